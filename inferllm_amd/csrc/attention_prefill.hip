@@ -58,6 +58,25 @@ __device__ __forceinline__ float pf_soft_cap(float x, float cap_log2) {
     return cap_log2 * (1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e));
 }
 
+// The (sequence, head) pair that place `slot_id % hb_per_xcd` of XCD `xcd` works on; false: none.
+// An XCD takes the same heads of every sequence (nh / 8 of them where 8 divides nh, neighbours, so
+// that a group shares its keys in one L2), never whole sequences: lengths of 64 to 4,096 tokens in
+// a batch of 8 (32 heads on 8) had the longest sequence on one XCD of eight: 1,225 us alone
+// instead of 322, and 41 ms of a 152 ms prompt step of 32 layers.
+__device__ __forceinline__ bool pf_pair(int xcd, int slot_id, int hb_per_xcd, int n_hb, int nh, int& h, int& b) {
+    const int j = slot_id % hb_per_xcd;
+    if (nh % 8 == 0) {
+        const int per = nh / 8;                 // hb_per_xcd = per * sequences
+        h = xcd * per + j % per;
+        b = j / per;
+        return true;
+    }
+    const int i = xcd * hb_per_xcd + j, n_seqs = n_hb / nh;
+    h = i / n_seqs;
+    b = i % n_seqs;
+    return i < n_hb;
+}
+
 template <int HD, bool PAGED>
 __global__ void __launch_bounds__(256, (HD <= 128 ? 2 : 1))
 attn_prefill_mfma_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out,
@@ -72,17 +91,16 @@ attn_prefill_mfma_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ ou
     __shared__ __attribute__((aligned(16))) bf16_t ks[PF_BN * KLD];
     __shared__ __attribute__((aligned(16))) bf16_t vts[DB * 32 * VLD];
 
-    // XCD x takes the (sequence, head) pairs [x * hb_per_xcd, (x + 1) * hb_per_xcd); within
-    // it, slots run over those pairs first and over query blocks, last block first, second
+    // XCD x takes hb_per_xcd of the (sequence, head) pairs; within it, slots run over those pairs
+    // first and over query blocks, last block first, second
     const int xcd = blockIdx.x % 8, slot_id = blockIdx.x / 8;
-    const int hb = xcd * hb_per_xcd + slot_id % hb_per_xcd;
-    if (hb >= n_hb) return;
+    int h, b;
+    if (!pf_pair(xcd, slot_id, hb_per_xcd, n_hb, nh, h, b)) return;
     // heavy half first (last query blocks, descending), then the light half ascending: when
     // all blocks are resident at once, the blocks that share a CU add up to about the same
     // (`zigzag`); with more blocks than fit at once, plain heaviest-first is better
     const int qi = slot_id / hb_per_xcd, top = zigzag ? (n_qblk + 1) / 2 : n_qblk;
     const int qb = qi < top ? n_qblk - 1 - qi : qi - top;
-    const int h = hb % nh, b = hb / nh;
     const int start = cu[b], len = cu[b + 1] - start;
     const int q0 = qb * PF_BM;
     if (q0 >= len) return;
@@ -305,11 +323,10 @@ attn_prefill_mfma2_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ o
     extern __shared__ __attribute__((aligned(16))) bf16_t pf_lds[];
 
     const int xcd = blockIdx.x % 8, slot_id = blockIdx.x / 8;
-    const int hb = xcd * hb_per_xcd + slot_id % hb_per_xcd;
-    if (hb >= n_hb) return;
+    int h, b;
+    if (!pf_pair(xcd, slot_id, hb_per_xcd, n_hb, nh, h, b)) return;
     const int qi = slot_id / hb_per_xcd, top = zigzag ? (n_qblk + 1) / 2 : n_qblk;
     const int qb = qi < top ? n_qblk - 1 - qi : qi - top;
-    const int h = hb % nh, b = hb / nh;
     const int start = cu[b], len = cu[b + 1] - start;
     const int q0 = qb * PF_BM;
     if (q0 >= len) return;

@@ -559,6 +559,24 @@ def test_gemm_f32_mfma(ydt, M, N, K):
     assert not ops().gemm_f32_mfma_fits(x.to(DEV).to(torch.bfloat16), w.to(DEV))
 
 
+@pytest.mark.parametrize("nh,nkv,lens", [(8, 8, [70, 1, 200]), (16, 2, [129, 40]), (5, 5, [3, 300, 64, 130]), (12, 4, [128, 127])])
+def test_attn_prefill_ragged_batches(nh, nkv, lens):
+    """Every (sequence, head) pair of a ragged batch is worked on once, whether 8 divides the heads (an
+    XCD takes the same heads of every sequence) or not: each sequence's rows are the bits of the
+    sequence alone."""
+    hd, T = 64, sum(lens)
+    qkv = rnd(T, (nh + 2 * nkv) * hd, seed=3).to(torch.bfloat16).to(DEV)
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    got = ops().attn_prefill(qkv, i32(cu), len(lens), max(lens), nh, nkv, hd, 0.125, 0)
+    close(got, R.attn_prefill(qkv.cpu(), torch.tensor(cu), len(lens), max(lens), nh, nkv, hd, 0.125, 0), torch.bfloat16)
+    for a, b in zip(cu, cu[1:]):
+        alone = ops().attn_prefill(qkv[a:b].contiguous(), i32([0, b - a]), 1, b - a, nh, nkv, hd, 0.125, 0)
+        assert torch.equal(got[a:b], alone)
+
+
 def _decode_copy(w, mode="plain", **geometry):
     o = ops()
     return o.Weight(w, o.tile_weight(w, o.tile_rows(w.shape[0], mode, **geometry)), mode)
