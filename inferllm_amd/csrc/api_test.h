@@ -12,6 +12,10 @@ extern "C" {
 // The sums are the same bits either way.
 void illm_set_rows_f32_tiles(int tiles);
 
+// illm_gemm_f32_mfma: outputs of a block along each side, 64 or 128 (0: the library's choice).  The
+// sums are the same bits either way.
+void illm_set_f32_tile(int t);
+
 // Whether float32 prompts with head sizes 32, 64, 96 and 128 take the attention kernel on the
 // matrix cores' float32 instruction (1, default) or the multiply-add kernel of every other size (0).
 void illm_set_attn_f32_mfma(int on);

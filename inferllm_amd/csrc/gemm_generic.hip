@@ -10,6 +10,8 @@
 //
 // The reference's float product is the same sum (src/kern/naive/naive.cpp:363-379);
 // its GPU path calls cublasSgemm (src/kern/gpu/kernel_gpu.cu:420-435).
+#include <mutex>
+
 #include "api.h"
 #include "api_test.h"
 #include "common.h"
@@ -85,99 +87,160 @@ extern "C" int illm_gemm_generic(const void* X, int x_dt, const void* W, int w_d
 // ---------------------------------------------------------------- many rows, float32
 // The same product for float32 X and W with K a multiple of 16, on the matrix cores' float32
 // instruction (MFMA 32x32x2: float32 operands, float32 products and sums; nothing is rounded to
-// a shorter type).  The multiply-add tile above reaches 45 TFLOP/s, 0.57 of what the vector units
-// give without packed instructions; the matrix cores' float32 rate is twice the vector units'.
-// A block of four waves takes 128 x 128 outputs, a wave 64 x 64 (2 x 2 MFMA tiles); both
-// operands go through LDS k-major (16 k a stage, two buffers, the next stage's loads in flight
-// while this one is multiplied).  The MFMA's rows are W's (n) and its columns X's (m), so a lane
-// holds 4 consecutive n of one m: 16-byte stores.  An output element is summed over k in
-// ascending pairs whatever its row's place in the batch.
+// a shorter type).  A block of four waves takes T x T outputs, a wave T/2 x T/2.  Both operands go
+// through LDS as rows of 32 k (two buffers, the next two stages' loads in flight in two register
+// sets while this one is multiplied), read 16 bytes a lane: half-wave h takes k 8 c + 4 h .. + 3
+// of a chunk of 8, so one LDS read is the operand of four MFMAs and the k of an MFMA are
+// 8 c + j and 8 c + 4 + j.  The MFMA's rows are W's (n) and its columns X's (m), so a lane
+// holds 4 consecutive n of one m: 16-byte stores.  An output element is summed over k in one
+// order whatever its row's place, the number of rows or T.
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4v_t __attribute__((ext_vector_type(4)));
 
-#define FM_T 128     // outputs of a block along m and along n
-#define FM_K 16      // k a stage
-#define FM_LD 130    // LDS row stride in floats (4 * FM_LD = 8 mod 32: the stores of a half-wave,
-                     // 8 rows x 4 k-quads, fall into 32 different banks)
+#define FM_K 32      // k a stage
+#define FM_LD 36     // LDS row stride in floats: the 16-byte reads of 8 rows fall into 32 different banks
 
-__global__ void __launch_bounds__(256)
+template <int T>
+__global__ void __launch_bounds__(256, 2)
 gemm_f32_mfma_kernel(const float* __restrict__ X, const float* __restrict__ W, void* __restrict__ Y,
-                     int y_dt, int M, int N, int K) {
-    __shared__ float xs[2][FM_K][FM_LD];
-    __shared__ float ws[2][FM_K][FM_LD];
+                     int y_dt, int M, int N, int K, int m_tiles) {
+    constexpr int NT = T / 64;                 // MFMA tiles of a wave along each side
+    constexpr int NL = T / 32;                 // 16-byte pieces a thread brings of each operand a stage
+    extern __shared__ __attribute__((aligned(16))) float lds[];         // [buffer][X rows, W rows][FM_LD]
+    constexpr int BUF = 2 * T * FM_LD;
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
     const int r = lane & 31, kh = lane >> 5;
     const int wm = wave & 1, wn = wave >> 1;
-    const int m0 = blockIdx.y * FM_T, n0 = blockIdx.x * FM_T;
+    // the blocks that share rows of W run next to each other on one XCD (block ids go round the 8)
+    const int xcd = blockIdx.x & 7, j8 = blockIdx.x >> 3;
+    const int m0 = (j8 % m_tiles) * T, n0 = ((j8 / m_tiles) * 8 + xcd) * T;
+    if (n0 >= N) return;
 
-    // staging: thread t brings 4 k (quad t % 4) of rows t / 4 and t / 4 + 64 of both operands;
-    // rows beyond the matrix read its last row (their outputs are not stored)
-    const int s_row = tid >> 2, s_kq = tid & 3;
-    const float* xsrc[2];
-    const float* wsrc[2];
+    // staging: thread t brings 4 k (quad t % 8) of rows t / 8 + 32 e of both operands, the stage's k as
+    // a scalar offset (address and mask instructions a stage cost a tenth of the time); rows beyond the matrix read its last row (their
+    // outputs are not stored).  K = 32 n + 16: the last stage's loads start 16 k earlier and count
+    // from the 17th k on; stages past the end are zeros.
+    const int s_row = tid >> 3, s_k = (tid & 7) * 4;
+    uint32_t xo[NL], wo[NL];                   // bytes from the block's first row
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        xsrc[e] = X + (size_t)min(m0 + s_row + 64 * e, M - 1) * K + s_kq * 4;
-        wsrc[e] = W + (size_t)min(n0 + s_row + 64 * e, N - 1) * K + s_kq * 4;
+    for (int e = 0; e < NL; ++e) {
+        xo[e] = (uint32_t)(min(s_row + 32 * e, M - 1 - m0) * K + min(s_k, K - 4)) * 4u;
+        wo[e] = (uint32_t)(min(s_row + 32 * e, N - 1 - n0) * K + min(s_k, K - 4)) * 4u;
     }
-    float4 xg[2], wg[2];
-    auto fetch = [&](int k0) __attribute__((always_inline)) {
+    const char* const xbase = (const char*)(X + (size_t)m0 * K);
+    const char* const wbase = (const char*)(W + (size_t)n0 * K);
+    const bool in_part = K >= FM_K ? s_k >= FM_K / 2 : s_k < K;
+    struct Set { f32x4v_t x[NL], w[NL]; };
+    const int full = K / FM_K, stages = (K + FM_K - 1) / FM_K;
+    auto fetch = [&](Set& g, int st) __attribute__((always_inline)) {
+        const size_t at = (size_t)max(0, min(st * FM_K, K - FM_K)) * 4;
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            xg[e] = *(const float4*)(xsrc[e] + k0);
-            wg[e] = *(const float4*)(wsrc[e] + k0);
+        for (int e = 0; e < NL; ++e) {
+            g.x[e] = *(const f32x4v_t*)(xbase + at + xo[e]);
+            g.w[e] = *(const f32x4v_t*)(wbase + at + wo[e]);
         }
     };
-    auto stage = [&](int buf) __attribute__((always_inline)) {
+    auto stage = [&](Set& g, int st) __attribute__((always_inline)) {
+        float* xs = lds + (st & 1) * BUF + s_row * FM_LD + s_k;
+        if (st >= full) {
+            const bool in = st < stages && in_part;
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int row = s_row + 64 * e;
-            xs[buf][s_kq * 4 + 0][row] = xg[e].x; xs[buf][s_kq * 4 + 1][row] = xg[e].y;
-            xs[buf][s_kq * 4 + 2][row] = xg[e].z; xs[buf][s_kq * 4 + 3][row] = xg[e].w;
-            ws[buf][s_kq * 4 + 0][row] = wg[e].x; ws[buf][s_kq * 4 + 1][row] = wg[e].y;
-            ws[buf][s_kq * 4 + 2][row] = wg[e].z; ws[buf][s_kq * 4 + 3][row] = wg[e].w;
+            for (int e = 0; e < NL; ++e) {
+                const f32x4v_t zero = {0.f, 0.f, 0.f, 0.f};
+                g.x[e] = in ? g.x[e] : zero;
+                g.w[e] = in ? g.w[e] : zero;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < NL; ++e) {
+            *(f32x4v_t*)(xs + 32 * e * FM_LD) = g.x[e];
+            *(f32x4v_t*)(xs + (T + 32 * e) * FM_LD) = g.w[e];
         }
     };
-    f32x16_t acc[2][2];                    // [n tile][m tile]
+    f32x16_t acc[NT][NT];                    // [n tile][m tile]
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NT; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    struct Ops { f32x4v_t a[NT], b[NT]; };     // a wave's operands of 8 k
+    auto operands = [&](Ops& o, int st, int c) __attribute__((always_inline)) {
+        const float* xb = lds + (st & 1) * BUF + (wm * (T / 2) + r) * FM_LD + 4 * kh + 8 * c;
+        const float* wb = lds + (st & 1) * BUF + (T + wn * (T / 2) + r) * FM_LD + 4 * kh + 8 * c;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) o.a[i] = *(const f32x4v_t*)(wb + 32 * i * FM_LD);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) o.b[j] = *(const f32x4v_t*)(xb + 32 * j * FM_LD);
+    };
+    auto multiply = [&](const Ops& o) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(o.a[i][s], o.b[j][s], acc[i][j], 0, 0, 0);
+        if constexpr (T == 64) __builtin_amdgcn_sched_barrier(0);
+    };
 
-    fetch(0);
-    stage(0);
+    Set g0, g1;
+    Ops o0, o1;
+    fetch(g0, 0);
+    fetch(g1, 1);
+    stage(g0, 0);
     __syncthreads();
-    int buf = 0;
-    for (int k0 = 0; k0 < K; k0 += FM_K, buf ^= 1) {
-        const bool more = k0 + FM_K < K;
-        if (more) fetch(k0 + FM_K);
+    // Stage st is multiplied while st + 1 waits in one register set and st + 2 is asked for into the
+    // other (stages past the end are zeros).  T = 64: a chunk's operands are read while the chunk
+    // before it is multiplied, the next stage's first ones too: its writes and the barrier stand
+    // before this stage's last products, so that a block alone on its compute unit goes on (256 rows,
+    // 12288 x 4096: 243 -> 226 us).  T = 128: the other block of the compute unit fills the gap, and
+    // the order by stages is the faster one (2,048 rows of 4096 x 11008: 137 TFLOP/s against 125).
+    auto turn = [&](Set& next, Set& after, int st) __attribute__((always_inline)) {
+        fetch(after, st + 2);
+        if constexpr (T == 64) {
+            operands(o1, st, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(o0);
+            operands(o0, st, 2);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(o1);
+            operands(o1, st, 3);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(o0);
+            stage(next, st + 1);
+            __syncthreads();
+            operands(o0, st + 1, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(o1);
+        } else {
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < FM_K / 2; ++s) {
-            float a[2], b[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) a[i] = ws[buf][2 * s + kh][wn * 64 + 32 * i + r];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) b[j] = xs[buf][2 * s + kh][wm * 64 + 32 * j + r];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+            for (int c = 0; c < FM_K / 8; ++c) {
+                Ops o;
+                operands(o, st, c);
+                multiply(o);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            stage(next, st + 1);
+            __syncthreads();
         }
-        if (more) stage(buf ^ 1);          // (last read before the barrier that ended the stage before)
-        __syncthreads();
+    };
+    if constexpr (T == 64) operands(o0, 0, 0);
+    for (int st = 0; st < stages; st += 2) {
+        turn(g1, g0, st);
+        turn(g0, g1, st + 1);
     }
-    // acc[i][j][v]: n = n0 + wn * 64 + 32 i + 8 (v / 4) + 4 kh + v % 4, m = m0 + wm * 64 + 32 j + r
+    // acc[i][j][v]: n = n0 + wn * T/2 + 32 i + 8 (v / 4) + 4 kh + v % 4, m = m0 + wm * T/2 + 32 j + r
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int m = m0 + wm * 64 + 32 * j + r;
+    for (int j = 0; j < NT; ++j) {
+        const int m = m0 + wm * (T / 2) + 32 * j + r;
         if (m >= M) continue;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < NT; ++i)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const int n = n0 + wn * 64 + 32 * i + 8 * g + 4 * kh;
+                const int n = n0 + wn * (T / 2) + 32 * i + 8 * g + 4 * kh;
                 const size_t at = (size_t)m * N + n;
                 if (n + 3 < N && (N & 3) == 0 && y_dt == ILLM_F32) {
                     *(float4*)((float*)Y + at) = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1],
@@ -191,16 +254,56 @@ gemm_f32_mfma_kernel(const float* __restrict__ X, const float* __restrict__ W, v
     }
 }
 
+static int g_f32_tile = 0;
+extern "C" void illm_set_f32_tile(int t) { g_f32_tile = t == 64 || t == 128 ? t : 0; }
+
+// A kernel that needs more dynamic LDS than it may have without asking: asked for once per device.
+template <int T>
+static int f32_lds_ready(size_t bytes) {
+    static bool ready[64] = {};
+    static std::mutex lock;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return ILLM_ERR_LAUNCH;
+    std::lock_guard<std::mutex> hold(lock);
+    if (!ready[dev]) {
+        if (hipFuncSetAttribute((const void*)gemm_f32_mfma_kernel<T>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
+            return ILLM_ERR_LAUNCH;
+        ready[dev] = true;
+    }
+    return ILLM_OK;
+}
+
+template <int T>
+static int launch_f32_mfma(const float* X, const float* W, void* Y, int y_dt, int M, int N, int K, hipStream_t st) {
+    const long long mt = (M + T - 1) / T, nt = (N + T - 1) / T, blocks = (nt + 7) / 8 * 8 * mt;
+    if (blocks > 0x7fffffffLL) return ILLM_ERR_ARG;
+    const size_t lds = (size_t)4 * T * FM_LD * sizeof(float);
+    const int rc = f32_lds_ready<T>(lds);
+    if (rc != ILLM_OK) return rc;
+    hipLaunchKernelGGL(gemm_f32_mfma_kernel<T>, dim3((unsigned)blocks), dim3(256), lds, st, X, W, Y, y_dt, M, N, K, (int)mt);
+    return illm_launch_status();
+}
+
 // float32 X [M, K] and W [N, K], K % 16 == 0; Y float32 or bfloat16.  Else ILLM_ERR_ARG.
 extern "C" int illm_gemm_f32_mfma(const float* X, const float* W, void* Y, int y_dt, int M, int N,
                                   int K, void* stream) {
-    if (M <= 0 || N <= 0 || K <= 0 || (K % FM_K) || !illm_dtype_ok(y_dt) || !X || !W || !Y)
+    if (M <= 0 || N <= 0 || K <= 0 || (K % 16) || !illm_dtype_ok(y_dt) || !X || !W || !Y)
         return ILLM_ERR_ARG;
-    const int gy = (M + FM_T - 1) / FM_T;
-    if (gy > 65535) return ILLM_ERR_ARG;
-    hipLaunchKernelGGL(gemm_f32_mfma_kernel, dim3((N + FM_T - 1) / FM_T, gy), dim3(256), 0,
-                       (hipStream_t)stream, X, W, Y, y_dt, M, N, K);
-    return illm_launch_status();
+    const long long m128 = (M + 127) / 128, b128 = m128 * ((N + 127) / 128);
+    const long long b64 = (long long)((M + 63) / 64) * ((N + 63) / 64);
+    if (m128 > 65535) return ILLM_ERR_ARG;
+    if (K >= 1 << 22)                      // a block's rows would pass 2 GiB
+        return illm_gemm_generic(X, ILLM_F32, W, ILLM_F32, Y, y_dt, M, N, K, stream);
+    // Blocks of 128 x 128 finish in rounds of one a compute unit (256 blocks of K = 4,096: 275 us, 512
+    // 505, 768 776), those of 64 x 64 in rounds of a quarter of that at 0.9 of the rate (256 88 us, 512
+    // 155, 1,024 283): the larger ones where their rounds are nearly full.  Measured at 129 to 2,048
+    // rows of the 7B shapes; with 128 x 128 alone, stages of 16 k and one stage ahead, 256 rows took
+    // 314 us (4096 x 4096), 320 (12288 x 4096), 830 (4096 x 11008) and 543 (22016 x 4096), now 88, 223,
+    // 240 and 425; 2,048 rows 546, 1,590, 1,480 and 3,040, now 510, 1,510, 1,345 and 2,780.
+    const bool big = g_f32_tile ? g_f32_tile == 128 : 10 * 1024 * ((b128 + 255) / 256) <= 11 * b64;
+    return big ? launch_f32_mfma<128>(X, W, Y, y_dt, M, N, K, (hipStream_t)stream)
+               : launch_f32_mfma<64>(X, W, Y, y_dt, M, N, K, (hipStream_t)stream);
 }
 
 
@@ -213,7 +316,6 @@ extern "C" int illm_gemm_f32_mfma(const float* X, const float* W, void* Y, int y
 // MFMA whose four k are 4 g + j + 16 q, the same four for both operands, so nothing is
 // permuted.  The waves' sums are added through LDS in wave order: the order of a sum depends on
 // K only, not on the row's place or on the number of rows.
-typedef float f32x4v_t __attribute__((ext_vector_type(4)));
 
 template <int RT, int CT>                      // tiles of 16 rows of X, tiles of 16 rows of W
 __global__ void __launch_bounds__(512)

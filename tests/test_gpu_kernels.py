@@ -559,6 +559,27 @@ def test_gemm_f32_mfma(ydt, M, N, K):
     assert not ops().gemm_f32_mfma_fits(x.to(DEV).to(torch.bfloat16), w.to(DEV))
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 16), (64, 64, 32), (65, 129, 48), (129, 64, 64), (192, 520, 80), (130, 1030, 112),
+                                   (257, 65, 4096)])
+def test_gemm_f32_mfma_tiles(M, N, K):
+    """Both block sizes of the many-row float32 product give the same bits, at edges of their tiles, of
+    a stage of 32 k and of the eight column tiles that go round the chip; against 64 bits within
+    sums of K products in any order (each within K 2^-24 of the sum of their magnitudes)."""
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+    want = x.double() @ w.double().t()
+    room = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    got = []
+    lib = ops()._lib()
+    try:
+        for tile in (64, 128):
+            lib.illm_set_f32_tile(tile)
+            got.append(ops().gemm_f32_mfma(x.to(DEV), w.to(DEV), torch.float32))
+    finally:
+        lib.illm_set_f32_tile(0)
+    assert torch.equal(got[0], got[1])
+    assert bool(((got[0].double().cpu() - want).abs() <= room).all())
+
+
 @pytest.mark.parametrize("nh,nkv,lens", [(8, 8, [70, 1, 200]), (16, 2, [129, 40]), (5, 5, [3, 300, 64, 130]), (12, 4, [128, 127])])
 def test_attn_prefill_ragged_batches(nh, nkv, lens):
     """Every (sequence, head) pair of a ragged batch is worked on once, whether 8 divides the heads (an
