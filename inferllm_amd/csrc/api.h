@@ -107,6 +107,13 @@ int illm_gemm_generic(const void* X, int x_dt, const void* W, int w_dt, void* Y,
 int illm_gemm_f32_mfma(const float* X, const float* W, void* Y, int y_dt, int M, int N, int K,
                        void* stream);
 
+// Products of up to 256 bfloat16 rows from row-major W, K % 64 == 0, N % 4 == 0 (csrc/gemm_tiles.hip): K
+// cut into `splits` parts (illm_gemm_tiles_splits(N, K), or any number that leaves no part empty) as
+// float32 planes [splits][M][N].
+int illm_gemm_tiles_splits(int N, int K);
+int illm_gemm_tiles_planes(const void* X, const void* W, float* Y, int M, int N, int K, int splits,
+                           void* stream);
+
 // The same product for M <= 128 rows of float32 X and W with K % 32 == 0, W read once, on the
 // matrix cores' float32 instruction with operands straight from memory.
 int illm_gemm_rows_f32_mfma(const float* X, const float* W, void* Y, int y_dt, int M, int N, int K,

@@ -775,6 +775,38 @@ def linear_planes(x: torch.Tensor, w: "Weight", splits: int = 0) -> torch.Tensor
     return y
 
 
+CUT_ROWS = (129, 256)     # rows `linear_cut` takes: below, `linear_planes` reads the decode copy; above, the
+                          # vendor GEMM has tiles enough
+CUT_MIN_K = 4096          # product and the norm that adds the planes against the vendor GEMM and its norm, us
+                          # at 129 / 192 / 256 rows: 4096 x 4096 28 / 39 / 29 -> 20 / 23 / 26, 4096 x 11008
+                          # 60 / 61 / 58 -> 37 / 42 / 48, 8192 x 28672 315 / 242 / 328 -> 157 / 181 / 204,
+                          # 2048 x 5376 21 / 22 / 24 -> 16 / 18 / 20; 2048 x 2048 13 / 14 / 15 -> 13 / 14 / 17
+
+
+def linear_cut_fits(x, w) -> bool:
+    """Whether `linear_cut` takes these operands and is the faster way: 129 to 256 bfloat16 rows and a
+    row-major matrix (its plain copy) with few rows for its length (K >= N, K a multiple of 64)."""
+    w = plain_weight(w)
+    return (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and x.dim() == 2 and w.dim() == 2 and CUT_ROWS[0] <= x.shape[0] <= CUT_ROWS[1]
+            and x.shape[1] == w.shape[1] and w.is_contiguous() and w.shape[1] % 64 == 0
+            and w.shape[0] % 4 == 0 and CUT_MIN_K <= w.shape[1] and w.shape[0] <= w.shape[1]
+            and w.shape[0] <= _plan.rules.planes_most_cols and w.numel() * 2 < 0xffffffff)
+
+
+def linear_cut(x: torch.Tensor, w, splits: int = 0) -> torch.Tensor:
+    """x . w^T as float32 planes [S, M, N] whose sum over S is the product, for 129 to 256 rows
+    (csrc/gemm_tiles.hip, row-major w).  The planes go to `add_rmsnorm` as `delta`."""
+    x, w = x.contiguous(), plain_weight(w)
+    _gpu(x, w)
+    M, K = x.shape
+    N = w.shape[0]
+    S = splits or _lib().illm_gemm_tiles_splits(N, K)
+    y = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
+    _check(_lib().illm_gemm_tiles_planes(_p(x), _p(w), _p(y), M, N, K, S, _stream()), "linear_cut")
+    return y
+
+
 def linear(x, w, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     """y = x . w^T, w stored [out, in] (src/kern/naive/naive.cpp:363-379).  x may be
     `NormedRows`, w a `Weight`."""

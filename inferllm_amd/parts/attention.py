@@ -124,6 +124,9 @@ class Attention(Mixer):
         if (next_norm is not None and getattr(next_norm, "adds_planes", False)
                 and ops.linear_planes_fits(o, self.w_o) and ops.linear_planes_pays(o, self.w_o)):
             return ops.linear_planes(o, self.w_o)
+        if (next_norm is not None and getattr(next_norm, "adds_planes", False)
+                and ops.linear_cut_fits(o, self.w_o)):
+            return ops.linear_cut(o, self.w_o)
         if residual is not None and ops.linear_add_fits(o, self.w_o, residual):
             return ops.linear_add(o, self.w_o, residual,
                                   next_norm.rms_params() if next_norm is not None else None,

@@ -49,6 +49,9 @@ class SwiGLU(FeedForward):
         if (next_norm is not None and getattr(next_norm, "adds_planes", False)
                 and ops.linear_planes_fits(a, self.w_down) and ops.linear_planes_pays(a, self.w_down)):
             return ops.linear_planes(a, self.w_down)
+        if (next_norm is not None and getattr(next_norm, "adds_planes", False)
+                and ops.linear_cut_fits(a, self.w_down)):
+            return ops.linear_cut(a, self.w_down)
         if residual is not None and ops.linear_add_fits(a, self.w_down, residual):
             return ops.linear_add(a, self.w_down, residual,
                                   next_norm.rms_params() if next_norm is not None else None,

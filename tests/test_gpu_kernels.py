@@ -824,6 +824,27 @@ def test_linear_planes(M, N, K, splits, tiles_per_wave):
     torch.testing.assert_close(dev.cpu(), ref_x, atol=2e-4 * math.sqrt(K), rtol=1e-5)
 
 
+@pytest.mark.parametrize("M,N,K,splits", [(129, 64, 4096, 0), (192, 4096, 4096, 0), (193, 68, 4160, 3), (256, 132, 4096, 64),
+                                          (160, 260, 11008, 0), (1, 4, 64, 1), (200, 4096, 192, 3)])
+def test_linear_cut(M, N, K, splits):
+    """The product of 129 to 256 rows with K cut over blocks, from the row-major matrix: the planes add up
+    to x . w^T (any order of K float32 sums: K 2^-24 of the sum of magnitudes) at edges of the tiles, with
+    parts of one stage and of unequal length, and repeat bit for bit."""
+    o = ops()
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=1), rnd(N, K, dtype=torch.bfloat16, seed=2)
+    xd, wd = x.to(DEV), w.to(DEV)
+    planes = o.linear_cut(xd, wd, splits)
+    assert planes.dtype == torch.float32 and planes.shape[1:] == (M, N) and (not splits or planes.shape[0] == splits)
+    want = x.double() @ w.double().t()
+    room = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert bool(((planes.double().sum(0).cpu() - want).abs() <= room).all())
+    assert torch.equal(o.linear_cut(xd, o.Weight(wd), splits), planes)
+    fits = 129 <= M <= 256 and N <= K and K >= 4096
+    assert o.linear_cut_fits(xd, wd) == fits and not o.linear_cut_fits(xd.float(), wd)
+    with pytest.raises(Exception):
+        o.linear_cut(xd, wd, K // 64 + 1)                      # a part without a stage
+
+
 def test_linear_planes_refuses_what_it_does_not_take():
     o = ops()
     w = rnd(64, 256, dtype=torch.bfloat16).to(DEV)
