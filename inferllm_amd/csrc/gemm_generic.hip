@@ -89,13 +89,14 @@ extern "C" int illm_gemm_generic(const void* X, int x_dt, const void* W, int w_d
 // instruction (MFMA 32x32x2: float32 operands, float32 products and sums; nothing is rounded to
 // a shorter type).  A block of four waves takes T x T outputs, a wave T/2 x T/2.  Both operands go
 // through LDS as rows of 32 k (two buffers, the next two stages' loads in flight in two register
-// sets while this one is multiplied), read 16 bytes a lane: half-wave h takes k 8 c + 4 h .. + 3
-// of a chunk of 8, so one LDS read is the operand of four MFMAs and the k of an MFMA are
-// 8 c + j and 8 c + 4 + j.  The MFMA's rows are W's (n) and its columns X's (m), so a lane
-// holds 4 consecutive n of one m: 16-byte stores.  An output element is summed over k in one
-// order whatever its row's place, the number of rows or T.
+// sets while this one is multiplied), a chunk of 8 k as its even ones, then its odd ones, read 16
+// bytes a lane: half-wave 0 takes the even ones, so that one LDS read is the operand of four
+// MFMAs, each of two neighbouring k.  The MFMA's rows are W's (n) and its columns X's (m), so a
+// lane holds 4 consecutive n of one m: 16-byte stores.  An output element is summed over k in
+// ascending pairs whatever its row's place, the number of rows or T.
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef float f32x4v_t __attribute__((ext_vector_type(4)));
+typedef float f32x2v_t __attribute__((ext_vector_type(2)));
 
 #define FM_K 32      // k a stage
 #define FM_LD 36     // LDS row stride in floats: the 16-byte reads of 8 rows fall into 32 different banks
@@ -141,7 +142,7 @@ gemm_f32_mfma_kernel(const float* __restrict__ X, const float* __restrict__ W, v
         }
     };
     auto stage = [&](Set& g, int st) __attribute__((always_inline)) {
-        float* xs = lds + (st & 1) * BUF + s_row * FM_LD + s_k;
+        float* xs = lds + (st & 1) * BUF + s_row * FM_LD + (s_k & ~7) + (s_k & 4) / 2;
         if (st >= full) {
             const bool in = st < stages && in_part;
 #pragma unroll
@@ -153,8 +154,11 @@ gemm_f32_mfma_kernel(const float* __restrict__ X, const float* __restrict__ W, v
         }
 #pragma unroll
         for (int e = 0; e < NL; ++e) {
-            *(f32x4v_t*)(xs + 32 * e * FM_LD) = g.x[e];
-            *(f32x4v_t*)(xs + (T + 32 * e) * FM_LD) = g.w[e];
+            float* ws = xs + T * FM_LD;
+            *(f32x2v_t*)(xs + 32 * e * FM_LD) = (f32x2v_t){g.x[e][0], g.x[e][2]};
+            *(f32x2v_t*)(xs + 32 * e * FM_LD + 4) = (f32x2v_t){g.x[e][1], g.x[e][3]};
+            *(f32x2v_t*)(ws + 32 * e * FM_LD) = (f32x2v_t){g.w[e][0], g.w[e][2]};
+            *(f32x2v_t*)(ws + 32 * e * FM_LD + 4) = (f32x2v_t){g.w[e][1], g.w[e][3]};
         }
     };
     f32x16_t acc[NT][NT];                    // [n tile][m tile]
@@ -195,7 +199,7 @@ gemm_f32_mfma_kernel(const float* __restrict__ X, const float* __restrict__ W, v
     // before it is multiplied, the next stage's first ones too: its writes and the barrier stand
     // before this stage's last products, so that a block alone on its compute unit goes on (256 rows,
     // 12288 x 4096: 243 -> 226 us).  T = 128: the other block of the compute unit fills the gap, and
-    // the order by stages is the faster one (2,048 rows of 4096 x 11008: 137 TFLOP/s against 125).
+    // the order by stages is the faster one (2,048 rows of 4096 x 11008: 1,345 against 1,474 us).
     auto turn = [&](Set& next, Set& after, int st) __attribute__((always_inline)) {
         fetch(after, st + 2);
         if constexpr (T == 64) {
@@ -295,12 +299,12 @@ extern "C" int illm_gemm_f32_mfma(const float* X, const float* W, void* Y, int y
     if (m128 > 65535) return ILLM_ERR_ARG;
     if (K >= 1 << 22)                      // a block's rows would pass 2 GiB
         return illm_gemm_generic(X, ILLM_F32, W, ILLM_F32, Y, y_dt, M, N, K, stream);
-    // Blocks of 128 x 128 finish in rounds of one a compute unit (256 blocks of K = 4,096: 275 us, 512
-    // 505, 768 776), those of 64 x 64 in rounds of a quarter of that at 0.9 of the rate (256 88 us, 512
-    // 155, 1,024 283): the larger ones where their rounds are nearly full.  Measured at 129 to 2,048
+    // Blocks of 128 x 128 finish in rounds of one a compute unit (256 blocks of K = 4,096: 280 us, 512
+    // 535, 768 800), those of 64 x 64 in rounds of a quarter of that at 0.9 of the rate (256 91 us, 512
+    // 157, 1,024 300): the larger ones where their rounds are nearly full.  Measured at 129 to 2,048
     // rows of the 7B shapes; with 128 x 128 alone, stages of 16 k and one stage ahead, 256 rows took
-    // 314 us (4096 x 4096), 320 (12288 x 4096), 830 (4096 x 11008) and 543 (22016 x 4096), now 88, 223,
-    // 240 and 425; 2,048 rows 546, 1,590, 1,480 and 3,040, now 510, 1,510, 1,345 and 2,780.
+    // 314 us (4096 x 4096), 318 (12288 x 4096), 829 (4096 x 11008) and 545 (22016 x 4096), now 91, 236,
+    // 249 and 438; 2,048 rows 562, 1,584, 1,447 and 2,973, now 540, 1,585, 1,428 and 2,894.
     const bool big = g_f32_tile ? g_f32_tile == 128 : 10 * 1024 * ((b128 + 255) / 256) <= 11 * b64;
     return big ? launch_f32_mfma<128>(X, W, Y, y_dt, M, N, K, (hipStream_t)stream)
                : launch_f32_mfma<64>(X, W, Y, y_dt, M, N, K, (hipStream_t)stream);
