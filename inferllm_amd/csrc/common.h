@@ -82,6 +82,19 @@ __device__ __forceinline__ uint4 ld16_stream(const void* p) {
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// A buffer of `bytes` (at most 4 GiB) from p on: loads beyond it give zeros.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t illm_buffer(const void* p, size_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)(uint32_t)min(bytes, (size_t)0xffffffffu), 0x00020000);
+}
+
+// 16 bytes a lane from memory straight into LDS: lane l's land at to + l.  lane_at and stage_at (the same
+// in all lanes) are byte offsets into the buffer.
+__device__ __forceinline__ void ld16_lds(__amdgpu_buffer_rsrc_t rs, illm_u32x4_t* to, uint32_t lane_at,
+                                         uint32_t stage_at) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)to, 16, (int)lane_at,
+                                             (int)stage_at, 0, 0);
+}
+
 // The wave's number within its block, as a value the compiler knows to be the same in all
 // lanes: loops and branches on it run on the scalar unit instead of under lane masks.
 __device__ __forceinline__ int wave_index() {

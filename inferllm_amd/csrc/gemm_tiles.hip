@@ -19,16 +19,6 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 #define GT_K 64                                   // k a stage
 
-// A buffer of `bytes` from p on: loads beyond it give zeros.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t gt_buffer(const void* p, size_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)(uint32_t)min(bytes, (size_t)0xffffffffu), 0x00020000);
-}
-
-// 16 bytes a lane straight into LDS: lane l's bytes land at to + l.
-__device__ __forceinline__ void gt_load(__amdgpu_buffer_rsrc_t rs, illm_u32x4_t* to, uint32_t lane_at, uint32_t stage_at) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)to, 16, (int)lane_at, (int)stage_at, 0, 0);
-}
-
 // TM x TN: rows of X and of W a block takes; WM x WN waves; NS stages in LDS.
 template <int TM, int TN, int WM, int WN, int NS>
 __global__ void __launch_bounds__(64 * WM * WN, 1)
@@ -49,8 +39,8 @@ gemm_tiles_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, fl
 
     // A load instruction brings 8 rows of 128 bytes; 16-byte piece c of row t stands at place c ^ (t % 8)
     // of the row, so that the 16 rows an MFMA operand reads at once lie in different banks.
-    const __amdgpu_buffer_rsrc_t xr = gt_buffer(X, (size_t)M * K * 2);
-    const __amdgpu_buffer_rsrc_t wr = gt_buffer(W, (size_t)N * K * 2);
+    const __amdgpu_buffer_rsrc_t xr = illm_buffer(X, (size_t)M * K * 2);
+    const __amdgpu_buffer_rsrc_t wr = illm_buffer(W, (size_t)N * K * 2);
     uint32_t xo[LX], wo[LW];
     const int lr = lane >> 3, lc = (lane & 7) ^ lr;
 #pragma unroll
@@ -60,9 +50,9 @@ gemm_tiles_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, fl
     auto load = [&](illm_u32x4_t* b, int s) __attribute__((always_inline)) {
         const uint32_t at = (uint32_t)min(s, last) * (GT_K * 2);               // (past the end: not used)
 #pragma unroll
-        for (int i = 0; i < LW; ++i) gt_load(wr, b + (TM + (i * WAVES + wave) * 8) * 8, wo[i], at);
+        for (int i = 0; i < LW; ++i) ld16_lds(wr, b + (TM + (i * WAVES + wave) * 8) * 8, wo[i], at);
 #pragma unroll
-        for (int i = 0; i < LX; ++i) gt_load(xr, b + (i * WAVES + wave) * 64, xo[i], at);
+        for (int i = 0; i < LX; ++i) ld16_lds(xr, b + (i * WAVES + wave) * 64, xo[i], at);
     };
     f32x4_t acc[NT][MT];
 #pragma unroll

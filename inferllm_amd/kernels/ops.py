@@ -1486,13 +1486,24 @@ MOE_MFMA_FROM = 0        # (token, choice) pairs an expert on average from which
                          # K took 253 + 166 us for 64 tokens, bound by its sums across lanes)
 
 
+MOE_TILES_FROM = 1.5     # pairs an expert on average from which the kernel with both operands in LDS, in
+                         # tiles of 128 pairs, takes bfloat16 experts whose sizes are multiples of 64
+                         # (64 experts of 1408 x 2048, 6 a token, both products, us; tiles of 16 to 64
+                         # pairs -> of 128: 8 tokens 159 -> 164, 16 217 -> 206, 64 303 -> 236, 300 387
+                         # -> 252, 2,964 1,023 -> 608; the same bits)
+
+
 def _moe_tiling(dtype: torch.dtype, E: int, F: int, NP: int, n_exp: int):
     """(on the matrix cores?, rows a tile, upper bound of tiles) for NP (token, choice) pairs."""
-    # many pairs an expert (prompts): tiles of up to 64 rows; few (single tokens): tiles of 16 rows
-    # on the matrix cores, or of 8 rows with a wave a column (float32, odd sizes)
+    # tiles of 128 rows from MOE_TILES_FROM pairs an expert on, as far as a load's 32-bit offset reaches;
+    # other sizes: up to 64 rows; few pairs (single tokens): 16 rows on the matrix cores, or 8 rows with a
+    # wave a column (float32, odd sizes)
     per_expert = NP / max(1, n_exp)
     mfma = dtype == torch.bfloat16 and E % 32 == 0 and F % 32 == 0 and per_expert >= MOE_MFMA_FROM
     rows = (64 if per_expert >= 48 else 32 if per_expert >= 24 else 16) if mfma else _lib().illm_moe_tile_rows()
+    if mfma and per_expert >= MOE_TILES_FROM and E % 64 == 0 and F % 64 == 0 and 2 * NP * max(E, F) < 1 << 32 \
+            and 4 * (max(E, F) + 128) * max(E, F) < 1 << 32:
+        rows = 128
     return mfma, rows, max(1, min(NP, NP // rows + n_exp))
 
 

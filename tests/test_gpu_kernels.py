@@ -598,6 +598,55 @@ def test_attn_prefill_ragged_batches(nh, nkv, lens):
         assert torch.equal(got[a:b], alone)
 
 
+@pytest.mark.parametrize("T,E,F,NE,top,act", [(1, 64, 64, 2, 1, "silu"), (9, 128, 192, 4, 2, "clamped_swish"), (129, 192, 64, 1, 1, "silu"),
+                                              (300, 64, 320, 3, 2, "silu"), (257, 256, 128, 2, 2, "relu_squared"), (40, 448, 64, 5, 5, "silu")])
+def test_moe_tiles_of_128_pairs(T, E, F, NE, top, act):
+    """The experts' products in tiles of up to 128 pairs give the bits of the kernel for 16 pairs (the same
+    products summed over k in the same order), at tiles of one row, whole ones and remainders, column
+    blocks that are not full, with and without gates and weights on the input."""
+    o = ops()
+    gated = act != "relu_squared"
+    g = torch.Generator().manual_seed(5)
+    h = rnd(T, E, dtype=torch.bfloat16, seed=1).to(DEV)
+    wu = (rnd(NE, F * (2 if gated else 1), E, seed=2) * 0.1).to(torch.bfloat16).to(DEV)
+    wd = (rnd(NE, E, F, seed=3) * 0.1).to(torch.bfloat16).to(DEV)
+    idx = torch.stack([torch.randperm(NE, generator=g)[:top] for _ in range(T)]).to(torch.int32).to(DEV)
+    wt = torch.rand(T, top, generator=g).to(DEV) if act == "clamped_swish" else None
+    real, got = o._moe_tiling, []
+    try:
+        for rows in (16, 128):
+            o._moe_tiling = lambda dtype, e, f, np, n: (True, rows, max(1, min(np, np // rows + n)))
+            got.append(o.moe_experts(h, idx, wu, wd, None, act, 7.0 if act == "clamped_swish" else 0.0, wt))
+    finally:
+        o._moe_tiling = real
+    assert torch.equal(got[0], got[1]) and bool(torch.isfinite(got[1].float()).all())
+    assert real(torch.bfloat16, E, F, 2 * NE, NE)[1] == 128 and real(torch.bfloat16, E, F + 32, 2 * NE, NE)[1] != 128
+
+
+@pytest.mark.parametrize("xdt", DTYPES)
+@pytest.mark.parametrize("T,NE,K", [(1, 1, 4), (8, 64, 2048), (9, 65, 2052), (16, 7, 6144), (17, 33, 260), (100, 64, 512)])
+def test_few_outputs_rows(xdt, T, NE, K):
+    """A router's product at the edges of its two kernels: 8 tokens a block, waves of 256 k, 4 outputs a
+    wave; float32 sums in any order (K 2^-24 of the sum of magnitudes)."""
+    x, w = rnd(T, K, dtype=xdt, seed=1), rnd(NE, K, seed=2)
+    got = ops().few_outputs_f32(x.to(DEV), w.to(DEV)).double().cpu()
+    room = (K + 8) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert bool(((got - x.double() @ w.double().t()).abs() <= room).all())
+
+
+def test_moe_route_places():
+    """The choice by places: ties go to the lower index, as in the search that odd scores (not finite, or
+    more than 64 outputs) take; weights are the scores."""
+    o = ops()
+    for NE in (1, 5, 64, 65):
+        z = (rnd(50, NE, seed=4) * 2).round().div(2).to(DEV)                 # many equal scores
+        top = min(6, NE)
+        idx, wt = o.moe_route(z, None, top)
+        want = torch.sort(torch.softmax(z.double().cpu(), -1).float(), dim=-1, descending=True, stable=True)
+        assert torch.equal(idx.long().cpu(), want.indices[:, :top])
+        torch.testing.assert_close(wt.cpu(), want.values[:, :top], atol=0, rtol=1e-5)
+
+
 def _decode_copy(w, mode="plain", **geometry):
     o = ops()
     return o.Weight(w, o.tile_weight(w, o.tile_rows(w.shape[0], mode, **geometry)), mode)
