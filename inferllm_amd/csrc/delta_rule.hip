@@ -283,29 +283,44 @@ delta_step_kernel(const float* __restrict__ qn, const float* __restrict__ kn,
         if (live && i0 + ii < dk) sp[(size_t)(i0 + ii) * dv] = s[ii];
 }
 
-// The same recurrence for long runs of tokens (16 parts a column, part p holding rows p, p + 16, ...).  What bounds it is the chain of
-// dependent operations a token, so nothing may wait for memory inside it: the k, q and decay rows of
-// DELTA_CHUNK tokens go through LDS in two buffers, the next chunk's loads (and its v and beta, in
-// registers) are issued before this chunk's arithmetic and stored after it.  One wave a block;
-// dynamic LDS: 2 * DELTA_CHUNK * 3 * 16 NS floats (with a removal vector 4 in place of 3).
+// The same recurrence for long runs of tokens.  A block of four waves takes 16 columns of the state, a wave
+// four of them, 16 parts a column, part p holding rows p, p + 16, ....  Nothing may wait for memory
+// inside the chain of a token's operations: the k, q and decay rows of DELTA_CHUNK tokens, the
+// block's columns of v and the tokens' factors go through LDS in two buffers, the next chunk's loads are
+// issued before this chunk's arithmetic and stored after it.  A part's rows lie together in LDS, up to four
+// a read; one decay for all rows (SCALAR) is one of the tokens' factors.
+// What bounded a wave with rows of its own, read word by word, was the number of its instructions (24 LDS
+// reads a token beside 24 multiply-adds, and all of a token's rows loaded for four columns): 64 heads of
+// 128 x 64, 8 sequences of 61 to 1,024 tokens, 765 -> 256 us; one sequence of 2,048, 16 delta-rule heads of
+// 128 x 128 with a decay a row, 804 -> 645 (there the chain of a token bounds it).  The same bits.
+// Dynamic LDS: 2 * delta_chunk_floats(..) floats.
 #define DELTA_CHUNK 8
-template <int NS, int RULE>
-__global__ void __launch_bounds__(64)
+static constexpr int delta_rows(int rule, bool scalar) { return 2 + (scalar ? 0 : 1) + (rule == RULE_REMOVAL ? 1 : 0); }
+static constexpr int delta_chunk_floats(int ns, int rule, bool scalar) {
+    return DELTA_CHUNK * delta_rows(rule, scalar) * 16 * ns + 18 * DELTA_CHUNK;
+}
+
+template <int NS, int RULE, bool SCALAR>
+__global__ void __launch_bounds__(256)
 delta_scan_long_kernel(const float* __restrict__ qn, const float* __restrict__ kn,
                        const float* __restrict__ vv, const float* __restrict__ beta,
                        const float* __restrict__ dec, int DW, float* __restrict__ state,
                        const int32_t* __restrict__ cu, const int32_t* __restrict__ seq_slot,
                        float* __restrict__ o, int G, int H, int dk, int dv, const float* __restrict__ removal) {
     constexpr bool CORRECT = RULE == RULE_DELTA || RULE == RULE_REMOVAL;
-    constexpr int NVEC = RULE == RULE_REMOVAL ? 4 : 3;  // rows a token in LDS
-    constexpr int PARTS = 16, COLS = 4;
-    constexpr int TC = RULE == RULE_REMOVAL ? DELTA_CHUNK / 2 : DELTA_CHUNK;    // (a fourth row a token: fewer tokens, or registers run out)
-    constexpr int DKP = PARTS * NS;                     // a row of k, q or decays in LDS, filled up
-    constexpr int JJ = (DKP + 63) / 64;                 // pieces of 64 floats in it
+    constexpr int NR = delta_rows(RULE, SCALAR);        // rows a token: k, q, the decays, the removal vector
+    constexpr int PARTS = 16, COLS = 4, TC = DELTA_CHUNK;
+    constexpr int DKP = PARTS * NS;                     // a row in LDS, filled up
+    constexpr int ELS = TC * NR * DKP, PER = (ELS + 255) / 256;
+    constexpr int CHUNK = delta_chunk_floats(NS, RULE, SCALAR);
     constexpr int NA = NS >= 4 ? 4 : NS;
-    extern __shared__ float stage[];                    // [2][TC][k | q | decay | removal?][DKP]
-    const int b = blockIdx.z, h = blockIdx.y, lane = threadIdx.x;
-    const int part = lane % PARTS, col = blockIdx.x * COLS + lane / PARTS;
+    constexpr int V = NS >= 4 ? 4 : NS;                 // rows a read; row p + 16 (V a + e) stands at (16 a + p) V + e
+    typedef float vec_t __attribute__((ext_vector_type(V)));
+    typedef float f32x4_t __attribute__((ext_vector_type(4)));
+    // [2][rows [TC][NR][DKP] | v [16 columns][TC] | beta [TC] | one decay a token [TC]]
+    extern __shared__ __attribute__((aligned(16))) float stage[];
+    const int b = blockIdx.z, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = wave_index();
+    const int part = lane % PARTS, wcol = wave * COLS + lane / PARTS, col = blockIdx.x * 16 + wcol;
     const int r0 = cu[b], n = cu[b + 1] - r0;
     if (n <= 0) return;
     const int slot = seq_slot[b], gh = h / (H / G);
@@ -313,100 +328,101 @@ delta_scan_long_kernel(const float* __restrict__ qn, const float* __restrict__ k
     float* sp = state + (((size_t)slot * H + h) * dk) * dv + col;
     float s[NS];
 #pragma unroll
-    for (int ii = 0; ii < NS; ++ii)      // row part + 16 ii: the 16 parts read neighbouring words of LDS
+    for (int ii = 0; ii < NS; ++ii)
         s[ii] = (live && part + PARTS * ii < dk) ? sp[(size_t)(part + PARTS * ii) * dv] : 0.f;
     const float* kbase = kn + ((size_t)r0 * G + gh) * dk;
     const float* qbase = qn + ((size_t)r0 * G + gh) * dk;
     const float* dbase = dec + ((size_t)r0 * H + h) * DW;
-    const float* vbase = vv + ((size_t)r0 * H + h) * dv + (live ? col : 0);
-    const float* bbase = beta + (size_t)r0 * H + h;
     const float* cbase = RULE == RULE_REMOVAL ? removal + ((size_t)r0 * H + h) * dk : nullptr;
-    const int cstep = H * dk;
-    float* op = o + ((size_t)r0 * H + h) * dv + col;
-    const int kstep = G * dk, dstep = H * DW, vstep = H * dv;
-    float sk[TC][JJ], sq[TC][JJ], sg[TC][JJ], sv[TC], sb[TC];
-    float sr[TC][RULE == RULE_REMOVAL ? JJ : 1];
+    const size_t kstep = (size_t)G * dk, dstep = (size_t)H * DW, cstep = (size_t)H * dk, vstep = (size_t)H * dv;
+
     // Rows beyond dk are filled with k = q = 0 and decay 1, and the tokens of the last chunk beyond
     // the sequence with k = q = v = beta = 0 and decay 1, which leave the state as it is: the
-    // arithmetic needs no bounds and no branches.  A whole chunk is loaded through pointers that
-    // step from token to token; the last, partial one with every row's place computed and clamped.
-    bool in_k[JJ];
+    // arithmetic needs no bounds and no branches.  (What is read for them lies within the tensors.)
+    const int row = tid % DKP, row_in = min(row, dk - 1);
+    const int first = DKP >= 64 ? __builtin_amdgcn_readfirstlane(tid / DKP) : tid / DKP;
+    const int at = ((row / PARTS / V) * PARTS + row % PARTS) * V + (row / PARTS) % V;
+    float sx[PER], sy = 0.f;
+    // element i of a thread: row `row` of kind x = (first + i 256 / DKP) of the chunk's TC * NR rows
+    auto load = [&](int t0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int jj = 0; jj < JJ; ++jj) in_k[jj] = lane + 64 * jj < dk;
-    const int jlast = dk - 1;
-#define DELTA_LOAD(T0)                                                                            \
-    if ((T0) + TC <= n) {                                                                         \
-        const float* kp = kbase + (size_t)(T0) * kstep;                                           \
-        const float* qp = qbase + (size_t)(T0) * kstep;                                           \
-        const float* dp = dbase + (size_t)(T0) * dstep;                                           \
-        const float* vp = vbase + (size_t)(T0) * vstep;                                           \
-        const float* bp = bbase + (size_t)(T0) * H;                                               \
-        const float* cp = cbase + (RULE == RULE_REMOVAL ? (size_t)(T0) * cstep : 0);              \
-        _Pragma("unroll") for (int tt = 0; tt < TC; ++tt) {                                       \
-            _Pragma("unroll") for (int jj = 0; jj < JJ; ++jj) {                                   \
-                const int j = in_k[jj] ? lane + 64 * jj : jlast;      /* read in bounds, then choose */ \
-                const float kx = kp[j], qx = qp[j], gx = dp[DW == 1 ? 0 : j];                     \
-                sk[tt][jj] = in_k[jj] ? kx : 0.f;                                                 \
-                sq[tt][jj] = in_k[jj] ? qx : 0.f;                                                 \
-                sg[tt][jj] = in_k[jj] ? gx : 1.f;                                                 \
-                if (RULE == RULE_REMOVAL) { const float cx = cp[j]; sr[tt][jj] = in_k[jj] ? cx : 0.f; } \
-            }                                                                                     \
-            sv[tt] = *vp;                                                                         \
-            sb[tt] = *bp;                                                                         \
-            kp += kstep; qp += kstep; dp += dstep; vp += vstep; bp += H;                          \
-            if (RULE == RULE_REMOVAL) cp += cstep;                                                \
-        }                                                                                         \
-    } else {                                                                                      \
-        _Pragma("unroll") for (int tt = 0; tt < TC; ++tt) {                                       \
-            const bool ok = (T0) + tt < n;                                                        \
-            const int at = ok ? (T0) + tt : n - 1;                                                \
-            _Pragma("unroll") for (int jj = 0; jj < JJ; ++jj) {                                   \
-                const int j = in_k[jj] ? lane + 64 * jj : jlast;                                  \
-                const bool use = ok && in_k[jj];                                                  \
-                sk[tt][jj] = use ? kbase[(size_t)at * kstep + j] : 0.f;                           \
-                sq[tt][jj] = use ? qbase[(size_t)at * kstep + j] : 0.f;                           \
-                sg[tt][jj] = use ? dbase[(size_t)at * dstep + (DW == 1 ? 0 : j)] : 1.f;           \
-                if (RULE == RULE_REMOVAL) sr[tt][jj] = use ? cbase[(size_t)at * cstep + j] : 0.f; \
-            }                                                                                     \
-            sv[tt] = ok ? vbase[(size_t)at * vstep] : 0.f;                                        \
-            sb[tt] = ok ? bbase[(size_t)at * H] : 0.f;                                            \
-        }                                                                                         \
-    }
-#define DELTA_STORE(BUF)                                                                          \
-    _Pragma("unroll") for (int tt = 0; tt < TC; ++tt) {                                           \
-        float* dst = stage + ((size_t)(BUF) * TC + tt) * NVEC * DKP;                              \
-        _Pragma("unroll") for (int jj = 0; jj < JJ; ++jj) {                                       \
-            const int j = lane + 64 * jj;                                                         \
-            if (j < DKP) {                                                                        \
-                dst[j] = sk[tt][jj]; dst[DKP + j] = sq[tt][jj]; dst[2 * DKP + j] = sg[tt][jj];    \
-                if (RULE == RULE_REMOVAL) dst[3 * DKP + j] = sr[tt][jj];                          \
-            }                                                                                     \
-        }                                                                                         \
-    }
-    DELTA_LOAD(0)
-    DELTA_STORE(0)
+        for (int i = 0; i < PER; ++i) {
+            const int x = first + i * 256 / DKP, tt = x / NR, kind = x % NR, tok = t0 + tt;
+            const int tc = tok < n ? tok : n - 1;
+            const bool ok = tok < n && row < dk;
+            const float* p = kind == 0 ? kbase + tc * kstep : qbase + tc * kstep;
+            if (!SCALAR && kind == 2) p = dbase + tc * dstep;
+            if (RULE == RULE_REMOVAL && kind == NR - 1) p = cbase + tc * cstep;
+            if (ELS % 256 == 0 || x < TC * NR) {
+                const float v = p[row_in];
+                sx[i] = ok ? v : !SCALAR && kind == 2 ? 1.f : 0.f;
+            }
+        }
+        if (tid < 16 * TC) {
+            const int tok = t0 + tid / 16, c = blockIdx.x * 16 + tid % 16;
+            const float v = vv[((size_t)r0 * H + h) * dv + (size_t)(tok < n ? tok : n - 1) * vstep + (c < dv ? c : dv - 1)];
+            sy = tok < n ? v : 0.f;
+        } else if (tid < 18 * TC) {
+            const int tok = t0 + tid % TC, tc = tok < n ? tok : n - 1;
+            const bool is_beta = tid < 17 * TC;
+            const float v = is_beta ? beta[(size_t)r0 * H + h + (size_t)tc * H] : SCALAR ? dbase[tc * dstep] : 1.f;
+            sy = tok < n ? v : is_beta ? 0.f : 1.f;
+        }
+    };
+    auto store = [&](int buf) __attribute__((always_inline)) {
+        float* dst = stage + buf * CHUNK;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int x = first + i * 256 / DKP;
+            if (ELS % 256 == 0 || x < TC * NR) dst[x * DKP + at] = sx[i];
+        }
+        if (tid < 16 * TC) dst[ELS + (tid % 16) * TC + tid / 16] = sy;
+        else if (tid < 18 * TC) dst[ELS + tid] = sy;
+    };
+    load(0);
+    store(0);
     __syncthreads();
-    const bool writes = part == 0 && live;
     for (int t0 = 0, buf = 0; t0 < n; t0 += TC, buf ^= 1) {
-        float cv[TC], cb[TC];
-#pragma unroll
-        for (int tt = 0; tt < TC; ++tt) { cv[tt] = sv[tt]; cb[tt] = sb[tt]; }
         const bool more = t0 + TC < n;
-        if (more) { DELTA_LOAD(t0 + TC) }
-        const float* src0 = stage + (size_t)buf * TC * NVEC * DKP + part;
-        float ovs[TC];
+        if (more) load(t0 + TC);
+        const float* chunk = stage + buf * CHUNK;
+        float cv[TC], cb[TC], cg[TC];
+#pragma unroll
+        for (int t4 = 0; t4 < TC; t4 += 4) {
+            const f32x4_t v4 = *(const f32x4_t*)(chunk + ELS + wcol * TC + t4), b4 = *(const f32x4_t*)(chunk + ELS + 16 * TC + t4);
+            const f32x4_t g4 = *(const f32x4_t*)(chunk + ELS + 17 * TC + t4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { cv[t4 + e] = v4[e]; cb[t4 + e] = b4[e]; cg[t4 + e] = g4[e]; }
+        }
+        auto rows_of = [&](const float* src, float* to) __attribute__((always_inline)) {
+#pragma unroll
+            for (int a = 0; a < NS / V; ++a) {
+                const vec_t r = *(const vec_t*)(src + a * PARTS * V);
+#pragma unroll
+                for (int e = 0; e < V; ++e) to[a * V + e] = r[e];
+            }
+        };
+        float mine = 0.f;                               // part t keeps token t's output
 #pragma unroll
         for (int tt = 0; tt < TC; ++tt) {
-            const float* src = src0 + tt * NVEC * DKP;
-            float kc[NS], pa[NA];
+            const float* src = chunk + tt * NR * DKP + part * V;
+            float kc[NS], qc[NS], gc[NS], rc[NS], pa[NA];
+            rows_of(src, kc);
+            rows_of(src + DKP, qc);
+            if (SCALAR) {
+#pragma unroll
+                for (int ii = 0; ii < NS; ++ii) gc[ii] = cg[tt];
+            } else {
+                rows_of(src + 2 * DKP, gc);
+            }
+            if (RULE == RULE_REMOVAL) rows_of(src + (NR - 1) * DKP, rc);
 #pragma unroll
             for (int a = 0; a < NA; ++a) pa[a] = 0.f;
 #pragma unroll
             for (int ii = 0; ii < NS; ++ii) {
-                kc[ii] = src[PARTS * ii];
                 if (RULE == RULE_BONUS) continue;
-                if (RULE != RULE_REMOVAL) s[ii] *= src[2 * DKP + PARTS * ii];
-                pa[ii % NA] = fmaf(s[ii], kc[ii], pa[ii % NA]);
+                if (RULE != RULE_REMOVAL) s[ii] *= gc[ii];
+                if (CORRECT) pa[ii % NA] = fmaf(s[ii], kc[ii], pa[ii % NA]);
             }
             float kv = 0.f;
             if (CORRECT) {
@@ -422,35 +438,30 @@ delta_scan_long_kernel(const float* __restrict__ qn, const float* __restrict__ k
 #pragma unroll
             for (int ii = 0; ii < NS; ++ii) {
                 if (RULE == RULE_BONUS) {
-                    pa[ii % NA] = fmaf(s[ii], src[DKP + PARTS * ii], pa[ii % NA]);
-                    s[ii] = fmaf(kc[ii], cv[tt], s[ii] * src[2 * DKP + PARTS * ii]);
+                    pa[ii % NA] = fmaf(s[ii], qc[ii], pa[ii % NA]);
+                    s[ii] = fmaf(kc[ii], cv[tt], s[ii] * gc[ii]);
                     continue;
                 }
                 if (RULE == RULE_REMOVAL) {
                     // (all but the last operation is off the chain that hangs on `read`)
-                    const float kept = fmaf(kc[ii], u, s[ii] * src[2 * DKP + PARTS * ii]);
-                    s[ii] = fmaf(-src[3 * DKP + PARTS * ii], read, kept);
+                    const float kept = fmaf(kc[ii], u, s[ii] * gc[ii]);
+                    s[ii] = fmaf(-rc[ii], read, kept);
                 } else
                     s[ii] = fmaf(kc[ii], u, s[ii]);
-                pa[ii % NA] = fmaf(s[ii], src[DKP + PARTS * ii], pa[ii % NA]);
+                pa[ii % NA] = fmaf(s[ii], qc[ii], pa[ii % NA]);
             }
             float ov = pa[0];
 #pragma unroll
             for (int a = 1; a < NA; ++a) ov += pa[a];
-            ovs[tt] = group_sum<PARTS>(ov);
-            if (RULE == RULE_BONUS) ovs[tt] = fmaf(cb[tt], cv[tt], ovs[tt]);
+            ov = group_sum<PARTS>(ov);
+            if (RULE == RULE_BONUS) ov = fmaf(cb[tt], cv[tt], ov);
+            mine = part == tt ? ov : mine;
         }
-        if (writes) {
-#pragma unroll
-            for (int tt = 0; tt < TC; ++tt)
-                if (t0 + tt < n) op[(size_t)tt * vstep] = ovs[tt];
-        }
-        op += (size_t)TC * vstep;
-        if (more) { DELTA_STORE(buf ^ 1) }
+        if (part < TC && live && t0 + part < n)
+            o[((size_t)r0 * H + h) * dv + (size_t)(t0 + part) * vstep + col] = mine;
+        if (more) store(buf ^ 1);
         __syncthreads();
     }
-#undef DELTA_LOAD
-#undef DELTA_STORE
 #pragma unroll
     for (int ii = 0; ii < NS; ++ii)
         if (live && part + PARTS * ii < dk) sp[(size_t)(part + PARTS * ii) * dv] = s[ii];
@@ -472,17 +483,19 @@ extern "C" int illm_gated_scan(const float* qn, const float* kn, const float* vv
     hipStream_t st = (hipStream_t)stream;
     if (max_rows >= 16) {
         const int ns = (dk + 15) / 16;
-        const size_t lds = (size_t)2 * DELTA_CHUNK * (removal ? 4 : 3) * 16 * (ns <= 1 ? 1 : ns <= 2 ? 2 : ns <= 4 ? 4 : ns <= 8 ? 8 : 16) * sizeof(float);
-        const dim3 grid((dv + 3) / 4, H, n_seqs);
-#define GOL_R(NS_, RULE_)                                                                         \
+        const dim3 grid((dv + 15) / 16, H, n_seqs);
+#define GOL_S(NS_, RULE_, SC_)                                                                    \
     do {                                                                                          \
+        constexpr size_t lds = (size_t)2 * delta_chunk_floats(NS_, RULE_, SC_) * sizeof(float);   \
         if (lds > 48 * 1024 &&                                                                    \
-            hipFuncSetAttribute((const void*)delta_scan_long_kernel<NS_, RULE_>,                  \
+            hipFuncSetAttribute((const void*)delta_scan_long_kernel<NS_, RULE_, SC_>,             \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) \
             return ILLM_ERR_LAUNCH;                                                               \
-        hipLaunchKernelGGL((delta_scan_long_kernel<NS_, RULE_>), grid, dim3(64), lds, st, qn, kn, vv, beta, \
+        hipLaunchKernelGGL((delta_scan_long_kernel<NS_, RULE_, SC_>), grid, dim3(256), lds, st, qn, kn, vv, beta, \
                            dec, DW, state, cu, seq_slot, o, G, H, dk, dv, removal);               \
     } while (0)
+#define GOL_R(NS_, RULE_)                                                                         \
+    do { if (DW == 1) GOL_S(NS_, RULE_, true); else GOL_S(NS_, RULE_, false); } while (0)
 #define GOL(NS_)                                                                                  \
     if (removal) GOL_R(NS_, RULE_REMOVAL);                                                        \
     else if (correct == 2) GOL_R(NS_, RULE_BONUS);                                                \
@@ -495,6 +508,7 @@ extern "C" int illm_gated_scan(const float* qn, const float* kn, const float* vv
         else { GOL(16); }
 #undef GOL
 #undef GOL_R
+#undef GOL_S
     } else {
         const int ns = (dk + 3) / 4;
         const dim3 grid((dv + 63) / 64, H, n_seqs);

@@ -647,6 +647,71 @@ def test_moe_route_places():
         torch.testing.assert_close(wt.cpu(), want.values[:, :top], atol=0, rtol=1e-5)
 
 
+@pytest.mark.parametrize("rule", ["plain", "delta", "bonus", "removal"])
+@pytest.mark.parametrize("G,H,dk,dv,vector", [(2, 4, 128, 20, False), (3, 3, 40, 17, True), (1, 1, 5, 3, False), (2, 2, 17, 16, True),
+                                              (1, 2, 130, 33, True)])
+def test_gated_scan_chunks(rule, G, H, dk, dv, vector):
+    """The recurrences for long runs: chunks of 8 tokens that end anywhere, blocks of 16 columns that are
+    not full, every count of rows a part, a decay a row or one for all; against a plain walk in 64 bits
+    (2,000 roundings of sums of a few units), and a run in two steps leaves the same bits."""
+    if rule == "removal":
+        G = H
+    lens = [16, 17, 33, 3, 24]
+    T = sum(lens)
+    q, k, v = rnd(T, G, dk, seed=1) * dk ** -0.5, rnd(T, G, dk, seed=2) * dk ** -0.5, rnd(T, H, dv, seed=3)
+    g = torch.Generator().manual_seed(4)
+    beta, dec = torch.rand(T, H, generator=g), torch.rand(T, H, dk if vector else 1, generator=g) * 0.4 + 0.6
+    rem = rnd(T, H, dk, seed=5) * dk ** -0.5 if rule == "removal" else None
+    start = rnd(len(lens), H, dk, dv, seed=6) * 0.5
+    want, r = torch.zeros(T, H, dv, dtype=torch.float64), 0
+    S = start.double().clone()
+    for b, n in enumerate(lens):
+        for t in range(r, r + n):
+            kk, qq = k[t].double().repeat_interleave(H // G, 0), q[t].double().repeat_interleave(H // G, 0)
+            vt, bt, gt = v[t].double(), beta[t].double()[:, None], dec[t].double()[:, :, None]
+            if rule == "bonus":
+                want[t] = (S[b] * qq[:, :, None]).sum(1) + bt * vt
+                S[b] = S[b] * gt + kk[:, :, None] * vt[:, None]
+                continue
+            if rule == "removal":
+                read = bt * (S[b] * kk[:, :, None]).sum(1)
+                S[b] = S[b] * gt + kk[:, :, None] * vt[:, None] - rem[t].double()[:, :, None] * read[:, None]
+            else:
+                S[b] = S[b] * gt
+                u = bt * (vt - ((S[b] * kk[:, :, None]).sum(1) if rule == "delta" else 0.0))
+                S[b] = S[b] + kk[:, :, None] * u[:, None]
+            want[t] = (S[b] * qq[:, :, None]).sum(1)
+        r += n
+
+    def run(spans, states):
+        """the rows `spans` (begin, end) of every sequence, its state in `states`"""
+        rows = torch.cat([torch.arange(a, b) for a, b in spans])
+        cu = [0]
+        for a, b in spans:
+            cu.append(cu[-1] + b - a)
+        i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+        d = [x[rows].contiguous().to(DEV) if x is not None else None for x in (q, k, v, beta, dec, rem)]
+        o = torch.empty(len(rows), H, dv, device=DEV)
+        lib, p = ops()._lib(), ops()._p
+        assert lib.illm_gated_scan(p(d[0]), p(d[1]), p(d[2]), p(d[3]), p(d[4]), dec.shape[2], p(states), p(i32(cu)),
+                                   p(i32(list(range(len(lens))))), p(o), len(lens), max(max(b - a for a, b in spans), 16), G, H, dk, dv,
+                                   {"plain": 0, "delta": 1, "bonus": 2, "removal": 0}[rule], p(d[5]), ops()._stream()) == 0
+        return o.cpu()
+
+    ends = [sum(lens[:i + 1]) for i in range(len(lens))]
+    spans = [(e - n, e) for e, n in zip(ends, lens)]
+    whole = start.clone().to(DEV)
+    got = run(spans, whole)
+    scale = want.abs().max()
+    assert float((got.double() - want).abs().max() / scale) < 2000 * 2.0 ** -24
+    assert float((whole.double().cpu() - S).abs().max() / S.abs().max()) < 2000 * 2.0 ** -24
+    halves = start.clone().to(DEV)
+    cuts = [(a, a + (b - a) // 2) for a, b in spans]
+    first, second = run(cuts, halves), run([(m, b) for (_, m), (_, b) in zip(cuts, spans)], halves)
+    assert torch.equal(halves, whole)
+    assert torch.equal(torch.cat([first[:cuts[0][1]], second[:lens[0] - cuts[0][1]]]), got[:lens[0]])
+
+
 def _decode_copy(w, mode="plain", **geometry):
     o = ops()
     return o.Weight(w, o.tile_weight(w, o.tile_rows(w.shape[0], mode, **geometry)), mode)
