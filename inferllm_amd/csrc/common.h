@@ -51,14 +51,43 @@ __device__ __forceinline__ void st_f(void* p, int dt, size_t i, float v) {
     else ((float*)p)[i] = v;
 }
 
-// four neighbouring elements (number 4 i4 .. 4 i4 + 3) as float32, and back
-__device__ __forceinline__ float4 ld_f4(const void* p, int dt, size_t i4) {
-    if (dt == ILLM_BF16) {
-        const uint2 u = ((const uint2*)p)[i4];
-        return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u),
-                           __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u));
-    }
-    return ((const float4*)p)[i4];
+// Four neighbouring elements (number 4 i4 .. 4 i4 + 3) as they lie in memory, without a branch on
+// the type: bfloat16 takes its 8 bytes twice.  A branch would hold the conversion, and with it the
+// wait for the load, so that loads that stand in a row would each take a trip to memory of their own.
+struct AnyRaw4 {
+    uint2 lo, hi;
+};
+
+__device__ __forceinline__ AnyRaw4 ld_raw4(const void* p, int dt, size_t i4) {
+    const char* at = (const char*)p + i4 * (dt == ILLM_BF16 ? 8 : 16);
+    AnyRaw4 r;
+    r.lo = *(const uint2*)at;
+    r.hi = *(const uint2*)(at + (dt == ILLM_BF16 ? 0 : 8));
+    return r;
+}
+
+// ... and as float32
+__device__ __forceinline__ float4 raw4_f(AnyRaw4 r, int dt) {
+    const bool half = dt == ILLM_BF16;
+    return make_float4(__uint_as_float(half ? r.lo.x << 16 : r.lo.x),
+                       __uint_as_float(half ? r.lo.x & 0xffff0000u : r.lo.y),
+                       __uint_as_float(half ? r.lo.y << 16 : r.hi.x),
+                       __uint_as_float(half ? r.lo.y & 0xffff0000u : r.hi.y));
+}
+
+// four neighbouring elements as float32, and back
+__device__ __forceinline__ float4 ld_f4(const void* p, int dt, size_t i4) { return raw4_f(ld_raw4(p, dt, i4), dt); }
+
+// Loads asked for before this stay before it: the compiler otherwise moves them into the branch that
+// uses them, behind a wait for other loads.
+__device__ __forceinline__ void loads_asked_for() { asm volatile("" ::: "memory"); }
+
+// ... or zeros where `on` is false, without a branch either: p's first four are then read, or `other`'s
+// (four float32) where p is null
+__device__ __forceinline__ float4 ld_f4_if(const void* p, int dt, size_t i4, bool on, const float* other) {
+    const bool there = p != nullptr;
+    const float4 v = ld_f4(there ? p : other, there ? dt : ILLM_F32, on && there ? i4 : 0);
+    return on && there ? v : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 __device__ __forceinline__ void st_f4(void* p, int dt, size_t i4, float4 v) {
@@ -114,15 +143,18 @@ __device__ __forceinline__ float wave_max(float v) {
 }
 
 // Sum over a block of up to 1024 threads; `red` holds 16 floats of LDS.  Every
-// thread gets the result; the order of the additions is fixed by the block size.
+// thread gets the result; the order of the additions is fixed by the block size.  NW: the block's
+// waves where they are known when the kernel is compiled.
+template <int NW = 0>
 __device__ __forceinline__ float block_sum(float v, float* red) {
     const int lane = threadIdx.x & (ILLM_WAVE - 1), w = threadIdx.x / ILLM_WAVE;
-    const int nw = (blockDim.x + ILLM_WAVE - 1) / ILLM_WAVE;
+    const int nw = NW ? NW : (blockDim.x + ILLM_WAVE - 1) / ILLM_WAVE;
     v = wave_sum(v);
     __syncthreads();
     if (lane == 0) red[w] = v;
     __syncthreads();
     float t = 0.f;
+#pragma unroll
     for (int i = 0; i < nw; ++i) t += red[i];
     return t;
 }

@@ -17,7 +17,7 @@ __device__ __forceinline__ float2 row_stats(const float* v, const bool* in, int 
         float s = 0.f;
 #pragma unroll
         for (int k = 0; k < N; ++k) s += v[k];
-        mean = block_sum(s, red) / (float)E;
+        mean = block_sum<4>(s, red) / (float)E;
     }
     float ss = 0.f;
 #pragma unroll
@@ -25,7 +25,7 @@ __device__ __forceinline__ float2 row_stats(const float* v, const bool* in, int 
         const float d = in[k / 4] ? v[k] - mean : 0.f;
         ss = fmaf(d, d, ss);
     }
-    ss = block_sum(ss, red);
+    ss = block_sum<4>(ss, red);
     return make_float2(mean, 1.0f / sqrtf(ss / (float)E + eps));
 }
 
@@ -40,20 +40,20 @@ post_add_norm_kernel(float* __restrict__ x, const void* __restrict__ a, int a_dt
     __shared__ float red[16];
     const int r = blockIdx.x, n4 = E / 4;
     const size_t ib4 = (size_t)(row_idx ? row_idx[r] : r) * n4, ob4 = (size_t)r * n4;
-    const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 xv[NV], av[NV], pwv[NV], pbv[NV], wv[NV], bv[NV];
     bool in[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const int i = threadIdx.x + 256 * k;
         in[k] = i < n4;
-        xv[k] = in[k] ? ((const float4*)x)[ib4 + i] : zero4;
-        av[k] = (a && in[k]) ? ld_f4(a, a_dt, ib4 + i) : zero4;
-        pwv[k] = (a && post_kind && in[k]) ? ld_f4(pw, pw_dt, i) : zero4;
-        pbv[k] = (a && pb && in[k]) ? ld_f4(pb, pw_dt, i) : zero4;
-        wv[k] = (out_kind && in[k]) ? ld_f4(w, w_dt, i) : zero4;
-        bv[k] = (out_kind && b && in[k]) ? ld_f4(b, w_dt, i) : zero4;
+        xv[k] = ld_f4_if(x, ILLM_F32, ib4 + i, in[k], x);
+        av[k] = ld_f4_if(a, a_dt, ib4 + i, in[k], x);
+        pwv[k] = ld_f4_if(a && post_kind ? pw : nullptr, pw_dt, i, in[k], x);
+        pbv[k] = ld_f4_if(a ? pb : nullptr, pw_dt, i, in[k], x);
+        wv[k] = ld_f4_if(out_kind ? w : nullptr, w_dt, i, in[k], x);
+        bv[k] = ld_f4_if(out_kind ? b : nullptr, w_dt, i, in[k], x);
     }
+    loads_asked_for();
     if (a) {
         float2 st = make_float2(0.f, 1.f);
         if (post_kind) st = row_stats<4 * NV>((const float*)av, in, post_kind, E, post_eps, red);
@@ -105,11 +105,11 @@ post_add_norm_any_kernel(float* __restrict__ x, const void* __restrict__ a, int 
         float mean = 0.f, s = 0.f;
         if (kind == ILLM_NORM_LAYER) {
             for (int i = threadIdx.x; i < E; i += 256) s += row[i];
-            mean = block_sum(s, red) / (float)E;
+            mean = block_sum<4>(s, red) / (float)E;
         }
         s = 0.f;
         for (int i = threadIdx.x; i < E; i += 256) s = fmaf(row[i] - mean, row[i] - mean, s);
-        s = block_sum(s, red);
+        s = block_sum<4>(s, red);
         return make_float2(mean, 1.0f / sqrtf(s / (float)E + e));
     };
     // (a thread reads and writes its own entries of `row` only)
@@ -212,7 +212,6 @@ post_mix_norm_kernel(PostMix m) {
     if (NV > 0) {
         const int n4 = E / 4;
         const size_t ib = in_row * n4, ob = (size_t)r * n4;
-        const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
         float4 x[NV ? NV : 1], a[NV ? NV : 1], b[NV && PAIR ? NV : 1], aw[NV && PAIR ? NV : 1], bw[NV && PAIR ? NV : 1];
         float4 pw[NV ? NV : 1], w[NV ? NV : 1], pl[NV ? NV : 1], old[NV && SHIFT ? NV : 1];
         constexpr bool AHEAD = SHIFT && NV > 0 && NV <= 2;
@@ -221,23 +220,24 @@ post_mix_norm_kernel(PostMix m) {
         for (int k = 0; k < NV; ++k) {
             const int i = threadIdx.x + 256 * k;
             const bool in = i < n4;
-            x[k] = in ? ((const float4*)m.x)[ib + i] : zero4;
-            a[k] = (m.a && in) ? ld_f4(m.a, m.a_dt, ib + i) : zero4;
+            x[k] = ld_f4_if(m.x, ILLM_F32, ib + i, in, m.x);
+            a[k] = ld_f4_if(m.a, m.a_dt, ib + i, in, m.x);
             if (PAIR) {
-                b[k] = in ? ld_f4(m.b, m.b_dt, ib + i) : zero4;
-                aw[k] = in ? ld_f4(m.aw, m.pair_dt, i) : zero4;
-                bw[k] = in ? ld_f4(m.bw, m.pair_dt, i) : zero4;
+                b[k] = ld_f4_if(m.b, m.b_dt, ib + i, in, m.x);
+                aw[k] = ld_f4_if(m.aw, m.pair_dt, i, in, m.x);
+                bw[k] = ld_f4_if(m.bw, m.pair_dt, i, in, m.x);
             }
-            pw[k] = (m.a && in) ? ld_f4(m.pw, m.pw_dt, i) : zero4;
-            pl[k] = (m.plus && in) ? ((const float4*)m.plus)[ib + i] : zero4;
-            w[k] = in ? ld_f4(m.w, m.w_dt, i) : zero4;
+            pw[k] = ld_f4_if(m.a ? m.pw : nullptr, m.pw_dt, i, in, m.x);
+            pl[k] = ld_f4_if(m.plus, ILLM_F32, ib + i, in, m.x);
+            w[k] = ld_f4_if(m.w, m.w_dt, i, in, m.x);
             if (AHEAD) {
 #pragma unroll
                 for (int s = 0; s < POST_MIX_AHEAD; ++s)
-                    if (s < m.S) mu[k][s] = in ? ((const float4*)m.mu)[(size_t)s * n4 + i] : zero4;
+                    mu[k][s] = ld_f4_if(m.mu, ILLM_F32, (size_t)s * n4 + i, in && s < m.S, m.x);
             }
-            if (SHIFT) old[k] = in ? ld_f4(m.tail, m.tail_dt, (size_t)slot * n4 + i) : zero4;
+            if (SHIFT) old[k] = ld_f4_if(m.tail, m.tail_dt, (size_t)slot * n4 + i, in, m.x);
         }
+        loads_asked_for();
         if (m.a) {
             if (PAIR) {
                 float sa = 0.f, sb = 0.f;
@@ -256,7 +256,7 @@ post_mix_norm_kernel(PostMix m) {
             float ss = 0.f;
 #pragma unroll
             for (int k = 0; k < NV; ++k) ss += sum_sq(a[k]);
-            ss = block_sum(ss, red);
+            ss = block_sum<4>(ss, red);
             const float inv = 1.0f / sqrtf(ss / (float)E + m.post_eps);
 #pragma unroll
             for (int k = 0; k < NV; ++k) {
@@ -274,7 +274,7 @@ post_mix_norm_kernel(PostMix m) {
             if (!m.row_idx && (m.a || m.plus) && i < n4) ((float4*)m.x)[ib + i] = x[k];
             ss += sum_sq(x[k]);
         }
-        ss = block_sum(ss, red);
+        ss = block_sum<4>(ss, red);
         const float inv = 1.0f / sqrtf(ss / (float)E + m.eps);
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
@@ -326,7 +326,7 @@ post_mix_norm_kernel(PostMix m) {
         }
         float ss = 0.f;
         for (int i = threadIdx.x; i < E; i += 256) ss = fmaf(y[i], y[i], ss);
-        ss = block_sum(ss, red);
+        ss = block_sum<4>(ss, red);
         inv = 1.0f / sqrtf(ss / (float)E + m.post_eps);
     }
     float ss = 0.f;
@@ -338,7 +338,7 @@ post_mix_norm_kernel(PostMix m) {
         row[i] = v;
         ss = fmaf(v, v, ss);
     }
-    ss = block_sum(ss, red);
+    ss = block_sum<4>(ss, red);
     inv = 1.0f / sqrtf(ss / (float)E + m.eps);
     for (int i = threadIdx.x; i < E; i += 256) {
         float h = (row[i] * inv) * ld_f(m.w, m.w_dt, i);

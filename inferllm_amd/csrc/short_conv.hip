@@ -21,7 +21,10 @@ __device__ __forceinline__ float conv_round(float v, int dt) {
 }
 
 // Four channels a thread where the rows allow (C, the offset and the strides multiples of 4): grid
-// (rows, ceil(C / 1024)).
+// (rows, ceil(C / 1024)).  Bound by trips to memory one after another: with TAPS (2 to 4) known when
+// the kernel is compiled it takes the slots, then every row, kept input and weight at once, whichever
+// of the two an input comes from.  TAPS 0: any number, a trip an input.
+template <int TAPS>
 __global__ void __launch_bounds__(256)
 short_conv_vec4_kernel(const void* __restrict__ X, int x_dt, int x_stride, int x_off,
                        const float* __restrict__ in_bias, const float* __restrict__ w,
@@ -33,56 +36,97 @@ short_conv_vec4_kernel(const void* __restrict__ X, int x_dt, int x_stride, int x
     const int K = taps - 1, slot = row_slot[r];
     int above[CONV_MAX_TAPS];
 #pragma unroll
-    for (int j = 1; j < CONV_MAX_TAPS; ++j) above[j] = (j <= K && r - j >= 0) ? row_slot[r - j] : -1;
+    for (int j = 1; j < (TAPS ? TAPS : CONV_MAX_TAPS); ++j) above[j] = (j <= K && r - j >= 0) ? row_slot[r - j] : -1;
     float4 ib = make_float4(0.f, 0.f, 0.f, 0.f);
     if (in_bias) ib = ((const float4*)in_bias)[c4];
-    // the rows above are asked for together with their slots, before it is known how many of them
-    // belong to this sequence (a row of another sequence is then read and dropped): one trip to
-    // memory instead of two in a row
-    float4 in[CONV_MAX_TAPS];                   // (indexed by constants only: the array stays in registers)
+    float4 in[TAPS ? TAPS : CONV_MAX_TAPS];     // in[j]: the input taps - 1 - j rows back (indexed by
+    float4 cur = make_float4(0.f, 0.f, 0.f, 0.f);       // constants only: the array stays in registers)
+    float y[4];
+    if (TAPS) {
+        int n = 0;                              // rows of the same sequence right above this one
 #pragma unroll
-    for (int j = 0; j < CONV_MAX_TAPS; ++j) {
-        if (j >= taps) continue;
-        const int rr = max(r - (K - j), 0);
-        in[j] = ld_f4(X, x_dt, ((size_t)rr * x_stride + x_off) / 4 + c4);
-    }
-    int n = 0;
+        for (int j = 1; j < TAPS; ++j)
+            if (n == j - 1 && above[j] == slot) n = j;
+        AnyRaw4 raw[TAPS ? TAPS : 1];
+        float4 cw[TAPS ? TAPS : 1];             // [4][TAPS]
 #pragma unroll
-    for (int j = 1; j < CONV_MAX_TAPS; ++j)
-        if (n == j - 1 && above[j] == slot) n = j;
-    float4 cur = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int j = 0; j < TAPS; ++j) {
+            const int back = TAPS - 1 - j;
+            const bool row = back <= n;
+            raw[j] = ld_raw4(row ? X : tail, row ? x_dt : tail_dt,
+                             row ? ((size_t)(r - back) * x_stride + x_off) / 4 + c4
+                                 : ((size_t)slot * K + (K - (back - n))) * (C / 4) + c4);
+            cw[j] = ((const float4*)w)[(size_t)TAPS * c4 + j];
+        }
+        const float4 b4 = ld_f4_if(bias, ILLM_F32, c4, true, w);
+        loads_asked_for();
+        y[0] = b4.x; y[1] = b4.y; y[2] = b4.z; y[3] = b4.w;
 #pragma unroll
-    for (int j = 0; j < CONV_MAX_TAPS; ++j) {
-        if (j >= taps) continue;
-        const int back = K - j;
-        if (back <= n) {
-            float4 v = in[j];
-            v.x += ib.x; v.y += ib.y; v.z += ib.z; v.w += ib.w;
-            if (in_bias) {
-                v.x = conv_round(v.x, tail_dt); v.y = conv_round(v.y, tail_dt);
-                v.z = conv_round(v.z, tail_dt); v.w = conv_round(v.w, tail_dt);
+        for (int j = 0; j < TAPS; ++j) {
+            const bool row = TAPS - 1 - j <= n;
+            float4 v = raw4_f(raw[j], row ? x_dt : tail_dt);
+            if (row) {
+                v.x += ib.x; v.y += ib.y; v.z += ib.z; v.w += ib.w;
+                if (in_bias) {
+                    v.x = conv_round(v.x, tail_dt); v.y = conv_round(v.y, tail_dt);
+                    v.z = conv_round(v.z, tail_dt); v.w = conv_round(v.w, tail_dt);
+                }
             }
             in[j] = v;
-        } else {
-            in[j] = ld_f4(tail, tail_dt, ((size_t)slot * K + (K - (back - n))) * (C / 4) + c4);
+            if (j == TAPS - 1) cur = v;
         }
-        if (back == 0) cur = in[j];
-    }
-    float y[4];
-    if (bias) { const float4 b4 = ((const float4*)bias)[c4]; y[0] = b4.x; y[1] = b4.y; y[2] = b4.z; y[3] = b4.w; }
-    else y[0] = y[1] = y[2] = y[3] = 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const float* cw = w + (size_t)(4 * c4 + e) * taps;
+        for (int e = 0; e < 4; ++e) {
 #pragma unroll
-        for (int j = 0; j < CONV_MAX_TAPS; ++j)
-            if (j < taps) y[e] = fmaf(cw[j], ((const float*)&in[j])[e], y[e]);
-        if (add_input) y[e] += ((const float*)&cur)[e];
+            for (int j = 0; j < TAPS; ++j) y[e] = fmaf(((const float*)cw)[e * TAPS + j], ((const float*)&in[j])[e], y[e]);
+            if (add_input) y[e] += ((const float*)&cur)[e];
+        }
+    } else {
+        // the rows above are asked for together with their slots, before it is known how many of them
+        // belong to this sequence (a row of another sequence is then read and dropped): one trip to
+        // memory instead of two in a row
+#pragma unroll
+        for (int j = 0; j < CONV_MAX_TAPS; ++j) {
+            if (j >= taps) continue;
+            const int rr = max(r - (K - j), 0);
+            in[j] = ld_f4(X, x_dt, ((size_t)rr * x_stride + x_off) / 4 + c4);
+        }
+        int n = 0;
+#pragma unroll
+        for (int j = 1; j < CONV_MAX_TAPS; ++j)
+            if (n == j - 1 && above[j] == slot) n = j;
+#pragma unroll
+        for (int j = 0; j < CONV_MAX_TAPS; ++j) {
+            if (j >= taps) continue;
+            const int back = K - j;
+            if (back <= n) {
+                float4 v = in[j];
+                v.x += ib.x; v.y += ib.y; v.z += ib.z; v.w += ib.w;
+                if (in_bias) {
+                    v.x = conv_round(v.x, tail_dt); v.y = conv_round(v.y, tail_dt);
+                    v.z = conv_round(v.z, tail_dt); v.w = conv_round(v.w, tail_dt);
+                }
+                in[j] = v;
+            } else {
+                in[j] = ld_f4(tail, tail_dt, ((size_t)slot * K + (K - (back - n))) * (C / 4) + c4);
+            }
+            if (back == 0) cur = in[j];
+        }
+        if (bias) { const float4 b4 = ((const float4*)bias)[c4]; y[0] = b4.x; y[1] = b4.y; y[2] = b4.z; y[3] = b4.w; }
+        else y[0] = y[1] = y[2] = y[3] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float* cw = w + (size_t)(4 * c4 + e) * taps;
+#pragma unroll
+            for (int j = 0; j < CONV_MAX_TAPS; ++j)
+                if (j < taps) y[e] = fmaf(cw[j], ((const float*)&in[j])[e], y[e]);
+            if (add_input) y[e] += ((const float*)&cur)[e];
+        }
     }
     st_f4(out, out_dt, ((size_t)r * out_stride) / 4 + c4, make_float4(y[0], y[1], y[2], y[3]));
     if (update_tail) {
 #pragma unroll
-        for (int j = 1; j < CONV_MAX_TAPS; ++j)
+        for (int j = 1; j < (TAPS ? TAPS : CONV_MAX_TAPS); ++j)
             if (j < taps) st_f4(tail, tail_dt, ((size_t)slot * K + (j - 1)) * (C / 4) + c4, in[j]);
     }
 }
@@ -142,9 +186,17 @@ extern "C" int illm_short_conv(const void* X, int x_dt, int x_stride, int x_off,
         return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
     if (C % 4 == 0 && x_off % 4 == 0 && x_stride % 4 == 0 && out_stride % 4 == 0) {
-        hipLaunchKernelGGL(short_conv_vec4_kernel, dim3(T, (C / 4 + 255) / 256), dim3(256), 0, (hipStream_t)stream,
-                           X, x_dt, x_stride, x_off, in_bias, w, bias, taps, tail, tail_dt, row_slot,
-                           add_input, out, out_dt, out_stride, C, taps > 1 ? update_tail : 0);
+        // (float4 reads of the taps want them 16-byte aligned)
+        const int t = (uintptr_t)w % 16 == 0 ? taps : 0;
+#define GO(TAPS_)                                                                                                 \
+    hipLaunchKernelGGL(short_conv_vec4_kernel<TAPS_>, dim3(T, (C / 4 + 255) / 256), dim3(256), 0,                  \
+                       (hipStream_t)stream, X, x_dt, x_stride, x_off, in_bias, w, bias, taps, tail, tail_dt, row_slot, \
+                       add_input, out, out_dt, out_stride, C, taps > 1 ? update_tail : 0)
+        if (t == 2) GO(2);
+        else if (t == 3) GO(3);
+        else if (t == 4) GO(4);
+        else GO(0);
+#undef GO
         return illm_launch_status();
     }
     hipLaunchKernelGGL(short_conv_kernel, dim3(T, (C + 255) / 256), dim3(256), 0, (hipStream_t)stream,
@@ -283,9 +335,13 @@ extern "C" int illm_clamped_swish_mul(const void* gate_up, void* out, int dt, in
 // With `row_idx` only those rows are formed and x is left as it is.  The convolution is for steps of
 // one row a sequence: the earlier inputs come from tail [slots][taps - 1][E], which is moved on.
 // grid (rows); 256 threads.  A thread owns NV groups of 4 consecutive columns (E % 4 == 0, E <= 1024
-// NV) and asks for everything it reads of a pass before it uses any of it; other widths take the
-// plain loop (NV 0), which keeps the row's sum in LDS (E floats) between the passes.
-template <int NV>
+// NV) and asks for everything it reads before it uses any of it, the kept inputs and the taps too
+// where their number is known when the kernel is compiled (TAPS 2 to 4, rows up to 4,096 columns;
+// TAPS 0: no convolution or any number); other widths take the plain loop (NV 0), which keeps the
+// row's sum in LDS (E floats) between the passes.
+// Bound by trips to memory one after another: 8 rows of 2,048 columns with 3 taps take 4.8 us, and took
+// 9.3 us where the type of each load was a branch with its wait and the taps came one by one.
+template <int NV, int TAPS>
 __global__ void __launch_bounds__(256)
 post_add_rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ a, int a_dt,
                         const void* __restrict__ post_w, int post_w_dt, float post_eps, float gain,
@@ -303,20 +359,35 @@ post_add_rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ a, int a
     if (NV > 0) {
         const int n4 = E / 4;
         float4 xv[NV > 0 ? NV : 1], av[NV > 0 ? NV : 1], pwv[NV > 0 ? NV : 1], wv4[NV > 0 ? NV : 1];
-        const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
+        float4 cwv[NV > 0 ? NV : 1][TAPS ? TAPS : 1], oldv[NV > 0 ? NV : 1][TAPS ? TAPS : 1];
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const int i4 = threadIdx.x + 256 * k;
-            xv[k] = i4 < n4 ? ((const float4*)(x + ib))[i4] : zero4;
-            av[k] = (a && i4 < n4) ? ld_f4(a, a_dt, ib / 4 + i4) : zero4;
-            pwv[k] = (a && i4 < n4) ? ld_f4(post_w, post_w_dt, i4) : zero4;
-            wv4[k] = i4 < n4 ? ld_f4(w, w_dt, i4) : zero4;
+            const bool in = i4 < n4;
+            xv[k] = ld_f4_if(x, ILLM_F32, ib / 4 + i4, in, x);
+            av[k] = ld_f4_if(a, a_dt, ib / 4 + i4, in, x);
+            pwv[k] = ld_f4_if(a ? post_w : nullptr, post_w_dt, i4, in, x);
+            wv4[k] = ld_f4_if(w, w_dt, i4, in, x);
+            if (TAPS) {
+#pragma unroll
+                for (int j = 0; j < TAPS; ++j) cwv[k][j] = ld_f4_if(conv_w, ILLM_F32, (size_t)TAPS * i4 + j, in, x);
+            }
         }
+        if (TAPS) {
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                const int i4 = threadIdx.x + 256 * k;
+#pragma unroll
+                for (int j = 0; j < TAPS - 1; ++j)
+                    oldv[k][j] = ld_f4_if(tail, tail_dt, ((size_t)slot * (TAPS - 1) + j) * n4 + i4, i4 < n4, x);
+            }
+        }
+        loads_asked_for();
         if (a) {
             float sa = 0.f;
 #pragma unroll
             for (int k = 0; k < NV; ++k) sa += av[k].x * av[k].x + av[k].y * av[k].y + av[k].z * av[k].z + av[k].w * av[k].w;
-            sa = block_sum(sa, red);
+            sa = block_sum<4>(sa, red);
             const float inv_a = 1.0f / sqrtf(sa / (float)E + post_eps);
 #pragma unroll
             for (int k = 0; k < NV; ++k) {
@@ -333,7 +404,7 @@ post_add_rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ a, int a
         float ss = 0.f;
 #pragma unroll
         for (int k = 0; k < NV; ++k) ss += xv[k].x * xv[k].x + xv[k].y * xv[k].y + xv[k].z * xv[k].z + xv[k].w * xv[k].w;
-        ss = block_sum(ss, red);
+        ss = block_sum<4>(ss, red);
         const float scale = 1.0f / sqrtf(ss / (float)E + eps);
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
@@ -342,7 +413,22 @@ post_add_rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ a, int a
             const float4 wv = wv4[k];
             float h[4] = {(xv[k].x * scale) * wv.x, (xv[k].y * scale) * wv.y, (xv[k].z * scale) * wv.z,
                           (xv[k].w * scale) * wv.w};
-            if (conv_w) {
+            if (TAPS) {
+                float hq[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    hq[e] = conv_round(h[e], out_dt);
+                    const float* cw = (const float*)cwv[k] + e * TAPS;      // [4][TAPS]: column 4 i4 + e's taps
+                    float c = 0.f;
+#pragma unroll
+                    for (int j = 0; j < TAPS - 1; ++j) c = fmaf(cw[j], ((const float*)&oldv[k][j])[e], c);
+                    c = fmaf(cw[TAPS - 1], hq[e], c);
+                    h[e] = hq[e] + c;
+                }
+#pragma unroll
+                for (int j = 1; j < TAPS - 1; ++j) st_f4(tail, tail_dt, ((size_t)slot * K + (j - 1)) * n4 + i4, oldv[k][j]);
+                st_f4(tail, tail_dt, ((size_t)slot * K + (K - 1)) * n4 + i4, make_float4(hq[0], hq[1], hq[2], hq[3]));
+            } else if (conv_w) {
                 float4 old[CONV_MAX_TAPS - 1];
 #pragma unroll
                 for (int j = 0; j < CONV_MAX_TAPS - 1; ++j)
@@ -376,7 +462,7 @@ post_add_rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ a, int a
             const float v = ld_f(a, a_dt, ib + i);
             sa = fmaf(v, v, sa);
         }
-        sa = block_sum(sa, red);
+        sa = block_sum<4>(sa, red);
         inv_a = 1.0f / sqrtf(sa / (float)E + post_eps);
     }
     float ss = 0.f;
@@ -389,7 +475,7 @@ post_add_rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ a, int a
         row[i] = v;
         ss = fmaf(v, v, ss);
     }
-    ss = block_sum(ss, red);
+    ss = block_sum<4>(ss, red);
     const float scale = 1.0f / sqrtf(ss / (float)E + eps);
     for (int i = threadIdx.x; i < E; i += 256) {
         float h = (row[i] * scale) * ld_f(w, w_dt, i);
@@ -425,24 +511,34 @@ extern "C" int illm_post_add_rmsnorm(float* x, const void* a, int a_dt, const vo
         return ILLM_ERR_ARG;
     if (rows == 0) return ILLM_OK;
     hipStream_t st = (hipStream_t)stream;
-#define GO(NV_, LDS_)                                                                                   \
-    hipLaunchKernelGGL(post_add_rmsnorm_kernel<NV_>, dim3(rows), dim3(256), LDS_, st, x, a, a_dt, post_w,   \
-                       post_w_dt, post_eps, gain, w, w_dt, out, out_dt, row_idx, E, eps, conv_w, taps, tail, \
+#define GO(NV_, TAPS_, LDS_)                                                                                 \
+    hipLaunchKernelGGL((post_add_rmsnorm_kernel<NV_, TAPS_>), dim3(rows), dim3(256), LDS_, st, x, a, a_dt, post_w, \
+                       post_w_dt, post_eps, gain, w, w_dt, out, out_dt, row_idx, E, eps, conv_w, taps, tail,      \
                        tail_dt, row_slot)
     if (E % 4 == 0 && E <= 8192) {
-        if (E <= 1024) GO(1, 0);
-        else if (E <= 2048) GO(2, 0);
-        else if (E <= 4096) GO(4, 0);
-        else GO(8, 0);
+        // (float4 reads of the taps want them 16-byte aligned)
+        const int t = conv_w && E <= 4096 && (uintptr_t)conv_w % 16 == 0 ? taps : 0;
+#define GO_TAPS(NV_)                       \
+    do {                                   \
+        if (t == 2) GO(NV_, 2, 0);         \
+        else if (t == 3) GO(NV_, 3, 0);    \
+        else if (t == 4) GO(NV_, 4, 0);    \
+        else GO(NV_, 0, 0);                \
+    } while (0)
+        if (E <= 1024) GO_TAPS(1);
+        else if (E <= 2048) GO_TAPS(2);
+        else if (E <= 4096) GO_TAPS(4);
+        else GO(8, 0, 0);
+#undef GO_TAPS
         return illm_launch_status();
     }
     const size_t lds = (size_t)E * sizeof(float);
     if (lds > 64 * 1024) return ILLM_ERR_ARG;
     if (lds > 48 * 1024 &&
-        hipFuncSetAttribute((const void*)post_add_rmsnorm_kernel<0>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipFuncSetAttribute((const void*)post_add_rmsnorm_kernel<0, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lds) != hipSuccess)
         return ILLM_ERR_LAUNCH;
-    GO(0, lds);
+    GO(0, 0, lds);
 #undef GO
     return illm_launch_status();
 }

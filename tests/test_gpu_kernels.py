@@ -1329,3 +1329,52 @@ def test_qkv_rope_store_of_many_rows(M, nh, nkv, hd, K, tb, kp, rows_shape):
     for gotc, wantc in ((kc_g.cpu(), kr), (vc_g.cpu(), vr)):
         assert torch.equal(torch.isnan(gotc), torch.isnan(wantc))        # the same rows, nothing else
         close(torch.nan_to_num(gotc), torch.nan_to_num(wantc), dtype, scale=sc)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("E", [4, 1024, 1028, 2052, 4096, 4100, 8196, 90])
+def test_passes_of_single_tokens_over_widths_and_taps(E, dtype):
+    """The passes that ask for all they read at once: groups of four columns a thread from none left over to one
+    more than a thread's share, and the widths that take the plain loops; 2 to 5 taps (compiled in up to 4)."""
+    g = torch.Generator().manual_seed(E)
+    o, T, V, buckets = ops(), 3, 11, 7
+    # float32: sums of up to 8,196 squares and 5 taps, relative error below 1e-5; bfloat16: the result's rounding,
+    # and one step more where the rounded input of the convolution falls on the other side
+    tol = 1e-5 if dtype == torch.float32 else 2 ** -7
+
+    def near(got, want, tol):
+        want = want.double()
+        assert float((got.double().cpu() - want).abs().max()) <= tol * max(1.0, float(want.abs().max()))
+    a, pw = (torch.randn(T, E, generator=g) * 3).to(dtype), torch.randn(E, generator=g) + 1
+    x, w = torch.randn(T, E, generator=g), (torch.randn(E, generator=g) + 1).to(dtype)
+    slots = torch.tensor([3, 0, 2], dtype=torch.int32)
+    for taps in (2, 3, 4, 5):
+        cw, tail = torch.randn(E, taps, generator=g), torch.randn(4, taps - 1, E, generator=g).to(dtype)
+        for post in (None, (a, pw, 1e-5, 0.3)):
+            x_want, x_got, t_want, t_got = x.clone(), x.to(DEV), tail.clone(), tail.to(DEV)
+            want = R.post_add_rmsnorm(x_want, o.PostNormed(*post) if post else None, w, 2e-5, dtype, None,
+                                      (cw, t_want, slots))
+            got = o.post_add_rmsnorm(x_got, o.PostNormed(a.to(DEV), pw.to(DEV), 1e-5, 0.3) if post else None,
+                                     w.to(DEV), 2e-5, dtype, None, (cw.to(DEV), t_got, slots.to(DEV)))
+            near(got, want, tol), near(x_got, x_want, 1e-5), near(t_got, t_want, tol)
+        # rows of two sequences (the second's first inputs are kept ones) and single rows; taps of an odd base
+        X, bias, odd = x.to(dtype), torch.randn(E, generator=g), torch.zeros(E * taps + 1)
+        odd[1:] = cw.reshape(-1)
+        for row_slot in (torch.tensor([1, 1, 2], dtype=torch.int32), slots):
+            for cwd in (cw.to(DEV), odd.to(DEV)[1:].view(E, taps)):
+                single = row_slot is slots
+                t_want, t_got = tail.clone(), tail.to(DEV)
+                want = R.short_conv(X, 0, E, cw, t_want, row_slot, torch.float32, bias, bias, False, update_tail=single)
+                got = o.short_conv(X.to(DEV), 0, E, cwd, t_got, row_slot.to(DEV), torch.float32, bias.to(DEV),
+                                   bias.to(DEV), False, update_tail=single)
+                near(got, want, tol), near(t_got, t_want, tol)
+    table, pairs = torch.randn(V, E, generator=g).to(dtype), torch.randn(buckets + 1, E, generator=g).to(dtype)
+    places = torch.randn(5, E, generator=g)
+    tokens, pos = torch.tensor([3, 10, 0], dtype=torch.int32), torch.tensor([0, 4, 2], dtype=torch.int32)
+    for pr, pl in ((pairs, places), (pairs, None), (None, places), (None, None)):
+        l_want, l_got = torch.tensor([1, 2, 4, 9], dtype=torch.int32), torch.tensor([1, 2, 4, 9], dtype=torch.int32).to(DEV)
+        put = lambda t: t.to(DEV) if t is not None else None
+        want = R.embed_pairs(tokens, pos, slots, table, 2.5, pr, buckets, 7, 3, pl, l_want, True)
+        got = o.embed_pairs(put(tokens), put(pos), put(slots), put(table), 2.5, put(pr), buckets, 7, 3, put(pl), l_got, True)
+        near(got, want, 1e-6)
+        assert torch.equal(l_got.cpu(), l_want)
