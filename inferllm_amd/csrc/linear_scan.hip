@@ -137,20 +137,27 @@ extern "C" int illm_ssm_finish(const float* o, const float* x, const float* D, c
 }
 
 // ---------------------------------------------------------------- matrix memory
-// grid (rows); 256 threads.  U [T, u_stride] = [q (H dk) | k (H dk) | v (H dv) | ...].
+// grid (rows, ceil(max(H dk, H (dv + 1)) / 256)); 256 threads, an entry of q, k and v each (a block a row, which
+// went through them one after another, took 9.3 us for 8 rows of 2,048, this 4.7).
+// U [T, u_stride] = [q (H dk) | k (H dk) | v (H dv) | ...].
+template <int DT>
 __global__ void __launch_bounds__(256)
-memory_rows_kernel(const void* __restrict__ U, int dt, int u_stride, float* __restrict__ qn,
+memory_rows_kernel(const void* __restrict__ U, int u_stride, float* __restrict__ qn,
                    float* __restrict__ kn, float* __restrict__ vv, int H, int dk, int dv, float qscale) {
     const size_t r = blockIdx.x;
-    const int nq = H * dk, nv = H * (dv + 1);
-    for (int i = threadIdx.x; i < nq; i += 256) {
-        qn[r * nq + i] = ld_f(U, dt, r * u_stride + i) * qscale;
-        kn[r * nq + i] = ld_f(U, dt, r * u_stride + nq + i);
+    const int nq = H * dk, nv = H * (dv + 1), i = blockIdx.y * 256 + threadIdx.x;
+    const int h = i / (dv + 1), j = i - h * (dv + 1);
+    float q = 0.f, k = 0.f, v = 1.0f;
+    if (i < nq) {
+        q = ld_f(U, DT, r * u_stride + i);
+        k = ld_f(U, DT, r * u_stride + nq + i);
     }
-    for (int i = threadIdx.x; i < nv; i += 256) {
-        const int h = i / (dv + 1), j = i - h * (dv + 1);
-        vv[r * nv + i] = j < dv ? ld_f(U, dt, r * u_stride + 2 * nq + h * dv + j) : 1.0f;
+    if (i < nv && j < dv) v = ld_f(U, DT, r * u_stride + 2 * nq + h * dv + j);
+    if (i < nq) {
+        qn[r * nq + i] = q * qscale;
+        kn[r * nq + i] = k;
     }
+    if (i < nv) vv[r * nv + i] = v;
 }
 
 // grid (sequences, H); one wave.  64 tokens at a time: every lane forms its token's two gates, then
@@ -200,8 +207,15 @@ extern "C" int illm_memory_prepare(const void* U, int dt, int u_stride, int i_of
         i_off + H > u_stride || f_off + H > u_stride)
         return ILLM_ERR_ARG;
     if (T == 0 || n_seqs == 0) return ILLM_OK;
-    hipLaunchKernelGGL(memory_rows_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, U, dt, u_stride, qn,
-                       kn, vv, H, dk, dv, 1.0f / sqrtf((float)dk));
+    const int widest = H * dk > H * (dv + 1) ? H * dk : H * (dv + 1);
+    if ((widest + 255) / 256 > 65535) return ILLM_ERR_ARG;
+    const dim3 grid(T, (widest + 255) / 256);
+    if (dt == ILLM_BF16)
+        hipLaunchKernelGGL(memory_rows_kernel<ILLM_BF16>, grid, dim3(256), 0, (hipStream_t)stream, U, u_stride, qn,
+                           kn, vv, H, dk, dv, 1.0f / sqrtf((float)dk));
+    else
+        hipLaunchKernelGGL(memory_rows_kernel<ILLM_F32>, grid, dim3(256), 0, (hipStream_t)stream, U, u_stride, qn,
+                           kn, vv, H, dk, dv, 1.0f / sqrtf((float)dk));
     if (hipGetLastError() != hipSuccess) return ILLM_ERR_LAUNCH;
     hipLaunchKernelGGL(memory_gates_kernel, dim3(n_seqs, H), dim3(64), 0, (hipStream_t)stream, U, dt,
                        u_stride, i_off, f_off, i_bias, f_bias, cap, m_state, cu, seq_slot, beta, dec, em, H);
@@ -268,6 +282,33 @@ gla_prepare_kernel(const void* __restrict__ U, int dt, int u_stride, int q_off, 
     for (int e = threadIdx.x; e < H; e += 256) beta[t * H + e] = 1.0f;
 }
 
+// The same four columns a thread where offsets, strides and widths are multiples of 4: grid
+// (rows, ceil(max(H dk, H dv) / 1024)).  A block a row, a column at a time, took 11.2 us for 8 rows of
+// 2,048, this 4.8; 2,964 rows 26 and 18.
+__global__ void __launch_bounds__(256)
+gla_prepare_vec4_kernel(const void* __restrict__ U, int dt, int u_stride, int q_off, int k_off, int v_off,
+                        const void* __restrict__ Z, int z_dt, int z_stride, const float* __restrict__ zb,
+                        float inv_tau, float* __restrict__ qn, float* __restrict__ kn, float* __restrict__ vv,
+                        float* __restrict__ beta, float* __restrict__ dec, int H, int dk, int dv) {
+    const size_t t = blockIdx.x;
+    const int g = blockIdx.y * 256 + threadIdx.x, nk4 = H * dk / 4, nv4 = H * dv / 4;
+    const float qs = 1.0f / sqrtf((float)dk);
+    const int gk = g < nk4 ? g : 0, gv = g < nv4 ? g : 0;
+    const float4 q = ld_f4(U, dt, (t * u_stride + q_off) / 4 + gk), k = ld_f4(U, dt, (t * u_stride + k_off) / 4 + gk);
+    const float4 z = ld_f4(Z, z_dt, t * z_stride / 4 + gk), b = ((const float4*)zb)[gk];
+    const float4 v = ld_f4(U, dt, (t * u_stride + v_off) / 4 + gv);
+    loads_asked_for();
+    if (g < nk4) {
+        ((float4*)qn)[t * nk4 + g] = make_float4(q.x * qs, q.y * qs, q.z * qs, q.w * qs);
+        ((float4*)kn)[t * nk4 + g] = k;
+        ((float4*)dec)[t * nk4 + g] = make_float4(
+            expf(ls_log_sigmoid(z.x + b.x) * inv_tau), expf(ls_log_sigmoid(z.y + b.y) * inv_tau),
+            expf(ls_log_sigmoid(z.z + b.z) * inv_tau), expf(ls_log_sigmoid(z.w + b.w) * inv_tau));
+    }
+    if (g < nv4) ((float4*)vv)[t * nv4 + g] = v;
+    if (g < H) beta[t * H + g] = 1.0f;
+}
+
 extern "C" int illm_gla_prepare(const void* U, int dt, int u_stride, int q_off, int k_off, int v_off,
                                 const void* Z, int z_dt, int z_stride, const float* zb, float tau,
                                 float* qn, float* kn, float* vv, float* beta, float* dec, int T, int H,
@@ -277,6 +318,16 @@ extern "C" int illm_gla_prepare(const void* U, int dt, int u_stride, int q_off, 
         v_off + H * dv > u_stride || H * dk > z_stride)
         return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
+    const int widest = H * dk > H * dv ? H * dk : H * dv;
+    // (dv >= 4: a row's H weights are within its groups of four)
+    if (((H * dk) | (H * dv) | q_off | k_off | v_off | u_stride | z_stride) % 4 == 0 && widest / 4 >= H &&
+        (widest / 4 + 255) / 256 <= 65535 &&
+        ((uintptr_t)U | (uintptr_t)Z | (uintptr_t)zb | (uintptr_t)qn | (uintptr_t)kn | (uintptr_t)vv | (uintptr_t)dec) % 16 == 0) {
+        hipLaunchKernelGGL(gla_prepare_vec4_kernel, dim3(T, (widest / 4 + 255) / 256), dim3(256), 0, (hipStream_t)stream,
+                           U, dt, u_stride, q_off, k_off, v_off, Z, z_dt, z_stride, zb, 1.0f / tau, qn, kn, vv, beta,
+                           dec, H, dk, dv);
+        return illm_launch_status();
+    }
     hipLaunchKernelGGL(gla_prepare_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, U, dt, u_stride,
                        q_off, k_off, v_off, Z, z_dt, z_stride, zb, 1.0f / tau, qn, kn, vv, beta, dec, H, dk, dv);
     return illm_launch_status();
@@ -371,6 +422,84 @@ lru_gates_kernel(const float* __restrict__ u, const float* __restrict__ Wt, cons
     }
 }
 
+// The same for steps of few rows: 32 outputs and 4 rows a block, grid (ceil(T / 4), nb, ceil(cb / 32)).  Eight
+// lanes take four outputs each of one input at a time (every 32nd input, so that a wave reads 8 inputs'
+// 128 bytes at once); the 32 slices' sums are added over the wave's lanes and then over the waves, in a fixed order.
+// Bound by the trips of a thread's inputs, of which it has cb / 32 instead of cb cb / 256: 8 rows of 2,048 channels
+// in 16 blocks take 6.0 us, and took 24.2 us with a block's outputs all in one place (32 blocks on the chip).
+#define LRU_FEW_ROWS 4
+__global__ void __launch_bounds__(256)
+lru_gates_few_kernel(const float* __restrict__ u, const float* __restrict__ Wt, const float* __restrict__ br,
+                     const float* __restrict__ bi, const float* __restrict__ lam, float rate,
+                     float* __restrict__ a_out, float* __restrict__ x_out, int T, int C, int cb) {
+    extern __shared__ float us[];                   // [cb][4 rows]
+    __shared__ float part[4][2][LRU_FEW_ROWS][32];  // the waves' sums
+    const int t0 = blockIdx.x * LRU_FEW_ROWS, b = blockIdx.y, nb = C / cb;
+    const int o_first = blockIdx.z * 32, rows = min(LRU_FEW_ROWS, T - t0);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int o = o_first + 4 * (lane & 7), sl = wave * 8 + (lane >> 3);
+    const float* wr = Wt + (size_t)b * cb * cb + (o < cb ? o : 0);
+    const float* wi = wr + (size_t)nb * cb * cb;
+    for (int i = tid; i < cb; i += 256) {
+        float4 x;
+        x.x = u[(size_t)t0 * C + (size_t)b * cb + i];
+        x.y = rows > 1 ? u[(size_t)(t0 + 1) * C + (size_t)b * cb + i] : 0.f;
+        x.z = rows > 2 ? u[(size_t)(t0 + 2) * C + (size_t)b * cb + i] : 0.f;
+        x.w = rows > 3 ? u[(size_t)(t0 + 3) * C + (size_t)b * cb + i] : 0.f;
+        ((float4*)us)[i] = x;
+    }
+    __syncthreads();
+    float s[2][LRU_FEW_ROWS][4];
+#pragma unroll
+    for (int k = 0; k < 8 * LRU_FEW_ROWS; ++k) ((float*)s)[k] = 0.f;
+#pragma unroll 4
+    for (int i = sl; i < cb; i += 32) {
+        const float4 w1 = *(const float4*)(wr + (size_t)i * cb), w2 = *(const float4*)(wi + (size_t)i * cb);
+        const float4 x4 = ((const float4*)us)[i];
+        const float x[4] = {x4.x, x4.y, x4.z, x4.w};
+#pragma unroll
+        for (int r = 0; r < LRU_FEW_ROWS; ++r) {
+            s[0][r][0] = fmaf(w1.x, x[r], s[0][r][0]); s[0][r][1] = fmaf(w1.y, x[r], s[0][r][1]);
+            s[0][r][2] = fmaf(w1.z, x[r], s[0][r][2]); s[0][r][3] = fmaf(w1.w, x[r], s[0][r][3]);
+            s[1][r][0] = fmaf(w2.x, x[r], s[1][r][0]); s[1][r][1] = fmaf(w2.y, x[r], s[1][r][1]);
+            s[1][r][2] = fmaf(w2.z, x[r], s[1][r][2]); s[1][r][3] = fmaf(w2.w, x[r], s[1][r][3]);
+        }
+    }
+    // over the lanes of the same outputs by halves: a lane keeps the half of its sums that its bit names
+    // and gives the other away, so that it ends with one gate's four outputs of one row pair's row
+    const bool up32 = lane & 32, up16 = lane & 16, up8 = lane & 8;
+    float h1[LRU_FEW_ROWS][4];
+#pragma unroll
+    for (int k = 0; k < 4 * LRU_FEW_ROWS; ++k) {
+        const float keep = up32 ? ((float*)s[1])[k] : ((float*)s[0])[k], give = up32 ? ((float*)s[0])[k] : ((float*)s[1])[k];
+        ((float*)h1)[k] = keep + __shfl_xor(give, 32);
+    }
+    float h2[2][4];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float keep = up16 ? ((float*)h1[2])[k] : ((float*)h1[0])[k], give = up16 ? ((float*)h1[0])[k] : ((float*)h1[2])[k];
+        ((float*)h2)[k] = keep + __shfl_xor(give, 16);
+    }
+    float4 h3;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float keep = up8 ? h2[1][k] : h2[0][k], give = up8 ? h2[0][k] : h2[1][k];
+        ((float*)&h3)[k] = keep + __shfl_xor(give, 8);
+    }
+    *(float4*)&part[wave][up32 ? 1 : 0][(up16 ? 2 : 0) + (up8 ? 1 : 0)][4 * (lane & 7)] = h3;
+    __syncthreads();
+    const int oo = tid & 31, r = tid >> 5;
+    if (r >= rows || o_first + oo >= cb) return;
+    const float ar = (part[0][0][r][oo] + part[1][0][r][oo]) + (part[2][0][r][oo] + part[3][0][r][oo]);
+    const float ai = (part[0][1][r][oo] + part[1][1][r][oo]) + (part[2][1][r][oo] + part[3][1][r][oo]);
+    const int c = b * cb + o_first + oo;
+    const float rg = ls_sigmoid(ar + br[c]), ig = ls_sigmoid(ai + bi[c]);
+    const float log_a = -rate * rg * ls_softplus(lam[c]);
+    a_out[(size_t)(t0 + r) * C + c] = expf(log_a);
+    // 1 - a^2 as -expm1(2 log a): a decay close to 1 keeps its digits
+    x_out[(size_t)(t0 + r) * C + c] = sqrtf(fmaxf(-expm1f(2.0f * log_a), 0.f)) * ig * us[(o_first + oo) * LRU_FEW_ROWS + r];
+}
+
 template <int ROWS>
 static int lru_gates_launch(const float* u, const float* Wt, const float* br, const float* bi,
                             const float* lam, float rate, float* a_out, float* x_out, int T, int C,
@@ -393,6 +522,13 @@ extern "C" int illm_lru_gates(const float* u, const float* Wt, const float* br, 
                               int nb, void* stream) {
     if (T < 0 || C <= 0 || nb <= 0 || C % nb || nb > 65535) return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
+    const int cb = C / nb;
+    if (T <= 128 && cb % 4 == 0 && cb <= 3072 && (uintptr_t)Wt % 16 == 0) {
+        hipLaunchKernelGGL(lru_gates_few_kernel, dim3((T + LRU_FEW_ROWS - 1) / LRU_FEW_ROWS, nb, (cb + 31) / 32), dim3(256),
+                           (size_t)cb * LRU_FEW_ROWS * sizeof(float), (hipStream_t)stream, u, Wt, br, bi, lam, rate,
+                           a_out, x_out, T, C, cb);
+        return illm_launch_status();
+    }
     // tiles of 16 rows where a block's inputs of 16 rows fit LDS (blocks of up to 1,024 channels)
     if (T <= 128 || C / nb > 1024)
         return lru_gates_launch<4>(u, Wt, br, bi, lam, rate, a_out, x_out, T, C, nb, (hipStream_t)stream);

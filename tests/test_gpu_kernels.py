@@ -1378,3 +1378,32 @@ def test_passes_of_single_tokens_over_widths_and_taps(E, dtype):
         got = o.embed_pairs(put(tokens), put(pos), put(slots), put(table), 2.5, put(pr), buckets, 7, 3, put(pl), l_got, True)
         near(got, want, 1e-6)
         assert torch.equal(l_got.cpu(), l_want)
+
+
+@pytest.mark.parametrize("T", [1, 4, 7, 128, 129])
+@pytest.mark.parametrize("nb, cb", [(2, 4), (3, 32), (1, 36), (2, 128), (1, 1028), (2, 30)])
+def test_recurrent_gates_of_few_rows(T, nb, cb):
+    """Blocks of channels around the 32 outputs and 32 slices a block takes; rows around its 4; 129 rows and widths
+    that are no multiple of 4 take the other kernel."""
+    g = torch.Generator().manual_seed(T + cb)
+    u = torch.randn(T, nb * cb, generator=g) * 2
+    wt = torch.randn(2, nb, cb, cb, generator=g) * min(0.5, 4.0 / cb ** 0.5)
+    rb, ib, lam = (torch.randn(nb * cb, generator=g) for _ in range(3))
+    for got, want in zip(ops().lru_gates(*(t.to(DEV) for t in (u, wt, rb, ib, lam)), 8.0),
+                         R.lru_gates(u, wt, rb, ib, lam, 8.0)):
+        # sums of up to 1,028 products of size 8 in float32, through functions of slope below 8
+        assert float((got.cpu().double() - want.double()).abs().max()) <= 1e-5 * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H, dk, dv", [(4, 256, 128), (1, 4, 4), (8, 132, 264), (16, 64, 64), (5, 12, 2)])
+def test_gated_linear_attention_rows_four_columns_a_load(H, dk, dv, dtype):
+    g = torch.Generator().manual_seed(H * dk)
+    for off in (0, 1):                                  # (an odd offset takes the loop by column)
+        U = (torch.randn(3, 2 * H * dk + H * dv + 8, generator=g) * 2).to(dtype)
+        Z, zb = (torch.randn(3, H * dk, generator=g) * 3).to(dtype), torch.randn(H * dk, generator=g)
+        args = (off, off + H * dk, off + 2 * H * dk)
+        want = R.gla_prepare(U, *args, Z, zb, 7.0, H, dk, dv)
+        got = ops().gla_prepare(U.to(DEV), *args, Z.to(DEV), zb.to(DEV), 7.0, H, dk, dv)
+        for a, b in zip(got, want):                     # (one exponential and one logarithm in float32)
+            assert float((a.cpu().double() - b.double()).abs().max()) <= 1e-5 * max(1.0, float(b.abs().max()))
