@@ -189,15 +189,6 @@ struct PostMix {
     float pair_eps, pair_scale, post_eps, gain, eps;
 };
 
-__device__ __forceinline__ float2 block_sum2(float u, float v, float* red) {
-    const int lane = threadIdx.x & (ILLM_WAVE - 1), w = threadIdx.x / ILLM_WAVE;
-    u = wave_sum(u); v = wave_sum(v);
-    __syncthreads();
-    if (lane == 0) { red[w] = u; red[8 + w] = v; }
-    __syncthreads();
-    return make_float2((red[0] + red[1]) + (red[2] + red[3]), (red[8] + red[9]) + (red[10] + red[11]));
-}
-__device__ __forceinline__ float sum_sq(const float4 v) { return (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w); }
 
 #define POST_MIX_AHEAD 5   // mixes whose weights are asked for with the row (rows of up to 2,048 columns)
 

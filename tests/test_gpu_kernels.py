@@ -1380,6 +1380,40 @@ def test_passes_of_single_tokens_over_widths_and_taps(E, dtype):
         assert torch.equal(l_got.cpu(), l_want)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nh, nkv, dk, dv, weights, mix", [(2, 1, 4, 8, True, True), (16, 4, 64, 64, True, False),
+                                                           (8, 2, 132, 128, False, True), (4, 4, 256, 260, True, True),
+                                                           (32, 8, 128, 128, True, True), (33, 1, 128, 64, True, True),
+                                                           (4, 2, 128, 128, False, False)])
+def test_norm_mix_and_store_four_columns_a_load(nh, nkv, dk, dv, weights, mix, dtype):
+    """Widths around a thread's share (1,024, 2,048 and 4,096 columns; 4,224 takes the loop by column), with and
+    without the norm and the mix of values, into a cache with a ring and into none."""
+    g = torch.Generator().manual_seed(nh * dk + dv)
+    o, page, pages, ring = ops(), 16, 6, 2
+    # float32: one rounding a step and a sum of up to 4,224 squares; bfloat16: the result's rounding (2^-8)
+    tol = 1e-5 if dtype == torch.float32 else 2 ** -8
+    pos, slot = torch.tensor([40, 3, 17], dtype=torch.int32), torch.tensor([1, 0, 2], dtype=torch.int32)
+    table = torch.randperm(pages, generator=g).view(3, 2).to(torch.int32)
+    k_off, v_off = nh * dk + 4, nh * dk + 4 + nkv * dk
+    rows = torch.randn(3, v_off + nkv * dv + 8, generator=g).to(dtype)
+    first = torch.randn(3, nkv * dv + 12, generator=g).to(dtype) if mix else None
+    lam = torch.tensor([0.3]) if mix else None
+    qw, kw = (torch.randn(n * dk, generator=g).to(dtype) if weights else None for n in (nh, nkv))
+    put = lambda t: t.to(DEV) if t is not None else None
+    for cached in (True, False):
+        kc = torch.randn(pages, nkv, page, dk, generator=g).to(dtype) if cached else None
+        vc = torch.randn(pages, nkv, page, dv, generator=g).to(dtype) if cached else None
+        r_want, r_got, kc_got, vc_got = rows.clone(), put(rows), put(kc), put(vc)
+        o.qkv_norm_mix_store(r_got, k_off, v_off, put(qw), put(kw), 1e-5, put(lam), put(first), 8, put(pos), put(slot),
+                             kc_got, vc_got, put(table), page, ring, nh, nkv, dk, dv)
+        R.qkv_norm_mix_store(r_want, k_off, v_off, qw, kw, 1e-5, lam, first, 8, pos, slot, kc, vc, table, page, ring,
+                             nh, nkv, dk, dv)
+        for got, want in ((r_got, r_want), (kc_got, kc), (vc_got, vc)):
+            if want is not None:
+                want = want.double()
+                assert float((got.double().cpu() - want).abs().max()) <= tol * max(1.0, float(want.abs().max()))
+
+
 @pytest.mark.parametrize("T", [1, 4, 7, 128, 129])
 @pytest.mark.parametrize("nb, cb", [(2, 4), (3, 32), (1, 36), (2, 128), (1, 1028), (2, 30)])
 def test_recurrent_gates_of_few_rows(T, nb, cb):
