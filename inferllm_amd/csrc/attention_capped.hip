@@ -23,6 +23,8 @@
 // plain ones on the vector units.
 #include <math.h>
 
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 
@@ -981,27 +983,33 @@ attn_cap_decode_kernel(const void* __restrict__ q, int q_stride, const void* __r
 // wave reads 8 rows of keys (and of values) an instruction, a whole 128-byte line a row, for all
 // the block's query heads at once; a score is 3 exchanges among the eight lanes.  Every group of
 // eight keeps its own running max, sum and weighted values (lane s of a group holds dims U s + 8 U j
-// ..), the next round's rows are asked for before this round's arithmetic, and the groups, then the
-// waves, are combined at the end in a fixed order.  `partial` as above.
+// ..), the next rounds' rows are asked for before this round's arithmetic, and the groups (by exchanges
+// between lanes and rows of lanes, no LDS), then the waves, are combined at the end in a fixed order.
+// Bound by trips to memory, few of which follow each other: q, the pages and two rounds of keys and values
+// are in flight at once.  `partial` as above; a range without keys leaves only its maximum and its sum.
+// With the merge, 16 ranges, 8 sequences of 1,040 keys, 16 heads of 128 over 4: bfloat16 22.4 -> 15.5 us, float32
+// 23.8 -> 16.0 against q read head by head, one round in flight and the sums through LDS.
 template <int CTRL>
 __device__ __forceinline__ float cap_dpp(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
 
-template <int DT>
-__device__ __forceinline__ void ld_unit(const void* p, size_t at, float* x) {
-    if (DT == ILLM_BF16) {
-        const uint4 r = *(const uint4*)((const bf16_t*)p + at);
-        const uint32_t w[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            x[2 * k] = __uint_as_float(w[k] << 16);
-            x[2 * k + 1] = __uint_as_float(w[k] & 0xffff0000u);
-        }
-    } else {
-        const float4 r = *(const float4*)((const float*)p + at);
-        x[0] = r.x; x[1] = r.y; x[2] = r.z; x[3] = r.w;
-    }
+// A lane's value and the one 16 (32) lanes away, in the order of their rows.
+__device__ __forceinline__ float2 cap_swap16(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+    return make_float2(__int_as_float(r[0]), __int_as_float(r[1]));
+}
+__device__ __forceinline__ float2 cap_swap32(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+    return make_float2(__int_as_float(r[0]), __int_as_float(r[1]));
+}
+// the sum over a wave's eight groups, without a trip through LDS: the other eight lanes of every sixteen, then
+// the row next to it, then the other half of the wave
+__device__ __forceinline__ float cap_sum_groups(float v) {
+    v += cap_dpp<0x128>(v);
+    float2 r = cap_swap16(v);
+    r = cap_swap32(r.x + r.y);
+    return r.x + r.y;
 }
 
 template <int DT, int KQ, int VQ, int DH>        // DH: query heads a block takes at most
@@ -1016,7 +1024,7 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
                              int keep, int kept, const float* __restrict__ sink) {
     constexpr int U = DT == ILLM_BF16 ? 8 : 4;          // elements of a unit
     constexpr int NK = U * KQ, NV = U * VQ;             // dims of a key, of a value, a lane holds
-    __shared__ float wacc[4][DH][8 * NV];
+    __shared__ __attribute__((aligned(16))) float wacc[4][DH][8 * NV];
     __shared__ float wm[4][DH], wl[4][DH];
     const int rep = nh / nkv, per_kv = (rep + DH - 1) / DH;
     const int kvh = blockIdx.x / per_kv, h0 = kvh * rep + (blockIdx.x % per_kv) * DH;
@@ -1028,8 +1036,18 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
     const int tiles = (seen.hi + 63) / 64, t0 = seen.lo / 64;
     const int per = (tiles - t0 + nsplit - 1) / nsplit;
     const int k_lo = max(seen.lo, (t0 + sp * per) * 64), k_hi = min(seen.hi, (t0 + (sp + 1) * per) * 64);
+    if (k_lo >= k_hi) {                            // no key: the merge leaves the range's values alone
+        if (nsplit > 1) {
+            if ((int)threadIdx.x < hb) {
+                float* pp = partial + (((size_t)b * nh + h0 + threadIdx.x) * nsplit + sp) * (dv + 2);
+                pp[dv] = NEG_INF; pp[dv + 1] = 0.f;
+            }
+            return;
+        }
+    }
     const float inv_cap = cap > 0.f ? 1.0f / cap : 0.f;
     float qv[DH][NK], acc[DH][NV], m[DH], l[DH], slope[DH];
+    illm_u32x4_t qr[DH][KQ];                       // (raw, as everything below: a conversion would wait for its load)
 #pragma unroll
     for (int i = 0; i < DH; ++i) {
         m[i] = NEG_INF; l[i] = 0.f;
@@ -1037,14 +1055,16 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
 #pragma unroll
         for (int c = 0; c < NV; ++c) acc[i][c] = 0.f;
 #pragma unroll
-        for (int j = 0; j < KQ; ++j) {
+        for (int j = 0; j < KQ; ++j) {             // (a head or a column that is not there reads one that is)
             const int d = U * sub + 8 * U * j;
-#pragma unroll
-            for (int c = 0; c < U; ++c) qv[i][U * j + c] = 0.f;
-            if (i < hb && d < dk) ld_unit<DT>(q, (size_t)b * q_stride + (size_t)(h0 + i) * dk + d, &qv[i][U * j]);
+            const size_t at = (size_t)b * q_stride + (size_t)(h0 + (i < hb ? i : 0)) * dk + (d < dk ? d : 0);
+            qr[i][j] = *(const illm_u32x4_t*)((const char*)q + at * (DT == ILLM_BF16 ? 2 : 4));
         }
     }
-    illm_u32x4_t kn[KQ], vn[VQ];                   // (raw: turned into floats when the round begins)
+    // two rounds in flight, one where a round's rows take more registers (float32 of more than 64 dims: 27.3
+    // us with two, 23.7 with one)
+    constexpr int AHEAD = KQ + VQ <= 4 ? 2 : 1;
+    illm_u32x4_t kn[AHEAD][KQ], vn[AHEAD][VQ];
     auto unit_floats = [&](const illm_u32x4_t r, float* x) __attribute__((always_inline)) {
         if (DT == ILLM_BF16) {
             const uint32_t wd[4] = {r.x, r.y, r.z, r.w};
@@ -1058,14 +1078,14 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
             x[2] = __uint_as_float(r.z); x[3] = __uint_as_float(r.w);
         }
     };
-    // the page of a round's key is looked up a round before its rows are asked for, so that a round
-    // waits for one trip to memory, not for two in a row
+    // the page of a round's key is looked up AHEAD rounds before its rows are asked for, and the rows AHEAD
+    // rounds before they are used
     auto page_of = [&](int base) __attribute__((always_inline)) {
         int lp = seen.at(min(base + grp, k_hi - 1)) / page_size;
         if (ring > 0 && lp >= kept) lp = kept + (lp - kept) % ring;
         return page_table[(size_t)slot * table_stride + lp];
     };
-    auto fetch = [&](int base, int page) __attribute__((always_inline)) {
+    auto fetch = [&](int s, int base, int page) __attribute__((always_inline)) {
         const int kj = seen.at(min(base + grp, k_hi - 1));
         const size_t row = ((size_t)page * nkv + kvh) * page_size + (kj % page_size);
         const size_t kat = row * dk, vat = row * dv;
@@ -1073,31 +1093,46 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
 #pragma unroll
         for (int j = 0; j < KQ; ++j) {
             const int d = U * sub + 8 * U * j;
-            kn[j] = illm_u32x4_t{0u, 0u, 0u, 0u};
-            if (d < dk) kn[j] = *(const illm_u32x4_t*)((const char*)kcache + (kat + d) * esz);
+            kn[s][j] = *(const illm_u32x4_t*)((const char*)kcache + (kat + (d < dk ? d : 0)) * esz);
         }
 #pragma unroll
         for (int j = 0; j < VQ; ++j) {
             const int d = U * sub + 8 * U * j;
-            vn[j] = illm_u32x4_t{0u, 0u, 0u, 0u};
-            if (d < dv) vn[j] = *(const illm_u32x4_t*)((const char*)vcache + (vat + d) * esz);
+            vn[s][j] = *(const illm_u32x4_t*)((const char*)vcache + (vat + (d < dv ? d : 0)) * esz);
         }
     };
-    int page_next = 0;
-    if (k_lo + 8 * w < k_hi) {
-        fetch(k_lo + 8 * w, page_of(k_lo + 8 * w));
-        page_next = page_of(k_lo + 8 * w + 32);
+    int pages[AHEAD];
+    const int r0 = k_lo + 8 * w;
+    if (k_lo < k_hi) {                             // (past the range: its last key again)
+        int p0[AHEAD];
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) p0[s] = page_of(r0 + 32 * s);
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) pages[s] = page_of(r0 + 32 * (AHEAD + s));
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) fetch(s, r0 + 32 * s, p0[s]);
     }
-    for (int base = k_lo + 8 * w; base < k_hi; base += 32) {
+#pragma unroll
+    for (int i = 0; i < DH; ++i)
+#pragma unroll
+        for (int j = 0; j < KQ; ++j) {
+            unit_floats(qr[i][j], &qv[i][U * j]);
+            const bool there = i < hb && U * sub + 8 * U * j < dk;
+#pragma unroll
+            for (int c = 0; c < U; ++c) qv[i][U * j + c] = there ? qv[i][U * j + c] : 0.f;
+        }
+    auto round = [&](auto S, int base) __attribute__((always_inline)) {
+        constexpr int s = S.value;
         float kc[NK], vc[NV];
 #pragma unroll
-        for (int j = 0; j < KQ; ++j) unit_floats(kn[j], &kc[U * j]);
+        for (int j = 0; j < KQ; ++j)                // (columns beyond dk: nothing; values beyond dv are not stored)
+            unit_floats(U * sub + 8 * U * j < dk ? kn[s][j] : illm_u32x4_t{0u, 0u, 0u, 0u}, &kc[U * j]);
 #pragma unroll
-        for (int j = 0; j < VQ; ++j) unit_floats(vn[j], &vc[U * j]);
-        if (base + 32 < k_hi) {
-            fetch(base + 32, page_next);
-            page_next = page_of(base + 64);
-        }
+        for (int j = 0; j < VQ; ++j) unit_floats(vn[s][j], &vc[U * j]);
+        // (without a branch, past the range its last row again: behind a branch the compiler can't count the
+        // loads in flight, and waits for all of them)
+        fetch(s, base + 32 * AHEAD, pages[s]);
+        pages[s] = page_of(base + 64 * AHEAD);
         const bool valid = base + grp < k_hi;
         const int kj = seen.at(base + grp);
 #pragma unroll
@@ -1125,27 +1160,29 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
 #pragma unroll
             for (int c = 0; c < NV; ++c) acc[i][c] = fmaf(p, vc[c], acc[i][c] * alpha);
         }
+    };
+    for (int base = r0; base < k_hi; base += 32 * AHEAD) {
+        round(std::integral_constant<int, 0>(), base);
+        if (AHEAD > 1) round(std::integral_constant<int, AHEAD - 1>(), base + 32);
     }
     // the wave's eight groups into one (every lane of a group holds the same m and l)
 #pragma unroll
     for (int i = 0; i < DH; ++i) {
         if (i >= hb) continue;
         float mm = m[i];
-        mm = fmaxf(mm, __shfl_xor(mm, 8, ILLM_WAVE));
-        mm = fmaxf(mm, __shfl_xor(mm, 16, ILLM_WAVE));
-        mm = fmaxf(mm, __shfl_xor(mm, 32, ILLM_WAVE));
+        mm = fmaxf(mm, cap_dpp<0x128>(mm));
+        float2 rows = cap_swap16(mm);
+        rows = cap_swap32(fmaxf(rows.x, rows.y));
+        mm = fmaxf(rows.x, rows.y);
         const float f = m[i] == NEG_INF ? 0.f : expf(m[i] - mm);
-        float lt = f * l[i];
-        lt += __shfl_xor(lt, 8, ILLM_WAVE);
-        lt += __shfl_xor(lt, 16, ILLM_WAVE);
-        lt += __shfl_xor(lt, 32, ILLM_WAVE);
+        const float lt = cap_sum_groups(f * l[i]);
+        float a[NV];
 #pragma unroll
-        for (int c = 0; c < NV; ++c) {
-            float a = f * acc[i][c];
-            a += __shfl_xor(a, 8, ILLM_WAVE);
-            a += __shfl_xor(a, 16, ILLM_WAVE);
-            a += __shfl_xor(a, 32, ILLM_WAVE);
-            if (grp == 0) wacc[w][i][U * sub + 8 * U * (c / U) + (c % U)] = a;
+        for (int c = 0; c < NV; ++c) a[c] = cap_sum_groups(f * acc[i][c]);
+        if (grp == 0) {
+#pragma unroll
+            for (int c = 0; c < NV; c += 4)
+                *(float4*)&wacc[w][i][U * sub + 8 * U * (c / U) + (c % U)] = make_float4(a[c], a[c + 1], a[c + 2], a[c + 3]);
         }
         if (lane == 0) { wm[w][i] = mm; wl[w][i] = lt; }
     }
@@ -1176,8 +1213,8 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
     }
 }
 
-// grid (heads, sequences): combine the splits' partial results in split order.  CAP_MERGE splits' maxima,
-// sums and values are asked for together before the first is used.
+// grid (heads, sequences), a thread a value dim (up to 256): combine the splits' partial results in split
+// order.  CAP_MERGE splits' maxima, sums and values are asked for together before the first is used.
 #define CAP_MERGE 16
 __global__ void attn_cap_merge_kernel(const float* __restrict__ partial, void* __restrict__ out,
                                       int dt, int nsplit, int nh, int dv, const void* __restrict__ gate,
@@ -1187,13 +1224,14 @@ __global__ void attn_cap_merge_kernel(const float* __restrict__ partial, void* _
     const float* pp = partial + ((size_t)b * nh + h) * nsplit * (dv + 2);
     const size_t step = dv + 2;
     float mm = NEG_INF;
-    for (int s0 = 0; s0 < nsplit; s0 += CAP_MERGE) {
-        float ms[CAP_MERGE];
+    if (nsplit > CAP_MERGE)
+        for (int s0 = 0; s0 < nsplit; s0 += CAP_MERGE) {
+            float ms[CAP_MERGE];
 #pragma unroll
-        for (int x = 0; x < CAP_MERGE; ++x) ms[x] = pp[(size_t)min(s0 + x, nsplit - 1) * step + dv];
+            for (int x = 0; x < CAP_MERGE; ++x) ms[x] = pp[(size_t)min(s0 + x, nsplit - 1) * step + dv];
 #pragma unroll
-        for (int x = 0; x < CAP_MERGE; ++x) mm = fmaxf(mm, ms[x]);
-    }
+            for (int x = 0; x < CAP_MERGE; ++x) mm = fmaxf(mm, ms[x]);
+        }
     float lt = 0.f;
     for (int d0 = 0; d0 < dv || d0 == 0; d0 += blockDim.x) {
         const int d = min(d0 + (int)threadIdx.x, dv - 1);
@@ -1206,11 +1244,16 @@ __global__ void attn_cap_merge_kernel(const float* __restrict__ partial, void* _
                 const float* p = pp + (size_t)min(s0 + x, nsplit - 1) * step;
                 ms[x] = p[dv]; ls[x] = p[dv + 1]; v[x] = p[d];
             }
+            if (nsplit <= CAP_MERGE) {
+#pragma unroll
+                for (int x = 0; x < CAP_MERGE; ++x) mm = fmaxf(mm, ms[x]);
+            }
 #pragma unroll
             for (int x = 0; x < CAP_MERGE; ++x) {
-                const float f = (s0 + x >= nsplit || ms[x] == NEG_INF) ? 0.f : expf(ms[x] - mm);
+                const bool keys = s0 + x < nsplit && ms[x] != NEG_INF;      // (a range without keys has no values)
+                const float f = keys ? expf(ms[x] - mm) : 0.f;
                 lt += f * ls[x];
-                a += f * v[x];
+                a = keys ? fmaf(f, v[x], a) : a;
             }
         }
         if (sink) add_sink(sink[h], mm, lt);
@@ -1285,7 +1328,7 @@ extern "C" int illm_attn_cap_decode(const void* q, int q_stride, void* out, int 
                            q_stride, kcache, vcache, page_table, table_stride, page_size, ring, seq_slot,
                            seq_len, partial, nsplit, nh, nkv, dk, dv, scale, cap, window, slopes, chunk, keep, kept);
     if (hipGetLastError() != hipSuccess) return ILLM_ERR_LAUNCH;
-    hipLaunchKernelGGL(attn_cap_merge_kernel, dim3(nh, B), dim3(64), 0, st, partial, out, dt, nsplit, nh, dv,
+    hipLaunchKernelGGL(attn_cap_merge_kernel, dim3(nh, B), dim3(dv <= 64 ? 64 : dv <= 128 ? 128 : 256), 0, st, partial, out, dt, nsplit, nh, dv,
                        gate, gate_stride, gate_off, gate_heads, lse, sink);
     return illm_launch_status();
 }

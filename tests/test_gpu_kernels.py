@@ -1441,3 +1441,27 @@ def test_gated_linear_attention_rows_four_columns_a_load(H, dk, dv, dtype):
         got = ops().gla_prepare(U.to(DEV), *args, Z.to(DEV), zb.to(DEV), 7.0, H, dk, dv)
         for a, b in zip(got, want):                     # (one exponential and one logarithm in float32)
             assert float((a.cpu().double() - b.double()).abs().max()) <= 1e-5 * max(1.0, float(b.abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nh, nkv, dk, dv", [(4, 1, 128, 128), (6, 2, 64, 32), (5, 1, 104, 72), (2, 2, 8, 128), (3, 1, 64, 8)])
+def test_capped_decode_ranges_and_rounds(nh, nkv, dk, dv, dtype):
+    """Key counts around a wave's rounds (32 keys) and the ranges' tiles (64), so that ranges are empty, end in their
+    first round or go past the two in flight; heads of a block that are not there; columns beyond the sizes."""
+    g = torch.Generator().manual_seed(nh * dk + dv)
+    lens, page = [1, 8, 31, 33, 64, 65, 97, 129, 200, 321], 16
+    B, per = len(lens), 21
+    table = torch.randperm(B * per, generator=g).view(B, per).to(torch.int32)
+    kc, vc = torch.randn(B * per, nkv, page, dk, generator=g).to(dtype), torch.randn(B * per, nkv, page, dv, generator=g).to(dtype)
+    q, slots = torch.randn(B, nh * dk, generator=g).to(dtype), torch.randperm(B, generator=g).to(torch.int32)
+    seq_len, slopes = torch.tensor(lens, dtype=torch.int32), torch.rand(nh, generator=g) * 0.1
+    put = lambda t: t.to(DEV)
+    for window, cap in ((0, 0.0), (70, 5.0)):
+        args = (nh, nkv, dk, dv, dk ** -0.5, cap, window)
+        want = R.attn_cap_decode(q, kc, vc, table, page, 0, slots, seq_len, *args, 1, slopes).double()
+        for nsplit in (1, 3, 16, 17):
+            got = ops().attn_cap_decode(put(q), put(kc), put(vc), put(table), page, 0, put(slots), put(seq_len), *args,
+                                        nsplit, put(slopes))
+            # float32: the scores' and sums' rounding; bfloat16: the result's (2^-9) and the exponential's
+            tol = 1e-5 if dtype == torch.float32 else 2 ** -8
+            assert float((got.double().cpu() - want).abs().max()) <= tol * max(1.0, float(want.abs().max())), (window, nsplit)
