@@ -256,7 +256,7 @@ attn_cap_rows_kernel(const void* __restrict__ q, int q_stride, void* __restrict_
                      const void* __restrict__ gate, int gate_stride, int gate_off, int gate_heads,
                      float* __restrict__ lse, int keep, int kept, int own_stride, int own_k,
                           int own_v_stride, int own_v, const float* __restrict__ sink) {
-    extern __shared__ float smem[];
+    extern __shared__ __attribute__((aligned(16))) float smem[];
     const int kp = dk + 1, vp = dv + 1;
     float* qs = smem;               // [CQ][kp]
     float* ks = qs + CQ * kp;       // [CK][kp]

@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(256)
 attn_prefill_generic_kernel(const void* __restrict__ qkv, void* __restrict__ out, int dt,
                             const int32_t* __restrict__ cu, int nh, int nkv, int hd, float scale,
                             int window, AttnPages pg) {
-    extern __shared__ float smem[];
+    extern __shared__ __attribute__((aligned(16))) float smem[];
     const int hp = hd + 1;
     float* qs = smem;            // [AQ][hp]
     float* ks = qs + AQ * hp;    // [AK][hp]

@@ -198,7 +198,7 @@ attn_pooled_rows_kernel(const void* __restrict__ q, int q_stride, void* __restri
                         int table_stride, int page_size, int nh, int nkv, int dk, int dv, float scale,
                         const float* __restrict__ head_scale, int window, int pool,
                         const float* __restrict__ lse) {
-    extern __shared__ float smem[];
+    extern __shared__ __attribute__((aligned(16))) float smem[];
     const int kp = dk + 1, vp = dv + 1;
     float* qs = smem;               // [PQ][kp]
     float* ks = qs + PQ * kp;       // [PK][kp]

@@ -68,7 +68,7 @@ gemm_rows_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ Wt, vo
                  int y_dt, int M, int N, int K, int tiles, int kp, GrRope rope, GrScale scale) {
     constexpr int UNITS = MT * 16 * GR_PIECE * 4;            // 16-byte units of a part's X piece
     constexpr int XU = (UNITS + TB * 64 - 1) / (TB * 64);    // units a thread stages
-    extern __shared__ uint4 lds[];       // X pieces [kp][2][UNITS]; afterwards the parts' sums
+    extern __shared__ __attribute__((aligned(16))) uint4 lds[];       // X pieces [kp][2][UNITS]; afterwards the parts' sums
     float* row_rs = (float*)(lds + (size_t)kp * 2 * UNITS);   // [16], behind the pieces (MT == 1)
     const int lane = threadIdx.x & 63, wave = wave_index();
     const int r = lane & 15, q = lane >> 4;

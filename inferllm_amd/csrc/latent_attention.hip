@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(256)
 latent_absorb_q_kernel(void* __restrict__ y, int dt, int ncols, const void* __restrict__ wuk,
                        int w_dt, void* __restrict__ qa, int qa_dt, int H, int dn, int dr, int R,
                        LatentStore st) {
-    extern __shared__ float qs[];
+    extern __shared__ __attribute__((aligned(16))) float qs[];
     const int b = blockIdx.x, h = blockIdx.y;
     if (FUSED && h == H) {
         latent_store_row(b, y, dt, ncols, H, dn, dr, R, st.rot, st.cos_sin, st.max_pos, st.nw, st.nw_dt,
@@ -248,7 +248,7 @@ __global__ void __launch_bounds__(256)
 latent_absorb_q_bf16_kernel(void* __restrict__ y, int dt, int ncols,
                             const bf16_t* __restrict__ wuk, void* __restrict__ qa, int qa_dt, int H,
                             int dn, int dr, int R, LatentStore st) {
-    extern __shared__ float sm[];
+    extern __shared__ __attribute__((aligned(16))) float sm[];
     float* qs = sm;                       // [dn + dr]
     float* part = sm + dn + dr;           // [groups][R]
     const int b = blockIdx.x, h = blockIdx.y;
@@ -367,7 +367,7 @@ latent_decode_kernel(const float* __restrict__ qa, const void* __restrict__ cach
                      const int32_t* __restrict__ seq_len, int len_more,
                      float* __restrict__ partial, int nsplit, int H, int R, int dr, float scale,
                      int window, int TK, int kstride) {
-    extern __shared__ size_t smem_raw[];
+    extern __shared__ __attribute__((aligned(16))) size_t smem_raw[];
     const int D = R + dr, HG = 4 * HGW;
     size_t* rowoff = smem_raw;                         // [TK]
     float* qs = (float*)(rowoff + TK);                 // [HG][D]
@@ -753,7 +753,8 @@ __global__ void __launch_bounds__(256)
 latent_merge_up_kernel(const float* __restrict__ partial, int nsplit, const void* __restrict__ wuv,
                        int w_dt, const void* __restrict__ y, int dt, int ncols, int gate_off,
                        void* __restrict__ out, int H, int R, int dv) {
-    extern __shared__ float ol[];                      // [R] combined sums, [nsplit] weights, then R % 4 == 0: [1024]
+    // [R] combined sums, [nsplit] weights, then, on 16 bytes, [1024] where R % 4 == 0
+    extern __shared__ __attribute__((aligned(16))) float ol[];
     float* ws = ol + R;
     __shared__ int filled;                             // ranges up to the last that holds keys
     const int b = blockIdx.x, h = blockIdx.y;
@@ -779,10 +780,10 @@ latent_merge_up_kernel(const float* __restrict__ partial, int nsplit, const void
         for (int s = lane; s < nsplit; s += 64) ws[s] = ws[s] / tot;
     }
     __syncthreads();
-    if (R % 4 == 0 && R <= 1024) {
+    if (R % 4 == 0 && R <= 1024 && (uintptr_t)partial % 16 == 0) {
         // a thread takes four neighbouring dims of every `turns`-th range, eight loads in flight
         const int r4 = R / 4, turns = 256 / r4, at = threadIdx.x % r4, mine = threadIdx.x / r4;
-        float* sums = ws + ((nsplit + 3) & ~3);        // [turns][R]
+        float* sums = ol + ((R + nsplit + 3) & ~3);    // [turns][R]
         if (mine < turns) {
             float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
             for (int s0 = mine; s0 < filled; s0 += 8 * turns) {

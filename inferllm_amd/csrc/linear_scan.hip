@@ -350,7 +350,7 @@ __global__ void __launch_bounds__(256)
 lru_gates_kernel(const float* __restrict__ u, const float* __restrict__ Wt, const float* __restrict__ br,
                  const float* __restrict__ bi, const float* __restrict__ lam, float rate,
                  float* __restrict__ a_out, float* __restrict__ x_out, int T, int C, int cb) {
-    extern __shared__ float us[];                   // [cb][ROWS], then the slices' partial sums
+    extern __shared__ __attribute__((aligned(16))) float us[];                   // [cb][ROWS], then the slices' partial sums
     const int t0 = blockIdx.x * ROWS, b = blockIdx.y, nb = C / cb;
     const int rows = min(ROWS, T - t0);
     for (int e = threadIdx.x; e < ROWS * cb; e += 256) {
@@ -432,7 +432,7 @@ __global__ void __launch_bounds__(256)
 lru_gates_few_kernel(const float* __restrict__ u, const float* __restrict__ Wt, const float* __restrict__ br,
                      const float* __restrict__ bi, const float* __restrict__ lam, float rate,
                      float* __restrict__ a_out, float* __restrict__ x_out, int T, int C, int cb) {
-    extern __shared__ float us[];                   // [cb][4 rows]
+    extern __shared__ __attribute__((aligned(16))) float us[];                   // [cb][4 rows]
     __shared__ float part[4][2][LRU_FEW_ROWS][32];  // the waves' sums
     const int t0 = blockIdx.x * LRU_FEW_ROWS, b = blockIdx.y, nb = C / cb;
     const int o_first = blockIdx.z * 32, rows = min(LRU_FEW_ROWS, T - t0);

@@ -97,7 +97,7 @@ post_add_norm_any_kernel(float* __restrict__ x, const void* __restrict__ a, int 
                          float gain, int out_kind, const void* __restrict__ w, const void* __restrict__ b,
                          int w_dt, float eps, void* __restrict__ out, int out_dt,
                          const int32_t* __restrict__ row_idx, int E) {
-    extern __shared__ float row[];
+    extern __shared__ __attribute__((aligned(16))) float row[];
     __shared__ float red[16];
     const int r = blockIdx.x;
     const size_t ib = (size_t)(row_idx ? row_idx[r] : r) * E, ob = (size_t)r * E;
@@ -195,7 +195,7 @@ struct PostMix {
 template <int NV, bool PAIR, bool SHIFT>
 __global__ void __launch_bounds__(256)
 post_mix_norm_kernel(PostMix m) {
-    extern __shared__ float row[];
+    extern __shared__ __attribute__((aligned(16))) float row[];
     __shared__ float red[16];
     const int r = blockIdx.x, E = m.E;
     const size_t in_row = m.row_idx ? m.row_idx[r] : r;

@@ -349,7 +349,7 @@ post_add_rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ a, int a
                         const int32_t* __restrict__ row_idx, int E, float eps,
                         const float* __restrict__ conv_w, int taps, void* __restrict__ tail, int tail_dt,
                         const int32_t* __restrict__ row_slot) {
-    extern __shared__ float row[];
+    extern __shared__ __attribute__((aligned(16))) float row[];
     __shared__ float red[16];
     const int r = blockIdx.x;
     const int in_row = row_idx ? row_idx[r] : r;

@@ -32,7 +32,7 @@ stream_mix_norm_kernel(float* __restrict__ x, const void* __restrict__ y1, int y
                        const float* __restrict__ read, const void* __restrict__ w, int w_dt,
                        void* __restrict__ h, int h_dt, const int32_t* __restrict__ row_idx, int E,
                        float eps) {
-    extern __shared__ float smem[];
+    extern __shared__ __attribute__((aligned(16))) float smem[];
     float* us = smem;
     float* red = smem + E;
     const size_t r = blockIdx.x;
