@@ -14,9 +14,10 @@
 
 // ---------------------------------------------------------------- router
 // z[t, e] = sum_k x[t, k] w[e, k] with a float32 matrix of few rows (a router): float32 products
-// and sums.  A wave takes 4 outputs and 8 tokens at a time (a chunk of a row of w serves 8 tokens,
-// a chunk of a token's row 4 outputs), lanes over K; every sum runs over K in the same order
-// whatever its companions.  grid (ceil(T / 8), ceil(NE / 16)).
+// and sums.  Every sum runs over K in the same order whatever its companions and their number, so
+// that near-tied experts are the same for a prompt's row and for the same token alone: a wave's lanes
+// take four neighbouring k each (one where K % 4), 256 (64) a turn, and the lanes' sums are added
+// half by half of the wave, then by quarters, down to neighbours.
 __device__ __forceinline__ float4 ld4_f32(const void* p, int dt, size_t i) {
     if (dt == ILLM_BF16) {
         const uint2 u = *(const uint2*)((const bf16_t*)p + i);
@@ -26,152 +27,150 @@ __device__ __forceinline__ float4 ld4_f32(const void* p, int dt, size_t i) {
     return *(const float4*)((const float*)p + i);
 }
 
-template <int EW>
+// wave_sum without a trip through LDS, the same additions in the same order: the other half of the wave, the
+// row of sixteen lanes beside, then within a row the lane 8, 4, 2 and 1 on (once lanes l and l ^ 8 hold the
+// same number, the lane 4 on holds that of l ^ 4, and so on down).
+template <int CTRL>
+__device__ __forceinline__ float few_dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float few_wave_sum(float v) {
+    auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+    v = __int_as_float(r[0]) + __int_as_float(r[1]);
+    r = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+    v = __int_as_float(r[0]) + __int_as_float(r[1]);
+    v += few_dpp<0x128>(v);
+    v += few_dpp<0x124>(v);
+    v += few_dpp<0x122>(v);
+    v += few_dpp<0x121>(v);
+    return v;
+}
+
+// Up to 16 tokens (single tokens of a batch): a wave an output of a token, V neighbouring k a lane, eight
+// turns of the lanes asked for before the first is used.  Bound by that trip to memory; with 8 tokens a wave it
+// was the chain of its loads and of 8 sums of 6 exchanges each: 64 outputs of K = 2,048 for 8 tokens 14.2 -> 2.2
+// us, 160 of 5,120 29.6 -> 4.7 (two tokens a wave 2.8 and 4.8, four 3.6 and 6.8).  grid (T, ceil(NE / 4)).
+template <int DT, int V>
+__global__ void __launch_bounds__(256)
+few_outputs_few_tokens_kernel(const void* __restrict__ x, const float* __restrict__ w, float* __restrict__ z, int NE,
+                              int K) {
+    constexpr int AHEAD = 8;
+    const size_t t = blockIdx.x;
+    const int e = blockIdx.y * 4 + wave_index(), lane = threadIdx.x & 63;
+    if (e >= NE) return;
+    const float* wr = w + (size_t)e * K;
+    float acc = 0.f;
+    for (int k0 = lane * V; k0 < K; k0 += 64 * V * AHEAD) {
+        float wv[AHEAD][V], xv[AHEAD][V];
+#pragma unroll
+        for (int a = 0; a < AHEAD; ++a) {               // (past K: the first turn's again, not used)
+            const int k = k0 + 64 * V * a < K ? k0 + 64 * V * a : k0;
+            if (V == 4) {
+                *(float4*)wv[a] = *(const float4*)(wr + k);
+                *(float4*)xv[a] = ld4_f32(x, DT, t * K + k);
+            } else {
+                wv[a][0] = wr[k];
+                xv[a][0] = ld_f(x, DT, t * K + k);
+            }
+        }
+        loads_asked_for();
+#pragma unroll
+        for (int a = 0; a < AHEAD; ++a) {
+            if (k0 + 64 * V * a >= K) continue;
+#pragma unroll
+            for (int j = 0; j < V; ++j) acc += xv[a][j] * wv[a][j];
+        }
+    }
+    acc = few_wave_sum(acc);
+    if (lane == 0) z[t * NE + e] = acc;
+}
+
+// More tokens: a wave takes 4 outputs and 8 tokens at a time (a chunk of a row of w serves 8 tokens, a chunk of
+// a token's row 4 outputs).  grid (ceil(T / 8), ceil(NE / 16)).
 __global__ void __launch_bounds__(256)
 few_outputs_f32_kernel(const void* __restrict__ x, int x_dt, const float* __restrict__ w,
                        float* __restrict__ z, int T, int NE, int K) {
     const int t0 = blockIdx.x * 8;
-    const int e0 = (blockIdx.y * 4 + wave_index()) * EW, lane = threadIdx.x & 63;
+    const int e0 = (blockIdx.y * 4 + wave_index()) * 4, lane = threadIdx.x & 63;
     if (e0 >= NE) return;
     const int nt = T - t0 < 8 ? T - t0 : 8;
-    const float* wr[EW];
+    const float* wr[4];
     size_t xr[8];
 #pragma unroll
-    for (int j = 0; j < EW; ++j) wr[j] = w + (size_t)(e0 + j < NE ? e0 + j : NE - 1) * K;
+    for (int j = 0; j < 4; ++j) wr[j] = w + (size_t)(e0 + j < NE ? e0 + j : NE - 1) * K;
 #pragma unroll
     for (int i = 0; i < 8; ++i) xr[i] = (size_t)(i < nt ? t0 + i : t0) * K;
-    float acc[8][EW];
+    float v[32];                                        // sum 4 i + j: token i, output j
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < EW; ++j) acc[i][j] = 0.f;
+    for (int i = 0; i < 32; ++i) v[i] = 0.f;
     if (K % 4 == 0) {
         // four neighbouring k a lane: one 16-byte load of w and one of 8 or 16 bytes of x
 #pragma unroll 2
         for (int k = lane * 4; k < K; k += 256) {
-            float4 wv[EW], xv[8];
+            float4 wv[4], xv[8];
 #pragma unroll
-            for (int j = 0; j < EW; ++j) wv[j] = *(const float4*)(wr[j] + k);
+            for (int j = 0; j < 4; ++j) wv[j] = *(const float4*)(wr[j] + k);
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 xv[i] = i < nt ? ld4_f32(x, x_dt, xr[i] + k) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int i = 0; i < 8; ++i)
 #pragma unroll
-                for (int j = 0; j < EW; ++j) {
-                    acc[i][j] += xv[i].x * wv[j].x; acc[i][j] += xv[i].y * wv[j].y;
-                    acc[i][j] += xv[i].z * wv[j].z; acc[i][j] += xv[i].w * wv[j].w;
+                for (int j = 0; j < 4; ++j) {
+                    v[4 * i + j] += xv[i].x * wv[j].x; v[4 * i + j] += xv[i].y * wv[j].y;
+                    v[4 * i + j] += xv[i].z * wv[j].z; v[4 * i + j] += xv[i].w * wv[j].w;
                 }
         }
     } else {
 #pragma unroll 4
         for (int k = lane; k < K; k += 64) {
-            float wv[EW], xv[8];
+            float wv[4], xv[8];
 #pragma unroll
-            for (int j = 0; j < EW; ++j) wv[j] = wr[j][k];
+            for (int j = 0; j < 4; ++j) wv[j] = wr[j][k];
 #pragma unroll
             for (int i = 0; i < 8; ++i) xv[i] = i < nt ? ld_f(x, x_dt, xr[i] + k) : 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i)
 #pragma unroll
-                for (int j = 0; j < EW; ++j) acc[i][j] += xv[i] * wv[j];
+                for (int j = 0; j < 4; ++j) v[4 * i + j] += xv[i] * wv[j];
         }
     }
-    if constexpr (EW == 4) {
-        // 32 sums over 64 lanes by halving: at the step that pairs lanes l and l ^ b a lane keeps the sums
-        // whose number has l's bit b, and sum 4 i + j ends in lane 4 i + j (and 32 on)
-        float v[32];
+    // 32 sums over 64 lanes by halving: at the step that pairs lanes l and l ^ b a lane keeps the sums whose
+    // number has that step's bit where l has b, 1 for b = 32 up to 16 for b = 2
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[4 * i + j] = acc[i][j];
-#pragma unroll
-        for (int b = 1, n = 16; b < 32; b <<= 1, n >>= 1) {
-            const bool up = (lane & b) != 0;
-#pragma unroll
-            for (int i = 0; i < n; ++i) {
-                const float keep = up ? v[2 * i + 1] : v[2 * i], send = up ? v[2 * i] : v[2 * i + 1];
-                v[i] = keep + __shfl_xor(send, b, ILLM_WAVE);
-            }
-        }
-        const float sum = v[0] + __shfl_xor(v[0], 32, ILLM_WAVE);
-        const int i = lane >> 2, j = lane & 3;
-        if (lane < 32 && i < nt && e0 + j < NE) z[(size_t)(t0 + i) * NE + e0 + j] = sum;
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        if (i >= nt) continue;
-#pragma unroll
-        for (int j = 0; j < EW; ++j) {
-            const float v = wave_sum(acc[i][j]);
-            if (lane == 0 && e0 + j < NE) z[(size_t)(t0 + i) * NE + e0 + j] = v;
-        }
-    }
-}
-
-// Up to 16 tokens (single tokens of a batch): a block an output and up to 8 tokens, its eight waves taking
-// 256 k in turn (K % 4 == 0), so that a router's whole row is asked for at once; a wave's 8 sums are added
-// over its lanes by halving, the waves' sums in wave order.  What bounded a wave an output walking K by
-// itself was the chain of its loads and of 8 sums of 6 exchanges each: 64 outputs of K = 2,048 for 8
-// tokens 26 -> 5 us.
-__global__ void __launch_bounds__(512)
-few_outputs_few_tokens_kernel(const void* __restrict__ x, int x_dt, const float* __restrict__ w,
-                              float* __restrict__ z, int T, int NE, int K) {
-    __shared__ float part[8][8];
-    const int t0 = blockIdx.x * 8, e = blockIdx.y, wave = wave_index(), lane = threadIdx.x & 63;
-    float acc[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] = 0.f;
-    for (int k = (wave * 64 + lane) * 4; k < K; k += 2048) {
-        const float4 wv = *(const float4*)(w + (size_t)e * K + k);
-        float4 xv[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) xv[i] = ld4_f32(x, x_dt, (size_t)min(t0 + i, T - 1) * K + k);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            acc[i] += xv[i].x * wv.x; acc[i] += xv[i].y * wv.y;
-            acc[i] += xv[i].z * wv.z; acc[i] += xv[i].w * wv.w;
-        }
-    }
-    // at the step that pairs lanes l and l ^ b a lane keeps the sums whose number has l's bit b: lane l is
-    // left with token l % 8's over its eighth of the lanes
-#pragma unroll
-    for (int b = 1, n = 4; b < 8; b <<= 1, n >>= 1) {
+    for (int b = 32, n = 16; b > 1; b >>= 1, n >>= 1) {
         const bool up = (lane & b) != 0;
 #pragma unroll
         for (int i = 0; i < n; ++i) {
-            const float keep = up ? acc[2 * i + 1] : acc[2 * i], send = up ? acc[2 * i] : acc[2 * i + 1];
-            acc[i] = keep + __shfl_xor(send, b, ILLM_WAVE);
+            const float keep = up ? v[2 * i + 1] : v[2 * i], send = up ? v[2 * i] : v[2 * i + 1];
+            v[i] = keep + __shfl_xor(send, b, ILLM_WAVE);
         }
     }
-    float v = acc[0];
-    v += __shfl_xor(v, 8, ILLM_WAVE);
-    v += __shfl_xor(v, 16, ILLM_WAVE);
-    v += __shfl_xor(v, 32, ILLM_WAVE);
-    if (lane < 8) part[wave][lane] = v;
-    __syncthreads();
-    if (threadIdx.x < 8 && t0 + (int)threadIdx.x < T) {
-        float sum = part[0][threadIdx.x];
-#pragma unroll
-        for (int i = 1; i < 8; ++i) sum += part[i][threadIdx.x];
-        z[(size_t)(t0 + threadIdx.x) * NE + e] = sum;
-    }
+    const float sum = v[0] + __shfl_xor(v[0], 1, ILLM_WAVE);
+    const int mine = (int)(__brev((uint32_t)lane) >> 26) & 31;      // lane bit 5 is the sum's bit 0, .., bit 1 its bit 4
+    const int i = mine >> 2, j = mine & 3;
+    if (!(lane & 1) && i < nt && e0 + j < NE) z[(size_t)(t0 + i) * NE + e0 + j] = sum;
 }
 
 extern "C" int illm_few_outputs_f32(const void* x, int x_dt, const float* w, float* z, int T, int NE,
                                     int K, void* stream) {
     if (T < 0 || NE <= 0 || NE > 65535 * 4 || K <= 0 || !illm_dtype_ok(x_dt)) return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
-    if (T <= 16 && K % 4 == 0 && NE <= 65535)
-        hipLaunchKernelGGL(few_outputs_few_tokens_kernel, dim3((T + 7) / 8, NE), dim3(512), 0, (hipStream_t)stream, x,
-                           x_dt, w, z, T, NE, K);
-    else if (T <= 16)   // few tokens: an output a wave, so that more waves share the reading
-        hipLaunchKernelGGL(few_outputs_f32_kernel<1>, dim3((T + 7) / 8, (NE + 3) / 4), dim3(256), 0,
-                           (hipStream_t)stream, x, x_dt, w, z, T, NE, K);
-    else
-        hipLaunchKernelGGL(few_outputs_f32_kernel<4>, dim3((T + 7) / 8, (NE + 15) / 16), dim3(256), 0,
-                           (hipStream_t)stream, x, x_dt, w, z, T, NE, K);
+    hipStream_t st = (hipStream_t)stream;
+    if (T <= 16) {
+#define GO(DT_, V_)                                                                                          \
+    hipLaunchKernelGGL((few_outputs_few_tokens_kernel<DT_, V_>), dim3(T, (NE + 3) / 4), dim3(256), 0, st, x, w, \
+                       z, NE, K)
+        if (K % 4) {
+            if (x_dt == ILLM_BF16) GO(ILLM_BF16, 1);
+            else GO(ILLM_F32, 1);
+        } else if (x_dt == ILLM_BF16) GO(ILLM_BF16, 4);
+        else GO(ILLM_F32, 4);
+#undef GO
+        return illm_launch_status();
+    }
+    hipLaunchKernelGGL(few_outputs_f32_kernel, dim3((T + 7) / 8, (NE + 15) / 16), dim3(256), 0, st, x, x_dt, w, z, T,
+                       NE, K);
     return illm_launch_status();
 }
 

@@ -626,12 +626,24 @@ def test_moe_tiles_of_128_pairs(T, E, F, NE, top, act):
 @pytest.mark.parametrize("xdt", DTYPES)
 @pytest.mark.parametrize("T,NE,K", [(1, 1, 4), (8, 64, 2048), (9, 65, 2052), (16, 7, 6144), (17, 33, 260), (100, 64, 512)])
 def test_few_outputs_rows(xdt, T, NE, K):
-    """A router's product at the edges of its two kernels: 8 tokens a block, waves of 256 k, 4 outputs a
-    wave; float32 sums in any order (K 2^-24 of the sum of magnitudes)."""
+    """A router's product at the edges of its two kernels (up to 16 tokens, eight turns of 256 k; 8 tokens a block,
+    4 outputs a wave); float32 sums in any order (K 2^-24 of the sum of magnitudes)."""
     x, w = rnd(T, K, dtype=xdt, seed=1), rnd(NE, K, seed=2)
     got = ops().few_outputs_f32(x.to(DEV), w.to(DEV)).double().cpu()
     room = (K + 8) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
     assert bool(((got - x.double() @ w.double().t()).abs() <= room).all())
+
+
+@pytest.mark.parametrize("xdt", DTYPES)
+@pytest.mark.parametrize("NE,K", [(64, 2048), (7, 6144), (33, 260), (5, 4), (65, 2050), (3, 61)])
+def test_few_outputs_of_a_row_alone_and_among_others(xdt, NE, K):
+    """A row's sums are the same bits alone, among 16 (the most of one kernel), 17 and 100 rows: a token's
+    near-tied experts don't hang on its company."""
+    x, w = rnd(100, K, dtype=xdt, seed=1).to(DEV), rnd(NE, K, seed=2).to(DEV)
+    every = ops().few_outputs_f32(x, w)
+    for T in (1, 2, 3, 15, 16, 17, 99):
+        for at in (0, 100 - T):
+            assert torch.equal(ops().few_outputs_f32(x[at:at + T].contiguous(), w), every[at:at + T]), (T, at)
 
 
 def test_moe_route_places():
