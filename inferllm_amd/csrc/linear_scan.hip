@@ -422,82 +422,94 @@ lru_gates_kernel(const float* __restrict__ u, const float* __restrict__ Wt, cons
     }
 }
 
-// The same for steps of few rows: 32 outputs and 4 rows a block, grid (ceil(T / 4), nb, ceil(cb / 32)).  Eight
-// lanes take four outputs each of one input at a time (every 32nd input, so that a wave reads 8 inputs'
-// 128 bytes at once); the 32 slices' sums are added over the wave's lanes and then over the waves, in a fixed order.
-// Bound by the trips of a thread's inputs, of which it has cb / 32 instead of cb cb / 256: 8 rows of 2,048 channels
-// in 16 blocks take 6.0 us, and took 24.2 us with a block's outputs all in one place (32 blocks on the chip).
+// The same for steps of few rows and maps of 64 channels or more, sum for sum in the same order (a row's gates are
+// the same bits alone and among many): 32 outputs and 4 rows a block, grid (ceil(T / 4), nb, ceil(cb / 32)); a
+// wave has both gates of the outputs and one of the slices that a map's inputs are cut into, S waves.
+// Bound by the trips to memory of a thread's inputs, AHEAD of which are under way twice over; a block with all
+// outputs of a map had 8 of each gate and left compute units idle: 16 maps of 128 x 128, 8 rows 14.3 -> 5.5 us,
+// 128 rows 15.3 -> 8.9; 8 of 256 x 256, 8 rows 38.6 -> 11.3; 16 of 64 x 64, 1 row 5.9 -> 3.9.  (Below 64 the tiles of many
+// rows: 16 of 32 x 32, 1 row 4.1 us against 5.2.)
 #define LRU_FEW_ROWS 4
+template <int AHEAD>
 __global__ void __launch_bounds__(256)
 lru_gates_few_kernel(const float* __restrict__ u, const float* __restrict__ Wt, const float* __restrict__ br,
                      const float* __restrict__ bi, const float* __restrict__ lam, float rate,
-                     float* __restrict__ a_out, float* __restrict__ x_out, int T, int C, int cb) {
-    extern __shared__ __attribute__((aligned(16))) float us[];                   // [cb][4 rows]
-    __shared__ float part[4][2][LRU_FEW_ROWS][32];  // the waves' sums
-    const int t0 = blockIdx.x * LRU_FEW_ROWS, b = blockIdx.y, nb = C / cb;
-    const int o_first = blockIdx.z * 32, rows = min(LRU_FEW_ROWS, T - t0);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int o = o_first + 4 * (lane & 7), sl = wave * 8 + (lane >> 3);
-    const float* wr = Wt + (size_t)b * cb * cb + (o < cb ? o : 0);
-    const float* wi = wr + (size_t)nb * cb * cb;
-    for (int i = tid; i < cb; i += 256) {
+                     float* __restrict__ a_out, float* __restrict__ x_out, int T, int C, int cb, int S) {
+    extern __shared__ __attribute__((aligned(16))) float us[];        // [cb][4 rows]
+    __shared__ float part[4][LRU_FEW_ROWS][64];                       // the slices' sums
+    const int t0 = blockIdx.x * LRU_FEW_ROWS, b = blockIdx.y, nb = C / cb, rows = min(LRU_FEW_ROWS, T - t0);
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
+    const int o = blockIdx.z * 32 + (lane & 31);
+    const float* const wp = Wt + ((size_t)(lane >= 32 ? nb : 0) + b) * cb * cb + min(o, cb - 1);
+    const float* const up = u + (size_t)t0 * C + (size_t)b * cb;
+    const int per = (cb + S - 1) / S, lo = wave * per, hi = min(cb, lo + per);
+    float w0[AHEAD], w1[AHEAD];
+    auto ask = [&](float* w, int i0) __attribute__((always_inline)) {           // (past the range: its last, not used)
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) w[k] = wp[(size_t)min(i0 + k, cb - 1) * cb];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    ask(w0, lo);
+    for (int i = tid; i < cb; i += blockDim.x) {
         float4 x;
-        x.x = u[(size_t)t0 * C + (size_t)b * cb + i];
-        x.y = rows > 1 ? u[(size_t)(t0 + 1) * C + (size_t)b * cb + i] : 0.f;
-        x.z = rows > 2 ? u[(size_t)(t0 + 2) * C + (size_t)b * cb + i] : 0.f;
-        x.w = rows > 3 ? u[(size_t)(t0 + 3) * C + (size_t)b * cb + i] : 0.f;
+        x.x = up[i];
+        x.y = rows > 1 ? up[(size_t)C + i] : 0.f;
+        x.z = rows > 2 ? up[2 * (size_t)C + i] : 0.f;
+        x.w = rows > 3 ? up[3 * (size_t)C + i] : 0.f;
         ((float4*)us)[i] = x;
     }
     __syncthreads();
-    float s[2][LRU_FEW_ROWS][4];
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto take = [&](float w, int i) __attribute__((always_inline)) {
+        const float4 x = ((const float4*)us)[i];
+        acc.x = fmaf(w, x.x, acc.x); acc.y = fmaf(w, x.y, acc.y);
+        acc.z = fmaf(w, x.z, acc.z); acc.w = fmaf(w, x.w, acc.w);
+    };
+    auto multiply = [&](const float* w, int i0) __attribute__((always_inline)) {
+        if (i0 + AHEAD <= hi) {
 #pragma unroll
-    for (int k = 0; k < 8 * LRU_FEW_ROWS; ++k) ((float*)s)[k] = 0.f;
-#pragma unroll 4
-    for (int i = sl; i < cb; i += 32) {
-        const float4 w1 = *(const float4*)(wr + (size_t)i * cb), w2 = *(const float4*)(wi + (size_t)i * cb);
-        const float4 x4 = ((const float4*)us)[i];
-        const float x[4] = {x4.x, x4.y, x4.z, x4.w};
+            for (int k = 0; k < AHEAD; ++k) take(w[k], i0 + k);
+        } else {
 #pragma unroll
-        for (int r = 0; r < LRU_FEW_ROWS; ++r) {
-            s[0][r][0] = fmaf(w1.x, x[r], s[0][r][0]); s[0][r][1] = fmaf(w1.y, x[r], s[0][r][1]);
-            s[0][r][2] = fmaf(w1.z, x[r], s[0][r][2]); s[0][r][3] = fmaf(w1.w, x[r], s[0][r][3]);
-            s[1][r][0] = fmaf(w2.x, x[r], s[1][r][0]); s[1][r][1] = fmaf(w2.y, x[r], s[1][r][1]);
-            s[1][r][2] = fmaf(w2.z, x[r], s[1][r][2]); s[1][r][3] = fmaf(w2.w, x[r], s[1][r][3]);
+            for (int k = 0; k < AHEAD; ++k)
+                if (i0 + k < hi) take(w[k], i0 + k);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int i0 = lo; i0 < hi; i0 += 2 * AHEAD) {
+        ask(w1, i0 + AHEAD);
+        multiply(w0, i0);
+        ask(w0, i0 + 2 * AHEAD);
+        multiply(w1, i0 + AHEAD);
+    }
+    if (S > 1) {
+#pragma unroll
+        for (int r = 0; r < LRU_FEW_ROWS; ++r) part[wave][r][lane] = ((const float*)&acc)[r];
+        __syncthreads();
+        if (wave > 0) return;
+        for (int s = 1; s < S; ++s) {
+            acc.x += part[s][0][lane]; acc.y += part[s][1][lane];
+            acc.z += part[s][2][lane]; acc.w += part[s][3][lane];
         }
     }
-    // over the lanes of the same outputs by halves: a lane keeps the half of its sums that its bit names
-    // and gives the other away, so that it ends with one gate's four outputs of one row pair's row
-    const bool up32 = lane & 32, up16 = lane & 16, up8 = lane & 8;
-    float h1[LRU_FEW_ROWS][4];
+    // lanes below 32 hold their output's first gate, those above its second: rows 0 and 1 to the ones, 2 and 3 to the others
+    const bool high = lane >= 32;
+    const float4 oth = make_float4(__shfl_xor(acc.x, 32, ILLM_WAVE), __shfl_xor(acc.y, 32, ILLM_WAVE),
+                                   __shfl_xor(acc.z, 32, ILLM_WAVE), __shfl_xor(acc.w, 32, ILLM_WAVE));
+    if (o >= cb) return;
+    const int c = b * cb + o;
+    const float sp = ls_softplus(lam[c]), b1 = br[c], b2 = bi[c];
 #pragma unroll
-    for (int k = 0; k < 4 * LRU_FEW_ROWS; ++k) {
-        const float keep = up32 ? ((float*)s[1])[k] : ((float*)s[0])[k], give = up32 ? ((float*)s[0])[k] : ((float*)s[1])[k];
-        ((float*)h1)[k] = keep + __shfl_xor(give, 32);
+    for (int k = 0; k < 2; ++k) {
+        const int r = (high ? 2 : 0) + k;
+        if (r >= rows) continue;
+        const float ar = high ? (k ? oth.w : oth.z) : (k ? acc.y : acc.x), ai = high ? (k ? acc.w : acc.z) : (k ? oth.y : oth.x);
+        const float rg = ls_sigmoid(ar + b1), ig = ls_sigmoid(ai + b2);
+        const float log_a = -rate * rg * sp;
+        a_out[(size_t)(t0 + r) * C + c] = expf(log_a);
+        // 1 - a^2 as -expm1(2 log a): a decay close to 1 keeps its digits
+        x_out[(size_t)(t0 + r) * C + c] = sqrtf(fmaxf(-expm1f(2.0f * log_a), 0.f)) * ig * us[o * LRU_FEW_ROWS + r];
     }
-    float h2[2][4];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const float keep = up16 ? ((float*)h1[2])[k] : ((float*)h1[0])[k], give = up16 ? ((float*)h1[0])[k] : ((float*)h1[2])[k];
-        ((float*)h2)[k] = keep + __shfl_xor(give, 16);
-    }
-    float4 h3;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const float keep = up8 ? h2[1][k] : h2[0][k], give = up8 ? h2[0][k] : h2[1][k];
-        ((float*)&h3)[k] = keep + __shfl_xor(give, 8);
-    }
-    *(float4*)&part[wave][up32 ? 1 : 0][(up16 ? 2 : 0) + (up8 ? 1 : 0)][4 * (lane & 7)] = h3;
-    __syncthreads();
-    const int oo = tid & 31, r = tid >> 5;
-    if (r >= rows || o_first + oo >= cb) return;
-    const float ar = (part[0][0][r][oo] + part[1][0][r][oo]) + (part[2][0][r][oo] + part[3][0][r][oo]);
-    const float ai = (part[0][1][r][oo] + part[1][1][r][oo]) + (part[2][1][r][oo] + part[3][1][r][oo]);
-    const int c = b * cb + o_first + oo;
-    const float rg = ls_sigmoid(ar + br[c]), ig = ls_sigmoid(ai + bi[c]);
-    const float log_a = -rate * rg * ls_softplus(lam[c]);
-    a_out[(size_t)(t0 + r) * C + c] = expf(log_a);
-    // 1 - a^2 as -expm1(2 log a): a decay close to 1 keeps its digits
-    x_out[(size_t)(t0 + r) * C + c] = sqrtf(fmaxf(-expm1f(2.0f * log_a), 0.f)) * ig * us[(o_first + oo) * LRU_FEW_ROWS + r];
 }
 
 template <int ROWS>
@@ -523,10 +535,21 @@ extern "C" int illm_lru_gates(const float* u, const float* Wt, const float* br, 
     if (T < 0 || C <= 0 || nb <= 0 || C % nb || nb > 65535) return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
     const int cb = C / nb;
-    if (T <= 128 && cb % 4 == 0 && cb <= 3072 && (uintptr_t)Wt % 16 == 0) {
-        hipLaunchKernelGGL(lru_gates_few_kernel, dim3((T + LRU_FEW_ROWS - 1) / LRU_FEW_ROWS, nb, (cb + 31) / 32), dim3(256),
-                           (size_t)cb * LRU_FEW_ROWS * sizeof(float), (hipStream_t)stream, u, Wt, br, bi, lam, rate,
-                           a_out, x_out, T, C, cb);
+    if (T <= 128 && cb >= 64 && cb <= 4096) {
+        const int S = cb < 256 ? 256 / cb : 1;
+        const size_t lds = (size_t)cb * LRU_FEW_ROWS * sizeof(float);
+#define GO(AHEAD_)                                                                                                 \
+    do {                                                                                                           \
+        if (lds > 48 * 1024 && hipFuncSetAttribute((const void*)lru_gates_few_kernel<AHEAD_>,                        \
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) \
+            return ILLM_ERR_LAUNCH;                                                                                \
+        hipLaunchKernelGGL(lru_gates_few_kernel<AHEAD_>, dim3((T + LRU_FEW_ROWS - 1) / LRU_FEW_ROWS, nb, (cb + 31) / 32), \
+                           dim3(64 * S), lds, (hipStream_t)stream, u, Wt, br, bi, lam, rate, a_out, x_out, \
+                           T, C, cb, S);                                                                           \
+    } while (0)
+        if ((cb + S - 1) / S <= 32) GO(16);
+        else GO(32);
+#undef GO
         return illm_launch_status();
     }
     // tiles of 16 rows where a block's inputs of 16 rows fit LDS (blocks of up to 1,024 channels)

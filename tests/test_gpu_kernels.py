@@ -1429,8 +1429,8 @@ def test_norm_mix_and_store_four_columns_a_load(nh, nkv, dk, dv, weights, mix, d
 @pytest.mark.parametrize("T", [1, 4, 7, 128, 129])
 @pytest.mark.parametrize("nb, cb", [(2, 4), (3, 32), (1, 36), (2, 128), (1, 1028), (2, 30)])
 def test_recurrent_gates_of_few_rows(T, nb, cb):
-    """Blocks of channels around the 32 outputs and 32 slices a block takes; rows around its 4; 129 rows and widths
-    that are no multiple of 4 take the other kernel."""
+    """Blocks of channels around the 32 outputs a block takes; rows around its 4; 129 rows and blocks below 64
+    channels take the other kernel."""
     g = torch.Generator().manual_seed(T + cb)
     u = torch.randn(T, nb * cb, generator=g) * 2
     wt = torch.randn(2, nb, cb, cb, generator=g) * min(0.5, 4.0 / cb ** 0.5)
@@ -1439,6 +1439,22 @@ def test_recurrent_gates_of_few_rows(T, nb, cb):
                          R.lru_gates(u, wt, rb, ib, lam, 8.0)):
         # sums of up to 1,028 products of size 8 in float32, through functions of slope below 8
         assert float((got.cpu().double() - want.double()).abs().max()) <= 1e-5 * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("nb, cb", [(2, 4), (3, 36), (3, 64), (2, 65), (16, 128), (1, 129), (2, 200), (2, 256), (1, 1028), (1, 3072),
+                                    (1, 4096)])
+def test_recurrent_gates_of_a_row_alone_and_among_others(nb, cb):
+    """A row's gates are the same bits alone, among 128 rows (the most of one kernel) and among 129: blocks narrower
+    and wider than a thread block, with a last slice of their inputs cut short, up to the widest that was ever taken."""
+    g = torch.Generator().manual_seed(cb)
+    u = (torch.randn(129, nb * cb, generator=g) * 2).to(DEV)
+    maps = [t.to(DEV) for t in (torch.randn(2, nb, cb, cb, generator=g) * min(0.5, 4.0 / cb ** 0.5),
+                                *(torch.randn(nb * cb, generator=g) for _ in range(3)))]
+    every = ops().lru_gates(u, *maps, 8.0)
+    for T in (1, 3, 4, 5, 128):
+        for at in (0, 129 - T):
+            for a, b in zip(ops().lru_gates(u[at:at + T].contiguous(), *maps, 8.0), every):
+                assert torch.equal(a, b[at:at + T]), (T, at)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
