@@ -109,7 +109,7 @@ int illm_gemm_f32_mfma(const float* X, const float* W, void* Y, int y_dt, int M,
 
 // Products of up to 256 bfloat16 rows from row-major W, K % 64 == 0, N % 4 == 0 (csrc/gemm_tiles.hip): K
 // cut into `splits` parts (illm_gemm_tiles_splits(N, K), or any number that leaves no part empty) as
-// float32 planes [splits][M][N].
+// float32 planes [splits][M][N].  X, W and Y on 16-byte addresses.
 int illm_gemm_tiles_splits(int N, int K);
 int illm_gemm_tiles_planes(const void* X, const void* W, float* Y, int M, int N, int K, int splits,
                            void* stream);

@@ -131,11 +131,13 @@ extern "C" int illm_gemm_tiles_splits(int N, int K) {
 }
 
 // X [M <= 256, K], W [N, K], K % 64 == 0, N % 4 == 0, planes Y float32 [splits][M][N], no part of K empty; X
-// and W each within the 4 GiB that a load's 32-bit offset reaches.  Else ILLM_ERR_ARG.
+// and W each within the 4 GiB that a load's 32-bit offset reaches; X, W and Y on 16-byte addresses (a lane brings or
+// stores 16 bytes at a time).  Else ILLM_ERR_ARG.
 extern "C" int illm_gemm_tiles_planes(const void* X, const void* W, float* Y, int M, int N, int K, int splits,
                                       void* stream) {
     if (!X || !W || !Y || M <= 0 || M > 256 || N <= 0 || K <= 0 || K % GT_K || N % 4 || splits < 1 || splits > 65535 ||
-        (long long)(N + 63) * K * 2 >= 0xffffffffLL || 256LL * K * 2 >= 0xffffffffLL)
+        (long long)(N + 63) * K * 2 >= 0xffffffffLL || 256LL * K * 2 >= 0xffffffffLL ||
+        ((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16)
         return ILLM_ERR_ARG;
     const int every = K / GT_K, per = (every + splits - 1) / splits;
     if ((long long)(splits - 1) * per >= every) return ILLM_ERR_ARG;

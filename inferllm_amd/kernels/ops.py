@@ -71,6 +71,11 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+def _on16(*tensors: Optional[torch.Tensor]) -> bool:
+    """Whether the tensors' first elements lie on 16-byte addresses (views may begin anywhere)."""
+    return all(t is None or t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def _need(cond: bool, msg: str) -> None:
     if not cond:
         raise KernelError(msg)
@@ -783,15 +788,26 @@ CUT_MIN_K = 4096          # product and the norm that adds the planes against th
                           # 2048 x 5376 21 / 22 / 24 -> 16 / 18 / 20; 2048 x 2048 13 / 14 / 15 -> 13 / 14 / 17
 
 
+CUT_SHORT_ROWS = 192     # up to these it is the faster way for every number of columns; above, with one stage less in
+                         # flight, not where blocks of 64 columns and parts of 512 k (the shortest) leave the chip idle and
+                         # the matrix is no small one (us at 129 / 192 / 256 rows, K = 4,096: 64 columns 14 / 14 / 14 -> 9 / 10 / 12,
+                         # 256 14 / 15 / 15 -> 10 / 11 / 12, 768 15 / 15 / 16 -> 12 / 14 / 16, 1,024 16 / 16 / 16 -> 13 / 15 / 18, 1,536
+                         # 17 / 20 / 21 -> 16 / 17 / 19; K = 8,192: 256 14 / 14 / 14 -> 12 / 13 / 15, 1,024 23 / 24 / 24 -> 15 / 17 / 20)
+
+
 def linear_cut_fits(x, w) -> bool:
     """Whether `linear_cut` takes these operands and is the faster way: 129 to 256 bfloat16 rows and a
-    row-major matrix (its plain copy) with few rows for its length (K >= N, K a multiple of 64)."""
+    row-major matrix (its plain copy) with few rows for its length (K >= N, K a multiple of 64), both on
+    16-byte addresses and within a load's 32-bit offset."""
     w = plain_weight(w)
-    return (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+    if not (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and x.dim() == 2 and w.dim() == 2 and CUT_ROWS[0] <= x.shape[0] <= CUT_ROWS[1]
-            and x.shape[1] == w.shape[1] and w.is_contiguous() and w.shape[1] % 64 == 0
-            and w.shape[0] % 4 == 0 and CUT_MIN_K <= w.shape[1] and w.shape[0] <= w.shape[1]
-            and w.shape[0] <= _plan.rules.planes_most_cols and w.numel() * 2 < 0xffffffff)
+            and x.shape[1] == w.shape[1] and w.is_contiguous()):
+        return False
+    M, (N, K) = x.shape[0], w.shape
+    return (K % 64 == 0 and N % 4 == 0 and CUT_MIN_K <= K and N <= K and N <= _plan.rules.planes_most_cols
+            and (M <= CUT_SHORT_ROWS or N * K <= 1 << 20 or (N + 63) // 64 * (K // 512) >= 192) and 2 * max(N + 63, 256) * K < 0xffffffff
+            and _on16(w) and (_on16(x) or not x.is_contiguous()))
 
 
 def linear_cut(x: torch.Tensor, w, splits: int = 0) -> torch.Tensor:

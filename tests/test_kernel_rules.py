@@ -1,0 +1,37 @@
+"""The rules that send a call to one kernel or another, and what the library refuses before it launches anything:
+no GPU is needed for either."""
+import torch
+
+from inferllm_amd.kernels import ops
+
+ERR_ARG = 1
+AT = 1 << 20                                               # an address that nothing reads: the call is refused
+
+
+def test_the_cut_product_is_given_only_what_it_takes():
+    """`linear_cut_fits` against the library's own limits: sizes near 4 GiB and views that begin off a 16-byte
+    address go to the product they took before."""
+    def fits(M, N, K, x_at=0, w_at=0, **kw):
+        x = torch.empty(x_at + M * K, dtype=torch.bfloat16, **kw)[x_at:].view(M, K)
+        w = torch.empty(w_at + N * K, dtype=torch.bfloat16, **kw)[w_at:].view(N, K)
+        return ops.linear_cut_fits(x, w)
+
+    lib = ops._lib()
+    rc = lambda M, N, K, X=AT, W=AT, Y=AT: lib.illm_gemm_tiles_planes(X, W, Y, M, N, K, 1, None)  # noqa: E731
+    assert fits(129, 4096, 4096) and fits(256, 4096, 4096) and not fits(128, 4096, 4096) and not fits(257, 4096, 4096)
+    # more than 192 rows, too few blocks: the vendor's product
+    assert fits(192, 1024, 4096) and not fits(193, 1024, 4096) and fits(193, 1536, 4096) and fits(256, 256, 4096)
+    # the last K that the planes' offsets reach (N + 63 rows of W, 256 of X), and the next
+    for N in (1536, 4096):
+        last = (0xffffffff - 1) // (2 * (N + 63)) // 64 * 64
+        assert fits(200, N, last, device="meta") and not fits(200, N, last + 64, device="meta")
+        assert rc(200, N, last + 64) == ERR_ARG
+    assert rc(150, 4, (0xffffffff // 512 // 64 + 1) * 64) == ERR_ARG
+    assert not fits(150, 4, (0xffffffff // 512 // 64 + 1) * 64, device="meta")
+    for off in (1, 4):                                     # 2 and 8 bytes off
+        assert not fits(129, 2048, 4096, x_at=off) and not fits(129, 2048, 4096, w_at=off)
+    for off in (2, 4, 8):
+        assert rc(129, 64, 4096, X=AT + off) == rc(129, 64, 4096, W=AT + off) == rc(129, 64, 4096, Y=AT + off) == ERR_ARG
+    # rows that are columns of wider ones are copied first
+    wide = torch.empty(129, 4104, dtype=torch.bfloat16)[:, 1:4097]
+    assert ops.linear_cut_fits(wide, torch.empty(2048, 4096, dtype=torch.bfloat16))
