@@ -807,7 +807,7 @@ moe_rows_mfma_lds_kernel(const bf16_t* __restrict__ X, int x_div, const bf16_t* 
 // 128 rows of W (gated: 64 gate rows and their 64 up rows), a wave 64 x 64; both operands go straight from
 // memory into LDS, 64 k (a row's 128 bytes) a stage, X's rows gathered by the load, two stages, one barrier
 // each.  A load instruction brings 8 rows; 16-byte piece c of row t stands at place c ^ (t % 8) of the row.
-// X and an expert's W each within the 4 GiB that a load's 32-bit offset reaches.
+// X and an expert's W each within the 4 GiB that a load's 32-bit offset reaches; X, W and Y on 16-byte addresses.
 // What bounded the waves that read their rows of W themselves was that stream (16 rows x 64 bytes an
 // instruction, one step ahead) and a tile's W read once for every 64 pairs.  64 experts of 1408 x 2048, both
 // products: 2,964 tokens 1,023 -> 608 us (505 TFLOP/s), 64 tokens 303 -> 236 (1.1 GB of experts at 4.7 TB/s).
@@ -925,7 +925,9 @@ extern "C" int illm_moe_rows_mfma(const void* X, int x_div, const void* W, int g
     if (max_tiles == 0) return ILLM_OK;
     hipStream_t st = (hipStream_t)stream;
     if (tile_rows == 128) {
-        if (K % 64 || N % 4 || (long long)(gated ? 2 : 1) * (N + 128) * K * 2 >= 0xffffffffLL) return ILLM_ERR_ARG;
+        if (K % 64 || N % 4 || (long long)(gated ? 2 : 1) * (N + 128) * K * 2 >= 0xffffffffLL ||
+            ((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16)
+            return ILLM_ERR_ARG;
         const int cols = (N + (gated ? 63 : 127)) / (gated ? 64 : 128);
         const long long blocks = 8LL * ((cols + 7) / 8) * max_tiles;
         if (blocks > 0x7fffffffLL) return ILLM_ERR_ARG;

@@ -1523,9 +1523,14 @@ def _moe_tiling(dtype: torch.dtype, E: int, F: int, NP: int, n_exp: int):
     return mfma, rows, max(1, min(NP, NP // rows + n_exp))
 
 
-def _moe_group(idx: torch.Tensor, n_exp: int, dtype: torch.dtype, E: int, F: int):
+def _moe_group(idx: torch.Tensor, n_exp: int, dtype: torch.dtype, E: int, F: int, on16: bool = True):
+    """The pairs grouped by expert.  `on16`: the rows and the experts' matrices lie on 16-byte addresses, as the
+    tiles of 128 pairs want them (straight into LDS, 16 bytes a lane)."""
     NP = idx.numel()
     mfma, rows, max_tiles = _moe_tiling(dtype, E, F, NP, n_exp)
+    if rows == 128 and not on16:
+        rows = 16
+        max_tiles = max(1, min(NP, NP // rows + n_exp))
     order = torch.empty((NP,), dtype=torch.int32, device=idx.device)
     tiles = torch.empty((3 * max_tiles + 1,), dtype=torch.int32, device=idx.device)
     _check(_lib().illm_moe_group(_p(idx), NP, n_exp, _p(order), _p(tiles), max_tiles, rows,
@@ -1575,7 +1580,10 @@ def moe_experts(h: torch.Tensor, idx: torch.Tensor, w_gate_up: torch.Tensor, w_d
           and w_gate_up.dtype == h.dtype and w_down.dtype == h.dtype and idx.shape[0] == T,
           "moe_experts: shapes or dtypes")
     NP = T * top
-    order, tiles, max_tiles, rows, mfma = grouped if grouped is not None else _moe_group(idx, n_exp, h.dtype, E, F)
+    on16 = _on16(h, w_gate_up, w_down)
+    if grouped is None or (grouped[3] == 128 and not on16):
+        grouped = _moe_group(idx, n_exp, h.dtype, E, F, on16)
+    order, tiles, max_tiles, rows, mfma = grouped
     act = torch.empty((NP, F), dtype=h.dtype, device=h.device)
     y = torch.empty((NP, E), dtype=h.dtype, device=h.device)
     if mfma:

@@ -623,6 +623,24 @@ def test_moe_tiles_of_128_pairs(T, E, F, NE, top, act):
     assert real(torch.bfloat16, E, F, 2 * NE, NE)[1] == 128 and real(torch.bfloat16, E, F + 32, 2 * NE, NE)[1] != 128
 
 
+def test_moe_experts_of_views_that_begin_anywhere():
+    """Rows and experts' matrices whose first element is no multiple of 16 bytes give the bits of copies that are,
+    with the pairs grouped beforehand and not."""
+    o, T, E, F, NE, top = ops(), 130, 128, 192, 3, 2
+    h, wu, wd = (rnd(*s, dtype=torch.bfloat16, seed=i).to(DEV) * 0.3 for i, s in enumerate([(T, E), (NE, 2 * F, E), (NE, E, F)]))
+    idx = torch.stack([torch.randperm(NE)[:top] for _ in range(T)]).to(torch.int32).to(DEV)
+    want = o.moe_experts(h, idx, wu, wd)
+
+    def off(t):
+        v = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:].view(t.shape)
+        return v.copy_(t)
+    plan = o._moe_group(idx, NE, h.dtype, E, F)
+    assert plan[3] == 128
+    for a, b, c in ((off(h), wu, wd), (h, off(wu), wd), (h, wu, off(wd))):
+        assert torch.equal(o.moe_experts(a, idx, b, c), want)
+        assert torch.equal(o.moe_experts(a, idx, b, c, plan), want)
+
+
 @pytest.mark.parametrize("xdt", DTYPES)
 @pytest.mark.parametrize("T,NE,K", [(1, 1, 4), (8, 64, 2048), (9, 65, 2052), (16, 7, 6144), (17, 33, 260), (100, 64, 512)])
 def test_few_outputs_rows(xdt, T, NE, K):

@@ -35,3 +35,12 @@ def test_the_cut_product_is_given_only_what_it_takes():
     # rows that are columns of wider ones are copied first
     wide = torch.empty(129, 4104, dtype=torch.bfloat16)[:, 1:4097]
     assert ops.linear_cut_fits(wide, torch.empty(2048, 4096, dtype=torch.bfloat16))
+
+
+def test_the_experts_tiles_of_128_pairs_refuse_other_addresses():
+    """Rows and matrices go straight into LDS 16 bytes a lane: what does not lie on 16 bytes is refused (the caller
+    groups such pairs for the kernels of 16 to 64)."""
+    call = lambda rows=128, X=AT, W=AT, Y=AT: ops._lib().illm_moe_rows_mfma(  # noqa: E731
+        X, 1, W, 0, rows, AT, AT, 1, Y, 64, 64, 0, 0.0, None, None)
+    for off in (2, 8):
+        assert call(X=AT + off) == call(W=AT + off) == call(Y=AT + off) == ERR_ARG
