@@ -1027,7 +1027,7 @@ moe_combine_kernel(const void* __restrict__ h, int dt, const int32_t* __restrict
     }
 }
 
-// The same with V neighbouring columns a thread (16-byte loads; E % V == 0, top <= MOE_COMBINE_TOP) and a
+// The same with V neighbouring columns a thread (16-byte loads from 16-byte addresses; E % V == 0, top <= MOE_COMBINE_TOP) and a
 // block a token: the gate's dot product is formed once a token, and all of a thread's rows are asked for
 // together (2,964 tokens of 2,048, 6 chosen: 200 -> 40 us; 8 tokens 10.5 -> 6.5).
 template <int DT, int V>
@@ -1085,7 +1085,8 @@ extern "C" int illm_moe_combine(const void* h, int dt, const int32_t* idx, const
         (E + 255) / 256 > 65535)
         return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
-    if (top <= MOE_COMBINE_TOP && E % (dt == ILLM_BF16 ? 8 : 4) == 0) {
+    const uintptr_t at = (uintptr_t)h | (uintptr_t)Y | (uintptr_t)shared | (uintptr_t)out;
+    if (top <= MOE_COMBINE_TOP && E % (dt == ILLM_BF16 ? 8 : 4) == 0 && at % 16 == 0) {
         if (dt == ILLM_BF16)
             hipLaunchKernelGGL((moe_combine_vec_kernel<ILLM_BF16, 8>), dim3(T), dim3(256), 0, (hipStream_t)stream, h, idx,
                                wt, Y, shared, sg, sg_dt, out, E, top, NEr);

@@ -623,6 +623,27 @@ def test_moe_tiles_of_128_pairs(T, E, F, NE, top, act):
     assert real(torch.bfloat16, E, F, 2 * NE, NE)[1] == 128 and real(torch.bfloat16, E, F + 32, 2 * NE, NE)[1] != 128
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_moe_combine_of_views_that_begin_anywhere(dtype):
+    """The weighted sum reads 16 bytes at a time only from addresses that are multiples of 16: views that begin
+    elsewhere (by column, a gate's sum in another order) are as close to 64 bits."""
+    o, T, E, top = ops(), 5, 64, 3
+    h, y, sh, sg = rnd(T, E, dtype=dtype, seed=1), rnd(T * top, E, dtype=dtype, seed=2), rnd(T, E, dtype=dtype, seed=3), rnd(E, seed=4)
+    idx = torch.randint(0, 5, (T, top), generator=torch.Generator().manual_seed(5)).to(torch.int32)
+    wt = torch.rand(T, top, generator=torch.Generator().manual_seed(6))
+    rows = torch.where((idx < 4)[:, :, None], y.double().view(T, top, E), h.double()[:, None])
+    want = (rows * wt.double()[:, :, None]).sum(1) + torch.sigmoid(h.double() @ sg.double())[:, None] * sh.double()
+
+    def off(t):
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:].view(t.shape).copy_(t)
+    on = [t.to(DEV) for t in (h, y, sh)]
+    for k in range(4):
+        a, b, c = [off(t) if i == k else t for i, t in enumerate(on)]
+        got = o.moe_combine(a, idx.to(DEV), wt.to(DEV), b, 4, c, sg.to(DEV)).double().cpu()
+        # a sum of 64 products through a sigmoid, five more products: a few hundred roundings of 2^-24
+        assert float((got - want).abs().max()) <= 300 * 2.0 ** -24 * float(want.abs().max())
+
+
 def test_moe_experts_of_views_that_begin_anywhere():
     """Rows and experts' matrices whose first element is no multiple of 16 bytes give the bits of copies that are,
     with the pairs grouped beforehand and not."""
