@@ -1029,7 +1029,11 @@ moe_combine_kernel(const void* __restrict__ h, int dt, const int32_t* __restrict
 
 // The same with V neighbouring columns a thread (16-byte loads from 16-byte addresses; E % V == 0, top <= MOE_COMBINE_TOP) and a
 // block a token: the gate's dot product is formed once a token, and all of a thread's rows are asked for
-// together (2,964 tokens of 2,048, 6 chosen: 200 -> 40 us; 8 tokens 10.5 -> 6.5).
+// together (2,964 tokens of 2,048, 6 chosen: 157 -> 25 us; 8 tokens 7.0 -> 5.0).  Up to MOE_COMBINE_FEW tokens a
+// block 256 V columns of a token, each with the gate's product for itself: tokens of 7,168, 8 chosen, one block
+// against several, by column first: 8 tokens 12.7, 14.4, 7.9 us; 128 tokens 37, 14.7, 9.4; 256 tokens in float32
+// 49, 17.8, 22.4.
+#define MOE_COMBINE_FEW 128
 template <int DT, int V>
 __global__ void __launch_bounds__(256)
 moe_combine_vec_kernel(const void* __restrict__ h, const int32_t* __restrict__ idx, const float* __restrict__ wt,
@@ -1049,7 +1053,7 @@ moe_combine_vec_kernel(const void* __restrict__ h, const int32_t* __restrict__ i
         d = block_sum(d, red);
         gate = 1.0f / (1.0f + expf(-d));
     }
-    for (int i = threadIdx.x * V; i < E; i += 256 * V) {
+    for (int i = (blockIdx.y * 256 + threadIdx.x) * V; i < E; i += gridDim.y * 256 * V) {
         float acc[V], hv[V], v[V];
         ldv<DT, V>(h, t * E + i, hv);
 #pragma unroll
@@ -1087,12 +1091,13 @@ extern "C" int illm_moe_combine(const void* h, int dt, const int32_t* idx, const
     if (T == 0) return ILLM_OK;
     const uintptr_t at = (uintptr_t)h | (uintptr_t)Y | (uintptr_t)shared | (uintptr_t)out;
     if (top <= MOE_COMBINE_TOP && E % (dt == ILLM_BF16 ? 8 : 4) == 0 && at % 16 == 0) {
+        const int V = dt == ILLM_BF16 ? 8 : 4, parts = T <= MOE_COMBINE_FEW ? (E + 256 * V - 1) / (256 * V) : 1;
         if (dt == ILLM_BF16)
-            hipLaunchKernelGGL((moe_combine_vec_kernel<ILLM_BF16, 8>), dim3(T), dim3(256), 0, (hipStream_t)stream, h, idx,
-                               wt, Y, shared, sg, sg_dt, out, E, top, NEr);
+            hipLaunchKernelGGL((moe_combine_vec_kernel<ILLM_BF16, 8>), dim3(T, parts), dim3(256), 0, (hipStream_t)stream, h,
+                               idx, wt, Y, shared, sg, sg_dt, out, E, top, NEr);
         else
-            hipLaunchKernelGGL((moe_combine_vec_kernel<ILLM_F32, 4>), dim3(T), dim3(256), 0, (hipStream_t)stream, h, idx,
-                               wt, Y, shared, sg, sg_dt, out, E, top, NEr);
+            hipLaunchKernelGGL((moe_combine_vec_kernel<ILLM_F32, 4>), dim3(T, parts), dim3(256), 0, (hipStream_t)stream, h,
+                               idx, wt, Y, shared, sg, sg_dt, out, E, top, NEr);
         return illm_launch_status();
     }
     hipLaunchKernelGGL(moe_combine_kernel, dim3(T, (E + 255) / 256), dim3(256), 0, (hipStream_t)stream,

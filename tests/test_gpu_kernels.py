@@ -624,6 +624,24 @@ def test_moe_tiles_of_128_pairs(T, E, F, NE, top, act):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("E", [1024, 1032, 2048, 2056, 4104])
+def test_moe_combine_of_wide_rows(E, dtype):
+    """Rows around a block's columns (1,024 in float32, 2,048 in bfloat16): with few tokens several blocks a token, the
+    same bits as among 129, where one block walks them all."""
+    o, T, top = ops(), 129, 3
+    h, y, sh = (rnd(n, E, dtype=dtype, seed=i).to(DEV) for i, n in enumerate((T, T * top, T)))
+    sg, g = rnd(E, seed=4).to(DEV), torch.Generator().manual_seed(5)
+    idx, wt = torch.randint(0, 5, (T, top), generator=g).to(torch.int32), torch.rand(T, top, generator=g)
+    every = o.moe_combine(h, idx.to(DEV), wt.to(DEV), y, 4, sh, sg)
+    some = o.moe_combine(h[:128], idx[:128].to(DEV), wt[:128].to(DEV), y[:128 * top], 4, sh[:128], sg)
+    assert torch.equal(some, every[:128])
+    d = lambda t: t.double().cpu()  # noqa: E731
+    rows = torch.where((idx < 4)[:, :, None], d(y).view(T, top, E), d(h)[:, None])
+    want = (rows * wt.double()[:, :, None]).sum(1) + torch.sigmoid(d(h) @ d(sg))[:, None] * d(sh)
+    assert float((d(every) - want).abs().max()) <= (E + 200) * 2.0 ** -24 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_moe_combine_of_views_that_begin_anywhere(dtype):
     """The weighted sum reads 16 bytes at a time only from addresses that are multiples of 16: views that begin
     elsewhere (by column, a gate's sum in another order) are as close to 64 bits."""
