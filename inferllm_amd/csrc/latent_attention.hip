@@ -558,10 +558,16 @@ extern "C" int illm_latent_attn_decode(const float* qa, const void* cache, int d
 // is two 8-byte loads from the transposed copy.  Keys that are not seen get weight 0 and their
 // loaded values are masked (a freed page may hold anything).  The sums stay in registers
 // (R / 16 accumulators of 4); statistics in float32.
+// Bound by trips to memory one after another.  Latents of more than 256 dims (RT 32) ask for a tile's first values
+// ahead of its keys and for U steps of 32 dims of keys together; U is 9 where 288 divides the key's dims and 6
+// elsewhere, so that no width goes a step at a time for long.  Narrower ones have few such trips and lose
+// more to the registers: keys and values in turn (walk alone, us: 512 + 64 dims, 1 sequence of 3,000 keys 17.5 -> 15.3,
+// 32 heads, 32 sequences of 1,000 to 2,000 63.5 -> 60.4; 192 + 64 in this order 9.4 and 31.2, with the values early 10.3
+// and 35.8).
 typedef __bf16 la_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float la_f32x4_t __attribute__((ext_vector_type(4)));
 
-template <int RT>
+template <int RT, int U>
 __global__ void __launch_bounds__(64)
 latent_decode_mfma_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restrict__ cache,
                           const bf16_t* __restrict__ cache_t,
@@ -579,6 +585,7 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restric
     const int per = (tile1 - tile0 + nsplit - 1) / nsplit;
     const int ta = tile0 + split * per;
     const int tb = ta + per < tile1 ? ta + per : tile1;
+    asm volatile("" ::"s"(slot));                    // (asked for with the length, not behind the branch)
     if (ta >= tb) {                                  // a range without keys: its sums are not read
         if (q == 0 && h0 + r < H) {
             float* dst = partial + (((size_t)b * H + h0 + r) * nsplit + split) * (size_t)(R + 4);
@@ -603,11 +610,9 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restric
         const bf16_t* kp0 = cache + ((size_t)phys * page_size + rowb + r) * D + 8 * q;
         const bf16_t* kp1 = kp0 + (size_t)16 * D;
         la_f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
-        // The tile's values are asked for with its keys: the first row groups before them, the rest
-        // before the softmax, so that a tile is a chain of three trips to memory instead of nine
-        // (8 sequences of 61 to 1,040 keys, 512 + 64 dims: 17.8 -> 14.1 us).
         const bf16_t* tp = cache_t + ((size_t)phys * R + r) * page_size + rowb + 4 * q;
-        constexpr int CH = RT < 16 ? RT : 16;        // row groups whose loads are in flight together
+        constexpr bool EARLY = RT > 16;
+        constexpr int CH = EARLY ? 16 : RT < 8 ? RT : 8;            // row groups whose loads are in flight together
         uint2 c0[CH], c1[CH];
         auto values = [&](int r0) __attribute__((always_inline)) {
 #pragma unroll
@@ -617,21 +622,23 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restric
                 c1[u] = *(const uint2*)(tp + (size_t)rt * 16 * page_size + 16);
             }
         };
-        values(0);
-        __builtin_amdgcn_sched_barrier(0);
-        // nine steps of 32 dims at a time: all their loads are asked for before the first product
+        if constexpr (EARLY) {
+            values(0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // U steps of 32 dims at a time: all their loads are asked for before the first product
         int d0 = 0;
-        for (; d0 + 288 <= D; d0 += 288) {
-            la_bf16x8_t qv[9], ka[9], kb[9];
+        for (; d0 + 32 * U <= D; d0 += 32 * U) {
+            la_bf16x8_t qv[U], ka[U], kb[U];
 #pragma unroll
-            for (int u = 0; u < 9; ++u) {
+            for (int u = 0; u < U; ++u) {
                 qv[u] = *(const la_bf16x8_t*)(qp + d0 + 32 * u);
                 ka[u] = *(const la_bf16x8_t*)(kp0 + d0 + 32 * u);
                 kb[u] = *(const la_bf16x8_t*)(kp1 + d0 + 32 * u);
             }
-            __builtin_amdgcn_sched_barrier(0);       // (else every product's loads are put right before it)
+            if constexpr (EARLY) __builtin_amdgcn_sched_barrier(0);  // (else every product's loads are put right before it)
 #pragma unroll
-            for (int u = 0; u < 9; ++u) {
+            for (int u = 0; u < U; ++u) {
                 s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[u], qv[u], s0, 0, 0, 0);
                 s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[u], qv[u], s1, 0, 0, 0);
             }
@@ -683,21 +690,26 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restric
         const uint32_t k67 = (ok[6] ? 0xffffu : 0u) | (ok[7] ? 0xffff0000u : 0u);
 #pragma unroll
         for (int r0 = 0; r0 < RT; r0 += CH) {
-            la_bf16x8_t cv[CH];
-#pragma unroll
-            for (int u = 0; u < CH; ++u) {
+            if constexpr (!EARLY) values(r0);
+            auto masked = [&](int u) __attribute__((always_inline)) {
                 uint4 cu;
                 cu.x = c0[u].x & k01; cu.y = c0[u].y & k23; cu.z = c1[u].x & k45; cu.w = c1[u].y & k67;
-                cv[u] = *(const la_bf16x8_t*)&cu;
+                return *(const la_bf16x8_t*)&cu;
+            };
+            la_bf16x8_t cv[EARLY ? CH : 1];          // (early: out of the way of the next groups' loads)
+            if constexpr (EARLY) {
+#pragma unroll
+                for (int u = 0; u < CH; ++u) cv[u] = masked(u);
+                if (r0 + CH < RT) values(r0 + CH);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            if (r0 + CH < RT) values(r0 + CH);
-            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int u = 0; u < CH; ++u) {
                 const int rt = r0 + u;
                 if (rt * 16 < R) {
+                    const la_bf16x8_t c = EARLY ? cv[EARLY ? u : 0] : masked(u);
                     o[rt][0] *= alpha; o[rt][1] *= alpha; o[rt][2] *= alpha; o[rt][3] *= alpha;
-                    o[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cv[u], pv, o[rt], 0, 0, 0);
+                    o[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, pv, o[rt], 0, 0, 0);
                 }
             }
         }
@@ -731,24 +743,27 @@ extern "C" int illm_latent_attn_decode_mfma(const void* qa, const void* cache, c
     if (groups > 65535) return ILLM_ERR_ARG;
     const dim3 grid(B, nsplit, groups);
     hipStream_t st = (hipStream_t)stream;
-#define GO(RT_)                                                                                   \
-    hipLaunchKernelGGL((latent_decode_mfma_kernel<RT_>), grid, dim3(64), 0, st,                    \
+#define GO(RT_, U_)                                                                               \
+    hipLaunchKernelGGL((latent_decode_mfma_kernel<RT_, U_>), grid, dim3(64), 0, st,                \
                        (const bf16_t*)qa, (const bf16_t*)cache, (const bf16_t*)cache_t, page_table, table_stride,     \
                        page_size, ring, seq_slot, seq_len, len_more, partial, nsplit, H, R, dr,    \
                        scale, window)
-    if (R <= 64) GO(4);
-    else if (R <= 128) GO(8);
-    else if (R <= 256) GO(16);
-    else GO(32);
+    if (R <= 64) GO(4, 6);
+    else if (R <= 128) GO(8, 6);
+    else if (R <= 256) GO(16, 6);
+    else if ((R + dr) % 288) GO(32, 6);
+    else GO(32, 9);
 #undef GO
     return illm_launch_status();
 }
 
 // grid (B, H, chunks of 32 value dims): combine the splits, multiply the combined latent sum by
 // W_uv's rows of the head (a wave a value dim, lanes over the latent dims) and by the head's
-// output gate.  Every chunk's block combines the splits for itself: those that hold keys (the ranges are
-// cut for the longest sequence), 16 bytes a lane, eight loads in flight (8 sequences of 61 to 1,040 keys in
-// 64 ranges: 17.1 -> 9.7 us with a thread a dim walking all of them).
+// output gate.  Every chunk's block combines the splits for itself, those up to the last that holds keys (the
+// ranges are cut for the longest sequence): a few by a thread a dim, more in 16-byte loads by all threads, eight
+// loads in flight either way, in an order that their number and R fix (512 dims: 63 ranges 10.5 -> 7.7 us with a
+// thread a dim walking all of them one by one, 16 of 64 sequences 28.4 -> 22.3; 128 dims: 64 ranges 7.5 -> 6.5, 4 ranges 5.9
+// -> 6.0, and 7.2 with the second pass through LDS).
 __global__ void __launch_bounds__(256)
 latent_merge_up_kernel(const float* __restrict__ partial, int nsplit, const void* __restrict__ wuv,
                        int w_dt, const void* __restrict__ y, int dt, int ncols, int gate_off,
@@ -761,26 +776,34 @@ latent_merge_up_kernel(const float* __restrict__ partial, int nsplit, const void
     const float* base = partial + ((size_t)b * H + h) * nsplit * (size_t)(R + 4);
     const int w = wave_index(), lane = threadIdx.x & 63;
     if (w == 0) {
-        // the ranges' (max, weight): lane s holds range s, s + 64, ...; weights exp(m_s - M) / total
-        float M = -INFINITY;
-        for (int s = lane; s < nsplit; s += 64) M = fmaxf(M, base[(size_t)s * (R + 4) + R]);
+        // the ranges' (max, sum), asked for together: lane s holds range s, s + 64, ...; weights exp(m_s - M) / total
+        auto at = [&](int s, int i, float none) __attribute__((always_inline)) {
+            return s < nsplit ? base[(size_t)s * (R + 4) + R + i] : none;
+        };
+        const float m0 = at(lane, 0, -INFINITY), l0 = at(lane, 1, 0.f);
+        float M = m0;
+        for (int s = lane + 64; s < nsplit; s += 64) M = fmaxf(M, at(s, 0, -INFINITY));
         M = wave_max(M);
-        float tot = 0.f;
+        float tot = 0.f, e0 = 0.f;
         int last = 0;
-        for (int s = lane; s < nsplit; s += 64) {
-            const float ms = base[(size_t)s * (R + 4) + R];
+        for (int s0 = 0; s0 < nsplit; s0 += 64) {
+            const float ms = s0 ? at(s0 + lane, 0, -INFINITY) : m0, ls = s0 ? at(s0 + lane, 1, 0.f) : l0;
             const float e = ms == -INFINITY ? 0.f : expf(ms - M);
-            ws[s] = e;
-            tot += ms == -INFINITY ? 0.f : base[(size_t)s * (R + 4) + R + 1] * e;
-            last = ms == -INFINITY ? last : s + 1;
+            tot += ls * e;
+            if (s0) { if (s0 + lane < nsplit) ws[s0 + lane] = e; }
+            else e0 = e;
+            const unsigned long long some = __ballot(ms != -INFINITY);
+            if (some) last = s0 + 64 - __clzll(some);
         }
-        for (int d = 32; d > 0; d >>= 1) last = max(last, __shfl_xor(last, d, 64));
-        if (lane == 0) filled = last;
         tot = wave_sum(tot);
-        for (int s = lane; s < nsplit; s += 64) ws[s] = ws[s] / tot;
+        if (lane == 0) filled = last;
+        if (lane < nsplit) ws[lane] = e0 / tot;
+        for (int s = lane + 64; s < nsplit; s += 64) ws[s] = ws[s] / tot;
     }
     __syncthreads();
-    if (R % 4 == 0 && R <= 1024 && (uintptr_t)partial % 16 == 0) {
+    // (few ranges, narrow latents: walking them costs less than the second pass through LDS)
+    const bool few = filled <= (R <= 256 ? 24 : 8);
+    if (!few && R % 4 == 0 && R <= 1024 && (uintptr_t)partial % 16 == 0) {
         // a thread takes four neighbouring dims of every `turns`-th range, eight loads in flight
         const int r4 = R / 4, turns = 256 / r4, at = threadIdx.x % r4, mine = threadIdx.x / r4;
         float* sums = ol + ((R + nsplit + 3) & ~3);    // [turns][R]
@@ -809,9 +832,16 @@ latent_merge_up_kernel(const float* __restrict__ partial, int nsplit, const void
             ol[r] = a;
         }
     } else {
+        // a thread a dim, range after range, eight loads in flight
         for (int r = threadIdx.x; r < R; r += 256) {
             float a = 0.f;
-            for (int s = 0; s < filled; ++s) a += base[(size_t)s * (R + 4) + r] * ws[s];
+            for (int s0 = 0; s0 < filled; s0 += 8) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = base[(size_t)min(s0 + u, filled - 1) * (R + 4) + r];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) a += s0 + u < filled ? v[u] * ws[s0 + u] : 0.f;
+            }
             ol[r] = a;
         }
     }

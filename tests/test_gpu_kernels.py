@@ -1550,3 +1550,33 @@ def test_capped_decode_ranges_and_rounds(nh, nkv, dk, dv, dtype):
             # float32: the scores' and sums' rounding; bfloat16: the result's (2^-9) and the exponential's
             tol = 1e-5 if dtype == torch.float32 else 2 ** -8
             assert float((got.double().cpu() - want).abs().max()) <= tol * max(1.0, float(want.abs().max())), (window, nsplit)
+
+
+@pytest.mark.parametrize("dtype, Rk, dr", [(torch.bfloat16, r, d) for r, d in ((16, 8), (64, 32), (128, 64), (208, 64), (256, 72), (320, 64),
+                                                                             (384, 192), (512, 32), (512, 64))] +
+                         [(torch.float32, 30, 8), (torch.float32, 64, 32), (torch.float32, 500, 12)])
+def test_latent_single_tokens_over_widths_and_ranges(dtype, Rk, dr, monkeypatch):
+    """Key widths on either side of the groups of 6 and 9 steps of 32 dims, the last step whole and in part; ranges
+    without keys (up to 63 of 64) whose sums nobody writes and nobody may read: the partial results begin as NaN; as few
+    and as many ranges as either way of combining them takes."""
+    o, g, H, dv, page = ops(), torch.Generator().manual_seed(Rk + dr), 3, 40, 64
+    lens = [1, 31, 33, 64, 300, 800, 1090]
+    B, per = len(lens), 18
+    table = torch.randperm(B * per, generator=g).view(B, per).to(torch.int32)
+    cache = torch.randn(B * per, page, Rk + dr, generator=g).to(dtype)
+    mfma = dtype == torch.bfloat16
+    ct = cache[:, :, :Rk].transpose(1, 2).contiguous().unsqueeze(-1) if mfma else None
+    qa = (torch.randn(B, H, Rk + dr, generator=g) * 0.3).to(dtype)
+    y, wuv = torch.randn(B, H + 2, generator=g).to(dtype), (torch.randn(H * dv, Rk, generator=g) * Rk ** -0.5).to(dtype)
+    slot, ln = torch.randperm(B, generator=g).to(torch.int32), torch.tensor(lens, dtype=torch.int32)
+    put = lambda t: t.to(DEV) if t is not None else None  # noqa: E731
+    want = R.latent_attn_decode(qa, y, wuv, 2, cache, table, page, 0, slot, ln, 0, H, dr, Rk, dv, 0.2, 0, 1).double()
+    args = (put(qa), put(y), put(wuv), 2, put(cache), put(table), page, 0, put(slot), put(ln), 0, H, dr, Rk, dv, 0.2, 0)
+    ct, real = put(ct), torch.empty
+    for nsplit in (1, 3, 8, 9, 16, 24, 25, 35, 64):
+        with monkeypatch.context() as m:
+            m.setattr(torch, "empty", lambda *a, **k: real(*a, **k).fill_(float("nan")))
+            got = o.latent_attn_decode(*args, nsplit, ct).double().cpu()
+        assert bool(torch.isfinite(got).all()), nsplit
+        # bfloat16: a weight's and a result's rounding (2^-9 each, 2^-8 beside the norm's share); float32 sums of up to 1,090
+        assert float((got - want).norm() / want.norm()) < (2 ** -7 if mfma else 2e-5), nsplit
