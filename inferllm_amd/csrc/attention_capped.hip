@@ -164,12 +164,12 @@ qkv_norm_mix_store_vec4_kernel(void* __restrict__ rows, int dt, int row_len, int
     for (int n = 0; n < NV; ++n) {
         const int i = threadIdx.x + 256 * n;
         const bool iq = qw && i < nq, ik = i < nk, iv = i < nv, ikw = kw && ik, il = lam && iv;
-        q[n] = ld_f4(rows, dt, iq ? base + i : base);
-        qg[n] = ld_f4(iq ? qw : rows, iq ? w_dt : dt, iq ? (size_t)i : base);
-        k[n] = ld_f4(rows, dt, ik ? base + k_at + i : base);
-        kg[n] = ld_f4(ikw ? kw : rows, ikw ? w_dt : dt, ikw ? (size_t)i : base);
-        v[n] = ld_f4(rows, dt, iv ? base + v_at + i : base);
-        f[n] = ld_f4(il ? first : rows, dt, il ? f_at + i : base);
+        q[n] = ld_f4_any(rows, dt, iq ? base + i : base);
+        qg[n] = ld_f4_any(iq ? qw : rows, iq ? w_dt : dt, iq ? (size_t)i : base);
+        k[n] = ld_f4_any(rows, dt, ik ? base + k_at + i : base);
+        kg[n] = ld_f4_any(ikw ? kw : rows, ikw ? w_dt : dt, ikw ? (size_t)i : base);
+        v[n] = ld_f4_any(rows, dt, iv ? base + v_at + i : base);
+        f[n] = ld_f4_any(il ? first : rows, dt, il ? f_at + i : base);
         if (!iq) q[n] = zero4;
         if (!ik) k[n] = zero4;
     }

@@ -51,9 +51,20 @@ __device__ __forceinline__ void st_f(void* p, int dt, size_t i, float v) {
     else ((float*)p)[i] = v;
 }
 
-// Four neighbouring elements (number 4 i4 .. 4 i4 + 3) as they lie in memory, without a branch on
-// the type: bfloat16 takes its 8 bytes twice.  A branch would hold the conversion, and with it the
-// wait for the load, so that loads that stand in a row would each take a trip to memory of their own.
+// four neighbouring elements (number 4 i4 .. 4 i4 + 3) as float32, and back (st_f4)
+__device__ __forceinline__ float4 ld_f4(const void* p, int dt, size_t i4) {
+    if (dt == ILLM_BF16) {
+        const uint2 u = ((const uint2*)p)[i4];
+        return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u),
+                           __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u));
+    }
+    return ((const float4*)p)[i4];
+}
+
+// The same as they lie in memory, without a branch on the type: bfloat16 takes its 8 bytes twice.  A branch
+// would hold the conversion, and with it the wait for the load, so that loads that stand in a row would each
+// take a trip to memory of their own.  (float32 takes two loads for one: where that is most of the traffic the
+// type belongs into the kernel.)
 struct AnyRaw4 {
     uint2 lo, hi;
 };
@@ -75,18 +86,20 @@ __device__ __forceinline__ float4 raw4_f(AnyRaw4 r, int dt) {
                        __uint_as_float(half ? r.lo.y & 0xffff0000u : r.hi.y));
 }
 
-// four neighbouring elements as float32, and back
-__device__ __forceinline__ float4 ld_f4(const void* p, int dt, size_t i4) { return raw4_f(ld_raw4(p, dt, i4), dt); }
+__device__ __forceinline__ float4 ld_f4_any(const void* p, int dt, size_t i4) { return raw4_f(ld_raw4(p, dt, i4), dt); }
 
 // Loads asked for before this stay before it: the compiler otherwise moves them into the branch that
 // uses them, behind a wait for other loads.
 __device__ __forceinline__ void loads_asked_for() { asm volatile("" ::: "memory"); }
 
 // ... or zeros where `on` is false, without a branch either: p's first four are then read, or `other`'s
-// (four float32) where p is null
+// (four float32) where p is null.  F32: p is known to be float32 when the kernel is compiled.
+template <bool F32 = false>
 __device__ __forceinline__ float4 ld_f4_if(const void* p, int dt, size_t i4, bool on, const float* other) {
     const bool there = p != nullptr;
-    const float4 v = ld_f4(there ? p : other, there ? dt : ILLM_F32, on && there ? i4 : 0);
+    const void* const from = there ? p : other;
+    const size_t at = on && there ? i4 : 0;
+    const float4 v = F32 ? ((const float4*)from)[at] : ld_f4_any(from, there ? dt : ILLM_F32, at);
     return on && there ? v : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 

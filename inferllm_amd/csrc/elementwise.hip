@@ -40,7 +40,7 @@ extern "C" int illm_embed(const int32_t* tokens, const void* table, int table_dt
 // The token's row under an RMS norm: out = v / sqrt(mean(v^2) + eps) * w with v = table[id] * scale.  `copy`
 // (null: none) takes the rows a second time.  grid (rows); 256 threads, NV groups of 4 columns a thread, the row
 // and the weights asked for together; NV 0: any width.
-template <int NV>
+template <int NV, bool F32>
 __global__ void __launch_bounds__(256)
 embed_norm_kernel(const int32_t* __restrict__ tokens, const void* __restrict__ table, int table_dt,
                   const void* __restrict__ w, int w_dt, float* __restrict__ out, float* __restrict__ copy, int E,
@@ -56,8 +56,8 @@ embed_norm_kernel(const int32_t* __restrict__ tokens, const void* __restrict__ t
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const size_t i = threadIdx.x + 256 * k;
-            v[k] = ld_f4_if(table, table_dt, src + i, i < n4, nullptr);
-            g[k] = ld_f4_if(w, w_dt, i, i < n4, nullptr);
+            v[k] = ld_f4_if<F32>(table, table_dt, src + i, i < n4, nullptr);
+            g[k] = ld_f4_if<F32>(w, w_dt, i, i < n4, nullptr);
         }
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
@@ -96,15 +96,18 @@ extern "C" int illm_embed_norm(const int32_t* tokens, const void* table, int tab
                                float* out, float* copy, int T, int E, int V, float scale, float eps, void* stream) {
     if (T < 0 || E <= 0 || V <= 0 || !illm_dtype_ok(table_dt) || !illm_dtype_ok(w_dt)) return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
-#define GO(NV_)                                                                                            \
-    hipLaunchKernelGGL(embed_norm_kernel<NV_>, dim3(T), dim3(256), 0, (hipStream_t)stream, tokens, table, table_dt, w, \
-                       w_dt, out, copy, E, V, scale, eps)
-    if (E % 4 || E > 8192) GO(0);
+#define GO_F(NV_, F32_)                                                                                    \
+    hipLaunchKernelGGL((embed_norm_kernel<NV_, F32_>), dim3(T), dim3(256), 0, (hipStream_t)stream, tokens, table, \
+                       table_dt, w, w_dt, out, copy, E, V, scale, eps)
+#define GO(NV_) do { if (f32) GO_F(NV_, true); else GO_F(NV_, false); } while (0)
+    const bool f32 = table_dt == ILLM_F32 && w_dt == ILLM_F32;
+    if (E % 4 || E > 8192) GO_F(0, false);
     else if (E <= 1024) GO(1);
     else if (E <= 2048) GO(2);
     else if (E <= 4096) GO(4);
     else GO(8);
 #undef GO
+#undef GO_F
     return illm_launch_status();
 }
 
@@ -162,12 +165,12 @@ embed_pairs_kernel(const int32_t* __restrict__ tokens, const int32_t* __restrict
         for (int k = 0; k < NV; ++k) {
             const size_t i = threadIdx.x + 256 * k;
             v[k] = ld_f4_if(table, table_dt, src / 4 + i, i < n4, nullptr);
-            q[k] = ld_f4(places ? places : table, places ? places_dt : table_dt, places && i < n4 ? pos * n4 + i : 0);
+            q[k] = ld_f4_any(places ? places : table, places ? places_dt : table_dt, places && i < n4 ? pos * n4 + i : 0);
         }
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const size_t i = threadIdx.x + 256 * k;
-            p[k] = ld_f4(pairs ? pairs : table, pairs ? pairs_dt : table_dt, pairs && i < n4 ? pair * n4 + i : 0);
+            p[k] = ld_f4_any(pairs ? pairs : table, pairs ? pairs_dt : table_dt, pairs && i < n4 ? pair * n4 + i : 0);
         }
         loads_asked_for();
 #pragma unroll

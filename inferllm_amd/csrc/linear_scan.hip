@@ -294,9 +294,9 @@ gla_prepare_vec4_kernel(const void* __restrict__ U, int dt, int u_stride, int q_
     const int g = blockIdx.y * 256 + threadIdx.x, nk4 = H * dk / 4, nv4 = H * dv / 4;
     const float qs = 1.0f / sqrtf((float)dk);
     const int gk = g < nk4 ? g : 0, gv = g < nv4 ? g : 0;
-    const float4 q = ld_f4(U, dt, (t * u_stride + q_off) / 4 + gk), k = ld_f4(U, dt, (t * u_stride + k_off) / 4 + gk);
-    const float4 z = ld_f4(Z, z_dt, t * z_stride / 4 + gk), b = ((const float4*)zb)[gk];
-    const float4 v = ld_f4(U, dt, (t * u_stride + v_off) / 4 + gv);
+    const float4 q = ld_f4_any(U, dt, (t * u_stride + q_off) / 4 + gk), k = ld_f4_any(U, dt, (t * u_stride + k_off) / 4 + gk);
+    const float4 z = ld_f4_any(Z, z_dt, t * z_stride / 4 + gk), b = ((const float4*)zb)[gk];
+    const float4 v = ld_f4_any(U, dt, (t * u_stride + v_off) / 4 + gv);
     loads_asked_for();
     if (g < nk4) {
         ((float4*)qn)[t * nk4 + g] = make_float4(q.x * qs, q.y * qs, q.z * qs, q.w * qs);

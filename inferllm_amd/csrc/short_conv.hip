@@ -58,7 +58,7 @@ short_conv_vec4_kernel(const void* __restrict__ X, int x_dt, int x_stride, int x
                                  : ((size_t)slot * K + (K - (back - n))) * (C / 4) + c4);
             cw[j] = ((const float4*)w)[(size_t)TAPS * c4 + j];
         }
-        const float4 b4 = ld_f4_if(bias, ILLM_F32, c4, true, w);
+        const float4 b4 = ld_f4_if<true>(bias, ILLM_F32, c4, true, w);
         loads_asked_for();
         y[0] = b4.x; y[1] = b4.y; y[2] = b4.z; y[3] = b4.w;
 #pragma unroll
@@ -341,7 +341,7 @@ extern "C" int illm_clamped_swish_mul(const void* gate_up, void* out, int dt, in
 // row's sum in LDS (E floats) between the passes.
 // Bound by trips to memory one after another: 8 rows of 2,048 columns with 3 taps take 4.8 us, and took
 // 9.3 us where the type of each load was a branch with its wait and the taps came one by one.
-template <int NV, int TAPS>
+template <int NV, int TAPS, bool F32>
 __global__ void __launch_bounds__(256)
 post_add_rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ a, int a_dt,
                         const void* __restrict__ post_w, int post_w_dt, float post_eps, float gain,
@@ -364,13 +364,13 @@ post_add_rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ a, int a
         for (int k = 0; k < NV; ++k) {
             const int i4 = threadIdx.x + 256 * k;
             const bool in = i4 < n4;
-            xv[k] = ld_f4_if(x, ILLM_F32, ib / 4 + i4, in, x);
-            av[k] = ld_f4_if(a, a_dt, ib / 4 + i4, in, x);
-            pwv[k] = ld_f4_if(a ? post_w : nullptr, post_w_dt, i4, in, x);
-            wv4[k] = ld_f4_if(w, w_dt, i4, in, x);
+            xv[k] = ld_f4_if<true>(x, ILLM_F32, ib / 4 + i4, in, x);
+            av[k] = ld_f4_if<F32>(a, a_dt, ib / 4 + i4, in, x);
+            pwv[k] = ld_f4_if<F32>(a ? post_w : nullptr, post_w_dt, i4, in, x);
+            wv4[k] = ld_f4_if<F32>(w, w_dt, i4, in, x);
             if (TAPS) {
 #pragma unroll
-                for (int j = 0; j < TAPS; ++j) cwv[k][j] = ld_f4_if(conv_w, ILLM_F32, (size_t)TAPS * i4 + j, in, x);
+                for (int j = 0; j < TAPS; ++j) cwv[k][j] = ld_f4_if<true>(conv_w, ILLM_F32, (size_t)TAPS * i4 + j, in, x);
             }
         }
         if (TAPS) {
@@ -379,7 +379,7 @@ post_add_rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ a, int a
                 const int i4 = threadIdx.x + 256 * k;
 #pragma unroll
                 for (int j = 0; j < TAPS - 1; ++j)
-                    oldv[k][j] = ld_f4_if(tail, tail_dt, ((size_t)slot * (TAPS - 1) + j) * n4 + i4, i4 < n4, x);
+                    oldv[k][j] = ld_f4_if<F32>(tail, tail_dt, ((size_t)slot * (TAPS - 1) + j) * n4 + i4, i4 < n4, x);
             }
         }
         loads_asked_for();
@@ -511,34 +511,38 @@ extern "C" int illm_post_add_rmsnorm(float* x, const void* a, int a_dt, const vo
         return ILLM_ERR_ARG;
     if (rows == 0) return ILLM_OK;
     hipStream_t st = (hipStream_t)stream;
-#define GO(NV_, TAPS_, LDS_)                                                                                 \
-    hipLaunchKernelGGL((post_add_rmsnorm_kernel<NV_, TAPS_>), dim3(rows), dim3(256), LDS_, st, x, a, a_dt, post_w, \
+#define GO_F(NV_, TAPS_, F_, LDS_)                                                                               \
+    hipLaunchKernelGGL((post_add_rmsnorm_kernel<NV_, TAPS_, F_>), dim3(rows), dim3(256), LDS_, st, x, a, a_dt, post_w, \
                        post_w_dt, post_eps, gain, w, w_dt, out, out_dt, row_idx, E, eps, conv_w, taps, tail,      \
                        tail_dt, row_slot)
+#define GO(NV_, TAPS_) do { if (f32) GO_F(NV_, TAPS_, true, 0); else GO_F(NV_, TAPS_, false, 0); } while (0)
     if (E % 4 == 0 && E <= 8192) {
+        const bool f32 = w_dt == ILLM_F32 && (!a || (a_dt == ILLM_F32 && post_w_dt == ILLM_F32)) &&
+                         (!conv_w || tail_dt == ILLM_F32);
         // (float4 reads of the taps want them 16-byte aligned)
         const int t = conv_w && E <= 4096 && (uintptr_t)conv_w % 16 == 0 ? taps : 0;
-#define GO_TAPS(NV_)                       \
-    do {                                   \
-        if (t == 2) GO(NV_, 2, 0);         \
-        else if (t == 3) GO(NV_, 3, 0);    \
-        else if (t == 4) GO(NV_, 4, 0);    \
-        else GO(NV_, 0, 0);                \
+#define GO_TAPS(NV_)                    \
+    do {                                \
+        if (t == 2) GO(NV_, 2);         \
+        else if (t == 3) GO(NV_, 3);    \
+        else if (t == 4) GO(NV_, 4);    \
+        else GO(NV_, 0);                \
     } while (0)
         if (E <= 1024) GO_TAPS(1);
         else if (E <= 2048) GO_TAPS(2);
         else if (E <= 4096) GO_TAPS(4);
-        else GO(8, 0, 0);
+        else GO(8, 0);
 #undef GO_TAPS
+#undef GO
         return illm_launch_status();
     }
     const size_t lds = (size_t)E * sizeof(float);
     if (lds > 64 * 1024) return ILLM_ERR_ARG;
     if (lds > 48 * 1024 &&
-        hipFuncSetAttribute((const void*)post_add_rmsnorm_kernel<0, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipFuncSetAttribute((const void*)post_add_rmsnorm_kernel<0, 0, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lds) != hipSuccess)
         return ILLM_ERR_LAUNCH;
-    GO(0, 0, lds);
-#undef GO
+    GO_F(0, 0, false, lds);
+#undef GO_F
     return illm_launch_status();
 }
