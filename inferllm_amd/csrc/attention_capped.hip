@@ -1123,17 +1123,18 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
         }
     auto round = [&](auto S, int base) __attribute__((always_inline)) {
         constexpr int s = S.value;
+        const bool valid = base + grp < k_hi;
         float kc[NK], vc[NV];
 #pragma unroll
         for (int j = 0; j < KQ; ++j)                // (columns beyond dk: nothing; values beyond dv are not stored)
             unit_floats(U * sub + 8 * U * j < dk ? kn[s][j] : illm_u32x4_t{0u, 0u, 0u, 0u}, &kc[U * j]);
 #pragma unroll
-        for (int j = 0; j < VQ; ++j) unit_floats(vn[s][j], &vc[U * j]);
+        for (int j = 0; j < VQ; ++j)                // (past the range: zeros, or its last row's infinities times 0 were NaN)
+            unit_floats(valid ? vn[s][j] : illm_u32x4_t{0u, 0u, 0u, 0u}, &vc[U * j]);
         // (without a branch, past the range its last row again: behind a branch the compiler can't count the
         // loads in flight, and waits for all of them)
         fetch(s, base + 32 * AHEAD, pages[s]);
         pages[s] = page_of(base + 64 * AHEAD);
-        const bool valid = base + grp < k_hi;
         const int kj = seen.at(base + grp);
 #pragma unroll
         for (int i = 0; i < DH; ++i) {

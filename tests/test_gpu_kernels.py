@@ -1580,3 +1580,25 @@ def test_latent_single_tokens_over_widths_and_ranges(dtype, Rk, dr, monkeypatch)
         assert bool(torch.isfinite(got).all()), nsplit
         # bfloat16: a weight's and a result's rounding (2^-9 each, 2^-8 beside the norm's share); float32 sums of up to 1,090
         assert float((got - want).norm() / want.norm()) < (2 ** -7 if mfma else 2e-5), nsplit
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dk, dv", [(128, 128), (64, 32)])
+def test_capped_decode_of_infinite_values(dk, dv, dtype):
+    """An infinity in the last key's value reaches its own dim as an infinity and no other: rounds of 32 keys that are
+    full, that end early, and whole rounds past the range."""
+    g, o, page, nh, nkv = torch.Generator().manual_seed(dk), ops(), 16, 4, 1
+    lens = [8, 31, 32, 33, 64, 96, 128]
+    B, per = len(lens), 8
+    table = torch.arange(B * per, dtype=torch.int32).view(B, per)
+    kc, vc = (torch.randn(B * per, nkv, page, d, generator=g).to(dtype) for d in (dk, dv))
+    for b, n in enumerate(lens):
+        vc[table[b, (n - 1) // page], 0, (n - 1) % page, 5] = float("inf")
+    q = torch.randn(B, nh * dk, generator=g).to(dtype)
+    put = lambda t: t.to(DEV)  # noqa: E731
+    for nsplit in (1, 2, 5):
+        got = o.attn_cap_decode(put(q), put(kc), put(vc), put(table), page, 0, put(torch.arange(B, dtype=torch.int32)),
+                                put(torch.tensor(lens, dtype=torch.int32)), nh, nkv, dk, dv, dk ** -0.5, 0.0, 0, nsplit)
+        got = got.float().cpu().view(B, nh, dv)
+        assert bool((got[:, :, 5] == float("inf")).all()), nsplit
+        assert bool(torch.isfinite(got[:, :, [d for d in range(dv) if d != 5]]).all()), nsplit
