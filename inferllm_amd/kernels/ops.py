@@ -1509,6 +1509,11 @@ MOE_TILES_FROM = 1.5     # pairs an expert on average from which the kernel with
                          # -> 252, 2,964 1,023 -> 608; the same bits)
 
 
+def _moe_few_rows(per_expert: float) -> int:
+    """Rows a tile of the matrix-core kernels that read what lies at any address."""
+    return 64 if per_expert >= 48 else 32 if per_expert >= 24 else 16
+
+
 def _moe_tiling(dtype: torch.dtype, E: int, F: int, NP: int, n_exp: int):
     """(on the matrix cores?, rows a tile, upper bound of tiles) for NP (token, choice) pairs."""
     # tiles of 128 rows from MOE_TILES_FROM pairs an expert on, as far as a load's 32-bit offset reaches;
@@ -1516,7 +1521,7 @@ def _moe_tiling(dtype: torch.dtype, E: int, F: int, NP: int, n_exp: int):
     # wave a column (float32, odd sizes)
     per_expert = NP / max(1, n_exp)
     mfma = dtype == torch.bfloat16 and E % 32 == 0 and F % 32 == 0 and per_expert >= MOE_MFMA_FROM
-    rows = (64 if per_expert >= 48 else 32 if per_expert >= 24 else 16) if mfma else _lib().illm_moe_tile_rows()
+    rows = _moe_few_rows(per_expert) if mfma else _lib().illm_moe_tile_rows()
     if mfma and per_expert >= MOE_TILES_FROM and E % 64 == 0 and F % 64 == 0 and 2 * NP * max(E, F) < 1 << 32 \
             and 4 * (max(E, F) + 128) * max(E, F) < 1 << 32:
         rows = 128
@@ -1529,7 +1534,7 @@ def _moe_group(idx: torch.Tensor, n_exp: int, dtype: torch.dtype, E: int, F: int
     NP = idx.numel()
     mfma, rows, max_tiles = _moe_tiling(dtype, E, F, NP, n_exp)
     if rows == 128 and not on16:
-        rows = 16
+        rows = _moe_few_rows(NP / max(1, n_exp))
         max_tiles = max(1, min(NP, NP // rows + n_exp))
     order = torch.empty((NP,), dtype=torch.int32, device=idx.device)
     tiles = torch.empty((3 * max_tiles + 1,), dtype=torch.int32, device=idx.device)

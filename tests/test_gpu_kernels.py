@@ -674,7 +674,7 @@ def test_moe_experts_of_views_that_begin_anywhere():
         v = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:].view(t.shape)
         return v.copy_(t)
     plan = o._moe_group(idx, NE, h.dtype, E, F)
-    assert plan[3] == 128
+    assert plan[3] == 128 and o._moe_group(idx, NE, h.dtype, E, F, False)[3] == 64
     for a, b, c in ((off(h), wu, wd), (h, off(wu), wd), (h, wu, off(wd))):
         assert torch.equal(o.moe_experts(a, idx, b, c), want)
         assert torch.equal(o.moe_experts(a, idx, b, c, plan), want)
