@@ -1502,11 +1502,35 @@ MOE_MFMA_FROM = 0        # (token, choice) pairs an expert on average from which
                          # K took 253 + 166 us for 64 tokens, bound by its sums across lanes)
 
 
-MOE_TILES_FROM = 1.5     # pairs an expert on average from which the kernel with both operands in LDS, in
-                         # tiles of 128 pairs, takes bfloat16 experts whose sizes are multiples of 64
-                         # (64 experts of 1408 x 2048, 6 a token, both products, us; tiles of 16 to 64
-                         # pairs -> of 128: 8 tokens 159 -> 164, 16 217 -> 206, 64 303 -> 236, 300 387
-                         # -> 252, 2,964 1,023 -> 608; the same bits)
+# Where the kernel with both operands in LDS, in tiles of 128 pairs, takes bfloat16 experts whose sizes are
+# multiples of 64.  It beats the smaller tiles from 24 pairs an expert on with every stack (their kernels for 32
+# and 64 pairs are the slow ones); with fewer pairs where the stack has blocks enough for the chip (columns of 64
+# and of 128) and a matrix is large enough for its pairs to be worth a block.  us, both products, tiles of 16 pairs -> of 128:
+#   experts        pairs an expert: 2           4           6           12          24
+#   64 of 1408 x 2048         226 -> 223  249 -> 238  295 -> 241  379 -> 244  350 -> 253
+#   32 of 4096 x 2048         427 -> 364  414 -> 360  461 -> 379  532 -> 382  551 -> 393
+#   8 of 14336 x 4096         526 -> 576  758 -> 632  788 -> 634  830 -> 636  816 -> 645
+#   8 of 8192 x 4096          342 -> 406  364 -> 386  369 -> 387  405 -> 389  603 -> 394
+#   24 of 1536 x 1536          82 ->  99   86 -> 101   90 -> 101  122 -> 102  134 -> 106
+#   128 of 768 x 2048         226 -> 257  239 -> 265  315 -> 274  382 -> 282  360 -> 300
+#   256 of 256 x 1024          81 -> 118   89 -> 126   98 -> 129  117 -> 137  176 -> 153
+#   16 of 512 x 512            18 ->  22   18 ->  22   18 ->  22   20 ->  25   50 ->  27
+#   8 of 2048 x 1024           40 ->  58   41 ->  58   43 ->  58   48 ->  59  109 ->  61
+#   2 of 4096 x 4096           65 -> 131   67 -> 131   71 -> 131   79 -> 131  274 -> 133
+# (2,964 tokens of the first, 6 chosen: 1,023 -> 608.)  The same bits.
+MOE_TILES_ALWAYS = 24              # pairs an expert on average
+MOE_TILES_BLOCKS = (256, 512)      # blocks of the thinner product: none with fewer than the first, from 12 pairs an
+                                   # expert on with fewer than the second, from 1.5 on with more
+MOE_TILES_WORK = 1 << 23           # pairs an expert times its F E
+
+
+def _moe_tiles_pay(E: int, F: int, NP: int, n_exp: int) -> bool:
+    per_expert = NP / max(1, n_exp)
+    if per_expert >= MOE_TILES_ALWAYS:
+        return True
+    blocks = n_exp * min(F // 64, (E + 127) // 128)
+    return (blocks >= MOE_TILES_BLOCKS[0] and per_expert >= (12 if blocks < MOE_TILES_BLOCKS[1] else 1.5)
+            and per_expert * F * E >= MOE_TILES_WORK)
 
 
 def _moe_few_rows(per_expert: float) -> int:
@@ -1516,13 +1540,12 @@ def _moe_few_rows(per_expert: float) -> int:
 
 def _moe_tiling(dtype: torch.dtype, E: int, F: int, NP: int, n_exp: int):
     """(on the matrix cores?, rows a tile, upper bound of tiles) for NP (token, choice) pairs."""
-    # tiles of 128 rows from MOE_TILES_FROM pairs an expert on, as far as a load's 32-bit offset reaches;
-    # other sizes: up to 64 rows; few pairs (single tokens): 16 rows on the matrix cores, or 8 rows with a
-    # wave a column (float32, odd sizes)
+    # tiles of 128 rows where they pay, as far as a load's 32-bit offset reaches; else up to 64 rows; few pairs
+    # (single tokens): 16 rows on the matrix cores, or 8 rows with a wave a column (float32, odd sizes)
     per_expert = NP / max(1, n_exp)
     mfma = dtype == torch.bfloat16 and E % 32 == 0 and F % 32 == 0 and per_expert >= MOE_MFMA_FROM
     rows = _moe_few_rows(per_expert) if mfma else _lib().illm_moe_tile_rows()
-    if mfma and per_expert >= MOE_TILES_FROM and E % 64 == 0 and F % 64 == 0 and 2 * NP * max(E, F) < 1 << 32 \
+    if mfma and _moe_tiles_pay(E, F, NP, n_exp) and E % 64 == 0 and F % 64 == 0 and 2 * NP * max(E, F) < 1 << 32 \
             and 4 * (max(E, F) + 128) * max(E, F) < 1 << 32:
         rows = 128
     return mfma, rows, max(1, min(NP, NP // rows + n_exp))

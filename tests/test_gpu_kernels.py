@@ -620,7 +620,7 @@ def test_moe_tiles_of_128_pairs(T, E, F, NE, top, act):
     finally:
         o._moe_tiling = real
     assert torch.equal(got[0], got[1]) and bool(torch.isfinite(got[1].float()).all())
-    assert real(torch.bfloat16, E, F, 2 * NE, NE)[1] == 128 and real(torch.bfloat16, E, F + 32, 2 * NE, NE)[1] != 128
+    assert real(torch.bfloat16, E, F, 24 * NE, NE)[1] == 128 and real(torch.bfloat16, E, F + 32, 24 * NE, NE)[1] != 128
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
