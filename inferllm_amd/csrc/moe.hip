@@ -267,8 +267,9 @@ moe_route_row(const float* zr, const void* __restrict__ corr, int corr_dt, int N
     }
     // Up to 64 outputs, all choice scores finite: an output's place is the number of outputs ahead of it
     // (a larger score, or the same and a lower index), counted in one pass over the lanes instead of
-    // `top` searches of 12 exchanges each (64 outputs, 6 chosen: 9.0 -> 4.6 us).
-    if (NE <= 64 && groups == 0 && __all(lane >= NE || fabsf(c[0]) < INFINITY)) {
+    // `top` searches of 12 exchanges each (64 outputs, 6 chosen: 9.0 -> 4.6 us).  A search costs as much as
+    // counting some 20 outputs: of 64 outputs 1 or 2 chosen take 3.8 and 4.6 us by searches, 5.5 by counting.
+    if (NE <= 64 && NE <= 20 * top && groups == 0 && __all(lane >= NE || fabsf(c[0]) < INFINITY)) {
         int place = 0;
         for (int j = 0; j < NE; ++j) {
             const float o = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c[0]), j));

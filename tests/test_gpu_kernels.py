@@ -709,11 +709,11 @@ def test_moe_route_places():
     o = ops()
     for NE in (1, 5, 64, 65):
         z = (rnd(50, NE, seed=4) * 2).round().div(2).to(DEV)                 # many equal scores
-        top = min(6, NE)
-        idx, wt = o.moe_route(z, None, top)
         want = torch.sort(torch.softmax(z.double().cpu(), -1).float(), dim=-1, descending=True, stable=True)
-        assert torch.equal(idx.long().cpu(), want.indices[:, :top])
-        torch.testing.assert_close(wt.cpu(), want.values[:, :top], atol=0, rtol=1e-5)
+        for top in sorted({1, min(3, NE), min(4, NE), min(6, NE)}):          # (3 of 64: searches, 4: places)
+            idx, wt = o.moe_route(z, None, top)
+            assert torch.equal(idx.long().cpu(), want.indices[:, :top])
+            torch.testing.assert_close(wt.cpu(), want.values[:, :top], atol=0, rtol=1e-5)
 
 
 @pytest.mark.parametrize("rule", ["plain", "delta", "bonus", "removal"])
