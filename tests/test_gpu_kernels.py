@@ -1453,10 +1453,12 @@ def test_passes_of_single_tokens_over_widths_and_taps(E, dtype):
 @pytest.mark.parametrize("nh, nkv, dk, dv, weights, mix", [(2, 1, 4, 8, True, True), (16, 4, 64, 64, True, False),
                                                            (8, 2, 132, 128, False, True), (4, 4, 256, 260, True, True),
                                                            (32, 8, 128, 128, True, True), (33, 1, 128, 64, True, True),
-                                                           (4, 2, 128, 128, False, False)])
+                                                           (4, 2, 128, 128, False, False), (16, 4, 128, 128, False, True),
+                                                           (3, 1, 32, 16, False, True), (2, 1, 248, 252, False, True), (2, 1, 252, 256, False, True),
+                                                           (40, 8, 128, 128, False, True)])
 def test_norm_mix_and_store_four_columns_a_load(nh, nkv, dk, dv, weights, mix, dtype):
-    """Widths around a thread's share (1,024, 2,048 and 4,096 columns; 4,224 takes the loop by column), with and
-    without the norm and the mix of values, into a cache with a ring and into none."""
+    """Widths around a thread's share (1,024, 2,048 and 4,096 columns; 4,224 takes the loop by column, and below 256
+    without the norm), with and without the norm and the mix of values, into a cache with a ring and into none."""
     g = torch.Generator().manual_seed(nh * dk + dv)
     o, page, pages, ring = ops(), 16, 6, 2
     # float32: one rounding a step and a sum of up to 4,224 squares; bfloat16: the result's rounding (2^-8)
