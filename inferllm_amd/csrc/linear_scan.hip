@@ -319,8 +319,9 @@ extern "C" int illm_gla_prepare(const void* U, int dt, int u_stride, int q_off, 
         return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
     const int widest = H * dk > H * dv ? H * dk : H * dv;
-    // (dv >= 4: a row's H weights are within its groups of four)
-    if (((H * dk) | (H * dv) | q_off | k_off | v_off | u_stride | z_stride) % 4 == 0 && widest / 4 >= H &&
+    // Rows of at most 256 columns are one turn of a block's threads a column each: 4 heads of 64 take 3.0 us that way
+    // and 3.4 by groups of four.  (dv >= 4: a row's H weights are within its groups of four.)
+    if (widest > 256 && ((H * dk) | (H * dv) | q_off | k_off | v_off | u_stride | z_stride) % 4 == 0 && widest / 4 >= H &&
         (widest / 4 + 255) / 256 <= 65535 &&
         ((uintptr_t)U | (uintptr_t)Z | (uintptr_t)zb | (uintptr_t)qn | (uintptr_t)kn | (uintptr_t)vv | (uintptr_t)dec) % 16 == 0) {
         hipLaunchKernelGGL(gla_prepare_vec4_kernel, dim3(T, (widest / 4 + 255) / 256), dim3(256), 0, (hipStream_t)stream,

@@ -1517,7 +1517,8 @@ def test_recurrent_gates_of_a_row_alone_and_among_others(nb, cb):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("H, dk, dv", [(4, 256, 128), (1, 4, 4), (8, 132, 264), (16, 64, 64), (5, 12, 2)])
+@pytest.mark.parametrize("H, dk, dv", [(4, 256, 128), (1, 4, 4), (8, 132, 264), (16, 64, 64), (5, 12, 2), (4, 64, 64), (2, 64, 128),
+                                       (2, 130, 64)])
 def test_gated_linear_attention_rows_four_columns_a_load(H, dk, dv, dtype):
     g = torch.Generator().manual_seed(H * dk)
     for off in (0, 1):                                  # (an odd offset takes the loop by column)
