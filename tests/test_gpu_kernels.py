@@ -1555,6 +1555,33 @@ def test_capped_decode_ranges_and_rounds(nh, nkv, dk, dv, dtype):
             assert float((got.double().cpu() - want).abs().max()) <= tol * max(1.0, float(want.abs().max())), (window, nsplit)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dk, dv", [(128, 128), (64, 32), (40, 200)])
+def test_capped_decode_of_ranges_without_keys(dk, dv, dtype, monkeypatch):
+    """Ragged lengths, so that up to 32 of 33 ranges hold no key; nobody writes such a range's values and nobody may
+    read them: the partial results begin as NaN.  As many ranges as the merge takes at once (16), one more and fewer."""
+    g, o, page, nh, nkv = torch.Generator().manual_seed(dv), ops(), 16, 6, 2
+    lens = [1, 31, 64, 65, 300, 1056]
+    B, per = len(lens), 66
+    table = torch.randperm(B * per, generator=g).view(B, per).to(torch.int32)
+    kc, vc = (torch.randn(B * per, nkv, page, d, generator=g).to(dtype) for d in (dk, dv))
+    q, slots = torch.randn(B, nh * dk, generator=g).to(dtype), torch.randperm(B, generator=g).to(torch.int32)
+    seq_len, sink = torch.tensor(lens, dtype=torch.int32), torch.randn(nh, generator=g)
+    put = lambda t: t.to(DEV) if t is not None else None  # noqa: E731
+    args, real = (nh, nkv, dk, dv, dk ** -0.5, 0.0, 0), torch.empty
+    on = [put(t) for t in (q, kc, vc, table)]
+    slots_d, len_d = put(slots), put(seq_len)
+    for sk in (None, sink):
+        want = R.attn_cap_decode(q, kc, vc, table, page, 0, slots, seq_len, *args, 1, sink=sk).double()
+        for nsplit in (2, 15, 16, 17, 33):
+            with monkeypatch.context() as m:
+                m.setattr(torch, "empty", lambda *a, **k: real(*a, **k).fill_(float("nan")))
+                got = o.attn_cap_decode(*on, page, 0, slots_d, len_d, *args, nsplit, sink=put(sk)).double().cpu()
+            assert bool(torch.isfinite(got).all()), nsplit
+            tol = 1e-5 if dtype == torch.float32 else 2 ** -8     # (as for the ranges and rounds above)
+            assert float((got - want).abs().max()) <= tol * max(1.0, float(want.abs().max())), nsplit
+
+
 @pytest.mark.parametrize("dtype, Rk, dr", [(torch.bfloat16, r, d) for r, d in ((16, 8), (64, 32), (128, 64), (208, 64), (256, 72), (320, 64),
                                                                              (384, 192), (512, 32), (512, 64))] +
                          [(torch.float32, 30, 8), (torch.float32, 64, 32), (torch.float32, 500, 12)])

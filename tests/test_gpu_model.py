@@ -96,6 +96,31 @@ def test_short_prompts_at_head_size_128(tmp_path_factory, copies):
         eng.free_slot(s)
 
 
+@pytest.mark.parametrize("lens", [[129], [100, 60], [192], [193], [7, 249]])
+def test_steps_of_129_to_256_rows(tmp_path_factory, monkeypatch, lens):
+    """Steps of 129 to 256 rows whose o and down matrices are thin (256 x 4096): K cut over the blocks, the planes added
+    by the next norm, in both layers; one prompt and two, at the edges of the two tile heights."""
+    from inferllm_amd import StepEntry
+    from inferllm_amd.kernels import ops
+    calls = []
+    real = ops.linear_cut
+    monkeypatch.setattr(ops, "linear_cut", lambda x, w, *a: calls.append(x.shape[0]) or real(x, w, *a))
+    monkeypatch.setitem(CONFIGS, "cut", dict(CONFIGS["D"], num_attention_heads=32, num_key_value_heads=8,
+                                             intermediate_size=4096, vocab_size=300))
+    eng, plain, config = setup(tmp_path_factory, "cut", "bfloat16")
+    reqs = requests_for(config, lens, seed=4)
+    slots = [eng.alloc_slot() for _ in reqs]
+    got = eng.step([StepEntry(s, r, list(range(len(r)))) for s, r in zip(slots, reqs)]).clone()
+    assert calls == [sum(lens)] * 4, calls
+    at = 0
+    for r in reqs:
+        assert err(got[at:at + len(r)], plain(r)) < BUDGET["bfloat16"], len(r)
+        at += len(r)
+    for s in slots:
+        eng.free_slot(s)
+    eng.cache.check()
+
+
 def test_steps_of_17_to_64_rows(tmp_path_factory, monkeypatch):
     """Steps of 17 to 128 rows (here 24 to 64: a prompt of that length, or that many sequences decoding) read the
     decode copy of the down projection with K cut into ranges, whose planes the next norm adds
