@@ -198,8 +198,8 @@ gemm_f32_mfma_kernel(const float* __restrict__ X, const float* __restrict__ W, v
     // other (stages past the end are zeros).  T = 64: a chunk's operands are read while the chunk
     // before it is multiplied, the next stage's first ones too: its writes and the barrier stand
     // before this stage's last products, so that a block alone on its compute unit goes on (256 rows,
-    // 12288 x 4096: 243 -> 226 us).  T = 128: the other block of the compute unit fills the gap, and
-    // the order by stages is the faster one (2,048 rows of 4096 x 11008: 1,345 against 1,474 us).
+    // 12288 x 4096: 260 -> 249 us, 4096 x 11008: 227 -> 217).  T = 128: the other block of the compute unit
+    // fills the gap, and the order by stages is as fast (2,048 rows of 4096 x 11008: 1,422 us, 1,431 so).
     auto turn = [&](Set& next, Set& after, int st) __attribute__((always_inline)) {
         fetch(after, st + 2);
         if constexpr (T == 64) {
