@@ -12,8 +12,8 @@ extern "C" {
 // The sums are the same bits either way.
 void illm_set_rows_f32_tiles(int tiles);
 
-// illm_gemm_f32_mfma: outputs of a block along each side, 64 or 128 (0: the library's choice).  The
-// sums are the same bits either way.
+// illm_gemm_f32_mfma: outputs of a block along each side, 64 or 128, or 16 for the kernel of short K (stages of
+// 16 k, blocks of 128 x 128; 0: the library's choice).  The sums are the same bits either way.
 void illm_set_f32_tile(int t);
 
 // Whether float32 prompts with head sizes 32, 64, 96 and 128 take the attention kernel on the

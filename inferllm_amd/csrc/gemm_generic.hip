@@ -231,10 +231,11 @@ gemm_f32_mfma_kernel(const float* __restrict__ X, const float* __restrict__ W, v
         }
     };
     if constexpr (T == 64) operands(o0, 0, 0);
-    for (int st = 0; st < stages; st += 2) {
+    for (int st = 0; st + 1 < stages; st += 2) {
         turn(g1, g0, st);
         turn(g0, g1, st + 1);
     }
+    if (stages & 1) turn(g1, g0, stages - 1);
     // acc[i][j][v]: n = n0 + wn * T/2 + 32 i + 8 (v / 4) + 4 kh + v % 4, m = m0 + wm * T/2 + 32 j + r
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
@@ -258,8 +259,109 @@ gemm_f32_mfma_kernel(const float* __restrict__ X, const float* __restrict__ W, v
     }
 }
 
+// The same for short K, where the kernel above has more stages in flight than there are: blocks of 128 x 128,
+// stages of 16 k, one ahead, operands k-major in LDS (33 KB, so that four blocks share a compute unit and
+// their stores of Y, which is what counts here, overlap).  4,096 rows of 4096 x 16 19 us, and 46 (35 in blocks of 64 x 64)
+// above; 2,048 rows of 2048 x 16 9.2 and 13.5.  The same pairs of k in the same order: the same bits.
+#define FS_T 128     // outputs of a block along m and along n
+#define FS_K 16      // k a stage
+#define FS_LD 130    // LDS row stride in floats (4 * FS_LD = 8 mod 32: the stores of a half-wave,
+                     // 8 rows x 4 k-quads, fall into 32 different banks)
+
+__global__ void __launch_bounds__(256)
+gemm_f32_short_kernel(const float* __restrict__ X, const float* __restrict__ W, void* __restrict__ Y,
+                     int y_dt, int M, int N, int K) {
+    __shared__ float xs[2][FS_K][FS_LD];
+    __shared__ float ws[2][FS_K][FS_LD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
+    const int r = lane & 31, kh = lane >> 5;
+    const int wm = wave & 1, wn = wave >> 1;
+    const int m0 = blockIdx.y * FS_T, n0 = blockIdx.x * FS_T;
+
+    // staging: thread t brings 4 k (quad t % 4) of rows t / 4 and t / 4 + 64 of both operands;
+    // rows beyond the matrix read its last row (their outputs are not stored)
+    const int s_row = tid >> 2, s_kq = tid & 3;
+    const float* xsrc[2];
+    const float* wsrc[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        xsrc[e] = X + (size_t)min(m0 + s_row + 64 * e, M - 1) * K + s_kq * 4;
+        wsrc[e] = W + (size_t)min(n0 + s_row + 64 * e, N - 1) * K + s_kq * 4;
+    }
+    float4 xg[2], wg[2];
+    auto fetch = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            xg[e] = *(const float4*)(xsrc[e] + k0);
+            wg[e] = *(const float4*)(wsrc[e] + k0);
+        }
+    };
+    auto stage = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int row = s_row + 64 * e;
+            xs[buf][s_kq * 4 + 0][row] = xg[e].x; xs[buf][s_kq * 4 + 1][row] = xg[e].y;
+            xs[buf][s_kq * 4 + 2][row] = xg[e].z; xs[buf][s_kq * 4 + 3][row] = xg[e].w;
+            ws[buf][s_kq * 4 + 0][row] = wg[e].x; ws[buf][s_kq * 4 + 1][row] = wg[e].y;
+            ws[buf][s_kq * 4 + 2][row] = wg[e].z; ws[buf][s_kq * 4 + 3][row] = wg[e].w;
+        }
+    };
+    f32x16_t acc[2][2];                    // [n tile][m tile]
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+    fetch(0);
+    stage(0);
+    __syncthreads();
+    int buf = 0;
+    for (int k0 = 0; k0 < K; k0 += FS_K, buf ^= 1) {
+        const bool more = k0 + FS_K < K;
+        if (more) fetch(k0 + FS_K);
+#pragma unroll
+        for (int s = 0; s < FS_K / 2; ++s) {
+            float a[2], b[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) a[i] = ws[buf][2 * s + kh][wn * 64 + 32 * i + r];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) b[j] = xs[buf][2 * s + kh][wm * 64 + 32 * j + r];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        if (more) stage(buf ^ 1);          // (last read before the barrier that ended the stage before)
+        __syncthreads();
+    }
+    // acc[i][j][v]: n = n0 + wn * 64 + 32 i + 8 (v / 4) + 4 kh + v % 4, m = m0 + wm * 64 + 32 j + r
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int m = m0 + wm * 64 + 32 * j + r;
+        if (m >= M) continue;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int n = n0 + wn * 64 + 32 * i + 8 * g + 4 * kh;
+                const size_t at = (size_t)m * N + n;
+                if (n + 3 < N && (N & 3) == 0 && y_dt == ILLM_F32) {
+                    *(float4*)((float*)Y + at) = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1],
+                                                             acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (n + v < N) st_f(Y, y_dt, at + v, acc[i][j][4 * g + v]);
+                }
+            }
+    }
+}
+
 static int g_f32_tile = 0;
-extern "C" void illm_set_f32_tile(int t) { g_f32_tile = t == 64 || t == 128 ? t : 0; }
+extern "C" void illm_set_f32_tile(int t) { g_f32_tile = t == 16 || t == 64 || t == 128 ? t : 0; }
 
 // A kernel that needs more dynamic LDS than it may have without asking: asked for once per device.
 template <int T>
@@ -299,13 +401,25 @@ extern "C" int illm_gemm_f32_mfma(const float* X, const float* W, void* Y, int y
     if (m128 > 65535) return ILLM_ERR_ARG;
     if (K >= 1 << 22)                      // a block's rows would pass 2 GiB
         return illm_gemm_generic(X, ILLM_F32, W, ILLM_F32, Y, y_dt, M, N, K, stream);
+    // Short K: writing Y is what counts.  The kernel for it from 512 of its blocks on, unless they are rows and columns
+    // beyond the matrix for more than a tenth (then up to K = 112), else blocks of 64 x 64.  us in that kernel / in blocks of
+    // 64 x 64 / of 128 x 128: 4,096 rows of 4096 x 16 19 / 32 / 49, x 96 41 / 46 / 47, x 320 108 / 122 / 109;
+    // 4,096 of 2048 x 48 18 / 20 / 22; 300 of 32000 x 48 20 / 24 / 32, x 160 46 / 41 / 49; 2,048 of 2048 x 32 11 / 9 / 11,
+    // x 128 19 / 17 / 19, x 320 35 / 33 / 34 (x 512 - / 51 / 48).
+    const bool few_k = K <= 320;
+    const bool is_short = g_f32_tile ? g_f32_tile == 16 : few_k && b128 >= 512 && (K <= 112 || 10 * b64 >= 36 * b128);
+    if (is_short) {
+        hipLaunchKernelGGL(gemm_f32_short_kernel, dim3((N + FS_T - 1) / FS_T, (unsigned)m128), dim3(256), 0, (hipStream_t)stream,
+                           X, W, Y, y_dt, M, N, K);
+        return illm_launch_status();
+    }
     // Blocks of 128 x 128 finish in rounds of one a compute unit (256 blocks of K = 4,096: 280 us, 512
     // 535, 768 800), those of 64 x 64 in rounds of a quarter of that at 0.9 of the rate (256 91 us, 512
     // 157, 1,024 300): the larger ones where their rounds are nearly full.  Measured at 129 to 2,048
     // rows of the 7B shapes; with 128 x 128 alone, stages of 16 k and one stage ahead, 256 rows took
     // 314 us (4096 x 4096), 318 (12288 x 4096), 829 (4096 x 11008) and 545 (22016 x 4096), now 91, 236,
     // 249 and 438; 2,048 rows 562, 1,584, 1,447 and 2,973, now 540, 1,585, 1,428 and 2,894.
-    const bool big = g_f32_tile ? g_f32_tile == 128 : 10 * 1024 * ((b128 + 255) / 256) <= 11 * b64;
+    const bool big = g_f32_tile ? g_f32_tile == 128 : !few_k && 10 * 1024 * ((b128 + 255) / 256) <= 11 * b64;
     return big ? launch_f32_mfma<128>(X, W, Y, y_dt, M, N, K, (hipStream_t)stream)
                : launch_f32_mfma<64>(X, W, Y, y_dt, M, N, K, (hipStream_t)stream);
 }

@@ -562,8 +562,8 @@ def test_gemm_f32_mfma(ydt, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(1, 1, 16), (64, 64, 32), (65, 129, 48), (129, 64, 64), (192, 520, 80), (130, 1030, 112),
                                    (257, 65, 4096)])
 def test_gemm_f32_mfma_tiles(M, N, K):
-    """Both block sizes of the many-row float32 product give the same bits, at edges of their tiles, of
-    a stage of 32 k and of the eight column tiles that go round the chip; against 64 bits within
+    """Both block sizes of the many-row float32 product and its kernel of short K (16) give the same bits, at edges of
+    their tiles, of a stage of 32 k and of the eight column tiles that go round the chip; against 64 bits within
     sums of K products in any order (each within K 2^-24 of the sum of their magnitudes)."""
     x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
     want = x.double() @ w.double().t()
@@ -571,12 +571,12 @@ def test_gemm_f32_mfma_tiles(M, N, K):
     got = []
     lib = ops()._lib()
     try:
-        for tile in (64, 128):
+        for tile in (16, 64, 128):
             lib.illm_set_f32_tile(tile)
             got.append(ops().gemm_f32_mfma(x.to(DEV), w.to(DEV), torch.float32))
     finally:
         lib.illm_set_f32_tile(0)
-    assert torch.equal(got[0], got[1])
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
     assert bool(((got[0].double().cpu() - want).abs() <= room).all())
 
 
