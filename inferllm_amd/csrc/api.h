@@ -107,6 +107,17 @@ int illm_gemm_generic(const void* X, int x_dt, const void* W, int w_dt, void* Y,
 int illm_gemm_f32_mfma(const float* X, const float* W, void* Y, int y_dt, int M, int N, int K,
                        void* stream);
 
+// The same product for float32 X and W with K % 32 == 0 on the matrix cores' bfloat16 instruction:
+// operands as the sum of three bfloat16 parts, six products of parts (csrc/gemm_f32_split.hip).  P: scratch of
+// 6 K illm_gemm_f32_split_rows(M) bytes.  splits 1: Y [M, N] in y_dt; more: float32 planes [splits][M][N] of parts of K
+// (illm_gemm_f32_split_parts, or any number that leaves no part empty).  All on 16-byte addresses.
+int illm_gemm_f32_split_rows(int M);
+int illm_gemm_f32_split_parts(int M, int N, int K);
+int illm_gemm_f32_split(const float* X, const float* W, void* P, size_t p_bytes, void* Y, int y_dt, int M, int N,
+                        int K, int splits, void* stream);
+// Y [n] (n % 4 == 0) in y_dt = the sum of float32 planes [S][n], in order.
+int illm_f32_planes_sum(const float* planes, void* Y, int y_dt, int S, size_t n, void* stream);
+
 // Products of up to 256 bfloat16 rows from row-major W, K % 64 == 0, N % 4 == 0 (csrc/gemm_tiles.hip): K
 // cut into `splits` parts (illm_gemm_tiles_splits(N, K), or any number that leaves no part empty) as
 // float32 planes [splits][M][N].  X, W and Y on 16-byte addresses.

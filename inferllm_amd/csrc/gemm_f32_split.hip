@@ -1,0 +1,327 @@
+// Y[M, N] = X[M, K] . W[N, K]^T, float32 throughout, by the matrix cores' bfloat16 instruction.
+//
+// A float32 number is the sum of three bfloat16 numbers exactly (8 bits of mantissa each, rounded to nearest
+// so that the rest is what the next one holds): x = x1 + x2 + x3, |x2| <= 2^-9 |x|, |x3| <= 2^-18 |x|.  Of the
+// nine products of two such sums the six largest are taken, each exact in the instruction's float32 sum;
+// what is left out is below 2^-26 of a product, a quarter of what one float32 rounding of it may lose.
+//
+// What bounds it: the matrix cores (six products at 16 times the rate of the float32 instruction), and from 17 to 64
+// rows W's bytes.  W comes straight into registers, each wave its own rows, and is parted beside the products (11
+// vector instructions a pair, between MFMAs); X's parts, made once by a small kernel in the order of the operands, go
+// straight into LDS and serve the four waves.  The largest product of each stage has a sum of its own, so that a sum
+// is rounded once a stage at its full size: 2.6 times closer to 64 bits than six roundings, for no vector work.
+// Against the float32 instruction (256 rows, us): 4096 x 4096 94 -> 55, 12288 x 4096 234 -> 155, 22016 x 4096 429 -> 267
+// (1.05 PFLOP/s of bfloat16 products; two blocks a compute unit hold 344 of 512 places), 4096 x 11008 219 -> 134;
+// 2,048 rows of 22016 x 4096 2,877 -> 1,576 (1.4 PFLOP/s).
+// (Published as bf16x6 and the like: Henry, Tang, Heinecke, "Leveraging the bfloat16 artificial intelligence
+// datatype for higher-precision computations", 2019.)
+#include "api.h"
+#include "common.h"
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+#define SP_K 32                                   // k a stage
+
+// two float32 as their three bfloat16 parts, each pair packed
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t& p1, uint32_t& p2, uint32_t& p3) {
+    p1 = pack_bf16x2(a, b);
+    a -= __uint_as_float(p1 << 16);
+    b -= __uint_as_float(p1 & 0xffff0000u);
+    p2 = pack_bf16x2(a, b);
+    a -= __uint_as_float(p2 << 16);
+    b -= __uint_as_float(p2 & 0xffff0000u);
+    p3 = pack_bf16x2(a, b);
+}
+
+// The 8 k of a lane: 4 q .. 4 q + 3 and 16 + 4 q .. 16 + 4 q + 3 of a stage's 32 (both operands alike), so that
+// a load of 16 bytes a lane reads 64 neighbouring bytes of a row.
+__device__ __forceinline__ void split8(f32x4_t lo, f32x4_t hi, illm_u32x4_t (&p)[3]) {
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        const f32x4_t v = h < 2 ? lo : hi;
+        uint32_t a, b, c;
+        split_pair(v[2 * (h & 1)], v[2 * (h & 1) + 1], a, b, c);
+        p[0][h] = a;
+        p[1][h] = b;
+        p[2][h] = c;
+    }
+}
+
+// X's parts in the order that the product's blocks bring them into LDS: [stage of 32 k][16 rows][part][lane].
+// Rows beyond M are zeros.
+__global__ void __launch_bounds__(256)
+f32_split_rows_kernel(const float* __restrict__ X, illm_u32x4_t* __restrict__ P, int M, int K, int tiles) {
+    const int lane = threadIdx.x & 63, tile = blockIdx.y;
+    const int stage = blockIdx.x * 4 + threadIdx.x / 64;
+    if (stage >= K / SP_K) return;
+    const int row = tile * 16 + (lane & 15);
+    f32x4_t lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+    if (row < M) {
+        const float* at = X + (size_t)row * K + stage * SP_K + 4 * (lane >> 4);
+        lo = *(const f32x4_t*)at;
+        hi = *(const f32x4_t*)(at + 16);
+    }
+    illm_u32x4_t p[3];
+    split8(lo, hi, p);
+    illm_u32x4_t* to = P + ((size_t)stage * tiles + tile) * 192 + lane;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) to[64 * i] = p[i];
+}
+
+// A block of four waves takes MT * 16 rows of X and 64 * NT of W; a wave all those rows and 16 * NT of W's.
+template <int MT, int NT, int NS>
+__global__ void __launch_bounds__(256, 2)
+gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restrict__ X, const float* __restrict__ W,
+                      void* __restrict__ Y, int y_dt, int M, int N, int K, int m_tiles, int splits) {
+    constexpr int UNITS = MT * 3;                                              // KB of X a stage
+    constexpr int LX = (UNITS + 3) / 4, L = LX + 2 * NT;                       // loads a wave a stage
+    __shared__ illm_u32x4_t st0[UNITS * 64], st1[UNITS * 64], st2[UNITS * 64];
+    __shared__ illm_u32x4_t st3[NS > 3 ? UNITS * 64 : 1], st4[NS > 3 ? UNITS * 64 : 1], st5[NS > 3 ? UNITS * 64 : 1];
+    const int lane = threadIdx.x & 63, wave = wave_index();
+    const int r = lane & 15, q = lane >> 4;
+    // the blocks that share rows of W run next to each other on one XCD (block ids go round the 8)
+    const int xcd = blockIdx.x & 7, j8 = blockIdx.x >> 3;
+    const int mt = j8 % m_tiles, n0 = ((j8 / m_tiles) * 8 + xcd) * (64 * NT);
+    if (n0 >= N) return;
+    const int every = K / SP_K, per = (every + splits - 1) / splits;
+    const int first = blockIdx.y * per, last = min(first + per, every) - 1;
+
+    const __amdgpu_buffer_rsrc_t xr = illm_buffer(P, (size_t)every * m_tiles * UNITS * 1024);
+    const uint32_t x_stage = (uint32_t)m_tiles * UNITS * 1024, x_lane = (uint32_t)mt * UNITS * 1024 + lane * 16;
+    auto load_x = [&](illm_u32x4_t* b, int s) __attribute__((always_inline)) {
+        const uint32_t at = (uint32_t)min(s, last) * x_stage;
+#pragma unroll
+        for (int i = 0; i < LX; ++i) {
+            const int u = min(i * 4 + wave, UNITS - 1);
+            ld16_lds(xr, b + u * 64, x_lane + u * 1024, at);
+        }
+    };
+    struct Raw { f32x4_t lo[NT], hi[NT]; };
+    struct Parts { illm_u32x4_t w[NT][3]; };
+    uint32_t wo[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) wo[i] = (uint32_t)(min(n0 + (wave * NT + i) * 16 + r, N - 1) - n0) * (uint32_t)K * 4u + 16u * q;
+    const char* const wbase = (const char*)(W + (size_t)n0 * K);
+    auto load_w = [&](Raw& g, int s) __attribute__((always_inline)) {
+        const char* const at = wbase + (size_t)min(s, last) * (SP_K * 4);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            g.lo[i] = *(const f32x4_t*)(at + wo[i]);
+            g.hi[i] = *(const f32x4_t*)(at + wo[i] + 64);
+        }
+    };
+    f32x4_t acc[NT][MT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    // The large products have a sum of their own (one rounding a stage at its size), the five small ones another.
+    f32x4_t low[NT][MT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) low[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    auto split_part = [&](const Raw& g, Parts& p, int e) __attribute__((always_inline)) {     // the e-th pair of a lane
+        const f32x4_t v = e % 4 < 2 ? g.lo[e / 4] : g.hi[e / 4];
+        uint32_t a, b, c;
+        split_pair(v[2 * (e & 1)], v[2 * (e & 1) + 1], a, b, c);
+        p.w[e / 4][0][e % 4] = a;
+        p.w[e / 4][1][e % 4] = b;
+        p.w[e / 4][2][e % 4] = c;
+    };
+    auto multiply = [&](const illm_u32x4_t* b, const Parts& p, const Raw& next, Parts& pn) __attribute__((always_inline)) {
+        constexpr int PW[6] = {2, 0, 1, 0, 1, 0}, PX[6] = {0, 0, 1, 2, 0, 1};
+        constexpr int E = (4 * NT + MT - 1) / MT;                              // pairs of W split beside 16 rows of X
+        illm_u32x4_t xf[2][3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) xf[0][c] = b[c * 64 + lane];
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            if (j + 1 < MT) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) xf[(j + 1) & 1][c] = b[((j + 1) * 3 + c) * 64 + lane];
+            }
+#pragma unroll
+            for (int e = j * E; e < (j + 1) * E; ++e)
+                if (e < 4 * NT) split_part(next, pn, e);
+#pragma unroll
+            for (int t = 0; t < 6; ++t)
+#pragma unroll
+                for (int i = 0; i < NT; ++i) {
+                    f32x4_t& to = t == 1 ? acc[i][j] : low[i][j];
+                    to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&p.w[i][PW[t]],
+                                                                 *(const bf16x8_t*)&xf[j & 1][PX[t]], to, 0, 0, 0);
+                }
+            __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+#pragma unroll
+            for (int t = 0; t < 6 * NT; ++t) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, 2 * E / NT + 1, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    Raw g0, g1, g2, g3, g4, g5;
+    Parts p0, p1;
+    // Turn s: stage s of X stands in LDS and stage s + 1 of W in registers when every wave's loads of NS - 1 turns
+    // ago have arrived; those of the turns since may still be under way.  Nobody reads stage s - 1 any more.
+    auto turn = [&](illm_u32x4_t* cur, illm_u32x4_t* after, const Parts& p, Parts& pn, const Raw& next, Raw& ask,
+                    int s) __attribute__((always_inline)) {
+        constexpr int VM = (NS - 2) * L;
+        static_assert(VM < 64, "the wait count");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x0070 | (VM & 15) | ((VM >> 4) << 14));    // vmcnt(VM), lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        load_x(after, s + NS - 1);
+        load_w(ask, s + NS);
+        if (s <= last) multiply(cur, p, next, pn);
+    };
+    load_w(g0, first);
+    load_x(st0, first);
+    load_w(g1, first + 1);
+    load_x(st1, first + 1);
+    load_w(g2, first + 2);
+    if constexpr (NS > 3) {
+        load_x(st2, first + 2);
+        load_w(g3, first + 3);
+        load_x(st3, first + 3);
+        load_w(g4, first + 4);
+        load_x(st4, first + 4);
+        load_w(g5, first + 5);
+    }
+#pragma unroll
+    for (int e = 0; e < 4 * NT; ++e) split_part(g0, p0, e);
+    for (int s = first; s <= last; s += 6) {
+        if constexpr (NS == 3) {
+            turn(st0, st2, p0, p1, g1, g0, s);
+            turn(st1, st0, p1, p0, g2, g1, s + 1);
+            turn(st2, st1, p0, p1, g0, g2, s + 2);
+            turn(st0, st2, p1, p0, g1, g0, s + 3);
+            turn(st1, st0, p0, p1, g2, g1, s + 4);
+            turn(st2, st1, p1, p0, g0, g2, s + 5);
+        } else {
+            turn(st0, st5, p0, p1, g1, g0, s);
+            turn(st1, st0, p1, p0, g2, g1, s + 1);
+            turn(st2, st1, p0, p1, g3, g2, s + 2);
+            turn(st3, st2, p1, p0, g4, g3, s + 3);
+            turn(st4, st3, p0, p1, g5, g4, s + 4);
+            turn(st5, st4, p1, p0, g0, g5, s + 5);
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);             // no load into LDS outlives the block
+
+    // acc[i][j][v]: row (wave * NT + i) * 16 + 4 q + v of W's, row 16 j + r of X's.  A sum that is no finite
+    // number is taken again with plain multiply-adds: an infinity has no parts.
+    const int k0 = first * SP_K, k1 = (last + 1) * SP_K;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+        const int m = (mt * MT + j) * 16 + r;
+        if (m >= M) continue;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const int n = n0 + (wave * NT + i) * 16 + 4 * q;
+            f32x4_t v = acc[i][j] + low[i][j];
+            bool odd = false;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) odd |= (__float_as_uint(v[e]) & 0x7f800000u) == 0x7f800000u;
+            if (odd) {
+                for (int e = 0; e < 4; ++e) {
+                    if (n + e >= N) break;
+                    float t = 0.f;
+                    for (int k = k0; k < k1; ++k) t = fmaf(X[(size_t)m * K + k], W[(size_t)(n + e) * K + k], t);
+                    v[e] = t;
+                }
+            }
+            const size_t at = ((size_t)blockIdx.y * M + m) * N + n;
+            if (n + 3 < N && (N & 3) == 0 && y_dt == ILLM_F32) {
+                *(f32x4_t*)((float*)Y + at) = v;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) st_f(Y, y_dt, at + e, v[e]);
+            }
+        }
+    }
+}
+
+// Y = the planes' sum, in order; four elements a thread, n4 of them.
+__global__ void __launch_bounds__(256)
+f32_planes_sum_kernel(const float* __restrict__ planes, void* __restrict__ Y, int y_dt, int S, size_t n4) {
+    for (size_t i = blockIdx.x * 256ull + threadIdx.x; i < n4; i += gridDim.x * 256ull) {
+        f32x4_t v = ((const f32x4_t*)planes)[i];
+        for (int s = 1; s < S; ++s) v += ((const f32x4_t*)planes)[s * n4 + i];
+        st_f4(Y, y_dt, i, make_float4(v[0], v[1], v[2], v[3]));
+    }
+}
+
+struct SplitTiles { int mt, nt, m_tiles, blocks; };
+
+// Rows in equal tiles of at most 128.  Along W a block takes 64 or 128: a compute unit works through its blocks
+// in rounds of 256, and one of 128 takes 1.8 times one of 64 (245 rows, us with 128 / with 64: 12288 x 4096
+// 146 / 164, 22016 x 4096 263 / 252; 64 rows: 94 / 70 and 112 / 129; 900 rows of 22016 x 4096 789 / 850).
+static SplitTiles split_tiles(int M, int N, int splits) {
+    const int tiles = (M + 15) / 16, m_tiles = (tiles + 7) / 8, need = (tiles + m_tiles - 1) / m_tiles;
+    const int mt = need <= 2 ? need : need <= 4 ? 4 : need <= 6 ? 6 : 8;
+    const int b1 = (N + 63) / 64 * m_tiles, b2 = (N + 127) / 128 * m_tiles;
+    const bool wide = splits > 1 || 10 * 23 * ((b2 + 255) / 256) <= 10 * 13 * ((b1 + 255) / 256);
+    return {mt, wide ? 2 : 1, m_tiles, wide ? b2 : b1};
+}
+
+// Parts of K for about one block a compute unit where the tiles are fewer (than 160 of 64 columns): at most 8, each of
+// at least 16 stages, none empty.  The same for all rows up to 128.
+extern "C" int illm_gemm_f32_split_parts(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K < SP_K) return 1;
+    const SplitTiles t = split_tiles(M, N, 2);
+    if ((N + 63) / 64 * t.m_tiles >= 160) return 1;
+    const int every = K / SP_K, s = max(1, min(min(256 / t.blocks, 8), every / 16)), per = (every + s - 1) / s;
+    return (every + per - 1) / per;
+}
+
+// Rows of X as its parts are laid out (M filled up to whole tiles): 6 bytes of scratch for each of their K.
+extern "C" int illm_gemm_f32_split_rows(int M) {
+    if (M <= 0) return 0;
+    const SplitTiles t = split_tiles(M, 64, 1);
+    return t.m_tiles * t.mt * 16;
+}
+
+// float32 X [M, K] and W [N, K] on 16-byte addresses, K % 32 == 0; P: scratch of 6 K
+// illm_gemm_f32_split_rows(M) bytes (at most 4 GiB).  splits 1: Y [M, N], float32 or bfloat16; more: float32 planes [splits][M][N], no part
+// of K empty.
+extern "C" int illm_gemm_f32_split(const float* X, const float* W, void* P, size_t p_bytes, void* Y, int y_dt, int M,
+                                   int N, int K, int splits, void* stream) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % SP_K || K >= 1 << 22 || !illm_dtype_ok(y_dt) || !X || !W || !Y || !P ||
+        splits < 1 || splits > 65535 || (splits > 1 && y_dt != ILLM_F32) || ((uintptr_t)X | (uintptr_t)W | (uintptr_t)P | (uintptr_t)Y) % 16)
+        return ILLM_ERR_ARG;
+    const int every = K / SP_K, per = (every + splits - 1) / splits;
+    const SplitTiles t = split_tiles(M, N, splits);
+    const size_t need = (size_t)t.m_tiles * t.mt * 16 * K * 6;
+    const long long grid_x = ((long long)(t.blocks / t.m_tiles) + 7) / 8 * 8 * t.m_tiles;
+    if ((long long)(splits - 1) * per >= every || need > p_bytes || need > 0xffffffffu || grid_x > 0x7fffffff ||
+        t.m_tiles * t.mt > 65535)
+        return ILLM_ERR_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    hipLaunchKernelGGL(f32_split_rows_kernel, dim3((every + 3) / 4, t.m_tiles * t.mt), dim3(256), 0, st, X,
+                       (illm_u32x4_t*)P, M, K, t.m_tiles * t.mt);
+    const dim3 grid((unsigned)grid_x, splits);
+#define ILLM_SPLIT(MT, NT, NS)                                                                                      \
+    if (t.mt == MT && t.nt == NT)                                                                                   \
+        hipLaunchKernelGGL((gemm_f32_split_kernel<MT, NT, NS>), grid, dim3(256), 0, st, (const illm_u32x4_t*)P, X, W, \
+                           Y, y_dt, M, N, K, t.m_tiles, splits)
+    ILLM_SPLIT(1, 1, 6); ILLM_SPLIT(1, 2, 6); ILLM_SPLIT(2, 1, 6); ILLM_SPLIT(2, 2, 6);
+    ILLM_SPLIT(4, 1, 6); ILLM_SPLIT(4, 2, 6); ILLM_SPLIT(6, 1, 3); ILLM_SPLIT(6, 2, 3); ILLM_SPLIT(8, 1, 3);
+    ILLM_SPLIT(8, 2, 3);
+#undef ILLM_SPLIT
+    return illm_launch_status();
+}
+
+// Y [n], float32 or bfloat16, from float32 planes [S][n]; n a multiple of 4, all on 16-byte addresses.
+extern "C" int illm_f32_planes_sum(const float* planes, void* Y, int y_dt, int S, size_t n, void* stream) {
+    if (!planes || !Y || S < 1 || n % 4 || !illm_dtype_ok(y_dt) || ((uintptr_t)planes | (uintptr_t)Y) % 16) return ILLM_ERR_ARG;
+    if (n == 0) return ILLM_OK;
+    const size_t blocks = (n / 4 + 255) / 256;
+    hipLaunchKernelGGL(f32_planes_sum_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0,
+                       (hipStream_t)stream, planes, Y, y_dt, S, n / 4);
+    return illm_launch_status();
+}

@@ -573,14 +573,73 @@ def gemm_rows_f32_mfma_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def gemm_rows_f32_mfma(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     """x [M <= 128, K] . w [N, K]^T, both float32, W read once, on the matrix cores' float32
-    instruction.  A row's sum does not depend on the other rows or on their number."""
+    instruction; large matrices in bfloat16 parts (`gemm_f32_split`).  A row's sum does not depend on the other rows
+    or on their number."""
     _gpu(x, w)
     _need(gemm_rows_f32_mfma_fits(x, w), "gemm_rows_f32_mfma: operands not taken")
+    if _split_large(w) and gemm_f32_split_fits(x, w):
+        return gemm_f32_split(x, w, out_dtype)
     M, K = x.shape
     N = w.shape[0]
     y = torch.empty((M, N), dtype=out_dtype, device=x.device)
     _check(_lib().illm_gemm_rows_f32_mfma(_p(x), _p(w), _p(y), _code(y), M, N, K, _stream()),
            "gemm_rows_f32_mfma")
+    return y
+
+
+def gemm_f32_split_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether `gemm_f32_split` takes these operands."""
+    if not (x.dtype == torch.float32 and w.dtype == torch.float32 and x.dim() == 2 and w.dim() == 2
+            and x.shape[0] >= 1 and x.shape[1] == w.shape[1] and x.shape[1] % 32 == 0
+            and x.is_contiguous() and w.is_contiguous() and _on16(x, w)):
+        return False
+    return (x.shape[0] + 127) * 6 * x.shape[1] < 0xffffffff and x.shape[1] < 1 << 22
+
+
+def gemm_f32_split_pays(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether it is the faster way for operands that it takes.  Parting X and the sums of K's parts cost 4 to 8 us,
+    so short sums and small matrices stay with the kernels of the float32 instruction (whose time grows with K).
+    us there -> here, matrices cold: 33 / 100 rows of 2048 x 2048 17 / 38 -> 22 / 30;
+    17 rows of 4096 x 4096 28 -> 26, of 2048 x 2048 14 -> 20, of 8192 x 2048 27 -> 24; 9 of 4096 x 11008 55 -> 51, of
+    12288 x 4096 55 -> 58; 700 of 4096 x 1024 65 -> 49, of 1024 x 1024 25 -> 34; 2,048 of 1024 x 256 15 -> 19.  Large:
+    64 / 256 / 2,048 rows of 22016 x 4096 203 / 429 / 2,877 -> 118 / 267 / 1,576, of 4096 x 11008 135 / 219 / 1,412 ->
+    62 / 134 / 827.  Largest error against 64 bits 1.9e-6 -> 6.7e-7."""
+    M, (N, K) = x.shape[0], w.shape
+    if K < 2048:
+        return K >= 512 and M * N >= 1400000
+    if N < 1024:
+        return False
+    return M >= (9 if _split_large(w) or K >= 8192 else 17 if K >= 4096 or N * K >= 1 << 24 else 65)
+
+
+def _split_large(w: torch.Tensor) -> bool:
+    """Matrices whose products of up to 128 rows are parted whatever the rows (so that a row's bits do not depend on
+    their number): 16 rows of 12288 x 4096 60 -> 58 us, of 22016 x 4096 110 -> 98; 9 rows 55 -> 58 and 96 -> 97."""
+    return w.shape[0] >= 1024 and w.shape[1] >= 2048 and w.shape[0] * w.shape[1] >= 1 << 25
+
+
+def _f32_split(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, S: int) -> torch.Tensor:
+    """[M, N] (S = 1) or float32 planes [S, M, N]."""
+    _gpu(x, w)
+    (M, K), N = x.shape, w.shape[0]
+    parts = torch.empty(_lib().illm_gemm_f32_split_rows(M) * K * 6, dtype=torch.uint8, device=x.device)
+    y = torch.empty((M, N) if S == 1 else (S, M, N), dtype=out_dtype, device=x.device)
+    _check(_lib().illm_gemm_f32_split(_p(x), _p(w), _p(parts), ctypes.c_size_t(parts.numel()), _p(y), _code(y), M, N, K, S,
+                                      _stream()), "gemm_f32_split")
+    return y
+
+
+def gemm_f32_split(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
+    """x [M, K] . w [N, K]^T, both float32, as six products of bfloat16 parts on the matrix cores, no less precise
+    than a float32 sum of float32 products (csrc/gemm_f32_split.hip)."""
+    _need(gemm_f32_split_fits(x, w), "gemm_f32_split: operands not taken")
+    (M, K), N = x.shape, w.shape[0]
+    S = _lib().illm_gemm_f32_split_parts(M, N, K) if N % 4 == 0 else 1
+    if S == 1:
+        return _f32_split(x, w, out_dtype, 1)
+    planes = _f32_split(x, w, torch.float32, S)
+    y = torch.empty((M, N), dtype=out_dtype, device=x.device)
+    _check(_lib().illm_f32_planes_sum(_p(planes), _p(y), _code(y), S, ctypes.c_size_t(M * N), _stream()), "f32_planes_sum")
     return y
 
 
@@ -812,11 +871,13 @@ def linear_cut_fits(x, w) -> bool:
 
 def linear_cut(x: torch.Tensor, w, splits: int = 0) -> torch.Tensor:
     """x . w^T as float32 planes [S, M, N] whose sum over S is the product, for 129 to 256 rows
-    (csrc/gemm_tiles.hip, row-major w).  The planes go to `add_rmsnorm` as `delta`."""
+    (csrc/gemm_tiles.hip, row-major w) or float32 operands.  The planes go to `add_rmsnorm` as `delta`."""
     x, w = x.contiguous(), plain_weight(w)
     _gpu(x, w)
     M, K = x.shape
     N = w.shape[0]
+    if x.dtype == torch.float32:
+        return _f32_split(x, w, torch.float32, splits or _lib().illm_gemm_f32_split_parts(M, N, K))
     S = splits or _lib().illm_gemm_tiles_splits(N, K)
     y = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
     _check(_lib().illm_gemm_tiles_planes(_p(x), _p(w), _p(y), M, N, K, S, _stream()), "linear_cut")
@@ -837,6 +898,8 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     if isinstance(w, Weight) and not (x.dtype == torch.bfloat16 and 1 <= x.shape[0] <= SKINNY_BEST_ROWS):
         w = w.plain                                      # only the few-rows kernel reads the copy
     if x.dtype == torch.float32 or w.dtype == torch.float32:
+        if gemm_f32_split_fits(x, w) and gemm_f32_split_pays(x, w):
+            return gemm_f32_split(x, w, out_dtype)
         if x.shape[0] >= ROWS_F32_MFMA_FROM and gemm_rows_f32_mfma_fits(x, w):
             return gemm_rows_f32_mfma(x, w, out_dtype)
         if gemv_rows_f32_fits(x, w):

@@ -534,6 +534,32 @@ def test_gemm_rows_f32_mfma(ydt, M, N, K):
     assert not ops().gemm_rows_f32_mfma_fits(rnd(M, K + 16).to(DEV), rnd(N, K + 16).to(DEV))
 
 
+@pytest.mark.parametrize("M,N,K,S", [(1, 64, 32, 1), (9, 1027, 2048, 1), (16, 130, 96, 3), (17, 4096, 64, 2), (33, 129, 224, 7),
+                                     (65, 65, 160, 1), (96, 16400, 64, 1), (100, 500, 512, 4), (128, 1028, 992, 8),
+                                     (129, 12288, 96, 1), (257, 300, 416, 2), (400, 7, 352, 1)])
+def test_gemm_f32_split(M, N, K, S):
+    """The float32 product in bfloat16 parts, whole and as planes: within the rounding of float32 sums (a sum of K / 32
+    stages and a few more, each within 2^-23 of the sum of absolute products), edges of the tiles, a row's bits the
+    same alone and among others, and infinities, NaN and the largest numbers as plain multiply-adds have them."""
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+    xd, wd = x.to(DEV), w.to(DEV)
+    assert ops().gemm_f32_split_fits(xd, wd)
+    got = ops()._f32_split(xd, wd, torch.float32, S)
+    whole = got.sum(0) if S > 1 else got
+    bound = 2.0 ** -23 * (K / 32 + 16) * (x.double().abs() @ w.double().abs().t())
+    assert bool(((whole.double().cpu() - R.linear(x, w, torch.float64)).abs() <= bound).all())
+    alone = ops()._f32_split(xd[M - 1:].contiguous(), wd, torch.float32, S)
+    assert torch.equal(alone[..., 0, :], got[..., M - 1, :])
+    direct = ops().gemm_f32_split(xd, wd, torch.float32)          # with the library's own number of parts
+    assert bool(((direct.double().cpu() - R.linear(x, w, torch.float64)).abs() <= bound).all())
+    close(ops().gemm_f32_split(xd, wd, torch.bfloat16), R.linear(x, w, torch.float64), torch.bfloat16, scale=math.sqrt(K))
+    x[0, 3], w[1, 5], w[N - 1, K - 1] = float("inf"), float("nan"), 3.4028e38
+    got = ops().gemm_f32_split(x.to(DEV), w.to(DEV), torch.float32).cpu()
+    want = ops().gemm_generic(x.to(DEV), w.to(DEV), torch.float32).cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert not ops().gemm_f32_split_fits(rnd(M, K + 16).to(DEV), rnd(N, K + 16).to(DEV))
+
+
 @pytest.mark.parametrize("ydt", DTYPES)
 @pytest.mark.parametrize("M,N,K", [(129, 128, 16), (130, 33, 48), (200, 411, 80), (257, 129, 1008), (1, 5, 32),
                                    (300, 1000, 4096), (2048, 130, 512)])
