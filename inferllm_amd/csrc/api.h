@@ -19,6 +19,9 @@ int illm_embed(const int32_t* tokens, const void* table, int table_dt, float* ou
 int illm_embed_scaled(const int32_t* tokens, const void* table, int table_dt, float* out,
                       int T, int E, int V, float scale, void* stream);
 
+// Zeros to n pieces of device memory, `bytes` each (host arrays).
+int illm_zero_pieces(const uint64_t* at, const uint64_t* bytes, int n, void* stream);
+
 // out[t, :] = v / sqrt(mean(v^2) + eps) * w, v = table[tokens[t]] * scale; `copy` (null: none) takes it too.
 int illm_embed_norm(const int32_t* tokens, const void* table, int table_dt, const void* w, int w_dt, float* out,
                     float* copy, int T, int E, int V, float scale, float eps, void* stream);

@@ -118,6 +118,48 @@ copy_rows_kernel(const float* __restrict__ x, float* __restrict__ out, size_t n)
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step) out[i] = x[i];
 }
 
+// Zeros to several pieces of memory in one launch (the state of a sequence that begins: with a fill a tensor, 11 of
+// 1.9 us and 6 us of the host each, for every sequence of a batch).  A block's share is 16 KB of one piece; a piece's
+// first and last bytes, where it does not lie on 16, go one by one.
+#define ZERO_PIECES 16
+struct ZeroPieces {
+    char* at[ZERO_PIECES];
+    size_t bytes[ZERO_PIECES];
+};
+
+__global__ void __launch_bounds__(256)
+zero_pieces_kernel(ZeroPieces z) {
+    char* const at = z.at[blockIdx.y];
+    const size_t bytes = z.bytes[blockIdx.y];
+    const size_t head = min(bytes, (size_t)(-(intptr_t)at & 15)), whole = (bytes - head) / 16, tail = head + whole * 16;
+    const illm_u32x4_t zero = {0, 0, 0, 0};
+    for (size_t i = blockIdx.x * 1024ull + threadIdx.x, n = 0; n < 4 && i < whole; ++n, i += 256) ((illm_u32x4_t*)(at + head))[i] = zero;
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < head) at[threadIdx.x] = 0;
+        if (threadIdx.x < bytes - tail) at[tail + threadIdx.x] = 0;
+    }
+}
+
+extern "C" int illm_zero_pieces(const uint64_t* at, const uint64_t* bytes, int n, void* stream) {
+    if (n < 0 || (n && (!at || !bytes))) return ILLM_ERR_ARG;
+    for (int i = 0; i < n; i += ZERO_PIECES) {
+        ZeroPieces z = {};
+        const int m = n - i < ZERO_PIECES ? n - i : ZERO_PIECES;
+        size_t most = 0;
+        for (int j = 0; j < m; ++j) {
+            if (!at[i + j] && bytes[i + j]) return ILLM_ERR_ARG;
+            z.at[j] = (char*)at[i + j];
+            z.bytes[j] = bytes[i + j];
+            most = most < z.bytes[j] ? z.bytes[j] : most;
+        }
+        const size_t blocks = (most + 16383) / 16384;
+        if (blocks == 0) continue;
+        if (blocks > 0x7fffffff) return ILLM_ERR_ARG;
+        hipLaunchKernelGGL(zero_pieces_kernel, dim3((unsigned)blocks, m), dim3(256), 0, (hipStream_t)stream, z);
+    }
+    return illm_launch_status();
+}
+
 extern "C" int illm_copy_rows(const float* x, float* out, size_t n, void* stream) {
     if (!x || !out) return ILLM_ERR_ARG;
     if (n == 0) return ILLM_OK;

@@ -20,9 +20,10 @@ import os
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence
 
+import numpy as np
 import torch
 
-from ..cache.manager import CacheManager
+from ..cache.manager import CacheManager, to_device
 from ..kernels import ops
 from ..parts.base import StepContext
 from .model import DecoderModel
@@ -186,31 +187,48 @@ class StepRunner:
         self._prompt_uses: Dict[tuple, int] = {}
 
     # ------------------------------------------------------------ checks
-    def _phase(self, entries: Sequence[StepEntry]) -> bool:
-        """True for a step of whole prompts, False for a step of single tokens."""
+    def _ids(self, e: StepEntry) -> Sequence[int]:
+        """The entry's tokens, each found to be an id of the vocabulary (several integers as an array: a loop over
+        nine thousand tokens keeps the device waiting for a millisecond)."""
+        if len(e.tokens) > 8:
+            try:
+                ids = np.asarray(e.tokens)
+            except (TypeError, ValueError, RuntimeError):
+                ids = None
+            if (ids is not None and ids.ndim == 1 and ids.dtype.kind in "iu"
+                    and 0 <= int(ids.min()) and int(ids.max()) < self.vocab_size):
+                return ids
+        out = []
+        for t in e.tokens:
+            if not (0 <= int(t) < self.vocab_size):
+                raise StepError(f"slot {e.slot}: token id {t} outside the vocabulary "
+                                f"of {self.vocab_size}")
+            out.append(int(t))
+        return out
+
+    def _phase(self, entries: Sequence[StepEntry]):
+        """(True for a step of whole prompts or False for a step of single tokens, the entries' token ids)."""
         if not entries:
             raise StepError("a step needs at least one sequence")
         slots = [e.slot for e in entries]
         if len(set(slots)) != len(slots):
             raise StepError("a slot appears twice in one step")
+        ids = []
         for e in entries:
             if len(e.tokens) == 0:
                 raise StepError(f"slot {e.slot}: no tokens in this step")
-            for t in e.tokens:
-                if not (0 <= int(t) < self.vocab_size):
-                    raise StepError(f"slot {e.slot}: token id {t} outside the vocabulary "
-                                    f"of {self.vocab_size}")
+            ids.append(self._ids(e))
             for w in e.want:
                 if not (0 <= int(w) < len(e.tokens)):
                     raise StepError(f"slot {e.slot}: wanted place {w} is not among the "
                                     f"{len(e.tokens)} tokens of this step")
         starts = [self.cache.length(e.slot) == 0 for e in entries]
         if all(starts):
-            return True
+            return True, ids
         if not any(starts) and all(len(e.tokens) == 1 for e in entries):
-            return False
+            return False, ids
         if not self.model.one_token_mixers:
-            return True            # every mixer goes on from what it kept by any number of tokens
+            return True, ids       # every mixer goes on from what it kept by any number of tokens
         raise StepError("the sequences of a step must either all start at their first token "
                         "or all go on by one token: this model's "
                         f"{', '.join(self.model.one_token_mixers)} cannot go on by several")
@@ -230,7 +248,7 @@ class StepRunner:
         `borrow`: the result may be a view of memory that the next step writes again (a decode
         graph's output); a caller that has used it up by then saves a copy.  Without it the
         result is the caller's to keep."""
-        prefill = self._phase(entries)          # True: a step of several tokens per sequence
+        prefill, ids = self._phase(entries)     # True: a step of several tokens per sequence
         if self.plan is not None:
             ops.use_plan(self.plan)
         if device_tokens is not None:
@@ -250,7 +268,7 @@ class StepRunner:
             g = self._prompt_graph_for(entries, starts)
             if g is not None:
                 return self._replay_prompt(g, entries, starts, borrow)
-            return self._prefill(entries, starts)
+            return self._prefill(entries, starts, ids)
         return self._decode(entries, starts, device_tokens, borrow)
 
     def _prompt_graph_for(self, entries: Sequence[StepEntry], starts: Sequence[int]) -> Optional[_PromptGraph]:
@@ -334,27 +352,28 @@ class StepRunner:
             logits = logits[torch.tensor(order, dtype=torch.long, device=self.device)]
         return logits
 
-    def _prefill(self, entries: Sequence[StepEntry], starts: Sequence[int]) -> Optional[torch.Tensor]:
-        tokens: List[int] = []
-        pos: List[int] = []
-        slot: List[int] = []
+    def _prefill(self, entries: Sequence[StepEntry], starts: Sequence[int],
+                 ids: Sequence[Sequence[int]]) -> Optional[torch.Tensor]:
         cu = [0]
         want: List[int] = []
-        for e, start in zip(entries, starts):
-            n = len(e.tokens)
+        for e in entries:
             want.extend(cu[-1] + int(w) for w in e.want)
-            tokens.extend(int(t) for t in e.tokens)
-            pos.extend(range(start, start + n))
-            slot.extend([e.slot] * n)
-            cu.append(cu[-1] + n)
-        T, B = len(tokens), len(entries)
-        host = torch.tensor(tokens + pos + slot + cu + [e.slot for e in entries]
-                            + [s + len(e.tokens) for e, s in zip(entries, starts)]
-                            + [int(s) for s in starts] + want, dtype=torch.int32)
-        meta = host.to(self.device)
+            cu.append(cu[-1] + len(e.tokens))
+        T, B = cu[-1], len(entries)
+        sizes = (T, T, T, B + 1, B, B, B, len(want))
+        host = torch.empty(sum(sizes), dtype=torch.int32)
+        flat = host.numpy()
+        for e, start, tokens, at, to in zip(entries, starts, ids, cu, cu[1:]):
+            flat[at:to] = tokens
+            flat[T + at:T + to] = np.arange(start, start + to - at)
+            flat[2 * T + at:2 * T + to] = e.slot
+        flat[3 * T:] = (cu + [e.slot for e in entries] + [s + len(e.tokens) for e, s in zip(entries, starts)]
+                        + [int(s) for s in starts] + want)
+        meta = torch.empty(host.shape, dtype=torch.int32, device=self.device)
+        to_device(meta, host)
         o = 0
         parts = []
-        for n in (T, T, T, B + 1, B, B, B, len(want)):
+        for n in sizes:
             parts.append(meta[o:o + n])
             o += n
         ctx = StepContext(

@@ -141,6 +141,16 @@ def embed_norm(tokens: torch.Tensor, table: torch.Tensor, weight: torch.Tensor, 
     return out
 
 
+def zero_slot(tensors, slot: int) -> None:
+    """Row `slot` of every tensor to zeros (contiguous [slots, ...], any types), in one launch for 16 of them."""
+    rows = [t[slot] for t in tensors]
+    _gpu(*rows)
+    n = len(rows)
+    at = (ctypes.c_uint64 * n)(*[r.data_ptr() for r in rows])
+    size = (ctypes.c_uint64 * n)(*[r.numel() * r.element_size() for r in rows])
+    _check(_lib().illm_zero_pieces(at, size, n, _stream()), "zero_slot")
+
+
 def copy_rows(x: torch.Tensor) -> torch.Tensor:
     """A copy of float32 rows by a kernel of the library (also under graph capture)."""
     _gpu(x)

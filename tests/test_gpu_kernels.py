@@ -560,6 +560,22 @@ def test_gemm_f32_split(M, N, K, S):
     assert not ops().gemm_f32_split_fits(rnd(M, K + 16).to(DEV), rnd(N, K + 16).to(DEV))
 
 
+def test_zero_slot():
+    """A slot's row of every state tensor to zeros: 19 tensors (more than a launch takes), rows of 1 byte to 100 KB
+    that begin on and off 16 bytes, and nothing beside them."""
+    shapes = [(1,), (3,), (5, 7), (16,), (33,), (64, 129), (25000,), (2, 3, 4), (1021,)]
+    ts = [torch.ones((4,) + sh, dtype=dt, device=DEV) for sh in shapes for dt in (torch.float32, torch.bfloat16)]
+    ts.append(torch.ones((4, 17), dtype=torch.uint8, device=DEV))
+    for slot in (0, 2, 3):
+        for t in ts:
+            t.fill_(1)
+        ops().zero_slot(ts, slot)
+        for t in ts:
+            want = torch.ones_like(t)
+            want[slot] = 0
+            assert torch.equal(t, want)
+
+
 @pytest.mark.parametrize("ydt", DTYPES)
 @pytest.mark.parametrize("M,N,K", [(129, 128, 16), (130, 33, 48), (200, 411, 80), (257, 129, 1008), (1, 5, 32),
                                    (300, 1000, 4096), (2048, 130, 512)])
