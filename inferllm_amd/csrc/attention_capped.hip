@@ -1033,7 +1033,7 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
     const int rep = nh / nkv, per_kv = (rep + DH - 1) / DH;
     const int kvh = blockIdx.x / per_kv, h0 = kvh * rep + (blockIdx.x % per_kv) * DH;
     const int hb = min(DH, (kvh + 1) * rep - h0);
-    const int b = blockIdx.y, sp = blockIdx.z;
+    const int b = blockIdx.z, sp = blockIdx.y;
     const int w = wave_index(), lane = threadIdx.x & 63, grp = lane >> 3, sub = lane & 7;
     const int len = seq_len[b], slot = seq_slot[b];
     const SeenKeys seen = seen_keys(len, window, chunk, keep);
@@ -1295,7 +1295,8 @@ extern "C" int illm_attn_cap_decode(const void* q, int q_stride, void* out, int 
         int dh = g_attn_cap_heads;
         if (dh == 0)
             for (dh = 4; dh > 1 && (long)nkv * ((rep + dh - 1) / dh) * B * nsplit < 256;) dh /= 2;
-        const dim3 grid(nkv * ((rep + dh - 1) / dh), B, nsplit);
+        // (a sequence's ranges next to each other: the longest sequence's go to many compute units)
+        const dim3 grid(nkv * ((rep + dh - 1) / dh), nsplit, B);
         const int kq = (dk + 8 * unit - 1) / (8 * unit), vq = (dv + 8 * unit - 1) / (8 * unit);
 #define GO(DT_, KQ_, VQ_)                                                                          \
     if (dh == 1)                                                                                   \
