@@ -228,6 +228,10 @@ int illm_attn_decode_bf16_static(const void* qkv, void* out, const void* kcache,
 int illm_gemm_skinny_bf16(const void* X, const void* W, const void* Wt, void* Y, int y_dt, int M,
                           int N, int K, const float* ssq, int parts, float eps, int waves_wanted,
                           void* stream);
+// The same of at most 16 rows, an activation on the float32 sums: act 1 relu(y)^2, 2 gelu(y) by tanh, 0 none.
+int illm_gemm_skinny_act(const void* X, const void* W, const void* Wt, void* Y, int y_dt, int M, int N, int K,
+                         const float* ssq, int parts, float eps, int act, void* stream);
+
 
 // Y[M, N] (float32 residual rows) += X . W^T for M <= 16 bfloat16 rows.  nw != null (the weight of
 // the RMS norm that follows, bfloat16 or float32 [N]): also xb[M, N] = bfloat16(Y * nw) and

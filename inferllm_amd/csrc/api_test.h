@@ -26,6 +26,10 @@ void illm_set_attn_f32_mfma(int on);
 // more.
 void illm_set_prefill_two_buffers(int on);
 
+// illm_gemm_skinny_bf16 and _act, up to 8 rows from the tiled copy: half a tile a block, 0 never, 1 always, -1 (default)
+// where the tiles are few.
+void illm_set_skinny_half(int on);
+
 // illm_gemm_mid_bf16: tiles of W a wave takes, 1 or 2 (0, default: by the number of tiles).
 void illm_set_mid_tiles_per_wave(int n);
 // illm_gemm_mid_bf16: rows of X a launch takes, 64 or 128 (default); W is read once a launch.

@@ -195,6 +195,10 @@ __device__ __forceinline__ float block_max(float v, float* red) {
     return t;
 }
 
+__device__ __forceinline__ float gelu_tanh_f(float z) {
+    return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+}
+
 static inline int illm_launch_status() {
     return hipGetLastError() == hipSuccess ? ILLM_OK : ILLM_ERR_LAUNCH;
 }

@@ -327,10 +327,6 @@ __global__ void gelu_tanh_kernel(const void* __restrict__ x, void* __restrict__ 
     st_f(out, dt, i, 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))));
 }
 
-__device__ __forceinline__ float gelu_tanh_f(float z) {
-    return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-}
-
 // bfloat16 with n % 8 == 0: 8 values (16 bytes) a thread
 __global__ void __launch_bounds__(256)
 gelu_tanh_bf16x8_kernel(const bf16_t* __restrict__ x, bf16_t* __restrict__ out, size_t n8) {

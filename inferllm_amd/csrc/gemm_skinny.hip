@@ -62,7 +62,9 @@ struct SkResidual {
     float act_alpha;             // g = min(gate, limit), u = clamp(up, -limit, limit); else silu(gate) up
     int planes;                  // SK_PLAIN: > 1, W's rows are that many parts and part p, whose rows end at
     int ends[ILLM_MAX_PLANES];   // ends[p] (multiples of a block's rows but for the last), reads plane p of
-};                               // X [planes][M][K]
+                                 // X [planes][M][K]
+    int act;                     // SK_PLAIN without `accumulate`: 1 relu(y)^2, 2 gelu(y) (tanh), 0 y
+};
 
 // TILED (NTB == 1, K % 32 == 0): W is a copy laid out for this kernel, [tile][k-step][16 rows][32 k]
 // with tile = blockIdx.x holding the 16 rows that block works on (in its mode's order): a load
@@ -71,7 +73,10 @@ struct SkResidual {
 // ONE_SHOT: a wave asks for its whole share of K at once and holds no second piece (for K that
 // the block's waves cover in one piece each: the product of a short K is bound by the round
 // trips of a wave's pieces, not by bandwidth).
-template <int MT, int NTB, int SK_U, int MAXW, int MODE, bool TILED, bool ONE_SHOT = false>
+// HALF (TILED, MT == NTB == 1, at most 8 rows of X): a block takes 8 rows of a tile, so that a matrix of few tiles
+// occupies twice the compute units.  The MFMA's 16 rows of W are then its 8 at one k-step and at the next, its 16
+// columns the rows of X likewise, and the two quarters of the result that belong together are added at the end.
+template <int MT, int NTB, int SK_U, int MAXW, int MODE, bool TILED, bool ONE_SHOT = false, bool HALF = false>
 __global__ void __launch_bounds__(64 * MAXW)
 gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                    void* __restrict__ Y, int y_dt, int M, int N, int K, SkRope rope,
@@ -130,7 +135,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
         tot += __shfl_xor(tot, 32, ILLM_WAVE);
         if (lane < 16) row_rs[lane] = 1.0f / sqrtf(tot / (float)K + res.eps);
     }
-    const int n_base = blockIdx.x * (DUAL ? 8 * NTB : 16 * NTB);
+    const int n_base = blockIdx.x * (DUAL ? 8 * NTB : HALF ? 8 : 16 * NTB);
     if (MODE == SK_PLAIN && res.planes > 1) {
         int plane = 0;
         for (int p = 0; p + 1 < res.planes; ++p) plane += n_base >= res.ends[p] ? 1 : 0;
@@ -214,7 +219,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
     const bf16_t* xrow[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-        int mm = mt * 16 + r;
+        int mm = HALF ? r & 7 : mt * 16 + r;
         mm = mm < M ? mm : M - 1;
         xrow[mt] = X + (size_t)mm * K;
     }
@@ -233,12 +238,13 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
     const int w_row = lane >> 3, w_chunk = lane & 7;
     // TILED: this lane's 8 values of k-step 0 of the block's first tile; a last block may have
     // fewer than NTB tiles (SK_GATE_UP with NTB > 1)
-    const bf16_t* wtile = W + (size_t)blockIdx.x * NTB * ((K + 31) / 32) * 512 + (r * 4 + q) * 8;
+    const bf16_t* wtile = W + (size_t)(HALF ? blockIdx.x / 2 : blockIdx.x * NTB) * ((K + 31) / 32) * 512 +
+                          ((HALF ? (blockIdx.x & 1) * 8 + (r & 7) : r) * 4 + q) * 8;
     bool tile_ok[NTB];
 #pragma unroll
     for (int nt = 0; nt < NTB; ++nt) tile_ok[nt] = DUAL ? n_base + 8 * nt < N : tile_row[nt] < N || MODE != SK_PLAIN;
 
-    const int ksteps = (K + 31) / 32;
+    const int all_steps = (K + 31) / 32, ksteps = HALF ? (all_steps + 1) / 2 : all_steps;
     const int stride = waves * SK_U;
     uint4 a[NTB][SK_U], b[MT][SK_U];
     auto load = [&](int s0, uint4 (&aa)[NTB][SK_U], uint4 (&bb)[MT][SK_U]) {
@@ -248,13 +254,16 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
             const int kw = (s0 + (u & ~1)) * 32 + w_chunk * 8;
 #pragma unroll
             for (int nt = 0; nt < NTB; ++nt) {
-                if (TILED)
+                if (HALF) {
+                    const int st = 2 * (s0 + u) + (r >> 3);
+                    aa[nt][u] = st < all_steps ? ld16_stream(wtile + (size_t)st * 512) : make_uint4(0, 0, 0, 0);
+                } else if (TILED)
                     aa[nt][u] = (s0 + u < ksteps && tile_ok[nt])
                                     ? ld16_stream(wtile + ((size_t)nt * ksteps + s0 + u) * 512)
                                     : make_uint4(0, 0, 0, 0);
                 else aa[nt][u] = kw < K ? ld16_stream(wline[nt][u & 1] + kw) : make_uint4(0, 0, 0, 0);
             }
-            const int k = (s0 + u) * 32 + q * 8;
+            const int k = (HALF ? 2 * (s0 + u) + (r >> 3) : s0 + u) * 32 + q * 8;
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
                 bb[mt][u] = k < K ? *(const uint4*)(xrow[mt] + k) : make_uint4(0, 0, 0, 0);
@@ -307,7 +316,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
     }
     // acc[nt][mt][i] = Y[m = mt*16 + r][n = n_base + nt*16 + q*4 + i]
     constexpr int PER_WAVE = SK_REGION_FLOATS;
-    if (waves > 1 || MODE != SK_PLAIN) {
+    if (waves > 1 || MODE != SK_PLAIN || HALF) {
 #pragma unroll
         for (int nt = 0; nt < NTB; ++nt)
 #pragma unroll
@@ -391,14 +400,17 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
     // every thread of the block sums some of the (mt, lane) groups over the waves, tile by tile
     for (int grp = threadIdx.x; grp < MT * 64; grp += blockDim.x) {
         const int l2 = grp & 63, mt = grp >> 6;
+        if (HALF && (l2 & 40)) continue;
         f32x4_t v[NTB];
 #pragma unroll
         for (int nt = 0; nt < NTB; ++nt) {
-            if (waves > 1) {
+            if (waves > 1 || HALF) {
                 const int e = ((nt * MT + mt) * 64 + l2) * 4;
                 v[nt] = *(f32x4_t*)(red + e);
+                if (HALF) v[nt] += *(f32x4_t*)(red + e + 160);
                 for (int w = 1; w < waves; ++w) {
-                    const f32x4_t o = *(f32x4_t*)(red + (size_t)w * PER_WAVE + e);
+                    f32x4_t o = *(f32x4_t*)(red + (size_t)w * PER_WAVE + e);
+                    if (HALF) o += *(f32x4_t*)(red + (size_t)w * PER_WAVE + e + 160);
                     v[nt][0] += o[0]; v[nt][1] += o[1]; v[nt][2] += o[2]; v[nt][3] += o[3];
                 }
             } else {
@@ -452,14 +464,23 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
             const int n0 = tile_row[nt] + (l2 >> 4) * 4;
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                if (n0 + i < N) st_f(Y, y_dt, (size_t)mrow * N + n0 + i, v[nt][i] * rs);
+                if (n0 + i < N) {
+                    float y = v[nt][i] * rs;
+                    if (res.act == 1) {
+                        y = fmaxf(y, 0.f);
+                        y *= y;
+                    } else if (res.act == 2) {
+                        y = gelu_tanh_f(y);
+                    }
+                    st_f(Y, y_dt, (size_t)mrow * N + n0 + i, y);
+                }
         }
     }
 }
 
-static const SkResidual SK_NO_RESIDUAL = {0, nullptr, ILLM_BF16, nullptr, nullptr, nullptr, 0, 0.f, 0.f, 0.f, 0, {}};
+static const SkResidual SK_NO_RESIDUAL = {0, nullptr, ILLM_BF16, nullptr, nullptr, nullptr, 0, 0.f, 0.f, 0.f, 0, {}, 0};
 
-template <int MT, int NTB, int U, int MODE = SK_PLAIN, bool TILED = false, bool ONE_SHOT = false>
+template <int MT, int NTB, int U, int MODE = SK_PLAIN, bool TILED = false, bool ONE_SHOT = false, bool HALF = false>
 static int launch_skinny(const void* X, const void* W, void* Y, int y_dt, int M, int N, int K,
                          int waves, hipStream_t st, SkRope rope = SkRope(),
                          SkResidual res = SK_NO_RESIDUAL) {
@@ -468,10 +489,10 @@ static int launch_skinny(const void* X, const void* W, void* Y, int y_dt, int M,
     constexpr int REGS = (ONE_SHOT ? 1 : 2) * (NTB + MT) * U * 4 + NTB * 8 + NTB * MT * 4 + 40;
     constexpr int MAXW = REGS <= 128 ? 16 : (REGS <= 256 ? 8 : 4);
     waves = waves > MAXW ? MAXW : waves;
-    const int rows_per_block = DUAL ? 8 * NTB : 16 * NTB;
+    const int rows_per_block = DUAL ? 8 * NTB : HALF ? 8 : 16 * NTB;
     const int blocks = (N + rows_per_block - 1) / rows_per_block;
     const size_t smem = (size_t)waves * NTB * ((!TILED && U > MT) ? U : MT) * 1024 + 64;
-    hipLaunchKernelGGL((gemm_skinny_kernel<MT, NTB, U, MAXW, MODE, TILED, ONE_SHOT>), dim3(blocks), dim3(64 * waves),
+    hipLaunchKernelGGL((gemm_skinny_kernel<MT, NTB, U, MAXW, MODE, TILED, ONE_SHOT, HALF>), dim3(blocks), dim3(64 * waves),
                        smem, st, (const bf16_t*)X, (const bf16_t*)W, Y, y_dt, M, N, K, rope, res);
     return illm_launch_status();
 }
@@ -499,7 +520,7 @@ static int clamp_waves(int w, int ntb, int mt, int u, int K) {
 // W a block, u * 64 bytes of a W row per wave iteration, waves per block (clamped to what LDS
 // and K allow).  Up to 16 rows of X take ntb = 1, more take 2; u = 4 (measured best).
 static int skinny_from_matrix(const void* X, const void* W, void* Y, int y_dt, int M,
-                              int N, int K, int ntb, int u, int waves, void* stream) {
+                              int N, int K, int ntb, int u, int waves, const SkResidual& res, void* stream) {
     if (M <= 0 || M > 64 || N <= 0 || K <= 0 || (K % 8) || !illm_dtype_ok(y_dt))
         return ILLM_ERR_ARG;
     hipStream_t st = (hipStream_t)stream;
@@ -507,7 +528,7 @@ static int skinny_from_matrix(const void* X, const void* W, void* Y, int y_dt, i
     waves = clamp_waves(waves, ntb, mt, u, K);
 #define GO(MT_, NTB_, U_)                                                                     \
     if (mt == MT_ && ntb == NTB_ && u == U_)                                                  \
-        return launch_skinny<MT_, NTB_, U_>(X, W, Y, y_dt, M, N, K, waves, st)
+        return launch_skinny<MT_, NTB_, U_>(X, W, Y, y_dt, M, N, K, waves, st, SkRope(), res)
     GO(1, 1, 4); GO(2, 2, 4); GO(3, 2, 4); GO(4, 2, 4);
 #undef GO
     return ILLM_ERR_ARG;
@@ -522,23 +543,31 @@ static bool scale_args_ok(const float* ssq, int parts, int M) {
 // Wt != null: the tiled copy of W (see the kernel), used for M <= 16 and K % 32 == 0.
 static bool use_tiled(const void* Wt, int M, int K) { return Wt && M <= 16 && K % 32 == 0; }
 
-extern "C" int illm_gemm_skinny_bf16(const void* X, const void* W, const void* Wt, void* Y, int y_dt,
-                                     int M, int N, int K, const float* ssq, int parts, float eps,
-                                     int waves_wanted, void* stream) {
-    if (M <= 0 || M > 64 || N <= 0 || K <= 0 || (K % 8) || !illm_dtype_ok(y_dt) ||
-        !scale_args_ok(ssq, parts, M))
-        return ILLM_ERR_ARG;
+static int SK_HALF = -1;              // tuning and tests: 0 never, 1 wherever it can be, -1 the rule below
+extern "C" void illm_set_skinny_half(int on) { SK_HALF = on; }
+
+static int skinny_plain(const void* X, const void* W, const void* Wt, void* Y, int y_dt, int M, int N, int K,
+                        const SkResidual& res, int waves_wanted, void* stream) {
     const int ntb = M <= 16 ? 1 : 2, u = 4;
     const int blocks = (N + 16 * ntb - 1) / (16 * ntb);
     const int on_chip = use_tiled(Wt, M, K) ? SK_WAVES_ON_CHIP_TILED : SK_WAVES_ON_CHIP;
     int waves = waves_wanted > 0 ? waves_wanted : (on_chip + blocks / 2) / blocks;
     waves = waves < 1 ? 1 : waves;
-    if (!ssq && !use_tiled(Wt, M, K))
-        return skinny_from_matrix(X, W, Y, y_dt, M, N, K, ntb, u, waves, stream);
-    SkResidual res = SK_NO_RESIDUAL;
-    res.ssq = ssq; res.parts = parts; res.eps = eps;
+    if (!res.ssq && !use_tiled(Wt, M, K))
+        return skinny_from_matrix(X, W, Y, y_dt, M, N, K, ntb, u, waves, res, stream);
     waves = clamp_waves(waves, 1, 1, 4, K);
     if (use_tiled(Wt, M, K)) {
+        // Half a tile a block where the tiles do not fill the compute units (us with whole / half tiles at 8 rows: 2048 x
+        // 8192 14.9 / 11.0, x 4096 8.6 / 7.3, x 2048 5.7 / 5.0, x 512 3.6 / 3.5, x 64 2.9 / 3.1; 512 x 8192 12.3 / 9.0; at 1 row
+        // 2048 x 8192 12.8 / 8.5), not where they do (2560 x 4096 9.6 / 9.9, 4096 x 4096 9.4 / 10.8: X is read twice as often).
+        const bool half = M <= 8 && (SK_HALF >= 0 ? SK_HALF == 1 : blocks <= 128 && K >= 1024);
+        if (half) {
+            const int halves = (N + 7) / 8;
+            int wh = waves_wanted > 0 ? waves_wanted : (on_chip + halves / 2) / halves;
+            wh = clamp_waves(wh < 2 ? 2 : wh, 1, 1, 4, (K + 1) / 2);
+            return launch_skinny<1, 1, 4, SK_PLAIN, true, false, true>(X, Wt, Y, y_dt, M, N, K, wh, (hipStream_t)stream,
+                                                                       SkRope(), res);
+        }
         // with many tiles (the head) a block takes two: X is read half as often
         if (two_tiles_a_block(blocks)) {
             const int blocks2 = (blocks + 1) / 2;
@@ -551,6 +580,28 @@ extern "C" int illm_gemm_skinny_bf16(const void* X, const void* W, const void* W
                                                       (hipStream_t)stream, SkRope(), res);
     }
     return launch_skinny<1, 1, 4>(X, W, Y, y_dt, M, N, K, waves, (hipStream_t)stream, SkRope(), res);
+}
+
+extern "C" int illm_gemm_skinny_bf16(const void* X, const void* W, const void* Wt, void* Y, int y_dt,
+                                     int M, int N, int K, const float* ssq, int parts, float eps,
+                                     int waves_wanted, void* stream) {
+    if (M <= 0 || M > 64 || N <= 0 || K <= 0 || (K % 8) || !illm_dtype_ok(y_dt) ||
+        !scale_args_ok(ssq, parts, M))
+        return ILLM_ERR_ARG;
+    SkResidual res = SK_NO_RESIDUAL;
+    res.ssq = ssq; res.parts = parts; res.eps = eps;
+    return skinny_plain(X, W, Wt, Y, y_dt, M, N, K, res, waves_wanted, stream);
+}
+
+// The same of at most 16 rows with an activation on the float32 sums: act 1 relu(y)^2, 2 gelu(y) by tanh.
+extern "C" int illm_gemm_skinny_act(const void* X, const void* W, const void* Wt, void* Y, int y_dt, int M, int N, int K,
+                                    const float* ssq, int parts, float eps, int act, void* stream) {
+    if (M <= 0 || M > 16 || N <= 0 || K <= 0 || (K % 8) || !illm_dtype_ok(y_dt) || !scale_args_ok(ssq, parts, M) ||
+        act < 0 || act > 2)
+        return ILLM_ERR_ARG;
+    SkResidual res = SK_NO_RESIDUAL;
+    res.ssq = ssq; res.parts = parts; res.eps = eps; res.act = act;
+    return skinny_plain(X, W, Wt, Y, y_dt, M, N, K, res, 0, stream);
 }
 
 // The product whose parts of W read rows of X of their own: X [planes][M][K], W's rows ends[p - 1] .. ends[p] - 1

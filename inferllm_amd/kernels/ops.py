@@ -1094,6 +1094,26 @@ def gemm_skinny_bf16(x, w, out_dtype: torch.dtype) -> torch.Tensor:
     return y
 
 
+_LINEAR_ACTS = {"relu_squared": 1, "gelu_tanh": 2}
+
+
+def linear_act(x, w, act: str) -> torch.Tensor:
+    """An activation of x . w^T: up to 16 bfloat16 rows in the product's kernel, on the float32 sums (a kernel of its
+    own takes 4.5 us a layer of a decode step); else the product, then the activation."""
+    code = _LINEAR_ACTS.get(act, 0)
+    M, K = x.shape
+    if not (code and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.shape[1] == K
+            and 1 <= M <= SKINNY_BEST_ROWS and K % 8 == 0 and plain_weight(w).is_cuda):
+        return globals()[act](linear(x, w))
+    xt, ssq, parts, eps = _operand(x)
+    w, wt = _w(w)
+    _gpu(xt, w)
+    y = torch.empty((M, w.shape[0]), dtype=torch.bfloat16, device=xt.device)
+    _check(_lib().illm_gemm_skinny_act(_p(xt), _p(w), wt, _p(y), _code(y), M, w.shape[0], K, ssq, parts, eps, code,
+                                       _stream()), "linear_act")
+    return y
+
+
 QKV_ROPE_WAVES = 0       # waves per block of the fused kernel; 0: the kernel's own choice
 GATE_UP_WAVES = 0        # the same for the fused gate|up product
 PLAIN_WAVES = 0          # and for the plain few-rows product

@@ -109,9 +109,10 @@ class DenseActivation(FeedForward):
         return (("plain", self.w_down, {}),)
 
     def forward(self, h, ctx: StepContext):
-        act = getattr(ops, _ACTIVATIONS[self.activation])
-        z = ops.linear(h, self.w_up)
-        return ops.linear(act(z) if self.act is None else act(z, self.act), self.w_down)
+        act = _ACTIVATIONS[self.activation]
+        z = (ops.linear_act(h, self.w_up, act) if self.act is None
+             else getattr(ops, act)(ops.linear(h, self.w_up), self.act))
+        return ops.linear(z, self.w_down)
 
 
 @register_part("feed_forward", "clamped_gated")
@@ -256,6 +257,6 @@ class RoutedExperts(FeedForward):
         shared = None
         if self.Fs:
             inner = (ops.gate_up_silu(h, self.w_shared_gate_up) if self.gated
-                     else ops.relu_squared(ops.linear(h, self.w_shared_gate_up)))
+                     else ops.linear_act(h, self.w_shared_gate_up, "relu_squared"))
             shared = ops.linear(inner, self.w_shared_down)
         return ops.moe_combine(h, idx, weight, y, self.n_real, shared, self.w_sg)

@@ -560,6 +560,40 @@ def test_gemm_f32_split(M, N, K, S):
     assert not ops().gemm_f32_split_fits(rnd(M, K + 16).to(DEV), rnd(N, K + 16).to(DEV))
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (8, 24, 96), (3, 2048, 1056), (8, 2040, 4096), (7, 520, 2048), (5, 100, 1024),
+                                   (8, 2048, 8192), (9, 2048, 1024), (16, 40, 64)])
+def test_skinny_half_tiles_and_activations(M, N, K):
+    """Products of up to 8 rows with half a tile a block (odd numbers of k-steps, a last tile of few rows, a block's waves
+    more than its pieces) against whole tiles and 64 bits, a norm taken by the product, and activations on its sums."""
+    x, w = rnd(M, K, seed=1).to(torch.bfloat16), rnd(N, K, seed=2).to(torch.bfloat16)
+    tiled = ops().decode_weight(w.to(DEV), "plain", True)
+    assert isinstance(tiled, ops().Weight)
+    want = R.linear(x, w, torch.float64)
+    bound = 2.0 ** -23 * (K / 32 + 32) * (x.double().abs() @ w.double().abs().t())
+    lib = ops()._lib()
+    acts = {"relu_squared": lambda t: t.clamp(min=0) ** 2,
+            "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh")}
+    normed = ops().NormedRows(x.float().to(DEV), torch.ones(K, device=DEV), 1e-5, torch.bfloat16, x.to(DEV),
+                              (x.float() ** 2).view(M, K // 32, 32).sum(-1).contiguous().to(DEV))
+    scale = torch.rsqrt((x.double() ** 2).mean(1, keepdim=True) + 1e-5)
+    try:
+        for half in (0, 1, -1):
+            lib.illm_set_skinny_half(half)
+            got = ops().linear(x.to(DEV), tiled, torch.float32).double().cpu()
+            assert bool(((got - want).abs() <= bound).all())
+            got = ops().linear(normed, tiled, torch.float32).double().cpu()
+            assert bool(((got - want * scale).abs() <= 2 * bound * scale + 1e-12).all())
+            for name, act in acts.items():
+                for rows in (x.to(DEV), normed):
+                    z = want * (scale if rows is normed else 1.0)
+                    close(ops().linear_act(rows, tiled, name), act(z), torch.bfloat16, scale=float(act(z).abs().max()))
+                    close(ops().linear_act(rows, w.to(DEV), name), act(z), torch.bfloat16, scale=float(act(z).abs().max()))
+    finally:
+        lib.illm_set_skinny_half(-1)
+    many = rnd(40, K, seed=3).to(torch.bfloat16).to(DEV)              # beyond the few rows: a kernel of its own
+    assert torch.equal(ops().linear_act(many, tiled, "gelu_tanh"), ops().gelu_tanh(ops().linear(many, tiled)))
+
+
 def test_zero_slot():
     """A slot's row of every state tensor to zeros: 19 tensors (more than a launch takes), rows of 1 byte to 100 KB
     that begin on and off 16 bytes, and nothing beside them."""
