@@ -587,8 +587,10 @@ attn_cap_rows_mfma_kernel(const void* __restrict__ q, int q_stride, void* __rest
 // a lane holds its weights: key 16 s + 8 b + 4 h + i at place 16 s + 8 h + 4 b + i.
 typedef __bf16 cap_bf16x8_t __attribute__((ext_vector_type(8)));
 
-template <int KT, int VT>
-__global__ void __launch_bounds__(256, 2)
+// GROUPS 2: eight waves, of which the second four take every second tile of keys for the same rows, and add what they
+// have at the end: half as many turns behind each other for the block that the launch waits for.
+template <int KT, int VT, int GROUPS>
+__global__ void __launch_bounds__(256 * GROUPS, 2)
 attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out,
                           const int32_t* __restrict__ cu, const int32_t* __restrict__ seq_slot,
                           const int32_t* __restrict__ seq_start, const bf16_t* __restrict__ kcache,
@@ -601,8 +603,12 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
     constexpr int DKP = 32 * KT, DVP = 32 * VT, KLD = DKP + 8, VLD = MK + 8;
     constexpr int KP = (MK * DKP / 8 + 255) / 256;             // 16-byte pieces of a key tile a thread brings
     constexpr int VP = ((MK / 2) * (DVP / 8) + 255) / 256;     // pairs of keys x 8 value dims a thread brings
-    __shared__ __attribute__((aligned(16))) bf16_t ks[MK * KLD];
-    __shared__ __attribute__((aligned(16))) bf16_t vs[DVP * VLD];
+    constexpr int PART = MK * KLD + DVP * VLD;                 // a group's tile
+    constexpr int EXCHANGE = GROUPS > 1 ? (4 * 64 * 16 * 4 + 4 * 64 * 8) / 2 : 0;
+    __shared__ __attribute__((aligned(16))) bf16_t tiles[GROUPS * PART > EXCHANGE ? GROUPS * PART : EXCHANGE];
+    const int grp = GROUPS > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 256)) : 0;
+    bf16_t* const ks = tiles + grp * PART;
+    bf16_t* const vs = ks + MK * KLD;
     const int b = blockIdx.z, h = blockIdx.y;
     const int start = cu[b], len = cu[b + 1] - start;
     const int q0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * MQ;
@@ -610,7 +616,7 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
     const int pos0 = seq_start[b], slot = seq_slot[b];
     const int total = pos0 + len;
     const int kvh = h / (nh / nkv);
-    const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
+    const int tid = threadIdx.x & 255, lane = tid & 63, wave = wave_index() & 3;
     const int col = lane & 31, half = lane >> 5;
     const int qrow = q0 + 32 * wave + col;
     const int qpos = pos0 + qrow;
@@ -691,16 +697,20 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
     const int wq_lo = pos0 + q0 + 32 * wave, wq_hi = wq_lo + 31;
     const int wc_lo = chunk > 0 ? (wq_lo / chunk) * chunk : 0;
     const int c_lo = chunk > 0 ? (qpos / chunk) * chunk : 0;
-    const int k_last = k_lo + ((k_hi - 1 - k_lo) / MK) * MK;
     const int k_first = min(k_lo, ((keep + MK - 1) / MK) * MK);    // tiles [0, k_first): the kept tokens'
-    int k_next = k_first > 0 ? 0 : k_lo;
-    fetch(k_next);
-    for (int k0 = k_next; k0 < k_hi; k0 = k_next) {
+    const int n_first = k_first / MK, n_tiles = n_first + (k_hi - k_lo + MK - 1) / MK;
+    auto tile_at = [&](int n) __attribute__((always_inline)) {     // (past the end: the last again, not used)
+        n = min(n, n_tiles - 1);
+        return n < n_first ? n * MK : k_lo + (n - n_first) * MK;
+    };
+    fetch(tile_at(grp));
+    for (int n = grp; n < n_tiles + grp; n += GROUPS) {
+        const int k0 = tile_at(n);
         __syncthreads();
         stage();
         __syncthreads();
-        k_next = k0 + MK == k_first ? k_lo : k0 + MK;
-        fetch(min(k_next, k_last));               // (unconditional: the last tile is asked for twice)
+        fetch(tile_at(n + GROUPS));
+        if (GROUPS > 1 && n >= n_tiles) continue;
         if (!wave_has_rows || k0 > wq_hi || k0 + MK - 1 < wc_lo ||
             (window > 0 && k0 >= keep && k0 + MK - 1 <= wq_lo - window))
             continue;
@@ -760,6 +770,36 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
             }
         }
     }
+    if constexpr (GROUPS > 1) {
+        static_assert(GROUPS == 2, "two groups");
+        float* const ex = (float*)tiles;                       // [wave][16][lane], then (m, l) a lane
+        float2* const ml = (float2*)(ex + 4 * 64 * 16);
+        __syncthreads();
+        if (grp) ml[wave * 64 + lane] = make_float2(m_i, l_i);
+        float own = 1.f, other = 0.f;
+#pragma unroll
+        for (int t = 0; t < VT; ++t) {
+            if (grp) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) ex[(wave * 16 + v) * 64 + lane] = o[t][v];
+            }
+            __syncthreads();
+            if (!grp) {
+                if (t == 0) {
+                    const float2 x = ml[wave * 64 + lane];
+                    const float m_new = fmaxf(m_i, x.x);
+                    own = m_i == NEG_INF ? 0.f : __expf(m_i - m_new);
+                    other = x.x == NEG_INF ? 0.f : __expf(x.x - m_new);
+                    l_i = l_i * own + x.y * other;
+                    m_i = m_new;
+                }
+#pragma unroll
+                for (int v = 0; v < 16; ++v) o[t][v] = o[t][v] * own + ex[(wave * 16 + v) * 64 + lane] * other;
+            }
+            __syncthreads();
+        }
+        if (grp) return;
+    }
     if (qrow < len) {
         if (sink) add_sink(sink[h], m_i, l_i);
         const float inv = 1.0f / l_i;
@@ -790,10 +830,12 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
 // cores' float32 instruction also for bfloat16 storage.
 static int g_attn_cap_mfma = 1;
 extern "C" void illm_set_attn_cap_mfma(int on) { g_attn_cap_mfma = on < 0 || on > 2 ? 1 : on; }
+static int g_attn_cap_groups = 0;
+extern "C" void illm_set_attn_cap_groups(int n) { g_attn_cap_groups = n == 1 || n == 2 ? n : 0; }
 static int g_attn_cap_heads = 0;
 extern "C" void illm_set_attn_cap_heads(int n) { g_attn_cap_heads = (n == 1 || n == 2 || n == 4) ? n : 0; }
 
-extern "C" int illm_attn_cap_rows(const void* q, int q_stride, void* out, int dt, const int32_t* cu,
+extern "C" int illm_attn_cap_rows_of(const void* q, int q_stride, void* out, int dt, const int32_t* cu,
                                   const int32_t* seq_slot, const int32_t* seq_start,
                                   const void* kcache, const void* vcache, const int32_t* page_table,
                                   int table_stride, int page_size, int ring, int n_seqs, int max_rows,
@@ -801,7 +843,7 @@ extern "C" int illm_attn_cap_rows(const void* q, int q_stride, void* out, int dt
                                   const float* slopes, int chunk, const void* gate, int gate_stride,
                                   int gate_off, int gate_heads, float* lse, int keep, int kept,
                                   int own_stride, int own_k, int own_v_stride, int own_v, const float* sink,
-                                  void* stream) {
+                                  int rows, void* stream) {
     if (keep < 0 || kept < 0 || (keep > 0 && (window <= 0 || chunk > 0)) || own_stride < 0 ||
         (own_stride && (own_k < 0 || own_v < 0 || own_k + nkv * dk > own_stride || own_v + nkv * dv > own_v_stride)))
         return ILLM_ERR_ARG;
@@ -828,8 +870,17 @@ extern "C" int illm_attn_cap_rows(const void* q, int q_stride, void* out, int dt
         const bool bf16_rows = dt == ILLM_BF16 && g_attn_cap_mfma == 1 && dk % 8 == 0 && dv % 8 == 0 && q_stride % 8 == 0 &&
                                own_stride % 8 == 0 && own_k % 8 == 0 && own_v_stride % 8 == 0 && own_v % 8 == 0;
         if (bf16_rows) {
-#define GOB(KT_, VT_)                                                                              \
-    hipLaunchKernelGGL((attn_cap_rows_bf16_kernel<KT_, VT_>), grid, dim3(256), 0, (hipStream_t)stream, \
+            // Two groups of waves where the blocks that have rows are too few to fill the chip by themselves (at most
+            // rows / 128 + sequences a head); us with one / two groups: 8 sequences of 1,024 to 61 rows, 16 heads of 128 in
+            // chunks 87 / 66, 32 heads 94 / 112; 4 of 500 to 100, 32 heads 46 / 34; one of 200 22 / 19; one of 4,000, 16 heads
+            // 233 / 246; 16 of 128, 32 heads 22 / 31.  Heads of up to 64: 8 of 1,024 to 61 74 / 48, one of 4,000 167 / 141, 64
+            // of 300 85 / 102.
+            const long long tiles = (max_rows + MQ - 1) / MQ * (long long)n_seqs;
+            const long long blocks = (rows > 0 && rows / MQ + n_seqs < tiles ? rows / MQ + n_seqs : tiles) * nh;
+            const int groups = g_attn_cap_groups ? g_attn_cap_groups : blocks < (dk <= 64 && dv <= 64 ? 1025 : 512) ? 2 : 1;
+#define GOB(KT_, VT_) do { if (groups == 2) GOB_G(KT_, VT_, 2); else GOB_G(KT_, VT_, 1); } while (0)
+#define GOB_G(KT_, VT_, G_)                                                                        \
+    hipLaunchKernelGGL((attn_cap_rows_bf16_kernel<KT_, VT_, G_>), grid, dim3(256 * G_), 0, (hipStream_t)stream, \
                        (const bf16_t*)q, q_stride, (bf16_t*)out, cu, seq_slot, seq_start, (const bf16_t*)kcache, \
                        (const bf16_t*)vcache, page_table, table_stride, page_size, ring, nh, nkv, dk, dv, scale, cap, \
                        window, slopes, chunk, (const bf16_t*)gate, gate_stride, gate_off, gate_heads, lse, keep, kept, \
@@ -841,6 +892,7 @@ extern "C" int illm_attn_cap_rows(const void* q, int q_stride, void* out, int dt
                           case 3: GOB_V(3) break; default: GOB_V(4) break; }
 #undef GOB_V
 #undef GOB
+#undef GOB_G
         } else if (dt == ILLM_BF16) { GO_K(ILLM_BF16) } else { GO_K(ILLM_F32) }
 #undef GO_K
 #undef GO_V
@@ -857,6 +909,21 @@ extern "C" int illm_attn_cap_rows(const void* q, int q_stride, void* out, int dt
                        page_table, table_stride, page_size, ring, nh, nkv, dk, dv, scale, cap, window, slopes,
                        chunk, gate, gate_stride, gate_off, gate_heads, lse, keep, kept, own_stride, own_k, own_v_stride, own_v, sink);
     return illm_launch_status();
+}
+
+extern "C" int illm_attn_cap_rows(const void* q, int q_stride, void* out, int dt, const int32_t* cu,
+                                  const int32_t* seq_slot, const int32_t* seq_start,
+                                  const void* kcache, const void* vcache, const int32_t* page_table,
+                                  int table_stride, int page_size, int ring, int n_seqs, int max_rows,
+                                  int nh, int nkv, int dk, int dv, float scale, float cap, int window,
+                                  const float* slopes, int chunk, const void* gate, int gate_stride,
+                                  int gate_off, int gate_heads, float* lse, int keep, int kept,
+                                  int own_stride, int own_k, int own_v_stride, int own_v, const float* sink,
+                                  void* stream) {
+    return illm_attn_cap_rows_of(q, q_stride, out, dt, cu, seq_slot, seq_start, kcache, vcache, page_table, table_stride,
+                                 page_size, ring, n_seqs, max_rows, nh, nkv, dk, dv, scale, cap, window, slopes, chunk, gate,
+                                 gate_stride, gate_off, gate_heads, lse, keep, kept, own_stride, own_k, own_v_stride, own_v,
+                                 sink, 0, stream);
 }
 
 // The keys a single token sees, numbered without a gap: with `keep` first tokens before the window the

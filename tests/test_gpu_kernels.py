@@ -594,6 +594,64 @@ def test_skinny_half_tiles_and_activations(M, N, K):
     assert torch.equal(ops().linear_act(many, tiled, "gelu_tanh"), ops().gelu_tanh(ops().linear(many, tiled)))
 
 
+@pytest.mark.parametrize("d,window,chunk,keep", [(128, 0, 0, 0), (128, 0, 96, 0), (64, 70, 0, 0), (32, 40, 0, 33), (40, 0, 0, 0)])
+def test_attn_cap_rows_groups(d, window, chunk, keep):
+    """Prompts' attention with the keys' tiles in turn by two groups of waves against one group (the same sums in
+    another order): odd and even numbers of tiles, a sequence of one row, masks that leave a group without keys, sinks
+    and the softmax's sums."""
+    nh, nkv, lens = 4, 2, [1, 31, 33, 128, 200, 7]
+    T, B = sum(lens), len(lens)
+    q = rnd(T, (nh + 2 * nkv) * d, seed=1).to(torch.bfloat16).to(DEV)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    slot, start = torch.arange(B, dtype=torch.int32, device=DEV), torch.zeros(B, dtype=torch.int32, device=DEV)
+    cache = torch.zeros(1, nkv, 64, d, dtype=torch.bfloat16, device=DEV)
+    table = torch.zeros(B, 4, dtype=torch.int32, device=DEV)
+    slopes, sink = rnd(nh, seed=2).abs().to(DEV) * 0.1, rnd(nh, seed=3).to(DEV)
+    lib, got = ops()._lib(), []
+    try:
+        for groups in (1, 2, 0):
+            lib.illm_set_attn_cap_groups(groups)
+            lse = torch.empty(T, nh, device=DEV)
+            out = ops().attn_cap_rows(q, cu, slot, start, cache, cache, table, 64, 0, B, max(lens), nh, nkv, d, d, d ** -0.5,
+                                      0.0, window, slopes=slopes, chunk=chunk, lse=lse, keep=keep, kept=0,
+                                      own=(nh * d, (nh + nkv) * d), sink=sink)
+            got.append((out.float(), lse))
+    finally:
+        lib.illm_set_attn_cap_groups(0)
+    for out, lse in got[1:]:
+        assert float((out - got[0][0]).abs().max()) <= 2.0 ** -8 * float(got[0][0].abs().max())
+        assert float((lse - got[0][1]).abs().max()) <= 1e-5 * float(got[0][1].abs().max())
+
+
+@pytest.mark.parametrize("dt,taps,shape", [(torch.bfloat16, 4, (2, 4, 8, 16)), (torch.float32, 3, (1, 2, 4, 36)), (torch.bfloat16, 2, (2, 2, 6, 20))])
+def test_ssm_prepare_rows(dt, taps, shape):
+    """A state-space mixer's inputs of prompts, four channels a thread, against the kernel of a channel a thread (which
+    odd offsets still take): the same bits, sequences of 1 to 40 rows, tails of earlier steps."""
+    G, H, N, dv = shape
+    lens, C = [1, 2, 40, 3, 17], H * dv + 2 * G * N
+    T = sum(lens)
+    slot = torch.cat([torch.full((n,), 4 - i, dtype=torch.int32) for i, n in enumerate(lens)]).to(DEV)
+    cols = rnd(T, C + H, seed=1)
+    wide, odd = torch.zeros(T, C + H + 8), torch.zeros(T, C + H + 8)
+    wide[:, 4:4 + C + H], odd[:, 3:3 + C + H] = cols, cols
+    wide[:, 4 + C:4 + C + H], odd[:, 3 + C:3 + C + H] = cols[:, C:], cols[:, C:]
+    tail = rnd(5, taps - 1, C, seed=2).to(dt).to(DEV)
+    w, b, a, db = (t.to(DEV) for t in (rnd(C, taps, seed=3), rnd(C, seed=4), rnd(H, seed=5), rnd(H, seed=6)))
+    run = lambda U, off: ops().ssm_prepare(U.to(dt).to(DEV), off, off + C, w, b, tail, slot, a, db, G, H, N, dv)
+    for x, y in zip(run(wide, 4), run(odd, 3)):
+        assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("E", [4, 96, 1024, 1028, 4096, 8196, 33])
+def test_embed_widths(E):
+    """Rows of the table by four columns a thread, and one (E odd)."""
+    for dt in DTYPES:
+        table = rnd(50, E, seed=1).to(dt).to(DEV)
+        ids = torch.tensor([0, 49, 7, 7, 60, -1], dtype=torch.int32, device=DEV)
+        want = table[ids.long().clamp(0, 49)].float() * 0.5
+        assert torch.equal(ops().embed(ids, table, 0.5), want)
+
+
 def test_zero_slot():
     """A slot's row of every state tensor to zeros: 19 tensors (more than a launch takes), rows of 1 byte to 100 KB
     that begin on and off 16 bytes, and nothing beside them."""
