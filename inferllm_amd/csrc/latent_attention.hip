@@ -148,12 +148,41 @@ latent_pack_kernel(const void* __restrict__ y, int dt, int ncols, const void* __
     }
 }
 
+// bfloat16, every width a multiple of 8: 16 bytes a thread and turn (2,964 rows of 16 heads of 192: 57 us an element).
+__global__ void __launch_bounds__(256)
+latent_pack_vec8_kernel(const bf16_t* __restrict__ y, int ncols, const bf16_t* __restrict__ kvu,
+                        const bf16_t* __restrict__ kr, bf16_t* __restrict__ out, int H, int dn, int dr, int dv, int P) {
+    const size_t t = blockIdx.x;
+    const int HP = H * P, dq = dn + dr;
+    const bf16_t* const kv = kvu + t * (size_t)(H * (dn + dv));
+    for (int e = threadIdx.x * 8; e < 3 * HP; e += 256 * 8) {
+        const int which = e / HP, rem = e - which * HP;
+        const int h = rem / P, d = rem - h * P;
+        const bf16_t* from = nullptr;
+        if (which == 0) {
+            if (d < dq) from = y + t * ncols + (size_t)h * dq + d;
+        } else if (which == 1) {
+            if (d < dn) from = kv + (size_t)h * dn + d;
+            else if (d < dq) from = kr + t * dr + (d - dn);
+        } else if (d < dv) {
+            from = kv + (size_t)H * dn + (size_t)h * dv + d;
+        }
+        *(uint4*)(out + t * (size_t)(3 * HP) + e) = from ? *(const uint4*)from : make_uint4(0, 0, 0, 0);
+    }
+}
+
 extern "C" int illm_latent_pack(const void* y, int dt, int ncols, const void* kvu, const void* kr,
                                 void* out, int T, int H, int dn, int dr, int dv, int P,
                                 void* stream) {
     if (T < 0 || H <= 0 || dn < 0 || dr < 0 || dv <= 0 || P < dn + dr || P < dv || !illm_dtype_ok(dt))
         return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
+    if (dt == ILLM_BF16 && (ncols | dn | dr | dv | P) % 8 == 0 &&
+        ((uintptr_t)y | (uintptr_t)kvu | (uintptr_t)kr | (uintptr_t)out) % 16 == 0) {
+        hipLaunchKernelGGL(latent_pack_vec8_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)y, ncols,
+                           (const bf16_t*)kvu, (const bf16_t*)kr, (bf16_t*)out, H, dn, dr, dv, P);
+        return illm_launch_status();
+    }
     hipLaunchKernelGGL(latent_pack_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, y, dt, ncols,
                        kvu, kr, out, H, dn, dr, dv, P);
     return illm_launch_status();
@@ -172,11 +201,35 @@ latent_gate_kernel(const void* __restrict__ attn, const void* __restrict__ y, in
     }
 }
 
+// bfloat16, dv and P multiples of 8: 16 bytes a thread and turn (2,964 rows of 2,048: 17 us an element).
+__global__ void __launch_bounds__(256)
+latent_gate_vec8_kernel(const bf16_t* __restrict__ attn, const bf16_t* __restrict__ y, int ncols, int gate_off,
+                        bf16_t* __restrict__ out, int H, int dv, int P) {
+    const size_t t = blockIdx.x;
+    for (int e = threadIdx.x * 8; e < H * dv; e += 256 * 8) {
+        const int h = e / dv, v = e - h * dv;
+        const float g = bf16_to_f32(y[t * ncols + gate_off + h]);
+        const uint4 a = *(const uint4*)(attn + t * (size_t)(H * P) + (size_t)h * P + v);
+        const float s = 1.0f / (1.0f + expf(-g));
+        const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+        uint32_t o[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            o[k] = pack_bf16x2(__uint_as_float(w[k] << 16) * s, __uint_as_float(w[k] & 0xffff0000u) * s);
+        *(uint4*)(out + t * (size_t)(H * dv) + e) = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+}
+
 extern "C" int illm_latent_gate(const void* attn, const void* y, int dt, int ncols, int gate_off,
                                 void* out, int T, int H, int dv, int P, void* stream) {
     if (T < 0 || H <= 0 || dv <= 0 || P < dv || gate_off < 0 || gate_off + H > ncols || !illm_dtype_ok(dt))
         return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
+    if (dt == ILLM_BF16 && (dv | P) % 8 == 0 && ((uintptr_t)attn | (uintptr_t)out) % 16 == 0) {
+        hipLaunchKernelGGL(latent_gate_vec8_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)attn,
+                           (const bf16_t*)y, ncols, gate_off, (bf16_t*)out, H, dv, P);
+        return illm_launch_status();
+    }
     hipLaunchKernelGGL(latent_gate_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, attn, y, dt,
                        ncols, gate_off, out, H, dv, P);
     return illm_launch_status();

@@ -79,6 +79,70 @@ ssm_prepare_kernel(const void* __restrict__ U, int dt, int u_stride, int x_off, 
     }
 }
 
+// The same of prompts (no tails written) where four channels lie together: a thread takes four channels of `rows` rows
+// one after the other, its weights in registers, every input read once (a thread a channel and row read the weights
+// and the rows before again for each: 2,964 rows of 6,144 channels 209 us).  grid (ceil(T / rows), ceil(C / 1024)).  The
+// taps are added in the same order: the same bits.
+template <int DT, int TAPS>
+__global__ void __launch_bounds__(256)
+ssm_prepare_rows_kernel(const void* __restrict__ U, int u_stride, int x_off, int dt_off, const float* __restrict__ conv_w,
+                        const float* __restrict__ conv_b, const void* __restrict__ tail,
+                        const int32_t* __restrict__ row_slot, const float* __restrict__ a_log,
+                        const float* __restrict__ dt_bias, float* __restrict__ qn, float* __restrict__ kn,
+                        float* __restrict__ vv, float* __restrict__ beta, float* __restrict__ dec, int T, int G, int H,
+                        int N, int dv, int rows) {
+    constexpr int K = TAPS - 1;
+    const int inner = H * dv, GN = G * N, C = inner + 2 * GN;
+    const int r0 = blockIdx.x * rows, r1 = min(r0 + rows, T);
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 4;
+    if (blockIdx.y == 0) {
+        for (int i = threadIdx.x; i < (r1 - r0) * H; i += 256) {
+            const int h = i % H;
+            const size_t r = r0 + i / H;
+            const float step = ls_softplus(ld_f(U, DT, r * u_stride + dt_off + h) + dt_bias[h]);
+            beta[r * H + h] = step;
+            dec[r * H + h] = expf(-expf(a_log[h]) * step);
+        }
+    }
+    if (c >= C) return;
+    float w[4 * TAPS];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) *(float4*)(w + 4 * j) = ((const float4*)(conv_w + (size_t)c * TAPS))[j];
+    const float4 bias = *(const float4*)(conv_b + c);
+    auto input = [&](int r) { return ld_f4(U, DT, ((size_t)r * u_stride + x_off + c) / 4); };
+    float4 x[TAPS], next = input(r0);
+    int had = -1;
+    float* to = c < inner ? vv + c : c < inner + GN ? kn + (c - inner) : qn + (c - inner - GN);
+    const size_t to_row = c < inner ? inner : GN;
+    for (int r = r0; r < r1; ++r) {
+        const int slot = row_slot[r];
+        if (slot != had) {                              // the inputs ahead of the sequence's first row here
+            int before = 0;
+            while (before < K && r - before - 1 >= 0 && row_slot[r - before - 1] == slot) ++before;
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                const int d = K - j;                    // tap j looks d tokens back
+                x[j] = d <= before ? input(r - d) : ld_f4(tail, DT, (((size_t)slot * K + (K - (d - before))) * C + c) / 4);
+            }
+            had = slot;
+        }
+        x[K] = next;
+        if (r + 1 < r1) next = input(r + 1);
+        float4 a = bias;
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) {
+            a.x = fmaf(w[j], x[j].x, a.x);
+            a.y = fmaf(w[TAPS + j], x[j].y, a.y);
+            a.z = fmaf(w[2 * TAPS + j], x[j].z, a.z);
+            a.w = fmaf(w[3 * TAPS + j], x[j].w, a.w);
+        }
+        *(float4*)(to + r * to_row) = make_float4(a.x * ls_sigmoid(a.x), a.y * ls_sigmoid(a.y), a.z * ls_sigmoid(a.z),
+                                                  a.w * ls_sigmoid(a.w));
+#pragma unroll
+        for (int j = 0; j < K; ++j) x[j] = x[j + 1];
+    }
+}
+
 extern "C" int illm_ssm_prepare(const void* U, int dt, int u_stride, int x_off, int dt_off,
                                 const float* conv_w, const float* conv_b, int taps, void* tail,
                                 const int32_t* row_slot, const float* a_log, const float* dt_bias,
@@ -90,6 +154,24 @@ extern "C" int illm_ssm_prepare(const void* U, int dt, int u_stride, int x_off, 
         return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
     const int C = H * dv + 2 * G * N, most = (C + 255) / 256;
+    const size_t unit = dt == ILLM_BF16 ? 8 : 16;
+    if (!update_tail && taps >= 2 && taps <= 4 && T > 16 && (H * dv) % 4 == 0 && (G * N) % 4 == 0 && u_stride % 4 == 0 &&
+        x_off % 4 == 0 && ((uintptr_t)U | (uintptr_t)tail) % unit == 0 &&
+        ((uintptr_t)conv_w | (uintptr_t)conv_b | (uintptr_t)qn | (uintptr_t)kn | (uintptr_t)vv) % 16 == 0) {
+        // as many rows a thread, up to 8, as leave about 1,024 blocks
+        const int by = (C + 1023) / 1024, rows = max(1, min(8, (int)((long long)T * by / 1024)));
+        const dim3 grid((T + rows - 1) / rows, by);
+#define ROWS(DT_, TAPS_)                                                                                              \
+    hipLaunchKernelGGL((ssm_prepare_rows_kernel<DT_, TAPS_>), grid, dim3(256), 0, (hipStream_t)stream, U, u_stride, x_off, \
+                       dt_off, conv_w, conv_b, tail, row_slot, a_log, dt_bias, qn, kn, vv, beta, dec, T, G, H, N, dv, rows)
+        if (dt == ILLM_BF16) {
+            if (taps == 4) ROWS(ILLM_BF16, 4); else if (taps == 3) ROWS(ILLM_BF16, 3); else ROWS(ILLM_BF16, 2);
+        } else {
+            if (taps == 4) ROWS(ILLM_F32, 4); else if (taps == 3) ROWS(ILLM_F32, 3); else ROWS(ILLM_F32, 2);
+        }
+#undef ROWS
+        return illm_launch_status();
+    }
     int nb = T >= 2048 ? 1 : (2048 + T - 1) / T;        // enough blocks to fill the chip when the rows are few
     nb = nb > most ? most : nb;
     hipLaunchKernelGGL(ssm_prepare_kernel, dim3(T, nb), dim3(256), 0, (hipStream_t)stream, U, dt, u_stride,
