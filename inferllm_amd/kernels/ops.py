@@ -867,8 +867,11 @@ CUT_SHORT_ROWS = 192     # up to these it is the faster way for every number of 
 def linear_cut_fits(x, w) -> bool:
     """Whether `linear_cut` takes these operands and is the faster way: 129 to 256 bfloat16 rows and a
     row-major matrix (its plain copy) with few rows for its length (K >= N, K a multiple of 64), both on
-    16-byte addresses and within a load's 32-bit offset."""
+    16-byte addresses and within a load's 32-bit offset; or float32 operands whose K `gemm_f32_split` cuts."""
     w = plain_weight(w)
+    if isinstance(x, torch.Tensor) and x.dtype == torch.float32 and w.dtype == torch.float32:
+        return (gemm_f32_split_fits(x, w) and gemm_f32_split_pays(x, w) and w.shape[0] % 4 == 0
+                and _lib().illm_gemm_f32_split_parts(x.shape[0], w.shape[0], w.shape[1]) > 1)
     if not (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and x.dim() == 2 and w.dim() == 2 and CUT_ROWS[0] <= x.shape[0] <= CUT_ROWS[1]
             and x.shape[1] == w.shape[1] and w.is_contiguous()):
