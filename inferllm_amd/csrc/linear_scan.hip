@@ -263,10 +263,11 @@ memory_gates_kernel(const void* __restrict__ U, int dt, int u_stride, int i_off,
         const float ig = ok ? cap * tanhf((ld_f(U, dt, row * u_stride + i_off + h) + bi) * inv_cap) : -INFINITY;
         const float fg = ok ? ls_log_sigmoid(cap * tanhf((ld_f(U, dt, row * u_stride + f_off + h) + bf) * inv_cap)) : 0.f;
         float m_before = 0.f, m_mine = 0.f;
-#pragma unroll
-        for (int l = 0; l < 64; ++l) {
-            const float fl = __shfl(fg, l, 64), il = __shfl(ig, l, 64);
-            const float m_new = fmaxf(fl + m, il);      // a lane beyond the sequence leaves m as it is
+        const int tokens = min(64, n - t0);             // (all 64 turns took 6 us of a single token's step)
+        for (int l = 0; l < tokens; ++l) {
+            const float fl = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(fg), l));
+            const float il = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ig), l));
+            const float m_new = fmaxf(fl + m, il);
             if (lane == l) { m_before = m; m_mine = m_new; }
             m = m_new;
         }
