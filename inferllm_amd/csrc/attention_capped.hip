@@ -590,7 +590,7 @@ typedef __bf16 cap_bf16x8_t __attribute__((ext_vector_type(8)));
 // GROUPS 2: eight waves, of which the second four take every second tile of keys for the same rows, and add what they
 // have at the end: half as many turns behind each other for the block that the launch waits for.
 template <int KT, int VT, int GROUPS>
-__global__ void __launch_bounds__(256 * GROUPS, 2)
+__global__ void __launch_bounds__(256 * GROUPS, KT <= 2 && VT <= 2 ? 4 : 2)      // (128 registers: 1,500 rows of 64 230 -> 199 us)
 attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out,
                           const int32_t* __restrict__ cu, const int32_t* __restrict__ seq_slot,
                           const int32_t* __restrict__ seq_start, const bf16_t* __restrict__ kcache,
@@ -635,30 +635,44 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
         }
     }
     illm_u32x4_t kreg[KP], vreg[VP][2];
-    auto key_at = [&](int kj) __attribute__((always_inline)) {
-        kj = min(kj, total - 1);                               // keys past the end: a valid row, masked below
-        return own_stride ? (size_t)(start + kj) * own_stride + own_k + (size_t)kvh * dk
-                          : cache_row_offset(page_table, table_stride, slot, kj, page_size, ring, nkv, kvh, dk, kept);
+    // A tile's keys lie behind each other: in the step's own rows, or in a page where pages are whole tiles (then the
+    // page is looked up once for the wave, and a tile ahead of its loads, not by every lane before each of its loads).
+    const bool by_page = !own_stride && page_size % MK == 0;
+    auto page_at = [&](int k0) __attribute__((always_inline)) {
+        if (!by_page) return 0;
+        int lp = k0 / page_size;
+        if (ring > 0 && lp >= kept) lp = kept + (lp - kept) % ring;
+        return page_table[(size_t)slot * table_stride + lp];
     };
-    auto value_at = [&](int kj) __attribute__((always_inline)) {
-        kj = min(kj, total - 1);
-        return own_stride ? (size_t)(start + kj) * own_v_stride + own_v + (size_t)kvh * dv
-                          : cache_row_offset(page_table, table_stride, slot, kj, page_size, ring, nkv, kvh, dv, kept);
-    };
-    auto fetch = [&](int k0) __attribute__((always_inline)) {
+    auto fetch = [&](int k0, int page) __attribute__((always_inline)) {
+        const int rows = min(MK, total - k0);                  // keys past the end: a valid row, masked below
+        const size_t page_row = ((size_t)page * nkv + kvh) * page_size + k0 % page_size;
+        const size_t kb = own_stride ? (size_t)(start + k0) * own_stride + own_k + (size_t)kvh * dk : page_row * dk;
+        const size_t vb = own_stride ? (size_t)(start + k0) * own_v_stride + own_v + (size_t)kvh * dv : page_row * dv;
+        const int ks_row = own_stride ? own_stride : dk, vs_row = own_stride ? own_v_stride : dv;
+        auto key_at = [&](int row) __attribute__((always_inline)) {
+            row = min(row, rows - 1);
+            return own_stride || by_page ? kb + (size_t)((uint32_t)row * (uint32_t)ks_row)
+                                         : cache_row_offset(page_table, table_stride, slot, k0 + row, page_size, ring, nkv, kvh, dk, kept);
+        };
+        auto value_at = [&](int row) __attribute__((always_inline)) {
+            row = min(row, rows - 1);
+            return own_stride || by_page ? vb + (size_t)((uint32_t)row * (uint32_t)vs_row)
+                                         : cache_row_offset(page_table, table_stride, slot, k0 + row, page_size, ring, nkv, kvh, dv, kept);
+        };
 #pragma unroll
         for (int i = 0; i < KP; ++i) {
             const int e = tid + 256 * i, row = e / (DKP / 8), d = 8 * (e % (DKP / 8));
             kreg[i] = zero4;
-            if (row < MK && d < dk) kreg[i] = *(const illm_u32x4_t*)(kcache + key_at(k0 + row) + d);
+            if (row < MK && d < dk) kreg[i] = *(const illm_u32x4_t*)(kcache + key_at(row) + d);
         }
 #pragma unroll
         for (int i = 0; i < VP; ++i) {
             const int e = tid + 256 * i, row = 2 * (e % (MK / 2)), d = 8 * (e / (MK / 2));
             vreg[i][0] = vreg[i][1] = zero4;
             if (d < dv) {
-                vreg[i][0] = *(const illm_u32x4_t*)(vcache + value_at(k0 + row) + d);
-                vreg[i][1] = *(const illm_u32x4_t*)(vcache + value_at(k0 + row + 1) + d);
+                vreg[i][0] = *(const illm_u32x4_t*)(vcache + value_at(row) + d);
+                vreg[i][1] = *(const illm_u32x4_t*)(vcache + value_at(row + 1) + d);
             }
         }
     };
@@ -703,13 +717,15 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
         n = min(n, n_tiles - 1);
         return n < n_first ? n * MK : k_lo + (n - n_first) * MK;
     };
-    fetch(tile_at(grp));
+    fetch(tile_at(grp), page_at(tile_at(grp)));
+    int page = page_at(tile_at(grp + GROUPS));
     for (int n = grp; n < n_tiles + grp; n += GROUPS) {
         const int k0 = tile_at(n);
         __syncthreads();
         stage();
         __syncthreads();
-        fetch(tile_at(n + GROUPS));
+        fetch(tile_at(n + GROUPS), page);
+        page = page_at(tile_at(n + 2 * GROUPS));
         if (GROUPS > 1 && n >= n_tiles) continue;
         if (!wave_has_rows || k0 > wq_hi || k0 + MK - 1 < wc_lo ||
             (window > 0 && k0 >= keep && k0 + MK - 1 <= wq_lo - window))
@@ -806,6 +822,8 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
         if (lse && half == 0) lse[(size_t)(start + qrow) * nh + h] = m_i + logf(l_i);
         const size_t ob = (size_t)(start + qrow) * nh * dv + (size_t)h * dv;
         const size_t gb = (size_t)(start + qrow) * gate_stride + gate_off + (size_t)h * (gate_heads ? 1 : dv);
+        // (a gate a value dim, on 8 bytes: four at once)
+        const bool gate4 = gate && !gate_heads && ((uintptr_t)gate % 8 | gate_stride % 4 | gate_off % 4) == 0;
 #pragma unroll
         for (int t = 0; t < VT; ++t)
 #pragma unroll
@@ -814,9 +832,16 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
                 if (d >= dv) continue;
                 float y[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    y[i] = o[t][4 * g + i] * inv;
-                    if (gate) y[i] *= 1.0f / (1.0f + expf(-bf16_to_f32(gate[gb + (gate_heads ? 0 : d + i)])));
+                for (int i = 0; i < 4; ++i) y[i] = o[t][4 * g + i] * inv;
+                if (gate4) {
+                    const uint2 u = *(const uint2*)(gate + gb + d);
+                    const uint32_t w[4] = {u.x << 16, u.x & 0xffff0000u, u.y << 16, u.y & 0xffff0000u};
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) y[i] *= 1.0f / (1.0f + expf(-__uint_as_float(w[i])));
+                } else if (gate) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        y[i] *= 1.0f / (1.0f + expf(-bf16_to_f32(gate[gb + (gate_heads ? 0 : d + i)])));
                 }
                 uint2 w;
                 w.x = pack_bf16x2(y[0], y[1]);
@@ -872,12 +897,14 @@ extern "C" int illm_attn_cap_rows_of(const void* q, int q_stride, void* out, int
         if (bf16_rows) {
             // Two groups of waves where the blocks that have rows are too few to fill the chip by themselves (at most
             // rows / 128 + sequences a head); us with one / two groups: 8 sequences of 1,024 to 61 rows, 16 heads of 128 in
-            // chunks 87 / 66, 32 heads 94 / 112; 4 of 500 to 100, 32 heads 46 / 34; one of 200 22 / 19; one of 4,000, 16 heads
-            // 233 / 246; 16 of 128, 32 heads 22 / 31.  Heads of up to 64: 8 of 1,024 to 61 74 / 48, one of 4,000 167 / 141, 64
+            // chunks 97 / 84 from the step's rows, 91 / 68 from pages (without chunks 71 / 80, 65 / 60: rows without masks have
+            // less to do a tile), 32 heads 111 / 159; 4 of 500 to 100, 32 heads 55 / 50, 48 / 36; one of 4,000, 16 heads
+            // 233 / 246; 16 of 128, 32 heads 22 / 31.  Heads of up to 64: 8 of 1,024 to 61 82 / 55, one of 4,000 167 / 141, 64
             // of 300 85 / 102.
             const long long tiles = (max_rows + MQ - 1) / MQ * (long long)n_seqs;
             const long long blocks = (rows > 0 && rows / MQ + n_seqs < tiles ? rows / MQ + n_seqs : tiles) * nh;
-            const int groups = g_attn_cap_groups ? g_attn_cap_groups : blocks < (dk <= 64 && dv <= 64 ? 1025 : 512) ? 2 : 1;
+            const int most = dk <= 64 && dv <= 64 ? 1025 : own_stride && !slopes && chunk <= 0 ? 385 : 512;
+            const int groups = g_attn_cap_groups ? g_attn_cap_groups : blocks < most ? 2 : 1;
 #define GOB(KT_, VT_) do { if (groups == 2) GOB_G(KT_, VT_, 2); else GOB_G(KT_, VT_, 1); } while (0)
 #define GOB_G(KT_, VT_, G_)                                                                        \
     hipLaunchKernelGGL((attn_cap_rows_bf16_kernel<KT_, VT_, G_>), grid, dim3(256 * G_), 0, (hipStream_t)stream, \
