@@ -18,7 +18,7 @@ cache), the LLaMA-3-8B shape with 16 prompts of 64 to 4,096 tokens and with 8 se
 engine's generation loop, whose stopwatch starts after the warm-up steps.  Every decode point has a
 `..._hbm_frac` beside it: the bytes its step has to read (every weight once, the
 cache of its live sequences) / its time / the HBM peak.  Peaks are the published ones
-of MI355X (HBM 8 TB/s, dense bf16 MFMA 2.5 PFLOP/s, float32 157.3 TFLOP/s).
+of MI355X (HBM 8 TB/s, dense bf16 MFMA 2.5 PFLOP/s; float32, whose large products are six bf16 ones, a sixth of it).
 The run fails (non-zero) if any timed run produced a non-finite logit or the same
 greedy token everywhere.
 
@@ -42,7 +42,7 @@ import sys
 import time
 
 HBM_PEAK_GBS = 8000.0
-PEAK_TFLOPS = {"bf16": 2500.0, "fp32": 157.3}
+PEAK_TFLOPS = {"bf16": 2500.0, "fp32": 2500.0 / 6}      # (float32: six bfloat16 products for one)
 
 LLAMA2_7B = {"architectures": ["LlamaForCausalLM"], "hidden_size": 4096, "intermediate_size": 11008,
              "num_hidden_layers": 32, "num_attention_heads": 32, "num_key_value_heads": 32,
