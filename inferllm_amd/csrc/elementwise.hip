@@ -490,7 +490,10 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ x, const void* __restrict
 
 // The same with every element of the row held in registers: each thread owns NV
 // groups of 4 consecutive floats, all loads are issued before the first use, and x is
-// read once.  Needs E % 4 == 0 and E <= 1024 * NV.
+// read once.  Needs E % 4 == 0 and E <= 4 * TH * NV.
+// BY256 (TH 1024): the row's sum of squares in the order of blocks of 256 threads, so that a row of 129 to 512 has the
+// bits that it has among more: each group of four columns' sum goes to LDS, and the first 256 threads add their
+// 4 NV of them (the groups a narrow block's thread owns) before the sum over the waves.
 __device__ __forceinline__ float4 ld4_f(const void* p, int dt, size_t i4) {
     if (dt == ILLM_BF16) {
         const uint2 u = ((const uint2*)p)[i4];
@@ -511,7 +514,14 @@ __device__ __forceinline__ void st4_f(void* p, int dt, size_t i4, float4 v) {
     }
 }
 
-template <int NV, int TH>
+// Four columns' sum of squares.  (The two orders stand as rows have had them: the first where a thread has one group.)
+template <int NV>
+__device__ __forceinline__ float group_sq(float4 v) {
+    const float first = NV == 1 ? fmaf(v.y, v.y, v.x * v.x) : fmaf(v.x, v.x, v.y * v.y);
+    return fmaf(v.w, v.w, fmaf(v.z, v.z, first));
+}
+
+template <int NV, int TH, bool BY256 = false>
 __global__ void __launch_bounds__(TH)
 add_rmsnorm_vec_kernel(float* __restrict__ x, const void* __restrict__ delta, int delta_dt,
                        int planes, size_t plane_stride4, const void* __restrict__ delta2,
@@ -564,9 +574,19 @@ add_rmsnorm_vec_kernel(float* __restrict__ x, const void* __restrict__ delta, in
         }
     }
     float ss = 0.f;
+    if constexpr (BY256) {
+        __shared__ float part[TH * NV];
 #pragma unroll
-    for (int j = 0; j < NV; ++j)
-        ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+        for (int j = 0; j < NV; ++j)
+            part[threadIdx.x + TH * j] = group_sq<2>(v[j]);
+        __syncthreads();
+        if (threadIdx.x < 256)
+#pragma unroll
+            for (int k = 0; k < TH / 256 * NV; ++k) ss += part[threadIdx.x + 256 * k];
+    } else {
+#pragma unroll
+        for (int j = 0; j < NV; ++j) ss += group_sq<NV>(v[j]);
+    }
     ss = block_sum(ss, red);
     const float scale = 1.0f / sqrtf(ss / (float)E + eps);
 #pragma unroll
@@ -599,16 +619,19 @@ extern "C" int illm_add2_rmsnorm_two(float* x, const void* delta, int delta_dt, 
         return ILLM_ERR_ARG;
     if (rows == 0) return ILLM_OK;
     hipStream_t st = (hipStream_t)stream;
-#define VEC(NV_, TH_)                                                                         \
-    hipLaunchKernelGGL((add_rmsnorm_vec_kernel<NV_, TH_>), dim3(rows), dim3(TH_), 0, st, x,   \
+#define VEC(NV_, TH_, ...)                                                                    \
+    hipLaunchKernelGGL((add_rmsnorm_vec_kernel<NV_, TH_ __VA_OPT__(,) __VA_ARGS__>), dim3(rows), dim3(TH_), 0, st, x, \
                        delta, delta_dt, planes, plane_stride / 4, delta2, delta2_dt, w, w_dt, out,  \
                        out_dt, row_idx, E, eps, w2, out2)
     // few rows (decoding, short prompts): wide blocks, one group of 4 floats per thread, to shorten the row's
-    // critical path; many rows: narrow blocks so that more rows are in flight per CU (us, narrow / wide, with a bfloat16
-    // delta: 160 rows of 2,048 3.8 / 3.5, of 4,096 5.1 / 4.0, with four planes 5.8 / 4.3; 512 rows of 2,048 4.6 / 4.6, of
-    // 4,096 6.5 / 6.1, of 8,192 10.7 / 8.5)
-    if (E % 4 == 0 && rows <= (E <= 2048 ? 256 : 512) && E > 1024 && E <= 4096) VEC(1, 1024);
-    else if (E % 4 == 0 && rows <= 512 && E > 4096 && E <= 8192) VEC(2, 1024);
+    // critical path; many rows: narrow blocks so that more rows are in flight per CU (us, narrow / wide in the narrow
+    // order, with a bfloat16 delta: 130 / 192 / 256 / 300 rows of 2,048 3.2 / 3.3 / 3.5 / 3.6 against 3.1 / 3.3 / 3.4 / 3.6,
+    // of 4,096 4.3 / 4.5 / 4.7 / 4.9 against 3.6 / 3.9 / 4.2 / 5.0; 130 / 256 / 512 rows of 8,192 6.4 / 7.2 / 8.8 against
+    // 4.7 / 5.7 / 8.0)
+    if (E % 4 == 0 && rows <= 128 && E > 1024 && E <= 4096) VEC(1, 1024);
+    else if (E % 4 == 0 && rows <= 128 && E > 4096 && E <= 8192) VEC(2, 1024);
+    else if (E % 4 == 0 && rows <= 256 && E > 1024 && E <= 4096) VEC(1, 1024, true);
+    else if (E % 4 == 0 && rows <= 512 && E > 4096 && E <= 8192) VEC(2, 1024, true);
     else if (E % 4 == 0 && E <= 1024) VEC(1, 256);
     else if (E % 4 == 0 && E <= 2048) VEC(2, 256);
     else if (E % 4 == 0 && E <= 4096) VEC(4, 256);

@@ -97,6 +97,22 @@ def test_add_rmsnorm_adds_planes(out_dtype, S, T, E):
     assert torch.equal(xg2.cpu(), x)
 
 
+@pytest.mark.parametrize("T,E", [(129, 1028), (160, 2048), (256, 2052), (129, 4096), (257, 4092), (300, 4100), (512, 8192)])
+def test_norm_of_a_row_among_129_to_512_and_among_more(T, E):
+    """From 129 rows on, a row's normed values and its sum have the same bits whatever the number of rows."""
+    many = 520
+    x, w = rnd(many, E, seed=1), (1 + rnd(E, seed=2) * 0.1).to(DEV)
+    for planes, dtype in ((0, torch.bfloat16), (1, torch.bfloat16), (3, torch.float32)):
+        delta = rnd(planes, many, E, seed=3).to(dtype) if planes else None
+        got = []
+        for n in (T, many):
+            xs = x[:n].contiguous().to(DEV)
+            d = None if delta is None else delta[:, :n].contiguous().to(DEV)
+            out = ops().add_rmsnorm(xs, d if planes != 1 else d[0], w, 1e-5, torch.float32)
+            got.append((out, xs))
+        assert torch.equal(got[0][0], got[1][0][:T]) and torch.equal(got[0][1], got[1][1][:T])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("T,F", [(4, 10), (5, 130), (3, 11008), (1, 173), (70, 64), (2, 2056)])
 def test_silu_mul(dtype, T, F):
