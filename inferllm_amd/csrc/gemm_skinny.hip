@@ -66,6 +66,12 @@ struct SkResidual {
     int act;                     // SK_PLAIN without `accumulate`: 1 relu(y)^2, 2 gelu(y) (tanh), 0 y
 };
 
+// The value of the lane 8 further within 16.
+__device__ __forceinline__ uint4 turn8(uint4 v) {
+    auto t = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x128, 0xf, 0xf, true); };   // row_ror:8
+    return make_uint4(t(v.x), t(v.y), t(v.z), t(v.w));
+}
+
 // TILED (NTB == 1, K % 32 == 0): W is a copy laid out for this kernel, [tile][k-step][16 rows][32 k]
 // with tile = blockIdx.x holding the 16 rows that block works on (in its mode's order): a load
 // instruction then reads 1 KB that is contiguous and already in operand order, so the lines need
@@ -74,8 +80,10 @@ struct SkResidual {
 // the block's waves cover in one piece each: the product of a short K is bound by the round
 // trips of a wave's pieces, not by bandwidth).
 // HALF (TILED, MT == NTB == 1, at most 8 rows of X): a block takes 8 rows of a tile, so that a matrix of few tiles
-// occupies twice the compute units.  The MFMA's 16 rows of W are then its 8 at one k-step and at the next, its 16
-// columns the rows of X likewise, and the two quarters of the result that belong together are added at the end.
+// occupies twice the compute units.  A load brings two k-steps, lanes r < 8 the even one, the others the odd one, of W and X
+// alike; a product of the even step is followed by one of both operands turned by 8 lanes, so that rows 0 .. 7 and
+// columns 0 .. 7 of the sums take the steps one after the other, in whole tiles' order and with whole tiles' waves: the
+// same bits.  (The other three quarters of the sums are never read.)
 template <int MT, int NTB, int SK_U, int MAXW, int MODE, bool TILED, bool ONE_SHOT = false, bool HALF = false>
 __global__ void __launch_bounds__(64 * MAXW)
 gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
@@ -244,9 +252,11 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
 #pragma unroll
     for (int nt = 0; nt < NTB; ++nt) tile_ok[nt] = DUAL ? n_base + 8 * nt < N : tile_row[nt] < N || MODE != SK_PLAIN;
 
-    const int all_steps = (K + 31) / 32, ksteps = HALF ? (all_steps + 1) / 2 : all_steps;
-    const int stride = waves * SK_U;
+    const int ksteps = (K + 31) / 32;
+    const int stride = waves * SK_U, turn = HALF ? 2 * stride : stride;      // k-steps from a wave's piece to the next
     uint4 a[NTB][SK_U], b[MT][SK_U];
+    // HALF: the k-step of this lane's u-th load, of two pieces of the wave
+    auto step_of = [&](int s0, int u) { return s0 + (2 * u >= SK_U ? stride : 0) + (2 * u) % SK_U + (r >> 3); };
     auto load = [&](int s0, uint4 (&aa)[NTB][SK_U], uint4 (&bb)[MT][SK_U]) {
 #pragma unroll
         for (int u = 0; u < SK_U; ++u) {
@@ -255,15 +265,15 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
 #pragma unroll
             for (int nt = 0; nt < NTB; ++nt) {
                 if (HALF) {
-                    const int st = 2 * (s0 + u) + (r >> 3);
-                    aa[nt][u] = st < all_steps ? ld16_stream(wtile + (size_t)st * 512) : make_uint4(0, 0, 0, 0);
+                    const int st = step_of(s0, u);
+                    aa[nt][u] = st < ksteps ? ld16_stream(wtile + (size_t)st * 512) : make_uint4(0, 0, 0, 0);
                 } else if (TILED)
                     aa[nt][u] = (s0 + u < ksteps && tile_ok[nt])
                                     ? ld16_stream(wtile + ((size_t)nt * ksteps + s0 + u) * 512)
                                     : make_uint4(0, 0, 0, 0);
                 else aa[nt][u] = kw < K ? ld16_stream(wline[nt][u & 1] + kw) : make_uint4(0, 0, 0, 0);
             }
-            const int k = (HALF ? 2 * (s0 + u) + (r >> 3) : s0 + u) * 32 + q * 8;
+            const int k = (HALF ? step_of(s0, u) : s0 + u) * 32 + q * 8;
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
                 bb[mt][u] = k < K ? *(const uint4*)(xrow[mt] + k) : make_uint4(0, 0, 0, 0);
@@ -271,14 +281,14 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
     };
     int s0 = wave * SK_U;
     if (s0 < ksteps) load(s0, a, b);
-    for (; s0 < ksteps; s0 += stride) {
+    for (; s0 < ksteps; s0 += turn) {
         // the next piece is on its way while this one is multiplied
         uint4 an[ONE_SHOT ? 1 : NTB][SK_U], bn[ONE_SHOT ? 1 : MT][SK_U];
-        const bool more = !ONE_SHOT && s0 + stride < ksteps;
+        const bool more = !ONE_SHOT && s0 + turn < ksteps;
         if constexpr (ONE_SHOT) {
             if (s0 != wave * SK_U) load(s0, a, b);       // (a K longer than one piece a wave)
         } else {
-            if (more) load(s0 + stride, an, bn);
+            if (more) load(s0 + turn, an, bn);
         }
         if (!TILED) {
 #pragma unroll
@@ -301,6 +311,11 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                 for (int mt = 0; mt < MT; ++mt)
                     acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                         *(const bf16x8_t*)&am, *(bf16x8_t*)&b[mt][u], acc[nt][mt], 0, 0, 0);
+                if constexpr (HALF) {
+                    const uint4 a8 = turn8(am), b8 = turn8(b[0][u]);
+                    acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a8, *(const bf16x8_t*)&b8,
+                                                                        acc[0][0], 0, 0, 0);
+                }
             }
         if constexpr (!ONE_SHOT) {
             if (more) {
@@ -400,17 +415,15 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
     // every thread of the block sums some of the (mt, lane) groups over the waves, tile by tile
     for (int grp = threadIdx.x; grp < MT * 64; grp += blockDim.x) {
         const int l2 = grp & 63, mt = grp >> 6;
-        if (HALF && (l2 & 40)) continue;
+        if (HALF && (l2 & 40)) continue;                    // (rows and columns 0 .. 7)
         f32x4_t v[NTB];
 #pragma unroll
         for (int nt = 0; nt < NTB; ++nt) {
             if (waves > 1 || HALF) {
                 const int e = ((nt * MT + mt) * 64 + l2) * 4;
                 v[nt] = *(f32x4_t*)(red + e);
-                if (HALF) v[nt] += *(f32x4_t*)(red + e + 160);
                 for (int w = 1; w < waves; ++w) {
-                    f32x4_t o = *(f32x4_t*)(red + (size_t)w * PER_WAVE + e);
-                    if (HALF) o += *(f32x4_t*)(red + (size_t)w * PER_WAVE + e + 160);
+                    const f32x4_t o = *(f32x4_t*)(red + (size_t)w * PER_WAVE + e);
                     v[nt][0] += o[0]; v[nt][1] += o[1]; v[nt][2] += o[2]; v[nt][3] += o[3];
                 }
             } else {
@@ -557,17 +570,14 @@ static int skinny_plain(const void* X, const void* W, const void* Wt, void* Y, i
         return skinny_from_matrix(X, W, Y, y_dt, M, N, K, ntb, u, waves, res, stream);
     waves = clamp_waves(waves, 1, 1, 4, K);
     if (use_tiled(Wt, M, K)) {
-        // Half a tile a block where the tiles do not fill the compute units (us with whole / half tiles at 8 rows: 2048 x
-        // 8192 14.9 / 11.0, x 4096 8.6 / 7.3, x 2048 5.7 / 5.0, x 512 3.6 / 3.5, x 64 2.9 / 3.1; 512 x 8192 12.3 / 9.0; at 1 row
-        // 2048 x 8192 12.8 / 8.5), not where they do (2560 x 4096 9.6 / 9.9, 4096 x 4096 9.4 / 10.8: X is read twice as often).
+        // Half a tile a block where the tiles do not fill the compute units (us with whole / half tiles at 8 rows, matrices
+        // cold: 2048 x 8192 14.4 / 10.1, x 4096 8.2 / 6.6, x 2048 5.7 / 5.0, x 1024 4.4 / 4.1; 1024 x 4096 7.6 / 6.1, 512 x 8192
+        // 12.3 / 8.8, 64 x 1024 3.8 / 3.6; at 1 row 2048 x 8192 11.1 / 8.4, x 1024 3.8 / 3.8), not where they do (2560 x 4096
+        // 9.7 / 10.9, at 1 row 7.7 / 9.1: X is read twice as often).
         const bool half = M <= 8 && (SK_HALF >= 0 ? SK_HALF == 1 : blocks <= 128 && K >= 1024);
-        if (half) {
-            const int halves = (N + 7) / 8;
-            int wh = waves_wanted > 0 ? waves_wanted : (on_chip + halves / 2) / halves;
-            wh = clamp_waves(wh < 2 ? 2 : wh, 1, 1, 4, (K + 1) / 2);
-            return launch_skinny<1, 1, 4, SK_PLAIN, true, false, true>(X, Wt, Y, y_dt, M, N, K, wh, (hipStream_t)stream,
+        if (half)
+            return launch_skinny<1, 1, 4, SK_PLAIN, true, false, true>(X, Wt, Y, y_dt, M, N, K, waves, (hipStream_t)stream,
                                                                        SkRope(), res);
-        }
         // with many tiles (the head) a block takes two: X is read half as often
         if (two_tiles_a_block(blocks)) {
             const int blocks2 = (blocks + 1) / 2;

@@ -610,6 +610,27 @@ def test_skinny_half_tiles_and_activations(M, N, K):
     assert torch.equal(ops().linear_act(many, tiled, "gelu_tanh"), ops().gelu_tanh(ops().linear(many, tiled)))
 
 
+@pytest.mark.parametrize("N,K", [(2048, 8192), (2040, 4096), (512, 1056), (520, 2048), (1030, 2080), (64, 1024)])
+def test_skinny_rows_alone_and_among_16(N, K):
+    """A row's sums have the same bits in steps of 1 to 16 rows: with half a tile a block (up to 8 rows) as with whole
+    ones, and as a norm's consumer."""
+    x, w = rnd(16, K, seed=1).to(torch.bfloat16).to(DEV), rnd(N, K, seed=2).to(torch.bfloat16).to(DEV)
+    tiled, nw = ops().decode_weight(w, "plain", True), torch.ones(K, device=DEV)
+    ssq = (x.float() ** 2).view(16, K // 32, 32).sum(-1)
+    want = ops().linear(x, tiled, torch.float32)
+    lib = ops()._lib()
+    normed = lambda M: ops().NormedRows(x[:M].float(), nw, 1e-5, torch.bfloat16, x[:M].contiguous(), ssq[:M].contiguous())
+    want_normed = ops().linear(normed(16), tiled, torch.float32)
+    try:
+        for half in (1, 0, -1):
+            lib.illm_set_skinny_half(half)
+            for M in (1, 3, 7, 8, 9):
+                assert torch.equal(ops().linear(x[:M].contiguous(), tiled, torch.float32), want[:M])
+                assert torch.equal(ops().linear(normed(M), tiled, torch.float32), want_normed[:M])
+    finally:
+        lib.illm_set_skinny_half(-1)
+
+
 @pytest.mark.parametrize("d,window,chunk,keep", [(128, 0, 0, 0), (128, 0, 96, 0), (64, 70, 0, 0), (32, 40, 0, 33), (40, 0, 0, 0)])
 def test_attn_cap_rows_groups(d, window, chunk, keep):
     """Prompts' attention with the keys' tiles in turn by two groups of waves against one group (the same sums in
