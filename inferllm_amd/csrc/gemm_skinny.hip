@@ -63,7 +63,7 @@ struct SkResidual {
     int planes;                  // SK_PLAIN: > 1, W's rows are that many parts and part p, whose rows end at
     int ends[ILLM_MAX_PLANES];   // ends[p] (multiples of a block's rows but for the last), reads plane p of
                                  // X [planes][M][K]
-    int act;                     // SK_PLAIN without `accumulate`: 1 relu(y)^2, 2 gelu(y) (tanh), 0 y
+    int act;                     // SK_PLAIN without `accumulate`, ACT: 1 relu(y)^2, 2 gelu(y) (tanh), y rounded to Y's type
 };
 
 // The value of the lane 8 further within 16.
@@ -84,7 +84,8 @@ __device__ __forceinline__ uint4 turn8(uint4 v) {
 // alike; a product of the even step is followed by one of both operands turned by 8 lanes, so that rows 0 .. 7 and
 // columns 0 .. 7 of the sums take the steps one after the other, in whole tiles' order and with whole tiles' waves: the
 // same bits.  (The other three quarters of the sums are never read.)
-template <int MT, int NTB, int SK_U, int MAXW, int MODE, bool TILED, bool ONE_SHOT = false, bool HALF = false>
+// ACT: the results go through res.act.  (A variant of its own: the test alone cost every product 0.15 us.)
+template <int MT, int NTB, int SK_U, int MAXW, int MODE, bool TILED, bool ONE_SHOT = false, bool HALF = false, bool ACT = false>
 __global__ void __launch_bounds__(64 * MAXW)
 gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                    void* __restrict__ Y, int y_dt, int M, int N, int K, SkRope rope,
@@ -479,11 +480,14 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
             for (int i = 0; i < 4; ++i)
                 if (n0 + i < N) {
                     float y = v[nt][i] * rs;
-                    if (res.act == 1) {
-                        y = fmaxf(y, 0.f);
-                        y *= y;
-                    } else if (res.act == 2) {
-                        y = gelu_tanh_f(y);
+                    if constexpr (ACT) {
+                        if (y_dt == ILLM_BF16) y = bf16_to_f32(f32_to_bf16(y));     // as the activation alone reads it
+                        if (res.act == 1) {
+                            y = fmaxf(y, 0.f);
+                            y *= y;
+                        } else {
+                            y = gelu_tanh_f(y);
+                        }
                     }
                     st_f(Y, y_dt, (size_t)mrow * N + n0 + i, y);
                 }
@@ -493,7 +497,8 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
 
 static const SkResidual SK_NO_RESIDUAL = {0, nullptr, ILLM_BF16, nullptr, nullptr, nullptr, 0, 0.f, 0.f, 0.f, 0, {}, 0};
 
-template <int MT, int NTB, int U, int MODE = SK_PLAIN, bool TILED = false, bool ONE_SHOT = false, bool HALF = false>
+template <int MT, int NTB, int U, int MODE = SK_PLAIN, bool TILED = false, bool ONE_SHOT = false, bool HALF = false,
+          bool ACT = false>
 static int launch_skinny(const void* X, const void* W, void* Y, int y_dt, int M, int N, int K,
                          int waves, hipStream_t st, SkRope rope = SkRope(),
                          SkResidual res = SK_NO_RESIDUAL) {
@@ -505,7 +510,7 @@ static int launch_skinny(const void* X, const void* W, void* Y, int y_dt, int M,
     const int rows_per_block = DUAL ? 8 * NTB : HALF ? 8 : 16 * NTB;
     const int blocks = (N + rows_per_block - 1) / rows_per_block;
     const size_t smem = (size_t)waves * NTB * ((!TILED && U > MT) ? U : MT) * 1024 + 64;
-    hipLaunchKernelGGL((gemm_skinny_kernel<MT, NTB, U, MAXW, MODE, TILED, ONE_SHOT, HALF>), dim3(blocks), dim3(64 * waves),
+    hipLaunchKernelGGL((gemm_skinny_kernel<MT, NTB, U, MAXW, MODE, TILED, ONE_SHOT, HALF, ACT>), dim3(blocks), dim3(64 * waves),
                        smem, st, (const bf16_t*)X, (const bf16_t*)W, Y, y_dt, M, N, K, rope, res);
     return illm_launch_status();
 }
@@ -533,7 +538,7 @@ static int clamp_waves(int w, int ntb, int mt, int u, int K) {
 // W a block, u * 64 bytes of a W row per wave iteration, waves per block (clamped to what LDS
 // and K allow).  Up to 16 rows of X take ntb = 1, more take 2; u = 4 (measured best).
 static int skinny_from_matrix(const void* X, const void* W, void* Y, int y_dt, int M,
-                              int N, int K, int ntb, int u, int waves, const SkResidual& res, void* stream) {
+                              int N, int K, int ntb, int u, int waves, void* stream) {
     if (M <= 0 || M > 64 || N <= 0 || K <= 0 || (K % 8) || !illm_dtype_ok(y_dt))
         return ILLM_ERR_ARG;
     hipStream_t st = (hipStream_t)stream;
@@ -541,7 +546,7 @@ static int skinny_from_matrix(const void* X, const void* W, void* Y, int y_dt, i
     waves = clamp_waves(waves, ntb, mt, u, K);
 #define GO(MT_, NTB_, U_)                                                                     \
     if (mt == MT_ && ntb == NTB_ && u == U_)                                                  \
-        return launch_skinny<MT_, NTB_, U_>(X, W, Y, y_dt, M, N, K, waves, st, SkRope(), res)
+        return launch_skinny<MT_, NTB_, U_>(X, W, Y, y_dt, M, N, K, waves, st)
     GO(1, 1, 4); GO(2, 2, 4); GO(3, 2, 4); GO(4, 2, 4);
 #undef GO
     return ILLM_ERR_ARG;
@@ -559,6 +564,7 @@ static bool use_tiled(const void* Wt, int M, int K) { return Wt && M <= 16 && K 
 static int SK_HALF = -1;              // tuning and tests: 0 never, 1 wherever it can be, -1 the rule below
 extern "C" void illm_set_skinny_half(int on) { SK_HALF = on; }
 
+template <bool ACT>
 static int skinny_plain(const void* X, const void* W, const void* Wt, void* Y, int y_dt, int M, int N, int K,
                         const SkResidual& res, int waves_wanted, void* stream) {
     const int ntb = M <= 16 ? 1 : 2, u = 4;
@@ -566,30 +572,30 @@ static int skinny_plain(const void* X, const void* W, const void* Wt, void* Y, i
     const int on_chip = use_tiled(Wt, M, K) ? SK_WAVES_ON_CHIP_TILED : SK_WAVES_ON_CHIP;
     int waves = waves_wanted > 0 ? waves_wanted : (on_chip + blocks / 2) / blocks;
     waves = waves < 1 ? 1 : waves;
-    if (!res.ssq && !use_tiled(Wt, M, K))
-        return skinny_from_matrix(X, W, Y, y_dt, M, N, K, ntb, u, waves, res, stream);
+    if (!ACT && !res.ssq && !use_tiled(Wt, M, K))
+        return skinny_from_matrix(X, W, Y, y_dt, M, N, K, ntb, u, waves, stream);
     waves = clamp_waves(waves, 1, 1, 4, K);
     if (use_tiled(Wt, M, K)) {
         // Half a tile a block where the tiles do not fill the compute units (us with whole / half tiles at 8 rows, matrices
-        // cold: 2048 x 8192 14.4 / 10.1, x 4096 8.2 / 6.6, x 2048 5.7 / 5.0, x 1024 4.4 / 4.1; 1024 x 4096 7.6 / 6.1, 512 x 8192
-        // 12.3 / 8.8, 64 x 1024 3.8 / 3.6; at 1 row 2048 x 8192 11.1 / 8.4, x 1024 3.8 / 3.8), not where they do (2560 x 4096
-        // 9.7 / 10.9, at 1 row 7.7 / 9.1: X is read twice as often).
+        // cold: 2048 x 8192 14.7 / 9.9, x 4096 7.8 / 6.4, x 2048 5.4 / 4.8, x 1024 4.0 / 3.9; 1024 x 4096 7.4 / 5.9, 512 x 8192
+        // 12.0 / 8.6, 64 x 1024 3.7 / 3.5; at 1 row 2048 x 8192 11.0 / 8.3, x 1024 3.6 / 3.7), not where they do (2560 x 4096
+        // 9.3 / 10.8, at 1 row 7.5 / 8.7: X is read twice as often).
         const bool half = M <= 8 && (SK_HALF >= 0 ? SK_HALF == 1 : blocks <= 128 && K >= 1024);
         if (half)
-            return launch_skinny<1, 1, 4, SK_PLAIN, true, false, true>(X, Wt, Y, y_dt, M, N, K, waves, (hipStream_t)stream,
-                                                                       SkRope(), res);
+            return launch_skinny<1, 1, 4, SK_PLAIN, true, false, true, ACT>(X, Wt, Y, y_dt, M, N, K, waves,
+                                                                            (hipStream_t)stream, SkRope(), res);
         // with many tiles (the head) a block takes two: X is read half as often
         if (two_tiles_a_block(blocks)) {
             const int blocks2 = (blocks + 1) / 2;
             int w2 = waves_wanted > 0 ? waves_wanted : (on_chip + blocks2 / 2) / blocks2;
-            return launch_skinny<1, 2, 4, SK_PLAIN, true>(X, Wt, Y, y_dt, M, N, K,
+            return launch_skinny<1, 2, 4, SK_PLAIN, true, false, false, ACT>(X, Wt, Y, y_dt, M, N, K,
                                                           clamp_waves(w2 < 1 ? 1 : w2, 2, 1, 4, K),
                                                           (hipStream_t)stream, SkRope(), res);
         }
-        return launch_skinny<1, 1, 4, SK_PLAIN, true>(X, Wt, Y, y_dt, M, N, K, waves,
+        return launch_skinny<1, 1, 4, SK_PLAIN, true, false, false, ACT>(X, Wt, Y, y_dt, M, N, K, waves,
                                                       (hipStream_t)stream, SkRope(), res);
     }
-    return launch_skinny<1, 1, 4>(X, W, Y, y_dt, M, N, K, waves, (hipStream_t)stream, SkRope(), res);
+    return launch_skinny<1, 1, 4, SK_PLAIN, false, false, false, ACT>(X, W, Y, y_dt, M, N, K, waves, (hipStream_t)stream, SkRope(), res);
 }
 
 extern "C" int illm_gemm_skinny_bf16(const void* X, const void* W, const void* Wt, void* Y, int y_dt,
@@ -600,10 +606,11 @@ extern "C" int illm_gemm_skinny_bf16(const void* X, const void* W, const void* W
         return ILLM_ERR_ARG;
     SkResidual res = SK_NO_RESIDUAL;
     res.ssq = ssq; res.parts = parts; res.eps = eps;
-    return skinny_plain(X, W, Wt, Y, y_dt, M, N, K, res, waves_wanted, stream);
+    return skinny_plain<false>(X, W, Wt, Y, y_dt, M, N, K, res, waves_wanted, stream);
 }
 
-// The same of at most 16 rows with an activation on the float32 sums: act 1 relu(y)^2, 2 gelu(y) by tanh.
+// The same of at most 16 rows with an activation of the results as Y's type holds them (the bits of the product and the
+// activation one after the other): act 1 relu(y)^2, 2 gelu(y) by tanh.
 extern "C" int illm_gemm_skinny_act(const void* X, const void* W, const void* Wt, void* Y, int y_dt, int M, int N, int K,
                                     const float* ssq, int parts, float eps, int act, void* stream) {
     if (M <= 0 || M > 16 || N <= 0 || K <= 0 || (K % 8) || !illm_dtype_ok(y_dt) || !scale_args_ok(ssq, parts, M) ||
@@ -611,7 +618,8 @@ extern "C" int illm_gemm_skinny_act(const void* X, const void* W, const void* Wt
         return ILLM_ERR_ARG;
     SkResidual res = SK_NO_RESIDUAL;
     res.ssq = ssq; res.parts = parts; res.eps = eps; res.act = act;
-    return skinny_plain(X, W, Wt, Y, y_dt, M, N, K, res, 0, stream);
+    return act ? skinny_plain<true>(X, W, Wt, Y, y_dt, M, N, K, res, 0, stream)
+               : skinny_plain<false>(X, W, Wt, Y, y_dt, M, N, K, res, 0, stream);
 }
 
 // The product whose parts of W read rows of X of their own: X [planes][M][K], W's rows ends[p - 1] .. ends[p] - 1

@@ -631,6 +631,18 @@ def test_skinny_rows_alone_and_among_16(N, K):
         lib.illm_set_skinny_half(-1)
 
 
+@pytest.mark.parametrize("name", ["relu_squared", "gelu_tanh"])
+@pytest.mark.parametrize("N,K", [(2048, 1056), (100, 1024), (4104, 96)])
+def test_an_activation_in_the_product_and_behind_it(name, N, K):
+    """`linear_act` has the bits of the product and the activation one after the other, from either copy of the matrix
+    and for any number of rows."""
+    x, w = rnd(20, K, seed=1).to(torch.bfloat16).to(DEV), rnd(N, K, seed=2, std=K ** -0.5).to(torch.bfloat16).to(DEV)
+    for W in (w, ops().decode_weight(w, "plain", True)):
+        for M in (1, 5, 8, 9, 16, 17):
+            rows = x[:M].contiguous()
+            assert torch.equal(ops().linear_act(rows, W, name), getattr(ops(), name)(ops().linear(rows, W)))
+
+
 @pytest.mark.parametrize("d,window,chunk,keep", [(128, 0, 0, 0), (128, 0, 96, 0), (64, 70, 0, 0), (32, 40, 0, 33), (40, 0, 0, 0)])
 def test_attn_cap_rows_groups(d, window, chunk, keep):
     """Prompts' attention with the keys' tiles in turn by two groups of waves against one group (the same sums in
