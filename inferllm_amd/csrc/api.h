@@ -473,15 +473,6 @@ int illm_attn_cap_rows(const void* q, int q_stride, void* out, int dt, const int
                        const void* gate, int gate_stride, int gate_off, int gate_heads, float* lse,
                        int keep, int kept, int own_stride, int own_k, int own_v_stride, int own_v,
                        const float* sink, void* stream);
-// The same; rows: the step's rows in all, from which the blocks' shape is chosen (0: not known).
-int illm_attn_cap_rows_of(const void* q, int q_stride, void* out, int dt, const int32_t* cu,
-                       const int32_t* seq_slot, const int32_t* seq_start, const void* kcache,
-                       const void* vcache, const int32_t* page_table, int table_stride,
-                       int page_size, int ring, int n_seqs, int max_rows, int nh, int nkv, int dk,
-                       int dv, float scale, float cap, int window, const float* slopes, int chunk,
-                       const void* gate, int gate_stride, int gate_off, int gate_heads, float* lse,
-                       int keep, int kept, int own_stride, int own_k, int own_v_stride, int own_v,
-                       const float* sink, int rows, void* stream);
 int illm_attn_cap_decode(const void* q, int q_stride, void* out, int dt, const void* kcache,
                          const void* vcache, const int32_t* page_table, int table_stride,
                          int page_size, int ring, const int32_t* seq_slot, const int32_t* seq_len,

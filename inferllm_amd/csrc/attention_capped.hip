@@ -587,10 +587,14 @@ attn_cap_rows_mfma_kernel(const void* __restrict__ q, int q_stride, void* __rest
 // a lane holds its weights: key 16 s + 8 b + 4 h + i at place 16 s + 8 h + 4 b + i.
 typedef __bf16 cap_bf16x8_t __attribute__((ext_vector_type(8)));
 
-// GROUPS 2: eight waves, of which the second four take every second tile of keys for the same rows, and add what they
-// have at the end: half as many turns behind each other for the block that the launch waits for.
-template <int KT, int VT, int GROUPS>
-__global__ void __launch_bounds__(256 * GROUPS, KT <= 2 && VT <= 2 ? 4 : 2)      // (128 registers: 1,500 rows of 64 230 -> 199 us)
+// A tile's keys lie behind each other in the step's own rows (FROM 0) or in a page where pages are whole tiles (1: the page
+// is looked up once for the wave and a tile ahead of its loads); in other pages (2) every lane looks its own up.
+// (Variants, since all three in one took 8 to 14 registers more: 1,500 rows, 16 heads of 64 115 -> 108 us, 8 sequences of 1,024 to
+// 61 rows, 16 heads of 128 own 70 -> 65, pages 71 -> 67; a look a lane before each load had taken 87 there.)
+enum { CAP_OWN_ROWS = 0, CAP_TILED_PAGES = 1, CAP_ANY_PAGES = 2 };
+
+template <int KT, int VT, int FROM>
+__global__ void __launch_bounds__(256, 2)
 attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out,
                           const int32_t* __restrict__ cu, const int32_t* __restrict__ seq_slot,
                           const int32_t* __restrict__ seq_start, const bf16_t* __restrict__ kcache,
@@ -603,12 +607,8 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
     constexpr int DKP = 32 * KT, DVP = 32 * VT, KLD = DKP + 8, VLD = MK + 8;
     constexpr int KP = (MK * DKP / 8 + 255) / 256;             // 16-byte pieces of a key tile a thread brings
     constexpr int VP = ((MK / 2) * (DVP / 8) + 255) / 256;     // pairs of keys x 8 value dims a thread brings
-    constexpr int PART = MK * KLD + DVP * VLD;                 // a group's tile
-    constexpr int EXCHANGE = GROUPS > 1 ? (4 * 64 * 16 * 4 + 4 * 64 * 8) / 2 : 0;
-    __shared__ __attribute__((aligned(16))) bf16_t tiles[GROUPS * PART > EXCHANGE ? GROUPS * PART : EXCHANGE];
-    const int grp = GROUPS > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 256)) : 0;
-    bf16_t* const ks = tiles + grp * PART;
-    bf16_t* const vs = ks + MK * KLD;
+    __shared__ __attribute__((aligned(16))) bf16_t ks[MK * KLD];
+    __shared__ __attribute__((aligned(16))) bf16_t vs[DVP * VLD];
     const int b = blockIdx.z, h = blockIdx.y;
     const int start = cu[b], len = cu[b + 1] - start;
     const int q0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * MQ;
@@ -616,7 +616,7 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
     const int pos0 = seq_start[b], slot = seq_slot[b];
     const int total = pos0 + len;
     const int kvh = h / (nh / nkv);
-    const int tid = threadIdx.x & 255, lane = tid & 63, wave = wave_index() & 3;
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
     const int col = lane & 31, half = lane >> 5;
     const int qrow = q0 + 32 * wave + col;
     const int qpos = pos0 + qrow;
@@ -635,29 +635,26 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
         }
     }
     illm_u32x4_t kreg[KP], vreg[VP][2];
-    // A tile's keys lie behind each other: in the step's own rows, or in a page where pages are whole tiles (then the
-    // page is looked up once for the wave, and a tile ahead of its loads, not by every lane before each of its loads).
-    const bool by_page = !own_stride && page_size % MK == 0;
     auto page_at = [&](int k0) __attribute__((always_inline)) {
-        if (!by_page) return 0;
+        if (FROM != CAP_TILED_PAGES) return 0;
         int lp = k0 / page_size;
         if (ring > 0 && lp >= kept) lp = kept + (lp - kept) % ring;
         return page_table[(size_t)slot * table_stride + lp];
     };
     auto fetch = [&](int k0, int page) __attribute__((always_inline)) {
         const int rows = min(MK, total - k0);                  // keys past the end: a valid row, masked below
-        const size_t page_row = ((size_t)page * nkv + kvh) * page_size + k0 % page_size;
-        const size_t kb = own_stride ? (size_t)(start + k0) * own_stride + own_k + (size_t)kvh * dk : page_row * dk;
-        const size_t vb = own_stride ? (size_t)(start + k0) * own_v_stride + own_v + (size_t)kvh * dv : page_row * dv;
-        const int ks_row = own_stride ? own_stride : dk, vs_row = own_stride ? own_v_stride : dv;
+        const size_t page_row = FROM == CAP_TILED_PAGES ? ((size_t)page * nkv + kvh) * page_size + k0 % page_size : 0;
+        const size_t kb = FROM == CAP_OWN_ROWS ? (size_t)(start + k0) * own_stride + own_k + (size_t)kvh * dk : page_row * dk;
+        const size_t vb = FROM == CAP_OWN_ROWS ? (size_t)(start + k0) * own_v_stride + own_v + (size_t)kvh * dv : page_row * dv;
+        const int ks_row = FROM == CAP_OWN_ROWS ? own_stride : dk, vs_row = FROM == CAP_OWN_ROWS ? own_v_stride : dv;
         auto key_at = [&](int row) __attribute__((always_inline)) {
             row = min(row, rows - 1);
-            return own_stride || by_page ? kb + (size_t)((uint32_t)row * (uint32_t)ks_row)
+            return FROM != CAP_ANY_PAGES ? kb + (size_t)((uint32_t)row * (uint32_t)ks_row)
                                          : cache_row_offset(page_table, table_stride, slot, k0 + row, page_size, ring, nkv, kvh, dk, kept);
         };
         auto value_at = [&](int row) __attribute__((always_inline)) {
             row = min(row, rows - 1);
-            return own_stride || by_page ? vb + (size_t)((uint32_t)row * (uint32_t)vs_row)
+            return FROM != CAP_ANY_PAGES ? vb + (size_t)((uint32_t)row * (uint32_t)vs_row)
                                          : cache_row_offset(page_table, table_stride, slot, k0 + row, page_size, ring, nkv, kvh, dv, kept);
         };
 #pragma unroll
@@ -717,16 +714,15 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
         n = min(n, n_tiles - 1);
         return n < n_first ? n * MK : k_lo + (n - n_first) * MK;
     };
-    fetch(tile_at(grp), page_at(tile_at(grp)));
-    int page = page_at(tile_at(grp + GROUPS));
-    for (int n = grp; n < n_tiles + grp; n += GROUPS) {
+    fetch(tile_at(0), page_at(tile_at(0)));
+    int page = page_at(tile_at(1));
+    for (int n = 0; n < n_tiles; ++n) {
         const int k0 = tile_at(n);
         __syncthreads();
         stage();
         __syncthreads();
-        fetch(tile_at(n + GROUPS), page);
-        page = page_at(tile_at(n + 2 * GROUPS));
-        if (GROUPS > 1 && n >= n_tiles) continue;
+        fetch(tile_at(n + 1), page);
+        page = page_at(tile_at(n + 2));
         if (!wave_has_rows || k0 > wq_hi || k0 + MK - 1 < wc_lo ||
             (window > 0 && k0 >= keep && k0 + MK - 1 <= wq_lo - window))
             continue;
@@ -786,36 +782,6 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
             }
         }
     }
-    if constexpr (GROUPS > 1) {
-        static_assert(GROUPS == 2, "two groups");
-        float* const ex = (float*)tiles;                       // [wave][16][lane], then (m, l) a lane
-        float2* const ml = (float2*)(ex + 4 * 64 * 16);
-        __syncthreads();
-        if (grp) ml[wave * 64 + lane] = make_float2(m_i, l_i);
-        float own = 1.f, other = 0.f;
-#pragma unroll
-        for (int t = 0; t < VT; ++t) {
-            if (grp) {
-#pragma unroll
-                for (int v = 0; v < 16; ++v) ex[(wave * 16 + v) * 64 + lane] = o[t][v];
-            }
-            __syncthreads();
-            if (!grp) {
-                if (t == 0) {
-                    const float2 x = ml[wave * 64 + lane];
-                    const float m_new = fmaxf(m_i, x.x);
-                    own = m_i == NEG_INF ? 0.f : __expf(m_i - m_new);
-                    other = x.x == NEG_INF ? 0.f : __expf(x.x - m_new);
-                    l_i = l_i * own + x.y * other;
-                    m_i = m_new;
-                }
-#pragma unroll
-                for (int v = 0; v < 16; ++v) o[t][v] = o[t][v] * own + ex[(wave * 16 + v) * 64 + lane] * other;
-            }
-            __syncthreads();
-        }
-        if (grp) return;
-    }
     if (qrow < len) {
         if (sink) add_sink(sink[h], m_i, l_i);
         const float inv = 1.0f / l_i;
@@ -855,12 +821,10 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
 // cores' float32 instruction also for bfloat16 storage.
 static int g_attn_cap_mfma = 1;
 extern "C" void illm_set_attn_cap_mfma(int on) { g_attn_cap_mfma = on < 0 || on > 2 ? 1 : on; }
-static int g_attn_cap_groups = 0;
-extern "C" void illm_set_attn_cap_groups(int n) { g_attn_cap_groups = n == 1 || n == 2 ? n : 0; }
 static int g_attn_cap_heads = 0;
 extern "C" void illm_set_attn_cap_heads(int n) { g_attn_cap_heads = (n == 1 || n == 2 || n == 4) ? n : 0; }
 
-extern "C" int illm_attn_cap_rows_of(const void* q, int q_stride, void* out, int dt, const int32_t* cu,
+extern "C" int illm_attn_cap_rows(const void* q, int q_stride, void* out, int dt, const int32_t* cu,
                                   const int32_t* seq_slot, const int32_t* seq_start,
                                   const void* kcache, const void* vcache, const int32_t* page_table,
                                   int table_stride, int page_size, int ring, int n_seqs, int max_rows,
@@ -868,7 +832,7 @@ extern "C" int illm_attn_cap_rows_of(const void* q, int q_stride, void* out, int
                                   const float* slopes, int chunk, const void* gate, int gate_stride,
                                   int gate_off, int gate_heads, float* lse, int keep, int kept,
                                   int own_stride, int own_k, int own_v_stride, int own_v, const float* sink,
-                                  int rows, void* stream) {
+                                  void* stream) {
     if (keep < 0 || kept < 0 || (keep > 0 && (window <= 0 || chunk > 0)) || own_stride < 0 ||
         (own_stride && (own_k < 0 || own_v < 0 || own_k + nkv * dk > own_stride || own_v + nkv * dv > own_v_stride)))
         return ILLM_ERR_ARG;
@@ -895,19 +859,14 @@ extern "C" int illm_attn_cap_rows_of(const void* q, int q_stride, void* out, int
         const bool bf16_rows = dt == ILLM_BF16 && g_attn_cap_mfma == 1 && dk % 8 == 0 && dv % 8 == 0 && q_stride % 8 == 0 &&
                                own_stride % 8 == 0 && own_k % 8 == 0 && own_v_stride % 8 == 0 && own_v % 8 == 0;
         if (bf16_rows) {
-            // Two groups of waves where the blocks that have rows are too few to fill the chip by themselves (at most
-            // rows / 128 + sequences a head); us with one / two groups: 8 sequences of 1,024 to 61 rows, 16 heads of 128 in
-            // chunks 97 / 84 from the step's rows, 91 / 68 from pages (without chunks 71 / 80, 65 / 60: rows without masks have
-            // less to do a tile), 32 heads 111 / 159; 4 of 500 to 100, 32 heads 55 / 50, 48 / 36; one of 4,000, 16 heads
-            // 233 / 246; 16 of 128, 32 heads 22 / 31.  Heads of up to 64: 8 of 1,024 to 61 82 / 55, one of 4,000 167 / 141, 64
-            // of 300 85 / 102.
-            const long long tiles = (max_rows + MQ - 1) / MQ * (long long)n_seqs;
-            const long long blocks = (rows > 0 && rows / MQ + n_seqs < tiles ? rows / MQ + n_seqs : tiles) * nh;
-            const int most = dk <= 64 && dv <= 64 ? 1025 : own_stride && !slopes && chunk <= 0 ? 385 : 512;
-            const int groups = g_attn_cap_groups ? g_attn_cap_groups : blocks < most ? 2 : 1;
-#define GOB(KT_, VT_) do { if (groups == 2) GOB_G(KT_, VT_, 2); else GOB_G(KT_, VT_, 1); } while (0)
-#define GOB_G(KT_, VT_, G_)                                                                        \
-    hipLaunchKernelGGL((attn_cap_rows_bf16_kernel<KT_, VT_, G_>), grid, dim3(256 * G_), 0, (hipStream_t)stream, \
+#define GOB(KT_, VT_)                                                                              \
+    do {                                                                                           \
+        if (own_stride) GOB_F(KT_, VT_, CAP_OWN_ROWS);                                             \
+        else if (page_size % MK == 0) GOB_F(KT_, VT_, CAP_TILED_PAGES);                            \
+        else GOB_F(KT_, VT_, CAP_ANY_PAGES);                                                       \
+    } while (0)
+#define GOB_F(KT_, VT_, FROM_)                                                                     \
+    hipLaunchKernelGGL((attn_cap_rows_bf16_kernel<KT_, VT_, FROM_>), grid, dim3(256), 0, (hipStream_t)stream, \
                        (const bf16_t*)q, q_stride, (bf16_t*)out, cu, seq_slot, seq_start, (const bf16_t*)kcache, \
                        (const bf16_t*)vcache, page_table, table_stride, page_size, ring, nh, nkv, dk, dv, scale, cap, \
                        window, slopes, chunk, (const bf16_t*)gate, gate_stride, gate_off, gate_heads, lse, keep, kept, \
@@ -919,7 +878,7 @@ extern "C" int illm_attn_cap_rows_of(const void* q, int q_stride, void* out, int
                           case 3: GOB_V(3) break; default: GOB_V(4) break; }
 #undef GOB_V
 #undef GOB
-#undef GOB_G
+#undef GOB_F
         } else if (dt == ILLM_BF16) { GO_K(ILLM_BF16) } else { GO_K(ILLM_F32) }
 #undef GO_K
 #undef GO_V
@@ -936,21 +895,6 @@ extern "C" int illm_attn_cap_rows_of(const void* q, int q_stride, void* out, int
                        page_table, table_stride, page_size, ring, nh, nkv, dk, dv, scale, cap, window, slopes,
                        chunk, gate, gate_stride, gate_off, gate_heads, lse, keep, kept, own_stride, own_k, own_v_stride, own_v, sink);
     return illm_launch_status();
-}
-
-extern "C" int illm_attn_cap_rows(const void* q, int q_stride, void* out, int dt, const int32_t* cu,
-                                  const int32_t* seq_slot, const int32_t* seq_start,
-                                  const void* kcache, const void* vcache, const int32_t* page_table,
-                                  int table_stride, int page_size, int ring, int n_seqs, int max_rows,
-                                  int nh, int nkv, int dk, int dv, float scale, float cap, int window,
-                                  const float* slopes, int chunk, const void* gate, int gate_stride,
-                                  int gate_off, int gate_heads, float* lse, int keep, int kept,
-                                  int own_stride, int own_k, int own_v_stride, int own_v, const float* sink,
-                                  void* stream) {
-    return illm_attn_cap_rows_of(q, q_stride, out, dt, cu, seq_slot, seq_start, kcache, vcache, page_table, table_stride,
-                                 page_size, ring, n_seqs, max_rows, nh, nkv, dk, dv, scale, cap, window, slopes, chunk, gate,
-                                 gate_stride, gate_off, gate_heads, lse, keep, kept, own_stride, own_k, own_v_stride, own_v,
-                                 sink, 0, stream);
 }
 
 // The keys a single token sees, numbered without a gap: with `keep` first tokens before the window the

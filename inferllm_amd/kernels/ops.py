@@ -1868,13 +1868,13 @@ def attn_cap_rows(q: torch.Tensor, cu_seqlens: torch.Tensor, seq_slot: torch.Ten
     _i32(cu_seqlens, n_seqs + 1); _i32(seq_slot, n_seqs); _i32(seq_start, n_seqs); _i32(page_table)
     _cap_cache_ok(q, kcache, vcache, page_table, page_size, nh, nkv, dk, dv, "attn_cap_rows")
     out = torch.empty((q.shape[0], nh * dv), dtype=q.dtype, device=q.device)
-    _check(_lib().illm_attn_cap_rows_of(
+    _check(_lib().illm_attn_cap_rows(
         _p(q), q.shape[1], _p(out), _code(q), _p(cu_seqlens), _p(seq_slot), _p(seq_start),
         _p(q if own is not None else kcache), _p(values if own is not None else vcache), _p(page_table),
         page_table.shape[1], page_size, ring, n_seqs, max_rows, nh, nkv,
         dk, dv, ctypes.c_float(scale), ctypes.c_float(cap), window, _p(slopes), int(chunk), _p(gate),
         gate.shape[1] if gate is not None else 0, gate_off, 1 if gate_heads else 0, _p(lse), int(keep),
-        int(kept), own_stride, own_k, own_v_stride, own_v, _p(sink), q.shape[0], _stream()),
+        int(kept), own_stride, own_k, own_v_stride, own_v, _p(sink), _stream()),
         f"attn_cap_rows (sizes {dk}, {dv})")
     return out
 

@@ -643,33 +643,54 @@ def test_an_activation_in_the_product_and_behind_it(name, N, K):
             assert torch.equal(ops().linear_act(rows, W, name), getattr(ops(), name)(ops().linear(rows, W)))
 
 
-@pytest.mark.parametrize("d,window,chunk,keep", [(128, 0, 0, 0), (128, 0, 96, 0), (64, 70, 0, 0), (32, 40, 0, 33), (40, 0, 0, 0)])
-def test_attn_cap_rows_groups(d, window, chunk, keep):
-    """Prompts' attention with the keys' tiles in turn by two groups of waves against one group (the same sums in
-    another order): odd and even numbers of tiles, a sequence of one row, masks that leave a group without keys, sinks
-    and the softmax's sums."""
-    nh, nkv, lens = 4, 2, [1, 31, 33, 128, 200, 7]
+@pytest.mark.parametrize("d,window,chunk,own", [(128, 0, 0, 1), (128, 0, 96, 0), (64, 70, 0, 0), (64, 0, 0, 1)])
+def test_capped_prompt_alone_and_among_others(d, window, chunk, own):
+    """A prompt's attention has the same bits whatever prompts stand beside it in the step."""
+    nh, nkv, lens = 16, 4, [300] + [128] * 70
+    T, B, page = sum(lens), len(lens), 64
+    rows = rnd(T, (nh + 2 * nkv) * d, seed=1).to(torch.bfloat16).to(DEV)
+    table = torch.arange(B * 5, dtype=torch.int32, device=DEV).view(B, 5)
+    kc, vc = (rnd(B * 5, nkv, page, d, seed=s).to(torch.bfloat16).to(DEV) for s in (2, 3))
+    got = []
+    for n in (1, B):
+        cu = torch.tensor([0] + torch.tensor(lens[:n]).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+        slot, start = torch.arange(n, dtype=torch.int32, device=DEV), torch.zeros(n, dtype=torch.int32, device=DEV)
+        got.append(ops().attn_cap_rows(rows[:sum(lens[:n])].contiguous(), cu, slot, start, kc, vc, table, page, 0, n, 300, nh,
+                                       nkv, d, d, d ** -0.5, 0.0, window, chunk=chunk,
+                                       own=(nh * d, (nh + nkv) * d) if own else None))
+    assert torch.equal(got[0], got[1][:300])
+
+
+@pytest.mark.parametrize("d,window,chunk,keep", [(128, 50, 0, 70), (64, 0, 90, 0), (40, 33, 0, 0), (128, 0, 0, 0)])
+def test_capped_prompt_over_pages_of_any_size(d, window, chunk, keep):
+    """Rows over the cache (steps that go on from it, shuffled pages, kept pages, rings that have gone round) have the
+    same bits whether pages are whole tiles of keys (64, 96: looked up once a tile) or not (20, 48), and are right."""
+    nh, nkv, starts, lens = 4, 2, [0, 45, 500], [70, 33, 140]
     T, B = sum(lens), len(lens)
-    q = rnd(T, (nh + 2 * nkv) * d, seed=1).to(torch.bfloat16).to(DEV)
-    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
-    slot, start = torch.arange(B, dtype=torch.int32, device=DEV), torch.zeros(B, dtype=torch.int32, device=DEV)
-    cache = torch.zeros(1, nkv, 64, d, dtype=torch.bfloat16, device=DEV)
-    table = torch.zeros(B, 4, dtype=torch.int32, device=DEV)
-    slopes, sink = rnd(nh, seed=2).abs().to(DEV) * 0.1, rnd(nh, seed=3).to(DEV)
-    lib, got = ops()._lib(), []
-    try:
-        for groups in (1, 2, 0):
-            lib.illm_set_attn_cap_groups(groups)
-            lse = torch.empty(T, nh, device=DEV)
-            out = ops().attn_cap_rows(q, cu, slot, start, cache, cache, table, 64, 0, B, max(lens), nh, nkv, d, d, d ** -0.5,
-                                      0.0, window, slopes=slopes, chunk=chunk, lse=lse, keep=keep, kept=0,
-                                      own=(nh * d, (nh + nkv) * d), sink=sink)
-            got.append((out.float(), lse))
-    finally:
-        lib.illm_set_attn_cap_groups(0)
-    for out, lse in got[1:]:
-        assert float((out - got[0][0]).abs().max()) <= 2.0 ** -8 * float(got[0][0].abs().max())
-        assert float((lse - got[0][1]).abs().max()) <= 1e-5 * float(got[0][1].abs().max())
+    g = torch.Generator().manual_seed(1)
+    q = rnd(T, nh * d, seed=1).to(torch.bfloat16)
+    k, v = (rnd(B, 640, nkv, d, seed=s).to(torch.bfloat16) for s in (2, 3))
+    cu = torch.tensor([0, 70, 103, 243], dtype=torch.int32)
+    slot, start = torch.tensor([2, 0, 1], dtype=torch.int32), torch.tensor(starts, dtype=torch.int32)
+    gate = rnd(T, nh * d + 4, seed=4).to(torch.bfloat16)
+    outs = []
+    for page in (64, 96, 48, 20):
+        kept = -(-keep // page)
+        ring = -(-(140 + 50) // page) + 1 if window else 0
+        per = kept + ring if ring else -(-640 // page)
+        table = torch.randperm(B * per, generator=g).view(B, per).to(torch.int32)
+        kc, vc = (torch.zeros(B * per, nkv, page, d, dtype=torch.bfloat16) for _ in range(2))
+        for b in range(B):
+            for pos in range(starts[b] + lens[b]):
+                at, r = R.cache_offsets(table, int(slot[b]), pos, page, ring, kept)
+                kc[at, :, r], vc[at, :, r] = k[b, pos], v[b, pos]
+        args = (page, ring, B, max(lens), nh, nkv, d, d, d ** -0.5, 0.0, window)
+        dev = [t.to(DEV) for t in (q, cu, slot, start, kc, vc, table)]
+        outs.append(ops().attn_cap_rows(*dev, *args, chunk=chunk, keep=keep, kept=kept, gate=gate.to(DEV), gate_off=4).cpu())
+    want = R.attn_cap_rows(q, cu, slot, start, kc, vc, table, *args, chunk=chunk, keep=keep, kept=kept, gate=gate, gate_off=4)
+    close(outs[-1], want, torch.bfloat16)
+    for got in outs[:-1]:
+        assert torch.equal(got, outs[-1])
 
 
 @pytest.mark.parametrize("dt,taps,shape", [(torch.bfloat16, 4, (2, 4, 8, 16)), (torch.float32, 3, (1, 2, 4, 36)), (torch.bfloat16, 2, (2, 2, 6, 20))])
