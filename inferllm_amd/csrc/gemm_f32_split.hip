@@ -72,7 +72,7 @@ f32_split_rows_kernel(const float* __restrict__ X, illm_u32x4_t* __restrict__ P,
 // A block of four waves takes MT * 16 rows of X and 64 * NT of W; a wave all those rows and 16 * NT of W's.
 template <int MT, int NT, int NS>
 __global__ void __launch_bounds__(256, 2)
-gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restrict__ X, const float* __restrict__ W,
+gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restrict__ X, const float* W,
                       void* __restrict__ Y, int y_dt, int M, int N, int K, int m_tiles, int splits) {
     constexpr int UNITS = MT * 3;                                              // KB of X a stage
     constexpr int LX = (UNITS + 3) / 4, L = LX + 2 * NT;                       // loads a wave a stage
@@ -178,19 +178,25 @@ gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restric
         load_w(ask, s + NS);
         if (s <= last) multiply(cur, p, next, pn);
     };
-    load_w(g0, first);
-    load_x(st0, first);
-    load_w(g1, first + 1);
-    load_x(st1, first + 1);
-    load_w(g2, first + 2);
+    // The counted waits need the loads in this order: what a wave has under way behind the wait of turn 0 must be later than
+    // stage 0 of X, which other waves read behind the barrier.  (The scheduler is held by the barriers here and in `turn`;
+    // selection is since W's pointer is not __restrict__: loads of memory that nothing writes float to any place.)
+    auto ask_ahead = [&](Raw& g, illm_u32x4_t* b, int s) __attribute__((always_inline)) {
+        load_w(g, s);
+        load_x(b, s);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    ask_ahead(g0, st0, first);
+    ask_ahead(g1, st1, first + 1);
     if constexpr (NS > 3) {
-        load_x(st2, first + 2);
-        load_w(g3, first + 3);
-        load_x(st3, first + 3);
-        load_w(g4, first + 4);
-        load_x(st4, first + 4);
+        ask_ahead(g2, st2, first + 2);
+        ask_ahead(g3, st3, first + 3);
+        ask_ahead(g4, st4, first + 4);
         load_w(g5, first + 5);
+    } else {
+        load_w(g2, first + 2);
     }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int e = 0; e < 4 * NT; ++e) split_part(g0, p0, e);
     for (int s = first; s <= last; s += 6) {

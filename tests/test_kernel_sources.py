@@ -1,8 +1,10 @@
 """What the kernels' sources have to say for themselves, read as text: facts that no run on the hardware shows."""
 import os
 import re
+import subprocess
 
 import inferllm_amd
+from inferllm_amd.kernels import build
 
 CSRC = os.path.join(os.path.dirname(inferllm_amd.__file__), "csrc")
 SOURCES = {f: open(os.path.join(CSRC, f)).read() for f in sorted(os.listdir(CSRC)) if f.endswith((".hip", ".h"))}
@@ -17,3 +19,28 @@ def test_dynamic_lds_is_declared_on_16_bytes():
             found += 1
             assert "__attribute__((aligned(16)))" in line, (name, line)
     assert found >= 20
+
+
+def test_the_float32_parts_loads_are_issued_in_the_order_their_waits_count(tmp_path):
+    """The product in bfloat16 parts waits for "all but the youngest n" loads before other waves read what a wave brought
+    into LDS: in the compiled code W's loads (registers) and X's (LDS) stand stage by stage, and no load moves
+    from one turn to another."""
+    out = str(tmp_path / "parts.s")
+    subprocess.run([build._hipcc()] + build.HIPCC_FLAGS + ["--offload-device-only", "-S", "-o", out,
+                                                           os.path.join(CSRC, "gemm_f32_split.hip")], check=True,
+                   stderr=subprocess.DEVNULL)
+    kernels = re.findall(r"^_Z\w*gemm_f32_split_kernelILi(\d+)ELi(\d+)ELi(\d+)E\w*:(.*?)s_endpgm", open(out).read(),
+                         re.S | re.M)
+    assert len(kernels) >= 10
+    for mt, nt, ns, body in kernels:
+        mt, nt, ns = int(mt), int(nt), int(ns)
+        x, w = "X" * ((3 * mt + 3) // 4), "W" * (2 * nt)
+        stages = []
+        for part in body.split("s_barrier")[:4]:
+            loads = [line for line in part.splitlines() if re.search(r"\b(buffer|global)_load", line)]
+            stages.append("".join("X" if "lds" in line else "W" for line in loads))
+        # ahead of the first wait ns - 1 stages and W of one more; then a stage a turn
+        assert stages[0] == (w + x) * (ns - 1) + w, (mt, nt, ns, stages[0])
+        assert stages[1:] == [x + w] * 3, (mt, nt, ns, stages)
+        waits = re.findall(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)\s*\n\s*s_barrier", body)
+        assert waits and set(waits) == {str((ns - 2) * len(x + w))}, (mt, nt, ns, waits)
