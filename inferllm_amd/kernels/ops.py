@@ -583,12 +583,9 @@ def gemm_rows_f32_mfma_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def gemm_rows_f32_mfma(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     """x [M <= 128, K] . w [N, K]^T, both float32, W read once, on the matrix cores' float32
-    instruction; large matrices in bfloat16 parts (`gemm_f32_split`).  A row's sum does not depend on the other rows
-    or on their number."""
+    instruction.  A row's sum does not depend on the other rows or on their number."""
     _gpu(x, w)
     _need(gemm_rows_f32_mfma_fits(x, w), "gemm_rows_f32_mfma: operands not taken")
-    if _split_large(w) and gemm_f32_split_fits(x, w):
-        return gemm_f32_split(x, w, out_dtype)
     M, K = x.shape
     N = w.shape[0]
     y = torch.empty((M, N), dtype=out_dtype, device=x.device)
