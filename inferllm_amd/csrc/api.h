@@ -112,12 +112,13 @@ int illm_gemm_f32_mfma(const float* X, const float* W, void* Y, int y_dt, int M,
 
 // The same product for float32 X and W with K % 32 == 0 on the matrix cores' bfloat16 instruction:
 // operands as the sum of three bfloat16 parts, six products of parts (csrc/gemm_f32_split.hip).  P: scratch of
-// 6 K illm_gemm_f32_split_rows(M) bytes.  splits 1: Y [M, N] in y_dt; more: float32 planes [splits][M][N] of parts of K
-// (illm_gemm_f32_split_parts, or any number that leaves no part empty).  All on 16-byte addresses.
+// 6 K illm_gemm_f32_split_rows(M) bytes.  K is summed in parts of `per` stages of 32 (0: one), the parts added in order:
+// planes 0: Y [M, N] in y_dt, per a multiple of 6; else Y the parts' float32 planes.  All on 16-byte addresses.
 int illm_gemm_f32_split_rows(int M);
-int illm_gemm_f32_split_parts(int M, int N, int K);
+int illm_gemm_f32_split_per(int M, int N, int K);       // the library's `per`, the same up to 128 rows and above
+int illm_gemm_f32_split_planes(int M, int N, int K);    // whether planes are the faster way
 int illm_gemm_f32_split(const float* X, const float* W, void* P, size_t p_bytes, void* Y, int y_dt, int M, int N,
-                        int K, int splits, void* stream);
+                        int K, int per, int planes, void* stream);
 // Y [n] (n % 4 == 0) in y_dt = the sum of float32 planes [S][n], in order.
 int illm_f32_planes_sum(const float* planes, void* Y, int y_dt, int S, size_t n, void* stream);
 

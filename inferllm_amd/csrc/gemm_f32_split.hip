@@ -69,11 +69,13 @@ f32_split_rows_kernel(const float* __restrict__ X, illm_u32x4_t* __restrict__ P,
     for (int i = 0; i < 3; ++i) to[64 * i] = p[i];
 }
 
-// A block of four waves takes MT * 16 rows of X and 64 * NT of W; a wave all those rows and 16 * NT of W's.
-template <int MT, int NT, int NS>
+// A block of four waves takes MT * 16 rows of X and 64 * NT of W; a wave all those rows and 16 * NT of W's.  K is summed in
+// parts of `per` stages, and the parts' sums are added in order: by whoever reads the planes, a part a block (grid y), or in
+// here (FOLD, per a multiple of 6), one part after the other.  Both ways give the same bits.
+template <int MT, int NT, int NS, bool FOLD>
 __global__ void __launch_bounds__(256, 2)
 gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restrict__ X, const float* W,
-                      void* __restrict__ Y, int y_dt, int M, int N, int K, int m_tiles, int splits) {
+                      void* __restrict__ Y, int y_dt, int M, int N, int K, int m_tiles, int per) {
     constexpr int UNITS = MT * 3;                                              // KB of X a stage
     constexpr int LX = (UNITS + 3) / 4, L = LX + 2 * NT;                       // loads a wave a stage
     __shared__ illm_u32x4_t st0[UNITS * 64], st1[UNITS * 64], st2[UNITS * 64];
@@ -84,8 +86,8 @@ gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restric
     const int xcd = blockIdx.x & 7, j8 = blockIdx.x >> 3;
     const int mt = j8 % m_tiles, n0 = ((j8 / m_tiles) * 8 + xcd) * (64 * NT);
     if (n0 >= N) return;
-    const int every = K / SP_K, per = (every + splits - 1) / splits;
-    const int first = blockIdx.y * per, last = min(first + per, every) - 1;
+    const int every = K / SP_K;
+    const int first = FOLD ? 0 : blockIdx.y * per, last = FOLD ? every - 1 : min(first + per, every) - 1;
 
     const __amdgpu_buffer_rsrc_t xr = illm_buffer(P, (size_t)every * m_tiles * UNITS * 1024);
     const uint32_t x_stage = (uint32_t)m_tiles * UNITS * 1024, x_lane = (uint32_t)mt * UNITS * 1024 + lane * 16;
@@ -199,6 +201,27 @@ gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restric
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int e = 0; e < 4 * NT; ++e) split_part(g0, p0, e);
+    // What a part's sums are: acc[i][j][v] is row (wave * NT + i) * 16 + 4 q + v of W's, row 16 j + r of X's.  A sum that is
+    // no finite number is taken again with plain multiply-adds: an infinity has no parts.
+    auto part_sum = [&](int i, int j, int s0, int s1) __attribute__((always_inline)) {
+        const int m = (mt * MT + j) * 16 + r, n = n0 + (wave * NT + i) * 16 + 4 * q;
+        f32x4_t v = acc[i][j] + low[i][j];
+        bool odd = false;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) odd |= (__float_as_uint(v[e]) & 0x7f800000u) == 0x7f800000u;
+        if (odd && m < M) {
+            for (int e = 0; e < 4; ++e) {
+                if (n + e >= N) break;
+                float t = 0.f;
+                for (int k = s0 * SP_K; k <= s1 * SP_K + SP_K - 1; ++k)
+                    t = fmaf(X[(size_t)m * K + k], W[(size_t)(n + e) * K + k], t);
+                v[e] = t;
+            }
+        }
+        return v;
+    };
+    f32x4_t tot[FOLD ? NT : 1][FOLD ? MT : 1];
+    int part = first;                               // FOLD: where the part under way began
     for (int s = first; s <= last; s += 6) {
         if constexpr (NS == 3) {
             turn(st0, st2, p0, p1, g1, g0, s);
@@ -215,31 +238,31 @@ gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restric
             turn(st4, st3, p0, p1, g5, g4, s + 4);
             turn(st5, st4, p1, p0, g0, g5, s + 5);
         }
+        if constexpr (FOLD) {
+            if (s + 6 - part < per && s + 6 <= last) continue;
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int j = 0; j < MT; ++j) {
+                    const f32x4_t v = part_sum(i, j, part, min(s + 5, last));
+                    tot[i][j] = part == 0 ? v : tot[i][j] + v;
+                    acc[i][j] = low[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+                }
+            part = s + 6;
+        }
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);             // no load into LDS outlives the block
 
-    // acc[i][j][v]: row (wave * NT + i) * 16 + 4 q + v of W's, row 16 j + r of X's.  A sum that is no finite
-    // number is taken again with plain multiply-adds: an infinity has no parts.
-    const int k0 = first * SP_K, k1 = (last + 1) * SP_K;
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
         const int m = (mt * MT + j) * 16 + r;
-        if (m >= M) continue;
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
             const int n = n0 + (wave * NT + i) * 16 + 4 * q;
-            f32x4_t v = acc[i][j] + low[i][j];
-            bool odd = false;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) odd |= (__float_as_uint(v[e]) & 0x7f800000u) == 0x7f800000u;
-            if (odd) {
-                for (int e = 0; e < 4; ++e) {
-                    if (n + e >= N) break;
-                    float t = 0.f;
-                    for (int k = k0; k < k1; ++k) t = fmaf(X[(size_t)m * K + k], W[(size_t)(n + e) * K + k], t);
-                    v[e] = t;
-                }
-            }
+            f32x4_t v;
+            if constexpr (FOLD) v = tot[i][j];
+            else v = part_sum(i, j, first, last);
+            if (m >= M) continue;
             const size_t at = ((size_t)blockIdx.y * M + m) * N + n;
             if (n + 3 < N && (N & 3) == 0 && y_dt == ILLM_F32) {
                 *(f32x4_t*)((float*)Y + at) = v;
@@ -266,58 +289,73 @@ struct SplitTiles { int mt, nt, m_tiles, blocks; };
 
 // Rows in equal tiles of at most 128.  Along W a block takes 64 or 128: a compute unit works through its blocks
 // in rounds of 256, and one of 128 takes 1.8 times one of 64 (245 rows, us with 128 / with 64: 12288 x 4096
-// 146 / 164, 22016 x 4096 263 / 252; 64 rows: 94 / 70 and 112 / 129; 900 rows of 22016 x 4096 789 / 850).
-static SplitTiles split_tiles(int M, int N, int splits) {
+// 146 / 164, 22016 x 4096 263 / 252; 64 rows: 94 / 70 and 112 / 129; 900 rows of 22016 x 4096 789 / 850).  A block of a part
+// takes 128, one that adds up its parts 64 (their sums need the registers).
+static SplitTiles split_tiles(int M, int N, bool planes, bool fold) {
     const int tiles = (M + 15) / 16, m_tiles = (tiles + 7) / 8, need = (tiles + m_tiles - 1) / m_tiles;
     const int mt = need <= 2 ? need : need <= 4 ? 4 : need <= 6 ? 6 : 8;
     const int b1 = (N + 63) / 64 * m_tiles, b2 = (N + 127) / 128 * m_tiles;
-    const bool wide = splits > 1 || 10 * 23 * ((b2 + 255) / 256) <= 10 * 13 * ((b1 + 255) / 256);
+    const bool wide = !fold && (planes || 10 * 23 * ((b2 + 255) / 256) <= 10 * 13 * ((b1 + 255) / 256));
     return {mt, wide ? 2 : 1, m_tiles, wide ? b2 : b1};
 }
 
-// Parts of K for about one block a compute unit where the tiles are fewer (than 160 of 64 columns): at most 8, each of
-// at least 16 stages, none empty.  The same for all rows up to 128.
-extern "C" int illm_gemm_f32_split_parts(int M, int N, int K) {
-    if (M <= 0 || N <= 0 || K < SP_K) return 1;
-    const SplitTiles t = split_tiles(M, N, 2);
-    if ((N + 63) / 64 * t.m_tiles >= 160) return 1;
-    const int every = K / SP_K, s = max(1, min(min(256 / t.blocks, 8), every / 16)), per = (every + s - 1) / s;
-    return (every + per - 1) / per;
+// Stages of 32 k in a part of K, 0 where K is one part.  A row's bits hang on them, so they are the same for all numbers
+// of rows up to 128 and for all above: parts for about one block a compute unit at 128 and at 256 rows where the tiles are
+// fewer (than 160 of 64 columns), at most 8, each of at least 16 stages; a multiple of 6 (a round of the kernel's loop).
+extern "C" int illm_gemm_f32_split_per(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K < SP_K) return 0;
+    const int m_tiles = M <= 128 ? 1 : 2, blocks = (N + 127) / 128 * m_tiles;
+    if ((N + 63) / 64 * m_tiles >= 160) return 0;
+    const int every = K / SP_K, s = max(1, min(min(256 / blocks, 8), every / 16)), per = ((every + s - 1) / s + 5) / 6 * 6;
+    return per >= every ? 0 : per;
+}
+
+// Whether the parts of so many rows are taken by a block each (planes that somebody adds) and not one after the other by the
+// same blocks: up to 128 MB of planes (us, planes and their sum / in one: 245 / 1,024 / 2,048 rows of 4096 x 4096 60 / 177 /
+// 346 against 95 / 180 / 364, of 4096 x 11008 124 / 430 / 841 against 240 / 457 / 909, of 2048 x 2048 33 / 61 / 107 against
+// 51 / 56 / 97; all of K in one part, as it had been from 257 rows on, 4096 x 4096 163 / 314 at 1,024 / 2,048).
+extern "C" int illm_gemm_f32_split_planes(int M, int N, int K) {
+    const int per = illm_gemm_f32_split_per(M, N, K);
+    if (!per || N % 4) return 0;
+    return (long long)((K / SP_K + per - 1) / per) * M * N <= 1 << 25;
 }
 
 // Rows of X as its parts are laid out (M filled up to whole tiles): 6 bytes of scratch for each of their K.
 extern "C" int illm_gemm_f32_split_rows(int M) {
     if (M <= 0) return 0;
-    const SplitTiles t = split_tiles(M, 64, 1);
+    const SplitTiles t = split_tiles(M, 64, false, true);
     return t.m_tiles * t.mt * 16;
 }
 
-// float32 X [M, K] and W [N, K] on 16-byte addresses, K % 32 == 0; P: scratch of 6 K
-// illm_gemm_f32_split_rows(M) bytes (at most 4 GiB).  splits 1: Y [M, N], float32 or bfloat16; more: float32 planes [splits][M][N], no part
-// of K empty.
+// float32 X [M, K] and W [N, K] on 16-byte addresses, K % 32 == 0; P: scratch of 6 K illm_gemm_f32_split_rows(M) bytes
+// (at most 4 GiB).  per: stages of 32 k in a part of K, 0 for one part.  planes 0: Y [M, N], float32 or bfloat16, per a
+// multiple of 6; else the parts' float32 planes [ceil(K / 32 per)][M][N].
 extern "C" int illm_gemm_f32_split(const float* X, const float* W, void* P, size_t p_bytes, void* Y, int y_dt, int M,
-                                   int N, int K, int splits, void* stream) {
+                                   int N, int K, int per, int planes, void* stream) {
     if (M <= 0 || N <= 0 || K <= 0 || K % SP_K || K >= 1 << 22 || !illm_dtype_ok(y_dt) || !X || !W || !Y || !P ||
-        splits < 1 || splits > 65535 || (splits > 1 && y_dt != ILLM_F32) || ((uintptr_t)X | (uintptr_t)W | (uintptr_t)P | (uintptr_t)Y) % 16)
+        per < 0 || (planes && y_dt != ILLM_F32) || ((uintptr_t)X | (uintptr_t)W | (uintptr_t)P | (uintptr_t)Y) % 16)
         return ILLM_ERR_ARG;
-    const int every = K / SP_K, per = (every + splits - 1) / splits;
-    const SplitTiles t = split_tiles(M, N, splits);
+    const int every = K / SP_K;
+    if (per == 0 || per >= every) per = every;
+    const bool fold = !planes && per < every;
+    const int parts = planes ? (every + per - 1) / per : 1;
+    const SplitTiles t = split_tiles(M, N, parts > 1, fold);
     const size_t need = (size_t)t.m_tiles * t.mt * 16 * K * 6;
     const long long grid_x = ((long long)(t.blocks / t.m_tiles) + 7) / 8 * 8 * t.m_tiles;
-    if ((long long)(splits - 1) * per >= every || need > p_bytes || need > 0xffffffffu || grid_x > 0x7fffffff ||
+    if ((fold && per % 6) || parts > 65535 || need > p_bytes || need > 0xffffffffu || grid_x > 0x7fffffff ||
         t.m_tiles * t.mt > 65535)
         return ILLM_ERR_ARG;
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(f32_split_rows_kernel, dim3((every + 3) / 4, t.m_tiles * t.mt), dim3(256), 0, st, X,
                        (illm_u32x4_t*)P, M, K, t.m_tiles * t.mt);
-    const dim3 grid((unsigned)grid_x, splits);
-#define ILLM_SPLIT(MT, NT, NS)                                                                                      \
-    if (t.mt == MT && t.nt == NT)                                                                                   \
-        hipLaunchKernelGGL((gemm_f32_split_kernel<MT, NT, NS>), grid, dim3(256), 0, st, (const illm_u32x4_t*)P, X, W, \
-                           Y, y_dt, M, N, K, t.m_tiles, splits)
-    ILLM_SPLIT(1, 1, 6); ILLM_SPLIT(1, 2, 6); ILLM_SPLIT(2, 1, 6); ILLM_SPLIT(2, 2, 6);
-    ILLM_SPLIT(4, 1, 6); ILLM_SPLIT(4, 2, 6); ILLM_SPLIT(6, 1, 3); ILLM_SPLIT(6, 2, 3); ILLM_SPLIT(8, 1, 3);
-    ILLM_SPLIT(8, 2, 3);
+    const dim3 grid((unsigned)grid_x, parts);
+#define ILLM_SPLIT(MT, NT, NS, FOLD)                                                                                \
+    if (t.mt == MT && t.nt == NT && fold == FOLD)                                                                   \
+        hipLaunchKernelGGL((gemm_f32_split_kernel<MT, NT, NS, FOLD>), grid, dim3(256), 0, st, (const illm_u32x4_t*)P, X, \
+                           W, Y, y_dt, M, N, K, t.m_tiles, per)
+#define ILLM_SPLIT_ROWS(MT, NS) ILLM_SPLIT(MT, 1, NS, false); ILLM_SPLIT(MT, 2, NS, false); ILLM_SPLIT(MT, 1, NS, true)
+    ILLM_SPLIT_ROWS(1, 6); ILLM_SPLIT_ROWS(2, 6); ILLM_SPLIT_ROWS(4, 6); ILLM_SPLIT_ROWS(6, 3); ILLM_SPLIT_ROWS(8, 3);
+#undef ILLM_SPLIT_ROWS
 #undef ILLM_SPLIT
     return illm_launch_status();
 }

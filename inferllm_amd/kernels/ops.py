@@ -604,35 +604,36 @@ def gemm_f32_split_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def gemm_f32_split_pays(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether it is the faster way for operands that it takes.  Parting X and the sums of K's parts cost 4 to 8 us,
-    so short sums and small matrices stay with the kernels of the float32 instruction (whose time grows with K).
-    us there -> here, matrices cold: 33 / 100 rows of 2048 x 2048 17 / 38 -> 22 / 30;
-    17 rows of 4096 x 4096 28 -> 26, of 2048 x 2048 14 -> 20, of 8192 x 2048 27 -> 24; 9 of 4096 x 11008 55 -> 51, of
-    12288 x 4096 55 -> 58; 700 of 4096 x 1024 65 -> 49, of 1024 x 1024 25 -> 34; 2,048 of 1024 x 256 15 -> 19.  Large:
-    64 / 256 / 2,048 rows of 22016 x 4096 203 / 429 / 2,877 -> 118 / 267 / 1,576, of 4096 x 11008 135 / 219 / 1,412 ->
-    62 / 134 / 827.  Largest error against 64 bits 1.9e-6 -> 6.7e-7."""
+    """Whether it is the faster way for operands that it takes.  The matrix decides, once for 9 to 128 rows and once for all
+    above: a row's bits are the same whatever the number of rows in either range.  us by the float32 instruction -> here,
+    matrices cold; 9 / 16 / 33 / 128 rows: 22016 x 4096 98 / 112 / 162 / 357 -> 99 / 100 / 120 / 157, 12288 x 4096 53 / 59 / 97 /
+    241 -> 53 / 54 / 70 / 103, 6144 x 4096 36 / 40 / 56 / 155 -> 33 / 33 / 34 / 50, 2048 x 8192 32 / 37 / 55 / 154 -> 32 / 33 /
+    36 / 50, 4096 x 4096 20 / 23 / 34 / 80 -> 26 / 26 / 30 / 38 (the slower way up to 16 rows by 3 to 5 us, of 230 that a layer of
+    such matrices takes; 3 less as planes for a norm); 8192 x 2048, which stays there, 19 / 21 / 30 / 81 -> 24 / 24 / 25 / 38.
+    129 / 256 / 2,048 rows: 22016 x 4096 365 / 439 / 2,865 -> 220 / 265 / 1,580, 4096 x 4096 82 / 84 / 532 -> 46 / 56 / 345,
+    4096 x 11008 221 / 226 / 1,405 -> 105 / 127 / 850, 1024 x 2048 42 / 42 / 77 -> 26 / 31 / 64, 6144 x 1024 41 / 40 / 211 -> 25 /
+    31 / 124, 4096 x 1536 33 / 34 / 206 -> 28 / 33 / 135, 12288 x 512 31 / 33 / 219 -> 23 / 28 / 129; 4096 x 1024, which stays, 25 /
+    24 / 141 -> 27 / 31 / 88, as does 2048 x 1536, 32 / 33 / 111 -> 27 / 32 / 76, for 400 rows of it 33 -> 34."""
     M, (N, K) = x.shape[0], w.shape
-    if K < 2048:
-        return K >= 512 and M * N >= 1400000
-    if N < 1024:
+    if M < ROWS_F32_MFMA_FROM or N < 1024:
         return False
-    return M >= (9 if _split_large(w) or K >= 8192 else 17 if K >= 4096 or N * K >= 1 << 24 else 65)
-
-
-def _split_large(w: torch.Tensor) -> bool:
-    """Matrices whose products of up to 128 rows are parted whatever the rows (so that a row's bits do not depend on
-    their number): 16 rows of 12288 x 4096 60 -> 58 us, of 22016 x 4096 110 -> 98; 9 rows 55 -> 58 and 96 -> 97."""
-    return w.shape[0] >= 1024 and w.shape[1] >= 2048 and w.shape[0] * w.shape[1] >= 1 << 25
+    if M <= 128:
+        return K >= 2048 and (N * K >= 3 << 23 or K >= 8192 or (K >= 4096 and N * K >= 1 << 24))
+    return K >= 2048 or (K >= 512 and N >= 4096 and N * K >= 3 << 21)
 
 
 def _f32_split(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, S: int) -> torch.Tensor:
-    """[M, N] (S = 1) or float32 planes [S, M, N]."""
+    """[M, N] (S = 1), or float32 planes [S, M, N] of parts of K that are added in order (S = 0: the library's parts)."""
     _gpu(x, w)
     (M, K), N = x.shape, w.shape[0]
+    every = K // 32
+    per = -(-every // S) if S > 1 else _lib().illm_gemm_f32_split_per(M, N, K) or every
+    planes = -(-every // per) if S != 1 else 0
+    _need(S <= 1 or planes == S, f"gemm_f32_split: {S} parts of {every} stages")
     parts = torch.empty(_lib().illm_gemm_f32_split_rows(M) * K * 6, dtype=torch.uint8, device=x.device)
-    y = torch.empty((M, N) if S == 1 else (S, M, N), dtype=out_dtype, device=x.device)
-    _check(_lib().illm_gemm_f32_split(_p(x), _p(w), _p(parts), ctypes.c_size_t(parts.numel()), _p(y), _code(y), M, N, K, S,
-                                      _stream()), "gemm_f32_split")
+    y = torch.empty((planes, M, N) if planes else (M, N), dtype=out_dtype, device=x.device)
+    _check(_lib().illm_gemm_f32_split(_p(x), _p(w), _p(parts), ctypes.c_size_t(parts.numel()), _p(y), _code(y), M, N, K, per,
+                                      1 if planes else 0, _stream()), "gemm_f32_split")
     return y
 
 
@@ -641,12 +642,12 @@ def gemm_f32_split(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype) -> 
     than a float32 sum of float32 products (csrc/gemm_f32_split.hip)."""
     _need(gemm_f32_split_fits(x, w), "gemm_f32_split: operands not taken")
     (M, K), N = x.shape, w.shape[0]
-    S = _lib().illm_gemm_f32_split_parts(M, N, K) if N % 4 == 0 else 1
-    if S == 1:
+    if not _lib().illm_gemm_f32_split_planes(M, N, K):
         return _f32_split(x, w, out_dtype, 1)
-    planes = _f32_split(x, w, torch.float32, S)
+    planes = _f32_split(x, w, torch.float32, 0)
     y = torch.empty((M, N), dtype=out_dtype, device=x.device)
-    _check(_lib().illm_f32_planes_sum(_p(planes), _p(y), _code(y), S, ctypes.c_size_t(M * N), _stream()), "f32_planes_sum")
+    _check(_lib().illm_f32_planes_sum(_p(planes), _p(y), _code(y), planes.shape[0], ctypes.c_size_t(M * N), _stream()),
+           "f32_planes_sum")
     return y
 
 
@@ -867,8 +868,8 @@ def linear_cut_fits(x, w) -> bool:
     16-byte addresses and within a load's 32-bit offset; or float32 operands whose K `gemm_f32_split` cuts."""
     w = plain_weight(w)
     if isinstance(x, torch.Tensor) and x.dtype == torch.float32 and w.dtype == torch.float32:
-        return (gemm_f32_split_fits(x, w) and gemm_f32_split_pays(x, w) and w.shape[0] % 4 == 0
-                and _lib().illm_gemm_f32_split_parts(x.shape[0], w.shape[0], w.shape[1]) > 1)
+        return (gemm_f32_split_fits(x, w) and gemm_f32_split_pays(x, w)
+                and bool(_lib().illm_gemm_f32_split_planes(x.shape[0], w.shape[0], w.shape[1])))
     if not (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and x.dim() == 2 and w.dim() == 2 and CUT_ROWS[0] <= x.shape[0] <= CUT_ROWS[1]
             and x.shape[1] == w.shape[1] and w.is_contiguous()):
@@ -887,7 +888,7 @@ def linear_cut(x: torch.Tensor, w, splits: int = 0) -> torch.Tensor:
     M, K = x.shape
     N = w.shape[0]
     if x.dtype == torch.float32:
-        return _f32_split(x, w, torch.float32, splits or _lib().illm_gemm_f32_split_parts(M, N, K))
+        return _f32_split(x, w, torch.float32, splits)
     S = splits or _lib().illm_gemm_tiles_splits(N, K)
     y = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
     _check(_lib().illm_gemm_tiles_planes(_p(x), _p(w), _p(y), M, N, K, S, _stream()), "linear_cut")

@@ -578,6 +578,24 @@ def test_gemm_f32_split(M, N, K, S):
     assert not ops().gemm_f32_split_fits(rnd(M, K + 16).to(DEV), rnd(N, K + 16).to(DEV))
 
 
+@pytest.mark.parametrize("N,K", [(12288, 2048), (4096, 4096), (1024, 8192), (4098, 4096), (2048, 2048), (4096, 1024), (12288, 512), (1028, 2080)])
+def test_f32_rows_alone_and_among_others(N, K):
+    """A row of a float32 product has the same bits in steps of 9 to 128 rows, and in steps of more, with the parts of K
+    as planes or one after the other: from `linear` and, where it takes them, as `linear_cut`'s planes added in order."""
+    x, w = rnd(1100, K, seed=1).to(DEV), rnd(N, K, seed=2).to(DEV)
+    for sizes in ((128, 9, 16, 17, 64, 65, 100), (1100, 129, 200, 257, 384, 500, 640, 900)):
+        want = ops().linear(x[:sizes[0]].contiguous(), w)
+        for M in sizes:
+            rows = x[:M].contiguous()
+            assert torch.equal(ops().linear(rows, w), want[:M])
+            if ops().linear_cut_fits(rows, w):
+                planes = ops().linear_cut(rows, w)
+                got = planes[0].clone()
+                for p in planes[1:]:
+                    got += p
+                assert torch.equal(got, want[:M])
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 32), (8, 24, 96), (3, 2048, 1056), (8, 2040, 4096), (7, 520, 2048), (5, 100, 1024),
                                    (8, 2048, 8192), (9, 2048, 1024), (16, 40, 64)])
 def test_skinny_half_tiles_and_activations(M, N, K):

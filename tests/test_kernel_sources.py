@@ -29,9 +29,9 @@ def test_the_float32_parts_loads_are_issued_in_the_order_their_waits_count(tmp_p
     subprocess.run([build._hipcc()] + build.HIPCC_FLAGS + ["--offload-device-only", "-S", "-o", out,
                                                            os.path.join(CSRC, "gemm_f32_split.hip")], check=True,
                    stderr=subprocess.DEVNULL)
-    kernels = re.findall(r"^_Z\w*gemm_f32_split_kernelILi(\d+)ELi(\d+)ELi(\d+)E\w*:(.*?)s_endpgm", open(out).read(),
+    kernels = re.findall(r"^_Z\w*gemm_f32_split_kernelILi(\d+)ELi(\d+)ELi(\d+)ELb[01]E\w*:(.*?)\.Lfunc_end", open(out).read(),
                          re.S | re.M)
-    assert len(kernels) >= 10
+    assert len(kernels) >= 15
     for mt, nt, ns, body in kernels:
         mt, nt, ns = int(mt), int(nt), int(ns)
         x, w = "X" * ((3 * mt + 3) // 4), "W" * (2 * nt)
