@@ -596,6 +596,27 @@ def test_f32_rows_alone_and_among_others(N, K):
                 assert torch.equal(got, want[:M])
 
 
+@pytest.mark.parametrize("K", [64, 512])
+@pytest.mark.parametrize("M,N", [(17, 130), (129, 68)])
+def test_gemm_f32_split_over_the_range_of_float32(M, N, K):
+    """The parts hold a float32 number exactly from the smallest normal one up: rows and matrices of any magnitude
+    (beyond 2^104, and where the sums pass 2^80, by plain multiply-adds), subnormals among larger numbers, and operands
+    of one sign whose left-out products of parts all add up.  Errors within what float32 sums of K products may
+    have, 2^-24 for each addition of the sum of absolute products, and 2^-24 of it for what is left out."""
+    g = torch.Generator().manual_seed(1)
+    for ex, ew in ((0, 0), (-118, 0), (-124, 0), (-124, 100), (0, -122), (60, -125), (100, -100), (112, -100), (-100, 112), (60, 58)):
+        x, w = torch.randn(M, K, generator=g).clamp(-4, 4) * 2.0 ** ex, torch.randn(N, K, generator=g).clamp(-4, 4) * 2.0 ** ew
+        x[0, ::2] *= 2.0 ** -20
+        got = ops().gemm_f32_split(x.to(DEV), w.to(DEV), torch.float32).double().cpu()
+        bound = 2.0 ** -24 * (K + 1) * (x.double().abs() @ w.double().abs().t()) + 2.0 ** -148
+        assert bool(((got - x.double() @ w.double().t()).abs() <= bound).all()), (ex, ew)
+    one = torch.tensor([0x3f807fc0], dtype=torch.int32).view(torch.float32)
+    x, w = one.expand(M, K).contiguous(), -one.expand(N, K).contiguous()
+    want = x.double() @ w.double().t()
+    err = lambda y: float(((y.double().cpu() - want) / want).abs().max())  # noqa: E731
+    assert err(ops().gemm_f32_split(x.to(DEV), w.to(DEV), torch.float32)) <= 2.0 ** -24 * (K / 32 + 2)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 32), (8, 24, 96), (3, 2048, 1056), (8, 2040, 4096), (7, 520, 2048), (5, 100, 1024),
                                    (8, 2048, 8192), (9, 2048, 1024), (16, 40, 64)])
 def test_skinny_half_tiles_and_activations(M, N, K):
