@@ -78,22 +78,22 @@ f32_split_rows_kernel(const float* __restrict__ X, illm_u32x4_t* __restrict__ P,
     for (int i = 0; i < 3; ++i) to[64 * i] = p[i];
 }
 
-// A block of four waves takes MT * 16 rows of X and 64 * NT of W; a wave all those rows and 16 * NT of W's.  K is summed in
+// A block of NW waves takes MT * 16 rows of X and 16 * NW * NT of W; a wave all those rows and 16 * NT of W's.  K is summed in
 // parts of `per` stages, and the parts' sums are added in order: by whoever reads the planes, a part a block (grid y), or in
 // here (FOLD, per a multiple of 6), one part after the other.  Both ways give the same bits.
-template <int MT, int NT, int NS, bool FOLD>
-__global__ void __launch_bounds__(256, 2)
+template <int MT, int NT, int NS, bool FOLD, int NW = 4>
+__global__ void __launch_bounds__(64 * NW, 2)
 gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restrict__ X, const float* W,
                       void* __restrict__ Y, int y_dt, int M, int N, int K, int m_tiles, int per) {
     constexpr int UNITS = MT * 3;                                              // KB of X a stage
-    constexpr int LX = (UNITS + 3) / 4, L = LX + 2 * NT;                       // loads a wave a stage
+    constexpr int LX = (UNITS + NW - 1) / NW, L = LX + 2 * NT;                       // loads a wave a stage
     __shared__ illm_u32x4_t st0[UNITS * 64], st1[UNITS * 64], st2[UNITS * 64];
     __shared__ illm_u32x4_t st3[NS > 3 ? UNITS * 64 : 1], st4[NS > 3 ? UNITS * 64 : 1], st5[NS > 3 ? UNITS * 64 : 1];
     const int lane = threadIdx.x & 63, wave = wave_index();
     const int r = lane & 15, q = lane >> 4;
     // the blocks that share rows of W run next to each other on one XCD (block ids go round the 8)
     const int xcd = blockIdx.x & 7, j8 = blockIdx.x >> 3;
-    const int mt = j8 % m_tiles, n0 = ((j8 / m_tiles) * 8 + xcd) * (64 * NT);
+    const int mt = j8 % m_tiles, n0 = ((j8 / m_tiles) * 8 + xcd) * (16 * NW * NT);
     if (n0 >= N) return;
     const int every = K / SP_K;
     const int first = FOLD ? 0 : blockIdx.y * per, last = FOLD ? every - 1 : min(first + per, every) - 1;
@@ -104,7 +104,7 @@ gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restric
         const uint32_t at = (uint32_t)min(s, last) * x_stage;
 #pragma unroll
         for (int i = 0; i < LX; ++i) {
-            const int u = min(i * 4 + wave, UNITS - 1);
+            const int u = min(i * NW + wave, UNITS - 1);
             ld16_lds(xr, b + u * 64, x_lane + u * 1024, at);
         }
     };
@@ -294,18 +294,21 @@ f32_planes_sum_kernel(const float* __restrict__ planes, void* __restrict__ Y, in
     }
 }
 
-struct SplitTiles { int mt, nt, m_tiles, blocks; };
+struct SplitTiles { int mt, nt, m_tiles, blocks, waves; };
 
 // Rows in equal tiles of at most 128.  Along W a block takes 64 or 128: a compute unit works through its blocks
 // in rounds of 256, and one of 128 takes 1.8 times one of 64 (245 rows, us with 128 / with 64: 12288 x 4096
 // 146 / 164, 22016 x 4096 263 / 252; 64 rows: 94 / 70 and 112 / 129; 900 rows of 22016 x 4096 789 / 850).  A block of a part
-// takes 128, one that adds up its parts 64 (their sums need the registers).
+// takes 128, one that adds up its parts 64 (their sums need the registers).  Up to 16 rows, where W's bytes bound it, 32 from
+// more than 256 blocks of 64 on (9 rows, us with 128 / 64 / 32: 32000 x 4096 138 / 123 / 122, 22016 x 4096 - / 105 / 91, 12288 x
+// 4096 - / 55 / 62).
 static SplitTiles split_tiles(int M, int N, bool planes, bool fold) {
     const int tiles = (M + 15) / 16, m_tiles = (tiles + 7) / 8, need = (tiles + m_tiles - 1) / m_tiles;
     const int mt = need <= 2 ? need : need <= 4 ? 4 : need <= 6 ? 6 : 8;
     const int b1 = (N + 63) / 64 * m_tiles, b2 = (N + 127) / 128 * m_tiles;
+    if (mt == 1 && !planes && !fold) return b1 > 256 ? SplitTiles{1, 1, 1, (N + 31) / 32, 2} : SplitTiles{1, 1, 1, b1, 4};
     const bool wide = !fold && (planes || 10 * 23 * ((b2 + 255) / 256) <= 10 * 13 * ((b1 + 255) / 256));
-    return {mt, wide ? 2 : 1, m_tiles, wide ? b2 : b1};
+    return {mt, wide ? 2 : 1, m_tiles, wide ? b2 : b1, 4};
 }
 
 // Stages of 32 k in a part of K, 0 where K is one part.  A row's bits hang on them, so they are the same for all numbers
@@ -358,12 +361,14 @@ extern "C" int illm_gemm_f32_split(const float* X, const float* W, void* P, size
     hipLaunchKernelGGL(f32_split_rows_kernel, dim3((every + 3) / 4, t.m_tiles * t.mt), dim3(256), 0, st, X,
                        (illm_u32x4_t*)P, M, K, t.m_tiles * t.mt);
     const dim3 grid((unsigned)grid_x, parts);
-#define ILLM_SPLIT(MT, NT, NS, FOLD)                                                                                \
-    if (t.mt == MT && t.nt == NT && fold == FOLD)                                                                   \
-        hipLaunchKernelGGL((gemm_f32_split_kernel<MT, NT, NS, FOLD>), grid, dim3(256), 0, st, (const illm_u32x4_t*)P, X, \
-                           W, Y, y_dt, M, N, K, t.m_tiles, per)
-#define ILLM_SPLIT_ROWS(MT, NS) ILLM_SPLIT(MT, 1, NS, false); ILLM_SPLIT(MT, 2, NS, false); ILLM_SPLIT(MT, 1, NS, true)
-    ILLM_SPLIT_ROWS(1, 6); ILLM_SPLIT_ROWS(2, 6); ILLM_SPLIT_ROWS(4, 6); ILLM_SPLIT_ROWS(6, 3); ILLM_SPLIT_ROWS(8, 3);
+#define ILLM_SPLIT(MT, NT, NS, FOLD, IF, ...)                                                                        \
+    if (t.mt == MT && t.nt == NT && fold == FOLD && IF)                                                                \
+        hipLaunchKernelGGL((gemm_f32_split_kernel<MT, NT, NS, FOLD __VA_OPT__(,) __VA_ARGS__>), grid, dim3(64 * t.waves), 0, \
+                           st, (const illm_u32x4_t*)P, X, W, Y, y_dt, M, N, K, t.m_tiles, per)
+#define ILLM_SPLIT_ROWS(MT, NS) ILLM_SPLIT(MT, 1, NS, false, t.waves == 4); ILLM_SPLIT(MT, 2, NS, false, true); ILLM_SPLIT(MT, 1, NS, true, true)
+    ILLM_SPLIT(1, 1, 6, false, t.waves == 2, 2);
+    ILLM_SPLIT_ROWS(1, 6);
+    ILLM_SPLIT_ROWS(2, 6); ILLM_SPLIT_ROWS(4, 6); ILLM_SPLIT_ROWS(6, 3); ILLM_SPLIT_ROWS(8, 3);
 #undef ILLM_SPLIT_ROWS
 #undef ILLM_SPLIT
     return illm_launch_status();

@@ -606,8 +606,8 @@ def gemm_f32_split_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
 def gemm_f32_split_pays(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether it is the faster way for operands that it takes.  The matrix decides, once for 9 to 128 rows and once for all
     above: a row's bits are the same whatever the number of rows in either range.  us by the float32 instruction -> here,
-    matrices cold; 9 / 16 / 33 / 128 rows: 22016 x 4096 98 / 112 / 162 / 357 -> 99 / 100 / 120 / 157, 12288 x 4096 53 / 59 / 97 /
-    241 -> 53 / 54 / 70 / 103, 6144 x 4096 36 / 40 / 56 / 155 -> 33 / 33 / 34 / 50, 2048 x 8192 32 / 37 / 55 / 154 -> 32 / 33 /
+    matrices cold; 9 / 16 / 33 / 128 rows: 22016 x 4096 98 / 112 / 162 / 357 -> 91 / 91 / 122 / 157, 12288 x 4096 53 / 59 / 97 /
+    241 -> 55 / 55 / 70 / 103, 6144 x 4096 36 / 40 / 56 / 155 -> 33 / 33 / 34 / 50, 2048 x 8192 32 / 37 / 55 / 154 -> 32 / 33 /
     36 / 50, 4096 x 4096 20 / 23 / 34 / 80 -> 26 / 26 / 30 / 38 (the slower way up to 16 rows by 3 to 5 us, of 230 that a layer of
     such matrices takes; 3 less as planes for a norm); 8192 x 2048, which stays there, 19 / 21 / 30 / 81 -> 24 / 24 / 25 / 38.
     129 / 256 / 2,048 rows: 22016 x 4096 365 / 439 / 2,865 -> 220 / 265 / 1,580, 4096 x 4096 82 / 84 / 532 -> 46 / 56 / 345,

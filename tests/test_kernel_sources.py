@@ -29,12 +29,12 @@ def test_the_float32_parts_loads_are_issued_in_the_order_their_waits_count(tmp_p
     subprocess.run([build._hipcc()] + build.HIPCC_FLAGS + ["--offload-device-only", "-S", "-o", out,
                                                            os.path.join(CSRC, "gemm_f32_split.hip")], check=True,
                    stderr=subprocess.DEVNULL)
-    kernels = re.findall(r"^_Z\w*gemm_f32_split_kernelILi(\d+)ELi(\d+)ELi(\d+)ELb[01]E\w*:(.*?)\.Lfunc_end", open(out).read(),
+    kernels = re.findall(r"^_Z\w*gemm_f32_split_kernelILi(\d+)ELi(\d+)ELi(\d+)ELb[01]ELi(\d+)E\w*:(.*?)\.Lfunc_end", open(out).read(),
                          re.S | re.M)
     assert len(kernels) >= 15
-    for mt, nt, ns, body in kernels:
-        mt, nt, ns = int(mt), int(nt), int(ns)
-        x, w = "X" * ((3 * mt + 3) // 4), "W" * (2 * nt)
+    for *sizes, body in kernels:
+        mt, nt, ns, waves = map(int, sizes)
+        x, w = "X" * -(-3 * mt // waves), "W" * (2 * nt)
         stages = []
         for part in body.split("s_barrier")[:4]:
             loads = [line for line in part.splitlines() if re.search(r"\b(buffer|global)_load", line)]
@@ -42,5 +42,5 @@ def test_the_float32_parts_loads_are_issued_in_the_order_their_waits_count(tmp_p
         # ahead of the first wait ns - 1 stages and W of one more; then a stage a turn
         assert stages[0] == (w + x) * (ns - 1) + w, (mt, nt, ns, stages[0])
         assert stages[1:] == [x + w] * 3, (mt, nt, ns, stages)
-        waits = re.findall(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)\s*\n\s*s_barrier", body)
-        assert waits and set(waits) == {str((ns - 2) * len(x + w))}, (mt, nt, ns, waits)
+        counts = re.findall(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)\s*\n\s*s_barrier", body)
+        assert counts and set(counts) == {str((ns - 2) * len(x + w))}, (mt, nt, ns, counts)
