@@ -210,24 +210,51 @@ gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restric
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int e = 0; e < 4 * NT; ++e) split_part(g0, p0, e);
-    // What a part's sums are: acc[i][j][v] is row (wave * NT + i) * 16 + 4 q + v of W's, row 16 j + r of X's.  A sum that is
-    // no finite number is taken again with plain multiply-adds: an infinity has no parts.
-    auto part_sum = [&](int i, int j, int s0, int s1) __attribute__((always_inline)) {
-        const int m = (mt * MT + j) * 16 + r, n = n0 + (wave * NT + i) * 16 + 4 * q;
-        f32x4_t v = (acc[i][j] + low[i][j]) * SP_DOWN;
-        bool odd = false;
+    // A part's sums, left in `low`: [i][j][v] is row (wave * NT + i) * 16 + 4 q + v of W's, row 16 j + r of X's.  Those that are
+    // no finite numbers (an infinity has no parts) are taken again by the wave on the float32 instruction: all of its tiles
+    // at once, so that data full of NaN takes the time of both instructions and no more (256 rows of 4096 x 4096,
+    // us alone: finite 71, all of X NaN 162, one number of it 158; a lane's own multiply-adds had taken 7,922 and 724).
+    auto odd = [](float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; };
+    auto part_sums = [&](int s0, int s1) __attribute__((always_inline)) {
+        bool again = false;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) odd |= (__float_as_uint(v[e]) & 0x7f800000u) == 0x7f800000u;
-        if (odd && m < M) {
-            for (int e = 0; e < 4; ++e) {
-                if (n + e >= N) break;
-                float t = 0.f;
-                for (int k = s0 * SP_K; k <= s1 * SP_K + SP_K - 1; ++k)
-                    t = fmaf(X[(size_t)m * K + k], W[(size_t)(n + e) * K + k], t);
-                v[e] = t;
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                low[i][j] = (acc[i][j] + low[i][j]) * SP_DOWN;
+                acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) again |= odd(low[i][j][e]);
             }
+        if (!__any(again)) return;
+        const char* const xb = (const char*)(X + (size_t)mt * MT * 16 * K);
+        uint32_t xo[MT];
+#pragma unroll
+        for (int j = 0; j < MT; ++j) xo[j] = (uint32_t)min(j * 16 + r, M - 1 - mt * MT * 16) * (uint32_t)K * 4u + 16u * q;
+#pragma unroll 1
+        for (int k = s0 * SP_K; k < (s1 + 1) * SP_K; k += 16) {
+            f32x4_t xv[MT], wv[NT];
+#pragma unroll
+            for (int i = 0; i < NT; ++i) wv[i] = *(const f32x4_t*)(wbase + (size_t)k * 4 + wo[i]);
+#pragma unroll
+            for (int j = 0; j < MT; ++j) xv[j] = *(const f32x4_t*)(xb + (size_t)k * 4 + xo[j]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+#pragma unroll
+                    for (int j = 0; j < MT; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[i][e], xv[j][e], acc[i][j], 0, 0, 0);
         }
-        return v;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (odd(low[i][j][e])) low[i][j][e] = acc[i][j][e];
+                acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            }
     };
     f32x4_t tot[FOLD ? NT : 1][FOLD ? MT : 1];
     int part = first;                               // FOLD: where the part under way began
@@ -249,18 +276,19 @@ gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restric
         }
         if constexpr (FOLD) {
             if (s + 6 - part < per && s + 6 <= last) continue;
+            part_sums(part, min(s + 5, last));
 #pragma unroll
             for (int i = 0; i < NT; ++i)
 #pragma unroll
                 for (int j = 0; j < MT; ++j) {
-                    const f32x4_t v = part_sum(i, j, part, min(s + 5, last));
-                    tot[i][j] = part == 0 ? v : tot[i][j] + v;
-                    acc[i][j] = low[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+                    tot[i][j] = part == 0 ? low[i][j] : tot[i][j] + low[i][j];
+                    low[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
                 }
             part = s + 6;
         }
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);             // no load into LDS outlives the block
+    if constexpr (!FOLD) part_sums(first, last);
 
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
@@ -270,7 +298,7 @@ gemm_f32_split_kernel(const illm_u32x4_t* __restrict__ P, const float* __restric
             const int n = n0 + (wave * NT + i) * 16 + 4 * q;
             f32x4_t v;
             if constexpr (FOLD) v = tot[i][j];
-            else v = part_sum(i, j, first, last);
+            else v = low[i][j];
             if (m >= M) continue;
             const size_t at = ((size_t)blockIdx.y * M + m) * N + n;
             if (n + 3 < N && (N & 3) == 0 && y_dt == ILLM_F32) {

@@ -617,6 +617,29 @@ def test_gemm_f32_split_over_the_range_of_float32(M, N, K):
     assert err(ops().gemm_f32_split(x.to(DEV), w.to(DEV), torch.float32)) <= 2.0 ** -24 * (K / 32 + 2)
 
 
+def test_gemm_f32_split_takes_no_longer_for_nan():
+    """Sums that are no finite numbers are taken again on the float32 instruction: a prompt whose activations have all
+    become NaN takes a few times as long as a sound one, not a hundred times."""
+    x, w = rnd(256, 4096, seed=1).to(DEV), rnd(4096, 4096, seed=2).to(DEV)
+
+    def least(f, rows):
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record(); f(rows, w, torch.float32); b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times[1:])
+    bad = torch.full_like(x, float("nan"))
+    assert ops().gemm_f32_split(bad, w, torch.float32).isnan().all()
+    limit = 2 * least(ops().gemm_f32_mfma, x) + 2 * least(ops().gemm_f32_split, x)
+    for rows in (bad, torch.full_like(x, float("inf")), torch.full_like(x, 3e38)):
+        assert least(ops().gemm_f32_split, rows) <= limit
+    x[7, 100] = float("nan")
+    got = ops().gemm_f32_split(x, w, torch.float32)
+    assert got[7].isnan().all() and int(got.isnan().sum()) == 4096
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 32), (8, 24, 96), (3, 2048, 1056), (8, 2040, 4096), (7, 520, 2048), (5, 100, 1024),
                                    (8, 2048, 8192), (9, 2048, 1024), (16, 40, 64)])
 def test_skinny_half_tiles_and_activations(M, N, K):
