@@ -351,13 +351,13 @@ extern "C" int illm_gemm_f32_split_per(int M, int N, int K) {
 }
 
 // Whether the parts of so many rows are taken by a block each (planes that somebody adds) and not one after the other by the
-// same blocks: up to 128 MB of planes (us, planes and their sum / in one: 245 / 1,024 / 2,048 rows of 4096 x 4096 60 / 177 /
+// same blocks: up to 128 MB of planes and 256 MB of X's parts (us, planes and their sum / in one: 245 / 1,024 / 2,048 rows of 4096 x 4096 60 / 177 /
 // 346 against 95 / 180 / 364, of 4096 x 11008 124 / 430 / 841 against 240 / 457 / 909, of 2048 x 2048 33 / 61 / 107 against
 // 51 / 56 / 97; all of K in one part, as it had been from 257 rows on, 4096 x 4096 163 / 314 at 1,024 / 2,048).
 extern "C" int illm_gemm_f32_split_planes(int M, int N, int K) {
     const int per = illm_gemm_f32_split_per(M, N, K);
     if (!per || N % 4) return 0;
-    return (long long)((K / SP_K + per - 1) / per) * M * N <= 1 << 25;
+    return (long long)((K / SP_K + per - 1) / per) * M * N <= 1 << 25 && 6LL * M * K <= 1 << 28;
 }
 
 // Rows of X as its parts are laid out (M filled up to whole tiles): 6 bytes of scratch for each of their K.

@@ -28,7 +28,7 @@ nothing depends on a stopwatch).
 from __future__ import annotations
 
 import ctypes
-from typing import Dict, Optional
+from typing import Dict, List, Optional, Tuple
 
 import torch
 
@@ -594,13 +594,23 @@ def gemm_rows_f32_mfma(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype)
     return y
 
 
+F32_SPLIT_SCRATCH = 1 << 28      # bytes of X's parts (6 an element) at a time: more rows go in pieces
+
+
 def gemm_f32_split_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether `gemm_f32_split` takes these operands."""
-    if not (x.dtype == torch.float32 and w.dtype == torch.float32 and x.dim() == 2 and w.dim() == 2
-            and x.shape[0] >= 1 and x.shape[1] == w.shape[1] and x.shape[1] % 32 == 0
-            and x.is_contiguous() and w.is_contiguous() and _on16(x, w)):
-        return False
-    return (x.shape[0] + 127) * 6 * x.shape[1] < 0xffffffff and x.shape[1] < 1 << 22
+    return (x.dtype == torch.float32 and w.dtype == torch.float32 and x.dim() == 2 and w.dim() == 2
+            and x.shape[0] >= 1 and x.shape[1] == w.shape[1] and x.shape[1] % 32 == 0 and x.shape[1] <= 1 << 18
+            and x.is_contiguous() and w.is_contiguous() and _on16(x, w))
+
+
+def _f32_split_pieces(M: int, K: int) -> List[Tuple[int, int]]:
+    """(first row, rows) of the pieces that M rows go in: multiples of 128 but the last, about equal, none with more scratch
+    than `F32_SPLIT_SCRATCH`."""
+    most = max(128, F32_SPLIT_SCRATCH // (6 * K) // 128 * 128)
+    n = -(-M // most)
+    step = -(-M // (128 * n)) * 128
+    return [(r, min(step, M - r)) for r in range(0, M, step)]
 
 
 def gemm_f32_split_pays(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -630,10 +640,13 @@ def _f32_split(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, S: int)
     per = -(-every // S) if S > 1 else _lib().illm_gemm_f32_split_per(M, N, K) or every
     planes = -(-every // per) if S != 1 else 0
     _need(S <= 1 or planes == S, f"gemm_f32_split: {S} parts of {every} stages")
-    parts = torch.empty(_lib().illm_gemm_f32_split_rows(M) * K * 6, dtype=torch.uint8, device=x.device)
+    pieces = [(0, M)] if planes else _f32_split_pieces(M, K)
+    parts = torch.empty(max(_lib().illm_gemm_f32_split_rows(n) for _, n in pieces) * K * 6, dtype=torch.uint8, device=x.device)
     y = torch.empty((planes, M, N) if planes else (M, N), dtype=out_dtype, device=x.device)
-    _check(_lib().illm_gemm_f32_split(_p(x), _p(w), _p(parts), ctypes.c_size_t(parts.numel()), _p(y), _code(y), M, N, K, per,
-                                      1 if planes else 0, _stream()), "gemm_f32_split")
+    for r, n in pieces:
+        _check(_lib().illm_gemm_f32_split(_p(x[r:]), _p(w), _p(parts), ctypes.c_size_t(parts.numel()),
+                                          _p(y if planes else y[r:]), _code(y), n, N, K, per, 1 if planes else 0, _stream()),
+               "gemm_f32_split")
     return y
 
 

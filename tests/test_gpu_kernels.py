@@ -617,6 +617,18 @@ def test_gemm_f32_split_over_the_range_of_float32(M, N, K):
     assert err(ops().gemm_f32_split(x.to(DEV), w.to(DEV), torch.float32)) <= 2.0 ** -24 * (K / 32 + 2)
 
 
+def test_gemm_f32_split_in_pieces(monkeypatch):
+    """Rows in pieces of at most so much scratch: the bits of one call, with the parts of K of all rows."""
+    for M, N, K in ((300, 4098, 2048), (513, 130, 1056), (700, 12288, 512)):
+        x, w = rnd(M, K, seed=1).to(DEV), rnd(N, K, seed=2).to(DEV)
+        for dtype in DTYPES:
+            want = ops()._f32_split(x, w, dtype, 1)
+            monkeypatch.setattr(ops(), "F32_SPLIT_SCRATCH", 6 * K * 256)
+            assert len(ops()._f32_split_pieces(M, K)) > 1
+            assert torch.equal(ops()._f32_split(x, w, dtype, 1), want)
+            monkeypatch.undo()
+
+
 def test_gemm_f32_split_takes_no_longer_for_nan():
     """Sums that are no finite numbers are taken again on the float32 instruction: a prompt whose activations have all
     become NaN takes a few times as long as a sound one, not a hundred times."""

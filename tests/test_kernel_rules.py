@@ -55,3 +55,25 @@ def test_the_experts_tiles_of_128_pairs_are_taken_where_they_pay():
                             (2, 4096, 4096, 24), (32, 2048, 4096, 1.5)):
         for p in (1, 1.5, 2, 3, 4, 6, 8, 12, 16, 24, 64, 500):
             assert (rows(NE, F, E, p) == 128) == (p >= first), (NE, F, E, p)
+
+
+def test_float32_rows_in_pieces_that_the_product_in_parts_takes():
+    """Any number of rows, on and beyond what the library takes in one call (4 GiB of scratch, 65,535 tiles): pieces
+    that hold every row once, each with no more scratch than the limit says, and no row refused that another product
+    had taken."""
+    lib = ops._lib()
+    for K in (512, 2048, 4096, 11008, 1 << 18):
+        for M in (1, 127, 128, 129, 2048, 4064, 4065, 65536, (1 << 20) - 128, 1 << 20, (1 << 20) + 1, 3000000):
+            pieces = ops._f32_split_pieces(M, K)
+            assert [r for r, _ in pieces] == [0] + [r + n for r, n in pieces][:-1] and sum(n for _, n in pieces) == M
+            for r, n in pieces:
+                rows = lib.illm_gemm_f32_split_rows(n)
+                assert r % 128 == 0 and n <= rows < n + 128 and rows // 16 <= 65535
+                assert rows * K * 6 <= max(ops.F32_SPLIT_SCRATCH, 128 * 6 * K) <= 0xffffffff
+    x, w = torch.empty((1 << 20) + 1, 512, device="meta"), torch.empty(16384, 512, device="meta")
+    assert ops.gemm_f32_split_fits(x, w) and ops.gemm_f32_split_pays(x, w)
+    # planes and their scratch are bounded too
+    for M, N, K in ((4096, 1024, 11008), (16384, 1024, 2048), (2048, 4096, 11008), (300, 1024, 1 << 18)):
+        if lib.illm_gemm_f32_split_planes(M, N, K):
+            planes = -(-K // 32 // lib.illm_gemm_f32_split_per(M, N, K))
+            assert planes * M * N * 4 <= 1 << 27 and 6 * M * K <= ops.F32_SPLIT_SCRATCH
