@@ -142,13 +142,15 @@ def embed_norm(tokens: torch.Tensor, table: torch.Tensor, weight: torch.Tensor, 
 
 
 def zero_slot(tensors, slot: int) -> None:
-    """Row `slot` of every tensor to zeros (contiguous [slots, ...], any types), in one launch for 16 of them."""
+    """Row `slot` of every tensor to zeros (contiguous [slots, ...], any types, one device), in one launch for 16 of them
+    on that device."""
     rows = [t[slot] for t in tensors]
     _gpu(*rows)
     n = len(rows)
     at = (ctypes.c_uint64 * n)(*[r.data_ptr() for r in rows])
     size = (ctypes.c_uint64 * n)(*[r.numel() * r.element_size() for r in rows])
-    _check(_lib().illm_zero_pieces(at, size, n, _stream()), "zero_slot")
+    with torch.cuda.device(rows[0].device):
+        _check(_lib().illm_zero_pieces(at, size, n, _stream()), "zero_slot")
 
 
 def copy_rows(x: torch.Tensor) -> torch.Tensor:

@@ -77,3 +77,31 @@ def test_float32_rows_in_pieces_that_the_product_in_parts_takes():
         if lib.illm_gemm_f32_split_planes(M, N, K):
             planes = -(-K // 32 // lib.illm_gemm_f32_split_per(M, N, K))
             assert planes * M * N * 4 <= 1 << 27 and 6 * M * K <= ops.F32_SPLIT_SCRATCH
+
+
+def test_a_slot_is_zeroed_on_its_tensors_device(monkeypatch):
+    """A new sequence's state is cleared on the tensors' own card and its stream, whichever card is the current one."""
+    seen, current = [], ["another"]
+
+    class on:
+        def __init__(self, device):
+            self.device = device
+
+        def __enter__(self):
+            self.before, current[0] = current[0], self.device
+
+        def __exit__(self, *exc):
+            current[0] = self.before
+
+    class library:
+        @staticmethod
+        def illm_zero_pieces(at, size, n, stream):
+            seen.append((list(at), list(size), n, stream))
+            return 0
+    monkeypatch.setattr(torch.cuda, "device", on)
+    monkeypatch.setattr(ops, "_gpu", lambda *t: None)
+    monkeypatch.setattr(ops, "_lib", lambda: library)
+    monkeypatch.setattr(ops, "_stream", lambda: ("stream of", current[0]))
+    a, b = torch.zeros(4, 3, dtype=torch.float32), torch.zeros(4, 5, 2, dtype=torch.bfloat16)
+    ops.zero_slot([a, b], 2)
+    assert seen == [([a[2].data_ptr(), b[2].data_ptr()], [12, 20], 2, ("stream of", a.device))] and current == ["another"]
