@@ -121,6 +121,31 @@ def test_steps_of_129_to_256_rows(tmp_path_factory, monkeypatch, lens):
     eng.cache.check()
 
 
+@pytest.mark.parametrize("lens", [[128], [129], [100, 60], [7, 249], [300]])
+def test_float32_steps_whose_products_are_cut(tmp_path_factory, monkeypatch, lens):
+    """float32 steps of 129 rows and more whose o and down matrices (1024 x 2048) have their K in parts: the planes go to
+    the next norm, in both layers; up to 128 rows such matrices stay whole."""
+    from inferllm_amd import StepEntry
+    from inferllm_amd.kernels import ops
+    calls = []
+    real = ops.linear_cut
+    monkeypatch.setattr(ops, "linear_cut", lambda x, w, *a: calls.append(x.shape[0]) or real(x, w, *a))
+    monkeypatch.setitem(CONFIGS, "cut32", dict(CONFIGS["D"], hidden_size=1024, num_attention_heads=16, num_key_value_heads=4,
+                                               intermediate_size=2048, vocab_size=300))
+    eng, plain, config = setup(tmp_path_factory, "cut32", "float32")
+    reqs = requests_for(config, lens, seed=4)
+    slots = [eng.alloc_slot() for _ in reqs]
+    got = eng.step([StepEntry(s, r, list(range(len(r)))) for s, r in zip(slots, reqs)]).clone()
+    assert calls == ([sum(lens)] * 4 if sum(lens) > 128 else []), calls
+    at = 0
+    for r in reqs:
+        assert err(got[at:at + len(r)], plain(r)) < BUDGET["float32"], len(r)
+        at += len(r)
+    for s in slots:
+        eng.free_slot(s)
+    eng.cache.check()
+
+
 def test_steps_of_17_to_64_rows(tmp_path_factory, monkeypatch):
     """Steps of 17 to 128 rows (here 24 to 64: a prompt of that length, or that many sequences decoding) read the
     decode copy of the down projection with K cut into ranges, whose planes the next norm adds
