@@ -104,10 +104,6 @@ __device__ __forceinline__ void combine_block(const float* lds, int row_heads, i
     }
 }
 
-// The blocks of a sequence's ranges have neighbouring numbers (grid: heads, ranges, sequences): with the sequences
-// between, an XCD's compute units went round the sequences in step and one got the ranges of the longest alone.  16
-// sequences of 64 to 4,096 keys, 32/8 heads: 29.5 -> 24.2 us, 32/32: 61.8 -> 50.9; one of 4,000 before 15 of 200: 23.8 ->
-// 15.9 and 38.0 -> 34.4; equal lengths as before.
 // What the merge kernel passes over: a range without keys (its sums stay unwritten).
 __device__ __forceinline__ void no_keys(float* partial, int nsplit, int sp, size_t bh0, int n_heads, int hd) {
     if ((int)threadIdx.x < n_heads) {
@@ -124,6 +120,10 @@ struct DecMore {
 
 // LPR: lanes per key row (power of two, 8 dims each, LPR * 8 >= head_dim).
 // GC: query heads handled together (power of two >= heads per kv head, at most 8).
+// The blocks of a sequence's ranges have neighbouring numbers (grid: heads, ranges, sequences): with the sequences
+// between, an XCD's compute units went round the sequences in step and one got the ranges of the longest alone.  16
+// sequences of 64 to 4,096 keys, 32/8 heads: 29.5 -> 24.2 us, 32/32: 61.8 -> 50.9; one of 4,000 before 15 of 200: 23.8 ->
+// 15.9 and 38.0 -> 34.4; equal lengths as before.
 template <int LPR, int GC>
 __global__ void __launch_bounds__(GC <= 4 ? 512 : 256)
 attn_decode_bf16_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out,

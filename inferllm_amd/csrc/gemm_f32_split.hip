@@ -15,9 +15,9 @@
 // vector instructions a pair, between MFMAs); X's parts, made once by a small kernel in the order of the operands, go
 // straight into LDS and serve the four waves.  The largest product of each stage has a sum of its own, so that a sum
 // is rounded once a stage at its full size: 2.6 times closer to 64 bits than six roundings, for no vector work.
-// Against the float32 instruction (256 rows, us): 4096 x 4096 94 -> 55, 12288 x 4096 234 -> 155, 22016 x 4096 429 -> 267
-// (1.05 PFLOP/s of bfloat16 products; two blocks a compute unit hold 344 of 512 places), 4096 x 11008 219 -> 134;
-// 2,048 rows of 22016 x 4096 2,877 -> 1,576 (1.4 PFLOP/s).
+// Against the float32 instruction (256 rows, us): 4096 x 4096 84 -> 57, 12288 x 4096 232 -> 155 (192 blocks of 128 rows of W
+// for 256 compute units), 22016 x 4096 436 -> 263 (1.05 PFLOP/s of bfloat16 products; 688 blocks of 64 for 512 places), 4096 x
+// 11008 227 -> 126; 2,048 rows of 22016 x 4096 2,850 -> 1,590 (1.4 PFLOP/s).
 // (Published as bf16x6 and the like: Henry, Tang, Heinecke, "Leveraging the bfloat16 artificial intelligence
 // datatype for higher-precision computations", 2019.)
 #include "api.h"
