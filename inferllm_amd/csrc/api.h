@@ -229,7 +229,7 @@ int illm_attn_decode_bf16_static(const void* qkv, void* out, const void* kcache,
 int illm_gemm_skinny_bf16(const void* X, const void* W, const void* Wt, void* Y, int y_dt, int M,
                           int N, int K, const float* ssq, int parts, float eps, int waves_wanted,
                           void* stream);
-// The same of at most 16 rows, an activation of the results as Y's type holds them: act 1 relu(y)^2, 2 gelu(y) by tanh, 0 none.
+// The same of at most 16 rows, an activation on the float32 sums: act 1 relu(y)^2, 2 gelu(y) by tanh, 0 none.
 int illm_gemm_skinny_act(const void* X, const void* W, const void* Wt, void* Y, int y_dt, int M, int N, int K,
                          const float* ssq, int parts, float eps, int act, void* stream);
 

@@ -1114,8 +1114,8 @@ _LINEAR_ACTS = {"relu_squared": 1, "gelu_tanh": 2}
 
 
 def linear_act(x, w, act: str) -> torch.Tensor:
-    """An activation of x . w^T, the product rounded to its type first: up to 16 bfloat16 rows in the product's kernel (one
-    of its own takes 4.5 us a layer of a decode step), else in two; the same bits."""
+    """An activation of x . w^T: up to 16 bfloat16 rows (the few-rows product's) in the product's kernel, on the float32 sums
+    (a kernel of its own takes 4.5 us a layer of a decode step); else the product, then the activation."""
     code = _LINEAR_ACTS.get(act, 0)
     M, K = x.shape
     if not (code and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.shape[1] == K

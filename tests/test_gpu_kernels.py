@@ -710,13 +710,20 @@ def test_skinny_rows_alone_and_among_16(N, K):
 @pytest.mark.parametrize("name", ["relu_squared", "gelu_tanh"])
 @pytest.mark.parametrize("N,K", [(2048, 1056), (100, 1024), (4104, 96)])
 def test_an_activation_in_the_product_and_behind_it(name, N, K):
-    """`linear_act` has the bits of the product and the activation one after the other, from either copy of the matrix
-    and for any number of rows."""
-    x, w = rnd(20, K, seed=1).to(torch.bfloat16).to(DEV), rnd(N, K, seed=2, std=K ** -0.5).to(torch.bfloat16).to(DEV)
-    for W in (w, ops().decode_weight(w, "plain", True)):
-        for M in (1, 5, 8, 9, 16, 17):
-            rows = x[:M].contiguous()
-            assert torch.equal(ops().linear_act(rows, W, name), getattr(ops(), name)(ops().linear(rows, W)))
+    """`linear_act` of 1 to 16 rows: the same bits whatever their number, and no further from 64 bits than the product
+    rounded to bfloat16 and the activation of that; more rows are those two."""
+    x, w = rnd(20, K, seed=1).to(torch.bfloat16), rnd(N, K, seed=2, std=K ** -0.5).to(torch.bfloat16)
+    z = x.double() @ w.double().t()
+    want = z.clamp(min=0) ** 2 if name == "relu_squared" else torch.nn.functional.gelu(z, approximate="tanh")
+    off = lambda y: float((y.double().cpu() - want[:len(y)]).norm())  # noqa: E731
+    xd, act = x.to(DEV), getattr(ops(), name)
+    for W in (w.to(DEV), ops().decode_weight(w.to(DEV), "plain", True)):
+        whole = ops().linear_act(xd[:16].contiguous(), W, name)
+        assert off(whole) <= off(act(ops().linear(xd[:16].contiguous(), W)))
+        for M in (1, 5, 8, 9):
+            assert torch.equal(ops().linear_act(xd[:M].contiguous(), W, name), whole[:M])
+        rows = xd[:17].contiguous()
+        assert torch.equal(ops().linear_act(rows, W, name), act(ops().linear(rows, W)))
 
 
 @pytest.mark.parametrize("d,window,chunk,own", [(128, 0, 0, 1), (128, 0, 96, 0), (64, 70, 0, 0), (64, 0, 0, 1)])
