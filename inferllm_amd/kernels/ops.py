@@ -903,7 +903,9 @@ def linear_cut(x: torch.Tensor, w, splits: int = 0) -> torch.Tensor:
     M, K = x.shape
     N = w.shape[0]
     if x.dtype == torch.float32:
-        return _f32_split(x, w, torch.float32, splits)
+        _need(gemm_f32_split_fits(x, w), "linear_cut: operands not taken")
+        planes = _f32_split(x, w, torch.float32, splits)
+        return planes if planes.dim() == 3 else planes[None]
     S = splits or _lib().illm_gemm_tiles_splits(N, K)
     y = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
     _check(_lib().illm_gemm_tiles_planes(_p(x), _p(w), _p(y), M, N, K, S, _stream()), "linear_cut")

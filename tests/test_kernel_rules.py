@@ -1,5 +1,6 @@
 """The rules that send a call to one kernel or another, and what the library refuses before it launches anything:
 no GPU is needed for either."""
+import pytest
 import torch
 
 from inferllm_amd.kernels import ops
@@ -105,3 +106,16 @@ def test_a_slot_is_zeroed_on_its_tensors_device(monkeypatch):
     a, b = torch.zeros(4, 3, dtype=torch.float32), torch.zeros(4, 5, 2, dtype=torch.bfloat16)
     ops.zero_slot([a, b], 2)
     assert seen == [([a[2].data_ptr(), b[2].data_ptr()], [12, 20], 2, ("stream of", a.device))] and current == ["another"]
+
+
+def test_the_cut_product_refuses_float32_rows_with_another_matrix(monkeypatch):
+    """float32 rows with a bfloat16 matrix, or one of another width, are refused before anything reads them as float32."""
+    monkeypatch.setattr(ops, "_gpu", lambda *t: None)
+    monkeypatch.setattr(ops, "_f32_split", lambda x, w, dtype, S: torch.zeros((x.shape[0], w.shape[0]) if S == 1
+                                                                             else (S or 4, x.shape[0], w.shape[0])))
+    x = torch.zeros(140, 2048)
+    for w in (torch.zeros(1024, 2048, dtype=torch.bfloat16), torch.zeros(1024, 1024)):
+        with pytest.raises(ops.KernelError):
+            ops.linear_cut(x, w)
+    for splits, planes in ((0, 4), (1, 1), (3, 3)):
+        assert ops.linear_cut(x, torch.zeros(1024, 2048), splits).shape == (planes, 140, 1024)
