@@ -683,6 +683,103 @@ moe_rows_mfma_kernel(const bf16_t* __restrict__ X, int x_div, const bf16_t* __re
     }
 }
 
+// The value of the lane 8 further within 16.
+__device__ __forceinline__ moe_bf16x8_t moe_turn8(illm_u32x4_t v) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = (uint32_t)__builtin_amdgcn_mov_dpp((int)v[i], 0x128, 0xf, 0xf, true);   // row_ror:8
+    return *(const moe_bf16x8_t*)&v;
+}
+
+// The same for tiles of up to 16 pairs of few tokens, K % 64 == 0, W read in whole 128-byte lines: a load brings 64 k of 8
+// rows (lanes r < 8 hold the first 32 k of row r, the others the second 32 of row r - 8), and a product of the lines as
+// they are is followed by one of the lines turned by 8 lanes, so that rows 0 .. 7 of the sums take the steps of 32 k one
+// after the other, as above: the same bits.  (Rows 8 .. 15 of the sums are never read.)  Bound by reading the chosen
+// experts once.  A block is one (tile, group of columns), the groups of a tile one after the other: with the tile as the
+// faster index its blocks all went to one of the eight XCDs wherever the number of tiles is a multiple of 8, and 30 experts
+// make 3 tiles for some XCDs and 4 for others.  2,048 x 1,408, 64 experts, 6 a token, gate|up and down in us, matrices cold,
+// before / now: 4 tokens 68 + 24.2 / 47.9 + 24.8, 8 tokens 75.7 + 34.2 / 69.1 + 34.1, 16 tokens 121 + 96 / 102 + 53, 24
+// tokens 134 + 74 / 111 + 59 (2.8 to 5.8 TB/s).  NH: groups of 8 columns a wave takes; S: steps of 64 k a set of registers
+// holds, two sets in turn.
+template <int NH, bool GATED, int S>
+__global__ void __launch_bounds__(256)
+moe_lines_kernel(const bf16_t* __restrict__ X, int x_div, const bf16_t* __restrict__ W,
+                 const int32_t* __restrict__ order, const int32_t* __restrict__ tiles, int max_tiles,
+                 bf16_t* __restrict__ Y, int N, int K, int act_kind, float limit, const float* __restrict__ row_w,
+                 int groups) {
+    const int tile = blockIdx.x / groups, group = blockIdx.x - tile * groups;
+    if (tile >= tiles[3 * (size_t)max_tiles]) return;
+    const int e = tiles[3 * (size_t)tile], first = tiles[3 * (size_t)tile + 1], n = tiles[3 * (size_t)tile + 2];
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    const int n0 = (group * 4 + wave_index()) * 8 * NH;
+    if (n0 >= N) return;
+    constexpr int NW = GATED ? 2 * NH : NH;                           // (gate rows, then up rows)
+    const size_t wrows = GATED ? 2 * (size_t)N : (size_t)N;
+    const illm_u32x4_t* wp[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        const int row = min(n0 + (i % NH) * 8 + (r & 7), N - 1) + (i / NH) * N;
+        wp[i] = (const illm_u32x4_t*)(W + ((size_t)e * wrows + row) * K + (q + 4 * (r >> 3)) * 8);
+    }
+    const int pair = order[first + min(r, n - 1)];                    // rows beyond the tile: read, not written
+    const illm_u32x4_t* xp = (const illm_u32x4_t*)(X + (size_t)(pair / x_div) * K + q * 8);
+    moe_f32x4_t acc[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) acc[i] = (moe_f32x4_t){0.f, 0.f, 0.f, 0.f};
+    struct Set { illm_u32x4_t w[S][NW], x[S][2]; };
+    const int steps = K / 64;
+    auto load = [&](Set& s, int k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < S; ++u) {
+            const int at = min(k + u, steps - 1) * 8;                 // (past the end: not used)
+#pragma unroll
+            for (int i = 0; i < NW; ++i) s.w[u][i] = __builtin_nontemporal_load(wp[i] + at);
+            s.x[u][0] = xp[at];
+            s.x[u][1] = xp[at + 4];
+        }
+        __builtin_amdgcn_sched_barrier(0);                            // (else a product's loads are put right before it)
+    };
+    auto multiply = [&](const Set& s, int k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < S; ++u) {
+            if (k + u >= steps) continue;
+#pragma unroll
+            for (int i = 0; i < NW; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&s.w[u][i], *(const moe_bf16x8_t*)&s.x[u][0],
+                                                                 acc[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < NW; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(moe_turn8(s.w[u][i]), *(const moe_bf16x8_t*)&s.x[u][1], acc[i], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Set s0, s1;
+    load(s0, 0);
+    for (int k = 0; k < steps; k += 2 * S) {
+        load(s1, k + S);
+        multiply(s0, k);
+        load(s0, k + 2 * S);
+        multiply(s1, k + S);
+    }
+    // acc[h][i] belongs to the pair of row r and column n0 + 8 h + 4 q + i
+    if (r >= n || q >= 2) return;
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int col = n0 + 8 * h + 4 * q + i;
+            if (col >= N) continue;
+            float v = acc[h][i];
+            if (GATED) {
+                const float rw = row_w ? row_w[pair] : 1.0f;          // W (w x) = w (W x)
+                const float gate = bf16_to_f32(f32_to_bf16(v * rw));
+                const float upv = bf16_to_f32(f32_to_bf16(acc[(GATED ? NH : 0) + h][i] * rw));
+                v = moe_act(gate, upv, act_kind, limit);
+            } else
+                v = moe_plain_act(row_w ? v * row_w[pair] : v, act_kind, true);
+            Y[(size_t)pair * N + col] = f32_to_bf16(v);
+        }
+}
+
 // Tiles of 64 pairs (prompts), K % 64 == 0: as above with the tile's X rows shared by the block's
 // four waves through LDS, 64 k at a time in two buffers (a thread brings 32 bytes of one row; the
 // 16-byte pieces of a row are placed at piece ^ (row % 8), so that the 16 rows a product's operand
@@ -961,15 +1058,29 @@ extern "C" int illm_moe_rows_mfma(const void* X, int x_div, const void* W, int g
                            (const bf16_t*)X, x_div, (const bf16_t*)W, order, tiles, max_tiles,     \
                            (bf16_t*)Y, N, K, act_kind, limit, row_w);                              \
     } while (0)
-    if (tile_rows == 16 && (long)max_tiles * ((N + 255) / 256) < 512) {
-        // few tiles (single tokens): 16 columns a wave, so that more waves share the reading
-        if (K % 256 == 0) { if (gated) GO(1, 1, true, 8); else GO(1, 1, false, 8); }
-        else if (K % 128 == 0) { if (gated) GO(1, 1, true, 4); else GO(1, 1, false, 4); }
-        else if (K % 64 == 0) { if (gated) GO(1, 1, true, 2); else GO(1, 1, false, 2); }
-        else { if (gated) GO(1, 1, true, 1); else GO(1, 1, false, 1); }
-    } else if (tile_rows == 16) {
-        if (K % 64 == 0) { if (gated) GO(1, 4, true, 2); else GO(1, 4, false, 2); }
-        else { if (gated) GO(1, 4, true, 1); else GO(1, 4, false, 1); }
+    if (tile_rows == 16) {
+        // W by whole lines from 8 tiles on, and where the columns alone make blocks enough (1 token with 6 of 64 experts,
+        // 2,048 x 1,408: 21.5 + 10.2 us below, 25.0 + 12.5 by lines; 2 tokens 39.7 + 17.1 / 35.7 + 17.3).  The down
+        // products take 16 columns a wave while that leaves waves enough (2,048 x 1,408, us with 8 / 16 columns: 8 tokens
+        // 40.1 / 34.1, 16 tokens 65.5 / 53.1; 1,024 x 2,816 of 8 experts, 4 tokens 13.5 / 21.4).
+        const bool wide = !gated && (long long)max_tiles * N >= 32768;
+        const int groups = (N + (wide ? 63 : 31)) / (wide ? 64 : 32);
+        const long long blocks = (long long)max_tiles * groups;
+        if (K % 64 == 0 && (max_tiles >= 8 || (long)max_tiles * ((N + 255) / 256) >= 512) && blocks < (1 << 23)) {
+#define GO_LINES(NH_, G_, S_)                                                                      \
+    hipLaunchKernelGGL((moe_lines_kernel<NH_, G_, S_>), dim3((unsigned)blocks), dim3(256), 0, st, (const bf16_t*)X, x_div, \
+                       (const bf16_t*)W, order, tiles, max_tiles, (bf16_t*)Y, N, K, act_kind, limit, row_w, groups)
+            if (gated) GO_LINES(1, true, 2);
+            else if (wide) GO_LINES(2, false, 1);
+            else GO_LINES(1, false, 2);
+#undef GO_LINES
+        } else if ((long)max_tiles * ((N + 255) / 256) < 512) {
+            // few tiles: 16 columns a wave, so that more waves share the reading
+            if (K % 256 == 0) { if (gated) GO(1, 1, true, 8); else GO(1, 1, false, 8); }
+            else if (K % 128 == 0) { if (gated) GO(1, 1, true, 4); else GO(1, 1, false, 4); }
+            else if (K % 64 == 0) { if (gated) GO(1, 1, true, 2); else GO(1, 1, false, 2); }
+            else { if (gated) GO(1, 1, true, 1); else GO(1, 1, false, 1); }
+        } else { if (gated) GO(1, 4, true, 1); else GO(1, 4, false, 1); }
     }
     else if (tile_rows == 32) { if (gated) GO(2, 4, true, 1); else GO(2, 4, false, 1); }
     else { if (gated) GO(4, 2, true, 1); else GO(4, 4, false, 1); }    // wider column blocks measured slower

@@ -910,6 +910,32 @@ def test_moe_tiles_of_128_pairs(T, E, F, NE, top, act):
     assert real(torch.bfloat16, E, F, 24 * NE, NE)[1] == 128 and real(torch.bfloat16, E, F + 32, 24 * NE, NE)[1] != 128
 
 
+@pytest.mark.parametrize("T,E,F,NE,top,act", [(8, 64, 64, 9, 1, "silu"), (17, 192, 96, 8, 2, "clamped_swish"), (90, 64, 320, 3, 2, "relu_squared"),
+                                              (12, 2048, 64, 16, 3, "silu"), (20, 4160, 64, 9, 2, "relu_squared")])
+def test_moe_products_of_few_tokens_by_whole_lines(T, E, F, NE, top, act):
+    """Experts' products of 8 tiles and more of up to 16 pairs, read by whole lines, give a token the bits that it has
+    alone, where fewer tiles go to the kernel that reads 64 bytes of 16 rows: one step of 64 k and odd numbers of them,
+    full tiles and tiles of one pair, columns that end inside a block, 8 and 16 columns a wave."""
+    o, gated = ops(), act != "relu_squared"
+    g = torch.Generator().manual_seed(5)
+    h = rnd(T, E, dtype=torch.bfloat16, seed=1).to(DEV)
+    wu = (rnd(NE, F * (2 if gated else 1), E, seed=2) * 0.1).to(torch.bfloat16).to(DEV)
+    wd = (rnd(NE, E, F, seed=3) * 0.1).to(torch.bfloat16).to(DEV)
+    idx = torch.stack([torch.randperm(NE, generator=g)[:top] for _ in range(T)]).to(torch.int32).to(DEV)
+    wt = torch.rand(T, top, generator=g).to(DEV) if act == "clamped_swish" else None
+    real, lim = o._moe_tiling, 7.0 if act == "clamped_swish" else 0.0
+    try:
+        o._moe_tiling = lambda dtype, e, f, np, n: (True, 16, max(1, min(np, np // 16 + n)))
+        assert min(T * top, T * top // 16 + NE) >= 8 > top
+        got = o.moe_experts(h, idx, wu, wd, None, act, lim, wt).view(T, top, E)
+        for t in range(T):
+            alone = o.moe_experts(h[t:t + 1], idx[t:t + 1], wu, wd, None, act, lim, None if wt is None else wt[t:t + 1])
+            assert torch.equal(got[t], alone)
+    finally:
+        o._moe_tiling = real
+    assert bool(torch.isfinite(got.float()).all())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("E", [1024, 1032, 2048, 2056, 4104])
 def test_moe_combine_of_wide_rows(E, dtype):
