@@ -9,6 +9,7 @@
 // rows between tiles and changes no value.
 #include "api.h"
 #include "common.h"
+#include "gemm_turns.h"
 
 #define MOE_TILE 8
 
@@ -901,114 +902,100 @@ moe_rows_mfma_lds_kernel(const bf16_t* __restrict__ X, int x_div, const bf16_t* 
     }
 }
 
-// Tiles of up to 128 pairs (from 1.5 pairs an expert on), K % 64 == 0, N % 4 == 0: a block of 128 pairs and
-// 128 rows of W (gated: 64 gate rows and their 64 up rows), a wave 64 x 64; both operands go straight from
-// memory into LDS, 64 k (a row's 128 bytes) a stage, X's rows gathered by the load, two stages, one barrier
-// each.  A load instruction brings 8 rows; 16-byte piece c of row t stands at place c ^ (t % 8) of the row.
-// X and an expert's W each within the 4 GiB that a load's 32-bit offset reaches; X, W and Y on 16-byte addresses.
-// What bounded the waves that read their rows of W themselves was that stream (16 rows x 64 bytes an
-// instruction, one step ahead) and a tile's W read once for every 64 pairs.  64 experts of 1408 x 2048, both
-// products: 2,964 tokens 1,023 -> 608 us (505 TFLOP/s), 64 tokens 303 -> 236 (1.1 GB of experts at 4.7 TB/s).
-template <bool GATED>
-__global__ void __launch_bounds__(256, 2)
-moe_tiles_kernel(const bf16_t* __restrict__ X, int x_div, const bf16_t* __restrict__ W,
+// Tiles of up to 128 or 192 pairs (from 1.5 pairs an expert on), K % 64 == 0, N % 4 == 0 (192: N % 8): the loop of
+// gemm_turns.h over a tile's pairs, X's rows gathered by the loads, and 64 NT rows of W (gated: half of them gate rows, half
+// the up rows of the same columns).  X and an expert's W each within the 4 GiB that a load's 32-bit offset reaches; X, W
+// and Y on 16-byte addresses.  Block ids go round the 8 XCDs: an XCD takes a stretch of the (tile, columns) there are, the
+// columns of a tile one after the other, so that a tile's rows of X and, through an expert's tiles, its rows of W are read
+// into that L2 once.
+// A loop of two stages with one barrier each, both drained (four waves, tiles of 128 pairs by 128 rows of W, two blocks a
+// compute unit) -> this one; 64 experts of 1408 x 2048, 6 chosen, gate|up + down in us: 2,964 tokens 406 + 208 -> 289 + 149
+// (700 TFLOP/s; of the rows of 192 a third are padding), 1,000 tokens 199 + 97 -> 167 + 95, 64 tokens 174 + 73 -> 139 + 70
+// (bound by reading the experts); 8 experts of 8192 x 4096, 1,024 tokens, 2 chosen 478 + 285 -> 425 + 174.
+template <int MT0, int MT1, int NTH, bool GATED>
+__global__ void __launch_bounds__(512, 2)
+moe_turns_kernel(const bf16_t* __restrict__ X, int x_div, const bf16_t* __restrict__ W,
                  const int32_t* __restrict__ order, const int32_t* __restrict__ tiles, int max_tiles,
                  bf16_t* __restrict__ Y, int N, int K, int act_kind, float limit, const float* __restrict__ row_w) {
-    __shared__ illm_u32x4_t st0[256 * 8], st1[256 * 8];        // [pairs, then rows of W][8 pieces]
-    // Block ids go round the 8 XCDs: an XCD takes every eighth column block, and of a tile all of them one
-    // after the other, so that a tile's rows of X and, through an expert's tiles, its rows of W are read
-    // into that L2 once.
-    const int cols = (N + (GATED ? 63 : 127)) / (GATED ? 64 : 128), per_xcd = (cols + 7) / 8;
-    const int j8 = blockIdx.x >> 3, tile = j8 / per_xcd, col_block = (j8 % per_xcd) * 8 + (blockIdx.x & 7);
-    if (col_block >= cols || tile >= tiles[3 * (size_t)max_tiles]) return;     // the whole block leaves together
-    const int e = tiles[3 * (size_t)tile], first = tiles[3 * (size_t)tile + 1];
-    const int n = tiles[3 * (size_t)tile + 2];
-    const int wave = wave_index(), lane = threadIdx.x & 63;
-    const int r = lane & 15, q = lane >> 4, wm = wave & 1, wn = wave >> 1;
+    using T = Turns<MT0, MT1, NTH, NTH>;
+    constexpr int COLS = GATED ? T::BN / 2 : T::BN;
+    __shared__ illm_u32x4_t x0a[T::UX0], x1a[T::UX1], w0a[T::UW0], w1a[T::UW1];
+    __shared__ illm_u32x4_t x0b[T::UX0], x1b[T::UX1], w0b[T::UW0], w1b[T::UW1];
+    const int cols = (N + COLS - 1) / COLS, total = tiles[3 * (size_t)max_tiles] * cols;
+    if ((int)blockIdx.x >= total) return;                      // the whole block leaves together
+    const int xcd = blockIdx.x & 7, at = xcd * (total >> 3) + min(xcd, total & 7) + (blockIdx.x >> 3);
+    const int tile = at / cols, n0 = (at - tile * cols) * COLS;
+    const int e = tiles[3 * (size_t)tile], first = tiles[3 * (size_t)tile + 1], n = tiles[3 * (size_t)tile + 2];
+    T t;
+    t.begin();
+    const uint32_t K2 = (uint32_t)K * 2u;
     const size_t wrows = GATED ? 2 * (size_t)N : (size_t)N;
-    const int n0 = col_block * (GATED ? 64 : 128);
-    // rows of W: 16 rows a product; gated: a wave's four are 2 of gate rows and the same 2 of up rows
-    auto w_row = [&](int t) __attribute__((always_inline)) {
-        return GATED ? (((t >> 5) & 1) ? N : 0) + n0 + (t >> 6) * 32 + (t & 31) : n0 + t;
+    struct Loads {
+        const T& t;
+        __amdgpu_buffer_rsrc_t rx, rw;
+        uint32_t ox0[T::CX0], ox1[T::CX1], ow0[T::CW0], ow1[T::CW1], at, last;     // at: byte offset of stage s + 2
+        __device__ __forceinline__ void x1(illm_u32x4_t* to) const { t.load(to, rx, ox1, min(at - 128, last)); }
+        __device__ __forceinline__ void w0(illm_u32x4_t* to) const { t.load(to, rw, ow0, min(at, last)); }
+        __device__ __forceinline__ void x0(illm_u32x4_t* to) const { t.load(to, rx, ox0, min(at, last)); }
+        __device__ __forceinline__ void w1(illm_u32x4_t* to) { t.load(to, rw, ow1, min(at, last)); at += 128; }
+    } ld = {t, illm_buffer(X, 0xffffffffu), illm_buffer(W + (size_t)e * wrows * K, wrows * K * 2), {}, {}, {}, {}, 0, K2 - 128};
+    auto x_at = [&](int row) { return (uint32_t)(order[first + min(row, n - 1)] / x_div) * K2 + t.lc; };
+    auto w_at = [&](typename T::WAt w, int half) {
+        const int c = turns_column<NTH>(w.tile, w.row);
+        return (uint32_t)(n0 + (GATED ? w.wave * NTH * 16 + c + half * N : (2 * w.wave + half) * NTH * 16 + c)) * K2 + t.lc;
     };
-    const __amdgpu_buffer_rsrc_t xr = illm_buffer(X, 0xffffffffu);
-    const __amdgpu_buffer_rsrc_t wr = illm_buffer(W + (size_t)e * wrows * K, wrows * K * 2);
-    uint32_t xo[4], wo[4];
-    const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 16;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int t = (i * 4 + wave) * 8 + lr;
-        xo[i] = (uint32_t)(order[first + min(t, n - 1)] / x_div) * (uint32_t)K * 2u + lc;
-        wo[i] = (uint32_t)w_row(t) * (uint32_t)K * 2u + lc;
+    for (int i = 0; i < T::CX0; ++i) ld.ox0[i] = x_at(t.template x_row<MT0>(i, 0));
+#pragma unroll
+    for (int i = 0; i < T::CX1; ++i) ld.ox1[i] = x_at(t.template x_row<MT1>(i, MT0 * 16));
+#pragma unroll
+    for (int i = 0; i < NTH; ++i) {
+        ld.ow0[i] = w_at(t.template w_row<NTH>(i), 0);
+        ld.ow1[i] = w_at(t.template w_row<NTH>(i), 1);
     }
-    auto load = [&](illm_u32x4_t* b, int k) __attribute__((always_inline)) {
-        const uint32_t at = (uint32_t)min(k, K - 64) * 2;      // (past the end: not used)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            ld16_lds(xr, b + (i * 4 + wave) * 64, xo[i], at);
-            ld16_lds(wr, b + 1024 + (i * 4 + wave) * 64, wo[i], at);
-        }
-    };
-    moe_f32x4_t acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = (moe_f32x4_t){0.f, 0.f, 0.f, 0.f};
-    const int w_at = (128 + wn * 64 + r) * 8, x_at = (wm * 64 + r) * 8;
-    // a stage stands when every wave's loads of it have arrived; by then nobody reads the other buffer
-    // any more (a wave waits for its LDS reads too), so the next stage goes there
-    auto turn = [&](const illm_u32x4_t* cur, illm_u32x4_t* next, int k) __attribute__((always_inline)) {
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(0x0070);                    // vmcnt(0), lgkmcnt(0)
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        load(next, k + 64);
-        if (k >= K) return;
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            const int c = (kk * 4 + q) ^ (r & 7);
-            illm_u32x4_t wf[4], xf[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) wf[i] = cur[w_at + i * 128 + c];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) xf[j] = cur[x_at + j * 128 + c];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const moe_bf16x8_t*)&wf[i],
-                                                                        *(const moe_bf16x8_t*)&xf[j], acc[i][j], 0, 0, 0);
-        }
-    };
-    load(st0, 0);
-    for (int k = 0; k < K; k += 128) {
-        turn(st0, st1, k);
-        turn(st1, st0, k + 64);
+    t.clear();
+    ld.w0(w0a); ld.x0(x0a); ld.w1(w1a);                        // (stages past the end: the last one again, not used)
+    ld.x1(x1a);
+    ld.w0(w0b); ld.x0(x0b); ld.w1(w1b);
+    t.start(w0a);
+    const int stages = K / 64;
+    for (int s = 0; s < stages; s += 2) {
+        t.template stage<0>(x0a, x1a, w0a, w1a, x1b, w0b, ld);
+        if (s + 1 < stages) t.template stage<1>(x0b, x1b, w0b, w1b, x1a, w0a, ld);
     }
-    __builtin_amdgcn_s_waitcnt(0x0f70);                        // no load into LDS outlives the block
-    // acc[i][j][v]: row 64 wn + 16 i + 4 q + v of the block's rows of W, pair 64 wm + 16 j + r
+    t.end();
+    // acc[i][j][v]: pair wm MT 16 + 16 j + r, the i-th tile's column turns_column(i, 4 q + v)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int t = wm * 64 + 16 * j + r;
-        if (t >= n) continue;
-        const int pair = order[first + t];
+    for (int j = 0; j < T::MT; ++j) {
+        const int row = t.wm * T::MT * 16 + 16 * j + t.r;
+        if (row >= n) continue;
+        const int pair = order[first + row];
         const float rw = row_w ? row_w[pair] : 1.0f;           // W (w x) = w (W x)
 #pragma unroll
-        for (int i = 0; i < (GATED ? 2 : 4); ++i) {
-            const int col = n0 + wn * (GATED ? 32 : 64) + 16 * i + 4 * q;
+        for (int h = 0; h < (GATED ? 1 : 2); ++h) {
+            const int col = n0 + (GATED ? t.wn : 2 * t.wn + h) * NTH * 16 + t.q * 4 * NTH;
             if (col >= N) continue;
-            float v[4];
+            uint32_t o[2 * NTH];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if constexpr (GATED) {
-                    const float gate = bf16_to_f32(f32_to_bf16(acc[i][j][u] * rw));
-                    const float upv = bf16_to_f32(f32_to_bf16(acc[i + 2][j][u] * rw));
-                    v[u] = moe_act(gate, upv, act_kind, limit);
-                } else {
-                    v[u] = moe_plain_act(row_w ? acc[i][j][u] * rw : acc[i][j][u], act_kind, true);
+            for (int i = 0; i < NTH; ++i) {
+                float v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if constexpr (GATED) {
+                        const float gate = bf16_to_f32(f32_to_bf16(t.acc[i][j][u] * rw));
+                        const float upv = bf16_to_f32(f32_to_bf16(t.acc[NTH + i][j][u] * rw));
+                        v[u] = moe_act(gate, upv, act_kind, limit);
+                    } else {
+                        const float a = t.acc[h * NTH + i][j][u];
+                        v[u] = moe_plain_act(row_w ? a * rw : a, act_kind, true);
+                    }
                 }
+                o[2 * i] = pack_bf16x2(v[0], v[1]);
+                o[2 * i + 1] = pack_bf16x2(v[2], v[3]);
             }
-            *(uint2*)(Y + (size_t)pair * N + col) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+            bf16_t* const to = Y + (size_t)pair * N + col;
+            if constexpr (NTH == 2) *(uint4*)to = make_uint4(o[0], o[1], o[2], o[3]);
+            else *(uint2*)to = make_uint2(o[0], o[1]);
         }
     }
 }
@@ -1018,24 +1005,25 @@ extern "C" int illm_moe_rows_mfma(const void* X, int x_div, const void* W, int g
                                   void* Y, int N, int K, int act_kind, float limit,
                                   const float* row_w, void* stream) {
     if (!moe_act_ok(act_kind, gated) || x_div <= 0 || N <= 0 || K <= 0 || K % 32 || max_tiles < 0 || max_tiles > 2147483647 / 3 ||
-        (tile_rows != 16 && tile_rows != 32 && tile_rows != 64 && tile_rows != 128))
+        (tile_rows != 16 && tile_rows != 32 && tile_rows != 64 && tile_rows != 128 && tile_rows != 192))
         return ILLM_ERR_ARG;
     if (max_tiles == 0) return ILLM_OK;
     hipStream_t st = (hipStream_t)stream;
-    if (tile_rows == 128) {
-        if (K % 64 || N % 4 || (long long)(gated ? 2 : 1) * (N + 128) * K * 2 >= 0xffffffffLL ||
+    if (tile_rows == 128 || tile_rows == 192) {
+        // 192 pairs by 256 rows of W, one block a compute unit; 128 by 128, two (which one: `_moe_tiling`)
+        const int beyond = tile_rows == 192 ? 256 : 128;       // rows of W that a block's loads may go past the end
+        if (K % 64 || N % (tile_rows == 192 ? 8 : 4) || (long long)(gated ? 2 : 1) * (N + beyond) * K * 2 >= 0xffffffffLL ||
             ((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16)
             return ILLM_ERR_ARG;
-        const int cols = (N + (gated ? 63 : 127)) / (gated ? 64 : 128);
-        const long long blocks = 8LL * ((cols + 7) / 8) * max_tiles;
-        if (blocks > 0x7fffffffLL) return ILLM_ERR_ARG;
-        const dim3 grid((unsigned)blocks);
-        if (gated)
-            hipLaunchKernelGGL((moe_tiles_kernel<true>), grid, dim3(256), 0, st, (const bf16_t*)X, x_div, (const bf16_t*)W,
-                               order, tiles, max_tiles, (bf16_t*)Y, N, K, act_kind, limit, row_w);
-        else
-            hipLaunchKernelGGL((moe_tiles_kernel<false>), grid, dim3(256), 0, st, (const bf16_t*)X, x_div, (const bf16_t*)W,
-                               order, tiles, max_tiles, (bf16_t*)Y, N, K, act_kind, limit, row_w);
+        const int width = beyond / (gated ? 2 : 1);
+        const long long blocks = (long long)max_tiles * ((N + width - 1) / width);
+        if (blocks > 0x7fffffLL) return ILLM_ERR_ARG;
+#define GO_TURNS(MT0_, MT1_, NTH_, G_)                                                             \
+    hipLaunchKernelGGL((moe_turns_kernel<MT0_, MT1_, NTH_, G_>), dim3((unsigned)blocks), dim3(512), 0, st, (const bf16_t*)X, \
+                       x_div, (const bf16_t*)W, order, tiles, max_tiles, (bf16_t*)Y, N, K, act_kind, limit, row_w)
+        if (tile_rows == 192) { if (gated) GO_TURNS(4, 2, 2, true); else GO_TURNS(4, 2, 2, false); }
+        else { if (gated) GO_TURNS(2, 2, 1, true); else GO_TURNS(2, 2, 1, false); }
+#undef GO_TURNS
         return illm_launch_status();
     }
     if (tile_rows == 64 && K % 64 == 0) {

@@ -1613,7 +1613,7 @@ MOE_MFMA_FROM = 0        # (token, choice) pairs an expert on average from which
                          # K took 253 + 166 us for 64 tokens, bound by its sums across lanes)
 
 
-# Where the kernel with both operands in LDS, in tiles of 128 pairs, takes bfloat16 experts whose sizes are
+# Where the kernel with both operands in LDS, in tiles of 128 pairs or more, takes bfloat16 experts whose sizes are
 # multiples of 64.  It beats the smaller tiles from 24 pairs an expert on with every stack (their kernels for 32
 # and 64 pairs are the slow ones); with fewer pairs where the stack has blocks enough for the chip (columns of 64
 # and of 128) and a matrix is large enough for its pairs to be worth a block.  us, both products, tiles of 16 pairs -> of 128:
@@ -1628,11 +1628,17 @@ MOE_MFMA_FROM = 0        # (token, choice) pairs an expert on average from which
 #   16 of 512 x 512            18 ->  22   18 ->  22   18 ->  22   20 ->  25   50 ->  27
 #   8 of 2048 x 1024           40 ->  58   41 ->  58   43 ->  58   48 ->  59  109 ->  61
 #   2 of 4096 x 4096           65 -> 131   67 -> 131   71 -> 131   79 -> 131  274 -> 133
-# (2,964 tokens of the first, 6 chosen: 1,023 -> 608.)  The same bits.
+# (2,964 tokens of the first, 6 chosen: 1,023 -> 608.)  The same bits.  (Measured with the loop before the one
+# in turns, which takes 4 to 20 % less with few pairs an expert; tiles of 16 pairs take less now too.)
 MOE_TILES_ALWAYS = 24              # pairs an expert on average
 MOE_TILES_BLOCKS = (256, 512)      # blocks of the thinner product: none with fewer than the first, from 12 pairs an
                                    # expert on with fewer than the second, from 1.5 on with more
 MOE_TILES_WORK = 1 << 23           # pairs an expert times its F E
+# Tiles of 192 pairs and blocks of 256 rows of W from so many pairs an expert on, where that leaves every compute unit
+# a block.  us, gate|up + down, tiles of 128 -> of 192: 64 of 1408 x 2048 at 94 pairs 167 + 95 -> 174 + 94, at 278
+# 369 + 193 -> 289 + 149; 32 of 4096 x 2048 at 128 330 + 170 -> 237 + 139; 8 of 8192 x 4096 at 256 536 + 268 ->
+# 425 + 174; 16 of 512 x 512 at 256 (64 blocks) 15 + 11 -> 21 + 17.
+MOE_WIDE_FROM, MOE_WIDE_BLOCKS = 112, 256
 
 
 def _moe_tiles_pay(E: int, F: int, NP: int, n_exp: int) -> bool:
@@ -1647,6 +1653,13 @@ def _moe_tiles_pay(E: int, F: int, NP: int, n_exp: int) -> bool:
 def _moe_few_rows(per_expert: float) -> int:
     """Rows a tile of the matrix-core kernels that read what lies at any address."""
     return 64 if per_expert >= 48 else 32 if per_expert >= 24 else 16
+
+
+def _moe_wide(E: int, F: int, NP: int, n_exp: int) -> bool:
+    """Whether pairs that go in tiles of 128 go in tiles of 192."""
+    per_expert = NP / max(1, n_exp)
+    return (per_expert >= MOE_WIDE_FROM and 4 * (max(E, F) + 256) * max(E, F) < 1 << 32
+            and n_exp * -(-int(per_expert) // 192) * min(-(-F // 128), -(-E // 256)) >= MOE_WIDE_BLOCKS)
 
 
 def _moe_tiling(dtype: torch.dtype, E: int, F: int, NP: int, n_exp: int):
@@ -1664,11 +1677,14 @@ def _moe_tiling(dtype: torch.dtype, E: int, F: int, NP: int, n_exp: int):
 
 def _moe_group(idx: torch.Tensor, n_exp: int, dtype: torch.dtype, E: int, F: int, on16: bool = True):
     """The pairs grouped by expert.  `on16`: the rows and the experts' matrices lie on 16-byte addresses, as the
-    tiles of 128 pairs want them (straight into LDS, 16 bytes a lane)."""
+    tiles of 128 pairs and more want them (straight into LDS, 16 bytes a lane)."""
     NP = idx.numel()
     mfma, rows, max_tiles = _moe_tiling(dtype, E, F, NP, n_exp)
-    if rows == 128 and not on16:
-        rows = _moe_few_rows(NP / max(1, n_exp))
+    if rows >= 128:
+        if not on16:
+            rows = _moe_few_rows(NP / max(1, n_exp))
+        elif _moe_wide(E, F, NP, n_exp):
+            rows = 192
         max_tiles = max(1, min(NP, NP // rows + n_exp))
     order = torch.empty((NP,), dtype=torch.int32, device=idx.device)
     tiles = torch.empty((3 * max_tiles + 1,), dtype=torch.int32, device=idx.device)
@@ -1720,7 +1736,7 @@ def moe_experts(h: torch.Tensor, idx: torch.Tensor, w_gate_up: torch.Tensor, w_d
           "moe_experts: shapes or dtypes")
     NP = T * top
     on16 = _on16(h, w_gate_up, w_down)
-    if grouped is None or (grouped[3] == 128 and not on16):
+    if grouped is None or (grouped[3] >= 128 and not on16):
         grouped = _moe_group(idx, n_exp, h.dtype, E, F, on16)
     order, tiles, max_tiles, rows, mfma = grouped
     act = torch.empty((NP, F), dtype=h.dtype, device=h.device)

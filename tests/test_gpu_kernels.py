@@ -910,6 +910,31 @@ def test_moe_tiles_of_128_pairs(T, E, F, NE, top, act):
     assert real(torch.bfloat16, E, F, 24 * NE, NE)[1] == 128 and real(torch.bfloat16, E, F + 32, 24 * NE, NE)[1] != 128
 
 
+@pytest.mark.parametrize("T,E,F,NE,top,act", [(1, 64, 64, 2, 1, "silu"), (193, 192, 320, 1, 1, "clamped_swish"), (400, 448, 128, 3, 2, "silu"),
+                                              (385, 128, 192, 2, 2, "relu_squared"), (130, 64, 576, 5, 5, "silu")])
+def test_moe_tiles_of_192_pairs(T, E, F, NE, top, act):
+    """Tiles of up to 192 pairs in turns of two groups of waves give the bits of the kernel for 16 pairs: one stage of
+    64 k, odd and even numbers of them, tiles of one row, whole ones and remainders, columns that end inside a block."""
+    o = ops()
+    gated = act != "relu_squared"
+    g = torch.Generator().manual_seed(6)
+    h = rnd(T, E, dtype=torch.bfloat16, seed=1).to(DEV)
+    wu = (rnd(NE, F * (2 if gated else 1), E, seed=2) * 0.1).to(torch.bfloat16).to(DEV)
+    wd = (rnd(NE, E, F, seed=3) * 0.1).to(torch.bfloat16).to(DEV)
+    idx = torch.stack([torch.randperm(NE, generator=g)[:top] for _ in range(T)]).to(torch.int32).to(DEV)
+    wt = torch.rand(T, top, generator=g).to(DEV) if act == "clamped_swish" else None
+    real, got = o._moe_tiling, []
+    try:
+        for rows in (16, 192):
+            o._moe_tiling = lambda dtype, e, f, np, n: (True, rows, max(1, min(np, np // rows + n)))
+            got.append(o.moe_experts(h, idx, wu, wd, None, act, 7.0 if act == "clamped_swish" else 0.0, wt))
+    finally:
+        o._moe_tiling = real
+    assert torch.equal(got[0], got[1]) and bool(torch.isfinite(got[1].float()).all())
+    wide = lambda per, n: o._moe_wide(2048, 1408, per * n, n)  # noqa: E731
+    assert [wide(*c) for c in ((24, 64), (111, 64), (112, 64), (112, 8), (400, 8))] == [False, False, True, False, False]
+
+
 @pytest.mark.parametrize("T,E,F,NE,top,act", [(8, 64, 64, 9, 1, "silu"), (17, 192, 96, 8, 2, "clamped_swish"), (90, 64, 320, 3, 2, "relu_squared"),
                                               (12, 2048, 64, 16, 3, "silu"), (20, 4160, 64, 9, 2, "relu_squared")])
 def test_moe_products_of_few_tokens_by_whole_lines(T, E, F, NE, top, act):
