@@ -1019,9 +1019,9 @@ attn_cap_decode_kernel(const void* __restrict__ q, int q_stride, const void* __r
     if (threadIdx.x == 0) { pp[dv] = mm; pp[dv + 1] = lt; }
 }
 
-// Single tokens with key and value widths of up to 128 in steps of 4 (float32) or 8 (bfloat16).
+// Single tokens in float32 with key and value widths of up to 128 in steps of 4.
 // grid (kv heads x groups of up to 4 query heads that share them, sequences, splits); 256 threads.
-// Eight lanes take a key, each 16 bytes of a row at a time (a unit: 4 floats or 8 bfloat16), so a
+// Eight lanes take a key, each 16 bytes of a row at a time (a unit: 4 floats), so a
 // wave reads 8 rows of keys (and of values) an instruction, a whole 128-byte line a row, for all
 // the block's query heads at once; a score is 3 exchanges among the eight lanes.  Every group of
 // eight keeps its own running max, sum and weighted values (lane s of a group holds dims U s + 8 U j
@@ -1029,8 +1029,8 @@ attn_cap_decode_kernel(const void* __restrict__ q, int q_stride, const void* __r
 // between lanes and rows of lanes, no LDS), then the waves, are combined at the end in a fixed order.
 // Bound by trips to memory, few of which follow each other: q, the pages and two rounds of keys and values
 // are in flight at once.  `partial` as above; a range without keys leaves only its maximum and its sum.
-// With the merge, 16 ranges, 8 sequences of 1,040 keys, 16 heads of 128 over 4: bfloat16 22.4 -> 15.5 us, float32
-// 23.8 -> 16.0 against q read head by head, one round in flight and the sums through LDS.
+// With the merge, 16 ranges, 8 sequences of 1,040 keys, 16 heads of 128 over 4: 23.8 -> 16.0 us against q read
+// head by head, one round in flight and the sums through LDS.
 template <int CTRL>
 __device__ __forceinline__ float cap_dpp(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, 0xf, 0xf, true));
@@ -1054,17 +1054,17 @@ __device__ __forceinline__ float cap_sum_groups(float v) {
     return r.x + r.y;
 }
 
-template <int DT, int KQ, int VQ, int DH>        // DH: query heads a block takes at most
+template <int KQ, int VQ, int DH>                // DH: query heads a block takes at most
 __global__ void __launch_bounds__(256)
-attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const void* __restrict__ kcache,
-                             const void* __restrict__ vcache, const int32_t* __restrict__ page_table,
+attn_cap_decode_rows8_kernel(const float* __restrict__ q, int q_stride, const float* __restrict__ kcache,
+                             const float* __restrict__ vcache, const int32_t* __restrict__ page_table,
                              int table_stride, int page_size, int ring, const int32_t* __restrict__ seq_slot,
                              const int32_t* __restrict__ seq_len, float* __restrict__ partial, int nsplit,
                              int nh, int nkv, int dk, int dv, float scale, float cap, int window,
                              const float* __restrict__ slopes, int chunk, void* __restrict__ out,
                              const void* __restrict__ gate, int gate_stride, int gate_off, int gate_heads,
                              int keep, int kept, const float* __restrict__ sink) {
-    constexpr int U = DT == ILLM_BF16 ? 8 : 4;          // elements of a unit
+    constexpr int U = 4;                                // floats of a unit
     constexpr int NK = U * KQ, NV = U * VQ;             // dims of a key, of a value, a lane holds
     __shared__ __attribute__((aligned(16))) float wacc[4][DH][8 * NV];
     __shared__ float wm[4][DH], wl[4][DH];
@@ -1100,7 +1100,7 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
         for (int j = 0; j < KQ; ++j) {             // (a head or a column that is not there reads one that is)
             const int d = U * sub + 8 * U * j;
             const size_t at = (size_t)b * q_stride + (size_t)(h0 + (i < hb ? i : 0)) * dk + (d < dk ? d : 0);
-            qr[i][j] = *(const illm_u32x4_t*)((const char*)q + at * (DT == ILLM_BF16 ? 2 : 4));
+            qr[i][j] = *(const illm_u32x4_t*)(q + at);
         }
     }
     // two rounds in flight, one where a round's rows take more registers (float32 of more than 64 dims: 27.3
@@ -1108,17 +1108,8 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
     constexpr int AHEAD = KQ + VQ <= 4 ? 2 : 1;
     illm_u32x4_t kn[AHEAD][KQ], vn[AHEAD][VQ];
     auto unit_floats = [&](const illm_u32x4_t r, float* x) __attribute__((always_inline)) {
-        if (DT == ILLM_BF16) {
-            const uint32_t wd[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                x[2 * k] = __uint_as_float(wd[k] << 16);
-                x[2 * k + 1] = __uint_as_float(wd[k] & 0xffff0000u);
-            }
-        } else {
-            x[0] = __uint_as_float(r.x); x[1] = __uint_as_float(r.y);
-            x[2] = __uint_as_float(r.z); x[3] = __uint_as_float(r.w);
-        }
+        x[0] = __uint_as_float(r.x); x[1] = __uint_as_float(r.y);
+        x[2] = __uint_as_float(r.z); x[3] = __uint_as_float(r.w);
     };
     // the page of a round's key is looked up AHEAD rounds before its rows are asked for, and the rows AHEAD
     // rounds before they are used
@@ -1131,16 +1122,15 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
         const int kj = seen.at(min(base + grp, k_hi - 1));
         const size_t row = ((size_t)page * nkv + kvh) * page_size + (kj % page_size);
         const size_t kat = row * dk, vat = row * dv;
-        const size_t esz = DT == ILLM_BF16 ? 2 : 4;
 #pragma unroll
         for (int j = 0; j < KQ; ++j) {
             const int d = U * sub + 8 * U * j;
-            kn[s][j] = *(const illm_u32x4_t*)((const char*)kcache + (kat + (d < dk ? d : 0)) * esz);
+            kn[s][j] = *(const illm_u32x4_t*)(kcache + kat + (d < dk ? d : 0));
         }
 #pragma unroll
         for (int j = 0; j < VQ; ++j) {
             const int d = U * sub + 8 * U * j;
-            vn[s][j] = *(const illm_u32x4_t*)((const char*)vcache + (vat + (d < dv ? d : 0)) * esz);
+            vn[s][j] = *(const illm_u32x4_t*)(vcache + vat + (d < dv ? d : 0));
         }
     };
     int pages[AHEAD];
@@ -1195,9 +1185,8 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
             d += cap_dpp<0x141>(d);
             const float sc = valid ? soft_cap(d * scale, cap, inv_cap) - slope[i] * (float)(len - 1 - kj) : NEG_INF;
             const float m_new = fmaxf(m[i], sc);
-            // (bfloat16 keys and values: the hardware's exponential, float32 with an error of |x| 2^-24)
-            const float alpha = m_new == NEG_INF ? 1.f : DT == ILLM_BF16 ? __expf(m[i] - m_new) : expf(m[i] - m_new);
-            const float p = !valid ? 0.f : DT == ILLM_BF16 ? __expf(sc - m_new) : expf(sc - m_new);
+            const float alpha = m_new == NEG_INF ? 1.f : expf(m[i] - m_new);
+            const float p = !valid ? 0.f : expf(sc - m_new);
             l[i] = l[i] * alpha + p;
             m[i] = m_new;
 #pragma unroll
@@ -1246,8 +1235,175 @@ attn_cap_decode_rows8_kernel(const void* __restrict__ q, int q_stride, const voi
             if (sink) add_sink(sink[h0 + i], mm, lt);
             y *= 1.0f / lt;
             if (gate)
-                y *= 1.0f / (1.0f + expf(-ld_f(gate, DT, (size_t)b * gate_stride + gate_off + (gate_heads ? (size_t)(h0 + i) : (size_t)(h0 + i) * dv + d))));
-            st_f(out, DT, ((size_t)b * nh + h0 + i) * dv + d, y);
+                y *= 1.0f / (1.0f + expf(-ld_f(gate, ILLM_F32, (size_t)b * gate_stride + gate_off + (gate_heads ? (size_t)(h0 + i) : (size_t)(h0 + i) * dv + d))));
+            st_f(out, ILLM_F32, ((size_t)b * nh + h0 + i) * dv + d, y);
+            continue;
+        }
+        float* pp = partial + (((size_t)b * nh + h0 + i) * nsplit + sp) * (dv + 2);
+        pp[d] = y;
+        if (d == 0) { pp[dv] = mm; pp[dv + 1] = lt; }
+    }
+}
+
+// The same in bfloat16.  A wave takes 16 keys at a time: their products with up to four query heads on the matrix cores
+// (MFMA 16x16x32, keys as the rows, heads as the columns, so that a lane has four keys' scores of one head), the
+// softmax's weights in float32 through a piece of LDS, and the weighted values on the vector unit with two
+// neighbouring dims a lane: a value's row is one load instruction, the weights are the same for all lanes, and nothing
+// is left to add across lanes.  A head's sums do not depend on which others the block has.  Bound by the chain of
+// loads (length and slot, page, rows) and, before, by its own instructions: eight lanes a key and all dims of a
+// key for one head after the other took some 1,200 vector instructions for 16 keys and four heads, this some 300.
+// Attention and merge, 16 ranges, 16 heads of 128 over 4, 8 sequences of 61 to 1,040 keys: 16.0 -> 11.8 us,
+// in chunks of 1,024 14.5 -> 9.8; 64 sequences of 500 in one range 26.9 -> 24.9.
+typedef __bf16 cap_bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float cap_f32x4_t __attribute__((ext_vector_type(4)));
+
+template <int DH, int KC>                          // DH: query heads a block takes at most; KC: ceil(dk / 32)
+__global__ void __launch_bounds__(256)
+attn_cap_decode_keys16_kernel(const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kcache,
+                              const bf16_t* __restrict__ vcache, const int32_t* __restrict__ page_table,
+                              int table_stride, int page_size, int ring, const int32_t* __restrict__ seq_slot,
+                              const int32_t* __restrict__ seq_len, float* __restrict__ partial, int nsplit,
+                              int nh, int nkv, int dk, int dv, float scale, float cap, int window,
+                              const float* __restrict__ slopes, int chunk, void* __restrict__ out,
+                              const void* __restrict__ gate, int gate_stride, int gate_off, int gate_heads,
+                              int keep, int kept, const float* __restrict__ sink) {
+    __shared__ __attribute__((aligned(16))) float wacc[4][DH][128], weights[4][17][DH];    // [16]: the old sums' factor
+    __shared__ float wm[4][DH], wl[4][DH];
+    const int rep = nh / nkv, per_kv = (rep + DH - 1) / DH;
+    const int kvh = blockIdx.x / per_kv, h0 = kvh * rep + (blockIdx.x % per_kv) * DH;
+    const int hb = min(DH, (kvh + 1) * rep - h0);
+    const int b = blockIdx.z, sp = blockIdx.y;
+    const int w = wave_index(), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int len = seq_len[b], slot = seq_slot[b];
+    const SeenKeys seen = seen_keys(len, window, chunk, keep);
+    const int tiles = (seen.hi + 63) / 64, t0 = seen.lo / 64;
+    const int per = (tiles - t0 + nsplit - 1) / nsplit;
+    const int k_lo = max(seen.lo, (t0 + sp * per) * 64), k_hi = min(seen.hi, (t0 + (sp + 1) * per) * 64);
+    if (k_lo >= k_hi && nsplit > 1) {              // no key: the merge leaves the range's values alone
+        if ((int)threadIdx.x < hb) {
+            float* pp = partial + (((size_t)b * nh + h0 + threadIdx.x) * nsplit + sp) * (dv + 2);
+            pp[dv] = NEG_INF; pp[dv + 1] = 0.f;
+        }
+        return;
+    }
+    const float inv_cap = cap > 0.f ? 1.0f / cap : 0.f;
+    const int head = h0 + (r < hb ? r : 0);        // (columns beyond the block's heads: never read)
+    const float slope = slopes ? slopes[head] : 0.f;
+    illm_u32x4_t qf[KC];
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+        const int d = c * 32 + g * 8;
+        qf[c] = *(const illm_u32x4_t*)(q + (size_t)b * q_stride + (size_t)head * dk + (d < dk ? d : 0));
+    }
+    struct Rows { illm_u32x4_t k[KC]; uint32_t v[16]; };
+    // the cache row of this lane's key (key r of 16 from `base` on; past the range its last one)
+    auto row_of = [&](int base) __attribute__((always_inline)) {
+        const int kj = seen.at(min(base + r, k_hi - 1));
+        int lp = kj / page_size;
+        const int in = kj - lp * page_size;
+        if (ring > 0 && lp >= kept) lp = kept + (lp - kept) % ring;
+        return make_int2(page_table[(size_t)slot * table_stride + lp] * nkv + kvh, in);    // (head's part of a page, row in it)
+    };
+    auto fetch = [&](Rows& x, int2 row) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+            const int d = c * 32 + g * 8;
+            x.k[c] = *(const illm_u32x4_t*)(kcache + ((size_t)row.x * page_size + row.y) * dk + (d < dk ? d : 0));
+        }
+        const int at = 2 * lane < dv ? 2 * lane : 0;
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            x.v[j] = *(const uint32_t*)(vcache + ((size_t)__builtin_amdgcn_readlane(row.x, j) * page_size +
+                                                  __builtin_amdgcn_readlane(row.y, j)) * dv + at);
+        __builtin_amdgcn_sched_barrier(0);         // (else a row's load is put right before its use)
+    };
+    float acc[DH][2], m = NEG_INF, l = 0.f;
+#pragma unroll
+    for (int i = 0; i < DH; ++i) acc[i][0] = acc[i][1] = 0.f;
+    auto round = [&](const Rows& x, int base) __attribute__((always_inline)) {
+        cap_f32x4_t s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+            const bool there = c * 32 + g * 8 < dk;           // (columns beyond dk: nothing)
+            const illm_u32x4_t none = {0u, 0u, 0u, 0u}, kf = there ? x.k[c] : none, qc = there ? qf[c] : none;
+            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const cap_bf16x8_t*)&kf, *(const cap_bf16x8_t*)&qc, s, 0, 0, 0);
+        }
+        float tm = NEG_INF;                                   // s[i]: key base + 4 g + i with head r
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int k = base + 4 * g + i;
+            s[i] = k < k_hi ? soft_cap(s[i] * scale, cap, inv_cap) - slope * (float)(len - 1 - seen.at(k)) : NEG_INF;
+            tm = fmaxf(tm, s[i]);
+        }
+        float2 two = cap_swap16(tm);
+        two = cap_swap32(fmaxf(two.x, two.y));
+        const float m_new = fmaxf(m, fmaxf(two.x, two.y));
+        // (the hardware's exponential: float32 with an error of |x| 2^-24)
+        const float alpha = m_new == NEG_INF ? 1.f : __expf(m - m_new);
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float p = base + 4 * g + i < k_hi ? __expf(s[i] - m_new) : 0.f;
+            sum += p;
+            if (r < DH) weights[w][4 * g + i][r] = p;
+        }
+        if (r < DH && g == 0) weights[w][16][r] = alpha;
+        two = cap_swap16(sum);
+        two = cap_swap32(two.x + two.y);
+        l = l * alpha + (two.x + two.y);
+        m = m_new;
+#pragma unroll
+        for (int i = 0; i < DH; ++i) {
+            const float f = weights[w][16][i];
+            acc[i][0] *= f;
+            acc[i][1] *= f;
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {                        // (past the range: zeros, or infinities times 0 were NaN)
+            const uint32_t v = base + j < k_hi ? x.v[j] : 0u;
+            const float lo = __uint_as_float(v << 16), hi = __uint_as_float(v & 0xffff0000u);
+#pragma unroll
+            for (int i = 0; i < DH; ++i) {
+                const float p = weights[w][j][i];
+                acc[i][0] = fmaf(p, lo, acc[i][0]);
+                acc[i][1] = fmaf(p, hi, acc[i][1]);
+            }
+        }
+    };
+    int base = k_lo + 16 * w;
+    if (base < k_hi) {                             // the next rows are on their way while these are worked on
+        Rows x0, x1;
+        fetch(x0, row_of(base));
+        for (; base < k_hi; base += 128) {
+            if (base + 64 < k_hi) fetch(x1, row_of(base + 64));
+            round(x0, base);
+            if (base + 64 >= k_hi) break;
+            if (base + 128 < k_hi) fetch(x0, row_of(base + 128));
+            round(x1, base + 64);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < DH; ++i) *(float2*)&wacc[w][i][2 * lane] = make_float2(acc[i][0], acc[i][1]);
+    if (lane < DH) { wm[w][lane] = m; wl[w][lane] = l; }
+    __syncthreads();
+    // the four waves into one: the block's threads over all (head, value dim) pairs
+    for (int e = threadIdx.x; e < hb * dv; e += 256) {
+        const int i = e / dv, d = e - i * dv;
+        float mm = wm[0][i];
+        for (int x = 1; x < 4; ++x) mm = fmaxf(mm, wm[x][i]);
+        float lt = 0.f, y = 0.f;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const float f = wm[x][i] == NEG_INF ? 0.f : expf(wm[x][i] - mm);
+            lt += f * wl[x][i];
+            y += f * wacc[x][i][d];
+        }
+        if (nsplit == 1) {                              // the one range is the whole result: no merge
+            if (sink) add_sink(sink[h0 + i], mm, lt);
+            y *= 1.0f / lt;
+            if (gate)
+                y *= 1.0f / (1.0f + expf(-ld_f(gate, ILLM_BF16, (size_t)b * gate_stride + gate_off + (gate_heads ? (size_t)(h0 + i) : (size_t)(h0 + i) * dv + d))));
+            st_f(out, ILLM_BF16, ((size_t)b * nh + h0 + i) * dv + d, y);
             continue;
         }
         float* pp = partial + (((size_t)b * nh + h0 + i) * nsplit + sp) * (dv + 2);
@@ -1335,32 +1491,31 @@ extern "C" int illm_attn_cap_decode(const void* q, int q_stride, void* out, int 
             for (dh = 4; dh > 1 && (long)nkv * ((rep + dh - 1) / dh) * B * nsplit < 256;) dh /= 2;
         // (a sequence's ranges next to each other: the longest sequence's go to many compute units)
         const dim3 grid(nkv * ((rep + dh - 1) / dh), nsplit, B);
-        const int kq = (dk + 8 * unit - 1) / (8 * unit), vq = (dv + 8 * unit - 1) / (8 * unit);
-#define GO(DT_, KQ_, VQ_)                                                                          \
-    if (dh == 1)                                                                                   \
-        hipLaunchKernelGGL((attn_cap_decode_rows8_kernel<DT_, KQ_, VQ_, 1>), grid, dim3(256), 0, st, q, q_stride, \
-                           kcache, vcache, page_table, table_stride, page_size, ring, seq_slot, seq_len, partial, \
-                           nsplit, nh, nkv, dk, dv, scale, cap, window, slopes, chunk, out, gate, gate_stride, gate_off, gate_heads, \
-                           keep, kept, sink);                                                      \
-    else if (dh == 2)                                                                              \
-        hipLaunchKernelGGL((attn_cap_decode_rows8_kernel<DT_, KQ_, VQ_, 2>), grid, dim3(256), 0, st, q, q_stride, \
-                           kcache, vcache, page_table, table_stride, page_size, ring, seq_slot, seq_len, partial, \
-                           nsplit, nh, nkv, dk, dv, scale, cap, window, slopes, chunk, out, gate, gate_stride, gate_off, gate_heads, \
-                           keep, kept, sink);                                                      \
-    else                                                                                           \
-        hipLaunchKernelGGL((attn_cap_decode_rows8_kernel<DT_, KQ_, VQ_, 4>), grid, dim3(256), 0, st, q, q_stride, \
-                           kcache, vcache, page_table, table_stride, page_size, ring, seq_slot, seq_len, partial, \
-                           nsplit, nh, nkv, dk, dv, scale, cap, window, slopes, chunk, out, gate, gate_stride, gate_off, gate_heads, \
-                           keep, kept, sink)
-#define GO_V(DT_, KQ_)                                                                             \
-    switch (vq) { case 1: { GO(DT_, KQ_, 1); } break; case 2: { GO(DT_, KQ_, 2); } break;          \
-                  case 3: { GO(DT_, KQ_, 3); } break; default: { GO(DT_, KQ_, 4); } break; }
-#define GO_K(DT_)                                                                                  \
-    switch (kq) { case 1: GO_V(DT_, 1) break; case 2: GO_V(DT_, 2) break;                          \
-                  case 3: GO_V(DT_, 3) break; default: GO_V(DT_, 4) break; }
-        if (dt == ILLM_BF16) { GO_K(ILLM_BF16) } else { GO_K(ILLM_F32) }
+#define GO(KERNEL, T_, ...)                                                                        \
+    hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), grid, dim3(256), 0, st, (const T_*)q, q_stride, (const T_*)kcache, (const T_*)vcache, \
+                       page_table, table_stride, page_size, ring, seq_slot, seq_len, partial, nsplit, nh, nkv, dk, dv, \
+                       scale, cap, window, slopes, chunk, out, gate, gate_stride, gate_off, gate_heads, keep, kept, sink)
+        const int kc = (dk + 31) / 32, vc = (dv + 31) / 32;
+        if (dt == ILLM_BF16) {
+#define GO_K(DH_)                                                                                  \
+    switch (kc) { case 1: GO(attn_cap_decode_keys16_kernel, bf16_t, DH_, 1); break;                \
+                  case 2: GO(attn_cap_decode_keys16_kernel, bf16_t, DH_, 2); break;                \
+                  case 3: GO(attn_cap_decode_keys16_kernel, bf16_t, DH_, 3); break;                \
+                  default: GO(attn_cap_decode_keys16_kernel, bf16_t, DH_, 4); }
+            if (dh == 1) { GO_K(1) } else if (dh == 2) { GO_K(2) } else { GO_K(4) }
 #undef GO_K
+        } else {
+#define GO_H(KQ_, VQ_)                                                                             \
+    if (dh == 1) GO(attn_cap_decode_rows8_kernel, float, KQ_, VQ_, 1);                             \
+    else if (dh == 2) GO(attn_cap_decode_rows8_kernel, float, KQ_, VQ_, 2);                        \
+    else GO(attn_cap_decode_rows8_kernel, float, KQ_, VQ_, 4)
+#define GO_V(KQ_)                                                                                  \
+    switch (vc) { case 1: { GO_H(KQ_, 1); } break; case 2: { GO_H(KQ_, 2); } break;                \
+                  case 3: { GO_H(KQ_, 3); } break; default: { GO_H(KQ_, 4); } }
+            switch (kc) { case 1: GO_V(1) break; case 2: GO_V(2) break; case 3: GO_V(3) break; default: GO_V(4) }
 #undef GO_V
+#undef GO_H
+        }
 #undef GO
         if (nsplit == 1) return illm_launch_status();    // written whole by the kernel itself
     } else if (dt == ILLM_BF16)

@@ -1970,3 +1970,29 @@ def test_capped_decode_of_infinite_values(dk, dv, dtype):
         got = got.float().cpu().view(B, nh, dv)
         assert bool((got[:, :, 5] == float("inf")).all()), nsplit
         assert bool(torch.isfinite(got[:, :, [d for d in range(dv) if d != 5]]).all()), nsplit
+
+
+@pytest.mark.parametrize("nh, nkv, dk, dv", [(8, 2, 128, 128), (5, 1, 72, 40), (3, 3, 32, 8)])
+def test_capped_decode_steps_of_16_keys(nh, nkv, dk, dv):
+    """bfloat16 key counts around a wave's steps (16 keys, the next one 64 further on) that end in the first, the second
+    and the third of them; a head has the same bits whether a block takes four heads, two or one."""
+    g, o, page = torch.Generator().manual_seed(nh + dk), ops(), 32
+    lens = [15, 16, 17, 63, 79, 80, 81, 143, 145, 257]
+    B, per = len(lens), 9
+    table = torch.randperm(B * per, generator=g).view(B, per).to(torch.int32)
+    kc, vc = (torch.randn(B * per, nkv, page, d, generator=g).to(torch.bfloat16) for d in (dk, dv))
+    q, slots = torch.randn(B, nh * dk, generator=g).to(torch.bfloat16), torch.randperm(B, generator=g).to(torch.int32)
+    seq_len = torch.tensor(lens, dtype=torch.int32)
+    on = [t.to(DEV) for t in (q, kc, vc, table, slots, seq_len)]
+    want = R.attn_cap_decode(q, kc, vc, table, page, 0, slots, seq_len, nh, nkv, dk, dv, dk ** -0.5, 0.0, 0, 1).double()
+    try:
+        for nsplit in (1, 2):
+            got = []
+            for heads in (4, 2, 1):
+                o._lib().illm_set_attn_cap_heads(heads)
+                got.append(o.attn_cap_decode(*on[:4], page, 0, *on[4:], nh, nkv, dk, dv, dk ** -0.5, 0.0, 0, nsplit))
+            assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+            # (the result's rounding, 2^-9, and the exponential's)
+            assert float((got[0].double().cpu() - want).abs().max()) <= 2 ** -8 * max(1.0, float(want.abs().max())), nsplit
+    finally:
+        o._lib().illm_set_attn_cap_heads(0)
