@@ -14,6 +14,8 @@
 // Lanes of X rows >= M read row M - 1 and their results are dropped.
 //
 // The reference calls cublasSgemm with M = 1 here (src/kern/gpu/kernel_gpu.cu:420-435).
+#include <type_traits>
+
 #include "api.h"
 #include "api_test.h"
 #include "common.h"
@@ -66,6 +68,13 @@ struct SkResidual {
     int act;                     // SK_PLAIN without `accumulate`, ACT: 1 relu(y)^2, 2 gelu(y) (tanh) of the float32 sums
 };
 
+struct SkSecond {                // the second product of a sum: X [M, K], the tiled copy of W [N, K]
+    const bf16_t* X;
+    const bf16_t* W;
+    int K;
+};
+struct SkNone {};
+
 // The value of the lane 8 further within 16.
 __device__ __forceinline__ uint4 turn8(uint4 v) {
     auto t = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x128, 0xf, 0xf, true); };   // row_ror:8
@@ -85,11 +94,19 @@ __device__ __forceinline__ uint4 turn8(uint4 v) {
 // columns 0 .. 7 of the sums take the steps one after the other, in whole tiles' order and with whole tiles' waves: the
 // same bits.  (The other three quarters of the sums are never read.)
 // ACT: the results go through res.act.  (A variant of its own: the test alone cost every product 0.15 us.)
-template <int MT, int NTB, int SK_U, int MAXW, int MODE, bool TILED, bool ONE_SHOT = false, bool HALF = false, bool ACT = false>
+// TWO (TILED, MT == NTB == 1): the sum of two products with the same rows of results, the second one's pieces of K
+// after the first one's.  (SkSecond is read nowhere else.)
+// EVEN (TILED, MT == 1): K is whole pieces (a multiple of 32 SK_U), so that every load is unconditional and its base the same
+// in all lanes.  Behind a test of its own each load had a branch and a 64-bit address a lane to be made, and the compiler
+// waited where it could not count.  us, 8 / 16 rows, matrices cold: 4096 x 11008 19.2 / 23.3 -> 18.6 / 22.3, 8192 x 2048
+// 8.9 / 10.7 -> 8.4 / 10.0, 6144 x 2048 8.2 / 10.4 -> 7.9 / 9.6, 32000 x 4096 43.8 / 46.9 -> 42.3 / 45.5; gate|up 2 x 5376 x
+// 2048 11.2 / 13.5 -> 10.8 / 13.0; the sum of two products (TWO), which had no other way, 15.9 / 26.0 -> 12.0 / 18.6.
+template <int MT, int NTB, int SK_U, int MAXW, int MODE, bool TILED, bool ONE_SHOT = false, bool HALF = false, bool ACT = false,
+          bool EVEN = false, bool TWO = false>
 __global__ void __launch_bounds__(64 * MAXW)
 gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                    void* __restrict__ Y, int y_dt, int M, int N, int K, SkRope rope,
-                   SkResidual res) {
+                   SkResidual res, std::conditional_t<TWO, SkSecond, SkNone> two) {
     constexpr bool DUAL = MODE == SK_GATE_UP;
     // a wave's piece of LDS: first the staging of its W lines (NTB * SK_U KB, not TILED), then
     // its sums
@@ -247,18 +264,49 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
     const int w_row = lane >> 3, w_chunk = lane & 7;
     // TILED: this lane's 8 values of k-step 0 of the block's first tile; a last block may have
     // fewer than NTB tiles (SK_GATE_UP with NTB > 1)
-    const bf16_t* wtile = W + (size_t)(HALF ? blockIdx.x / 2 : blockIdx.x * NTB) * ((K + 31) / 32) * 512 +
-                          ((HALF ? (blockIdx.x & 1) * 8 + (r & 7) : r) * 4 + q) * 8;
+    const int tile_at = ((HALF ? (blockIdx.x & 1) * 8 + (r & 7) : r) * 4 + q) * 8;
+    const bf16_t* wtile = W + (size_t)(HALF ? blockIdx.x / 2 : blockIdx.x * NTB) * ((K + 31) / 32) * 512 + tile_at;
     bool tile_ok[NTB];
 #pragma unroll
     for (int nt = 0; nt < NTB; ++nt) tile_ok[nt] = DUAL ? n_base + 8 * nt < N : tile_row[nt] < N || MODE != SK_PLAIN;
 
-    const int ksteps = (K + 31) / 32;
+    const int ksteps1 = (K + 31) / 32;
+    int ksteps = ksteps1, lane_w = 0, lane_x1 = 0, lane_x2 = 0;
+    const bf16_t *tile1 = W, *tile2 = nullptr, *second_x = nullptr;
+    if constexpr (EVEN) {
+        const int tile = HALF ? blockIdx.x / 2 : blockIdx.x * NTB, odd = HALF ? r >> 3 : 0, row = min(HALF ? r & 7 : r, M - 1);
+        tile1 = W + (size_t)tile * ksteps1 * 512;
+        lane_w = tile_at + odd * 512;
+        lane_x1 = row * K + odd * 32 + q * 8;
+        if constexpr (TWO) {
+            ksteps += two.K / 32;
+            tile2 = two.W + (size_t)tile * (two.K / 32) * 512;
+            second_x = two.X;
+            lane_x2 = row * two.K + odd * 32 + q * 8;
+        }
+    }
     const int stride = waves * SK_U, turn = HALF ? 2 * stride : stride;      // k-steps from a wave's piece to the next
     uint4 a[NTB][SK_U], b[MT][SK_U];
     // HALF: the k-step of this lane's u-th load, of two pieces of the wave
     auto step_of = [&](int s0, int u) { return s0 + (2 * u >= SK_U ? stride : 0) + (2 * u) % SK_U + (r >> 3); };
     auto load = [&](int s0, uint4 (&aa)[NTB][SK_U], uint4 (&bb)[MT][SK_U]) {
+        if constexpr (EVEN) {
+            static_assert(!EVEN || (TILED && MT == 1), "");
+#pragma unroll
+            for (int u = 0; u < SK_U; ++u) {
+                const bool later = HALF && 2 * u >= SK_U;                         // (a wave's second piece of two)
+                const bool there = !later || s0 + stride < ksteps;
+                const int piece = later && there ? s0 + stride : s0;
+                const bool second = TWO && piece >= ksteps1;
+                const int st = piece - (second ? ksteps1 : 0) + (HALF ? 2 * u % SK_U : u);
+#pragma unroll
+                for (int nt = 0; nt < NTB; ++nt)            // (a tile that is not there: the first one, never stored)
+                    aa[nt][u] = ld16_stream((second ? tile2 : tile1) + ((size_t)(tile_ok[nt] ? nt * ksteps1 : 0) + st) * 512 + lane_w);
+                bb[0][u] = *(const uint4*)((TWO && second ? second_x : X) + st * 32 + (second ? lane_x2 : lane_x1));
+                if (later && !there) aa[0][u] = bb[0][u] = make_uint4(0, 0, 0, 0);
+            }
+            return;
+        }
 #pragma unroll
         for (int u = 0; u < SK_U; ++u) {
             // K is a multiple of 8: a lane's 8 values are all in or all out
@@ -497,10 +545,10 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
 static const SkResidual SK_NO_RESIDUAL = {0, nullptr, ILLM_BF16, nullptr, nullptr, nullptr, 0, 0.f, 0.f, 0.f, 0, {}, 0};
 
 template <int MT, int NTB, int U, int MODE = SK_PLAIN, bool TILED = false, bool ONE_SHOT = false, bool HALF = false,
-          bool ACT = false>
+          bool ACT = false, bool TWO = false>
 static int launch_skinny(const void* X, const void* W, void* Y, int y_dt, int M, int N, int K,
                          int waves, hipStream_t st, SkRope rope = SkRope(),
-                         SkResidual res = SK_NO_RESIDUAL) {
+                         SkResidual res = SK_NO_RESIDUAL, std::conditional_t<TWO, SkSecond, SkNone> two = {}) {
     constexpr bool DUAL = MODE == SK_GATE_UP;
     // registers a lane needs: operands of two pieces in flight (one if ONE_SHOT) and the accumulators
     constexpr int REGS = (ONE_SHOT ? 1 : 2) * (NTB + MT) * U * 4 + NTB * 8 + NTB * MT * 4 + 40;
@@ -509,8 +557,18 @@ static int launch_skinny(const void* X, const void* W, void* Y, int y_dt, int M,
     const int rows_per_block = DUAL ? 8 * NTB : HALF ? 8 : 16 * NTB;
     const int blocks = (N + rows_per_block - 1) / rows_per_block;
     const size_t smem = (size_t)waves * NTB * ((!TILED && U > MT) ? U : MT) * 1024 + 64;
-    hipLaunchKernelGGL((gemm_skinny_kernel<MT, NTB, U, MAXW, MODE, TILED, ONE_SHOT, HALF, ACT>), dim3(blocks), dim3(64 * waves),
-                       smem, st, (const bf16_t*)X, (const bf16_t*)W, Y, y_dt, M, N, K, rope, res);
+    // (EVEN pays where a wave goes through its pieces one by one: of half tiles a wave's last round would ask for pieces that
+    // are not there, 8 rows of 2048 x 2048 5.05 -> 6.02 us, and one piece a wave has nothing to count, 4096 x 4096 8.7 -> 9.1)
+    if constexpr (TWO || (TILED && MT == 1 && !HALF && !ONE_SHOT)) {
+        if (TWO || K % (32 * U) == 0) {
+            hipLaunchKernelGGL((gemm_skinny_kernel<MT, NTB, U, MAXW, MODE, TILED, ONE_SHOT, HALF, ACT, true, TWO>), dim3(blocks),
+                               dim3(64 * waves), smem, st, (const bf16_t*)X, (const bf16_t*)W, Y, y_dt, M, N, K, rope, res, two);
+            return illm_launch_status();
+        }
+    }
+    if constexpr (!TWO)
+        hipLaunchKernelGGL((gemm_skinny_kernel<MT, NTB, U, MAXW, MODE, TILED, ONE_SHOT, HALF, ACT>), dim3(blocks),
+                           dim3(64 * waves), smem, st, (const bf16_t*)X, (const bf16_t*)W, Y, y_dt, M, N, K, rope, res, two);
     return illm_launch_status();
 }
 
@@ -619,6 +677,26 @@ extern "C" int illm_gemm_skinny_act(const void* X, const void* W, const void* Wt
     res.ssq = ssq; res.parts = parts; res.eps = eps; res.act = act;
     return act ? skinny_plain<true>(X, W, Wt, Y, y_dt, M, N, K, res, 0, stream)
                : skinny_plain<false>(X, W, Wt, Y, y_dt, M, N, K, res, 0, stream);
+}
+
+// Y[M, N] (float32) = X . W^T + X2 . W2^T from the tiled copies Wt [N, K] and W2t [N, K2]: what two parts that read the same
+// rows leave for the residual stream, in one kernel with one sum and no rounding between.  M <= 16, K and K2 multiples of 128.
+// Half a tile a block by the rule above.  Matrices cold, us, both products / this at 1, 8 and 16 rows: 2048 x 2048 and x 8192
+// 12.1 / 10.0, 14.2 / 12.0, 22.4 / 18.6, 4096 x 4096 and x 16384 29.2 / 26.4, 32.5 / 29.6, 40.9 / 36.8.
+extern "C" int illm_gemm_skinny_sum(const void* X, const void* Wt, int K, const void* X2, const void* W2t, int K2, float* Y,
+                                    int M, int N, void* stream) {
+    if (M <= 0 || M > 16 || N <= 0 || K <= 0 || K % 128 || K2 <= 0 || K2 % 128 || K > 1 << 24 || K2 > 1 << 24 || !X || !Wt || !X2 ||
+        !W2t || !Y)
+        return ILLM_ERR_ARG;
+    const int blocks = (N + 15) / 16;
+    int waves = (SK_WAVES_ON_CHIP_TILED + blocks / 2) / blocks;
+    waves = clamp_waves(waves < 1 ? 1 : waves, 1, 1, 4, K + K2);
+    const SkSecond two = {(const bf16_t*)X2, (const bf16_t*)W2t, K2};
+    if (M <= 8 && (SK_HALF >= 0 ? SK_HALF == 1 : blocks <= 128 && K + K2 >= 1024))
+        return launch_skinny<1, 1, 4, SK_PLAIN, true, false, true, false, true>(X, Wt, Y, ILLM_F32, M, N, K, waves, (hipStream_t)stream,
+                                                                                SkRope(), SK_NO_RESIDUAL, two);
+    return launch_skinny<1, 1, 4, SK_PLAIN, true, false, false, false, true>(X, Wt, Y, ILLM_F32, M, N, K, waves, (hipStream_t)stream,
+                                                                             SkRope(), SK_NO_RESIDUAL, two);
 }
 
 // The product whose parts of W read rows of X of their own: X [planes][M][K], W's rows ends[p - 1] .. ends[p] - 1

@@ -1132,6 +1132,37 @@ def linear_act(x, w, act: str) -> torch.Tensor:
     return y
 
 
+class Product:
+    """x . w^T, not yet taken: a part's last product, left to a block that takes two of them in one kernel
+    (`linear_sum`); anything else asks for `tensor()`."""
+
+    def __init__(self, x: torch.Tensor, w):
+        self.x, self.w = x, w
+
+    def tensor(self) -> torch.Tensor:
+        return linear(self.x, self.w)
+
+
+def linear_sum_fits(a: Product, b: Product) -> bool:
+    """Whether `linear_sum` takes these: up to 16 bfloat16 rows and matrices with plain decode copies."""
+    return (all(isinstance(p.x, torch.Tensor) and isinstance(p.w, Weight) and p.w.tiled is not None and p.w.mode == "plain"
+                and p.x.dtype == torch.bfloat16 and p.x.dim() == 2 and p.x.shape[1] == p.w.shape[1] <= 1 << 24
+                and p.x.shape[1] % 128 == 0
+                and 1 <= p.x.shape[0] <= SKINNY_BEST_ROWS for p in (a, b))
+            and a.x.shape[0] == b.x.shape[0] and a.w.shape[0] == b.w.shape[0])
+
+
+def linear_sum(a: Product, b: Product) -> torch.Tensor:
+    """float32 [M, N]: the sum of the two products."""
+    _need(linear_sum_fits(a, b), "linear_sum: operands not taken")
+    _gpu(a.x, b.x, a.w.tiled, b.w.tiled)
+    M, N = a.x.shape[0], a.w.shape[0]
+    y = torch.empty((M, N), dtype=torch.float32, device=a.x.device)
+    _check(_lib().illm_gemm_skinny_sum(_p(a.x), _p(a.w.tiled), a.x.shape[1], _p(b.x), _p(b.w.tiled), b.x.shape[1], _p(y), M, N,
+                                       _stream()), "linear_sum")
+    return y
+
+
 QKV_ROPE_WAVES = 0       # waves per block of the fused kernel; 0: the kernel's own choice
 GATE_UP_WAVES = 0        # the same for the fused gate|up product
 PLAIN_WAVES = 0          # and for the plain few-rows product

@@ -277,6 +277,7 @@ class GatedAttention(Mixer):
     """
 
     graph_safe_prompts = True
+    may_leave_product = True
     takes_continuations = True
     takes_projected = True            # (its own products at column 0)
 
@@ -480,4 +481,4 @@ class GatedAttention(Mixer):
                 ops.attn_pooled_decode(rows, kc, vc, kp, vp, group.table, group.page_size, ctx.seq_slot,
                                        ctx.seq_len, nh, nkv, dk, dv, self.scale, None, window, self.pool,
                                        out=o, lse=lse)
-        return ops.linear(o, self.w_o)
+        return self.leave(o, self.w_o)

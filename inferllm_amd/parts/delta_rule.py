@@ -34,6 +34,7 @@ class GatedDeltaRule(Mixer):
     """
 
     graph_safe_prompts = True
+    may_leave_product = True
     takes_continuations = True
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, key_dim: int,
@@ -129,4 +130,4 @@ class GatedDeltaRule(Mixer):
                            ctx.max_rows if ctx.prefill else 1)
         y = ops.delta_finish(o, self.norm_w, P2 if self.rg else P, self.z_off, self.gate, self.eps,
                              ctx.act_dtype)
-        return ops.linear(y, self.w_o)
+        return self.leave(y, self.w_o)

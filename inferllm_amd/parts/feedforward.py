@@ -83,6 +83,7 @@ class DenseActivation(FeedForward):
     (p, q): softplus(p) z^2 + z / 2 for z > 0, (1/2 + softplus(q)) (e^z - 1 - z) + z / 2 else."""
 
     graph_safe_prompts = True
+    may_leave_product = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, activation: str = "relu_squared",
                  tensors=None):
@@ -112,7 +113,7 @@ class DenseActivation(FeedForward):
         act = _ACTIVATIONS[self.activation]
         z = (ops.linear_act(h, self.w_up, act) if self.act is None
              else getattr(ops, act)(ops.linear(h, self.w_up), self.act))
-        return ops.linear(z, self.w_down)
+        return self.leave(z, self.w_down)
 
 
 @register_part("feed_forward", "clamped_gated")
@@ -122,6 +123,7 @@ class ClampedGated(FeedForward):
     fused product, which in steps of few bfloat16 rows also applies the activation."""
 
     graph_safe_prompts = True
+    may_leave_product = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, limit: float, tensors=None):
         super().__init__(tensors)
@@ -143,7 +145,7 @@ class ClampedGated(FeedForward):
         return (("gate_up", self.w_gate_up, {}), ("plain", self.w_down, {}))
 
     def forward(self, h, ctx: StepContext):
-        return ops.linear(ops.gate_up_act(h, self.w_gate_up, self.limit), self.w_down)
+        return self.leave(ops.gate_up_act(h, self.w_gate_up, self.limit), self.w_down)
 
 
 @register_part("feed_forward", "routed_experts")

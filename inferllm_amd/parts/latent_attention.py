@@ -33,6 +33,7 @@ class LatentAttention(Mixer):
     """
 
     graph_safe_prompts = True
+    may_leave_product = True
     # rows that go on from earlier tokens are each treated as a single token over the cache, which
     # holds the step's own rows by then (a window's ring is kept from wrapping by the step function)
     takes_continuations = True
@@ -150,4 +151,4 @@ class LatentAttention(Mixer):
             o = ops.latent_attn_decode(qa, y, self.w_uv, self.gate_off, cache, group.table,
                                        group.page_size, group.ring, slots, lens, more, H, dr, R, dv,
                                        self.scale, window, nsplit, cache_t)
-        return ops.linear(o, self.w_o)
+        return self.leave(o, self.w_o)

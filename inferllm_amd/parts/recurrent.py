@@ -38,6 +38,7 @@ class StateSpaceDuality(Mixer):
     """
 
     graph_safe_prompts = True
+    may_leave_product = True
     takes_continuations = True
 
     def __init__(self, hidden_size: int, num_heads: int, groups: int, state_size: int, value_dim: int,
@@ -96,7 +97,7 @@ class StateSpaceDuality(Mixer):
         o = ops.delta_scan(qn, kn, vv, step, dec, S, ctx.cu_seqlens, ctx.seq_slot, ctx.n_seqs,
                            ctx.max_rows if ctx.prefill else 1, correct=False)
         y = ops.ssm_finish(o, vv, self.D, U, 0, self.norm_w, self.norm_groups, self.eps, ctx.act_dtype)
-        return ops.linear(y, self.w_o)
+        return self.leave(y, self.w_o)
 
 
 @register_part("mixer", "matrix_memory")
@@ -118,6 +119,7 @@ class MatrixMemory(Mixer):
     """
 
     graph_safe_prompts = True
+    may_leave_product = True
     takes_continuations = True
 
     def __init__(self, hidden_size: int, num_heads: int, key_dim: int, value_dim: int, gate_cap: float,
@@ -167,7 +169,7 @@ class MatrixMemory(Mixer):
         o = ops.delta_scan(qn, kn, vv, weight, dec, state["S"], ctx.cu_seqlens, ctx.seq_slot, ctx.n_seqs,
                            ctx.max_rows if ctx.prefill else 1, correct=False)
         y = ops.memory_finish(o, em, self.norm_w, U, self.z_off, self.eps, ctx.act_dtype)
-        return ops.linear(y, self.w_o)
+        return self.leave(y, self.w_o)
 
 
 @register_part("mixer", "gated_linear_attention")

@@ -1996,3 +1996,30 @@ def test_capped_decode_steps_of_16_keys(nh, nkv, dk, dv):
             assert float((got[0].double().cpu() - want).abs().max()) <= 2 ** -8 * max(1.0, float(want.abs().max())), nsplit
     finally:
         o._lib().illm_set_attn_cap_heads(0)
+
+
+@pytest.mark.parametrize("N, K, K2", [(48, 128, 128), (72, 256, 128), (2048, 128, 896), (2048, 2048, 8192), (4128, 384, 256)])
+def test_sum_of_two_products_of_few_rows(N, K, K2):
+    """x . w^T + x2 . w2^T in one kernel: one piece of 128 k of either product, odd numbers of them, more
+    pieces than waves and fewer, rows of W beyond the last tile; a row has the same bits alone, among 8 rows (half a tile a
+    block) and among 16; an infinity in one row's second operand stays in that row."""
+    o = ops()
+    x, x2 = (rnd(16, k, dtype=torch.bfloat16, seed=i).to(DEV) for i, k in enumerate((K, K2)))
+    w, w2 = ((rnd(N, k, seed=i + 2) * 0.1).to(torch.bfloat16).to(DEV) for i, k in enumerate((K, K2)))
+    a, b = (o.decode_weight(t, "plain", True) for t in (w, w2))
+    want = x.double() @ w.double().t() + x2.double() @ w2.double().t()
+    got = {}
+    for M in (1, 7, 8, 9, 16):
+        pair = o.Product(x[:M], a), o.Product(x2[:M], b)
+        assert o.linear_sum_fits(*pair)
+        got[M] = o.linear_sum(*pair)
+        # a float32 sum of K + K2 products
+        assert float((got[M].double() - want[:M]).abs().max()) <= (K + K2) * 2.0 ** -24 * float((x.abs().double() @ w.abs().double().t()
+                                                                              + x2.abs().double() @ w2.abs().double().t()).max())
+        assert torch.equal(got[M][:1], got[1])
+    assert torch.equal(got[16][:8], got[8])
+    x2[3, 5] = float("inf")
+    bad = o.linear_sum(o.Product(x[:8], a), o.Product(x2[:8], b))
+    rows = [0, 1, 2, 4, 5, 6, 7]
+    assert torch.equal(bad[rows], got[8][rows]) and not bool(torch.isfinite(bad[3]).any())
+    assert not o.linear_sum_fits(o.Product(x, w), o.Product(x2, b)) and not o.linear_sum_fits(o.Product(x[:4], a), o.Product(x2, b))
