@@ -99,7 +99,10 @@ class _DecodeGraph:
             max_len=self.max_len, cache=runner.cache, ragged=self.ragged)
 
 
-PROMPT_GRAPH_ROWS = (16, 32, 64, 96, 128, 192, 256)   # rows of the graphs that short prompt steps are replayed from
+# Rows of the graphs that short prompt steps are replayed from: from 64 on whole tiles of 16, from 128 on of 32 rows, since
+# every product's time grows with them (us a prompt, LLaMA-2-7B, in a bucket of 96 / 80 rows 4,627 / 4,464, 128 / 112
+# 5,157 / 4,960, 192 / 160 6,152 / 5,706).
+PROMPT_GRAPH_ROWS = (16, 32, 64, 80, 96, 112, 128, 160, 192, 224, 256)
 PROMPT_GRAPH_SEQS = (2, 4, 8, 16, 32)                 # and their sequences (one of them takes the padding rows)
 
 
