@@ -232,6 +232,9 @@ int illm_gemm_skinny_bf16(const void* X, const void* W, const void* Wt, void* Y,
 // The same of at most 16 rows, an activation on the float32 sums: act 1 relu(y)^2, 2 gelu(y) by tanh, 0 none.
 int illm_gemm_skinny_act(const void* X, const void* W, const void* Wt, void* Y, int y_dt, int M, int N, int K,
                          const float* ssq, int parts, float eps, int act, void* stream);
+// Many rows (csrc/gemm_turns.hip), bfloat16 on 16-byte addresses, K % 128 == 0, F % 8 == 0: Y [M, F] of W [2 F, K] = [gate | up]
+// (limit, alpha as for illm_gemm_skinny_gateup_act).
+int illm_gemm_turns_gate_up(const void* X, const void* W, void* Y, int M, int F, int K, float limit, float alpha, void* stream);
 // The sum of two products of at most 16 rows, float32 Y = X . W^T + X2 . W2^T, from the tiled copies (K, K2 % 128 == 0).
 int illm_gemm_skinny_sum(const void* X, const void* Wt, int K, const void* X2, const void* W2t, int K2, float* Y, int M,
                          int N, void* stream);

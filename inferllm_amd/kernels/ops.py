@@ -1274,11 +1274,28 @@ def gate_up_silu(x, w_gate_up) -> torch.Tensor:
     return gate_up_act(x, w_gate_up, 0.0)
 
 
+# From so many rows, and outputs of both products, gate and up with their activation are one kernel.  us, product and
+# activation -> one kernel: 2 x 4096 x 1024 of 256 / 500 rows 19 / 22 -> 19 / 19, 2 x 5376 x 2048 of 300 / 500 29 / 33 -> 30 / 33,
+# 2 x 2816 x 2048 of 500 / 1,000 29 / 36 -> 31 / 31, 2 x 1408 x 2048 of 1,000 / 2,048 28 / 33 -> 30 / 32, 2 x 1024 x 1024 of
+# 1,000 / 2,048 15 / 20 -> 18 / 18; 2 x 11008 x 4096 of 256 rows 69 -> 65, of 1,000 172 -> 178 (a second round of 88 tiles).
+TURNS_FROM, TURNS_OUTPUTS = 256, 1 << 22
+
+
+def gate_up_turns_fits(x, w) -> bool:
+    """Whether csrc/gemm_turns.hip takes the gate and up products of these rows and is the faster way."""
+    w = plain_weight(w)
+    return (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2
+            and x.is_cuda and w.is_cuda and x.shape[0] >= TURNS_FROM and x.shape[0] * w.shape[0] >= TURNS_OUTPUTS
+            and x.shape[1] == w.shape[1] and x.shape[1] % 128 == 0 and x.shape[1] <= 1 << 22 and w.shape[0] % 16 == 0
+            and w.shape[0] <= 1 << 30 and x.is_contiguous() and w.is_contiguous() and _on16(x, w))
+
+
 def gate_up_act(x, w_gate_up, limit: float = 0.0) -> torch.Tensor:
     """The gate and up products of w_gate_up = [Wg | Wu] ([2F, K]) and their activation: with `limit`
     0 silu(gate) * up, with `limit` > 0 the clamped gate g sigmoid(1.702 g) (u + 1), g = min(gate,
     limit), u = clamp(up, -limit, limit).  Few bfloat16 rows: one fused MFMA kernel (the activation
-    acts on the float32 sums).  Otherwise the product and `silu_mul` / `clamped_swish_mul`."""
+    acts on the float32 sums), and likewise many of them; otherwise the product and `silu_mul` /
+    `clamped_swish_mul`."""
     limit = float(limit)
     if isinstance(x, NormedRows) and (w_gate_up.dtype != torch.bfloat16 or w_gate_up.shape[0] % 2):
         x = x.rows()
@@ -1308,6 +1325,13 @@ def gate_up_act(x, w_gate_up, limit: float = 0.0) -> torch.Tensor:
         return y
     if isinstance(x, NormedRows):
         x = x.rows()
+    if gate_up_turns_fits(x, w_gate_up):
+        wp = plain_weight(w_gate_up)
+        _gpu(x, wp)
+        y = torch.empty((M, F2 // 2), dtype=x.dtype, device=x.device)
+        _check(_lib().illm_gemm_turns_gate_up(_p(x), _p(wp), _p(y), M, F2 // 2, K, ctypes.c_float(limit),
+                                              ctypes.c_float(SWISH_ALPHA), _stream()), "gate_up_act (many rows)")
+        return y
     both = linear(x, plain_weight(w_gate_up))
     return clamped_swish_mul(both, limit) if limit > 0 else silu_mul(both)
 

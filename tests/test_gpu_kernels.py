@@ -2023,3 +2023,39 @@ def test_sum_of_two_products_of_few_rows(N, K, K2):
     rows = [0, 1, 2, 4, 5, 6, 7]
     assert torch.equal(bad[rows], got[8][rows]) and not bool(torch.isfinite(bad[3]).any())
     assert not o.linear_sum_fits(o.Product(x, w), o.Product(x2, b)) and not o.linear_sum_fits(o.Product(x[:4], a), o.Product(x2, b))
+
+
+@pytest.mark.parametrize("M, F, K", [(1, 8, 128), (129, 136, 256), (257, 264, 384), (300, 2184, 128), (700, 40, 1024), (2100, 2056, 256)])
+def test_gate_up_of_many_rows_in_turns(M, F, K):
+    """Gate and up with their activation over tiles in turns: less than a tile and remainders along both sides, one stage
+    pair of K and more, more tiles than blocks (so that loads run on into the next tile), infinities that stay in their rows
+    and columns; the same rows have the same bits in every shape of tiles (other numbers of rows)."""
+    o, lib = ops(), ops()._lib()
+    x = rnd(M, K, dtype=torch.bfloat16, seed=1).to(DEV)
+    w = (rnd(2 * F, K, seed=2) * K ** -0.5).to(torch.bfloat16).to(DEV)
+
+    def run(rows, limit):
+        y = torch.full((rows + 1, F), 7.0, dtype=torch.bfloat16, device=DEV)
+        assert lib.illm_gemm_turns_gate_up(o._p(x), o._p(w), o._p(y), rows, F, K, limit, 1.702, None) == 0
+        assert bool((y[rows] == 7.0).all())
+        return y[:rows]
+    z = x.double() @ w.double().t()
+    for limit in (0.0, 1.5):
+        y = run(M, limit)
+        g, u = z[:, :F], z[:, F:]
+        if limit:
+            g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+            want = g * torch.sigmoid(1.702 * g) * (u + 1)
+        else:
+            want = g * torch.sigmoid(g) * u
+        # the result's rounding (half of the last of 8 bits: 2^-8 of a number that begins a power of two), and float32 sums of
+        # K products (of at most 4 x 4 K^-1/2 each) through a slope of up to 1.1
+        scale = want.abs() * 2.0 ** -8 + (g.abs() + u.abs() + 2) * K ** 0.5 * 16 * 2.0 ** -24
+        assert bool(((y.double() - want).abs() <= 1.01 * scale).all())
+        for rows in (1, M // 2 + 1, M):
+            assert torch.equal(run(rows, limit), y[:rows])
+    y, rows = run(M, 0.0), [i for i in range(M) if i != M // 3]
+    x[M // 3, 5] = float("inf")
+    bad = run(M, 0.0)
+    assert torch.equal(bad[rows], y[rows]) and bool(torch.isfinite(bad[rows].float()).all())
+    assert lib.illm_gemm_turns_gate_up(o._p(x), o._p(w), o._p(y), M, F, K + 64, 0.0, 1.0, None) != 0
