@@ -138,6 +138,7 @@ class KVGroup:
             self.tensors[t.name] = torch.zeros(shape, dtype=t.dtype or dtype, device=device)
         self.table_host = torch.full((n_slots + 1, self.pages_per_seq), self.spare_page,
                                      dtype=torch.int32)
+        self._table = self.table_host.numpy()    # the same memory: a row's part costs one call, not one a page
         self.table = self.table_host.to(device)
         self.held: Dict[int, List[int]] = {}     # slot -> pages in logical order
         self._dirty = set()
@@ -177,10 +178,10 @@ class KVGroup:
         if need - len(pages) > self.pool.n_free():
             raise CacheFull(f"cache full: {need - len(pages)} more pages of {self.page_size} tokens "
                             f"needed, {self.pool.n_free()} of {self.n_pages} free")
-        while len(pages) < need:
-            p = self.pool.alloc()
-            self.table_host[slot, len(pages)] = p
-            pages.append(p)
+        if need > len(pages):
+            got = self.pool.alloc_many(need - len(pages))
+            self._table[slot, len(pages):need] = got
+            pages.extend(got)
             self._dirty.add(slot)
 
     def shrink(self, slot: int, length: int, poison: bool = False) -> None:
@@ -195,7 +196,7 @@ class KVGroup:
             self._poison(gone)
         for p in gone:
             self.pool.free(p)
-        self.table_host[slot, need:need + len(gone)] = self.spare_page
+        self._table[slot, need:need + len(gone)] = self.spare_page
         self._dirty.add(slot)
 
     def release(self, slot: int, poison: bool = False) -> None:
@@ -204,7 +205,7 @@ class KVGroup:
             self._poison(pages)
         for p in pages:
             self.pool.free(p)
-        self.table_host[slot].fill_(self.spare_page)
+        self._table[slot] = self.spare_page
         self._dirty.add(slot)
 
     def upload(self) -> None:

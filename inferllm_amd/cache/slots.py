@@ -46,6 +46,15 @@ class FreeList:
         self._held.add(i)
         return i
 
+    def alloc_many(self, n: int) -> List[int]:
+        """What n calls of `alloc` give, or CacheFull and nothing."""
+        if n > len(self._free):
+            raise CacheFull(f"{n} {self.what}s wanted, {len(self._free)} of {self.n} are free")
+        got = self._free[-n:][::-1] if n > 0 else []
+        del self._free[len(self._free) - len(got):]
+        self._held.update(got)
+        return got
+
     def free(self, i: int) -> None:
         if i not in self._held:
             raise CacheError(f"{self.what} {i} is not held (freed twice, or never given out)")

@@ -71,6 +71,23 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+_streams: dict = {}
+
+
+def record(event) -> None:
+    """`event.record()` on the current stream (asking torch for the stream's object costs more than the record)."""
+    if _raw_stream is None:
+        return event.record()
+    device = torch.cuda.current_device()
+    key = (device, _raw_stream(device))
+    stream = _streams.get(key)
+    if stream is None:
+        if len(_streams) >= 64:
+            _streams.clear()
+        stream = _streams[key] = torch.cuda.current_stream()
+    event.record(stream)
+
+
 def _on16(*tensors: Optional[torch.Tensor]) -> bool:
     """Whether the tensors' first elements lie on 16-byte addresses (views may begin anywhere)."""
     return all(t is None or t.data_ptr() % 16 == 0 for t in tensors)
@@ -144,12 +161,13 @@ def embed_norm(tokens: torch.Tensor, table: torch.Tensor, weight: torch.Tensor, 
 def zero_slot(tensors, slot: int) -> None:
     """Row `slot` of every tensor to zeros (contiguous [slots, ...], any types, one device), in one launch for 16 of them
     on that device."""
-    rows = [t[slot] for t in tensors]
-    _gpu(*rows)
-    n = len(rows)
-    at = (ctypes.c_uint64 * n)(*[r.data_ptr() for r in rows])
-    size = (ctypes.c_uint64 * n)(*[r.numel() * r.element_size() for r in rows])
-    with torch.cuda.device(rows[0].device):
+    _gpu(*tensors)
+    n = len(tensors)
+    _need(all(t.dim() > 0 and 0 <= slot < t.shape[0] for t in tensors), f"zero_slot: row {slot} of every tensor")
+    sizes = [t.numel() // t.shape[0] * t.element_size() for t in tensors]       # (views of rows cost 2 us each)
+    at = (ctypes.c_uint64 * n)(*[t.data_ptr() + slot * b for t, b in zip(tensors, sizes)])
+    size = (ctypes.c_uint64 * n)(*sizes)
+    with torch.cuda.device(tensors[0].device):
         _check(_lib().illm_zero_pieces(at, size, n, _stream()), "zero_slot")
 
 
@@ -3066,8 +3084,11 @@ _sample_long_row_bytes = 0        # ILLM_SAMPLE_LONG_ROW_BYTES of csrc/api.h, as
 def sample(logits: torch.Tensor, temperature: float, top_k: int, top_p: float,
            repeat_penalty: float, last_tokens: Optional[torch.Tensor], seeds: torch.Tensor,
            counters: torch.Tensor) -> torch.Tensor:
-    """One draw per row; see csrc/sampling.hip.  seeds: int64 [B] (bit pattern used), counters int32 [B]."""
-    _gpu(logits, last_tokens, seeds, counters)
+    """One draw per row; see csrc/sampling.hip.  seeds: int64 [B] (bit pattern used), counters int32 [B], both on the
+    device or in pinned memory, which the kernel reads (and the caller leaves as it is until it has run)."""
+    _gpu(logits, last_tokens)
+    for t in (seeds, counters):
+        _need(t.is_contiguous() and (t.is_cuda or t.is_pinned()), "sample: seeds and counters on the device or in pinned memory")
     _need(logits.dtype == torch.float32 and logits.dim() == 2, "sample: float32 [B, V]")
     B, V = logits.shape
     _need(seeds.dtype == torch.int64 and seeds.numel() >= B, "sample: seeds int64 [B]")

@@ -45,10 +45,13 @@ class Sampler:
         # still wait for their copy when the next draw's are written
         self._stages: List[Optional[torch.Tensor]] = [None] * 4
         self._back: List[torch.Tensor] = []            # pinned buffers the drawn tokens come back in
+        self._copied: List[object] = []                # and the events behind their copies
         self._turn = 0
 
     def _upload(self, seeds, counters, windows):
-        """One pinned buffer, one copy: (seeds int64 [B], counters int32 [B], windows int32 [B, n] or None)."""
+        """One pinned buffer: (seeds int64 [B], counters int32 [B], windows int32 [B, n] or None).  Without windows the
+        kernel reads the few numbers where they are (a copy takes 10 us of the host and 3 of the device); with them one
+        copy brings everything over."""
         B = len(seeds)
         n = len(windows[0]) if windows else 0
         words = B * (3 + n)
@@ -63,7 +66,7 @@ class Sampler:
         flat[2 * B:3 * B] = counters
         if n:
             flat[3 * B:].reshape(B, n)[:] = windows
-        dev = host.to(self.device, non_blocking=True)
+        dev = host.to(self.device, non_blocking=True) if n else host
         return (dev[:2 * B].view(torch.int64), dev[2 * B:3 * B],
                 dev[3 * B:].view(B, n) if n else None)
 
@@ -105,12 +108,13 @@ class Sampler:
             return Draw(dev, dev, None)
         while len(self._back) < 4:
             self._back.append(torch.empty(1024, dtype=torch.int32, pin_memory=True))
+            self._copied.append(torch.cuda.Event())
         if self._back[self._turn].numel() < B:
             self._back[self._turn] = torch.empty(B, dtype=torch.int32, pin_memory=True)
         host = self._back[self._turn][:B]
         host.copy_(dev, non_blocking=True)
-        copied = torch.cuda.Event()
-        copied.record()
+        copied = self._copied[self._turn]
+        ops.record(copied)
         return Draw(dev, host, copied)
 
     def __call__(self, logits: torch.Tensor, seeds: Sequence[int], counters: Sequence[int],

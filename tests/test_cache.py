@@ -29,6 +29,26 @@ def test_free_list_refuses_double_free_and_exhaustion():
     f.check()
 
 
+@pytest.mark.parametrize("scatter", [False, True])
+def test_many_at_once_are_those_one_by_one(scatter):
+    """`alloc_many` gives what as many calls of `alloc` give, all that there are among them, or nothing and CacheFull."""
+    one, many = FreeList(7, "page", scatter), FreeList(7, "page", scatter)
+    for f in (one, many):
+        f.alloc(), f.alloc()
+        f.free(next(iter(f.held())))
+    for n in (0, 1, 3, 2):
+        assert many.alloc_many(n) == [one.alloc() for _ in range(n)]
+        many.check()
+    assert many.n_free() == one.n_free() == 0
+    with pytest.raises(CacheFull):
+        many.alloc_many(1)
+    many.free(5)
+    with pytest.raises(CacheFull):
+        many.alloc_many(2)
+    assert many.alloc_many(1) == [5]
+    many.check()
+
+
 def test_slots_and_pages_are_conserved_under_random_use():
     m = manager()
     rnd = random.Random(0)
