@@ -543,66 +543,110 @@ extern "C" int illm_gemm_rows_f32_mfma(const float* X, const float* W, void* Y, 
 
 // ---------------------------------------------------------------- few rows, float32
 // The same product for M <= 16 rows of float32 X and float32 W (decoding on the 32-bit path),
-// bound by reading W once: a block of 4 waves takes R = 64 / MR rows of W (MR = M rounded up to
-// 8 or 16), the waves split K in interleaved pieces of 256, a lane multiplies 4 consecutive k
+// bound by reading W once: a block of 4 waves takes R rows of W for MR rows of X (M rounded up to
+// 1, 2, 4, 8 or 16), the waves split K in interleaved pieces of 256, a lane multiplies 4 consecutive k
 // of every W row with every X row (plain multiply-adds, float32), and the R * MR sums of a wave
-// are added over its lanes by a halving exchange that leaves sum number l in lane l.  The waves'
-// sums are added in wave order.  The order of a sum depends on K only, not on the row's place.
-template <int MR>
+// are added over its lanes by a halving exchange that leaves sum number l in lane l (modulo their number; what is left of
+// the lanes' bits is added plainly, in the same tree).  The waves' sums are added in wave order.  The order of a sum
+// depends on K only, not on the row's place nor on MR.
+// AHEAD: a wave's next piece is asked for before this one is multiplied (few blocks).  Whole pieces are asked for without a
+// test.  us, matrices cold, 8 rows of sums for up to 8 of X, one piece at a time -> now, 1 and 4 rows: 4096 x 4096 15.4 / 15.2 ->
+// 12.7 / 14.3, 12288 x 4096 35.2 / 36.0 -> 31.9 / 33.9, 22016 x 4096 58.3 / 59.5 -> 55.0 / 56.6 (6.4 TB/s), 4096 x 11008 34.2 /
+// 34.5 -> 30.2 / 32.1, 512 x 96 3.7 / 3.8 -> 2.4 / 3.0.  The same bits.
+template <int MR, int R, bool AHEAD>
 __global__ void __launch_bounds__(256)
 gemv_rows_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, void* __restrict__ Y,
                      int y_dt, int M, int N, int K) {
-    constexpr int R = 64 / MR;
-    __shared__ float part[4][64];
+    constexpr int S = R * MR;
+    static_assert(S <= 64 && (S & (S - 1)) == 0, "");
+    __shared__ float part[4][S];
     const int lane = threadIdx.x & 63, wave = wave_index();
     const int n0 = blockIdx.x * R;
-    const float* wrow[R];
+    const float *wrow[R], *xrow[MR];
 #pragma unroll
-    for (int r = 0; r < R; ++r) wrow[r] = W + (size_t)min(n0 + r, N - 1) * K;
+    for (int r = 0; r < R; ++r) wrow[r] = W + (size_t)min(n0 + r, N - 1) * K + wave * 256;
+#pragma unroll
+    for (int m = 0; m < MR; ++m) xrow[m] = X + (size_t)min(m, M - 1) * K + wave * 256;
     float acc[R][MR];
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int m = 0; m < MR; ++m) acc[r][m] = 0.f;
 
-    for (int k = (wave * 64 + lane) * 4; k < K; k += 4 * 256) {      // K is a multiple of 4
-        f32x4v_t w[R];                                   // (W is used once: loads that do not stay in the caches)
+    struct Piece { f32x4v_t w[R]; };                         // (W is used once: loads that do not stay in the caches)
+    auto load = [&](Piece& p, int k) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) w[r] = __builtin_nontemporal_load((const f32x4v_t*)(wrow[r] + k));
+        for (int r = 0; r < R; ++r) p.w[r] = __builtin_nontemporal_load((const f32x4v_t*)(wrow[r] + k + lane * 4));
+        if (AHEAD) __builtin_amdgcn_sched_barrier(0);        // (else they are put right before their use)
+    };
+    auto multiply = [&](const Piece& p, int k) __attribute__((always_inline)) {
 #pragma unroll
         for (int m = 0; m < MR; ++m) {
-            const float4 x = *(const float4*)(X + (size_t)min(m, M - 1) * K + k);
+            const float4 x = *(const float4*)(xrow[m] + k + lane * 4);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 float a = acc[r][m];
-                a = fmaf(w[r].x, x.x, a);
-                a = fmaf(w[r].y, x.y, a);
-                a = fmaf(w[r].z, x.z, a);
-                a = fmaf(w[r].w, x.w, a);
+                a = fmaf(p.w[r].x, x.x, a);
+                a = fmaf(p.w[r].y, x.y, a);
+                a = fmaf(p.w[r].z, x.z, a);
+                a = fmaf(p.w[r].w, x.w, a);
                 acc[r][m] = a;
             }
         }
+    };
+    const int whole = (K - wave * 256) / 256, n = (whole + 3) / 4;         // this wave's whole pieces: 0, 1024, ...
+    if (MR == 8) {                                         // (whole pieces by themselves: 61 -> 63 us for 22016 x 4096)
+        for (int k = 0; k + wave * 256 + lane * 4 < K; k += 1024) {
+            Piece p;
+            load(p, k);
+            multiply(p, k);
+        }
+    } else if (!AHEAD) {
+        for (int i = 0; i < n; ++i) {
+            Piece p;
+            load(p, i * 1024);
+            multiply(p, i * 1024);
+        }
+    } else if (whole > 0) {
+        Piece p0, p1;
+        load(p0, 0);
+        for (int i = 0; i < n; i += 2) {
+            load(p1, min(i + 1, n - 1) * 1024);
+            multiply(p0, i * 1024);
+            if (i + 1 >= n) break;
+            load(p0, min(i + 2, n - 1) * 1024);
+            multiply(p1, (i + 1) * 1024);
+        }
     }
-    // 64 sums over 64 lanes: at the step that pairs lanes l and l ^ b a lane keeps the sums
-    // whose number has l's bit b; sum number e = r * MR + m ends in lane e
-    float v[64];
+    if (MR != 8 && K % 256 && K / 256 % 4 == wave && lane * 4 < K % 256) {            // the last piece, K is a multiple of 4
+        const int k = K / 1024 * 1024;
+        Piece p;
+        load(p, k);
+        multiply(p, k);
+    }
+    // at the step that pairs lanes l and l ^ b a lane keeps the sums whose number has l's bit b
+    float v[S];
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int m = 0; m < MR; ++m) v[r * MR + m] = acc[r][m];
 #pragma unroll
-    for (int b = 1, n = 32; b < 64; b <<= 1, n >>= 1) {
+    for (int b = 1, n2 = S / 2; b < 64; b <<= 1, n2 >>= 1) {
         const bool up = (lane & b) != 0;
+        if (b < S) {
 #pragma unroll
-        for (int i = 0; i < n; ++i) {
-            const float keep = up ? v[2 * i + 1] : v[2 * i];
-            const float send = up ? v[2 * i] : v[2 * i + 1];
-            v[i] = keep + __shfl_xor(send, b, ILLM_WAVE);
+            for (int i = 0; i < n2; ++i) {
+                const float keep = up ? v[2 * i + 1] : v[2 * i];
+                const float send = up ? v[2 * i] : v[2 * i + 1];
+                v[i] = keep + __shfl_xor(send, b, ILLM_WAVE);
+            }
+        } else {
+            v[0] += __shfl_xor(v[0], b, ILLM_WAVE);
         }
     }
-    part[wave][lane] = v[0];
+    if (lane < S) part[wave][lane] = v[0];
     __syncthreads();
-    if (wave == 0) {
+    if (wave == 0 && lane < S) {
         const float t = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
         const int r = lane / MR, m = lane % MR;
         if (m < M && n0 + r < N) st_f(Y, y_dt, (size_t)m * N + n0 + r, t);
@@ -614,11 +658,15 @@ extern "C" int illm_gemv_rows_f32(const float* X, const float* W, void* Y, int y
                                   int K, void* stream) {
     if (M <= 0 || M > 16 || N <= 0 || K <= 0 || (K % 4) || !illm_dtype_ok(y_dt)) return ILLM_ERR_ARG;
     hipStream_t st = (hipStream_t)stream;
-    // (a block of 16 rows of W for up to 4 rows of X was slower than this one of 8 at three of
-    // the four 7B shapes: 72 against 60 us for 22016 x 4096, 34 against 36 for 4096 x 11008)
-    if (M <= 8)
-        hipLaunchKernelGGL(gemv_rows_f32_kernel<8>, dim3((N + 7) / 8), dim3(256), 0, st, X, W, Y, y_dt, M, N, K);
-    else
-        hipLaunchKernelGGL(gemv_rows_f32_kernel<16>, dim3((N + 3) / 4), dim3(256), 0, st, X, W, Y, y_dt, M, N, K);
+    // (blocks of 16 rows of W were slower than these of 8: 72 against 60 us for 22016 x 4096)
+#define ILLM_GEMV(MR, R, AHEAD) \
+    hipLaunchKernelGGL((gemv_rows_f32_kernel<MR, R, AHEAD>), dim3((N + R - 1) / R), dim3(256), 0, st, X, W, Y, y_dt, M, N, K)
+    const bool ahead = N <= 8192;                  // (blocks enough hide the loads: 22016 x 4096 of 8 rows 61 -> 70 us)
+    if (M > 8) ILLM_GEMV(16, 4, true);
+    else if (M > 4) ILLM_GEMV(8, 8, false);
+    else if (M > 2) { if (ahead) ILLM_GEMV(4, 8, true); else ILLM_GEMV(4, 8, false); }
+    else if (M > 1) { if (ahead) ILLM_GEMV(2, 8, true); else ILLM_GEMV(2, 8, false); }
+    else { if (ahead) ILLM_GEMV(1, 8, true); else ILLM_GEMV(1, 8, false); }
+#undef ILLM_GEMV
     return illm_launch_status();
 }

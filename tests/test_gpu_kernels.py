@@ -2059,3 +2059,17 @@ def test_gate_up_of_many_rows_in_turns(M, F, K):
     bad = run(M, 0.0)
     assert torch.equal(bad[rows], y[rows]) and bool(torch.isfinite(bad[rows].float()).all())
     assert lib.illm_gemm_turns_gate_up(o._p(x), o._p(w), o._p(y), M, F, K + 64, 0.0, 1.0, None) != 0
+
+
+@pytest.mark.parametrize("N, K", [(8, 4), (9, 256), (1, 1024), (70, 260), (33, 1284), (8200, 2052), (24, 5120)])
+def test_float32_rows_of_every_number_have_the_same_bits(N, K):
+    """A row of X gives the same sums alone and among 2, 3, 4, 5, 8, 9 and 16, each of which goes to its own number of rows a
+    block: no whole piece of 256 k, one, pieces for some waves only, a last piece in part, odd and even numbers a wave,
+    one piece at a time and the next one ahead (8,192 rows of W and more)."""
+    o = ops()
+    x, w = rnd(16, K, seed=1).to(DEV), rnd(N, K, seed=2).to(DEV)
+    want = x.double() @ w.double().t()
+    all16 = o.gemv_rows_f32(x, w, torch.float32)
+    assert float((all16.double() - want).abs().max()) <= K * 2.0 ** -24 * float((x.abs().double() @ w.abs().double().t()).max())
+    for M in (1, 2, 3, 4, 5, 8, 9):
+        assert torch.equal(o.gemv_rows_f32(x[:M].contiguous(), w, torch.float32), all16[:M]), M
