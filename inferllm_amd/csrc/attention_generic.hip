@@ -363,7 +363,7 @@ extern "C" int illm_attn_prefill_paged_generic(const void* qkv, void* out, int d
 // 155 us for 520 keys at head size 128: every load of a wave touched 64 rows), and the eight
 // scores are summed over the wave together, each step handing half of them to the partner lane.
 // The waves' (sums, max, weight) are combined in wave order at the end; each block leaves
-// (acc[hd], max, sum) in `partial`.  Plain float32 arithmetic and expf.
+// (acc[hd], max, sum) in `partial`, or, being the only one, the result.  Plain float32 arithmetic and expf.
 // A wave asks for the keys and the values of its next eight keys together, before it works on
 // the eight it has: one trip to memory a round instead of two, and that one beside the arithmetic.
 template <int DT, int DL>                  // storage type; dims a lane holds (head sizes up to 64 DL)
@@ -373,7 +373,7 @@ attn_decode_generic_kernel(const void* __restrict__ qkv, const void* __restrict_
                            const int32_t* __restrict__ page_table, int table_stride,
                            int page_size, int ring, const int32_t* __restrict__ seq_slot,
                            const int32_t* __restrict__ seq_len, float* __restrict__ partial,
-                           int nsplit, int nh, int nkv, int hd, float scale, int window) {
+                           int nsplit, int nh, int nkv, int hd, float scale, int window, void* __restrict__ out) {
     constexpr int KU = 8;                  // keys a wave takes at a time
     __shared__ float wave_acc[4][256];
     __shared__ float wave_ml[4][2];
@@ -501,9 +501,10 @@ attn_decode_generic_kernel(const void* __restrict__ qkv, const void* __restrict_
     if (tid < hd) {
         float a = 0.f;
         for (int w = 0; w < 4; ++w) a += f[w] * wave_acc[w][tid];
-        pp[tid] = a;
+        if (nsplit == 1) st_f(out, DT, ((size_t)b * nh + h) * hd + tid, a * (1.0f / lb));   // the whole result: no merge
+        else pp[tid] = a;
     }
-    if (tid == 0) {
+    if (tid == 0 && nsplit > 1) {
         pp[hd] = mb;
         pp[hd + 1] = lb;
     }
@@ -545,7 +546,7 @@ extern "C" int illm_attn_decode_generic(const void* qkv, void* out, int dt, cons
 #define ILLM_DECODE_GENERIC(DT, DL)                                                                   \
     hipLaunchKernelGGL((attn_decode_generic_kernel<DT, DL>), dim3(nh, B, nsplit), dim3(256), 0,       \
                        (hipStream_t)stream, qkv, kcache, vcache, page_table, table_stride, page_size, \
-                       ring, seq_slot, seq_len, partial, nsplit, nh, nkv, hd, scale, window)
+                       ring, seq_slot, seq_len, partial, nsplit, nh, nkv, hd, scale, window, out)
     const int dl = (hd + 63) / 64;
     if (dt == ILLM_F32) {
         if (dl == 1) ILLM_DECODE_GENERIC(ILLM_F32, 1);
@@ -557,6 +558,7 @@ extern "C" int illm_attn_decode_generic(const void* qkv, void* out, int dt, cons
         else ILLM_DECODE_GENERIC(ILLM_BF16, 4);
     }
 #undef ILLM_DECODE_GENERIC
+    if (nsplit == 1) return illm_launch_status();
     hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(nh, B), dim3(64), 0, (hipStream_t)stream,
                        (const float*)partial, out, dt, nsplit, nh, hd);
     return illm_launch_status();

@@ -1462,6 +1462,9 @@ def attn_decode(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
             f"attn_decode_bf16 (head_dim {hd})")
         return out
     _need(not softcap, "attn_decode: a soft cap needs bfloat16 and a head size in steps of 8")
+    # (a range is whole tiles of 256 keys: with no more of them than ranges the others are empty, and one range needs
+    # no merge: 3 us of a step of a tiny model's layer)
+    nsplit = max(1, min(nsplit, -(-page_table.shape[1] * page_size // 256))) if ring <= 0 else nsplit
     partial = torch.empty((B, nh, nsplit, hd + 2), dtype=torch.float32, device=qkv.device)
     _check(_lib().illm_attn_decode_generic(
         _p(qkv), _p(out), _code(qkv), _p(kcache), _p(vcache), _p(page_table), page_table.shape[1],

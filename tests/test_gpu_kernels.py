@@ -391,6 +391,25 @@ def test_attn_decode(dtype, nh, nkv, hd, lens, window, nsplit):
     close(got, want, dtype, scale=2)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nh,nkv,hd,lens,window", [(4, 2, 24, [1, 255, 256], 0), (6, 2, 256, [33, 512, 600], 0),
+                                                   (3, 3, 120, [600, 90], 70)])
+def test_one_range_of_keys_needs_no_merge(dtype, nh, nkv, hd, lens, window):
+    """The general kernel as the only range of its sequence writes the result itself: the same bits as with
+    further, empty ranges and a merge, where all keys are in the first 256 of a table that could hold more."""
+    page = 16
+    pt, kc, vc, slots, seq_len = paged_case(dtype, nkv, hd, lens, page)
+    pt = torch.cat([pt, torch.full((pt.shape[0], 64), kc.shape[0] - 1, dtype=torch.int32)], dim=1)
+    qkv = rnd(len(lens), (nh + 2 * nkv) * hd, dtype=dtype, seed=11)
+    got = {n: ops().attn_decode(qkv.to(DEV), kc.to(DEV), vc.to(DEV), pt.to(DEV), page, 0, slots.to(DEV),
+                                seq_len.to(DEV), nh, nkv, hd, 1.0 / math.sqrt(hd), window, n).cpu() for n in (1, 4)}
+    for b, n in enumerate(lens):
+        if n <= 256:
+            assert torch.equal(got[1][b], got[4][b])
+    want = R.attn_decode(qkv, kc, vc, pt, page, 0, slots, seq_len, nh, nkv, hd, 1.0 / math.sqrt(hd), window, 1)
+    close(got[1], want, dtype, scale=2)
+
+
 @pytest.mark.parametrize("nh,nkv,hd,lens,window,nsplit", [
     (32, 32, 128, [600, 1, 64, 65], 0, 1), (32, 8, 128, [300, 70], 0, 3), (4, 4, 16, [7, 200], 0, 2),
     (8, 1, 64, [1000], 0, 32), (6, 2, 24, [5, 11, 130], 0, 2), (16, 1, 256, [257, 31], 0, 2),
