@@ -138,6 +138,8 @@ int illm_gemm_rows_f32_mfma(const float* X, const float* W, void* Y, int y_dt, i
 // (decoding on the 32-bit path); plain float32 multiply-adds.
 int illm_gemv_rows_f32(const float* X, const float* W, void* Y, int y_dt, int M, int N, int K,
                        void* stream);
+int illm_gemv_rows_f32_fused(const float* X, const float* W, float* Y, int M, int N, int K, const float* norm_w,
+                             float eps, int epi, float limit, float alpha, void* stream);
 
 // Causal attention over packed rows of whole prompts (keys and values of the step
 // itself).  cu_seqlens[n_seqs + 1]; window <= 0: all earlier keys.

@@ -553,18 +553,48 @@ extern "C" int illm_gemm_rows_f32_mfma(const float* X, const float* W, void* Y, 
 // test.  us, matrices cold, 8 rows of sums for up to 8 of X, one piece at a time -> now, 1 and 4 rows: 4096 x 4096 15.4 / 15.2 ->
 // 12.7 / 14.3, 12288 x 4096 35.2 / 36.0 -> 31.9 / 33.9, 22016 x 4096 58.3 / 59.5 -> 55.0 / 56.6 (6.4 TB/s), 4096 x 11008 34.2 /
 // 34.5 -> 30.2 / 32.1, 512 x 96 3.7 / 3.8 -> 2.4 / 3.0.  The same bits.
-template <int MR, int R, bool AHEAD>
+// What stood around the products of a decode step of few rows was launches (5.5 us each between the products of a 7B layer,
+// 2 to 3 for a tiny model's, of 5 to 20 rows of work), so they are taken into them:
+// NORM: X holds rows whose RMS norm (weight `nw`, `eps`) is to be multiplied: x nw is multiplied, the block, which reads the
+// whole rows anyway, sums their squares, and the sums are scaled by 1 / sqrt(mean + eps) at the end.
+// EPI GEMV_ADD: float32 Y += the product.  GEMV_ACT: W = [gate | up] of N rows each, a block takes R / 2 of either; Y = the
+// activation of the two sums (silu(gate) up, or the clamped one with limit > 0).
+enum { GEMV_PLAIN = 0, GEMV_ADD = 1, GEMV_ACT = 2 };
+
+// v[i] of all lanes summed, sum i (modulo S) in v[0] of lane i: at the step that pairs lanes l and l ^ b a lane keeps the sums
+// whose number has l's bit b
+template <int S>
+static __device__ __forceinline__ void lanes_sums(float (&v)[S], int lane) {
+#pragma unroll
+    for (int b = 1, n2 = S / 2; b < 64; b <<= 1, n2 >>= 1) {
+        const bool up = (lane & b) != 0;
+        if (b < S) {
+#pragma unroll
+            for (int i = 0; i < n2; ++i) {
+                const float keep = up ? v[2 * i + 1] : v[2 * i];
+                const float send = up ? v[2 * i] : v[2 * i + 1];
+                v[i] = keep + __shfl_xor(send, b, ILLM_WAVE);
+            }
+        } else {
+            v[0] += __shfl_xor(v[0], b, ILLM_WAVE);
+        }
+    }
+}
+
+template <int MR, int R, bool AHEAD, bool NORM = false, int EPI = GEMV_PLAIN>
 __global__ void __launch_bounds__(256)
 gemv_rows_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, void* __restrict__ Y,
-                     int y_dt, int M, int N, int K) {
-    constexpr int S = R * MR;
+                     int y_dt, int M, int N, int K, const float* __restrict__ nw, float eps, float limit, float alpha) {
+    constexpr int S = R * MR, RN = EPI == GEMV_ACT ? R / 2 : R;      // sums; columns of Y a block makes
     static_assert(S <= 64 && (S & (S - 1)) == 0, "");
     __shared__ float part[4][S];
+    __shared__ float part_ss[4][MR];
     const int lane = threadIdx.x & 63, wave = wave_index();
-    const int n0 = blockIdx.x * R;
+    const int n0 = blockIdx.x * RN;
     const float *wrow[R], *xrow[MR];
 #pragma unroll
-    for (int r = 0; r < R; ++r) wrow[r] = W + (size_t)min(n0 + r, N - 1) * K + wave * 256;
+    for (int r = 0; r < R; ++r)
+        wrow[r] = W + ((r < RN ? (size_t)0 : (size_t)N) + min(n0 + r % RN, N - 1)) * K + wave * 256;
 #pragma unroll
     for (int m = 0; m < MR; ++m) xrow[m] = X + (size_t)min(m, M - 1) * K + wave * 256;
     float acc[R][MR];
@@ -572,6 +602,9 @@ gemv_rows_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, v
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int m = 0; m < MR; ++m) acc[r][m] = 0.f;
+    float ss[MR];
+#pragma unroll
+    for (int m = 0; m < MR; ++m) ss[m] = 0.f;
 
     struct Piece { f32x4v_t w[R]; };                         // (W is used once: loads that do not stay in the caches)
     auto load = [&](Piece& p, int k) __attribute__((always_inline)) {
@@ -580,9 +613,14 @@ gemv_rows_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, v
         if (AHEAD) __builtin_amdgcn_sched_barrier(0);        // (else they are put right before their use)
     };
     auto multiply = [&](const Piece& p, int k) __attribute__((always_inline)) {
+        const float4 g = NORM ? *(const float4*)(nw + wave * 256 + k + lane * 4) : make_float4(1.f, 1.f, 1.f, 1.f);
 #pragma unroll
         for (int m = 0; m < MR; ++m) {
-            const float4 x = *(const float4*)(xrow[m] + k + lane * 4);
+            float4 x = *(const float4*)(xrow[m] + k + lane * 4);
+            if (NORM) {
+                ss[m] += (x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w);
+                x.x *= g.x; x.y *= g.y; x.z *= g.z; x.w *= g.w;
+            }
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 float a = acc[r][m];
@@ -624,32 +662,39 @@ gemv_rows_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, v
         load(p, k);
         multiply(p, k);
     }
-    // at the step that pairs lanes l and l ^ b a lane keeps the sums whose number has l's bit b
     float v[S];
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int m = 0; m < MR; ++m) v[r * MR + m] = acc[r][m];
-#pragma unroll
-    for (int b = 1, n2 = S / 2; b < 64; b <<= 1, n2 >>= 1) {
-        const bool up = (lane & b) != 0;
-        if (b < S) {
-#pragma unroll
-            for (int i = 0; i < n2; ++i) {
-                const float keep = up ? v[2 * i + 1] : v[2 * i];
-                const float send = up ? v[2 * i] : v[2 * i + 1];
-                v[i] = keep + __shfl_xor(send, b, ILLM_WAVE);
-            }
-        } else {
-            v[0] += __shfl_xor(v[0], b, ILLM_WAVE);
-        }
-    }
+    lanes_sums(v, lane);
     if (lane < S) part[wave][lane] = v[0];
+    if (NORM) {
+        lanes_sums(ss, lane);
+        if (lane < MR) part_ss[wave][lane] = ss[0];
+    }
     __syncthreads();
     if (wave == 0 && lane < S) {
-        const float t = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
+        float t = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
         const int r = lane / MR, m = lane % MR;
-        if (m < M && n0 + r < N) st_f(Y, y_dt, (size_t)m * N + n0 + r, t);
+        if (NORM) {
+            const float sum = ((part_ss[0][m] + part_ss[1][m]) + part_ss[2][m]) + part_ss[3][m];
+            t *= 1.0f / sqrtf(sum / (float)K + eps);
+        }
+        if (EPI == GEMV_ACT) {
+            const float u = __shfl(t, (lane + S / 2) & 63, ILLM_WAVE);     // (of the gates' lanes: the up sum)
+            if (limit > 0.f) {
+                const float g = fminf(t, limit);
+                t = g / (1.0f + expf(-alpha * g)) * (fminf(fmaxf(u, -limit), limit) + 1.0f);
+            } else {
+                t = (t / (1.0f + expf(-t))) * u;
+            }
+        }
+        if (m < M && r < RN && n0 + r < N) {
+            const size_t at = (size_t)m * N + n0 + r;
+            if (EPI == GEMV_ADD) ((float*)Y)[at] += t;
+            else st_f(Y, y_dt, at, t);
+        }
     }
 }
 
@@ -659,8 +704,9 @@ extern "C" int illm_gemv_rows_f32(const float* X, const float* W, void* Y, int y
     if (M <= 0 || M > 16 || N <= 0 || K <= 0 || (K % 4) || !illm_dtype_ok(y_dt)) return ILLM_ERR_ARG;
     hipStream_t st = (hipStream_t)stream;
     // (blocks of 16 rows of W were slower than these of 8: 72 against 60 us for 22016 x 4096)
-#define ILLM_GEMV(MR, R, AHEAD) \
-    hipLaunchKernelGGL((gemv_rows_f32_kernel<MR, R, AHEAD>), dim3((N + R - 1) / R), dim3(256), 0, st, X, W, Y, y_dt, M, N, K)
+#define ILLM_GEMV(MR, R, AHEAD)                                                                                      \
+    hipLaunchKernelGGL((gemv_rows_f32_kernel<MR, R, AHEAD>), dim3((N + R - 1) / R), dim3(256), 0, st, X, W, Y, y_dt, M, N, K, \
+                       (const float*)nullptr, 0.f, 0.f, 0.f)
     const bool ahead = N <= 8192;                  // (blocks enough hide the loads: 22016 x 4096 of 8 rows 61 -> 70 us)
     if (M > 8) ILLM_GEMV(16, 4, true);
     else if (M > 4) ILLM_GEMV(8, 8, false);
@@ -668,5 +714,38 @@ extern "C" int illm_gemv_rows_f32(const float* X, const float* W, void* Y, int y
     else if (M > 1) { if (ahead) ILLM_GEMV(2, 8, true); else ILLM_GEMV(2, 8, false); }
     else { if (ahead) ILLM_GEMV(1, 8, true); else ILLM_GEMV(1, 8, false); }
 #undef ILLM_GEMV
+    return illm_launch_status();
+}
+
+// The same for M <= 8 rows with what surrounds the product taken in: norm_w [K] (and eps) the RMS norm of X's rows, or null;
+// epi 0: Y [M, N] float32 = the product, 1: Y += the product (without a norm), 2: W [2 N, K] = [gate | up], Y = their activation (limit 0:
+// silu(gate) up; else the clamped one of `alpha`).
+extern "C" int illm_gemv_rows_f32_fused(const float* X, const float* W, float* Y, int M, int N, int K, const float* norm_w,
+                                        float eps, int epi, float limit, float alpha, void* stream) {
+    if (M <= 0 || M > 8 || N <= 0 || K <= 0 || (K % 4) || epi < GEMV_PLAIN || epi > GEMV_ACT ||
+        (norm_w && epi == GEMV_ADD))
+        return ILLM_ERR_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    const bool ahead = N <= 8192 / (epi == GEMV_ACT ? 2 : 1);        // (as above, by rows of W)
+#define ILLM_GEMV_F(MR, AHEAD, NORM, EPI)                                                                             \
+    hipLaunchKernelGGL((gemv_rows_f32_kernel<MR, 8, AHEAD, NORM, EPI>), dim3((N + (EPI == GEMV_ACT ? 3 : 7)) / (EPI == GEMV_ACT ? 4 : 8)), \
+                       dim3(256), 0, st, X, W, Y, (int)ILLM_F32, M, N, K, norm_w, eps, limit, alpha)
+#define ILLM_GEMV_M(NORM, EPI)                                                                                        \
+    do {                                                                                                              \
+        if (M > 4) ILLM_GEMV_F(8, false, NORM, EPI);                                                                  \
+        else if (M > 2) { if (ahead) ILLM_GEMV_F(4, true, NORM, EPI); else ILLM_GEMV_F(4, false, NORM, EPI); }        \
+        else if (M > 1) { if (ahead) ILLM_GEMV_F(2, true, NORM, EPI); else ILLM_GEMV_F(2, false, NORM, EPI); }        \
+        else { if (ahead) ILLM_GEMV_F(1, true, NORM, EPI); else ILLM_GEMV_F(1, false, NORM, EPI); }                   \
+    } while (0)
+    if (norm_w) {
+        if (epi == GEMV_ACT) ILLM_GEMV_M(true, GEMV_ACT);
+        else ILLM_GEMV_M(true, GEMV_PLAIN);
+    } else {
+        if (epi == GEMV_ACT) ILLM_GEMV_M(false, GEMV_ACT);
+        else if (epi == GEMV_ADD) ILLM_GEMV_M(false, GEMV_ADD);
+        else return illm_gemv_rows_f32(X, W, Y, ILLM_F32, M, N, K, stream);
+    }
+#undef ILLM_GEMV_M
+#undef ILLM_GEMV_F
     return illm_launch_status();
 }

@@ -532,16 +532,17 @@ def decode_weight(w: torch.Tensor, mode: str = "plain", copies=False, **geometry
 
 
 class NormedRows:
-    """Residual rows whose RMS norm the next product takes itself (few rows, bfloat16).
+    """Residual rows whose RMS norm the next product takes itself (few rows).
 
-    Left by `linear_add(..., norm=)`: `x` the float32 residual rows (the sum already in them),
+    Of bfloat16 activations, left by `linear_add(..., norm=)`: `x` the float32 residual rows (the sum already in them),
     `xb` = bfloat16(x * weight), `ssq[m][p]` partial sums of x^2.  A product of few rows reads
     `xb` and scales row m of its result by 1 / sqrt(sum_p ssq[m][p] / K + eps), which is the
     product of the normed rows since the scale is common to a row; anything else asks `rows()`
-    for the normed rows."""
+    for the normed rows.  Of float32 activations (`norm_left`) `xb` is `x` and `ssq` None: the product's kernel
+    reads whole rows and squares them itself."""
 
     def __init__(self, x: torch.Tensor, weight: torch.Tensor, eps: float, act_dtype: torch.dtype,
-                 xb: torch.Tensor, ssq: torch.Tensor):
+                 xb: torch.Tensor, ssq: Optional[torch.Tensor]):
         self.x, self.weight, self.eps, self.dtype = x, weight, float(eps), act_dtype
         self.xb, self.ssq = xb, ssq
         self.shape = x.shape
@@ -588,6 +589,38 @@ def gemv_rows_f32(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype) -> t
         _check(_lib().illm_gemv_rows_f32(_p(x[m0:m0 + rows]), _p(w), _p(y[m0:m0 + rows]), _code(y),
                                          rows, N, K, _stream()), "gemv_rows_f32")
     return y
+
+
+F32_FUSED_ROWS = 8         # rows of float32 whose products take the norm before them, the activation behind them and the add
+                           # to the residual rows into their kernel (4 rows, a 7B layer: 228 -> 206 us)
+
+
+def gemv_f32_fused_fits(x, w) -> bool:
+    """Whether a product of float32 rows is one that takes in what surrounds it."""
+    xt, w = x.x if isinstance(x, NormedRows) else x, plain_weight(w)
+    return xt.is_cuda and x.dtype == torch.float32 and xt.shape[0] <= F32_FUSED_ROWS and gemv_rows_f32_fits(xt, w)
+
+
+def _gemv_f32_fused(x, w, y: torch.Tensor, N: int, epi: int, limit: float = 0.0) -> torch.Tensor:
+    normed = isinstance(x, NormedRows)
+    xt = x.x if normed else x
+    _gpu(xt, w, y, x.weight if normed else None)
+    _check(_lib().illm_gemv_rows_f32_fused(_p(xt), _p(w), _p(y), xt.shape[0], N, xt.shape[1], _p(x.weight) if normed else None,
+                                           ctypes.c_float(x.eps if normed else 0.0), epi, ctypes.c_float(limit),
+                                           ctypes.c_float(SWISH_ALPHA), _stream()), "gemv_rows_f32_fused")
+    return y
+
+
+def norm_left(x: torch.Tensor, params, act_dtype: torch.dtype) -> Optional[NormedRows]:
+    """Few float32 residual rows x for a part that takes rows with their RMS norm (weight, eps) still to be taken, or
+    None where the norm has a kernel of its own."""
+    if (params is None or act_dtype != torch.float32 or x.dtype != torch.float32 or not x.is_cuda or x.dim() != 2
+            or not 1 <= x.shape[0] <= F32_FUSED_ROWS or x.shape[1] % 4 or not x.is_contiguous()):
+        return None
+    weight, eps = params
+    if weight.dtype != torch.float32 or weight.shape != (x.shape[1],) or not weight.is_contiguous():
+        return None
+    return NormedRows(x, weight, eps, act_dtype, x, None)
 
 
 ROWS_F32_MFMA_FROM = 9     # measured streaming over many matrices of the 7B shapes: up to 8 rows
@@ -685,8 +718,11 @@ def gemm_f32_split(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype) -> 
 
 
 def linear_add_fits(x, w, into: torch.Tensor) -> bool:
-    """Whether `linear_add` takes these operands (few bfloat16 rows into float32 rows)."""
+    """Whether `linear_add` takes these operands (few bfloat16 or float32 rows into float32 rows)."""
     w = plain_weight(w)
+    if isinstance(x, torch.Tensor) and x.dtype == torch.float32:
+        return (gemv_f32_fused_fits(x, w) and into.dtype == torch.float32 and into.is_contiguous()
+                and into.shape == (x.shape[0], w.shape[0]))
     return (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and x.dim() == 2 and w.dim() == 2 and into.dtype == torch.float32 and
             into.is_contiguous() and 1 <= x.shape[0] <= SKINNY_BEST_ROWS and x.shape[1] % 8 == 0
@@ -700,6 +736,9 @@ def linear_add(x: torch.Tensor, w, into: torch.Tensor, norm=None,
     that follows: the kernel also leaves what the next few-rows product needs to take that norm
     itself, returned as `NormedRows` (only if N % 8 == 0, else None as without `norm`)."""
     _need(linear_add_fits(x, w, into), "linear_add: operands not taken")
+    if x.dtype == torch.float32:
+        _gemv_f32_fused(x, plain_weight(w), into, into.shape[1], 1)
+        return norm_left(into, norm, act_dtype)
     w, wt = _w(w)
     _gpu(x, w, into)
     M, K = x.shape
@@ -934,8 +973,12 @@ def linear(x, w, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     """y = x . w^T, w stored [out, in] (src/kern/naive/naive.cpp:363-379).  x may be
     `NormedRows`, w a `Weight`."""
     if isinstance(x, NormedRows):
-        if w.dtype == torch.bfloat16:
+        if w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16:
             return gemm_skinny_bf16(x, w, out_dtype or x.dtype)
+        if out_dtype in (None, torch.float32) and gemv_f32_fused_fits(x, w):
+            w = plain_weight(w)
+            y = torch.empty((x.shape[0], w.shape[0]), dtype=torch.float32, device=x.x.device)
+            return _gemv_f32_fused(x, w, y, w.shape[0], 0)
         x = x.rows()
     out_dtype = out_dtype or x.dtype
     if (isinstance(w, Weight) and out_dtype == torch.float32 and rows_fits(x, w, "plain")
@@ -1315,7 +1358,11 @@ def gate_up_act(x, w_gate_up, limit: float = 0.0) -> torch.Tensor:
     acts on the float32 sums), and likewise many of them; otherwise the product and `silu_mul` /
     `clamped_swish_mul`."""
     limit = float(limit)
-    if isinstance(x, NormedRows) and (w_gate_up.dtype != torch.bfloat16 or w_gate_up.shape[0] % 2):
+    if w_gate_up.shape[0] % 2 == 0 and gemv_f32_fused_fits(x, w_gate_up):
+        w = plain_weight(w_gate_up)
+        y = torch.empty((x.shape[0], w.shape[0] // 2), dtype=torch.float32, device=w.device)
+        return _gemv_f32_fused(x, w, y, w.shape[0] // 2, 2, limit)
+    if isinstance(x, NormedRows) and (w_gate_up.dtype != torch.bfloat16 or x.dtype != torch.bfloat16 or w_gate_up.shape[0] % 2):
         x = x.rows()
     M, K = x.shape
     F2 = w_gate_up.shape[0]

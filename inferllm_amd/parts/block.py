@@ -35,6 +35,10 @@ class PreNormBlock(Block):
             if params is not None and pending.made_for(*params):
                 return pending if part.takes_normed_rows else pending.rows()
             pending = None                       # the sum is in x already; another norm follows
+        if pending is None and part.takes_normed_rows:
+            left = ops.norm_left(x, norm.rms_params(), ctx.act_dtype)
+            if left is not None:
+                return left
         return norm.forward(x, pending, ctx)
 
     def forward(self, x, pending, ctx: StepContext, line, writes_cache, next_norm=None):

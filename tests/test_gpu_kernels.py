@@ -2092,3 +2092,35 @@ def test_float32_rows_of_every_number_have_the_same_bits(N, K):
     assert float((all16.double() - want).abs().max()) <= K * 2.0 ** -24 * float((x.abs().double() @ w.abs().double().t()).max())
     for M in (1, 2, 3, 4, 5, 8, 9):
         assert torch.equal(o.gemv_rows_f32(x[:M].contiguous(), w, torch.float32), all16[:M]), M
+
+
+@pytest.mark.parametrize("F,K", [(5, 4), (96, 96), (131, 1028), (4100, 516), (33, 4096)])
+def test_float32_products_of_few_rows_with_what_surrounds_them(F, K):
+    """The norm in front, the activation behind and the add to the residual rows in the product's kernel: a part of a
+    piece of K, odd numbers of columns, one piece at a time and the next ahead, 1 to 8 rows.  Against 64 bits within the
+    bound of a sum of K float32 products; the add and the activation with the bits of the separate kernels; a row's bits
+    whatever the number of rows."""
+    o = ops()
+    x, w = (rnd(8, K, seed=1) * 3.0).to(DEV), rnd(2 * F, K, seed=2).to(DEV)
+    nw, eps = (rnd(K, seed=3) + 1.0).to(DEV), 1e-5
+    xn = x.double() / torch.sqrt((x.double() ** 2).mean(1, keepdim=True) + eps) * nw.double()
+    want = xn @ w.double().t()
+    bound = (K + 8) * 2.0 ** -24 * (xn.abs() @ w.double().abs().t())           # a sum's K roundings and those of the norm
+    left = o.norm_left(x, (nw, eps), torch.float32)
+    got = o.linear(left, w)
+    assert bool(((got.double() - want).abs() <= bound).all())
+    close(left.rows(), xn.float().cpu(), torch.float32)
+    sums, acts = o.linear(x, w), {lim: o.gate_up_act(x, w, lim) for lim in (0.0, 1.25)}
+    assert torch.equal(acts[0.0], o.silu_mul(sums)) and torch.equal(acts[1.25], o.clamped_swish_mul(sums, 1.25))
+    assert torch.equal(o.gate_up_act(left, w), o.silu_mul(got))
+    base = rnd(8, 2 * F, seed=4).to(DEV)
+    for M in (1, 2, 3, 5, 8):
+        xm, into = x[:M].contiguous(), base[:M].clone()
+        assert o.linear_add_fits(xm, w, into)
+        after = o.linear_add(xm, w, into, (torch.ones(2 * F, device=DEV), eps), torch.float32)
+        assert torch.equal(into, base[:M] + sums[:M])
+        assert (after is None) == (2 * F % 4 != 0) and (after is None or after.x is into)
+        part = o.norm_left(xm, (nw, eps), torch.float32)
+        assert torch.equal(o.linear(part, w), got[:M]) and torch.equal(o.gate_up_act(xm, w), acts[0.0][:M])
+    assert o.norm_left(torch.zeros(9, K, device=DEV), (nw, eps), torch.float32) is None
+    assert o.norm_left(x, (nw, eps), torch.bfloat16) is None and not o.linear_add_fits(x, w, base.to(torch.bfloat16))
