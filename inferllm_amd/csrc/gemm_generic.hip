@@ -554,12 +554,22 @@ extern "C" int illm_gemm_rows_f32_mfma(const float* X, const float* W, void* Y, 
 // 12.7 / 14.3, 12288 x 4096 35.2 / 36.0 -> 31.9 / 33.9, 22016 x 4096 58.3 / 59.5 -> 55.0 / 56.6 (6.4 TB/s), 4096 x 11008 34.2 /
 // 34.5 -> 30.2 / 32.1, 512 x 96 3.7 / 3.8 -> 2.4 / 3.0.  The same bits.
 // What stood around the products of a decode step of few rows was launches (5.5 us each between the products of a 7B layer,
-// 2 to 3 for a tiny model's, of 5 to 20 rows of work), so they are taken into them:
+// 2 to 3 for a tiny model's), so they are taken into them.  us of norm, product and what follows, as kernels -> in one, 1 / 4
+// rows: q|k|v 192 x 96 7.1 / 8.0 -> 3.4 / 4.0, 3072 x 1024 9.7 / 10.6 -> 5.6 / 6.8, 6144 x 2048 16.4 / 18.1 -> 12.2 / 13.4;
+// gate and up 2 x 256 x 96 6.2 / 7.3 -> 3.1 / 3.8, 2 x 8192 x 2048 26.2 / 27.5 -> 22.2 / 23.9, 2 x 11008 x 4096 60.5 / 62.2 -> 55.1
+// / 56.5; the add costs 0.4.
 // NORM: X holds rows whose RMS norm (weight `nw`, `eps`) is to be multiplied: x nw is multiplied, the block, which reads the
 // whole rows anyway, sums their squares, and the sums are scaled by 1 / sqrt(mean + eps) at the end.
 // EPI GEMV_ADD: float32 Y += the product.  GEMV_ACT: W = [gate | up] of N rows each, a block takes R / 2 of either; Y = the
-// activation of the two sums (silu(gate) up, or the clamped one with limit > 0).
-enum { GEMV_PLAIN = 0, GEMV_ADD = 1, GEMV_ACT = 2 };
+// activation of the two sums (silu(gate) up, or the clamped one with limit > 0).  GEMV_QKV: the rows of W are the q, k and
+// v heads, a block takes four pairs (i, i + hd / 2) of one; q rotated into Y, k rotated and v into the cache.
+enum { GEMV_PLAIN = 0, GEMV_ADD = 1, GEMV_ACT = 2, GEMV_QKV = 3 };
+struct GemvQkv {
+    const float* cos_sin;                  // [positions, hd / 2, 2]
+    const int32_t *row_pos, *row_slot, *page_table;
+    float *kcache, *vcache;
+    int table_stride, page_size, ring, nh, nkv, hd;
+};
 
 // v[i] of all lanes summed, sum i (modulo S) in v[0] of lane i: at the step that pairs lanes l and l ^ b a lane keeps the sums
 // whose number has l's bit b
@@ -582,21 +592,34 @@ static __device__ __forceinline__ void lanes_sums(float (&v)[S], int lane) {
 }
 
 template <int MR, int R, bool AHEAD, bool NORM = false, int EPI = GEMV_PLAIN>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, MR == 4 && !AHEAD ? 4 : 1)
 gemv_rows_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, void* __restrict__ Y,
-                     int y_dt, int M, int N, int K, const float* __restrict__ nw, float eps, float limit, float alpha) {
-    constexpr int S = R * MR, RN = EPI == GEMV_ACT ? R / 2 : R;      // sums; columns of Y a block makes
+                     int y_dt, int M, int N, int K, const float* __restrict__ nw, float eps, float limit, float alpha, GemvQkv a) {
+    constexpr bool HALVES = EPI == GEMV_ACT || EPI == GEMV_QKV;      // the second R / 2 rows of W belong to the first
+    constexpr int S = R * MR, RN = HALVES ? R / 2 : R;               // sums; columns (pairs) a block makes
     static_assert(S <= 64 && (S & (S - 1)) == 0, "");
     __shared__ float part[4][S];
     __shared__ float part_ss[4][MR];
     const int lane = threadIdx.x & 63, wave = wave_index();
     const int n0 = blockIdx.x * RN;
+    const int head = EPI == GEMV_QKV ? n0 / (a.hd / 2) : 0, pair0 = EPI == GEMV_QKV ? n0 - head * (a.hd / 2) : 0;
     const float *wrow[R], *xrow[MR];
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-        wrow[r] = W + ((r < RN ? (size_t)0 : (size_t)N) + min(n0 + r % RN, N - 1)) * K + wave * 256;
+    for (int r = 0; r < R; ++r) {
+        size_t at = (r < RN ? (size_t)0 : (size_t)N) + min(n0 + r % RN, N - 1);
+        if (EPI == GEMV_QKV) at = (size_t)head * a.hd + pair0 + r % RN + (r < RN ? 0 : a.hd / 2);
+        wrow[r] = W + at * K + wave * 256;
+    }
 #pragma unroll
     for (int m = 0; m < MR; ++m) xrow[m] = X + (size_t)min(m, M - 1) * K + wave * 256;
+    // (what the lanes that finish q, k and v need is a chain of three loads: its first before W, the next before the lanes'
+    // sums, the wait for either behind other work.  All of it at the end took a tiny model's step 2 us a layer longer)
+    const bool finishes = EPI == GEMV_QKV && wave == 0 && lane % MR < M && lane < S / 2;
+    int pos = 0, slot = 0;
+    if (finishes) {
+        pos = a.row_pos[lane % MR];
+        slot = a.row_slot[lane % MR];
+    }
     float acc[R][MR];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -662,6 +685,13 @@ gemv_rows_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, v
         load(p, k);
         multiply(p, k);
     }
+    float2 cs = make_float2(1.f, 0.f);
+    int page = 0;
+    if (finishes) {
+        if (head < a.nh + a.nkv) cs = *(const float2*)(a.cos_sin + ((size_t)pos * (a.hd / 2) + pair0 + lane / MR) * 2);
+        const int lp = pos / a.page_size;                                  // (`cache_row_offset` in two steps)
+        if (head >= a.nh) page = a.page_table[(size_t)slot * a.table_stride + (a.ring > 0 ? lp % a.ring : lp)];
+    }
     float v[S];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -690,6 +720,20 @@ gemv_rows_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, v
                 t = (t / (1.0f + expf(-t))) * u;
             }
         }
+        if (EPI == GEMV_QKV) {
+            const float u = __shfl(t, (lane + S / 2) & 63, ILLM_WAVE);     // (of the first rows' lanes: the partner's sum)
+            if (m < M && r < RN) {
+                const bool turned = head < a.nh + a.nkv;
+                const int kvh = turned ? head - a.nh : head - a.nh - a.nkv;
+                float* to = (float*)Y + ((size_t)m * (a.nh + 2 * a.nkv) + head) * a.hd + pair0 + r;
+                if (head >= a.nh)
+                    to = (turned ? a.kcache : a.vcache) +
+                         (((size_t)page * a.nkv + kvh) * a.page_size + pos % a.page_size) * a.hd + pair0 + r;
+                to[0] = turned ? t * cs.x - u * cs.y : t;
+                to[a.hd / 2] = turned ? t * cs.y + u * cs.x : u;
+            }
+            return;
+        }
         if (m < M && r < RN && n0 + r < N) {
             const size_t at = (size_t)m * N + n0 + r;
             if (EPI == GEMV_ADD) ((float*)Y)[at] += t;
@@ -706,7 +750,7 @@ extern "C" int illm_gemv_rows_f32(const float* X, const float* W, void* Y, int y
     // (blocks of 16 rows of W were slower than these of 8: 72 against 60 us for 22016 x 4096)
 #define ILLM_GEMV(MR, R, AHEAD)                                                                                      \
     hipLaunchKernelGGL((gemv_rows_f32_kernel<MR, R, AHEAD>), dim3((N + R - 1) / R), dim3(256), 0, st, X, W, Y, y_dt, M, N, K, \
-                       (const float*)nullptr, 0.f, 0.f, 0.f)
+                       (const float*)nullptr, 0.f, 0.f, 0.f, GemvQkv{})
     const bool ahead = N <= 8192;                  // (blocks enough hide the loads: 22016 x 4096 of 8 rows 61 -> 70 us)
     if (M > 8) ILLM_GEMV(16, 4, true);
     else if (M > 4) ILLM_GEMV(8, 8, false);
@@ -718,25 +762,28 @@ extern "C" int illm_gemv_rows_f32(const float* X, const float* W, void* Y, int y
 }
 
 // The same for M <= 8 rows with what surrounds the product taken in: norm_w [K] (and eps) the RMS norm of X's rows, or null;
-// epi 0: Y [M, N] float32 = the product, 1: Y += the product (without a norm), 2: W [2 N, K] = [gate | up], Y = their activation (limit 0:
-// silu(gate) up; else the clamped one of `alpha`).
+// epi 0: Y [M, N] float32 = the product, 1: Y += the product (without a norm), 2: W [2 N, K] = [gate | up], Y = their
+// activation (limit 0: silu(gate) up; else the clamped one of `alpha`).
+#define ILLM_GEMV_F(MR, AHEAD, NORM, EPI)                                                                             \
+    hipLaunchKernelGGL((gemv_rows_f32_kernel<MR, 8, AHEAD, NORM, EPI>), dim3(blocks), dim3(256), 0, (hipStream_t)stream, \
+                       X, W, Y, (int)ILLM_F32, M, N, K, norm_w, eps, limit, alpha, qkv)
+#define ILLM_GEMV_M(NORM, EPI)                                                                                        \
+    do {                                                                                                              \
+        if (M > 4) ILLM_GEMV_F(8, false, NORM, EPI);                                                                  \
+        else if (M > 2) { if (ahead) ILLM_GEMV_F(4, true, NORM, EPI); else ILLM_GEMV_F(4, false, NORM, EPI); }        \
+        else if (M > 1) { if (ahead) ILLM_GEMV_F(2, true, NORM, EPI); else ILLM_GEMV_F((NORM ? 4 : 2), false, NORM, EPI); } \
+        else { if (ahead) ILLM_GEMV_F(1, true, NORM, EPI); else ILLM_GEMV_F(1, false, NORM, EPI); }                   \
+    } while (0)
+// (2 rows with a norm, the next piece not ahead: sums for 4 rows, whose code is the better one: 2 x 8192 x 2048 25.8 -> 23.4 us,
+// 2 x 13824 x 5120 93.6 -> 86.1)
 extern "C" int illm_gemv_rows_f32_fused(const float* X, const float* W, float* Y, int M, int N, int K, const float* norm_w,
                                         float eps, int epi, float limit, float alpha, void* stream) {
     if (M <= 0 || M > 8 || N <= 0 || K <= 0 || (K % 4) || epi < GEMV_PLAIN || epi > GEMV_ACT ||
         (norm_w && epi == GEMV_ADD))
         return ILLM_ERR_ARG;
-    hipStream_t st = (hipStream_t)stream;
     const bool ahead = N <= 8192 / (epi == GEMV_ACT ? 2 : 1);        // (as above, by rows of W)
-#define ILLM_GEMV_F(MR, AHEAD, NORM, EPI)                                                                             \
-    hipLaunchKernelGGL((gemv_rows_f32_kernel<MR, 8, AHEAD, NORM, EPI>), dim3((N + (EPI == GEMV_ACT ? 3 : 7)) / (EPI == GEMV_ACT ? 4 : 8)), \
-                       dim3(256), 0, st, X, W, Y, (int)ILLM_F32, M, N, K, norm_w, eps, limit, alpha)
-#define ILLM_GEMV_M(NORM, EPI)                                                                                        \
-    do {                                                                                                              \
-        if (M > 4) ILLM_GEMV_F(8, false, NORM, EPI);                                                                  \
-        else if (M > 2) { if (ahead) ILLM_GEMV_F(4, true, NORM, EPI); else ILLM_GEMV_F(4, false, NORM, EPI); }        \
-        else if (M > 1) { if (ahead) ILLM_GEMV_F(2, true, NORM, EPI); else ILLM_GEMV_F(2, false, NORM, EPI); }        \
-        else { if (ahead) ILLM_GEMV_F(1, true, NORM, EPI); else ILLM_GEMV_F(1, false, NORM, EPI); }                   \
-    } while (0)
+    const int cols = epi == GEMV_ACT ? 4 : 8, blocks = (N + cols - 1) / cols;
+    const GemvQkv qkv{};
     if (norm_w) {
         if (epi == GEMV_ACT) ILLM_GEMV_M(true, GEMV_ACT);
         else ILLM_GEMV_M(true, GEMV_PLAIN);
@@ -745,7 +792,31 @@ extern "C" int illm_gemv_rows_f32_fused(const float* X, const float* W, float* Y
         else if (epi == GEMV_ADD) ILLM_GEMV_M(false, GEMV_ADD);
         else return illm_gemv_rows_f32(X, W, Y, ILLM_F32, M, N, K, stream);
     }
-#undef ILLM_GEMV_M
-#undef ILLM_GEMV_F
     return illm_launch_status();
 }
+
+// The q|k|v product of M <= 8 single tokens with the rotation of q and k (pairs (i, i + hd / 2) of a head, hd % 8 == 0) and
+// the store of k and v: row m at position row_pos[m] of slot row_slot[m].  Y [M, (nh + 2 nkv) hd]: only q is written.
+extern "C" int illm_gemv_qkv_f32(const float* X, const float* W, float* Y, int M, int K, const float* norm_w, float eps,
+                                 const float* cos_sin, const int32_t* row_pos, const int32_t* row_slot, float* kcache,
+                                 float* vcache, const int32_t* page_table, int table_stride, int page_size, int ring,
+                                 int nh, int nkv, int hd, void* stream) {
+    if (M <= 0 || M > 8 || K <= 0 || (K % 4) || nh <= 0 || nkv <= 0 || hd <= 0 || (hd % 8) || page_size <= 0 || table_stride <= 0)
+        return ILLM_ERR_ARG;
+    const GemvQkv qkv = {cos_sin, row_pos, row_slot, page_table, kcache, vcache, table_stride, page_size, ring, nh, nkv, hd};
+    const int N = (nh + 2 * nkv) * hd, blocks = N / 8;
+    const float limit = 0.f, alpha = 0.f;
+#define ILLM_GEMV_QKV(NORM)                                                                                           \
+    do {                                                                                                              \
+        if (M > 4) ILLM_GEMV_F(8, false, NORM, GEMV_QKV);                                                             \
+        else if (M > 2) ILLM_GEMV_F(4, true, NORM, GEMV_QKV);                                                         \
+        else if (M > 1) ILLM_GEMV_F(2, true, NORM, GEMV_QKV);                                                         \
+        else ILLM_GEMV_F(1, true, NORM, GEMV_QKV);                                                                    \
+    } while (0)
+    if (norm_w) ILLM_GEMV_QKV(true);
+    else ILLM_GEMV_QKV(false);
+#undef ILLM_GEMV_QKV
+    return illm_launch_status();
+}
+#undef ILLM_GEMV_M
+#undef ILLM_GEMV_F

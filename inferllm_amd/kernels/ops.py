@@ -560,7 +560,7 @@ class NormedRows:
 def _operand(x):
     """(tensor the kernel reads, ssq pointer, parts, eps) of a few-rows product's input."""
     if isinstance(x, NormedRows):
-        return x.xb, _p(x.ssq), x.ssq.shape[1], ctypes.c_float(x.eps)
+        return x.xb, _p(x.ssq), x.ssq.shape[1] if x.ssq is not None else 0, ctypes.c_float(x.eps)
     return x, None, 0, ctypes.c_float(0.0)
 
 
@@ -592,7 +592,7 @@ def gemv_rows_f32(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype) -> t
 
 
 F32_FUSED_ROWS = 8         # rows of float32 whose products take the norm before them, the activation behind them and the add
-                           # to the residual rows into their kernel (4 rows, a 7B layer: 228 -> 206 us)
+                           # to the residual rows into their kernel
 
 
 def gemv_f32_fused_fits(x, w) -> bool:
@@ -613,9 +613,11 @@ def _gemv_f32_fused(x, w, y: torch.Tensor, N: int, epi: int, limit: float = 0.0)
 
 def norm_left(x: torch.Tensor, params, act_dtype: torch.dtype) -> Optional[NormedRows]:
     """Few float32 residual rows x for a part that takes rows with their RMS norm (weight, eps) still to be taken, or
-    None where the norm has a kernel of its own."""
+    None where the norm has a kernel of its own: above 4 rows that is the faster way for wide rows (8 of 4,096, two
+    products: 109 us a norm of its own, 120 in the products; of 2,048: 41 and 37)."""
     if (params is None or act_dtype != torch.float32 or x.dtype != torch.float32 or not x.is_cuda or x.dim() != 2
-            or not 1 <= x.shape[0] <= F32_FUSED_ROWS or x.shape[1] % 4 or not x.is_contiguous()):
+            or not 1 <= x.shape[0] <= (F32_FUSED_ROWS if x.shape[1] <= 2048 else 4) or x.shape[1] % 4
+            or not x.is_contiguous()):
         return None
     weight, eps = params
     if weight.dtype != torch.float32 or weight.shape != (x.shape[1],) or not weight.is_contiguous():
@@ -721,8 +723,8 @@ def linear_add_fits(x, w, into: torch.Tensor) -> bool:
     """Whether `linear_add` takes these operands (few bfloat16 or float32 rows into float32 rows)."""
     w = plain_weight(w)
     if isinstance(x, torch.Tensor) and x.dtype == torch.float32:
-        return (gemv_f32_fused_fits(x, w) and into.dtype == torch.float32 and into.is_contiguous()
-                and into.shape == (x.shape[0], w.shape[0]))
+        return (gemv_f32_fused_fits(x, w) and (x.shape[0] <= 4 or w.shape[0] <= 2048)     # (where `norm_left` follows)
+                and into.dtype == torch.float32 and into.is_contiguous() and into.shape == (x.shape[0], w.shape[0]))
     return (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and x.dim() == 2 and w.dim() == 2 and into.dtype == torch.float32 and
             into.is_contiguous() and 1 <= x.shape[0] <= SKINNY_BEST_ROWS and x.shape[1] % 8 == 0
@@ -1232,7 +1234,9 @@ PLAIN_WAVES = 0          # and for the plain few-rows product
 def qkv_rope_store_fits(x, w_qkv, hd: int) -> bool:
     """Whether the one-kernel q|k|v product + rotation + cache store takes these operands: up to
     16 rows always, up to 128 (96 for small matrices) with a decode copy of the matrix in q|k|v
-    tile order."""
+    tile order; of float32 up to 8 (the cache being of the rows' type)."""
+    if gemv_f32_fused_fits(x, w_qkv):                # (12288 x 4096 of 4 rows: 36.6 us with a rotation of its own, 38.4 in one)
+        return hd % 8 == 0 and w_qkv.shape[0] <= 8192
     if not (x.dtype == torch.bfloat16 and w_qkv.dtype == torch.bfloat16 and hd % 16 == 0):
         return False
     if 1 <= x.shape[0] <= SKINNY_BEST_ROWS and x.shape[1] % 8 == 0:
@@ -1300,8 +1304,8 @@ def qkv_rope_store(x, w_qkv, cos_sin: torch.Tensor,
     """Decode only: x . Wqkv^T, q and k rotated (pairs (i, i + hd/2), all dims) at row_pos, q
     returned in rows [q | k | v] whose k and v parts are NOT filled, k and v stored in the cache.
     x may be `NormedRows`."""
-    xt, ssq, parts, eps = _operand(x)
     _need(qkv_rope_store_fits(x, w_qkv, hd), "qkv_rope_store: operands not taken")
+    xt, ssq, parts, eps = _operand(x)
     w_qkv, wt = _w(w_qkv, "qkv")
     _gpu(xt, w_qkv, cos_sin, row_pos, row_slot, kcache, vcache, page_table)
     _i32(row_pos, x.shape[0]); _i32(row_slot, x.shape[0]); _i32(page_table)
@@ -1310,10 +1314,18 @@ def qkv_rope_store(x, w_qkv, cos_sin: torch.Tensor,
     _need(w_qkv.shape == (N, K), f"qkv_rope_store: weight {tuple(w_qkv.shape)} vs ({N}, {K})")
     _need(cos_sin.dtype == torch.float32 and cos_sin.dim() == 3 and cos_sin.shape[1] * 2 == hd and
           cos_sin.shape[2] == 2, "qkv_rope_store: angle table must be float32 [max_pos, hd/2, 2]")
-    _need(kcache.dtype == torch.bfloat16 and kcache.shape[1:] == (nkv, page_size, hd) and
-          vcache.shape == kcache.shape and vcache.dtype == torch.bfloat16 and page_table.dim() == 2,
+    _need(kcache.dtype == x.dtype and kcache.shape[1:] == (nkv, page_size, hd) and
+          vcache.shape == kcache.shape and vcache.dtype == x.dtype and page_table.dim() == 2,
           "qkv_rope_store: cache shape or dtype")
-    y = torch.empty((M, N), dtype=torch.bfloat16, device=xt.device)
+    y = torch.empty((M, N), dtype=x.dtype, device=xt.device)
+    if x.dtype == torch.float32:
+        normed = isinstance(x, NormedRows)
+        _gpu(x.weight if normed else None)
+        _check(_lib().illm_gemv_qkv_f32(
+            _p(xt), _p(w_qkv), _p(y), M, K, _p(x.weight) if normed else None, eps, _p(cos_sin), _p(row_pos), _p(row_slot),
+            _p(kcache), _p(vcache), _p(page_table), page_table.shape[1], page_size, ring, nh, nkv, hd, _stream()),
+            "qkv_rope_store (float32)")
+        return y
     if wt is not None and K % 64 == 0 and M >= rows_from("qkv", w_qkv):
         _check(_lib().illm_qkv_rope_store_rows(
             _p(xt), wt, _p(y), M, K, _p(cos_sin), cos_sin.shape[0], _p(row_pos), _p(row_slot),

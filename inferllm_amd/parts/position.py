@@ -109,7 +109,7 @@ class Rotary(PositionEncoding):
     def project_qkv(self, h, w_qkv, ctx: StepContext, nh, nkv, hd, kcache, vcache, group):
         if (not ctx.prefill and kcache is not None and self.pairing == "half"
                 and self.rotary_dim == hd and ops.qkv_rope_store_fits(h, w_qkv, hd)
-                and kcache.dtype == torch.bfloat16):
+                and kcache.dtype == h.dtype):
             return ops.qkv_rope_store(h, w_qkv, self.table(ctx.device), ctx.row_pos, ctx.row_slot,
                                       kcache, vcache, group.table, group.page_size, group.ring,
                                       nh, nkv, hd)

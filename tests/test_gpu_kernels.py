@@ -2106,21 +2106,55 @@ def test_float32_products_of_few_rows_with_what_surrounds_them(F, K):
     xn = x.double() / torch.sqrt((x.double() ** 2).mean(1, keepdim=True) + eps) * nw.double()
     want = xn @ w.double().t()
     bound = (K + 8) * 2.0 ** -24 * (xn.abs() @ w.double().abs().t())           # a sum's K roundings and those of the norm
-    left = o.norm_left(x, (nw, eps), torch.float32)
-    got = o.linear(left, w)
+    left = o.norm_left(x[:8 if K <= 2048 else 4], (nw, eps), torch.float32)
+    n = left.shape[0]
+    got, want, bound, xn = o.linear(left, w), want[:n], bound[:n], xn[:n]
     assert bool(((got.double() - want).abs() <= bound).all())
     close(left.rows(), xn.float().cpu(), torch.float32)
     sums, acts = o.linear(x, w), {lim: o.gate_up_act(x, w, lim) for lim in (0.0, 1.25)}
     assert torch.equal(acts[0.0], o.silu_mul(sums)) and torch.equal(acts[1.25], o.clamped_swish_mul(sums, 1.25))
     assert torch.equal(o.gate_up_act(left, w), o.silu_mul(got))
     base = rnd(8, 2 * F, seed=4).to(DEV)
-    for M in (1, 2, 3, 5, 8):
+    for M in (1, 2, 3, 4, 5, 8):
         xm, into = x[:M].contiguous(), base[:M].clone()
-        assert o.linear_add_fits(xm, w, into)
+        assert torch.equal(o.gate_up_act(xm, w), acts[0.0][:M])
+        assert o.linear_add_fits(xm, w, into) == (M <= 4 or 2 * F <= 2048)
+        if not o.linear_add_fits(xm, w, into):
+            continue
         after = o.linear_add(xm, w, into, (torch.ones(2 * F, device=DEV), eps), torch.float32)
         assert torch.equal(into, base[:M] + sums[:M])
         assert (after is None) == (2 * F % 4 != 0) and (after is None or after.x is into)
         part = o.norm_left(xm, (nw, eps), torch.float32)
-        assert torch.equal(o.linear(part, w), got[:M]) and torch.equal(o.gate_up_act(xm, w), acts[0.0][:M])
+        assert (part is None) == (M > 4 and K > 2048)
+        if part is not None:
+            assert torch.equal(o.linear(part, w), got[:M]) and torch.equal(o.gate_up_act(part, w), o.silu_mul(got[:M]))
     assert o.norm_left(torch.zeros(9, K, device=DEV), (nw, eps), torch.float32) is None
     assert o.norm_left(x, (nw, eps), torch.bfloat16) is None and not o.linear_add_fits(x, w, base.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M,nh,nkv,hd,K,ring", [(1, 4, 2, 24, 96, 0), (3, 3, 1, 8, 1028, 2), (8, 16, 16, 128, 256, 0),
+                                                (5, 60, 1, 128, 516, 3), (4, 2, 2, 120, 4096, 0),
+                                                (2, 4, 4, 64, 2048, 0)])
+@pytest.mark.parametrize("normed", [False, True])
+def test_float32_qkv_rope_store_equals_the_three_steps(M, nh, nkv, hd, K, ring, normed):
+    """Few float32 rows: the product with rotation and store in one kernel against product, then `rope_store` (whose two
+    roundings a rotated value may take in another order)."""
+    from inferllm_amd.parts.position import rotary_table
+    o, page = ops(), 16
+    table = rotary_table(777.0, hd, 300, "cpu").to(DEV)
+    x, w = rnd(M, K, seed=1).to(DEV), rnd((nh + 2 * nkv) * hd, K, seed=2, std=0.1).to(DEV)
+    x = o.norm_left(x, ((rnd(K, seed=3) + 1.0).to(DEV), 1e-5), torch.float32) if normed else x
+    pos = torch.tensor([(37 * i + 5) % 290 for i in range(M)], dtype=torch.int32, device=DEV)
+    slot = torch.randperm(M + 2, generator=torch.Generator().manual_seed(9))[:M].to(torch.int32).to(DEV)
+    pt = torch.randperm((M + 2) * 19, generator=torch.Generator().manual_seed(4)).reshape(M + 2, 19).to(torch.int32).to(DEV)
+    caches = [[c.to(DEV) for c in make_cache((M + 2) * 19, nkv, page, hd, torch.float32)] for _ in range(2)]
+    assert o.qkv_rope_store_fits(x, w, hd)
+    got = o.qkv_rope_store(x, w, table, pos, slot, *caches[0], pt, page, ring, nh, nkv, hd)
+    want = o.linear(x, w)
+    size = float(want.abs().max())
+    o.rope_store(want, table, hd, 0, pos, slot, None, *caches[1], pt, page, ring, nh, nkv, hd)
+    near = lambda a, b: float((a - b).abs().max()) <= 2.0 ** -22 * size
+    assert near(got[:, :nh * hd], want[:, :nh * hd])
+    for a, b in zip(*caches):
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and near(torch.nan_to_num(a), torch.nan_to_num(b))
+    assert not o.qkv_rope_store_fits(x, w, hd + 4)
