@@ -239,9 +239,12 @@ __device__ int nth_equal_id(const float* s, int lo, int hi, const Keep& k, int r
 // pass from the mass per digit instead of 32 walks.  Measured with top_p alone: 32,000 ids
 // 557 -> 104 us (every pass in chunks and the exponentials recomputed in each, before), 128,256
 // ids and 16 rows 2,190 -> 400 us.
-constexpr int SAMPLE_REG_IDS = 32;      // ids a thread keeps in registers (IN_REGS: V <= 32 * SB)
+// A row of up to two ids a thread has its scores and probabilities in LDS: what a pass writes the next reads back, and the
+// scratch answered after some 700 ns, three times over (320 ids, temperature alone FIGURES; the same picks).
+constexpr int SAMPLE_REG_IDS = 32;      // ids a thread keeps in registers at most (V <= 32 * SB)
+constexpr int SAMPLE_LDS_IDS = 2;       // and in LDS
 
-template <bool IN_REGS>
+template <int REGS>                     // ids a thread keeps in registers, 0 for none
 __global__ void __launch_bounds__(SB)
 sample_kernel(const float* __restrict__ logits, float* __restrict__ scratch,
               int32_t* __restrict__ out, int V, float temp, int top_k, float top_p,
@@ -253,11 +256,15 @@ sample_kernel(const float* __restrict__ logits, float* __restrict__ scratch,
     __shared__ int sh_i;
     const int b = blockIdx.x, tid = threadIdx.x;
     const float* row = logits + (size_t)b * V;
-    float* s = scratch + (size_t)b * V;                       // scaled, penalised scores
-    float* pr = scratch + ((size_t)gridDim.x + b) * V;        // exp(s - max)
+    constexpr bool SMALL = REGS == SAMPLE_LDS_IDS;
+    __shared__ __attribute__((aligned(16))) float lds[SMALL ? 2 * SAMPLE_LDS_IDS * SB : 4];
+    float* s = SMALL ? lds : scratch + (size_t)b * V;         // scaled, penalised scores
+    float* pr = SMALL ? lds + SAMPLE_LDS_IDS * SB : scratch + ((size_t)gridDim.x + b) * V;        // exp(s - max)
     const int chunk = (V + SB - 1) / SB;
     const int lo = min(V, tid * chunk), hi = min(V, lo + chunk);
     const int nl = last_tokens ? min(n_last, 256) : 0;
+    const uint64_t seed = seeds[b];                           // (possibly the host's memory: asked for ahead of the passes)
+    const int counter = counters[b];
     if (tid < nl) last[tid] = last_tokens[(size_t)b * n_last + tid];
     __syncthreads();
 
@@ -279,8 +286,8 @@ sample_kernel(const float* __restrict__ logits, float* __restrict__ scratch,
 
     // The passes below walk the row's (id, key, probability): from registers, or from the
     // scratch again (a pass of 32,000 ids then waits for the cache four times over, 8 us).
-    constexpr int RV = SAMPLE_REG_IDS;
-    constexpr bool in_regs = IN_REGS;
+    constexpr bool in_regs = REGS > 0;
+    constexpr int RV = in_regs ? REGS : 1;
     uint32_t rkey[RV];
     float rp[RV];
     if constexpr (in_regs) {
@@ -414,7 +421,7 @@ sample_kernel(const float* __restrict__ logits, float* __restrict__ scratch,
     });
     float total;
     const float before = block_exclusive_scan<float>(mine, red_f, &total);
-    const float u = uniform_from(seeds[b], counters[b]);
+    const float u = uniform_from(seed, counter);
     const float target = u * total;
     __syncthreads();
     if (tid == 0) sh_i = -1;
@@ -1118,12 +1125,16 @@ extern "C" int illm_sample(const float* logits, float* scratch, int32_t* out, in
         hipLaunchKernelGGL((sample_topk_kernel<false, 0>), dim3(B), dim3(SB), 0, (hipStream_t)stream, logits,
                            scratch, out, V, temp, top_k, top_p, repeat_penalty, last_tokens, n_last,
                            seeds, counters);
+    else if (V <= SAMPLE_LDS_IDS * SB)
+        hipLaunchKernelGGL(sample_kernel<SAMPLE_LDS_IDS>, dim3(B), dim3(SB), 0, (hipStream_t)stream, logits,
+                           scratch, out, V, temp, top_k, top_p, repeat_penalty, last_tokens, n_last,
+                           seeds, counters);
     else if (V <= SAMPLE_REG_IDS * SB)
-        hipLaunchKernelGGL(sample_kernel<true>, dim3(B), dim3(SB), 0, (hipStream_t)stream, logits,
+        hipLaunchKernelGGL(sample_kernel<SAMPLE_REG_IDS>, dim3(B), dim3(SB), 0, (hipStream_t)stream, logits,
                            scratch, out, V, temp, top_k, top_p, repeat_penalty, last_tokens, n_last,
                            seeds, counters);
     else
-        hipLaunchKernelGGL(sample_kernel<false>, dim3(B), dim3(SB), 0, (hipStream_t)stream, logits,
+        hipLaunchKernelGGL(sample_kernel<0>, dim3(B), dim3(SB), 0, (hipStream_t)stream, logits,
                            scratch, out, V, temp, top_k, top_p, repeat_penalty, last_tokens, n_last,
                            seeds, counters);
     return illm_launch_status();
