@@ -240,7 +240,8 @@ __device__ int nth_equal_id(const float* s, int lo, int hi, const Keep& k, int r
 // 557 -> 104 us (every pass in chunks and the exponentials recomputed in each, before), 128,256
 // ids and 16 rows 2,190 -> 400 us.
 // A row of up to two ids a thread has its scores and probabilities in LDS: what a pass writes the next reads back, and the
-// scratch answered after some 700 ns, three times over (320 ids, temperature alone FIGURES; the same picks).
+// scratch answered after some 700 ns, three times over (320 ids, temperature alone 8.3 -> 6.4 us, with top_p 58 -> 27, and
+// 1,025 of 2,000 ids 102 -> 45, with the walks of two ids a thread instead of 32; the same picks).
 constexpr int SAMPLE_REG_IDS = 32;      // ids a thread keeps in registers at most (V <= 32 * SB)
 constexpr int SAMPLE_LDS_IDS = 2;       // and in LDS
 
@@ -754,6 +755,9 @@ sample_topk_merge_kernel(float* __restrict__ scratch, int32_t* __restrict__ out,
 //   edge    (top_p) the last digit; per part the mass above the threshold key and the ids at it
 //   draw    one block a row: how many ids at the threshold key stay (the lowest ids), the part
 //           that holds the target of the draw, and the id in it
+// Each kernel walks 8 ids a thread at most; what bounded them was chains in what surrounds that: the parts' fields loaded one
+// after the other, sums of a block by one LDS address, a thread's digits above its own.  us a draw, as those -> as below: 16
+// rows of 128,256 with top_p 124 -> 66, one row 116 -> 58, 8 of 32,000 97 -> 50, 64 of 128,256 177 -> 155.  The same picks.
 #define SP_MAX_PARTS 16
 typedef unsigned long long sp_u64;
 
@@ -779,6 +783,17 @@ __device__ __forceinline__ SpPart sp_part(int V, int parts, int p) {
     const int stretch = ((V + parts - 1) / parts + 3) / 4 * 4;
     const int first = min(V, p * stretch);
     return {first, min(stretch, V - first)};
+}
+
+// The sum over a row's parts of a field that each has left; the loads of all 16 together (a loop to `parts` waited for one
+// after the other).
+__device__ __forceinline__ sp_u64 sp_over_parts(const sp_u64* a, size_t stride, int parts) {
+    sp_u64 v[SP_MAX_PARTS], sum = 0;
+#pragma unroll
+    for (int q = 0; q < SP_MAX_PARTS; ++q) v[q] = a[q * stride];
+#pragma unroll
+    for (int q = 0; q < SP_MAX_PARTS; ++q) sum += q < parts ? v[q] : 0;
+    return sum;
 }
 
 __global__ void __launch_bounds__(SB)
@@ -835,12 +850,15 @@ __device__ __forceinline__ void sp_histogram(sp_u64 (*mhist)[256], sp_u64* out, 
 __global__ void __launch_bounds__(SB)
 sp_mass_kernel(float* __restrict__ scratch, SpRow* __restrict__ rows, int V, int n_rows, float top_p) {
     __shared__ sp_u64 mhist[SB / ILLM_WAVE][256];
-    __shared__ sp_u64 sh_total;
+    __shared__ sp_u64 red_u[SB / ILLM_WAVE];
     const int p = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, parts = gridDim.x;
     const SpPart part = sp_part(V, parts, p);
     SpRow& R = rows[b];
-    float mx = R.pmax[0];
-    for (int q = 1; q < parts; ++q) mx = fmaxf(mx, R.pmax[q]);
+    float pm[SP_MAX_PARTS], mx = R.pmax[0];
+#pragma unroll
+    for (int q = 0; q < SP_MAX_PARTS; ++q) pm[q] = R.pmax[q];
+#pragma unroll
+    for (int q = 1; q < SP_MAX_PARTS; ++q) mx = q < parts ? fmaxf(mx, pm[q]) : mx;
     const float* s = scratch + (size_t)b * V + part.first;
     float* pr = scratch + ((size_t)n_rows + b) * V + part.first;
     sp_u64 mine = 0;
@@ -849,12 +867,9 @@ sp_mass_kernel(float* __restrict__ scratch, SpRow* __restrict__ rows, int V, int
         pr[i] = e;
         mine += sp_fixed(e);
     });
-    if (tid == 0) sh_total = 0;
-    __syncthreads();
-    atomicAdd(&sh_total, mine);
-    __syncthreads();
+    mine = block_sum_t<sp_u64>(mine, red_u);
     if (tid == 0) {
-        R.ptotal[p] = sh_total;
+        R.ptotal[p] = mine;
         if (p == 0) { R.t[0] = 0u; R.above[0] = 0; }
     }
     if (top_p < 1.0f) {
@@ -869,29 +884,37 @@ sp_mass_kernel(float* __restrict__ scratch, SpRow* __restrict__ rows, int V, int
 // The threshold after `level` + 1 digits, from the masses per digit that pass `level` left: the
 // largest digit at which the mass from the top reaches what top_p needs.  Every block of the next
 // pass finds it for itself; the first of a row writes it down for the passes after.
-__device__ __forceinline__ void sp_decide(SpRow& R, int parts, int level, float top_p, sp_u64* digit_mass,
-                                          uint32_t* t_out, sp_u64* above_out, bool write) {
+__device__ __forceinline__ void sp_decide(SpRow& R, int parts, int level, float top_p, uint32_t* t_out, sp_u64* above_out,
+                                          bool write) {
     __shared__ int sh_digit;
-    __shared__ sp_u64 sh_above;
-    const int tid = threadIdx.x, shift = 24 - 8 * level;
-    sp_u64 total = 0;
-    for (int q = 0; q < parts; ++q) total += R.ptotal[q];
+    __shared__ sp_u64 sh_above, quarter[4];              // mass of the digits of a wave
+    const int tid = threadIdx.x, shift = 24 - 8 * level, lane = tid & (ILLM_WAVE - 1), wave = tid / ILLM_WAVE;
+    const sp_u64 total = sp_over_parts(R.ptotal, 1, parts), above = R.above[level];
+    const uint32_t t = R.t[level];
     sp_u64 need = (sp_u64)((double)top_p * (double)total);
     need = need > 0 ? need : 1;
+    // the mass from digit `tid` up: within its wave by a scan, then the waves above (a thread that walked the digits above
+    // its own took up to 255 reads of LDS in a row: 5 of the 17 us of a pass)
+    sp_u64 m = 0, up = 0;
     if (tid < 256) {
-        sp_u64 m = 0;
-        for (int q = 0; q < parts; ++q) m += R.hist[level & 1][q][tid];
-        digit_mass[tid] = m;
+        m = up = sp_over_parts(&R.hist[level & 1][0][tid], 256, parts);
+#pragma unroll
+        for (int o = 1; o < ILLM_WAVE; o <<= 1) {
+            const sp_u64 y = __shfl_down(up, o, ILLM_WAVE);
+            up += lane + o < ILLM_WAVE ? y : 0;
+        }
+        if (lane == 0) quarter[wave] = up;
     }
-    if (tid == 0) { sh_digit = 0; sh_above = R.above[level]; }
+    if (tid == 0) { sh_digit = 0; sh_above = above; }
     __syncthreads();
     if (tid < 256) {
-        sp_u64 over = R.above[level];
-        for (int d = tid + 1; d < 256; ++d) over += digit_mass[d];
-        if (over < need && over + digit_mass[tid] >= need) { sh_digit = tid; sh_above = over; }
+        sp_u64 over = above + (up - m);
+#pragma unroll
+        for (int w = 1; w < 4; ++w) over += w > wave ? quarter[w] : 0;
+        if (over < need && over + m >= need) { sh_digit = tid; sh_above = over; }
     }
     __syncthreads();
-    *t_out = R.t[level] | ((uint32_t)sh_digit << shift);
+    *t_out = t | ((uint32_t)sh_digit << shift);
     *above_out = sh_above;
     if (write && tid == 0) { R.t[level + 1] = *t_out; R.above[level + 1] = sh_above; }
     __syncthreads();
@@ -902,13 +925,12 @@ __global__ void __launch_bounds__(SB)
 sp_digit_kernel(const float* __restrict__ scratch, SpRow* __restrict__ rows, int V, int n_rows,
                 float top_p, int level) {
     __shared__ sp_u64 mhist[SB / ILLM_WAVE][256];
-    __shared__ sp_u64 digit_mass[256];
     const int p = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, parts = gridDim.x;
     const SpPart part = sp_part(V, parts, p);
     SpRow& R = rows[b];
     uint32_t t;
     sp_u64 above;
-    sp_decide(R, parts, level - 1, top_p, digit_mass, &t, &above, p == 0);
+    sp_decide(R, parts, level - 1, top_p, &t, &above, p == 0);
     const float* s = scratch + (size_t)b * V + part.first;
     const float* pr = scratch + ((size_t)n_rows + b) * V + part.first;
     auto walk = [&](auto f) __attribute__((always_inline)) {
@@ -922,15 +944,14 @@ sp_digit_kernel(const float* __restrict__ scratch, SpRow* __restrict__ rows, int
 __global__ void __launch_bounds__(SB)
 sp_edge_kernel(const float* __restrict__ scratch, SpRow* __restrict__ rows, int V, int n_rows,
                float top_p) {
-    __shared__ sp_u64 digit_mass[256];
-    __shared__ sp_u64 sh_gt, sh_one;
-    __shared__ int sh_eq;
+    __shared__ sp_u64 sh_one, red_u[SB / ILLM_WAVE];
+    __shared__ int red_i[SB / ILLM_WAVE];
     const int p = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, parts = gridDim.x;
     const SpPart part = sp_part(V, parts, p);
     SpRow& R = rows[b];
     uint32_t t;
     sp_u64 above;
-    sp_decide(R, parts, 3, top_p, digit_mass, &t, &above, p == 0);
+    sp_decide(R, parts, 3, top_p, &t, &above, p == 0);
     const float* s = scratch + (size_t)b * V + part.first;
     const float* pr = scratch + ((size_t)n_rows + b) * V + part.first;
     sp_u64 gt = 0, one = 0;
@@ -940,13 +961,12 @@ sp_edge_kernel(const float* __restrict__ scratch, SpRow* __restrict__ rows, int 
         if (key > t) gt += sp_fixed(pr[i]);
         else if (key == t) { eq += 1; one = sp_fixed(pr[i]); }
     });
-    if (tid == 0) { sh_gt = 0; sh_one = 0; sh_eq = 0; }
-    __syncthreads();
-    atomicAdd(&sh_gt, gt);
-    atomicAdd(&sh_eq, eq);
+    if (tid == 0) sh_one = 0;
+    gt = block_sum_t<sp_u64>(gt, red_u);
+    const int n_eq = block_sum_t<int>(eq, red_i);
     if (eq) atomicMax(&sh_one, one);
     __syncthreads();
-    if (tid == 0) { R.mass_gt[p] = sh_gt; R.n_eq[p] = sh_eq; R.one_fx[p] = sh_one; }
+    if (tid == 0) { R.mass_gt[p] = gt; R.n_eq[p] = n_eq; R.one_fx[p] = sh_one; }
 }
 
 __global__ void __launch_bounds__(SB)
@@ -961,9 +981,19 @@ sp_draw_kernel(const float* __restrict__ scratch, const SpRow* __restrict__ rows
     const float* s = scratch + (size_t)b * V;
     const float* pr = scratch + ((size_t)n_rows + b) * V;
     const bool all = !(top_p < 1.0f);                    // every id stays
-    // (every thread works these few numbers out for itself)
-    sp_u64 total = 0;
-    for (int q = 0; q < parts; ++q) total += R.ptotal[q];
+    const uint64_t seed = seeds[b];                      // (possibly the host's memory: asked for ahead of the passes)
+    const int counter = counters[b];
+    // (every thread works these few numbers out for itself; the parts' fields loaded together)
+    const sp_u64 total = sp_over_parts(R.ptotal, 1, parts);
+    int eqs[SP_MAX_PARTS];
+    sp_u64 masses[SP_MAX_PARTS], ones[SP_MAX_PARTS];
+#pragma unroll
+    for (int q = 0; q < SP_MAX_PARTS; ++q) {
+        const bool has = q < parts;
+        eqs[q] = has && !all ? R.n_eq[q] : 0;
+        ones[q] = has && !all ? R.one_fx[q] : 0;
+        masses[q] = has ? (all ? R.ptotal[q] : R.mass_gt[q]) : 0;
+    }
     uint32_t t = 0;
     int cut = V, part_of_cut = parts, eq_in_cut_part = 0;
     sp_u64 one = 0, kept_total = total;
@@ -973,22 +1003,24 @@ sp_draw_kernel(const float* __restrict__ scratch, const SpRow* __restrict__ rows
         t = R.t[4];
         const sp_u64 above = R.above[4];
         int n_eq = 0;
-        for (int q = 0; q < parts; ++q) { n_eq += R.n_eq[q]; one = one ? one : R.one_fx[q]; }
+#pragma unroll
+        for (int q = 0; q < SP_MAX_PARTS; ++q) { n_eq += eqs[q]; one = one ? one : ones[q]; }
         // ids at the threshold key that stay: as many as still needed to reach top_p, the lowest ids
         long long m = one > 0 ? (long long)((need - above + one - 1) / one) : n_eq;
         m = m < 1 ? 1 : (m > n_eq ? n_eq : m);
         kept_total = above + (sp_u64)m * one;
         int before = 0;
-        for (int q = 0; q < parts; ++q) {
-            if (m > before && m <= before + R.n_eq[q]) { part_of_cut = q; eq_in_cut_part = (int)m - before; }
-            before += R.n_eq[q];
+#pragma unroll
+        for (int q = 0; q < SP_MAX_PARTS; ++q) {
+            if (m > before && m <= before + eqs[q]) { part_of_cut = q; eq_in_cut_part = (int)m - before; }
+            before += eqs[q];
         }
         // the id of that last one: the eq_in_cut_part-th id at the key in its part
         const SpPart part = sp_part(V, parts, part_of_cut);
         const int chunk = (part.n + SB - 1) / SB;
         const int lo = part.first + min(part.n, tid * chunk), hi = min(part.first + part.n, lo + chunk);
         int mine = 0;
-        for (int i = lo; i < hi; ++i) mine += order_key(s[i]) == t ? 1 : 0;
+        each_in_order8(s, lo, hi, [&](int, float v) { mine += order_key(v) == t ? 1 : 0; });
         int all_eq;
         const int bef = block_exclusive_scan<int>(mine, red_i, &all_eq);
         __syncthreads();
@@ -1003,13 +1035,13 @@ sp_draw_kernel(const float* __restrict__ scratch, const SpRow* __restrict__ rows
         cut = sh_i;
         __syncthreads();
     }
-    auto stays = [&](int i) {
-        if (all) return true;
-        const uint32_t key = order_key(s[i]);
-        return key > t || (key == t && i <= cut);
+    auto stays_as = [&](int i, float v) {
+        const uint32_t key = order_key(v);
+        return all || key > t || (key == t && i <= cut);
     };
+    auto stays = [&](int i) { return stays_as(i, s[i]); };
     // the part that holds the target, by the parts' kept masses in id order
-    const float u = uniform_from(seeds[b], counters[b]);
+    const float u = uniform_from(seed, counter);
     sp_u64 target = (sp_u64)((double)u * (double)kept_total);
     target = target < kept_total ? target : (kept_total ? kept_total - 1 : 0);
     int pt = parts - 1;
@@ -1017,11 +1049,11 @@ sp_draw_kernel(const float* __restrict__ scratch, const SpRow* __restrict__ rows
     {
         sp_u64 acc = 0;
         bool found = false;
-        for (int q = 0; q < parts; ++q) {
-            const sp_u64 km = all ? R.ptotal[q]
-                                  : R.mass_gt[q] + one * (sp_u64)(q < part_of_cut ? R.n_eq[q]
-                                                                  : (q == part_of_cut ? eq_in_cut_part : 0));
-            if (!found && target < acc + km) { pt = q; before_part = acc; found = true; }
+#pragma unroll
+        for (int q = 0; q < SP_MAX_PARTS; ++q) {
+            const int eq_kept = q < part_of_cut ? eqs[q] : (q == part_of_cut ? eq_in_cut_part : 0);
+            const sp_u64 km = masses[q] + (all ? 0 : one * (sp_u64)eq_kept);
+            if (!found && q < parts && target < acc + km) { pt = q; before_part = acc; found = true; }
             acc += km;
         }
     }
@@ -1030,8 +1062,14 @@ sp_draw_kernel(const float* __restrict__ scratch, const SpRow* __restrict__ rows
     const int chunk = (part.n + SB - 1) / SB;
     const int lo = part.first + min(part.n, tid * chunk), hi = min(part.first + part.n, lo + chunk);
     sp_u64 mine = 0;
-    for (int i = lo; i < hi; ++i)
-        if (stays(i)) mine += sp_fixed(pr[i]);
+    for (int base = lo; base < hi; base += 8) {
+        float v[8], e[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) { v[u] = all ? 0.f : s[min(base + u, hi - 1)]; e[u] = pr[min(base + u, hi - 1)]; }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (base + u < hi && stays_as(base + u, v[u])) mine += sp_fixed(e[u]);
+    }
     sp_u64 part_total;
     const sp_u64 bef = block_exclusive_scan<sp_u64>(mine, red_u, &part_total);
     __syncthreads();

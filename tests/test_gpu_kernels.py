@@ -2158,3 +2158,20 @@ def test_float32_qkv_rope_store_equals_the_three_steps(M, nh, nkv, hd, K, ring, 
     for a, b in zip(*caches):
         assert torch.equal(torch.isnan(a), torch.isnan(b)) and near(torch.nan_to_num(a), torch.nan_to_num(b))
     assert not o.qkv_rope_store_fits(x, w, hd + 4)
+
+
+@pytest.mark.parametrize("V", [1, 2, 1023, 1024, 1025, 2047, 2048, 2049])
+@pytest.mark.parametrize("top_k,top_p", [(0, 1.0), (0, 0.8), (1500, 0.9)])
+def test_sample_of_short_rows(V, top_k, top_p):
+    """Rows whose scores stay in LDS, one and two ids a thread, and the first that do not: each draw's interval of the kept
+    ids' distribution holds its number, equal scores and a score of minus infinity among them."""
+    B = 5
+    logits = rnd(B, V, seed=8, std=2.0)
+    logits[1] = 0.0
+    logits[2] = (logits[2] * 2).round() / 2
+    logits[3, V // 2:V - 1] = float("-inf")
+    seeds, counters = torch.tensor([3, 99, 12345, -7, 2**62], dtype=torch.int64), torch.arange(B, dtype=torch.int32)
+    got = ops().sample(logits.to(DEV), 0.9, top_k, top_p, 1.0, None, seeds.to(DEV), counters.to(DEV)).cpu().tolist()
+    for b in range(B):
+        u = R.uniform(int(seeds[b]) & ((1 << 64) - 1), b)
+        assert interval_ok(logits[b], got[b], u, 0.9, top_k, top_p, 1.0, None), (b, got[b], u)
