@@ -6,16 +6,19 @@ Tensors must live on the GPU: there is no CPU path, and a missing or unbuildable
 library raises (`kernels.build.KernelLibraryError`).  Parts call these through the
 module (`ops.add_rmsnorm(...)`).
 
-Matrix products: float32 operands always go to the library's own float32 kernel
-(plain fused multiply-adds, fixed summation order).  bfloat16 operands go to the
+Matrix products: float32 operands always go to the library's own float32 kernels
+(fixed summation order).  bfloat16 operands go to the
 MFMA kernels of this library when the shape fits them (few rows: decoding), and
 to the vendor GEMM through `torch.matmul` otherwise, which is where the reference
 uses a vendor GEMM too (cublasSgemm, src/kern/gpu/kernel_gpu.cu:420-435).
 
+Gate and up of 256 rows and more with their activation are an own kernel as well
+(csrc/gemm_turns.hip).
+
 Five things ride on the products.  `Weight`: a matrix with a second copy in the
 kernels' own tile order (`decode_weight`).  `linear_add` / `NormedRows`: the
 residual add in the product's epilogue and the RMS norm that follows it taken by
-the next product (up to 16 rows).  `linear_planes`: the product of up to 128 rows (from
+the next product (up to 16 rows, of float32 up to 4 or 8).  `linear_planes`: the product of up to 128 rows (from
 17, or from fewer where the plan says that pays) with a long thin matrix, K cut into
 ranges whose float32 planes `add_rmsnorm` adds.  `linear_rows`, and `qkv_rope_store` and
 `gate_up_silu` from 17 rows on (from fewer where the plan says): products of up to 64 (128)

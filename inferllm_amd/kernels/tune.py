@@ -20,16 +20,16 @@ import sys
 
 def matrices(engine):
     """Distinct bfloat16 matrices that the engine's parts list as having several ways
-    (`Part.tunables`), as (shape, `ops.Weight` or tensor)."""
+    (`Part.tunables`), as shape -> (kind, `ops.Weight` or tensor)."""
     import torch
 
     from . import ops
     seen = {}
     for part in engine.model.every_part():
-        for _kind, w, _geometry in part.tunables():
+        for kind, w, _geometry in part.tunables():
             plain = ops.plain_weight(w) if isinstance(w, (ops.Weight, torch.Tensor)) else None
             if plain is not None and plain.dim() == 2 and plain.dtype == torch.bfloat16:
-                seen.setdefault(tuple(plain.shape), w)
+                seen.setdefault(tuple(plain.shape), (kind, w))
     return seen
 
 
@@ -61,7 +61,7 @@ def tune_config(cfg: dict, max_rows: int, repeats: int, say, rows_only: bool = F
     rows = {k: v for k, v in plan.rows_from.items() if v != rules.rows_from}
     if rows_only:
         return planes, cuts, rows
-    for (N, K), w in sorted(matrices(eng).items()):
+    for (N, K), (kind, w) in sorted(matrices(eng).items(), key=lambda e: e[0]):
         plain = ops.plain_weight(w)
         for rows32 in range(rules.pad_rows_above // 32 + 1, rules.pad_rows_to // 32 + 1):
             M = min(rows32 * 32, rules.pad_rows_to - 1)
@@ -70,7 +70,7 @@ def tune_config(cfg: dict, max_rows: int, repeats: int, say, rows_only: bool = F
             best = max(set(votes), key=votes.count)
             if best:
                 cuts[("pad", rows32, N, K)] = best
-        if N < rules.cut_min_cols:
+        if N < rules.cut_min_cols or kind == "gate_up":      # (many rows of gate|up are one kernel with the activation)
             continue
         for rows256 in range(rules.cut_min_rows // 256, max_rows // 256 + 1):
             M = rows256 * 256
