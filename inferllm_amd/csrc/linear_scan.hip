@@ -219,39 +219,17 @@ extern "C" int illm_ssm_finish(const float* o, const float* x, const float* D, c
 }
 
 // ---------------------------------------------------------------- matrix memory
-// grid (rows, ceil(max(H dk, H (dv + 1)) / 256)); 256 threads, an entry of q, k and v each (a block a row, which
-// went through them one after another, took 9.3 us for 8 rows of 2,048, this 4.7).
-// U [T, u_stride] = [q (H dk) | k (H dk) | v (H dv) | ...].
-template <int DT>
-__global__ void __launch_bounds__(256)
-memory_rows_kernel(const void* __restrict__ U, int u_stride, float* __restrict__ qn,
-                   float* __restrict__ kn, float* __restrict__ vv, int H, int dk, int dv, float qscale) {
-    const size_t r = blockIdx.x;
-    const int nq = H * dk, nv = H * (dv + 1), i = blockIdx.y * 256 + threadIdx.x;
-    const int h = i / (dv + 1), j = i - h * (dv + 1);
-    float q = 0.f, k = 0.f, v = 1.0f;
-    if (i < nq) {
-        q = ld_f(U, DT, r * u_stride + i);
-        k = ld_f(U, DT, r * u_stride + nq + i);
-    }
-    if (i < nv && j < dv) v = ld_f(U, DT, r * u_stride + 2 * nq + h * dv + j);
-    if (i < nq) {
-        qn[r * nq + i] = q * qscale;
-        kn[r * nq + i] = k;
-    }
-    if (i < nv) vv[r * nv + i] = v;
-}
-
-// grid (sequences, H); one wave.  64 tokens at a time: every lane forms its token's two gates, then
+// The gates of sequence b and head h, one wave.  64 tokens at a time: every lane forms its token's two gates, then
 // the running maximum goes through the 64 tokens in order (the lanes' values are read one after the
 // other as scalars), and every lane leaves its token's decay, weight and exp(-m).
-__global__ void __launch_bounds__(64)
-memory_gates_kernel(const void* __restrict__ U, int dt, int u_stride, int i_off, int f_off,
+template <int DT>
+static __device__ __forceinline__ void
+memory_gates(int b, int h, const void* __restrict__ U, int u_stride, int i_off, int f_off,
                     const float* __restrict__ i_bias, const float* __restrict__ f_bias, float cap,
                     float* __restrict__ m_state, const int32_t* __restrict__ cu,
                     const int32_t* __restrict__ seq_slot, float* __restrict__ beta,
                     float* __restrict__ dec, float* __restrict__ em, int H) {
-    const int b = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
     const int r0 = cu[b], n = cu[b + 1] - r0;
     if (n <= 0) return;
     const int slot = seq_slot[b];
@@ -260,8 +238,8 @@ memory_gates_kernel(const void* __restrict__ U, int dt, int u_stride, int i_off,
     for (int t0 = 0; t0 < n; t0 += 64) {
         const bool ok = t0 + lane < n;
         const size_t row = (size_t)(r0 + (ok ? t0 + lane : n - 1));
-        const float ig = ok ? cap * tanhf((ld_f(U, dt, row * u_stride + i_off + h) + bi) * inv_cap) : -INFINITY;
-        const float fg = ok ? ls_log_sigmoid(cap * tanhf((ld_f(U, dt, row * u_stride + f_off + h) + bf) * inv_cap)) : 0.f;
+        const float ig = ok ? cap * tanhf((ld_f(U, DT, row * u_stride + i_off + h) + bi) * inv_cap) : -INFINITY;
+        const float fg = ok ? ls_log_sigmoid(cap * tanhf((ld_f(U, DT, row * u_stride + f_off + h) + bf) * inv_cap)) : 0.f;
         float m_before = 0.f, m_mine = 0.f;
         const int tokens = min(64, n - t0);             // (all 64 turns took 6 us of a single token's step)
         for (int l = 0; l < tokens; ++l) {
@@ -280,6 +258,43 @@ memory_gates_kernel(const void* __restrict__ U, int dt, int u_stride, int i_off,
     if (lane == 0) m_state[(size_t)slot * H + h] = m;
 }
 
+// grid (gate blocks + rows, ceil(max(H dk, H (dv + 1)) / 256)); 256 threads, an entry of q, k and v each (a block a row, which
+// went through them one after another, took 9.3 us for 8 rows of 2,048, this 4.7).  The first blocks of the grid's first row
+// take four (sequence, head) pairs' gates each, which need nothing of the rest: as a kernel behind the
+// rows -> beside them, 16 heads of 128 x 128, 1 / 8 / 64 single tokens 5.0 / 4.6 / 5.1 -> 3.7 / 4.0 / 3.6 us, 8 sequences of 61 to
+// 1,024 tokens 87.9 -> 67.6, one of 2,048 147 -> 129 (the gates' chain of tokens bounds these).
+// U [T, u_stride] = [q (H dk) | k (H dk) | v (H dv) | ...].
+template <int DT>
+__global__ void __launch_bounds__(256)
+memory_prepare_kernel(const void* __restrict__ U, int u_stride, float* __restrict__ qn,
+                      float* __restrict__ kn, float* __restrict__ vv, int H, int dk, int dv, float qscale, int gate_blocks,
+                      int n_seqs, int i_off, int f_off, const float* __restrict__ i_bias, const float* __restrict__ f_bias,
+                      float cap, float* __restrict__ m_state, const int32_t* __restrict__ cu,
+                      const int32_t* __restrict__ seq_slot, float* __restrict__ beta, float* __restrict__ dec,
+                      float* __restrict__ em) {
+    if ((int)blockIdx.x < gate_blocks) {
+        const int unit = blockIdx.x * 4 + wave_index();
+        if (blockIdx.y == 0 && unit < n_seqs * H)
+            memory_gates<DT>(unit / H, unit % H, U, u_stride, i_off, f_off, i_bias, f_bias, cap, m_state, cu, seq_slot, beta,
+                             dec, em, H);
+        return;
+    }
+    const size_t r = blockIdx.x - gate_blocks;
+    const int nq = H * dk, nv = H * (dv + 1), i = blockIdx.y * 256 + threadIdx.x;
+    const int h = i / (dv + 1), j = i - h * (dv + 1);
+    float q = 0.f, k = 0.f, v = 1.0f;
+    if (i < nq) {
+        q = ld_f(U, DT, r * u_stride + i);
+        k = ld_f(U, DT, r * u_stride + nq + i);
+    }
+    if (i < nv && j < dv) v = ld_f(U, DT, r * u_stride + 2 * nq + h * dv + j);
+    if (i < nq) {
+        qn[r * nq + i] = q * qscale;
+        kn[r * nq + i] = k;
+    }
+    if (i < nv) vv[r * nv + i] = v;
+}
+
 extern "C" int illm_memory_prepare(const void* U, int dt, int u_stride, int i_off, int f_off,
                                    const float* i_bias, const float* f_bias, float cap, float* m_state,
                                    const int32_t* cu, const int32_t* seq_slot, float* qn, float* kn,
@@ -292,16 +307,16 @@ extern "C" int illm_memory_prepare(const void* U, int dt, int u_stride, int i_of
     if (T == 0 || n_seqs == 0) return ILLM_OK;
     const int widest = H * dk > H * (dv + 1) ? H * dk : H * (dv + 1);
     if ((widest + 255) / 256 > 65535) return ILLM_ERR_ARG;
-    const dim3 grid(T, (widest + 255) / 256);
-    if (dt == ILLM_BF16)
-        hipLaunchKernelGGL(memory_rows_kernel<ILLM_BF16>, grid, dim3(256), 0, (hipStream_t)stream, U, u_stride, qn,
-                           kn, vv, H, dk, dv, 1.0f / sqrtf((float)dk));
-    else
-        hipLaunchKernelGGL(memory_rows_kernel<ILLM_F32>, grid, dim3(256), 0, (hipStream_t)stream, U, u_stride, qn,
-                           kn, vv, H, dk, dv, 1.0f / sqrtf((float)dk));
-    if (hipGetLastError() != hipSuccess) return ILLM_ERR_LAUNCH;
-    hipLaunchKernelGGL(memory_gates_kernel, dim3(n_seqs, H), dim3(64), 0, (hipStream_t)stream, U, dt,
-                       u_stride, i_off, f_off, i_bias, f_bias, cap, m_state, cu, seq_slot, beta, dec, em, H);
+    const long long gate_blocks = ((long long)n_seqs * H + 3) / 4;
+    if (gate_blocks * 4 > 0x7fffffff || gate_blocks + T > 0x7fffffff) return ILLM_ERR_ARG;
+    const dim3 grid((unsigned)(gate_blocks + T), (widest + 255) / 256);
+#define ILLM_MEMORY_PREPARE(DT)                                                                                     \
+    hipLaunchKernelGGL(memory_prepare_kernel<DT>, grid, dim3(256), 0, (hipStream_t)stream, U, u_stride, qn, kn, vv, H, dk, dv, \
+                       1.0f / sqrtf((float)dk), (int)gate_blocks, n_seqs, i_off, f_off, i_bias, f_bias, cap, m_state, cu, \
+                       seq_slot, beta, dec, em)
+    if (dt == ILLM_BF16) ILLM_MEMORY_PREPARE(ILLM_BF16);
+    else ILLM_MEMORY_PREPARE(ILLM_F32);
+#undef ILLM_MEMORY_PREPARE
     return illm_launch_status();
 }
 

@@ -452,6 +452,29 @@ def test_matrix_memory_kernels_against_plain_torch(dtype):
         _near(got, want, 1e-5)
 
 
+@pytest.mark.parametrize("H,dk,dv,lens", [(5, 130, 100, [0, 3, 0, 0, 70, 1] + [0] * 25), (1, 8, 8, [1]), (7, 300, 4, [2, 129])])
+def test_matrix_memory_gates_beside_the_rows(H, dk, dv, lens):
+    """Gates and rows are blocks of one kernel: more gate blocks than rows, sequences without rows (whose maxima stay), counts
+    of (sequence, head) pairs that do not fill a block, several blocks a row."""
+    from inferllm_amd.kernels import ops
+    g = torch.Generator().manual_seed(11)
+    T, n = sum(lens), len(lens)
+    slots = torch.randperm(n + 2, generator=g)[:n].tolist()
+    cu, seq_slot, _ = _packed(lens, slots)
+    i_off = 2 * H * dk + H * dv
+    U = (torch.randn(T, i_off + 2 * H, generator=g) * 2).to(torch.bfloat16)
+    i_bias, f_bias, m = torch.randn(H, generator=g), torch.randn(H, generator=g) + 1, torch.randn(n + 2, H, generator=g)
+    m_want, m_got = m.clone(), m.cuda()
+    want = R.memory_prepare(U, i_off, i_off + H, i_bias, f_bias, 3.0, m_want, cu, seq_slot, n, H, dk, dv)
+    got = ops.memory_prepare(U.cuda(), i_off, i_off + H, i_bias.cuda(), f_bias.cuda(), 3.0, m_got, cu.cuda(), seq_slot.cuda(),
+                             n, H, dk, dv)
+    for a, b in zip(got, want):
+        _near(a, b, 1e-5)
+    _near(m_got, m_want, 1e-5)
+    for s, rows in zip(slots, lens):
+        assert rows or torch.equal(m_got[s].cpu(), m[s])
+
+
 @pytest.mark.parametrize("matrix_cores", [1, 2, 0])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_with_bias_chunks_and_gate_against_plain_torch(dtype, matrix_cores):
