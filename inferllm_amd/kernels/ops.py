@@ -30,7 +30,9 @@ nothing depends on a stopwatch).
 """
 from __future__ import annotations
 
+import collections
 import ctypes
+import threading
 from typing import Dict, List, Optional, Tuple
 
 import torch
@@ -3149,11 +3151,40 @@ _sample_long_row_bytes = 0        # ILLM_SAMPLE_LONG_ROW_BYTES of csrc/api.h, as
 def sample(logits: torch.Tensor, temperature: float, top_k: int, top_p: float,
            repeat_penalty: float, last_tokens: Optional[torch.Tensor], seeds: torch.Tensor,
            counters: torch.Tensor) -> torch.Tensor:
-    """One draw per row; see csrc/sampling.hip.  seeds: int64 [B] (bit pattern used), counters int32 [B], both on the
-    device or in pinned memory, which the kernel reads (and the caller leaves as it is until it has run)."""
-    _gpu(logits, last_tokens)
+    """One draw per row; see csrc/sampling.hip.  seeds: int64 [B] (bit pattern used), counters int32 [B]."""
+    _gpu(logits, last_tokens, seeds, counters)
+    return _sample(logits, temperature, top_k, top_p, repeat_penalty, last_tokens, seeds, counters)
+
+
+def sample_from_host(logits: torch.Tensor, temperature: float, top_k: int, top_p: float, seeds: torch.Tensor,
+                     counters: torch.Tensor) -> torch.Tensor:
+    """`sample` without a window of last tokens, the seeds and counters in pinned memory, where the kernel reads them.  The
+    memory is kept until the kernel has run, whoever lets go of it; what it holds the caller leaves as it is until then."""
+    _gpu(logits)
     for t in (seeds, counters):
-        _need(t.is_contiguous() and (t.is_cuda or t.is_pinned()), "sample: seeds and counters on the device or in pinned memory")
+        _need(t.is_contiguous() and t.is_pinned(), "sample_from_host: seeds and counters in pinned memory")
+    _need(not torch.cuda.is_current_stream_capturing(), "sample_from_host: a graph would read the numbers again")
+    out = _sample(logits, temperature, top_k, top_p, 1.0, None, seeds, counters)
+    keep_until_run(seeds, counters)
+    return out
+
+
+_kept: collections.deque = collections.deque()     # (event behind a kernel, the host memory that it reads), oldest first
+_kept_lock = threading.Lock()
+
+
+def keep_until_run(*tensors: torch.Tensor) -> None:
+    """Hold the tensors until the current stream has done what it was given so far.  (torch's pinned memory is free as soon
+    as its last tensor goes, unless torch itself has queued a copy of it.)"""
+    event = torch.cuda.Event()
+    record(event)
+    with _kept_lock:
+        while _kept and _kept[0][0].query():
+            _kept.popleft()
+        _kept.append((event, tensors))
+
+
+def _sample(logits, temperature, top_k, top_p, repeat_penalty, last_tokens, seeds, counters) -> torch.Tensor:
     _need(logits.dtype == torch.float32 and logits.dim() == 2, "sample: float32 [B, V]")
     B, V = logits.shape
     _need(seeds.dtype == torch.int64 and seeds.numel() >= B, "sample: seeds int64 [B]")

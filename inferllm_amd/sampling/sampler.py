@@ -41,6 +41,7 @@ class Sampler:
         params.validate()
         self.params = params
         self.device = device
+        self._pinned = torch.device(device).type == "cuda"
         # pinned [seeds (2 words each) | counters | windows], four in turn: a draw's numbers may
         # still wait for their copy when the next draw's are written
         self._stages: List[Optional[torch.Tensor]] = [None] * 4
@@ -50,16 +51,16 @@ class Sampler:
 
     def _upload(self, seeds, counters, windows):
         """One pinned buffer: (seeds int64 [B], counters int32 [B], windows int32 [B, n] or None).  Without windows the
-        kernel reads the few numbers where they are (a copy takes 10 us of the host and 3 of the device); with them one
-        copy brings everything over."""
+        kernel reads the few numbers where they are (a copy takes 10 us of the host and 3 of the device), and the buffer is
+        kept until it has, also where this sampler goes first (`ops.sample_from_host`); with them one copy brings
+        everything over."""
         B = len(seeds)
         n = len(windows[0]) if windows else 0
         words = B * (3 + n)
         stage = self._stages[self._turn]
         if stage is None or stage.numel() < words:
             stage = self._stages[self._turn] = torch.empty(
-                max(words, 1024), dtype=torch.int32,
-                pin_memory=torch.device(self.device).type == "cuda")
+                max(words, 1024), dtype=torch.int32, pin_memory=self._pinned)
         host = stage[:words]
         flat = host.numpy()                              # shares the pinned memory
         flat[:2 * B].view(np.int64)[:] = [_as_i64(int(s)) for s in seeds]
@@ -101,8 +102,11 @@ class Sampler:
             seeds_t, counters_t, last = self._upload(seeds, counters, rows)
             if last is not None and latest is not None:
                 last[:, -1].copy_(latest)
-            dev = ops.sample(logits.contiguous(), p.temperature, p.top_k, p.top_p,
-                             p.repeat_penalty, last, seeds_t, counters_t)
+            if last is None and self._pinned:
+                dev = ops.sample_from_host(logits.contiguous(), p.temperature, p.top_k, p.top_p, seeds_t, counters_t)
+            else:
+                dev = ops.sample(logits.contiguous(), p.temperature, p.top_k, p.top_p,
+                                 p.repeat_penalty, last, seeds_t, counters_t)
         B = dev.numel()
         if not dev.is_cuda:                  # stand-in kernels on the CPU (tests): nothing to wait for
             return Draw(dev, dev, None)

@@ -2175,3 +2175,27 @@ def test_sample_of_short_rows(V, top_k, top_p):
     for b in range(B):
         u = R.uniform(int(seeds[b]) & ((1 << 64) - 1), b)
         assert interval_ok(logits[b], got[b], u, 0.9, top_k, top_p, 1.0, None), (b, got[b], u)
+
+
+@pytest.mark.parametrize("V, top_p", [(300, 1.0), (5000, 0.9), (20000, 0.95)])
+def test_draws_outlive_their_samplers(V, top_p):
+    """Samplers that go as soon as their draw is under way, behind work that is not done, and pinned buffers of the same size
+    that are written at once: the draws use the seeds that they were given."""
+    from inferllm_amd.sampling import Sampler, SamplingParams
+    logits, params = rnd(8, V, seed=3).to(DEV), SamplingParams(temperature=1.5, top_p=top_p)
+    want, kept = [], []
+    for i in range(8):
+        kept.append(Sampler(params, DEV))
+        want.append(kept[-1](logits, list(range(100 * i, 100 * i + 8)), [i] * 8))
+    a = torch.randn(4096, 4096, device=DEV)
+    torch.cuda.synchronize()
+    for _ in range(20):
+        b = a @ a
+    draws, others = [], []
+    for i in range(8):
+        draws.append(Sampler(params, DEV).draw(logits, list(range(100 * i, 100 * i + 8)), [i] * 8))
+        others.append(torch.empty(1024, dtype=torch.int32, pin_memory=True).fill_(7))
+    assert [d.tokens() for d in draws] == want and b.shape == a.shape
+    with pytest.raises(Exception):
+        ops().sample(logits, 1.0, 0, 1.0, 1.0, None, torch.zeros(8, dtype=torch.int64, pin_memory=True),
+                     torch.zeros(8, dtype=torch.int32, device=DEV))

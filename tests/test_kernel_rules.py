@@ -119,3 +119,50 @@ def test_the_cut_product_refuses_float32_rows_with_another_matrix(monkeypatch):
             ops.linear_cut(x, w)
     for splits, planes in ((0, 4), (1, 1), (3, 3)):
         assert ops.linear_cut(x, torch.zeros(1024, 2048), splits).shape == (planes, 140, 1024)
+
+
+def test_a_draw_keeps_the_numbers_that_its_kernel_reads(monkeypatch):
+    """Seeds and counters in pinned memory are there until the kernel that reads them has run, also where the sampler and
+    the draw are gone before: here a buffer is let go of once the event behind its kernel has passed, and no sooner."""
+    import gc
+    import weakref
+
+    import numpy as np
+
+    from inferllm_amd.sampling import Sampler, SamplingParams
+    events = []
+
+    class event:
+        def __init__(self):
+            self.passed = False
+            events.append(self)
+
+        def query(self):
+            return self.passed
+
+    class library:
+        @staticmethod
+        def illm_sample(*a):
+            return 0
+    monkeypatch.setattr(torch.cuda, "Event", event)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.Tensor, "is_pinned", lambda t: True)
+    monkeypatch.setattr(ops, "record", lambda e: None)
+    monkeypatch.setattr(ops, "_gpu", lambda *t: None)
+    monkeypatch.setattr(ops, "_lib", lambda: library)
+    monkeypatch.setattr(ops, "_stream", lambda: None)
+    refs = []
+    for i in range(3):
+        sampler, numbers = Sampler(SamplingParams(temperature=0.8), "cuda:0"), np.zeros(1024, np.int32)
+        sampler._stages = [torch.from_numpy(numbers)] * 4
+        refs.append(weakref.ref(numbers))
+        sampler.draw(torch.zeros(2, 8), [1, 2], [0, 0])
+        del sampler, numbers
+        gc.collect()
+        assert [r() is not None for r in refs] == ([True], [True, True], [False, True, True])[i]
+        events[0].passed = i == 1
+    events[1].passed = events[2].passed = True
+    ops.keep_until_run(torch.zeros(1))
+    gc.collect()
+    assert [r() for r in refs] == [None] * 3
+    ops._kept.clear()
