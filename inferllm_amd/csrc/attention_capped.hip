@@ -1320,6 +1320,11 @@ attn_cap_decode_keys16_kernel(const bf16_t* __restrict__ q, int q_stride, const 
     float acc[DH][2], m = NEG_INF, l = 0.f;
 #pragma unroll
     for (int i = 0; i < DH; ++i) acc[i][0] = acc[i][1] = 0.f;
+    // (weights[w] goes between the lanes of one wave, whose LDS accesses run in program order: a fence for the compiler alone)
+    auto in_order = []() __attribute__((always_inline)) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     auto round = [&](const Rows& x, int base) __attribute__((always_inline)) {
         cap_f32x4_t s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1341,6 +1346,7 @@ attn_cap_decode_keys16_kernel(const bf16_t* __restrict__ q, int q_stride, const 
         // (the hardware's exponential: float32 with an error of |x| 2^-24)
         const float alpha = m_new == NEG_INF ? 1.f : __expf(m - m_new);
         float sum = 0.f;
+        in_order();
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float p = base + 4 * g + i < k_hi ? __expf(s[i] - m_new) : 0.f;
@@ -1348,6 +1354,7 @@ attn_cap_decode_keys16_kernel(const bf16_t* __restrict__ q, int q_stride, const 
             if (r < DH) weights[w][4 * g + i][r] = p;
         }
         if (r < DH && g == 0) weights[w][16][r] = alpha;
+        in_order();
         two = cap_swap16(sum);
         two = cap_swap32(two.x + two.y);
         l = l * alpha + (two.x + two.y);

@@ -44,3 +44,14 @@ def test_the_float32_parts_loads_are_issued_in_the_order_their_waits_count(tmp_p
         assert stages[1:] == [x + w] * 3, (mt, nt, ns, stages)
         counts = re.findall(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)\s*\n\s*s_barrier", body)
         assert counts and set(counts) == {str((ns - 2) * len(x + w))}, (mt, nt, ns, counts)
+
+
+def test_what_lanes_of_a_wave_hand_each_other_through_lds_is_fenced_for_the_compiler():
+    """The softmax's weights go from some lanes of a wave to all of them, with no barrier: the compiler, to which a lane's
+    loads are its own, is told by a fence before a round's stores and another between them and the loads."""
+    body = re.search(r"^attn_cap_decode_keys16_kernel\(.*?^}", SOURCES["attention_capped.hip"], re.S | re.M).group(0)
+    fence = re.search(r"auto (\w+) = \[\]\(\)[^{]*{([^}]*)}", body)
+    assert '__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront")' in fence.group(2)
+    assert "__builtin_amdgcn_wave_barrier()" in fence.group(2)
+    uses = re.findall(r"weights\[w\][^;=]*(=?)|" + fence.group(1) + r"(\(\));", body[fence.end():])
+    assert "".join("S" if store else "F" if call else "L" for store, call in uses) == "FSSFLL"
