@@ -11,10 +11,17 @@
 #include "api.h"
 #include "gemm_turns.h"
 
-// 1 / (1 + e^-z) by the hardware's exponential and reciprocal, each within 1 in the last place of float32: nothing is
-// under way on the matrix cores while a tile's results are formed, and by expf and a division they took 8 us of a round's 88.
-__device__ __forceinline__ float turns_sigmoid(float z) {
-    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
+// g / (1 + e^-(alpha g)), within 2 in the last place of float32 wherever the result is a normal number (expf and a division
+// 1.5): e^x as 2^(x log2 e) with the product's rounding and log2 e's taken along, and the denominator's quarter, so that
+// the reciprocal of a sum of up to 2^128 is no subnormal number, which the hardware makes zero.  Nothing is under way on the
+// matrix cores while a tile's results are formed: us of 2 x 11008 x 4096, 500 / 2,048 rows, by expf and a division 92.2 / 279,
+// by this 89.3 / 271, by a plain product, exponential and reciprocal (9 in the last place at -20, zero below -87.3) 87.8 / 266.
+__device__ __forceinline__ float turns_gated(float g, float alpha) {
+    const float z = fminf(fmaxf(alpha * g, -128.0f), 128.0f);          // (beyond: e^-z is infinite or nothing beside 1)
+    const float h = -1.44269502f * z;
+    const float rest = fmaf(-1.44269502f, z, -h) - 1.92596299e-8f * z;
+    const float d = 0.25f + 0.25f * (__builtin_amdgcn_exp2f(h) * fmaf(rest, 0.693147182f, 1.0f));
+    return (0.25f * g) * __builtin_amdgcn_rcpf(d);
 }
 
 struct TileAt { int m, n; };
@@ -104,7 +111,7 @@ gemm_turns_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, bf
                     const float g = t.acc[i][j][e], u = t.acc[NTH + i][j][e];
                     const float gc = limit > 0.f ? fminf(g, limit) : g;
                     const float uc = limit > 0.f ? fminf(fmaxf(u, -limit), limit) + 1.0f : u;
-                    v[e] = gc * turns_sigmoid(alpha * gc) * uc;
+                    v[e] = turns_gated(gc, alpha) * uc;
                 }
                 o[2 * i] = pack_bf16x2(v[0], v[1]);
                 o[2 * i + 1] = pack_bf16x2(v[2], v[3]);

@@ -2199,3 +2199,21 @@ def test_draws_outlive_their_samplers(V, top_p):
     with pytest.raises(Exception):
         ops().sample(logits, 1.0, 0, 1.0, 1.0, None, torch.zeros(8, dtype=torch.int64, pin_memory=True),
                      torch.zeros(8, dtype=torch.int32, device=DEV))
+
+
+def test_gates_far_below_zero_in_turns():
+    """g / (1 + e^-g) up is a normal number until e^-g is infinite: gates down to -88.5 by tiles in turns, and a limit's
+    slope of 1.702, against 64 bits within the result's rounding (2^-8 where a power of two begins) and float32's."""
+    o, lib = ops(), ops()._lib()
+    M, F, K = 5, 264, 128
+    gates = torch.linspace(-88.5, 40.0, F).mul(2 / K).bfloat16().mul(K / 2)      # exact sums of K / 2 equal products
+    w = torch.zeros(2 * F, K)
+    w[:F, ::2], w[F:, 1] = (gates / (K / 2))[:, None], 1.0
+    x, w, y = torch.ones(M, K, dtype=torch.bfloat16, device=DEV), w.bfloat16().to(DEV), torch.empty(M, F, dtype=torch.bfloat16, device=DEV)
+    for limit, slope, up in ((0.0, 1.0, 1.0), (50.0, 1.702, 2.0)):
+        assert lib.illm_gemm_turns_gate_up(o._p(x), o._p(w), o._p(y), M, F, K, limit, 1.702, None) == 0
+        z = gates.double() * torch.tensor(slope).double()
+        want = gates.double() / (1 + torch.exp(-z)) * up
+        want[torch.exp(-z.float()).isinf()] = 0.0
+        assert float(want[0].abs()) > 1e-37 or slope > 1
+        assert bool(((y.double().cpu() - want).abs() <= (2.0 ** -8 + 2e-5) * want.abs()).all())
