@@ -8,7 +8,10 @@
 // both products (us, in turn on one card): 2 x 14336 x 4096 of 9,061 rows 1,580 -> 1,470, of 512 109 -> 100; 2 x 11008 x 4096
 // of 9,061 / 2,048 / 500 rows 1,274 / 294 / 94 -> 1,172 / 286 / 89 (1.4 PFLOP/s, 688 tiles or 2.7 rounds of 256, one
 // round of 172); 2 x 5376 x 2048 of 2,964 rows 117 -> 106.  What bounds the large ones is the chip's power.
+#include <algorithm>
+
 #include "api.h"
+#include "api_test.h"
 #include "gemm_turns.h"
 
 // g / (1 + e^-(alpha g)), within 2 in the last place of float32 wherever the result is a normal number (expf and a division
@@ -124,18 +127,29 @@ gemm_turns_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, bf
     t.end();
 }
 
+static const struct { int m, n, cost; } TURNS_SHAPES[4] = {{256, 256, 88}, {192, 256, 73}, {128, 256, 59}, {256, 128, 58}};
+
+static long long turns_tiles(int M, int F, int shape) {
+    const auto s = TURNS_SHAPES[shape];
+    return ((long long)M + s.m - 1) / s.m * ((2LL * F + s.n - 1) / s.n);
+}
+
 // Tiles of 256 x 256, 192 x 256, 128 x 256 or 256 x 128 rows of X and of W: the least of rounds of 256 blocks times a
 // round's time (K = 4,096, us: 88, 73, 59 and 58).
 static int turns_shape(int M, int F) {
-    static const struct { int m, n, cost; } SHAPES[4] = {{256, 256, 88}, {192, 256, 73}, {128, 256, 59}, {256, 128, 58}};
     int best = 0;
     long long least = -1;
     for (int i = 0; i < 4; ++i) {
-        const long long tiles = ((long long)M + SHAPES[i].m - 1) / SHAPES[i].m * ((2LL * F + SHAPES[i].n - 1) / SHAPES[i].n);
-        const long long cost = (tiles + 255) / 256 * SHAPES[i].cost;
+        const long long cost = (turns_tiles(M, F, i) + 255) / 256 * TURNS_SHAPES[i].cost;
         if (least < 0 || cost < least) { best = i; least = cost; }
     }
     return best;
+}
+
+extern "C" int illm_gemm_turns_tiles(int M, int F, int* shape) {
+    const int s = turns_shape(M, F);
+    if (shape) *shape = s;
+    return (int)std::min(turns_tiles(M, F, s), 0x7fffffffLL);
 }
 
 // X [M, K], W [2 F, K] = [gate | up], Y [M, F], bfloat16 on 16-byte addresses, K % 128 == 0, F % 8 == 0.
@@ -146,13 +160,14 @@ extern "C" int illm_gemm_turns_gate_up(const void* X, const void* W, void* Y, in
         return ILLM_ERR_ARG;
     if (!(limit > 0.f)) alpha = 1.0f;
 #define ILLM_TURNS(I, MT0, MT1, NTH)                                                                                     \
-    case I: {                                                                                                            \
-        const long long tiles = (M + 32LL * (MT0 + MT1) - 1) / (32 * (MT0 + MT1)) * ((2LL * F + 128 * NTH - 1) / (128 * NTH)); \
-        if (tiles > 0x3fffffff) return ILLM_ERR_ARG;                                                                     \
+    case I:                                                                                                              \
         hipLaunchKernelGGL((gemm_turns_kernel<MT0, MT1, NTH>), dim3((unsigned)(tiles < 256 ? tiles : 256)), dim3(512), 0, \
                            (hipStream_t)stream, (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, M, F, K, limit, alpha);  \
-    } break
-    switch (turns_shape(M, F)) {
+        break
+    const int shape = turns_shape(M, F);
+    const long long tiles = turns_tiles(M, F, shape);
+    if (tiles > 0x3fffffff) return ILLM_ERR_ARG;
+    switch (shape) {
         ILLM_TURNS(0, 4, 4, 2);
         ILLM_TURNS(1, 4, 2, 2);
         ILLM_TURNS(2, 2, 2, 2);

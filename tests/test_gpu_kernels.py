@@ -2044,12 +2044,19 @@ def test_sum_of_two_products_of_few_rows(N, K, K2):
     assert not o.linear_sum_fits(o.Product(x, w), o.Product(x2, b)) and not o.linear_sum_fits(o.Product(x[:4], a), o.Product(x2, b))
 
 
-@pytest.mark.parametrize("M, F, K", [(1, 8, 128), (129, 136, 256), (257, 264, 384), (300, 2184, 128), (700, 40, 1024), (2100, 2056, 256)])
-def test_gate_up_of_many_rows_in_turns(M, F, K):
-    """Gate and up with their activation over tiles in turns: less than a tile and remainders along both sides, one stage
-    pair of K and more, more tiles than blocks (so that loads run on into the next tile), infinities that stay in their rows
-    and columns; the same rows have the same bits in every shape of tiles (other numbers of rows)."""
+@pytest.mark.parametrize("M, F, K, shape, tiles", [
+    (1, 8, 128, 3, 1), (129, 136, 256, 3, 3), (257, 264, 384, 3, 10), (300, 2184, 128, 3, 70), (700, 40, 1024, 3, 3),
+    (2100, 2056, 256, 1, 187), (500, 11008, 128, 0, 172), (300, 8328, 256, 2, 198), (1281, 10256, 384, 0, 486),
+    (2313, 8200, 128, 0, 650), (2050, 11016, 128, 1, 957), (520, 10888, 128, 2, 430), (1000, 11016, 256, 3, 692)])
+def test_gate_up_of_many_rows_in_turns(M, F, K, shape, tiles):
+    """Gate and up with their activation over tiles in turns: every shape of tiles, less than a tile and remainders along both
+    sides, one stage pair of K and more, two rounds of 256 blocks and more in every shape (so that loads run on into the next
+    tile), infinities that stay in their rows and columns; the same rows have the same bits in every shape of tiles (other
+    numbers of rows)."""
+    import ctypes
     o, lib = ops(), ops()._lib()
+    found = ctypes.c_int(-1)
+    assert (lib.illm_gemm_turns_tiles(M, F, ctypes.byref(found)), found.value) == (tiles, shape)
     x = rnd(M, K, dtype=torch.bfloat16, seed=1).to(DEV)
     w = (rnd(2 * F, K, seed=2) * K ** -0.5).to(torch.bfloat16).to(DEV)
 
