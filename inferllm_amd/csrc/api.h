@@ -141,7 +141,7 @@ int illm_gemv_rows_f32(const float* X, const float* W, void* Y, int y_dt, int M,
 int illm_gemv_rows_f32_fused(const float* X, const float* W, float* Y, int M, int N, int K, const float* norm_w,
                              float eps, int epi, float limit, float alpha, void* stream);
 int illm_gemv_qkv_f32(const float* X, const float* W, float* Y, int M, int K, const float* norm_w, float eps,
-                      const float* cos_sin, const int32_t* row_pos, const int32_t* row_slot, float* kcache,
+                      const float* cos_sin, int max_pos, const int32_t* row_pos, const int32_t* row_slot, float* kcache,
                       float* vcache, const int32_t* page_table, int table_stride, int page_size, int ring,
                       int nh, int nkv, int hd, void* stream);
 

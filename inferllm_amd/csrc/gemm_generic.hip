@@ -778,7 +778,7 @@ extern "C" int illm_gemv_rows_f32(const float* X, const float* W, void* Y, int y
 // 2 x 13824 x 5120 93.6 -> 86.1)
 extern "C" int illm_gemv_rows_f32_fused(const float* X, const float* W, float* Y, int M, int N, int K, const float* norm_w,
                                         float eps, int epi, float limit, float alpha, void* stream) {
-    if (M <= 0 || M > 8 || N <= 0 || K <= 0 || (K % 4) || epi < GEMV_PLAIN || epi > GEMV_ACT ||
+    if (!X || !W || !Y || M <= 0 || M > 8 || N <= 0 || K <= 0 || (K % 4) || epi < GEMV_PLAIN || epi > GEMV_ACT ||
         (norm_w && epi == GEMV_ADD))
         return ILLM_ERR_ARG;
     const bool ahead = N <= 8192 / (epi == GEMV_ACT ? 2 : 1);        // (as above, by rows of W)
@@ -798,10 +798,12 @@ extern "C" int illm_gemv_rows_f32_fused(const float* X, const float* W, float* Y
 // The q|k|v product of M <= 8 single tokens with the rotation of q and k (pairs (i, i + hd / 2) of a head, hd % 8 == 0) and
 // the store of k and v: row m at position row_pos[m] of slot row_slot[m].  Y [M, (nh + 2 nkv) hd]: only q is written.
 extern "C" int illm_gemv_qkv_f32(const float* X, const float* W, float* Y, int M, int K, const float* norm_w, float eps,
-                                 const float* cos_sin, const int32_t* row_pos, const int32_t* row_slot, float* kcache,
-                                 float* vcache, const int32_t* page_table, int table_stride, int page_size, int ring,
-                                 int nh, int nkv, int hd, void* stream) {
-    if (M <= 0 || M > 8 || K <= 0 || (K % 4) || nh <= 0 || nkv <= 0 || hd <= 0 || (hd % 8) || page_size <= 0 || table_stride <= 0)
+                                 const float* cos_sin, int max_pos, const int32_t* row_pos, const int32_t* row_slot,
+                                 float* kcache, float* vcache, const int32_t* page_table, int table_stride, int page_size,
+                                 int ring, int nh, int nkv, int hd, void* stream) {
+    if (!X || !W || !Y || M <= 0 || M > 8 || K <= 0 || (K % 4) || nh <= 0 || nkv <= 0 || hd <= 0 || (hd % 8) || !cos_sin ||
+        max_pos <= 0 || !row_pos || !row_slot || !kcache || !vcache || !page_table || page_size <= 0 || table_stride <= 0 ||
+        (nh + 2LL * nkv) * hd > 0x7fffffff)
         return ILLM_ERR_ARG;
     const GemvQkv qkv = {cos_sin, row_pos, row_slot, page_table, kcache, vcache, table_stride, page_size, ring, nh, nkv, hd};
     const int N = (nh + 2 * nkv) * hd, blocks = N / 8;

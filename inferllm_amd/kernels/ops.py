@@ -1327,8 +1327,9 @@ def qkv_rope_store(x, w_qkv, cos_sin: torch.Tensor,
         normed = isinstance(x, NormedRows)
         _gpu(x.weight if normed else None)
         _check(_lib().illm_gemv_qkv_f32(
-            _p(xt), _p(w_qkv), _p(y), M, K, _p(x.weight) if normed else None, eps, _p(cos_sin), _p(row_pos), _p(row_slot),
-            _p(kcache), _p(vcache), _p(page_table), page_table.shape[1], page_size, ring, nh, nkv, hd, _stream()),
+            _p(xt), _p(w_qkv), _p(y), M, K, _p(x.weight) if normed else None, eps, _p(cos_sin), cos_sin.shape[0],
+            _p(row_pos), _p(row_slot), _p(kcache), _p(vcache), _p(page_table), page_table.shape[1], page_size, ring, nh, nkv, hd,
+            _stream()),
             "qkv_rope_store (float32)")
         return y
     if wt is not None and K % 64 == 0 and M >= rows_from("qkv", w_qkv):

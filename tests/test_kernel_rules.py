@@ -166,3 +166,19 @@ def test_a_draw_keeps_the_numbers_that_its_kernel_reads(monkeypatch):
     gc.collect()
     assert [r() for r in refs] == [None] * 3
     ops._kept.clear()
+
+
+def test_float32_products_of_few_rows_refuse_what_is_not_there():
+    """The product with what surrounds it and the one with rotation and store: a null operand, an empty table, sizes that
+    they do not take, or heads whose rows pass the numbers' range, are refused before anything is launched."""
+    lib = ops._lib()
+    fused = dict(X=AT, W=AT, Y=AT, M=4, N=64, K=64, norm_w=AT, eps=1e-5, epi=0, limit=0.0, alpha=1.0, stream=None)
+    qkv = dict(X=AT, W=AT, Y=AT, M=4, K=64, norm_w=AT, eps=1e-5, cos_sin=AT, max_pos=32, row_pos=AT, row_slot=AT, kcache=AT,
+               vcache=AT, page_table=AT, table_stride=2, page_size=16, ring=0, nh=2, nkv=1, hd=64, stream=None)
+    for entry, good, bad in (
+            (lib.illm_gemv_rows_f32_fused, fused, dict(X=None, W=None, Y=None, M=9, N=0, K=66, epi=3)),
+            (lib.illm_gemv_qkv_f32, qkv, dict(X=None, W=None, Y=None, M=9, K=66, cos_sin=None, max_pos=0, row_pos=None,
+                                              row_slot=None, kcache=None, vcache=None, page_table=None, table_stride=0,
+                                              page_size=0, nh=1 << 25, nkv=0, hd=60))):
+        for name, value in bad.items():
+            assert entry(*dict(good, **{name: value}).values()) == ERR_ARG, name
