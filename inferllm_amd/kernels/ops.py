@@ -1366,7 +1366,8 @@ def gate_up_turns_fits(x, w) -> bool:
     return (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2
             and x.is_cuda and w.is_cuda and x.shape[0] >= TURNS_FROM and x.shape[0] * w.shape[0] >= TURNS_OUTPUTS
             and x.shape[1] == w.shape[1] and x.shape[1] % 128 == 0 and x.shape[1] <= 1 << 22 and w.shape[0] % 16 == 0
-            and w.shape[0] <= 1 << 30 and x.is_contiguous() and w.is_contiguous() and _on16(x, w))
+            and w.shape[0] <= 1 << 30 and x.is_contiguous() and w.is_contiguous() and _on16(x, w)
+            and not _plan.keeps_products(x.shape[0], *w.shape))
 
 
 def gate_up_act(x, w_gate_up, limit: float = 0.0) -> torch.Tensor:

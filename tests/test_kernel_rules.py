@@ -182,3 +182,28 @@ def test_float32_products_of_few_rows_refuse_what_is_not_there():
                                               page_size=0, nh=1 << 25, nkv=0, hd=60))):
         for name, value in bad.items():
             assert entry(*dict(good, **{name: value}).values()) == ERR_ARG, name
+
+
+def test_a_pinned_plan_keeps_the_gate_and_up_products_that_it_was_made_with():
+    """A plan saved before gate and up of many rows had a kernel of their own says nothing of it and keeps the products;
+    so do the matrices that a plan made by hand has cuts for.  What is saved now comes back as it was."""
+    import json
+
+    from inferllm_amd.kernels.plan import FIXED_CUTS, Plan
+    shape, cut = (22016, 4096), {(8, 22016, 4096): (8192,)}
+    old = Plan.fixed().to_dict()
+    old["cuts"].append([[8, 22016, 4096], [8192]])
+    del old["turns"]
+    old = Plan.from_dict(json.loads(json.dumps(old)))
+    assert old.cuts[8, 22016, 4096] == (8192,) and all(old.keeps_products(M, *shape) for M in (256, 1000, 2048))
+    for plan in (Plan.fixed(), Plan.fixed(measure=True), Plan(), Plan(measure=True), Plan(cuts=FIXED_CUTS), Plan(cuts=cut, turns=True)):
+        assert plan.turns is True and not any(plan.keeps_products(M, *shape) for M in (256, 1000, 2048))
+    own = Plan(cuts={**FIXED_CUTS, **cut})
+    assert [own.keeps_products(M, *shape) for M in (1792, 1793, 2048, 2049)] == [False, True, True, False]
+    measured = Plan(measure=True)
+    measured.cuts.update(cut)                          # (timed for another matrix of that shape)
+    for plan in (old, own, measured, Plan.fixed()):
+        again = Plan.from_dict(json.loads(json.dumps(plan.to_dict())))
+        assert again == plan and [again.keeps_products(M, *shape) for M in (1000, 2048)] == [plan.keeps_products(M, *shape)
+                                                                                              for M in (1000, 2048)]
+    assert old != Plan.from_dict(dict(old.to_dict(), turns=True))
