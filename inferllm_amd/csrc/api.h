@@ -241,6 +241,9 @@ int illm_gemm_skinny_act(const void* X, const void* W, const void* Wt, void* Y, 
 // Many rows (csrc/gemm_turns.hip), bfloat16 on 16-byte addresses, K % 128 == 0, F % 8 == 0: Y [M, F] of W [2 F, K] = [gate | up]
 // (limit, alpha as for illm_gemm_skinny_gateup_act).
 int illm_gemm_turns_gate_up(const void* X, const void* W, void* Y, int M, int F, int K, float limit, float alpha, void* stream);
+// The tiles that it takes M rows and F columns in, 256 of them a round, and (shape not null) their shape: 0: 256 x 256 rows
+// of X and of W, 1: 192 x 256, 2: 128 x 256, 3: 256 x 128.
+int illm_gemm_turns_tiles(int M, int F, int* shape);
 // The sum of two products of at most 16 rows, float32 Y = X . W^T + X2 . W2^T, from the tiled copies (K, K2 % 128 == 0).
 int illm_gemm_skinny_sum(const void* X, const void* Wt, int K, const void* X2, const void* W2t, int K2, float* Y, int M,
                          int N, void* stream);

@@ -54,10 +54,6 @@ void illm_set_rows_a_launch(int rows);
 // or not in steps of 4 use, instead of the matrix cores; 2 also bfloat16 rows to the one on their
 // float32 instruction (default 1: bfloat16 rows in steps of 8 the bfloat16 instruction).
 void illm_set_attn_cap_mfma(int on);
-// illm_gemm_turns_gate_up: the tiles that it takes M rows and F columns in, and their shape (0: 256 x 256 rows of X and of
-// W, 1: 192 x 256, 2: 128 x 256, 3: 256 x 128).  A launch has at most 256 blocks.
-int illm_gemm_turns_tiles(int M, int F, int* shape);
-
 // illm_attn_cap_decode, widths up to 128: query heads of a kv head that a block takes, 4, 2 or 1 (0,
 // the default: 4, or fewer while there are fewer than 256 blocks).
 void illm_set_attn_cap_heads(int n);

@@ -11,7 +11,6 @@
 #include <algorithm>
 
 #include "api.h"
-#include "api_test.h"
 #include "gemm_turns.h"
 
 // g / (1 + e^-(alpha g)), within 2 in the last place of float32 wherever the result is a normal number (expf and a division

@@ -1353,21 +1353,40 @@ def gate_up_silu(x, w_gate_up) -> torch.Tensor:
     return gate_up_act(x, w_gate_up, 0.0)
 
 
-# From so many rows, and outputs of both products, gate and up with their activation are one kernel.  us, product and
-# activation -> one kernel: 2 x 4096 x 1024 of 256 / 500 rows 19 / 22 -> 19 / 19, 2 x 5376 x 2048 of 300 / 500 29 / 33 -> 30 / 33,
-# 2 x 2816 x 2048 of 500 / 1,000 29 / 36 -> 31 / 31, 2 x 1408 x 2048 of 1,000 / 2,048 28 / 33 -> 30 / 32, 2 x 1024 x 1024 of
-# 1,000 / 2,048 15 / 20 -> 18 / 18; 2 x 11008 x 4096 of 256 rows 69 -> 65, of 1,000 172 -> 178 (a second round of 88 tiles).
-TURNS_FROM, TURNS_OUTPUTS = 256, 1 << 22
+# From so many rows, and outputs of both products, gate and up with their activation are one kernel.  us, weights cold,
+# product (in the plan's cuts) and activation -> one kernel:
+#   2 x 1024 x 1024   500 rows 17 -> 22, 1,000 19 -> 22, 2,048 23 -> 23, 2,198 25 -> 23, 2,775 32 -> 24
+#   2 x 1408 x 2048   1,000 rows 32 -> 34, 1,490 35 -> 35, 1,712 39 -> 36, 2,048 38 -> 37, 3,487 60 -> 47
+#   2 x 2816 x 2048   291 rows 24 -> 33, 500 33 -> 35, 745 35 -> 36, 855 39 -> 36, 2,048 69 -> 48
+#   2 x 5376 x 2048   272 rows 32 -> 35, 448 36 -> 37, 500 39 -> 37, 1,000 56 -> 48, 2,048 101 -> 83
+#   2 x 8192 x 4096   257 rows 59 -> 63, 332 64 -> 64, 406 69 -> 65, 1,000 110 -> 100, 2,048 201 -> 192
+#   2 x 11008 x 4096  256 rows 72 -> 68, 500 97 -> 90, 1,000 169 -> 170, 2,048 279 -> 264
+#   2 x 13824 x 5120  256 rows 96 -> 97, 500 143 -> 121, 1,000 267 -> 221, 2,048 473 -> 447
+#   2 x 28672 x 8192  256 rows 216 -> 191, 1,000 678 -> 669, 2,048 1,245 -> 1,244
+TURNS_FROM, TURNS_OUTPUTS = 256, 9 << 19
+# Not where the last of its few rounds of 256 blocks is nearly empty, and K long enough for the product to be a good one:
+# less than a third of the second round (2 x 14336 x 4096, 576 rows 140 -> 146; 2 x 13824 x 5120, 528 / 576 rows 180 / 180 -> 184
+# / 195; 2 x 11008 x 4096, 656 rows, a third of it 151 -> 138; of short K 2 x 6144 x 3072, 1,296 rows 122 -> 116), less than a
+# sixteenth of the third to sixth (2 x 11008 x 4096, 2,200 / 2,844 rows 326 / 418 -> 342 / 424; 24 tiles of 256 in the
+# thirteenth, 9,061 rows 1,279 -> 1,158).
+TURNS_ROUND_K = 4096
+
+
+def turns_pays(M: int, F: int, K: int) -> bool:
+    """Whether csrc/gemm_turns.hip is the faster way for M rows of gate and up (w [2 F, K])."""
+    if M < TURNS_FROM or M * 2 * F < TURNS_OUTPUTS:
+        return False
+    rounds, last = divmod(_lib().illm_gemm_turns_tiles(M, F, None) - 1, 256)          # full rounds before the last, its tiles - 1
+    return K < TURNS_ROUND_K or rounds == 0 or rounds > 5 or last + 1 >= (86 if rounds == 1 else 16)
 
 
 def gate_up_turns_fits(x, w) -> bool:
     """Whether csrc/gemm_turns.hip takes the gate and up products of these rows and is the faster way."""
     w = plain_weight(w)
     return (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 2
-            and x.is_cuda and w.is_cuda and x.shape[0] >= TURNS_FROM and x.shape[0] * w.shape[0] >= TURNS_OUTPUTS
-            and x.shape[1] == w.shape[1] and x.shape[1] % 128 == 0 and x.shape[1] <= 1 << 22 and w.shape[0] % 16 == 0
-            and w.shape[0] <= 1 << 30 and x.is_contiguous() and w.is_contiguous() and _on16(x, w)
-            and not _plan.keeps_products(x.shape[0], *w.shape))
+            and x.is_cuda and w.is_cuda and x.shape[1] == w.shape[1] and x.shape[1] % 128 == 0 and x.shape[1] <= 1 << 22
+            and w.shape[0] % 16 == 0 and w.shape[0] <= 1 << 30 and x.is_contiguous() and w.is_contiguous() and _on16(x, w)
+            and turns_pays(x.shape[0], w.shape[0] // 2, w.shape[1]) and not _plan.keeps_products(x.shape[0], *w.shape))
 
 
 def gate_up_act(x, w_gate_up, limit: float = 0.0) -> torch.Tensor:

@@ -12,8 +12,9 @@ the choice is a table by shape:
   (`python -m inferllm_amd.kernels.tune`: the majority of three measurements, and a way other
   than the rule's must win by 7 %), and for every other shape one rule: planes from 17 rows on,
   products of many rows whole.  Nothing is ever timed.  Gate and up of many rows are a kernel of
-  their own with the activation (`ops.gate_up_turns_fits`) and have no cuts, except under a plan
-  that was pinned before there was one (`Plan.turns`): it keeps the products and their bits.
+  their own with the activation, which has no cuts, but for sizes that `ops.turns_pays` leaves to the
+  product and under a plan that was pinned before there was that kernel (`Plan.turns`): it keeps
+  the products and their bits.
   The third table says from how few rows (below 17) the q|k|v product goes to the kernel that
   shares X through LDS (csrc/gemm_rows.hip) rather than to the few-rows kernel; gate|up and the
   head measured equal or worse there below 17 rows and have no entries.
@@ -69,6 +70,7 @@ FIXED_CUTS: Dict[tuple, tuple] = {
     ('pad', 6, 4096, 11008): ('pad', 256),
     ('pad', 6, 4096, 14336): ('pad', 256),
     (11, 8192, 8192): (4096,),
+    (12, 22016, 4096): (8192,),
     (13, 15360, 5120): (7680,),
     (13, 8192, 28672): (4096,),
     (14, 10240, 8192): (4096,),
@@ -100,6 +102,7 @@ FIXED_CUTS: Dict[tuple, tuple] = {
     (31, 15360, 5120): (8192,),
     (7, 10240, 8192): (8192,),
     (8, 10240, 8192): (8192,),
+    (9, 22016, 4096): (8192,),
 }
 
 

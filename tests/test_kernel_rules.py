@@ -207,3 +207,13 @@ def test_a_pinned_plan_keeps_the_gate_and_up_products_that_it_was_made_with():
         assert again == plan and [again.keeps_products(M, *shape) for M in (1000, 2048)] == [plan.keeps_products(M, *shape)
                                                                                               for M in (1000, 2048)]
     assert old != Plan.from_dict(dict(old.to_dict(), turns=True))
+
+
+@pytest.mark.parametrize("F, K, one_kernel, two", [
+    (11008, 4096, (256, 500, 768, 1000, 2048, 2112, 2305, 2816, 2881, 9061), (255, 2113, 2200, 2304, 2817, 2880)),
+    (14336, 4096, (256, 512, 577, 1000, 9061), (513, 576)), (13824, 5120, (500, 640, 2048), (528, 576)),
+    (6144, 3072, (384, 1296, 1344, 2048), (256, 383)), (8192, 4096, (288, 500, 2905), (256, 287)),
+    (2816, 2048, (838, 2048), (500, 837)), (1024, 1024, (2304, 9061), (1000, 2303))])
+def test_gate_up_and_activation_are_one_kernel_where_that_is_the_faster_way(F, K, one_kernel, two):
+    """Rows and outputs enough, and no last round that is nearly empty: both sides of every line."""
+    assert all(ops.turns_pays(M, F, K) for M in one_kernel) and not any(ops.turns_pays(M, F, K) for M in two)
