@@ -29,7 +29,8 @@ def matrices(engine):
         for kind, w, _geometry in part.tunables():
             plain = ops.plain_weight(w) if isinstance(w, (ops.Weight, torch.Tensor)) else None
             if plain is not None and plain.dim() == 2 and plain.dtype == torch.bfloat16:
-                seen.setdefault(tuple(plain.shape), (kind, w))
+                if seen.get(tuple(plain.shape), ("gate_up",))[0] == "gate_up":      # (other products have all the ways)
+                    seen[tuple(plain.shape)] = (kind, w)
     return seen
 
 
@@ -70,11 +71,13 @@ def tune_config(cfg: dict, max_rows: int, repeats: int, say, rows_only: bool = F
             best = max(set(votes), key=votes.count)
             if best:
                 cuts[("pad", rows32, N, K)] = best
-        if N < rules.cut_min_cols or kind == "gate_up":      # (many rows of gate|up are one kernel with the activation)
+        if N < rules.cut_min_cols:
             continue
         for rows256 in range(rules.cut_min_rows // 256, max_rows // 256 + 1):
             M = rows256 * 256
             x = torch.randn(M, K, device=plain.device).to(torch.bfloat16)
+            if kind == "gate_up" and ops.gate_up_turns_fits(x, plain):      # (one kernel with the activation, without cuts)
+                continue
             votes = [ops.measure_plan(x, plain, None, MARGIN) for _ in range(repeats)]
             best = max(set(votes), key=votes.count)
             if best:

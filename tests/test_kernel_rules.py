@@ -217,3 +217,18 @@ def test_a_pinned_plan_keeps_the_gate_and_up_products_that_it_was_made_with():
 def test_gate_up_and_activation_are_one_kernel_where_that_is_the_faster_way(F, K, one_kernel, two):
     """Rows and outputs enough, and no last round that is nearly empty: both sides of every line."""
     assert all(ops.turns_pays(M, F, K) for M in one_kernel) and not any(ops.turns_pays(M, F, K) for M in two)
+
+
+def test_tuning_times_a_product_that_has_the_shape_of_gate_and_up():
+    """Two matrices of one shape, one of them gate and up: the other's ways are those that are timed, whichever comes first."""
+    from inferllm_amd.kernels import tune
+    a, b = torch.zeros(64, 32, dtype=torch.bfloat16), torch.zeros(64, 32, dtype=torch.bfloat16)
+
+    class part:
+        def __init__(self, *listed):
+            self.tunables = lambda: listed
+
+    for parts in ([part(("gate_up", a, {})), part(("plain", b, {}))], [part(("plain", b, {}), ("gate_up", a, {}))]):
+        model = type("model", (), {"every_part": staticmethod(lambda: parts)})
+        (kind, w), = tune.matrices(type("engine", (), {"model": model})).values()
+        assert kind == "plain" and w is b
