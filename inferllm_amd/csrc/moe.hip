@@ -902,7 +902,7 @@ moe_rows_mfma_lds_kernel(const bf16_t* __restrict__ X, int x_div, const bf16_t* 
     }
 }
 
-// Tiles of up to 128 or 192 pairs (from 1.5 pairs an expert on), K % 64 == 0, N % 4 == 0 (192: N % 8): the loop of
+// Tiles of up to 128 or 192 pairs (from 3 to 24 pairs an expert on), K % 64 == 0, N % 4 == 0 (192: N % 8): the loop of
 // gemm_turns.h over a tile's pairs, X's rows gathered by the loads, and 64 NT rows of W (gated: half of them gate rows, half
 // the up rows of the same columns).  X and an expert's W each within the 4 GiB that a load's 32-bit offset reaches; X, W
 // and Y on 16-byte addresses.  Block ids go round the 8 XCDs: an XCD takes a stretch of the (tile, columns) there are, the

@@ -1775,26 +1775,32 @@ MOE_MFMA_FROM = 0        # (token, choice) pairs an expert on average from which
 
 
 # Where the kernel with both operands in LDS, in tiles of 128 pairs or more, takes bfloat16 experts whose sizes are
-# multiples of 64.  It beats the smaller tiles from 24 pairs an expert on with every stack (their kernels for 32
-# and 64 pairs are the slow ones); with fewer pairs where the stack has blocks enough for the chip (columns of 64
-# and of 128) and a matrix is large enough for its pairs to be worth a block.  us, both products, tiles of 16 pairs -> of 128:
-#   experts        pairs an expert: 2           4           6           12          24
-#   64 of 1408 x 2048         226 -> 223  249 -> 238  295 -> 241  379 -> 244  350 -> 253
-#   32 of 4096 x 2048         427 -> 364  414 -> 360  461 -> 379  532 -> 382  551 -> 393
-#   8 of 14336 x 4096         526 -> 576  758 -> 632  788 -> 634  830 -> 636  816 -> 645
-#   8 of 8192 x 4096          342 -> 406  364 -> 386  369 -> 387  405 -> 389  603 -> 394
-#   24 of 1536 x 1536          82 ->  99   86 -> 101   90 -> 101  122 -> 102  134 -> 106
-#   128 of 768 x 2048         226 -> 257  239 -> 265  315 -> 274  382 -> 282  360 -> 300
-#   256 of 256 x 1024          81 -> 118   89 -> 126   98 -> 129  117 -> 137  176 -> 153
-#   16 of 512 x 512            18 ->  22   18 ->  22   18 ->  22   20 ->  25   50 ->  27
-#   8 of 2048 x 1024           40 ->  58   41 ->  58   43 ->  58   48 ->  59  109 ->  61
-#   2 of 4096 x 4096           65 -> 131   67 -> 131   71 -> 131   79 -> 131  274 -> 133
-# (2,964 tokens of the first, 6 chosen: 1,023 -> 608.)  The same bits.  (Measured with the loop before the one
-# in turns, which takes 4 to 20 % less with few pairs an expert; tiles of 16 pairs take less now too.)
-MOE_TILES_ALWAYS = 24              # pairs an expert on average
-MOE_TILES_BLOCKS = (256, 512)      # blocks of the thinner product: none with fewer than the first, from 12 pairs an
-                                   # expert on with fewer than the second, from 1.5 on with more
-MOE_TILES_WORK = 1 << 23           # pairs an expert times its F E
+# multiples of 64, rather than tiles of 16 (the kernels for 32 and 64 pairs are slower than either).  The smaller tiles
+# take longer with every pair and most from 12 an expert on, where some experts of a step have a second tile and read
+# their matrices twice; the larger ones take the same time for all, which a stack with few blocks (columns of 64 and of
+# 128) or small matrices takes longer to be worth.  us, both products, matrices cold, tiles of 16 pairs -> of 128:
+#   experts        pairs an expert: 3           6           8           12          16          24
+#   64 of 1408 x 2048         191 -> 203  212 -> 208  232 -> 209  280 -> 211  352 -> 215  506 -> 215
+#   32 of 4096 x 2048         278 -> 286  302 -> 295  317 -> 297  386 -> 300  504 -> 302  716 -> 307
+#   128 of 768 x 2048         211 -> 211  241 -> 225  260 -> 226  312 -> 229  400 -> 233  575 -> 239
+#   256 of 256 x 1024          86 ->  85  101 ->  89  112 ->  90  132 ->  92  171 ->  93  236 ->  97
+#   64 of 1024 x 1024          81 ->  77   90 ->  80   98 ->  80  116 ->  81  148 ->  82  204 ->  85
+#   32 of 2048 x 4096         312 -> 291  352 -> 301  360 -> 300  398 -> 300  526 -> 302  711 -> 306
+#   8 of 14336 x 4096         466 -> 494  492 -> 496  521 -> 497  714 -> 511  868 -> 511 1175 -> 511
+#   8 of 8192 x 4096          352 -> 297  356 -> 298  361 -> 299  454 -> 300  548 -> 302  723 -> 302
+#   24 of 1536 x 1536          76 ->  84   83 ->  86   89 ->  85   99 ->  88  126 ->  88  173 ->  91
+#   16 of 2048 x 2048          82 -> 103   86 -> 102   89 -> 102  115 -> 102  142 -> 103  197 -> 104
+#   8 of 3072 x 3072           90 ->  99   98 -> 100  104 -> 100  134 -> 102  183 -> 103  208 -> 105
+#   8 of 2048 x 1024           30 ->  43   32 ->  44   33 ->  43   50 ->  44   57 ->  45   66 ->  45
+#   16 of 512 x 512            16 ->  21   16 ->  21   17 ->  21   22 ->  22   25 ->  23   26 ->  23
+#   4 of 8192 x 2048          108 -> 146  128 -> 147  121 -> 146  139 -> 148  172 -> 149  208 -> 149
+#   2 of 4096 x 4096           67 ->  94   70 ->  94   72 ->  94   77 ->  95   83 ->  95  143 ->  97
+# The same bits.
+MOE_TILES_FROM = (3, 6, 12, 24)    # pairs an expert on average: of stacks with blocks enough and long rows (E), of those
+                                   # with blocks or matrices enough, of others of eight experts or more, of fewer (whose
+                                   # pairs are spread evenly)
+MOE_TILES_BLOCKS = (256, 512)      # blocks of the thinner product: enough with large matrices, and with any
+MOE_TILES_WORK, MOE_TILES_LONG = 1 << 24, 4096       # F E of a large matrix; E of long rows
 # Tiles of 192 pairs and blocks of 256 rows of W from so many pairs an expert on, where that leaves every compute unit
 # a block.  us, gate|up + down, tiles of 128 -> of 192: 64 of 1408 x 2048 at 94 pairs 167 + 95 -> 174 + 94, at 278
 # 369 + 193 -> 289 + 149; 32 of 4096 x 2048 at 128 330 + 170 -> 237 + 139; 8 of 8192 x 4096 at 256 536 + 268 ->
@@ -1803,12 +1809,10 @@ MOE_WIDE_FROM, MOE_WIDE_BLOCKS = 112, 256
 
 
 def _moe_tiles_pay(E: int, F: int, NP: int, n_exp: int) -> bool:
-    per_expert = NP / max(1, n_exp)
-    if per_expert >= MOE_TILES_ALWAYS:
-        return True
     blocks = n_exp * min(F // 64, (E + 127) // 128)
-    return (blocks >= MOE_TILES_BLOCKS[0] and per_expert >= (12 if blocks < MOE_TILES_BLOCKS[1] else 1.5)
-            and per_expert * F * E >= MOE_TILES_WORK)
+    enough = blocks >= MOE_TILES_BLOCKS[1] or (blocks >= MOE_TILES_BLOCKS[0] and F * E >= MOE_TILES_WORK)
+    kind = (0 if E >= MOE_TILES_LONG and blocks >= MOE_TILES_BLOCKS[1] else 1) if enough else 2 if n_exp >= 8 else 3
+    return NP / max(1, n_exp) >= MOE_TILES_FROM[kind]
 
 
 def _moe_few_rows(per_expert: float) -> int:

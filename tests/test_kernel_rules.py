@@ -48,12 +48,12 @@ def test_the_experts_tiles_of_128_pairs_refuse_other_addresses():
 
 
 def test_the_experts_tiles_of_128_pairs_are_taken_where_they_pay():
-    """Stacks that leave compute units idle, or whose matrices are small, keep the smaller tiles up to 24 pairs an expert
-    (experts, F, E -> the fewest pairs an expert in tiles of 128, measured to be no slower from there on)."""
+    """Stacks that leave compute units idle, or whose matrices are small, keep the smaller tiles up to 12 pairs an expert, of
+    few experts up to 24 (experts, F, E -> the fewest pairs an expert in tiles of 128, measured to be no slower from there on)."""
     rows = lambda NE, F, E, p: ops._moe_tiling(torch.bfloat16, E, F, int(p * NE), NE)[1]  # noqa: E731
-    for NE, F, E, first in ((64, 1408, 2048, 3), (32, 4096, 2048, 1.5), (8, 14336, 4096, 12), (24, 1536, 1536, 12), (128, 768, 2048, 6),
-                            (256, 256, 1024, 24), (16, 512, 512, 24), (4, 1024, 1024, 24), (8, 2048, 1024, 24),
-                            (2, 4096, 4096, 24), (32, 2048, 4096, 1.5)):
+    for NE, F, E, first in ((64, 1408, 2048, 6), (32, 4096, 2048, 6), (8, 14336, 4096, 6), (24, 1536, 1536, 12), (128, 768, 2048, 6),
+                            (256, 256, 1024, 6), (16, 512, 512, 12), (4, 1024, 1024, 24), (8, 2048, 1024, 12), (16, 2048, 2048, 12),
+                            (2, 4096, 4096, 24), (32, 2048, 4096, 3), (8, 8192, 4096, 6), (64, 1024, 1024, 6)):
         for p in (1, 1.5, 2, 3, 4, 6, 8, 12, 16, 24, 64, 500):
             assert (rows(NE, F, E, p) == 128) == (p >= first), (NE, F, E, p)
 
