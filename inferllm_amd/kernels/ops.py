@@ -3178,31 +3178,31 @@ def sample(logits: torch.Tensor, temperature: float, top_k: int, top_p: float,
            counters: torch.Tensor) -> torch.Tensor:
     """One draw per row; see csrc/sampling.hip.  seeds: int64 [B] (bit pattern used), counters int32 [B]."""
     _gpu(logits, last_tokens, seeds, counters)
-    return _sample(logits, temperature, top_k, top_p, repeat_penalty, last_tokens, seeds, counters)
+    B = logits.shape[0] if logits.dim() == 2 else 0
+    _need(seeds.dtype == torch.int64 and seeds.numel() >= B, "sample: seeds int64 [B]")
+    _i32(counters, B)
+    return _sample(logits, temperature, top_k, top_p, repeat_penalty, last_tokens, _p(seeds), _p(counters))
 
 
-def sample_from_host(logits: torch.Tensor, temperature: float, top_k: int, top_p: float, seeds: torch.Tensor,
-                     counters: torch.Tensor) -> torch.Tensor:
-    """`sample` without a window of last tokens, the seeds and counters in pinned memory, where the kernel reads them.  The
-    memory is kept until the kernel has run, whoever lets go of it; what it holds the caller leaves as it is until then."""
+def sample_from_host(logits: torch.Tensor, temperature: float, top_k: int, top_p: float, numbers: torch.Tensor) -> torch.Tensor:
+    """`sample` without a window of last tokens, from `numbers` int32 [3 n], n >= B, in pinned memory, where the kernel reads
+    them: n seeds of two words each, then n counters.  They have to be there, as they are, until the kernel has run, whoever
+    lets go of them (`keep_until`)."""
     _gpu(logits)
-    for t in (seeds, counters):
-        _need(t.is_contiguous() and t.is_pinned(), "sample_from_host: seeds and counters in pinned memory")
+    at, n = numbers.data_ptr(), numbers.numel() // 3
+    _need(logits.dim() == 2 and numbers.dtype == torch.int32 and n >= logits.shape[0] and numbers.is_contiguous()
+          and numbers.is_pinned(), "sample_from_host: seeds and counters int32 [3 n] in pinned memory")
     _need(not torch.cuda.is_current_stream_capturing(), "sample_from_host: a graph would read the numbers again")
-    out = _sample(logits, temperature, top_k, top_p, 1.0, None, seeds, counters)
-    keep_until_run(seeds, counters)
-    return out
+    return _sample(logits, temperature, top_k, top_p, 1.0, None, ctypes.c_void_p(at), ctypes.c_void_p(at + 8 * n))
 
 
-_kept: collections.deque = collections.deque()     # (event behind a kernel, the host memory that it reads), oldest first
+_kept: collections.deque = collections.deque()     # (event, tensors), oldest first
 _kept_lock = threading.Lock()
 
 
-def keep_until_run(*tensors: torch.Tensor) -> None:
-    """Hold the tensors until the current stream has done what it was given so far.  (torch's pinned memory is free as soon
-    as its last tensor goes, unless torch itself has queued a copy of it.)"""
-    event = torch.cuda.Event()
-    record(event)
+def keep_until(event, *tensors: torch.Tensor) -> None:
+    """Hold host memory that a kernel reads until `event`, recorded behind the kernel and not again, has passed.  (torch's
+    pinned memory is free as soon as its last tensor goes, unless torch itself has queued a copy of it.)"""
     with _kept_lock:
         while _kept and _kept[0][0].query():
             _kept.popleft()
@@ -3212,8 +3212,7 @@ def keep_until_run(*tensors: torch.Tensor) -> None:
 def _sample(logits, temperature, top_k, top_p, repeat_penalty, last_tokens, seeds, counters) -> torch.Tensor:
     _need(logits.dtype == torch.float32 and logits.dim() == 2, "sample: float32 [B, V]")
     B, V = logits.shape
-    _need(seeds.dtype == torch.int64 and seeds.numel() >= B, "sample: seeds int64 [B]")
-    _i32(counters, B); _i32(last_tokens)
+    _i32(last_tokens)
     n_last = 0
     if last_tokens is not None:
         _need(last_tokens.dim() == 2 and last_tokens.shape[0] == B, "sample: last_tokens [B, n]")
@@ -3231,11 +3230,11 @@ def _sample(logits, temperature, top_k, top_p, repeat_penalty, last_tokens, seed
         rows = torch.empty((B, (_sample_long_row_bytes + 7) // 8), dtype=torch.int64, device=logits.device)
         _check(_lib().illm_sample_long(
             _p(logits), _p(scratch), _p(rows), _p(out), B, V, ctypes.c_float(temperature),
-            ctypes.c_float(top_p), ctypes.c_float(repeat_penalty), _p(last_tokens), n_last, _p(seeds),
-            _p(counters), _stream()), "sample_long")
+            ctypes.c_float(top_p), ctypes.c_float(repeat_penalty), _p(last_tokens), n_last, seeds,
+            counters, _stream()), "sample_long")
         return out
     _check(_lib().illm_sample(
         _p(logits), _p(scratch), _p(out), B, V, ctypes.c_float(temperature), int(top_k),
-        ctypes.c_float(top_p), ctypes.c_float(repeat_penalty), _p(last_tokens), n_last, _p(seeds),
-        _p(counters), _stream()), "sample")
+        ctypes.c_float(top_p), ctypes.c_float(repeat_penalty), _p(last_tokens), n_last, seeds,
+        counters, _stream()), "sample")
     return out

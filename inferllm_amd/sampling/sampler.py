@@ -46,14 +46,10 @@ class Sampler:
         # still wait for their copy when the next draw's are written
         self._stages: List[Optional[torch.Tensor]] = [None] * 4
         self._back: List[torch.Tensor] = []            # pinned buffers the drawn tokens come back in
-        self._copied: List[object] = []                # and the events behind their copies
         self._turn = 0
 
-    def _upload(self, seeds, counters, windows):
-        """One pinned buffer: (seeds int64 [B], counters int32 [B], windows int32 [B, n] or None).  Without windows the
-        kernel reads the few numbers where they are (a copy takes 10 us of the host and 3 of the device), and the buffer is
-        kept until it has, also where this sampler goes first (`ops.sample_from_host`); with them one copy brings
-        everything over."""
+    def _stage(self, seeds, counters, windows):
+        """The draw's numbers in one pinned buffer, int32: seeds (two words each), counters, windows or none."""
         B = len(seeds)
         n = len(windows[0]) if windows else 0
         words = B * (3 + n)
@@ -67,9 +63,7 @@ class Sampler:
         flat[2 * B:3 * B] = counters
         if n:
             flat[3 * B:].reshape(B, n)[:] = windows
-        dev = host.to(self.device, non_blocking=True) if n else host
-        return (dev[:2 * B].view(torch.int64), dev[2 * B:3 * B],
-                dev[3 * B:].view(B, n) if n else None)
+        return host
 
     def needs_histories(self) -> bool:
         """Whether a draw depends on the tokens before it (the repeat penalty's window)."""
@@ -87,6 +81,7 @@ class Sampler:
         is completed on the device."""
         p = self.params
         self._turn = (self._turn + 1) % 4
+        from_host = False
         if p.greedy:
             dev = ops.argmax(logits.contiguous())
         else:
@@ -99,26 +94,31 @@ class Sampler:
                     m = n - 1
                     rows = [[-1] * (m - min(m, len(h))) + (list(h[-m:]) if m else []) + [-1]
                             for h in histories]
-            seeds_t, counters_t, last = self._upload(seeds, counters, rows)
-            if last is not None and latest is not None:
-                last[:, -1].copy_(latest)
-            if last is None and self._pinned:
-                dev = ops.sample_from_host(logits.contiguous(), p.temperature, p.top_k, p.top_p, seeds_t, counters_t)
+            numbers, B = self._stage(seeds, counters, rows), len(seeds)
+            from_host = not rows and self._pinned
+            if from_host:
+                # the kernel reads the few numbers where they are (a copy takes 10 us of the host and 3 of the device)
+                dev = ops.sample_from_host(logits.contiguous(), p.temperature, p.top_k, p.top_p, numbers)
             else:
+                there = numbers.to(self.device, non_blocking=True)      # one copy for everything
+                last = there[3 * B:].view(B, -1) if rows else None
+                if last is not None and latest is not None:
+                    last[:, -1].copy_(latest)
                 dev = ops.sample(logits.contiguous(), p.temperature, p.top_k, p.top_p,
-                                 p.repeat_penalty, last, seeds_t, counters_t)
+                                 p.repeat_penalty, last, there[:2 * B].view(torch.int64), there[2 * B:3 * B])
         B = dev.numel()
         if not dev.is_cuda:                  # stand-in kernels on the CPU (tests): nothing to wait for
             return Draw(dev, dev, None)
         while len(self._back) < 4:
             self._back.append(torch.empty(1024, dtype=torch.int32, pin_memory=True))
-            self._copied.append(torch.cuda.Event())
         if self._back[self._turn].numel() < B:
             self._back[self._turn] = torch.empty(B, dtype=torch.int32, pin_memory=True)
         host = self._back[self._turn][:B]
         host.copy_(dev, non_blocking=True)
-        copied = self._copied[self._turn]
+        copied = torch.cuda.Event()          # (2.7 us; recording one again 4.7)
         ops.record(copied)
+        if from_host:                        # the numbers outlive the kernel, also where this sampler goes first
+            ops.keep_until(copied, self._stages[self._turn])
         return Draw(dev, host, copied)
 
     def __call__(self, logits: torch.Tensor, seeds: Sequence[int], counters: Sequence[int],

@@ -2200,7 +2200,8 @@ def test_draws_outlive_their_samplers(V, top_p):
         b = a @ a
     draws, others = [], []
     for i in range(8):
-        draws.append(Sampler(params, DEV).draw(logits, list(range(100 * i, 100 * i + 8)), [i] * 8))
+        more = i % 2                       # (a seed and a counter more than there are rows)
+        draws.append(Sampler(params, DEV).draw(logits, list(range(100 * i, 100 * i + 8 + more)), [i] * (8 + more)))
         others.append(torch.empty(1024, dtype=torch.int32, pin_memory=True).fill_(7))
     assert [d.tokens() for d in draws] == want and b.shape == a.shape
     with pytest.raises(Exception):

@@ -147,6 +147,7 @@ def test_a_draw_keeps_the_numbers_that_its_kernel_reads(monkeypatch):
     monkeypatch.setattr(torch.cuda, "Event", event)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     monkeypatch.setattr(torch.Tensor, "is_pinned", lambda t: True)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda t: True))
     monkeypatch.setattr(ops, "record", lambda e: None)
     monkeypatch.setattr(ops, "_gpu", lambda *t: None)
     monkeypatch.setattr(ops, "_lib", lambda: library)
@@ -155,6 +156,7 @@ def test_a_draw_keeps_the_numbers_that_its_kernel_reads(monkeypatch):
     for i in range(3):
         sampler, numbers = Sampler(SamplingParams(temperature=0.8), "cuda:0"), np.zeros(1024, np.int32)
         sampler._stages = [torch.from_numpy(numbers)] * 4
+        sampler._back = [torch.empty(2, dtype=torch.int32)] * 4
         refs.append(weakref.ref(numbers))
         sampler.draw(torch.zeros(2, 8), [1, 2], [0, 0])
         del sampler, numbers
@@ -162,7 +164,7 @@ def test_a_draw_keeps_the_numbers_that_its_kernel_reads(monkeypatch):
         assert [r() is not None for r in refs] == ([True], [True, True], [False, True, True])[i]
         events[0].passed = i == 1
     events[1].passed = events[2].passed = True
-    ops.keep_until_run(torch.zeros(1))
+    ops.keep_until(event(), torch.zeros(1))
     gc.collect()
     assert [r() for r in refs] == [None] * 3
     ops._kept.clear()
