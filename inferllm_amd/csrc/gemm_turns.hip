@@ -5,9 +5,9 @@
 // last product and the next one's first.  Block ids go round the 8 XCDs: an XCD takes a stretch of the tiles, in groups of
 // 8 along X, so that the 32 under way share 8 panels of X and 4 of W in its L2.
 // Against the vendor GEMM (cut along the columns where that was faster) and the activation behind it, which wrote and read
-// both products (us, in turn on one card): 2 x 14336 x 4096 of 9,061 rows 1,580 -> 1,470, of 512 109 -> 100; 2 x 11008 x 4096
-// of 9,061 / 2,048 / 500 rows 1,274 / 294 / 94 -> 1,172 / 286 / 89 (1.4 PFLOP/s, 688 tiles or 2.7 rounds of 256, one
-// round of 172); 2 x 5376 x 2048 of 2,964 rows 117 -> 106.  What bounds the large ones is the chip's power.
+// both products (us, in turn on one card, weights from memory): 2 x 14336 x 4096 of 9,061 rows 1,547 -> 1,495, of 512 108 -> 97;
+// 2 x 11008 x 4096 of 9,061 / 2,048 / 500 rows 1,283 / 289 / 99 -> 1,178 / 276 / 90 (1.34 PFLOP/s, 688 tiles or 2.7 rounds of 256,
+// one round of 172); 2 x 5376 x 2048 of 2,964 rows 119 -> 105.  What bounds the large ones is the chip's power.
 #include <algorithm>
 
 #include "api.h"
@@ -134,7 +134,7 @@ static long long turns_tiles(int M, int F, int shape) {
 }
 
 // Tiles of 256 x 256, 192 x 256, 128 x 256 or 256 x 128 rows of X and of W: the least of rounds of 256 blocks times a
-// round's time (K = 4,096, us: 88, 73, 59 and 58).
+// round's time (K = 4,096, us: 88, 73, 59 and 58; with the gate as it is now about 1 more each).
 static int turns_shape(int M, int F) {
     int best = 0;
     long long least = -1;

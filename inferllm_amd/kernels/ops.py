@@ -12,8 +12,8 @@ MFMA kernels of this library when the shape fits them (few rows: decoding), and
 to the vendor GEMM through `torch.matmul` otherwise, which is where the reference
 uses a vendor GEMM too (cublasSgemm, src/kern/gpu/kernel_gpu.cu:420-435).
 
-Gate and up of 256 rows and more with their activation are an own kernel as well
-(csrc/gemm_turns.hip).
+Gate and up of 256 rows and more with their activation are an own kernel as well where that is the
+faster way (csrc/gemm_turns.hip, `turns_pays`).
 
 Five things ride on the products.  `Weight`: a matrix with a second copy in the
 kernels' own tile order (`decode_weight`).  `linear_add` / `NormedRows`: the

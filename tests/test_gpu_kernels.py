@@ -2225,3 +2225,18 @@ def test_gates_far_below_zero_in_turns():
         want[torch.exp(-z.float()).isinf()] = 0.0
         assert float(want[0].abs()) > 1e-37 or slope > 1
         assert bool(((y.double().cpu() - want).abs() <= (2.0 ** -8 + 2e-5) * want.abs()).all())
+
+
+def test_gate_up_of_many_rows_under_plans(monkeypatch):
+    """One kernel by default; the product and its activation, to the bit, under a plan saved before that kernel and where its
+    last round of blocks is nearly empty."""
+    from inferllm_amd.kernels.plan import Plan
+    o = ops()
+    old = {k: v for k, v in Plan.fixed().to_dict().items() if k != "turns"}
+    for M, F, K, plan, one in ((500, 8192, 512, Plan.fixed(), True), (500, 8192, 512, Plan.from_dict(old), False),
+                               (520, 13824, 4096, Plan.fixed(), False)):
+        x = rnd(M, K, dtype=torch.bfloat16, seed=4).to(DEV)
+        w = (torch.randn(2 * F, K, device=DEV) * K ** -0.5).to(torch.bfloat16)
+        monkeypatch.setattr(o, "_plan", plan)
+        assert o.gate_up_turns_fits(x, w) == one
+        assert torch.equal(o.gate_up_act(x, w), o.silu_mul(o.linear(x, w))) != one
