@@ -13,11 +13,12 @@
 #include "api.h"
 #include "gemm_turns.h"
 
-// g / (1 + e^-(alpha g)), within 2 in the last place of float32 wherever the result is a normal number (expf and a division
-// 1.5): e^x as 2^(x log2 e) with the product's rounding and log2 e's taken along, and the denominator's quarter, so that
+// g / (1 + e^-(alpha g)), off by at most 4.1 x 2^-24 of it wherever the result is a normal number (expf and a division
+// 3.1): e^x as 2^(x log2 e) with the product's rounding and log2 e's taken along, and the denominator's quarter, so that
 // the reciprocal of a sum of up to 2^128 is no subnormal number, which the hardware makes zero.  Nothing is under way on the
 // matrix cores while a tile's results are formed: us of 2 x 11008 x 4096, 500 / 2,048 rows, by expf and a division 92.2 / 279,
-// by this 89.3 / 271, by a plain product, exponential and reciprocal (9 in the last place at -20, zero below -87.3) 87.8 / 266.
+// by this 89.3 / 271, by a plain product, exponential and reciprocal (18 x 2^-24 down to -20, 65 to -87, zero below -87.3)
+// 87.8 / 266.
 __device__ __forceinline__ float turns_gated(float g, float alpha) {
     const float z = fminf(fmaxf(alpha * g, -128.0f), 128.0f);          // (beyond: e^-z is infinite or nothing beside 1)
     const float h = -1.44269502f * z;
