@@ -552,6 +552,22 @@ int illm_memory_finish(const float* o, const float* em, const void* w, int w_dt,
                        int z_dt, int z_stride, int z_off, void* out, int out_dt, int T, int H, int dv,
                        float eps, void* stream);
 
+// ---- single tokens, one row a sequence, through such mixers (mixer_steps.hip): head sizes to 256, U, tail and out of type dt.
+// A matrix memory in one launch: U as for illm_memory_prepare with the output gate at z_off, state [slots, H, dk, dv + 1].
+int illm_memory_step(const void* U, int dt, int u_stride, int i_off, int f_off, int z_off, const float* i_bias,
+                     const float* f_bias, float cap, float* m_state, float* state, const int32_t* row_slot,
+                     const void* w, int w_dt, void* out, int B, int H, int dk, int dv, float eps, void* stream);
+// Gated linear attention in one launch: the decays' `ra` inner numbers at a_off (ra, a_off, u_stride % 4 == 0, U and w_a2 on
+// four elements), w_a2 [H dk, ra] of type dt; out = o / rms(o) * w [dv] * silu(z).
+int illm_gla_step(const void* U, int dt, int u_stride, int q_off, int k_off, int v_off, int z_off, int a_off, int ra,
+                  const void* w_a2, const float* a2_bias, float tau, float* state, const int32_t* row_slot,
+                  const void* w, int w_dt, void* out, int B, int H, int dk, int dv, float eps, void* stream);
+// A state-space mixer in two, its tail moved on (H dv / norm_groups <= 2048); y: scratch float32 [B, H dv].
+int illm_ssm_step(const void* U, int dt, int u_stride, int x_off, int dt_off, int z_off, const float* conv_w,
+                  const float* conv_b, int taps, void* tail, float* state, const int32_t* row_slot, const float* a_log,
+                  const float* dt_bias, const float* D, float* y, const void* w, int w_dt, int norm_groups, float eps,
+                  void* out, int B, int G, int H, int N, int dv, void* stream);
+
 // ---- short causal convolutions with a kept tail, a sublayer's own norm, a clamped gate (short_conv.hip)
 // y(t) = (add_input ? in(t) : 0) + bias[c] + sum_j w[c, j] in(t - (taps - 1 - j)), in(t) = X[t, x_off + c]
 // (+ in_bias[c]); inputs before a step's first row from tail [slots, taps - 1, C]; `update_tail` (one

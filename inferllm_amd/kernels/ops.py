@@ -2288,6 +2288,84 @@ def memory_finish(o: torch.Tensor, em: torch.Tensor, weight: torch.Tensor, Z: to
     return out
 
 
+def mixer_step_fits(U: torch.Tensor, dk: int, dv: int, act_dtype: torch.dtype) -> bool:
+    """Whether csrc/mixer_steps.hip takes single tokens of these projections and head sizes."""
+    return U.is_cuda and U.dtype == act_dtype and U.is_contiguous() and U.shape[0] <= 65535 and 0 < dk <= 256 and 0 < dv <= 256
+
+
+def memory_step(U: torch.Tensor, i_off: int, f_off: int, z_off: int, i_bias: torch.Tensor, f_bias: torch.Tensor, cap: float,
+                m_state: torch.Tensor, state: torch.Tensor, row_slot: torch.Tensor, weight: torch.Tensor, H: int, dk: int,
+                dv: int, eps: float) -> torch.Tensor:
+    """One row a sequence through a matrix memory in one launch: `memory_prepare`, the plain gated rule on state float32
+    [slots, H, dk, dv + 1] and `memory_finish` with the gate at U's column z_off.  Returns [rows, H dv] of U's dtype."""
+    _gpu(U, i_bias, f_bias, m_state, state, row_slot, weight)
+    B = U.shape[0]
+    _i32(row_slot, B)
+    _columns_ok(U, "memory_step", (0, H * (2 * dk + dv)), (i_off, H), (f_off, H), (z_off, H * dv))
+    _need(all(t.dtype == torch.float32 and t.shape == (H,) for t in (i_bias, f_bias)) and m_state.dtype == torch.float32
+          and m_state.dim() == 2 and m_state.shape[1] == H and state.dtype == torch.float32
+          and state.shape[1:] == (H, dk, dv + 1) and weight.shape == (H * dv,), "memory_step: shapes")
+    out = torch.empty((B, H * dv), dtype=U.dtype, device=U.device)
+    _check(_lib().illm_memory_step(_p(U), _code(U), U.shape[1], i_off, f_off, z_off, _p(i_bias), _p(f_bias),
+                                   ctypes.c_float(cap), _p(m_state), _p(state), _p(row_slot), _p(weight), _code(weight),
+                                   _p(out), B, H, dk, dv, ctypes.c_float(eps), _stream()), "memory_step")
+    return out
+
+
+def gla_step_fits(U: torch.Tensor, a_off: int, w_a2, dk: int, dv: int, act_dtype: torch.dtype) -> bool:
+    """Whether `gla_step` takes these: as `mixer_step_fits`, the decays' inner numbers in whole groups of four."""
+    w = plain_weight(w_a2)
+    return (mixer_step_fits(U, dk, dv, act_dtype) and w.dtype == U.dtype and w.is_contiguous()
+            and (w.shape[1] | a_off | U.shape[1]) % 4 == 0 and _on16(U, w))
+
+
+def gla_step(U: torch.Tensor, q_off: int, k_off: int, v_off: int, z_off: int, a_off: int, w_a2, a2_bias: torch.Tensor,
+             tau: float, state: torch.Tensor, row_slot: torch.Tensor, weight: torch.Tensor, H: int, dk: int, dv: int,
+             eps: float) -> torch.Tensor:
+    """One row a sequence through gated linear attention in one launch: the decays' outer product (its sums stay float32),
+    `gla_prepare`, the plain gated rule on state float32 [slots, H, dk, dv] and `delta_finish` with the silu of U's columns at
+    z_off.  Returns [rows, H dv] of U's dtype."""
+    w_a2 = plain_weight(w_a2)
+    _gpu(U, w_a2, a2_bias, state, row_slot, weight)
+    B, ra = U.shape[0], w_a2.shape[1]
+    _i32(row_slot, B)
+    _columns_ok(U, "gla_step", (q_off, H * dk), (k_off, H * dk), (v_off, H * dv), (z_off, H * dv), (a_off, ra))
+    _need(w_a2.shape == (H * dk, ra) and w_a2.dtype == U.dtype and a2_bias.dtype == torch.float32 and a2_bias.shape == (H * dk,)
+          and state.dtype == torch.float32 and state.shape[1:] == (H, dk, dv) and weight.shape == (dv,), "gla_step: shapes")
+    out = torch.empty((B, H * dv), dtype=U.dtype, device=U.device)
+    _check(_lib().illm_gla_step(_p(U), _code(U), U.shape[1], q_off, k_off, v_off, z_off, a_off, ra, _p(w_a2), _p(a2_bias),
+                                ctypes.c_float(tau), _p(state), _p(row_slot), _p(weight), _code(weight), _p(out), B, H, dk, dv,
+                                ctypes.c_float(eps), _stream()), "gla_step")
+    return out
+
+
+def ssm_step_fits(U: torch.Tensor, N: int, dv: int, part: int, act_dtype: torch.dtype) -> bool:
+    """Whether `ssm_step` takes these: as `mixer_step_fits`, the norm's parts of at most 2,048 columns."""
+    return mixer_step_fits(U, N, dv, act_dtype) and part <= 2048
+
+
+def ssm_step(U: torch.Tensor, x_off: int, dt_off: int, z_off: int, conv_w: torch.Tensor, conv_b: torch.Tensor,
+             tail: torch.Tensor, state: torch.Tensor, row_slot: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
+             D: torch.Tensor, weight: torch.Tensor, norm_groups: int, eps: float, G: int, H: int, N: int, dv: int) -> torch.Tensor:
+    """One row a sequence through a state-space mixer in two launches: `ssm_prepare` with the tail's update, the plain gated rule
+    on state float32 [slots, H, N, dv] and `ssm_finish`.  Returns [rows, H dv] of U's dtype."""
+    _gpu(U, conv_w, conv_b, tail, state, row_slot, a_log, dt_bias, D, weight)
+    B, C, taps = U.shape[0], H * dv + 2 * G * N, conv_w.shape[1]
+    _i32(row_slot, B)
+    _columns_ok(U, "ssm_step", (x_off, C), (dt_off, H), (z_off, H * dv))
+    _need(conv_w.dtype == torch.float32 and conv_w.shape == (C, taps) and conv_b.dtype == torch.float32 and conv_b.shape == (C,)
+          and tail.dim() == 3 and tail.shape[1:] == (max(taps - 1, 1), C) and tail.dtype == U.dtype
+          and all(t.dtype == torch.float32 and t.shape == (H,) for t in (a_log, dt_bias, D)) and state.dtype == torch.float32
+          and state.shape[1:] == (H, N, dv) and weight.shape == (H * dv,) and H % G == 0 and (H * dv) % norm_groups == 0,
+          "ssm_step: shapes")
+    y = torch.empty((B, H * dv), dtype=torch.float32, device=U.device)
+    out = torch.empty((B, H * dv), dtype=U.dtype, device=U.device)
+    _check(_lib().illm_ssm_step(_p(U), _code(U), U.shape[1], x_off, dt_off, z_off, _p(conv_w), _p(conv_b), taps, _p(tail),
+                                _p(state), _p(row_slot), _p(a_log), _p(dt_bias), _p(D), _p(y), _p(weight), _code(weight),
+                                int(norm_groups), ctypes.c_float(eps), _p(out), B, G, H, N, dv, _stream()), "ssm_step")
+    return out
+
+
 DELTA_GATES = {"silu": 0, "sigmoid": 1}
 
 

@@ -87,6 +87,11 @@ class StateSpaceDuality(Mixer):
         U = ops.linear(h, self.w_in)
         state = ctx.cache.state_line(line)
         S, tail = state["S"], state["tail"]
+        if not ctx.prefill and ops.ssm_step_fits(U, self.N, self.dv, self.inner // self.norm_groups, ctx.act_dtype):
+            y = ops.ssm_step(U, self.inner, 2 * self.inner + 2 * self.G * self.N, 0, self.conv_w, self.conv_b, tail, S, ctx.row_slot,
+                             self.a_log, self.dt_bias, self.D, self.norm_w, self.norm_groups, self.eps, self.G, self.H, self.N,
+                             self.dv)
+            return self.leave(y, self.w_o)
         qn, kn, vv, step, dec = ops.ssm_prepare(
             U, self.inner, 2 * self.inner + 2 * self.G * self.N, self.conv_w, self.conv_b, tail,
             ctx.row_slot, self.a_log, self.dt_bias, self.G, self.H, self.N, self.dv,
@@ -163,6 +168,10 @@ class MatrixMemory(Mixer):
     def forward(self, h, ctx: StepContext, line, writes_cache, position):
         U = ops.linear(h, self.w_in)
         state = ctx.cache.state_line(line)
+        if not ctx.prefill and ops.mixer_step_fits(U, self.dk, self.dv, ctx.act_dtype):
+            y = ops.memory_step(U, self.i_off, self.f_off, self.z_off, self.i_bias, self.f_bias, self.cap, state["m"], state["S"],
+                                ctx.row_slot, self.norm_w, self.H, self.dk, self.dv, self.eps)
+            return self.leave(y, self.w_o)
         qn, kn, vv, weight, dec, em = ops.memory_prepare(
             U, self.i_off, self.f_off, self.i_bias, self.f_bias, self.cap, state["m"], ctx.cu_seqlens,
             ctx.seq_slot, ctx.n_seqs, self.H, self.dk, self.dv)
@@ -229,9 +238,13 @@ class GatedLinearAttention(Mixer):
     def forward(self, h, ctx: StepContext, line, writes_cache, position):
         H, dk, dv = self.H, self.dk, self.dv
         U = ops.linear(h, self.w_in)
+        S = ctx.cache.state_line(line)["S"]
+        if not ctx.prefill and ops.gla_step_fits(U, self.a_off, self.w_a2, dk, dv, ctx.act_dtype):
+            y = ops.gla_step(U, 0, H * dk, 2 * H * dk, self.g_off, self.a_off, self.w_a2, self.a2_bias, self.tau, S, ctx.row_slot,
+                             self.norm_w, H, dk, dv, self.eps)
+            return ops.linear(y, self.w_o)
         Z = ops.linear(U[:, self.a_off:].contiguous(), self.w_a2)
         qn, kn, vv, weight, dec = ops.gla_prepare(U, 0, H * dk, 2 * H * dk, Z, self.a2_bias, self.tau, H, dk, dv)
-        S = ctx.cache.state_line(line)["S"]
         o = ops.delta_scan(qn, kn, vv, weight, dec, S, ctx.cu_seqlens, ctx.seq_slot, ctx.n_seqs,
                            ctx.max_rows if ctx.prefill else 1, correct=False)
         y = ops.delta_finish(o, self.norm_w, U, self.g_off, "silu", self.eps, ctx.act_dtype)
