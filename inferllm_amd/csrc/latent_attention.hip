@@ -293,57 +293,71 @@ latent_absorb_q_kernel(void* __restrict__ y, int dt, int ncols, const void* __re
     for (int e = threadIdx.x; e < dr; e += blockDim.x) st_f(qa, qa_dt, dst + R + e, qs[dn + e]);
 }
 
-// The same for bfloat16 W_uk with R % 8 == 0 and R <= 512: a thread holds 8 neighbouring latent
-// dims (one 16-byte load a row of W_uk) and takes every (256 / (R / 8))-th plain dim; the groups'
-// sums are added through LDS in group order.
-template <bool FUSED>
+// The same for bfloat16 W_uk with R % 8 == 0, grid (B, H or H + 1, chunks of COLS latent dims): a thread holds 8 neighbouring
+// latent dims (one 16-byte load a row of W_uk) of every 16th plain dim (512 dims a block: every 4th), 8 rows asked for ahead of the query's way through LDS;
+// the groups' sums are added through LDS in group order.  Bound by trips to memory one after another: with the store, 16
+// heads of 128 x 512, blocks of a head's 512 dims that asked for four rows of W_uk at a time took 5.0 us for one row and 7.2
+// for 8, this 3.9 and 6.2.  More blocks than the chip takes at once (64 rows: 10.7 us) keep the 512 dims a block: 9.7.
+template <bool FUSED, int COLS>
 __global__ void __launch_bounds__(256)
 latent_absorb_q_bf16_kernel(void* __restrict__ y, int dt, int ncols,
                             const bf16_t* __restrict__ wuk, void* __restrict__ qa, int qa_dt, int H,
                             int dn, int dr, int R, LatentStore st) {
-    extern __shared__ __attribute__((aligned(16))) float sm[];
-    float* qs = sm;                       // [dn + dr]
-    float* part = sm + dn + dr;           // [groups][R]
-    const int b = blockIdx.x, h = blockIdx.y;
+    constexpr int LANES = COLS / 8, GROUPS = 256 / LANES, AHEAD = 8;
+    extern __shared__ __attribute__((aligned(16))) float qs[];           // [dn + dr]
+    __shared__ __attribute__((aligned(16))) float part[GROUPS][COLS];
+    const int b = blockIdx.x, h = blockIdx.y, r0 = blockIdx.z * COLS;
     if (FUSED && h == H) {
-        latent_store_row(b, y, dt, ncols, H, dn, dr, R, st.rot, st.cos_sin, st.max_pos, st.nw, st.nw_dt,
-                         st.eps, st.row_pos, st.row_slot, nullptr, st.cache, st.page_table,
-                         st.table_stride, st.page_size, st.ring, nullptr, nullptr, st.cache_t, false);
+        if (blockIdx.z == 0)
+            latent_store_row(b, y, dt, ncols, H, dn, dr, R, st.rot, st.cos_sin, st.max_pos, st.nw, st.nw_dt,
+                             st.eps, st.row_pos, st.row_slot, nullptr, st.cache, st.page_table,
+                             st.table_stride, st.page_size, st.ring, nullptr, nullptr, st.cache_t, false);
         return;
     }
+    const int c = threadIdx.x % LANES, g = threadIdx.x / LANES;
+    const bool live = r0 + 8 * c < R;
+    const bf16_t* const wp = wuk + (size_t)h * dn * R + (live ? r0 + 8 * c : 0);
+    uint4 u[AHEAD];
+    auto ask = [&](int d0) __attribute__((always_inline)) {              // (past the last row: the last, times nothing)
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) u[k] = *(const uint4*)(wp + (size_t)min(d0 + g + GROUPS * k, dn - 1) * R);
+    };
+    if (dn > 0) ask(0);
+    loads_asked_for();
     const size_t src = (size_t)b * ncols + (size_t)h * (dn + dr);
     for (int d = threadIdx.x; d < dn + dr; d += 256) qs[d] = ld_f(y, dt, src + d);
     __syncthreads();
     if (FUSED) rotate_in_lds(qs, dn, st, b);
-    const int per_row = R / 8, groups = 256 / per_row;
-    const int c = threadIdx.x % per_row, g = threadIdx.x / per_row;
     float acc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.f;
-    if (g < groups) {
-        const bf16_t* wp = wuk + (size_t)h * dn * R + c * 8;
-#pragma unroll 4
-        for (int d = g; d < dn; d += groups) {
-            const uint4 u = *(const uint4*)(wp + (size_t)d * R);
+    for (int d0 = 0; d0 < dn; d0 += GROUPS * AHEAD) {
+        if (d0) ask(d0);
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) {
+            const int d = d0 + g + GROUPS * k;
+            if (d >= dn) continue;
             const float q = qs[d];
-            const uint32_t uw[4] = {u.x, u.y, u.z, u.w};
+            const uint32_t uw[4] = {u[k].x, u[k].y, u[k].z, u[k].w};
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 acc[2 * i] += q * __uint_as_float(uw[i] << 16);
                 acc[2 * i + 1] += q * __uint_as_float(uw[i] & 0xffff0000u);
             }
         }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) part[(size_t)g * R + c * 8 + i] = acc[i];
     }
+#pragma unroll
+    for (int i = 0; i < 8; i += 4) *(float4*)&part[g][c * 8 + i] = make_float4(acc[i], acc[i + 1], acc[i + 2], acc[i + 3]);
     __syncthreads();
     const size_t dst = ((size_t)b * H + h) * (size_t)(R + dr);
-    for (int r = threadIdx.x; r < R; r += 256) {
+    for (int r = threadIdx.x; r < min(COLS, R - r0); r += 256) {
         float a = 0.f;
-        for (int gg = 0; gg < groups; ++gg) a += part[(size_t)gg * R + r];
-        st_f(qa, qa_dt, dst + r, a);
+#pragma unroll
+        for (int gg = 0; gg < GROUPS; ++gg) a += part[gg][r];
+        st_f(qa, qa_dt, dst + r0 + r, a);
     }
-    for (int e = threadIdx.x; e < dr; e += 256) st_f(qa, qa_dt, dst + R + e, qs[dn + e]);
+    if (blockIdx.z == 0)
+        for (int e = threadIdx.x; e < dr; e += 256) st_f(qa, qa_dt, dst + R + e, qs[dn + e]);
 }
 
 template <bool FUSED>
@@ -351,14 +365,14 @@ static int launch_absorb_q(void* y, int dt, int ncols, const void* wuk, int w_dt
                            int B, int H, int dn, int dr, int R, const LatentStore& st,
                            hipStream_t stream) {
     const dim3 grid(B, FUSED ? H + 1 : H);
-    if (w_dt == ILLM_BF16 && R % 8 == 0 && R <= 512 && R >= 8) {
-        const int groups = 256 / (R / 8);
-        const size_t smem = ((size_t)(dn + dr) + (size_t)groups * R) * sizeof(float);
-        if (smem <= 48 * 1024) {
-            hipLaunchKernelGGL(latent_absorb_q_bf16_kernel<FUSED>, grid, dim3(256), smem, stream, y, dt,
+    if (w_dt == ILLM_BF16 && R % 8 == 0 && R <= 512 && R >= 8 && (dn + dr) * sizeof(float) <= 40 * 1024 && (uintptr_t)wuk % 16 == 0) {
+        if ((long long)B * H <= 512)
+            hipLaunchKernelGGL((latent_absorb_q_bf16_kernel<FUSED, 128>), dim3(grid.x, grid.y, (R + 127) / 128), dim3(256),
+                               (dn + dr) * sizeof(float), stream, y, dt, ncols, (const bf16_t*)wuk, qa, qa_dt, H, dn, dr, R, st);
+        else
+            hipLaunchKernelGGL((latent_absorb_q_bf16_kernel<FUSED, 512>), grid, dim3(256), (dn + dr) * sizeof(float), stream, y, dt,
                                ncols, (const bf16_t*)wuk, qa, qa_dt, H, dn, dr, R, st);
-            return illm_launch_status();
-        }
+        return illm_launch_status();
     }
     hipLaunchKernelGGL(latent_absorb_q_kernel<FUSED>, grid, dim3(256), (size_t)(dn + dr) * sizeof(float),
                        stream, y, dt, ncols, wuk, w_dt, qa, qa_dt, H, dn, dr, R, st);
@@ -611,16 +625,12 @@ extern "C" int illm_latent_attn_decode(const float* qa, const void* cache, int d
 // is two 8-byte loads from the transposed copy.  Keys that are not seen get weight 0 and their
 // loaded values are masked (a freed page may hold anything).  The sums stay in registers
 // (R / 16 accumulators of 4); statistics in float32.
-// Bound by trips to memory one after another.  Latents of more than 256 dims (RT 32) ask for a tile's first values
-// ahead of its keys and for U steps of 32 dims of keys together; U is 9 where 288 divides the key's dims and 6
-// elsewhere, so that no width goes a step at a time for long.  Narrower ones have few such trips and lose
-// more to the registers: keys and values in turn (walk alone, us: 512 + 64 dims, 1 sequence of 3,000 keys 17.5 -> 15.3,
-// 32 heads, 32 sequences of 1,000 to 2,000 63.5 -> 60.4; 192 + 64 in this order 9.4 and 31.2, with the values early 10.3
-// and 35.8).
+// Bound by trips to memory one after another; keys and values are asked for in turn (with the values early 192 + 64 dims took
+// 10.3 and 35.8 us for 1 sequence of 3,000 and 32 of 1,000 to 2,000, so 9.4 and 31.2).  Wider latents: the kernel after this.
 typedef __bf16 la_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float la_f32x4_t __attribute__((ext_vector_type(4)));
 
-template <int RT, int U>
+template <int RT>
 __global__ void __launch_bounds__(64)
 latent_decode_mfma_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restrict__ cache,
                           const bf16_t* __restrict__ cache_t,
@@ -664,21 +674,8 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restric
         const bf16_t* kp1 = kp0 + (size_t)16 * D;
         la_f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
         const bf16_t* tp = cache_t + ((size_t)phys * R + r) * page_size + rowb + 4 * q;
-        constexpr bool EARLY = RT > 16;
-        constexpr int CH = EARLY ? 16 : RT < 8 ? RT : 8;            // row groups whose loads are in flight together
+        constexpr int CH = RT < 8 ? RT : 8, U = 6;          // row groups whose loads are in flight together, steps of the scores
         uint2 c0[CH], c1[CH];
-        auto values = [&](int r0) __attribute__((always_inline)) {
-#pragma unroll
-            for (int u = 0; u < CH; ++u) {
-                const int rt = (r0 + u) * 16 < R ? r0 + u : 0;      // beyond R: loaded, not used
-                c0[u] = *(const uint2*)(tp + (size_t)rt * 16 * page_size);
-                c1[u] = *(const uint2*)(tp + (size_t)rt * 16 * page_size + 16);
-            }
-        };
-        if constexpr (EARLY) {
-            values(0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
         // U steps of 32 dims at a time: all their loads are asked for before the first product
         int d0 = 0;
         for (; d0 + 32 * U <= D; d0 += 32 * U) {
@@ -689,7 +686,6 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restric
                 ka[u] = *(const la_bf16x8_t*)(kp0 + d0 + 32 * u);
                 kb[u] = *(const la_bf16x8_t*)(kp1 + d0 + 32 * u);
             }
-            if constexpr (EARLY) __builtin_amdgcn_sched_barrier(0);  // (else every product's loads are put right before it)
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[u], qv[u], s0, 0, 0, 0);
@@ -743,26 +739,20 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restric
         const uint32_t k67 = (ok[6] ? 0xffffu : 0u) | (ok[7] ? 0xffff0000u : 0u);
 #pragma unroll
         for (int r0 = 0; r0 < RT; r0 += CH) {
-            if constexpr (!EARLY) values(r0);
-            auto masked = [&](int u) __attribute__((always_inline)) {
-                uint4 cu;
-                cu.x = c0[u].x & k01; cu.y = c0[u].y & k23; cu.z = c1[u].x & k45; cu.w = c1[u].y & k67;
-                return *(const la_bf16x8_t*)&cu;
-            };
-            la_bf16x8_t cv[EARLY ? CH : 1];          // (early: out of the way of the next groups' loads)
-            if constexpr (EARLY) {
 #pragma unroll
-                for (int u = 0; u < CH; ++u) cv[u] = masked(u);
-                if (r0 + CH < RT) values(r0 + CH);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int u = 0; u < CH; ++u) {
+                const int rt = (r0 + u) * 16 < R ? r0 + u : 0;      // beyond R: loaded, not used
+                c0[u] = *(const uint2*)(tp + (size_t)rt * 16 * page_size);
+                c1[u] = *(const uint2*)(tp + (size_t)rt * 16 * page_size + 16);
             }
 #pragma unroll
             for (int u = 0; u < CH; ++u) {
                 const int rt = r0 + u;
                 if (rt * 16 < R) {
-                    const la_bf16x8_t c = EARLY ? cv[EARLY ? u : 0] : masked(u);
+                    uint4 cu;
+                    cu.x = c0[u].x & k01; cu.y = c0[u].y & k23; cu.z = c1[u].x & k45; cu.w = c1[u].y & k67;
                     o[rt][0] *= alpha; o[rt][1] *= alpha; o[rt][2] *= alpha; o[rt][3] *= alpha;
-                    o[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, pv, o[rt], 0, 0, 0);
+                    o[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const la_bf16x8_t*)&cu, pv, o[rt], 0, 0, 0);
                 }
             }
         }
@@ -781,6 +771,145 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restric
     }
 }
 
+// The same by four waves a block where R > 256: a wave takes every fourth step of 32 dims of the scores, whose parts
+// meet in LDS, then the softmax (each wave for itself) and a quarter of the latent dims of the sums: a tile's keys and values, 90 KB
+// that a single wave asks for in five turns, are one trip of four waves.  U: steps a wave, 4 U >= D / 32.
+// One wave a block -> this, us, 16 heads of 512 + 64 dims: 1 sequence of 600 / 3,000 keys 8.9 / 15.4 -> 5.9 / 9.7, 8 of 400 9.7 ->
+// 6.5, 8 of 62 to 1,040 12.6 -> 10.7, 16 of 1,000 16.2 -> 13.2, 32 of 1,500 34.6 -> 33.7, 64 of 2,000 79.7 -> 78.1.
+template <int U>
+__global__ void __launch_bounds__(256)
+latent_decode_mfma_wide_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restrict__ cache, const bf16_t* __restrict__ cache_t,
+                               const int32_t* __restrict__ page_table, int table_stride, int page_size, int ring,
+                               const int32_t* __restrict__ seq_slot, const int32_t* __restrict__ seq_len, int len_more,
+                               float* __restrict__ partial, int nsplit, int H, int R, int dr, float scale, int window) {
+    constexpr int NV = 8;                                  // row groups of 16 latent dims a wave: R <= 512
+    __shared__ la_f32x4_t part[2][4][2][64];
+    const int D = R + dr;
+    const int b = blockIdx.x, split = blockIdx.y, h0 = blockIdx.z * 16;
+    const int lane = threadIdx.x & 63, w = wave_index(), r = lane & 15, q = lane >> 4;
+    const int len = seq_len[b] + len_more, slot = seq_slot[b];
+    const int lo = window > 0 ? (len - window > 0 ? len - window : 0) : 0;
+    const int tile0 = lo / 32, tile1 = (len - 1) / 32 + 1;
+    const int per = (tile1 - tile0 + nsplit - 1) / nsplit;
+    const int ta = tile0 + split * per;
+    const int tb = ta + per < tile1 ? ta + per : tile1;
+    asm volatile("" ::"s"(slot));                    // (asked for with the length, not behind the branch)
+    const int h = h0 + r;
+    float* const dst = partial + (((size_t)b * H + min(h, H - 1)) * nsplit + split) * (size_t)(R + 4);
+    if (ta >= tb) {                                  // a range without keys: its sums are not read
+        if (w == 0 && q == 0 && h < H) {
+            dst[R] = -INFINITY;
+            dst[R + 1] = 0.f;
+        }
+        return;
+    }
+    // the wave's dims of the lane's query row (heads beyond the last read the last one's; steps past the end are zeros)
+    const bf16_t* qp = qa + ((size_t)b * H + min(h, H - 1)) * D;
+    const la_bf16x8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    int at[U];
+    bool there[U];
+    la_bf16x8_t qv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int d = 32 * (w + 4 * u) + 8 * q;
+        there[u] = d < D;
+        at[u] = there[u] ? d : 0;
+        qv[u] = *(const la_bf16x8_t*)(qp + at[u]);
+    }
+    la_f32x4_t o[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) o[v] = (la_f32x4_t){0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    for (int tile = ta; tile < tb; ++tile) {
+        const int k0 = tile * 32;
+        int lp = k0 / page_size;
+        if (ring > 0) lp %= ring;
+        const int phys = page_table[(size_t)slot * table_stride + lp];
+        const int rowb = k0 % page_size;
+        const bf16_t* kp0 = cache + ((size_t)phys * page_size + rowb + r) * D;
+        const bf16_t* kp1 = kp0 + (size_t)16 * D;
+        const bf16_t* tp = cache_t + ((size_t)phys * R + r) * page_size + rowb + 4 * q;
+        la_bf16x8_t ka[U], kb[U];
+        uint2 c0[NV], c1[NV];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            ka[u] = *(const la_bf16x8_t*)(kp0 + at[u]);
+            kb[u] = *(const la_bf16x8_t*)(kp1 + at[u]);
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const size_t row = (size_t)min((w * NV + v) * 16, R - 16) * page_size;      // beyond R: loaded, not used
+            c0[v] = *(const uint2*)(tp + row);
+            c1[v] = *(const uint2*)(tp + row + 16);
+        }
+        __builtin_amdgcn_sched_barrier(0);           // (else every product's loads are put right before it)
+        la_f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const la_bf16x8_t x = there[u] ? qv[u] : zero8;
+            s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(there[u] ? ka[u] : zero8, x, s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(there[u] ? kb[u] : zero8, x, s1, 0, 0, 0);
+        }
+        la_f32x4_t (*sums)[2][64] = part[tile & 1];
+        sums[w][0][lane] = s0;
+        sums[w][1][lane] = s1;
+        __syncthreads();
+        s0 = (sums[0][0][lane] + sums[1][0][lane]) + (sums[2][0][lane] + sums[3][0][lane]);
+        s1 = (sums[0][1][lane] + sums[1][1][lane]) + (sums[2][1][lane] + sums[3][1][lane]);
+        float sc[8];
+        bool ok[8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int p0 = k0 + 4 * q + i, p1 = p0 + 16;
+            ok[i] = p0 >= lo && p0 < len;
+            ok[4 + i] = p1 >= lo && p1 < len;
+            sc[i] = ok[i] ? s0[i] * scale : -INFINITY;
+            sc[4 + i] = ok[4 + i] ? s1[i] * scale : -INFINITY;
+        }
+        float mt = sc[0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) mt = fmaxf(mt, sc[i]);
+        mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+        const float mn = fmaxf(m, mt);
+        const float alpha = m == -INFINITY ? 0.f : expf(m - mn);
+        float pw[8], ls = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            pw[i] = ok[i] ? expf(sc[i] - mn) : 0.f;
+            ls += pw[i];
+        }
+        ls += __shfl_xor(ls, 16, 64);
+        ls += __shfl_xor(ls, 32, 64);
+        l = l * alpha + ls;
+        m = mn;
+        uint4 pu;
+        pu.x = pack_bf16x2(pw[0], pw[1]); pu.y = pack_bf16x2(pw[2], pw[3]);
+        pu.z = pack_bf16x2(pw[4], pw[5]); pu.w = pack_bf16x2(pw[6], pw[7]);
+        const la_bf16x8_t pv = *(const la_bf16x8_t*)&pu;
+        const uint32_t k01 = (ok[0] ? 0xffffu : 0u) | (ok[1] ? 0xffff0000u : 0u);
+        const uint32_t k23 = (ok[2] ? 0xffffu : 0u) | (ok[3] ? 0xffff0000u : 0u);
+        const uint32_t k45 = (ok[4] ? 0xffffu : 0u) | (ok[5] ? 0xffff0000u : 0u);
+        const uint32_t k67 = (ok[6] ? 0xffffu : 0u) | (ok[7] ? 0xffff0000u : 0u);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            uint4 cu;
+            cu.x = c0[v].x & k01; cu.y = c0[v].y & k23; cu.z = c1[v].x & k45; cu.w = c1[v].y & k67;
+            o[v][0] *= alpha; o[v][1] *= alpha; o[v][2] *= alpha; o[v][3] *= alpha;
+            o[v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const la_bf16x8_t*)&cu, pv, o[v], 0, 0, 0);
+        }
+    }
+    // o[v][i] = sum of head h over latent dim 16 (8 w + v) + 4 q + i
+    if (h < H) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int d = (w * NV + v) * 16;
+            if (d < R) *(la_f32x4_t*)(dst + d + 4 * q) = o[v];               // rows of R + 4 floats: 16-byte aligned
+        }
+        if (w == 0 && q == 0) { dst[R] = m; dst[R + 1] = l; }
+    }
+}
+
 extern "C" int illm_latent_attn_decode_mfma(const void* qa, const void* cache, const void* cache_t,
                                             const int32_t* page_table, int table_stride,
                                             int page_size, int ring, const int32_t* seq_slot,
@@ -796,16 +925,17 @@ extern "C" int illm_latent_attn_decode_mfma(const void* qa, const void* cache, c
     if (groups > 65535) return ILLM_ERR_ARG;
     const dim3 grid(B, nsplit, groups);
     hipStream_t st = (hipStream_t)stream;
-#define GO(RT_, U_)                                                                               \
-    hipLaunchKernelGGL((latent_decode_mfma_kernel<RT_, U_>), grid, dim3(64), 0, st,                \
-                       (const bf16_t*)qa, (const bf16_t*)cache, (const bf16_t*)cache_t, page_table, table_stride,     \
-                       page_size, ring, seq_slot, seq_len, len_more, partial, nsplit, H, R, dr,    \
-                       scale, window)
-    if (R <= 64) GO(4, 6);
-    else if (R <= 128) GO(8, 6);
-    else if (R <= 256) GO(16, 6);
-    else if ((R + dr) % 288) GO(32, 6);
-    else GO(32, 9);
+#define GO(KERNEL, THREADS)                                                                        \
+    hipLaunchKernelGGL(KERNEL, grid, dim3(THREADS), 0, st, (const bf16_t*)qa, (const bf16_t*)cache, (const bf16_t*)cache_t, \
+                       page_table, table_stride, page_size, ring, seq_slot, seq_len, len_more, partial, nsplit, H, R, dr, scale, \
+                       window)
+    if (R <= 64) GO(latent_decode_mfma_kernel<4>, 64);
+    else if (R <= 128) GO(latent_decode_mfma_kernel<8>, 64);
+    else if (R <= 256) GO(latent_decode_mfma_kernel<16>, 64);
+    else if (R + dr <= 512) GO(latent_decode_mfma_wide_kernel<4>, 256);
+    else if (R + dr <= 640) GO(latent_decode_mfma_wide_kernel<5>, 256);
+    else if (R + dr <= 1024) GO(latent_decode_mfma_wide_kernel<8>, 256);
+    else GO(latent_decode_mfma_kernel<32>, 64);
 #undef GO
     return illm_launch_status();
 }
@@ -943,6 +1073,99 @@ latent_merge_up_kernel(const float* __restrict__ partial, int nsplit, const void
     }
 }
 
+// The same for 256 < R <= 512 and bfloat16 W_uv: everything is asked for at once, the block's 32 rows of W_uv (eight a wave),
+// the ranges' statistics and the first 16 ranges' sums, whether they hold keys or not (what a range without keys holds is
+// dropped).  us, 128 value dims, one trip after another -> this: one row and 19 ranges 6.6 -> 5.4,
+// 8 rows of 13 ranges 8.0 -> 6.1, of up to 33 8.4 -> 7.2; 16 of 32 10.0 both, 32 rows and more, whose blocks are more than the
+// chip takes at once and hide each other's trips, 15.3 -> 19.2.  Blocks of one head follow each other 8 apart where heads are a
+// multiple of 8: its rows of W_uv stay in one XCD's L2.
+__global__ void __launch_bounds__(256)
+latent_merge_up_wide_kernel(const float* __restrict__ partial, int nsplit, const bf16_t* __restrict__ wuv,
+                            const void* __restrict__ y, int dt, int ncols, int gate_off, void* __restrict__ out, int H, int R,
+                            int dv) {
+    extern __shared__ __attribute__((aligned(16))) float ws[];      // [nsplit] weights
+    __shared__ __attribute__((aligned(16))) float sums[2][512];
+    __shared__ int filled;                                // ranges up to the last that holds keys
+    const int h = blockIdx.x, b = blockIdx.y, lane = threadIdx.x & 63, w = wave_index();
+    const float* const base = partial + ((size_t)b * H + h) * nsplit * (size_t)(R + 4);
+    auto stat = [&](int s, int i, float none) __attribute__((always_inline)) {
+        return s < nsplit ? base[(size_t)s * (R + 4) + R + i] : none;
+    };
+    float m0 = -INFINITY, l0 = 0.f;
+    if (w == 0) { m0 = stat(lane, 0, -INFINITY); l0 = stat(lane, 1, 0.f); }
+    // a thread takes four neighbouring dims of every other range
+    const int dim = (threadIdx.x & 127) * 4, mine = threadIdx.x >> 7;
+    float4 v[8];
+    auto ask = [&](int s0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            v[u] = *(const float4*)(base + (size_t)min(s0 + 2 * u + mine, nsplit - 1) * (R + 4) + min(dim, R - 4));
+    };
+    ask(0);
+    const float gv = ld_f(y, dt, (size_t)b * ncols + gate_off + h);
+    const int at = min(lane * 8, R - 8), v0 = blockIdx.z * 32 + 8 * w;
+    uint4 up[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) up[j] = *(const uint4*)(wuv + ((size_t)h * dv + min(v0 + j, dv - 1)) * R + at);
+    loads_asked_for();
+    if (w == 0) {
+        // lane s holds range s, s + 64, ...; weights exp(m_s - M) / total
+        float M = m0;
+        for (int s = lane + 64; s < nsplit; s += 64) M = fmaxf(M, stat(s, 0, -INFINITY));
+        M = wave_max(M);
+        float tot = 0.f;
+        int last = 0;
+        for (int s0 = 0; s0 < nsplit; s0 += 64) {
+            const float ms = s0 ? stat(s0 + lane, 0, -INFINITY) : m0, ls = s0 ? stat(s0 + lane, 1, 0.f) : l0;
+            const float e = ms == -INFINITY ? 0.f : expf(ms - M);
+            tot += ls * e;
+            if (s0 + lane < nsplit) ws[s0 + lane] = e;
+            const unsigned long long some = __ballot(ms != -INFINITY);
+            if (some) last = s0 + 64 - __clzll(some);
+        }
+        tot = wave_sum(tot);
+        if (lane == 0) filled = last;
+        for (int s = lane; s < nsplit; s += 64) ws[s] = ws[s] / tot;
+    }
+    __syncthreads();
+    const int ranges = filled;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s0 = 0; s0 < ranges; s0 += 16) {
+        if (s0) ask(s0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int s = s0 + 2 * u + mine;
+            if (s >= ranges) continue;
+            const float g = ws[s];
+            a.x += v[u].x * g; a.y += v[u].y * g; a.z += v[u].z * g; a.w += v[u].w * g;
+        }
+    }
+    *(float4*)&sums[mine][dim] = a;
+    __syncthreads();
+    const float gate = 1.0f / (1.0f + expf(-gv));
+    float c[8], dot[8];
+    const bool live = lane * 8 < R;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) c[i] = live ? sums[0][at + i] + sums[1][at + i] : 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const uint32_t uw[4] = {up[j].x, up[j].y, up[j].z, up[j].w};
+        dot[j] = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            dot[j] += __uint_as_float(uw[i] << 16) * c[2 * i];
+            dot[j] += __uint_as_float(uw[i] & 0xffff0000u) * c[2 * i + 1];
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) dot[j] += __shfl_xor(dot[j], o, 64);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        if (lane == j && v0 + j < dv) st_f(out, dt, (size_t)b * H * dv + (size_t)h * dv + v0 + j, dot[j] * gate);
+}
+
 extern "C" int illm_latent_merge_up(const float* partial, int nsplit, const void* wuv, int w_dt,
                                     const void* y, int dt, int ncols, int gate_off, void* out,
                                     int B, int H, int R, int dv, void* stream) {
@@ -951,6 +1174,12 @@ extern "C" int illm_latent_merge_up(const float* partial, int nsplit, const void
         return ILLM_ERR_ARG;
     if (B == 0) return ILLM_OK;
     if ((dv + 31) / 32 > 65535) return ILLM_ERR_ARG;
+    if ((long long)B * H <= 128 && R > 256 && R <= 512 && R % 8 == 0 && w_dt == ILLM_BF16 && nsplit <= 8192 &&
+        ((uintptr_t)partial | (uintptr_t)wuv) % 16 == 0) {
+        hipLaunchKernelGGL(latent_merge_up_wide_kernel, dim3(H, B, (dv + 31) / 32), dim3(256), (size_t)nsplit * sizeof(float),
+                           (hipStream_t)stream, partial, nsplit, (const bf16_t*)wuv, y, dt, ncols, gate_off, out, H, R, dv);
+        return illm_launch_status();
+    }
     hipLaunchKernelGGL(latent_merge_up_kernel, dim3(B, H, (dv + 31) / 32), dim3(256), (size_t)(R + nsplit + 4 + (R % 4 == 0 && R <= 1024 ? 1024 : 0)) * sizeof(float),
                        (hipStream_t)stream, partial, nsplit, wuv, w_dt, y, dt, ncols, gate_off, out,
                        H, R, dv);
