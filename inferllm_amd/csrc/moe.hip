@@ -87,9 +87,13 @@ few_outputs_few_tokens_kernel(const void* __restrict__ x, const float* __restric
 }
 
 // More tokens: a wave takes 4 outputs and 8 tokens at a time (a chunk of a row of w serves 8 tokens, a chunk of
-// a token's row 4 outputs).  grid (ceil(T / 8), ceil(NE / 16)).
+// a token's row 4 outputs), V neighbouring k a lane, the next turn's loads on their way beside this turn's products.  Rows past
+// the last are the last again: a load behind a branch on the type or the row is waited for before the next is asked
+// for, which had been the kernel's time (64 outputs of K = 2,048 for 64 / 2,964 bfloat16 tokens
+// 15 / 73 -> 8.5 / 26 us, 160 of 5,120 for 2,964 444 -> 132).  grid (ceil(T / 8), ceil(NE / 16)).
+template <int DT, int V>
 __global__ void __launch_bounds__(256)
-few_outputs_f32_kernel(const void* __restrict__ x, int x_dt, const float* __restrict__ w,
+few_outputs_f32_kernel(const void* __restrict__ x, const float* __restrict__ w,
                        float* __restrict__ z, int T, int NE, int K) {
     const int t0 = blockIdx.x * 8;
     const int e0 = (blockIdx.y * 4 + wave_index()) * 4, lane = threadIdx.x & 63;
@@ -100,40 +104,51 @@ few_outputs_f32_kernel(const void* __restrict__ x, int x_dt, const float* __rest
 #pragma unroll
     for (int j = 0; j < 4; ++j) wr[j] = w + (size_t)(e0 + j < NE ? e0 + j : NE - 1) * K;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) xr[i] = (size_t)(i < nt ? t0 + i : t0) * K;
+    for (int i = 0; i < 8; ++i) xr[i] = (size_t)min(t0 + i, T - 1) * K;
     float v[32];                                        // sum 4 i + j: token i, output j
 #pragma unroll
     for (int i = 0; i < 32; ++i) v[i] = 0.f;
-    if (K % 4 == 0) {
-        // four neighbouring k a lane: one 16-byte load of w and one of 8 or 16 bytes of x
-#pragma unroll 2
-        for (int k = lane * 4; k < K; k += 256) {
-            float4 wv[4], xv[8];
+    // (as they lie in memory: 4, 8 or 16 bytes)
+    typedef float w_t __attribute__((ext_vector_type(V)));
+    typedef uint32_t h_t __attribute__((ext_vector_type(V == 4 ? 2 : 1)));
+    struct Turn { w_t w[4], x[DT == ILLM_F32 ? 8 : 1]; h_t h[DT == ILLM_BF16 ? 8 : 1]; };
+    auto ask = [&](Turn& t, int k) __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) wv[j] = *(const float4*)(wr[j] + k);
+        for (int j = 0; j < 4; ++j) t.w[j] = *(const w_t*)(wr[j] + k);
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-                xv[i] = i < nt ? ld4_f32(x, x_dt, xr[i] + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    v[4 * i + j] += xv[i].x * wv[j].x; v[4 * i + j] += xv[i].y * wv[j].y;
-                    v[4 * i + j] += xv[i].z * wv[j].z; v[4 * i + j] += xv[i].w * wv[j].w;
-                }
+        for (int i = 0; i < 8; ++i) {
+            if constexpr (DT == ILLM_F32) t.x[i] = *(const w_t*)((const float*)x + xr[i] + k);
+            else if constexpr (V == 4) t.h[i] = *(const h_t*)((const bf16_t*)x + xr[i] + k);
+            else t.h[i] = ((const bf16_t*)x)[xr[i] + k];
         }
-    } else {
-#pragma unroll 4
-        for (int k = lane; k < K; k += 64) {
-            float wv[4], xv[8];
+    };
+    auto add = [&](const Turn& t) __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) wv[j] = wr[j][k];
+        for (int i = 0; i < 8; ++i) {
+            float xv[V];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) xv[i] = i < nt ? ld_f(x, x_dt, xr[i] + k) : 0.f;
+            for (int e = 0; e < V; ++e) {
+                if constexpr (DT == ILLM_F32) xv[e] = t.x[i][e];
+                else xv[e] = __uint_as_float(V == 1 || !(e & 1) ? t.h[i][e / 2] << 16 : t.h[i][e / 2] & 0xffff0000u);
+            }
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) v[4 * i + j] += xv[i] * wv[j];
+                for (int e = 0; e < V; ++e) v[4 * i + j] += xv[e] * t.w[j][e];
+        }
+    };
+    const int first = lane * V, step = 64 * V;
+    if (first < K) {
+        Turn t0_, t1_;
+        ask(t0_, first);
+        for (int k = first; k < K; k += 2 * step) {
+            ask(t1_, k + step < K ? k + step : first);  // (past K: the first turn's again, not used)
+            __builtin_amdgcn_sched_barrier(0);
+            add(t0_);
+            if (k + step >= K) break;
+            ask(t0_, k + 2 * step < K ? k + 2 * step : first);
+            __builtin_amdgcn_sched_barrier(0);
+            add(t1_);
         }
     }
     // 32 sums over 64 lanes by halving: at the step that pairs lanes l and l ^ b a lane keeps the sums whose
@@ -170,8 +185,14 @@ extern "C" int illm_few_outputs_f32(const void* x, int x_dt, const float* w, flo
 #undef GO
         return illm_launch_status();
     }
-    hipLaunchKernelGGL(few_outputs_f32_kernel, dim3((T + 7) / 8, (NE + 15) / 16), dim3(256), 0, st, x, x_dt, w, z, T,
-                       NE, K);
+#define GO(DT_, V_)                                                                                          \
+    hipLaunchKernelGGL((few_outputs_f32_kernel<DT_, V_>), dim3((T + 7) / 8, (NE + 15) / 16), dim3(256), 0, st, x, w, z, T, NE, K)
+    if (K % 4) {
+        if (x_dt == ILLM_BF16) GO(ILLM_BF16, 1);
+        else GO(ILLM_F32, 1);
+    } else if (x_dt == ILLM_BF16) GO(ILLM_BF16, 4);
+    else GO(ILLM_F32, 4);
+#undef GO
     return illm_launch_status();
 }
 
