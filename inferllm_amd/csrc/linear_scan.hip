@@ -205,6 +205,49 @@ ssm_finish_kernel(const float* __restrict__ o, const float* __restrict__ x,
     }
 }
 
+// The same in one pass where four columns lie together: a thread holds up to four groups of four columns, o, x, z and w asked for
+// together.  Bound by memory's bytes: 2,964 rows of 4,096 columns in 8 parts, a column at a time and everything read twice, 59 us,
+// this 23.
+template <int E>
+__global__ void __launch_bounds__(256)
+ssm_finish_vec4_kernel(const float* __restrict__ o, const float* __restrict__ x, const float* __restrict__ D,
+                       const void* __restrict__ Z, int z_dt, int z_stride, int z_off, const void* __restrict__ w, int w_dt,
+                       void* __restrict__ out, int out_dt, int inner, int dv, int part, float eps) {
+    __shared__ float red[16];
+    const size_t r = blockIdx.x;
+    const int j0 = blockIdx.y * part;
+    float4 ov[E], xv[E], wv[E];
+    AnyRaw4 zr[E];
+    float d[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int j = j0 + min(4 * (int)(threadIdx.x + blockDim.x * e), part - 4);         // (past the part: its last, not used)
+        ov[e] = ((const float4*)o)[(r * inner + j) / 4];
+        xv[e] = ((const float4*)x)[(r * inner + j) / 4];
+        zr[e] = ld_raw4(Z, z_dt, (r * z_stride + z_off + j) / 4);
+        wv[e] = ld_f4_any(w, w_dt, j / 4);
+        d[e] = D[j / dv];
+    }
+    loads_asked_for();
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const float4 z = raw4_f(zr[e], z_dt);
+        ov[e] = make_float4(fmaf(d[e], xv[e].x, ov[e].x) * (z.x * ls_sigmoid(z.x)), fmaf(d[e], xv[e].y, ov[e].y) * (z.y * ls_sigmoid(z.y)),
+                            fmaf(d[e], xv[e].z, ov[e].z) * (z.z * ls_sigmoid(z.z)), fmaf(d[e], xv[e].w, ov[e].w) * (z.w * ls_sigmoid(z.w)));
+        if (4 * (int)(threadIdx.x + blockDim.x * e) < part) ss += sum_sq(ov[e]);
+    }
+    ss = block_sum(ss, red);
+    const float inv = 1.0f / sqrtf(ss / (float)part + eps);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int j = 4 * (int)(threadIdx.x + blockDim.x * e);
+        if (j < part)
+            st_f4(out, out_dt, (r * inner + j0 + j) / 4, make_float4((ov[e].x * inv) * wv[e].x, (ov[e].y * inv) * wv[e].y,
+                                                                     (ov[e].z * inv) * wv[e].z, (ov[e].w * inv) * wv[e].w));
+    }
+}
+
 extern "C" int illm_ssm_finish(const float* o, const float* x, const float* D, const void* Z, int z_dt,
                                int z_stride, int z_off, const void* w, int w_dt, void* out, int out_dt,
                                int T, int H, int dv, int norm_groups, float eps, void* stream) {
@@ -213,15 +256,31 @@ extern "C" int illm_ssm_finish(const float* o, const float* x, const float* D, c
         z_off < 0 || z_off + H * dv > z_stride)
         return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
+    const int part = (H * dv) / norm_groups;
+    auto four = [](int dt) { return (uintptr_t)(dt == ILLM_BF16 ? 8 : 16); };
+    if (part % 4 == 0 && part <= 4096 && dv % 4 == 0 && z_off % 4 == 0 && z_stride % 4 == 0 &&
+        ((uintptr_t)o | (uintptr_t)x) % 16 == 0 && (uintptr_t)Z % four(z_dt) == 0 && (uintptr_t)w % four(w_dt) == 0 &&
+        (uintptr_t)out % four(out_dt) == 0) {
+        const int units = part / 4, threads = units >= 256 ? 256 : (units + 63) / 64 * 64, each = (units + threads - 1) / threads;
+#define GO(E)                                                                                                          \
+    hipLaunchKernelGGL(ssm_finish_vec4_kernel<E>, dim3(T, norm_groups), dim3(threads), 0, (hipStream_t)stream, o, x, D, Z, z_dt, \
+                       z_stride, z_off, w, w_dt, out, out_dt, H * dv, dv, part, eps)
+        if (each <= 1) GO(1);
+        else if (each <= 2) GO(2);
+        else GO(4);
+#undef GO
+        return illm_launch_status();
+    }
     hipLaunchKernelGGL(ssm_finish_kernel, dim3(T, norm_groups), dim3(256), 0, (hipStream_t)stream, o, x, D,
                        Z, z_dt, z_stride, z_off, w, w_dt, out, out_dt, H * dv, dv, (H * dv) / norm_groups, eps);
     return illm_launch_status();
 }
 
 // ---------------------------------------------------------------- matrix memory
-// The gates of sequence b and head h, one wave.  64 tokens at a time: every lane forms its token's two gates, then
-// the running maximum goes through the 64 tokens in order (the lanes' values are read one after the
-// other as scalars), and every lane leaves its token's decay, weight and exp(-m).
+// The gates of sequence b and head h, one wave, 64 tokens at a time, the next ones' pre-activations on their way.  A token turns
+// the maximum m into max(f + m, i); two such steps, (f, i) and then (f', i'), are the one step (f + f', max(i + f', i')), so the
+// maxima of 64 tokens are a scan of six exchanges (one token after the other as scalars: 2,048 tokens of 16 heads of 128 129 us with the
+// rows' conversion beside it, now 42; 8 sequences of 61 to 1,024 68 -> 27).
 template <int DT>
 static __device__ __forceinline__ void
 memory_gates(int b, int h, const void* __restrict__ U, int u_stride, int i_off, int f_off,
@@ -235,21 +294,29 @@ memory_gates(int b, int h, const void* __restrict__ U, int u_stride, int i_off, 
     const int slot = seq_slot[b];
     const float bi = i_bias[h], bf = f_bias[h], inv_cap = 1.0f / cap;
     float m = m_state[(size_t)slot * H + h];
+    auto row_of = [&](int t0) { return (size_t)(r0 + min(t0 + lane, n - 1)); };
+    float iu = ld_f(U, DT, row_of(0) * u_stride + i_off + h), fu = ld_f(U, DT, row_of(0) * u_stride + f_off + h);
     for (int t0 = 0; t0 < n; t0 += 64) {
         const bool ok = t0 + lane < n;
-        const size_t row = (size_t)(r0 + (ok ? t0 + lane : n - 1));
-        const float ig = ok ? cap * tanhf((ld_f(U, DT, row * u_stride + i_off + h) + bi) * inv_cap) : -INFINITY;
-        const float fg = ok ? ls_log_sigmoid(cap * tanhf((ld_f(U, DT, row * u_stride + f_off + h) + bf) * inv_cap)) : 0.f;
-        float m_before = 0.f, m_mine = 0.f;
-        const int tokens = min(64, n - t0);             // (all 64 turns took 6 us of a single token's step)
-        for (int l = 0; l < tokens; ++l) {
-            const float fl = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(fg), l));
-            const float il = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ig), l));
-            const float m_new = fmaxf(fl + m, il);
-            if (lane == l) { m_before = m; m_mine = m_new; }
-            m = m_new;
+        const float ig = ok ? cap * tanhf((iu + bi) * inv_cap) : -INFINITY;
+        const float fg = ok ? ls_log_sigmoid(cap * tanhf((fu + bf) * inv_cap)) : 0.f;
+        if (t0 + 64 < n) {
+            iu = ld_f(U, DT, row_of(t0 + 64) * u_stride + i_off + h);
+            fu = ld_f(U, DT, row_of(t0 + 64) * u_stride + f_off + h);
         }
+        float F = fg, I = ig;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const float fp = __shfl_up(F, d, ILLM_WAVE), ip = __shfl_up(I, d, ILLM_WAVE);
+            if (lane >= d) {
+                I = fmaxf(ip + F, I);
+                F = fp + F;
+            }
+        }
+        const float m_mine = fmaxf(F + m, I), left = __shfl_up(m_mine, 1, ILLM_WAVE), m_before = lane ? left : m;
+        m = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(m_mine), 63));      // (past the last token: its maximum)
         if (ok) {
+            const size_t row = row_of(t0);
             dec[row * H + h] = expf(fg + m_before - m_mine);
             beta[row * H + h] = expf(ig - m_mine);
             em[row * H + h] = expf(-m_mine);
@@ -261,8 +328,7 @@ memory_gates(int b, int h, const void* __restrict__ U, int u_stride, int i_off, 
 // grid (gate blocks + rows, ceil(max(H dk, H (dv + 1)) / 256)); 256 threads, an entry of q, k and v each (a block a row, which
 // went through them one after another, took 9.3 us for 8 rows of 2,048, this 4.7).  The first blocks of the grid's first row
 // take four (sequence, head) pairs' gates each, which need nothing of the rest: as a kernel behind the
-// rows -> beside them, 16 heads of 128 x 128, 1 / 8 / 64 single tokens 5.0 / 4.6 / 5.1 -> 3.7 / 4.0 / 3.6 us, 8 sequences of 61 to
-// 1,024 tokens 87.9 -> 67.6, one of 2,048 147 -> 129 (the gates' chain of tokens bounds these).
+// rows -> beside them, 16 heads of 128 x 128, 1 / 8 / 64 single tokens 5.0 / 4.6 / 5.1 -> 3.7 / 4.0 / 3.6 us.
 // U [T, u_stride] = [q (H dk) | k (H dk) | v (H dv) | ...].
 template <int DT>
 __global__ void __launch_bounds__(256)
@@ -320,16 +386,45 @@ extern "C" int illm_memory_prepare(const void* U, int dt, int u_stride, int i_of
     return illm_launch_status();
 }
 
-// grid (rows, H); one wave.  o [T, H, dv + 1]: the last column is n . q.
+// grid (rows, ceil(H / 4)); a wave a head.  o [T, H, dv + 1]: the last column is n . q.
 //   y_j = o_j / (max(|n . q|, exp(-m)) + 1e-6);  out = y / sqrt(mean_j y^2 + eps) * w[h dv + j] * sigmoid(z)
-__global__ void __launch_bounds__(64)
+// Heads of up to 64 CS columns (CS 0: any) in one pass, a lane's columns, z and w asked for together: 2,964 rows of 16 heads of
+// 128, a block a head and everything read when it is needed 25 us, this 21.
+template <int CS>
+__global__ void __launch_bounds__(256)
 memory_finish_kernel(const float* __restrict__ o, const float* __restrict__ em,
                      const void* __restrict__ w, int w_dt, const void* __restrict__ Z, int z_dt,
                      int z_stride, int z_off, void* __restrict__ out, int out_dt, int H, int dv, float eps) {
     const size_t r = blockIdx.x;
-    const int h = blockIdx.y, lane = threadIdx.x;
+    const int h = blockIdx.y * 4 + wave_index(), lane = threadIdx.x & 63;
+    if (h >= H) return;
     const float* op = o + (r * H + h) * (dv + 1);
-    const float den = fmaxf(fabsf(op[dv]), em[r * H + h]) + 1e-6f;
+    const size_t z0 = r * z_stride + z_off + (size_t)h * dv;
+    const float nq = op[dv], e0 = em[r * H + h];
+    if constexpr (CS > 0) {
+        float y[CS], z[CS], wt[CS];
+#pragma unroll
+        for (int c = 0; c < CS; ++c) {
+            const int j = min(lane + 64 * c, dv - 1);
+            y[c] = op[j];
+            z[c] = ld_f(Z, z_dt, z0 + j);
+            wt[c] = ld_f(w, w_dt, (size_t)h * dv + j);
+        }
+        const float den = fmaxf(fabsf(nq), e0) + 1e-6f;
+        float ss = 0.f;
+#pragma unroll
+        for (int c = 0; c < CS; ++c) {
+            y[c] /= den;
+            if (lane + 64 * c < dv) ss += y[c] * y[c];
+        }
+        const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)dv + eps);
+#pragma unroll
+        for (int c = 0; c < CS; ++c)
+            if (lane + 64 * c < dv)
+                st_f(out, out_dt, (r * H + h) * dv + lane + 64 * c, (y[c] * inv) * wt[c] * ls_sigmoid(z[c]));
+        return;
+    }
+    const float den = fmaxf(fabsf(nq), e0) + 1e-6f;
     float ss = 0.f;
     for (int j = lane; j < dv; j += 64) {
         const float y = op[j] / den;
@@ -337,11 +432,9 @@ memory_finish_kernel(const float* __restrict__ o, const float* __restrict__ em,
     }
     ss = wave_sum(ss);
     const float inv = 1.0f / sqrtf(ss / (float)dv + eps);
-    for (int j = lane; j < dv; j += 64) {
-        const float z = ld_f(Z, z_dt, r * z_stride + z_off + (size_t)h * dv + j);
+    for (int j = lane; j < dv; j += 64)
         st_f(out, out_dt, (r * H + h) * dv + j,
-             ((op[j] / den) * inv) * ld_f(w, w_dt, (size_t)h * dv + j) * ls_sigmoid(z));
-    }
+             ((op[j] / den) * inv) * ld_f(w, w_dt, (size_t)h * dv + j) * ls_sigmoid(ld_f(Z, z_dt, z0 + j)));
 }
 
 extern "C" int illm_memory_finish(const float* o, const float* em, const void* w, int w_dt, const void* Z,
@@ -351,8 +444,14 @@ extern "C" int illm_memory_finish(const float* o, const float* em, const void* w
         !illm_dtype_ok(out_dt) || z_off < 0 || z_off + H * dv > z_stride)
         return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
-    hipLaunchKernelGGL(memory_finish_kernel, dim3(T, H), dim3(64), 0, (hipStream_t)stream, o, em, w, w_dt, Z,
-                       z_dt, z_stride, z_off, out, out_dt, H, dv, eps);
+#define GO(CS)                                                                                                         \
+    hipLaunchKernelGGL(memory_finish_kernel<CS>, dim3(T, (H + 3) / 4), dim3(256), 0, (hipStream_t)stream, o, em, w, w_dt, Z, \
+                       z_dt, z_stride, z_off, out, out_dt, H, dv, eps)
+    if (dv <= 64) GO(1);
+    else if (dv <= 128) GO(2);
+    else if (dv <= 256) GO(4);
+    else GO(0);
+#undef GO
     return illm_launch_status();
 }
 
@@ -611,6 +710,85 @@ lru_gates_few_kernel(const float* __restrict__ u, const float* __restrict__ Wt, 
     }
 }
 
+// Steps of many rows and maps of whole waves of outputs (cb % 64 == 0), again the same sums: 16 rows and up to 256 outputs a
+// block, grid (ceil(T / 16), nb, ceil(cb / 256)); a wave has 64 outputs' gates of one slice of the inputs.  The rows' inputs
+// are the same for a wave's lanes and come through the scalar cache, so that the loop is the weights' loads and multiply-adds
+// with a scalar operand (by way of LDS its reads took as long as they).  us, that kernel -> this: 200 / 2,964 rows of 16 maps of
+// 128 x 128 28 / 126 -> 19 / 86, 2,964 of 8 of 256 x 256 247 -> 137, of 16 of 256 x 256 334 -> 247.  (The next turn's weights ahead, or
+// 4 or 16 inputs a turn: no faster.)
+__global__ void __launch_bounds__(256)
+lru_gates_rows_kernel(const float* __restrict__ u, const float* __restrict__ Wt, const float* __restrict__ br,
+                      const float* __restrict__ bi, const float* __restrict__ lam, float rate,
+                      float* __restrict__ a_out, float* __restrict__ x_out, int T, int C, int cb, int S) {
+    constexpr int ROWS = 16, IN = 8;                     // IN: inputs a turn
+    extern __shared__ __attribute__((aligned(16))) float part[];      // [S - 1][cb][2 ROWS] sums of the slices after the first
+    const int t0 = blockIdx.x * ROWS, b = blockIdx.y, nb = C / cb, rows = min(ROWS, T - t0);
+    const int lane = threadIdx.x & 63, wave = wave_index(), chunks = S > 1 ? cb / 64 : 4;
+    const int sl = wave / chunks, o = (blockIdx.z * 4 + wave % chunks) * 64 + lane;
+    const bool live = sl < S && o < cb;                  // (a wave's lanes alike)
+    const int per = cb / S;
+    float ar[ROWS], ai[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) ar[r] = ai[r] = 0.f;
+    if (live) {
+        const float* const wr = Wt + (size_t)b * cb * cb + o;
+        const float* const wi = Wt + ((size_t)nb + b) * cb * cb + o;
+        const float* const up = u + (size_t)t0 * C + (size_t)b * cb;
+        for (int i0 = sl * per; i0 < (sl + 1) * per; i0 += IN) {
+            float w1[IN], w2[IN];
+#pragma unroll
+            for (int k = 0; k < IN; ++k) {
+                w1[k] = wr[(size_t)(i0 + k) * cb];
+                w2[k] = wi[(size_t)(i0 + k) * cb];
+            }
+#pragma unroll
+            for (int k4 = 0; k4 < IN; k4 += 4)
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) {
+                    const float4 x = *(const float4*)(up + (size_t)min(r, rows - 1) * C + i0 + k4);
+                    const float xs[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        ar[r] = fmaf(w1[k4 + k], xs[k], ar[r]);
+                        ai[r] = fmaf(w2[k4 + k], xs[k], ai[r]);
+                    }
+                }
+        }
+    }
+    if (S > 1) {
+        if (live && sl > 0) {
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                part[(((size_t)(sl - 1) * 2 * ROWS) + r) * cb + o] = ar[r];
+                part[(((size_t)(sl - 1) * 2 * ROWS) + ROWS + r) * cb + o] = ai[r];
+            }
+        }
+        __syncthreads();
+        if (sl == 0)
+            for (int s = 1; s < S; ++s)
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) {
+                    ar[r] += part[((size_t)(s - 1) * 2 * ROWS + r) * cb + o];
+                    ai[r] += part[((size_t)(s - 1) * 2 * ROWS + ROWS + r) * cb + o];
+                }
+    }
+    if (!live || sl > 0) return;
+    const int c = b * cb + o;
+    const float sp = ls_softplus(lam[c]), b1 = br[c], b2 = bi[c];
+    float x[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) x[r] = u[(size_t)min(t0 + r, T - 1) * C + c];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        if (r >= rows) continue;
+        const float rg = ls_sigmoid(ar[r] + b1), ig = ls_sigmoid(ai[r] + b2);
+        const float log_a = -rate * rg * sp;
+        a_out[(size_t)(t0 + r) * C + c] = expf(log_a);
+        // 1 - a^2 as -expm1(2 log a): a decay close to 1 keeps its digits
+        x_out[(size_t)(t0 + r) * C + c] = sqrtf(fmaxf(-expm1f(2.0f * log_a), 0.f)) * ig * x[r];
+    }
+}
+
 template <int ROWS>
 static int lru_gates_launch(const float* u, const float* Wt, const float* br, const float* bi,
                             const float* lam, float rate, float* a_out, float* x_out, int T, int C,
@@ -649,6 +827,13 @@ extern "C" int illm_lru_gates(const float* u, const float* Wt, const float* br, 
         if ((cb + S - 1) / S <= 32) GO(16);
         else GO(32);
 #undef GO
+        return illm_launch_status();
+    }
+    if (T > 128 && cb % 64 == 0 && cb <= 4096 && (uintptr_t)u % 16 == 0) {
+        const int S = cb < 256 ? 256 / cb : 1;
+        const size_t lds = (size_t)(S - 1) * cb * 32 * sizeof(float);
+        hipLaunchKernelGGL(lru_gates_rows_kernel, dim3((T + 15) / 16, nb, (cb + 255) / 256), dim3(256), lds, (hipStream_t)stream, u,
+                           Wt, br, bi, lam, rate, a_out, x_out, T, C, cb, S);
         return illm_launch_status();
     }
     // tiles of 16 rows where a block's inputs of 16 rows fit LDS (blocks of up to 1,024 channels)

@@ -90,3 +90,48 @@ def test_state_space_step(N, dv, G, H, taps, groups, dtype):
     _near(got, R.ssm_finish(o, v, D, U, 0, w, groups, 1e-5, torch.float32), dtype)
     _near(S_got, S, torch.float32)
     assert torch.equal(t_got.cpu(), tail)
+
+
+@pytest.mark.parametrize("H, dk, lens", [(3, 8, [64, 1, 65]), (2, 4, [63, 500]), (1, 4, [128])])
+def test_matrix_memory_gates_of_long_runs(H, dk, lens):
+    """Maxima by a scan of 64 tokens: its edges, gates that stay far below the maximum for many tokens (whose decays add up) and
+    gates that take it over."""
+    from inferllm_amd.kernels import ops
+    g = torch.Generator().manual_seed(sum(lens))
+    T, n, cap = sum(lens), len(lens), 15.0
+    i_off = 3 * H * dk
+    U = torch.randn(T, i_off + 2 * H, generator=g) * 4
+    U[::7, i_off:i_off + H] -= 40.0
+    slot = torch.randperm(n + 1, generator=g)[:n].to(torch.int32)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    bias, m = torch.randn(2, H, generator=g), torch.randn(n + 1, H, generator=g)
+    m_got = m.cuda()
+    got = ops.memory_prepare(U.cuda(), i_off, i_off + H, bias[0].cuda(), bias[1].cuda(), cap, m_got, cu.cuda(), slot.cuda(), n, H, dk, dk)
+    want = R.memory_prepare(U, i_off, i_off + H, bias[0], bias[1], cap, m, cu, slot, n, H, dk, dk)
+    for a, b in zip(got[3:], want[3:]):      # weight, decay, exp(-m): exponentials of numbers up to 15, whose sums of up to 64 round
+        assert bool(((a.double().cpu() - b.double()).abs() <= 64 * 15 * 2.0 ** -24 * b.double().abs() + 1e-30).all())
+    torch.testing.assert_close(m_got.cpu(), m, atol=64 * 15 * 2.0 ** -24, rtol=0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H, dv, groups", [(2, 4, 1), (4, 12, 2), (3, 100, 1), (8, 128, 2), (64, 64, 8), (33, 124, 1), (5, 66, 1)])
+def test_state_space_finish_four_columns_a_load(H, dv, groups, dtype):
+    from inferllm_amd.kernels import ops
+    g = torch.Generator().manual_seed(H * dv)
+    T, inner = 5, H * dv
+    o, x, D = torch.randn(T, H, dv, generator=g), torch.randn(T, H, dv, generator=g), torch.randn(H, generator=g)
+    Z, w = torch.randn(T, inner + 8, generator=g).to(dtype), torch.randn(inner, generator=g).to(dtype)
+    got = ops.ssm_finish(o.cuda(), x.cuda(), D.cuda(), Z.cuda(), 4, w.cuda(), groups, 1e-5, torch.float32)
+    _near(got, R.ssm_finish(o, x, D, Z, 4, w, groups, 1e-5, torch.float32), torch.float32)
+
+
+@pytest.mark.parametrize("nb, cb", [(2, 64), (3, 128), (1, 192), (2, 256), (1, 320), (1, 4096)])
+def test_recurrent_gates_of_many_rows(nb, cb):
+    """16 rows and up to 256 outputs a block: slices, waves and whole blocks without outputs, a last tile of one row."""
+    from inferllm_amd.kernels import ops
+    g = torch.Generator().manual_seed(cb)
+    T, C = 145, nb * cb
+    u, wt = torch.randn(T, C, generator=g), torch.randn(2, nb, cb, cb, generator=g) * cb ** -0.5
+    rb, ib, lam = torch.randn(3, C, generator=g)
+    for got, want in zip(ops.lru_gates(*(t.cuda() for t in (u, wt, rb, ib, lam)), 8.0), R.lru_gates(u, wt, rb, ib, lam, 8.0)):
+        _near(got, want, torch.float32)
