@@ -1345,6 +1345,78 @@ def qkv_rope_store(x, w_qkv, cos_sin: torch.Tensor,
     return y
 
 
+# csrc/gemm_short.hip takes q|k|v of 17 to 256 rows with rotation and cache store, and gate|up of 129 to 192 (to 160 with more than
+# SHORT_OUTPUTS columns each) with the activation.  us, weights cold, the vendor GEMM and the elementwise kernel -> these:
+#   q|k|v    6144 x 4096   96 rows 33 -> 19 (of it host time), 144 43 -> 24, 192 38 -> 26, 256 45 -> 34
+#            12288 x 4096  17 rows 36 -> 23, 96 36 -> 29, 160 43 -> 36, 256 55 -> 51
+#            15360 x 5120  17 rows 38 -> 33, 160 54 -> 48, 256 71 -> 67;  10240 x 8192  40 rows 46 -> 37, 160 77 -> 48, 256 95 -> 67
+#   gate|up  2 x 11008 x 4096  144 rows 60 -> 49, 192 65 -> 55, 224 68 -> 62, 256 64 -> 87 (128, the fused kernel of few rows: 45 -> 44)
+#            2 x 14336 x 4096  144 rows 68 -> 62, 192 76 -> 69, 224 76 -> 91;  2 x 13824 x 5120  160 rows 79 -> 76, 192 85 -> 83
+#            2 x 28672 x 8192  144 rows 204 -> 193, 160 206 -> 198, 192 214 -> 227
+SHORT_QKV, SHORT_GATE_UP, SHORT_OUTPUTS = 256, 192, 1 << 14
+
+
+def _short_fits(x, w, mode: str) -> bool:
+    return (isinstance(x, torch.Tensor) and isinstance(w, Weight) and w.tiled is not None and w.mode == mode
+            and x.dim() == 2 and x.dtype == torch.bfloat16 and w.plain.dtype == torch.bfloat16 and x.is_cuda and w.tiled.is_cuda
+            and x.shape[1] == w.plain.shape[1] and x.shape[1] % 64 == 0 and x.shape[1] >= 512 and w.plain.numel() < 1 << 31
+            and x.is_contiguous() and _on16(x, w.tiled) and not _plan.keeps_short(x.shape[0], *w.plain.shape))
+
+
+def qkv_short_fits(x, w_qkv, hd: int) -> bool:
+    """Whether csrc/gemm_short.hip takes the q|k|v product of these rows (`NormedRows` too), rotation and store with it."""
+    xt = x.xb if isinstance(x, NormedRows) else x
+    return hd % 16 == 0 and _short_fits(xt, w_qkv, "qkv") and SKINNY_BEST_ROWS < xt.shape[0] <= SHORT_QKV
+
+
+# From so many rows of single tokens also where csrc/gemm_rows.hip takes them (it is the faster way with few: it writes no planes).
+# us, both in a graph, rows kernel -> this one:  6144 x 4096  64 rows 17.9 -> 18.1, 128 34 -> 23;  12288 x 4096  96 rows 30.1 ->
+# 30.7, 112 33.1 -> 34.2, 128 37.0 -> 36.1;  3072 x 2048  112 rows 15.9 -> 14.2, 128 19.9 -> 14.6;  3072 x 1024  112 rows 11.0
+# -> 11.5, 128 13.2 -> 11.8;  15360 x 5120  48 rows 34 -> 37, 80 43 -> 42, 128 60 -> 47;  10240 x 8192  40 rows 38 -> 40, 64 47
+# -> 41, 128 62 -> 47.
+SHORT_STEPS, SHORT_STEPS_K = 113, 65
+
+
+def qkv_short_pays(M: int, K: int) -> bool:
+    return M >= (SHORT_STEPS if K <= 4096 else SHORT_STEPS_K)
+
+
+def gate_up_short_fits(x, w_gate_up) -> bool:
+    """Whether csrc/gemm_short.hip takes the gate and up products of these rows and is the faster way."""
+    return (_short_fits(x, w_gate_up, "gate_up") and w_gate_up.plain.shape[0] % 16 == 0
+            and ROWS_MAX < x.shape[0] <= (SHORT_GATE_UP if w_gate_up.plain.shape[0] <= 2 * SHORT_OUTPUTS else 160))
+
+
+def _short_planes(x: torch.Tensor, rows: int) -> torch.Tensor:
+    M, K = x.shape
+    return torch.empty((_lib().illm_gemm_short_splits(M, rows, K), M, rows), dtype=torch.float32, device=x.device)
+
+
+def qkv_short(x, w_qkv: "Weight", cos_sin: torch.Tensor, row_pos: torch.Tensor, row_slot: torch.Tensor,
+              slot_len: Optional[torch.Tensor], kcache: torch.Tensor, vcache: torch.Tensor, page_table: torch.Tensor,
+              page_size: int, ring: int, nh: int, nkv: int, hd: int) -> torch.Tensor:
+    """`linear` and `rope_store` (pairs (i, i + hd/2), all dims) of up to 256 rows: rows [q | k | v], q and k rotated, k and v
+    stored in the cache.  The rotation acts on the float32 sums."""
+    _need(qkv_short_fits(x, w_qkv, hd), "qkv_short: operands not taken")
+    x = x.rows() if isinstance(x, NormedRows) else x
+    _gpu(x, w_qkv.tiled, cos_sin, row_pos, row_slot, slot_len, kcache, vcache, page_table)
+    M, K = x.shape
+    N = (nh + 2 * nkv) * hd
+    _i32(row_pos, M); _i32(row_slot, M); _i32(slot_len); _i32(page_table)
+    _need(w_qkv.shape == (N, K), f"qkv_short: weight {tuple(w_qkv.shape)} vs ({N}, {K})")
+    _need(cos_sin.dtype == torch.float32 and cos_sin.dim() == 3 and cos_sin.shape[1] * 2 == hd and cos_sin.shape[2] == 2,
+          "qkv_short: angle table must be float32 [max_pos, hd/2, 2]")
+    _need(kcache.dtype == torch.bfloat16 and kcache.shape[1:] == (nkv, page_size, hd) and vcache.shape == kcache.shape
+          and vcache.dtype == torch.bfloat16 and page_table.dim() == 2, "qkv_short: cache shape or dtype")
+    planes = _short_planes(x, N)
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    _check(_lib().illm_gemm_short_qkv(
+        _p(x), _p(w_qkv.tiled), _p(planes), planes.numel() * 4, _p(y), M, K, _p(cos_sin), cos_sin.shape[0], _p(row_pos),
+        _p(row_slot), _p(slot_len), _p(kcache), _p(vcache), _p(page_table), page_table.shape[1], page_size, ring, nh, nkv, hd,
+        0, 0, _stream()), "qkv_short")
+    return y
+
+
 def gate_up_silu(x, w_gate_up) -> torch.Tensor:
     """silu(x . Wg^T) * (x . Wu^T) for w_gate_up = [Wg | Wu] stacked as [2F, K].
 
@@ -1428,6 +1500,13 @@ def gate_up_act(x, w_gate_up, limit: float = 0.0) -> torch.Tensor:
         return y
     if isinstance(x, NormedRows):
         x = x.rows()
+    if gate_up_short_fits(x, w_gate_up):
+        planes = _short_planes(x, F2)
+        y = torch.empty((M, F2 // 2), dtype=x.dtype, device=x.device)
+        _check(_lib().illm_gemm_short_gate_up(_p(x), _p(w_gate_up.tiled), _p(planes), planes.numel() * 4, _p(y), M, F2 // 2, K,
+                                              ctypes.c_float(limit), ctypes.c_float(SWISH_ALPHA), 0, 0, _stream()),
+               "gate_up_act (a short prompt's rows)")
+        return y
     if gate_up_turns_fits(x, w_gate_up):
         wp = plain_weight(w_gate_up)
         _gpu(x, wp)

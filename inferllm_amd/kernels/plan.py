@@ -13,7 +13,7 @@ the choice is a table by shape:
   than the rule's must win by 7 %), and for every other shape one rule: planes from 17 rows on,
   products of many rows whole.  Nothing is ever timed.  Gate and up of many rows are a kernel of
   their own with the activation, which has no cuts, but for sizes that `ops.turns_pays` leaves to the
-  product and under a plan that was pinned before there was that kernel (`Plan.turns`): it keeps
+  product and under a plan that was pinned before there was that kernel (`Plan.turns`, `Plan.short`): it keeps
   the products and their bits.
   The third table says from how few rows (below 17) the q|k|v product goes to the kernel that
   shares X through LDS (csrc/gemm_rows.hip) rather than to the few-rows kernel; gate|up and the
@@ -138,25 +138,33 @@ class Plan:
     def __init__(self, planes_from: Optional[dict] = None, cuts: Optional[dict] = None,
                  measure: bool = False, rows_from: Optional[dict] = None,
                  rows_most: Optional[dict] = None, rules: Optional[Rules] = None,
-                 turns: Optional[bool] = None):
-        """`turns`: whether gate and up of many rows may go to the kernel that has no cuts.  None: but for those
-        whose matrix `cuts` names here and the fixed tables do not."""
+                 turns: Optional[bool] = None, short: Optional[bool] = None):
+        """`turns`: whether gate and up of many rows may go to the kernel that has no cuts, `short`: whether those and
+        q|k|v of a short prompt's rows may go to theirs.  None: but for those whose matrix `cuts` names here and the
+        fixed tables do not."""
         self.planes_from: Dict[Tuple[int, int], int] = dict(planes_from or {})
         self.cuts: Dict[tuple, tuple] = dict(cuts or {})
         self.rows_from: Dict[tuple, int] = dict(rows_from or {})
         self.rows_most: Dict[tuple, int] = dict(rows_most or {})
         self.rules = rules or Rules()
         self.measure = bool(measure)
-        self._kept = frozenset() if turns is not None else frozenset(self.cuts) - frozenset(FIXED_CUTS)
-        self.turns = bool(turns) if turns is not None else None if self._kept else True
+        own = frozenset(self.cuts) - frozenset(FIXED_CUTS)
+        self._kept = frozenset() if turns is not None else own
+        self._kept_short = frozenset() if short is not None else own
+        self.turns = bool(turns) if turns is not None else None if own else True
+        self.short = bool(short) if short is not None else None if own else True
 
     @classmethod
     def fixed(cls, measure: bool = False) -> "Plan":
-        return cls(FIXED_PLANES_FROM, FIXED_CUTS, measure, FIXED_ROWS_FROM, FIXED_ROWS_MOST, turns=True)
+        return cls(FIXED_PLANES_FROM, FIXED_CUTS, measure, FIXED_ROWS_FROM, FIXED_ROWS_MOST, turns=True, short=True)
 
     def keeps_products(self, M: int, N: int, K: int) -> bool:
         """Whether M rows of gate and up (w [N, K]) stay a product in this plan's cuts and its activation."""
         return self.turns is False or (-(-M // 256), N, K) in self._kept
+
+    def keeps_short(self, M: int, N: int, K: int) -> bool:
+        """The same for up to 256 rows of gate and up or of q|k|v."""
+        return self.short is False or bool(self._kept_short & {(-(-M // 256), N, K), ("pad", -(-M // 32), N, K)})
 
     # ------------------------------------------------------------ as plain data
     def to_dict(self) -> dict:
@@ -165,20 +173,22 @@ class Plan:
                 "cuts": [[list(k), list(p)] for k, p in sorted(self.cuts.items(), key=repr)],
                 "rows_from": [[m, n, k, r] for (m, n, k), r in sorted(self.rows_from.items())],
                 "rows_most": [[m, n, k, r] for (m, n, k), r in sorted(self.rows_most.items())],
-                "rules": asdict(self.rules), "turns": self.turns}
+                "rules": asdict(self.rules), "turns": self.turns, "short": self.short}
 
     @classmethod
     def from_dict(cls, d: dict) -> "Plan":
-        """A pinned plan: what `to_dict` gave, nothing measured.  Without a word on "turns" it was made before the
-        kernel of that name, and keeps the products that its process had."""
+        """A pinned plan: what `to_dict` gave, nothing measured.  Without a word on "turns" or "short" it was made
+        before the kernel of that name, and keeps the products that its process had."""
         return cls({(int(n), int(k)): int(r) for n, k, r in d.get("planes_from", [])},
                    {tuple(k): tuple(p) for k, p in d.get("cuts", [])}, measure=False,
                    rows_from={(str(m), int(n), int(k)): int(r) for m, n, k, r in d.get("rows_from", [])},
                    rows_most={(str(m), int(n), int(k)): int(r) for m, n, k, r in d.get("rows_most", [])},
-                   rules=Rules(**{k: int(v) for k, v in d.get("rules", {}).items()}), turns=d.get("turns", False))
+                   rules=Rules(**{k: int(v) for k, v in d.get("rules", {}).items()}), turns=d.get("turns", False),
+                   short=d.get("short", False))
 
     def __eq__(self, other) -> bool:
         return (isinstance(other, Plan) and self.planes_from == other.planes_from
                 and self.cuts == other.cuts and self.rows_from == other.rows_from
                 and self.rows_most == other.rows_most and self.rules == other.rules
-                and self.turns == other.turns and self._kept == other._kept)
+                and self.turns == other.turns and self._kept == other._kept
+                and self.short == other.short and self._kept_short == other._kept_short)

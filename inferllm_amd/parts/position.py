@@ -107,12 +107,15 @@ class Rotary(PositionEncoding):
         return "qkv" if fused else "plain"
 
     def project_qkv(self, h, w_qkv, ctx: StepContext, nh, nkv, hd, kcache, vcache, group):
-        if (not ctx.prefill and kcache is not None and self.pairing == "half"
-                and self.rotary_dim == hd and ops.qkv_rope_store_fits(h, w_qkv, hd)
-                and kcache.dtype == h.dtype):
-            return ops.qkv_rope_store(h, w_qkv, self.table(ctx.device), ctx.row_pos, ctx.row_slot,
-                                      kcache, vcache, group.table, group.page_size, group.ring,
-                                      nh, nkv, hd)
+        if kcache is not None and self.pairing == "half" and self.rotary_dim == hd and kcache.dtype == h.dtype:
+            short = ops.qkv_short_fits(h, w_qkv, hd)
+            if not ctx.prefill and ops.qkv_rope_store_fits(h, w_qkv, hd) and not (short and ops.qkv_short_pays(*h.shape)):
+                return ops.qkv_rope_store(h, w_qkv, self.table(ctx.device), ctx.row_pos, ctx.row_slot,
+                                          kcache, vcache, group.table, group.page_size, group.ring,
+                                          nh, nkv, hd)
+            if short:
+                return ops.qkv_short(h, w_qkv, self.table(ctx.device), ctx.row_pos, ctx.row_slot, ctx.overwritten_lengths,
+                                     kcache, vcache, group.table, group.page_size, group.ring, nh, nkv, hd)
         return super().project_qkv(h, w_qkv, ctx, nh, nkv, hd, kcache, vcache, group)
 
 
