@@ -3,10 +3,10 @@
 // `add_rmsnorm` adds in order (the o and down projections of 129 to 256 rows).
 //
 // The vendor GEMM finds too few tiles for these (192 rows of the 7B shape: o 32 us, down 49 with its rows
-// filled up to 256).  Here a block takes all rows, 64 columns and its part of K, about one block a compute
-// unit: a part of K is what keeps the chip busy and X small.  Both operands go straight from memory into
+// filled up to 256).  Here a block takes all rows, 64 or 128 columns (`tiles_columns`) and its part of K, about one
+// block a compute unit: a part of K is what keeps the chip busy and X small.  Both operands go straight from memory into
 // LDS, 64 k (a row's 128 bytes) a stage, two or three stages ahead, one barrier a stage.  Measured with
-// the norm behind it at 192 rows, matrices cold: o 39 -> 23 us, down 61 -> 42.  What is left: with W's
+// the norm behind it at 192 rows, matrices cold: o 39 -> 21 us, down 61 -> 37.  What is left: with W's
 // lines taken from L2 a stage takes 60 % of the time, so the blocks wait for memory (up to 96 KB a
 // compute unit are under way); an extra wave that asks for W's lines 8 or 16 stages ahead gained nothing.
 // The same loop with whole K (q|k|v with its rotation 47 -> 42 us, gate|up 61 -> 60, 73 -> 78 at the 8B
@@ -122,10 +122,20 @@ gemm_tiles_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, fl
     }
 }
 
+// Columns a block takes.  A compute unit brings in about 38 GB/s of X (from L2) and W together: of 128 columns X is read
+// half as often, for twice the planes, which pays where a part of K is then at least 16 stages long.  us with the norm that
+// adds the planes, matrices cold, 160 / 256 rows, 64 -> 128 columns: 4096 x 11008 37.5 / 46.2 -> 34.9 / 43.4, 4096 x 14336
+// 43.6 / 53.6 -> 39.4 / 48.6, 8192 x 28672 155 / 192 -> 124 / 146; with parts of 8 stages 4096 x 4096 19.4 / 25.3 -> 21.6 / 27.6,
+// 2048 x 8192 19.4 / 24.9 -> 22.0 / 27.5.  (Within the 4 GiB of a load's offset.)
+static int tiles_columns(int N, int K) {
+    const int blocks = (N + 127) / 128;
+    return K / GT_K >= 16 * max(1, 256 / blocks) && (N + 127LL) * K * 2 < 0xffffffffLL ? 128 : 64;
+}
+
 // Parts of K for about one block a compute unit, each at least 8 stages long and none empty.
 extern "C" int illm_gemm_tiles_splits(int N, int K) {
     if (N <= 0 || K < GT_K) return 1;
-    const int blocks = (N + 63) / 64, every = K / GT_K;
+    const int columns = tiles_columns(N, K), blocks = (N + columns - 1) / columns, every = K / GT_K;
     const int s = max(1, min(256 / blocks, every / 8)), per = (every + s - 1) / s;
     return (every + per - 1) / per;
 }
@@ -141,12 +151,18 @@ extern "C" int illm_gemm_tiles_planes(const void* X, const void* W, float* Y, in
         return ILLM_ERR_ARG;
     const int every = K / GT_K, per = (every + splits - 1) / splits;
     if ((long long)(splits - 1) * per >= every) return ILLM_ERR_ARG;
-    const dim3 grid((N + 63) / 64, splits), block(512);
-    if (M <= 192)
-        hipLaunchKernelGGL((gemm_tiles_kernel<192, 64, 4, 2, 4>), grid, block, 0, (hipStream_t)stream, (const bf16_t*)X,
-                           (const bf16_t*)W, Y, M, N, K, splits);
-    else
-        hipLaunchKernelGGL((gemm_tiles_kernel<256, 64, 4, 2, 3>), grid, block, 0, (hipStream_t)stream, (const bf16_t*)X,
-                           (const bf16_t*)W, Y, M, N, K, splits);
+    const int columns = tiles_columns(N, K);
+    const dim3 grid((N + columns - 1) / columns, splits);
+#define ILLM_TILES(TM, TN, NS)                                                                                        \
+    hipLaunchKernelGGL((gemm_tiles_kernel<TM, TN, 4, 2, NS>), grid, dim3(512), 0, (hipStream_t)stream, (const bf16_t*)X, \
+                       (const bf16_t*)W, Y, M, N, K, splits)
+    if (columns == 64) {
+        if (M <= 192) ILLM_TILES(192, 64, 4);
+        else ILLM_TILES(256, 64, 3);
+    } else {
+        if (M <= 192) ILLM_TILES(192, 128, 3);
+        else ILLM_TILES(256, 128, 3);
+    }
+#undef ILLM_TILES
     return illm_launch_status();
 }

@@ -929,8 +929,8 @@ def linear_planes(x: torch.Tensor, w: "Weight", splits: int = 0) -> torch.Tensor
 CUT_ROWS = (129, 256)     # rows `linear_cut` takes: below, `linear_planes` reads the decode copy; above, the
                           # vendor GEMM has tiles enough
 CUT_MIN_K = 4096          # product and the norm that adds the planes against the vendor GEMM and its norm, us
-                          # at 129 / 192 / 256 rows: 4096 x 4096 28 / 39 / 29 -> 20 / 23 / 26, 4096 x 11008
-                          # 60 / 61 / 58 -> 37 / 42 / 48, 8192 x 28672 315 / 242 / 328 -> 157 / 181 / 204,
+                          # at 129 / 192 / 256 rows: 4096 x 4096 28 / 39 / 29 -> 18 / 21 / 25, 4096 x 11008
+                          # 60 / 61 / 58 -> 34 / 37 / 43, 8192 x 28672 315 / 242 / 328 -> 121 / 130 / 146,
                           # 2048 x 5376 21 / 22 / 24 -> 16 / 18 / 20; 2048 x 2048 13 / 14 / 15 -> 13 / 14 / 17
 
 

@@ -90,3 +90,17 @@ def test_a_pinned_plan_keeps_the_products_of_short_prompts_that_it_was_made_with
         again = Plan.from_dict(json.loads(json.dumps(plan.to_dict())))
         assert again == plan and again.short is plan.short
     assert not Plan.fixed().keeps_short(160, *shape) and not Plan().keeps_short(160, *shape)
+
+
+# csrc/gemm_tiles.hip with blocks of 128 columns: parts of K of 16 stages and more, of unequal length, a ragged last block, and the
+# rows at the edges of both variants
+@pytest.mark.gpu
+@pytest.mark.parametrize("M, N, K, splits", [(129, 4096, 8192, 8), (192, 8196, 3136, 3), (193, 4132, 7232, 7), (256, 16384, 2048, 2), (1, 8320, 4096, 3)])
+def test_cut_products_of_wide_blocks(M, N, K, splits):
+    """Any order of K float32 sums: K 2^-24 of the sum of magnitudes."""
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x, w = (torch.randn(n, K, device=DEV, generator=g).to(torch.bfloat16) for n in (M, N))
+    planes = ops.linear_cut(x, w)
+    assert planes.shape == (splits, M, N)
+    want, room = (x.double() @ w.double().t(), K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()))
+    assert bool(((planes.double().sum(0) - want).abs() <= room).all())
