@@ -256,8 +256,14 @@ int illm_gemm_short_qkv(const void* X, const void* Wt, void* P, size_t p_bytes, 
                         void* vcache, const int32_t* page_table, int table_stride, int page_size, int ring, int nh, int nkv,
                         int hd, int tb, int splits, void* stream);
 // The sum of two products of at most 16 rows, float32 Y = X . W^T + X2 . W2^T, from the tiled copies (K, K2 % 128 == 0).
+int illm_gemm_skinny_sum_parts(int M, int N, int K, int K2);
 int illm_gemm_skinny_sum(const void* X, const void* Wt, int K, const void* X2, const void* W2t, int K2, float* Y, int M,
-                         int N, void* stream);
+                         int N, int add, const void* nw, const void* nw2, int nw_dt, void* xb, void* xb2, float* ssq_out,
+                         void* stream);
+// Two products side by side: Y = X . W^T, Y2 = act(X2 . W2^T) (act 0 none, 1 relu(y)^2, 2 gelu(y) by tanh), bfloat16, from tiled
+// copies; M <= 16, K a multiple of 128; ssq as for illm_gemm_skinny_bf16.
+int illm_gemm_skinny_pair(const void* X, const void* Wt, void* Y, int N, const void* X2, const void* W2t, void* Y2, int N2, int act,
+                          int M, int K, const float* ssq, int parts, float eps, void* stream);
 
 
 // Y[M, N] (float32 residual rows) += X . W^T for M <= 16 bfloat16 rows.  nw != null (the weight of

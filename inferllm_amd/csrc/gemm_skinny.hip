@@ -72,6 +72,14 @@ struct SkSecond {                // the second product of a sum: X [M, K], the t
     const bf16_t* X;
     const bf16_t* W;
     int K;
+    const void* nw;              // the weight, like the residual's, of another norm of the same rows, or null, and its operand
+    bf16_t* xb;
+};
+struct SkPair {                  // the second of two products: X [M, K], the tiled copy of W [N, K], whose blocks begin at `from`
+    const bf16_t* X;
+    const bf16_t* W;
+    void* Y;
+    int N, from;
 };
 struct SkNone {};
 
@@ -96,18 +104,32 @@ __device__ __forceinline__ uint4 turn8(uint4 v) {
 // ACT: the results go through res.act.  (A variant of its own: the test alone cost every product 0.15 us.)
 // TWO (TILED, MT == NTB == 1): the sum of two products with the same rows of results, the second one's pieces of K
 // after the first one's.  (SkSecond is read nowhere else.)
+// PAIR (EVEN, ACT): two products of rows with the same scales, side by side; res.act is the second one's.
 // EVEN (TILED, MT == 1): K is whole pieces (a multiple of 32 SK_U), so that every load is unconditional and its base the same
 // in all lanes.  Behind a test of its own each load had a branch and a 64-bit address a lane to be made, and the compiler
 // waited where it could not count.  us, 8 / 16 rows, matrices cold: 4096 x 11008 19.2 / 23.3 -> 18.6 / 22.3, 8192 x 2048
 // 8.9 / 10.7 -> 8.4 / 10.0, 6144 x 2048 8.2 / 10.4 -> 7.9 / 9.6, 32000 x 4096 43.8 / 46.9 -> 42.3 / 45.5; gate|up 2 x 5376 x
 // 2048 11.2 / 13.5 -> 10.8 / 13.0; the sum of two products (TWO), which had no other way, 15.9 / 26.0 -> 12.0 / 18.6.
 template <int MT, int NTB, int SK_U, int MAXW, int MODE, bool TILED, bool ONE_SHOT = false, bool HALF = false, bool ACT = false,
-          bool EVEN = false, bool TWO = false>
+          bool EVEN = false, bool TWO = false, bool PAIR = false>
 __global__ void __launch_bounds__(64 * MAXW)
 gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                    void* __restrict__ Y, int y_dt, int M, int N, int K, SkRope rope,
-                   SkResidual res, std::conditional_t<TWO, SkSecond, SkNone> two) {
+                   SkResidual res, std::conditional_t<TWO, SkSecond, std::conditional_t<PAIR, SkPair, SkNone>> two) {
     constexpr bool DUAL = MODE == SK_GATE_UP;
+    unsigned block = blockIdx.x;
+    int act = res.act;                     // (changed in `res` the struct would go through scratch memory)
+    if constexpr (PAIR) {
+        if ((int)block >= two.from) {
+            block -= two.from;
+            X = two.X;
+            W = two.W;
+            Y = two.Y;
+            N = two.N;
+        } else {
+            act = 0;
+        }
+    }
     // a wave's piece of LDS: first the staging of its W lines (NTB * SK_U KB, not TILED), then
     // its sums
     constexpr int SK_REGION_FLOATS = NTB * ((!TILED && SK_U > MT) ? SK_U : MT) * 256;
@@ -161,8 +183,8 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
         tot += __shfl_xor(tot, 32, ILLM_WAVE);
         if (lane < 16) row_rs[lane] = 1.0f / sqrtf(tot / (float)K + res.eps);
     }
-    const int n_base = blockIdx.x * (DUAL ? 8 * NTB : HALF ? 8 : 16 * NTB);
-    if (MODE == SK_PLAIN && res.planes > 1) {
+    const int n_base = block * (DUAL ? 8 * NTB : HALF ? 8 : 16 * NTB);
+    if (MODE == SK_PLAIN && !PAIR && !TWO && res.planes > 1) {
         int plane = 0;
         for (int p = 0; p + 1 < res.planes; ++p) plane += n_base >= res.ends[p] ? 1 : 0;
         X += (size_t)plane * M * K;
@@ -192,14 +214,17 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
 
     // producer: the threads that will add to the residual rows fetch their 4 values and the norm
     // weights now, so that they arrive while W is streamed
-    float pre_y[4] = {0.f, 0.f, 0.f, 0.f}, pre_nw[4] = {0.f, 0.f, 0.f, 0.f};
-    if (MODE == SK_PLAIN && res.accumulate && threadIdx.x < 64 && (int)(threadIdx.x & 15) < M) {
+    float pre_y[4] = {0.f, 0.f, 0.f, 0.f}, pre_nw[4] = {0.f, 0.f, 0.f, 0.f}, pre_nw2[TWO ? 4 : 1] = {0.f};
+    if (MODE == SK_PLAIN && res.accumulate && threadIdx.x < (HALF ? 32 : 64) && (int)(threadIdx.x & 15) < M) {
         const int n0 = tile_row[0] + (threadIdx.x >> 4) * 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             if (n0 + i < N) {
                 pre_y[i] = ((const float*)Y)[(size_t)(threadIdx.x & 15) * N + n0 + i];
                 if (res.nw) pre_nw[i] = ld_f(res.nw, res.nw_dt, n0 + i);
+                if constexpr (TWO) {
+                    if (two.nw) pre_nw2[i] = ld_f(two.nw, res.nw_dt, n0 + i);
+                }
             }
     }
 
@@ -264,8 +289,8 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
     const int w_row = lane >> 3, w_chunk = lane & 7;
     // TILED: this lane's 8 values of k-step 0 of the block's first tile; a last block may have
     // fewer than NTB tiles (SK_GATE_UP with NTB > 1)
-    const int tile_at = ((HALF ? (blockIdx.x & 1) * 8 + (r & 7) : r) * 4 + q) * 8;
-    const bf16_t* wtile = W + (size_t)(HALF ? blockIdx.x / 2 : blockIdx.x * NTB) * ((K + 31) / 32) * 512 + tile_at;
+    const int tile_at = ((HALF ? (block & 1) * 8 + (r & 7) : r) * 4 + q) * 8;
+    const bf16_t* wtile = W + (size_t)(HALF ? block / 2 : block * NTB) * ((K + 31) / 32) * 512 + tile_at;
     bool tile_ok[NTB];
 #pragma unroll
     for (int nt = 0; nt < NTB; ++nt) tile_ok[nt] = DUAL ? n_base + 8 * nt < N : tile_row[nt] < N || MODE != SK_PLAIN;
@@ -274,7 +299,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
     int ksteps = ksteps1, lane_w = 0, lane_x1 = 0, lane_x2 = 0;
     const bf16_t *tile1 = W, *tile2 = nullptr, *second_x = nullptr;
     if constexpr (EVEN) {
-        const int tile = HALF ? blockIdx.x / 2 : blockIdx.x * NTB, odd = HALF ? r >> 3 : 0, row = min(HALF ? r & 7 : r, M - 1);
+        const int tile = HALF ? block / 2 : block * NTB, odd = HALF ? r >> 3 : 0, row = min(HALF ? r & 7 : r, M - 1);
         tile1 = W + (size_t)tile * ksteps1 * 512;
         lane_w = tile_at + odd * 512;
         lane_x1 = row * K + odd * 32 + q * 8;
@@ -503,6 +528,11 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                     if (res.nw)
                         *(uint2*)(res.xb + at) = make_uint2(pack_bf16x2(y[0] * pre_nw[0], y[1] * pre_nw[1]),
                                                             pack_bf16x2(y[2] * pre_nw[2], y[3] * pre_nw[3]));
+                    if constexpr (TWO) {            // (N % 8 == 0 where there are operands)
+                        if (two.nw)
+                            *(uint2*)(two.xb + at) = make_uint2(pack_bf16x2(y[0] * pre_nw2[0], y[1] * pre_nw2[1]),
+                                                                pack_bf16x2(y[2] * pre_nw2[2], y[3] * pre_nw2[3]));
+                    }
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
@@ -514,7 +544,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
             }
             if (res.nw) {
                 sq += __shfl_xor(sq, 16, ILLM_WAVE);
-                sq += __shfl_xor(sq, 32, ILLM_WAVE);
+                if constexpr (!HALF) sq += __shfl_xor(sq, 32, ILLM_WAVE);
                 if (l2 < 16 && mrow < M) res.ssq_out[(size_t)mrow * gridDim.x + blockIdx.x] = sq;
             }
             continue;
@@ -529,10 +559,10 @@ gemm_skinny_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                 if (n0 + i < N) {
                     float y = v[nt][i] * rs;
                     if constexpr (ACT) {
-                        if (res.act == 1) {
+                        if (act == 1) {
                             y = fmaxf(y, 0.f);
                             y *= y;
-                        } else {
+                        } else if (!PAIR || act) {
                             y = gelu_tanh_f(y);
                         }
                     }
@@ -683,20 +713,56 @@ extern "C" int illm_gemm_skinny_act(const void* X, const void* W, const void* Wt
 // rows leave for the residual stream, in one kernel with one sum and no rounding between.  M <= 16, K and K2 multiples of 128.
 // Half a tile a block by the rule above.  Matrices cold, us, both products / this at 1, 8 and 16 rows: 2048 x 2048 and x 8192
 // 12.1 / 10.0, 14.2 / 12.0, 22.4 / 18.6, 4096 x 4096 and x 16384 29.2 / 26.4, 32.5 / 29.6, 40.9 / 36.8.
+// add: Y += that, and with nw != null xb and ssq_out as illm_gemm_skinny_add leaves them, ssq_out [M][illm_gemm_skinny_sum_parts],
+// and with nw2 (of nw's type) xb2 = bfloat16(Y nw2).
+static bool sum_by_halves(int M, int N, long long K) {
+    return M <= 8 && (SK_HALF >= 0 ? SK_HALF == 1 : (N + 15) / 16 <= 128 && K >= 1024);
+}
+
+extern "C" int illm_gemm_skinny_sum_parts(int M, int N, int K, int K2) {
+    return M <= 0 || N <= 0 || K <= 0 || K2 <= 0 ? 0 : sum_by_halves(M, N, (long long)K + K2) ? (N + 7) / 8 : (N + 15) / 16;
+}
+
 extern "C" int illm_gemm_skinny_sum(const void* X, const void* Wt, int K, const void* X2, const void* W2t, int K2, float* Y,
-                                    int M, int N, void* stream) {
+                                    int M, int N, int add, const void* nw, const void* nw2, int nw_dt, void* xb, void* xb2,
+                                    float* ssq_out, void* stream) {
     if (M <= 0 || M > 16 || N <= 0 || K <= 0 || K % 128 || K2 <= 0 || K2 % 128 || K > 1 << 24 || K2 > 1 << 24 || !X || !Wt || !X2 ||
-        !W2t || !Y)
+        !W2t || !Y || (nw && (!add || !illm_dtype_ok(nw_dt) || !xb || !ssq_out || N % 8)) || (nw2 && (!nw || !xb2)))
         return ILLM_ERR_ARG;
     const int blocks = (N + 15) / 16;
     int waves = (SK_WAVES_ON_CHIP_TILED + blocks / 2) / blocks;
     waves = clamp_waves(waves < 1 ? 1 : waves, 1, 1, 4, K + K2);
-    const SkSecond two = {(const bf16_t*)X2, (const bf16_t*)W2t, K2};
-    if (M <= 8 && (SK_HALF >= 0 ? SK_HALF == 1 : blocks <= 128 && K + K2 >= 1024))
+    const SkSecond two = {(const bf16_t*)X2, (const bf16_t*)W2t, K2, nw2, (bf16_t*)xb2};
+    SkResidual res = SK_NO_RESIDUAL;
+    res.accumulate = add != 0; res.nw = nw; res.nw_dt = nw_dt; res.xb = (bf16_t*)xb; res.ssq_out = ssq_out;
+    if (sum_by_halves(M, N, (long long)K + K2))
         return launch_skinny<1, 1, 4, SK_PLAIN, true, false, true, false, true>(X, Wt, Y, ILLM_F32, M, N, K, waves, (hipStream_t)stream,
-                                                                                SkRope(), SK_NO_RESIDUAL, two);
+                                                                                SkRope(), res, two);
     return launch_skinny<1, 1, 4, SK_PLAIN, true, false, false, false, true>(X, Wt, Y, ILLM_F32, M, N, K, waves, (hipStream_t)stream,
-                                                                             SkRope(), SK_NO_RESIDUAL, two);
+                                                                             SkRope(), res, two);
+}
+
+// Two products, Y[M, N] = X . W^T and Y2[M, N2] = act(X2 . W2^T) (act as above, 0 none), bfloat16, from the tiled copies: what a
+// mixer and a feed-forward that read norms of the same rows begin with.  M <= 16, K a multiple of 128; ssq, of both, as for
+// illm_gemm_skinny_bf16.
+extern "C" int illm_gemm_skinny_pair(const void* X, const void* Wt, void* Y, int N, const void* X2, const void* W2t, void* Y2, int N2, int act,
+                                     int M, int K, const float* ssq, int parts, float eps, void* stream) {
+    if (M <= 0 || M > 16 || N <= 0 || N2 <= 0 || K <= 0 || K % 128 || !X || !Wt || !Y || !X2 || !W2t || !Y2 || act < 0 || act > 2 ||
+        !scale_args_ok(ssq, parts, M))
+        return ILLM_ERR_ARG;
+    SkResidual res = SK_NO_RESIDUAL;
+    res.ssq = ssq; res.parts = parts; res.eps = eps; res.act = act;
+    // One tile a block: with two, X is read half as often, but fewer waves have loads under way (us at 8 rows, cold, the two products
+    // apart / one tile / two: 10304 and 8192 x 2048 19.6 / 17.1 / 21.4, 5120 and 8192 x 2048 17.9 / 14.7 / 14.5, 3648 and 2304 x 2048
+    // 11.9 / 8.9 / 9.4, 2560 and 2176 x 512 7.0 / 4.4 / 5.4, 12288 and 16384 x 4096 47.2 / 43.6 / 44.9; at 16 rows the first 23.7 / 20.2 /
+    // 24.0, the second 21.8 / 17.0 / 15.0, the last 54.5 / 53.3 / 49.0).
+    const int from = (N + 15) / 16, blocks = from + (N2 + 15) / 16;
+    const int waves = clamp_waves((SK_WAVES_ON_CHIP_TILED + blocks / 2) / blocks, 1, 1, 4, K);
+    const SkPair two = {(const bf16_t*)X2, (const bf16_t*)W2t, Y2, N2, from};
+    hipLaunchKernelGGL((gemm_skinny_kernel<1, 1, 4, 16, SK_PLAIN, true, false, false, true, true, false, true>), dim3(blocks),
+                       dim3(64 * waves), (size_t)waves * 1024 + 64, (hipStream_t)stream, (const bf16_t*)X, (const bf16_t*)Wt, Y,
+                       ILLM_BF16, M, N, K, SkRope(), res, two);
+    return illm_launch_status();
 }
 
 // The product whose parts of W read rows of X of their own: X [planes][M][K], W's rows ends[p - 1] .. ends[p] - 1

@@ -552,6 +552,7 @@ class NormedRows:
         self.xb, self.ssq = xb, ssq
         self.shape = x.shape
         self._rows: Optional[torch.Tensor] = None
+        self.second: Optional["NormedRows"] = None      # the same rows for a second norm (`linear_sum`)
 
     def rows(self) -> torch.Tensor:
         if self._rows is None:
@@ -1220,15 +1221,60 @@ def linear_sum_fits(a: Product, b: Product) -> bool:
             and a.x.shape[0] == b.x.shape[0] and a.w.shape[0] == b.w.shape[0])
 
 
-def linear_sum(a: Product, b: Product) -> torch.Tensor:
-    """float32 [M, N]: the sum of the two products."""
+def linear_sum(a: Product, b: Product, into: Optional[torch.Tensor] = None, norm=None, norm2=None):
+    """float32 [M, N]: the sum of the two products.  `into` (float32 residual rows): added to these instead; norm = (weight,
+    eps) of the RMS norm that follows: as `linear_add`, what a few-rows product takes that norm with comes back, else None;
+    norm2: likewise of another norm of the same rows (same eps and type), as `second` of the first one's."""
     _need(linear_sum_fits(a, b), "linear_sum: operands not taken")
-    _gpu(a.x, b.x, a.w.tiled, b.w.tiled)
-    M, N = a.x.shape[0], a.w.shape[0]
-    y = torch.empty((M, N), dtype=torch.float32, device=a.x.device)
-    _check(_lib().illm_gemm_skinny_sum(_p(a.x), _p(a.w.tiled), a.x.shape[1], _p(b.x), _p(b.w.tiled), b.x.shape[1], _p(y), M, N,
-                                       _stream()), "linear_sum")
-    return y
+    _gpu(a.x, b.x, a.w.tiled, b.w.tiled, into)
+    M, N, K, K2 = a.x.shape[0], a.w.shape[0], a.x.shape[1], b.x.shape[1]
+    _need(into is None or (into.dtype == torch.float32 and into.shape == (M, N) and into.is_contiguous()),
+          "linear_sum: float32 rows of the sum's shape")
+    y = into if into is not None else torch.empty((M, N), dtype=torch.float32, device=a.x.device)
+    fits = lambda n: n is not None and n[0].dtype in _CODES and n[0].shape == (N,) and n[0].is_contiguous()  # noqa: E731
+    ws, xbs, ssq = [None, None], [None, None], None
+    if into is not None and N % 8 == 0 and fits(norm):
+        ws[0] = norm[0]
+        if fits(norm2) and norm2[0].dtype == norm[0].dtype and float(norm2[1]) == float(norm[1]):
+            ws[1] = norm2[0]
+        xbs = [torch.empty((M, N), dtype=torch.bfloat16, device=y.device) if w is not None else None for w in ws]
+        ssq = torch.empty((M, _lib().illm_gemm_skinny_sum_parts(M, N, K, K2)), dtype=torch.float32, device=y.device)
+        _gpu(*ws)
+    _check(_lib().illm_gemm_skinny_sum(_p(a.x), _p(a.w.tiled), K, _p(b.x), _p(b.w.tiled), K2, _p(y), M, N, int(into is not None),
+                                       _p(ws[0]), _p(ws[1]), _code(ws[0]) if ws[0] is not None else BF16, _p(xbs[0]), _p(xbs[1]),
+                                       _p(ssq), _stream()), "linear_sum")
+    if into is None:
+        return y
+    left = [NormedRows(into, w, norm[1], torch.bfloat16, xb, ssq) if w is not None else None for w, xb in zip(ws, xbs)]
+    if left[0] is not None:
+        left[0].second = left[1]
+    return left[0]
+
+
+def linear_pair_fits(x, a, x2, b, act: str) -> bool:
+    """Whether `linear_pair` takes these: up to 16 bfloat16 rows (or `NormedRows` of the same rows) and matrices with plain
+    decode copies."""
+    normed = isinstance(x, NormedRows)
+    if normed != isinstance(x2, NormedRows) or (normed and (x.ssq is not x2.ssq or x.eps != x2.eps)):
+        return False
+    return (act in ("", *_LINEAR_ACTS)
+            and all(isinstance(t, torch.Tensor) and t.dtype == torch.bfloat16 and t.dim() == 2 and 1 <= t.shape[0] <= SKINNY_BEST_ROWS
+                    and t.shape[1] % 128 == 0 and t.is_contiguous() and isinstance(w, Weight) and w.tiled is not None
+                    and w.mode == "plain" and w.shape[1] == t.shape[1]
+                    for t, w in ((x.xb if normed else x, a), (x2.xb if normed else x2, b)))
+            and x.shape == x2.shape)
+
+
+def linear_pair(x, a: "Weight", x2, b: "Weight", act: str):
+    """(x . a^T, act(x2 . b^T)) in one kernel, `act` "" (none) or one of `linear_act`'s, on the float32 sums."""
+    _need(linear_pair_fits(x, a, x2, b, act), "linear_pair: operands not taken")
+    (xt, ssq, parts, eps), (xt2, _, _, _) = _operand(x), _operand(x2)
+    _gpu(xt, xt2, a.tiled, b.tiled)
+    M, K = xt.shape
+    y, z = (torch.empty((M, w.shape[0]), dtype=torch.bfloat16, device=xt.device) for w in (a, b))
+    _check(_lib().illm_gemm_skinny_pair(_p(xt), _p(a.tiled), _p(y), a.shape[0], _p(xt2), _p(b.tiled), _p(z), b.shape[0],
+                                        _LINEAR_ACTS.get(act, 0), M, K, ssq, parts, eps, _stream()), "linear_pair")
+    return y, z
 
 
 QKV_ROPE_WAVES = 0       # waves per block of the fused kernel; 0: the kernel's own choice

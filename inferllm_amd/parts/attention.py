@@ -278,6 +278,7 @@ class GatedAttention(Mixer):
 
     graph_safe_prompts = True
     may_leave_product = True
+    reads_by_product = True
     takes_continuations = True
     takes_projected = True            # (its own products at column 0)
 

@@ -93,6 +93,10 @@ class Part:
     # `self.leave(x, w)`: the product, or `ops.Product` where its block has set `leaves_product`.
     may_leave_product = False
     leaves_product = False
+    # A mixer or feed-forward that reads its input through one plain product alone says so with `reads_by_product`: its
+    # `h` may be `ops.NormedRows`, `first_product` names the matrix and the activation behind it ("": none), and `forward`
+    # also takes that product's result as `projected` (a mixer as (result, 0)).
+    reads_by_product = False
     # Set by the model before `load`: whether the engine wants second copies of the matrices in
     # the few-rows kernels' tile order (False, True or "thin"; see `ops.decode_weight`).
     decode_copies = False
@@ -116,6 +120,9 @@ class Part:
 
     def leave(self, x: torch.Tensor, w):
         return ops.Product(x, w) if self.leaves_product else ops.linear(x, w)
+
+    def first_product(self):
+        return self.w_in, ""
 
     def tunables(self):
         """The part's products that have several equivalent ways, for whoever times them (an
@@ -165,6 +172,8 @@ class Norm(Part):
     # (a product whose K was split, `ops.linear_planes`).  Parts hand planes only to a norm that
     # says so.
     adds_planes = False
+    # the norm that a block takes of the same rows beside this one, set by the block (None: no other)
+    beside = None
 
     def rms_params(self):
         """(weight, eps) if the norm is a plain RMS norm that a product's kernel may take over

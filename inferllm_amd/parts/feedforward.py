@@ -84,6 +84,7 @@ class DenseActivation(FeedForward):
 
     graph_safe_prompts = True
     may_leave_product = True
+    reads_by_product = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, activation: str = "relu_squared",
                  tensors=None):
@@ -109,10 +110,15 @@ class DenseActivation(FeedForward):
     def tunables(self):
         return (("plain", self.w_down, {}),)
 
-    def forward(self, h, ctx: StepContext):
+    def first_product(self):
+        return self.w_up, _ACTIVATIONS[self.activation] if self.act is None else ""
+
+    def forward(self, h, ctx: StepContext, projected=None):
         act = _ACTIVATIONS[self.activation]
-        z = (ops.linear_act(h, self.w_up, act) if self.act is None
-             else getattr(ops, act)(ops.linear(h, self.w_up), self.act))
+        if self.act is None:
+            z = projected if projected is not None else ops.linear_act(h, self.w_up, act)
+        else:
+            z = getattr(ops, act)(projected if projected is not None else ops.linear(h, self.w_up), self.act)
         return self.leave(z, self.w_down)
 
 

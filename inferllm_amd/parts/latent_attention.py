@@ -34,6 +34,7 @@ class LatentAttention(Mixer):
 
     graph_safe_prompts = True
     may_leave_product = True
+    reads_by_product = True
     # rows that go on from earlier tokens are each treated as a single token over the cache, which
     # holds the step's own rows by then (a window's ring is kept from wrapping by the step function)
     takes_continuations = True
@@ -101,7 +102,7 @@ class LatentAttention(Mixer):
         self.transposed = (self.w_uk.dtype == torch.bfloat16 and self.R % 16 == 0 and self.R <= 512
                            and (self.R + self.dr) % 8 == 0)
 
-    def forward(self, h, ctx: StepContext, line, writes_cache, position):
+    def forward(self, h, ctx: StepContext, line, writes_cache, position, projected=None):
         H, dn, dr, dv, R = self.H, self.dn, self.dr, self.dv, self.R
         kept, group = ctx.cache.token_line(line)
         cache, cache_t = kept["latent"], kept.get("latent_t")
@@ -110,7 +111,7 @@ class LatentAttention(Mixer):
         window = self.window or 0
         table = position.table(ctx.device) if position is not None else None
         rot = position.rotary_dim if position is not None else 0
-        y = ops.linear(h, self.w_in)
+        y = projected[0] if projected is not None else ops.linear(h, self.w_in)
         if not self.gated:
             y = torch.cat([y, y.new_full((y.shape[0], H), 30.0)], dim=1)       # sigmoid(30) = 1
         whole = ctx.prefill and not ctx.continues

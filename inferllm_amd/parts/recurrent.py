@@ -39,6 +39,7 @@ class StateSpaceDuality(Mixer):
 
     graph_safe_prompts = True
     may_leave_product = True
+    reads_by_product = True
     takes_continuations = True
 
     def __init__(self, hidden_size: int, num_heads: int, groups: int, state_size: int, value_dim: int,
@@ -83,8 +84,8 @@ class StateSpaceDuality(Mixer):
     def tunables(self):
         return (("plain", self.w_o, {}),)
 
-    def forward(self, h, ctx: StepContext, line, writes_cache, position):
-        U = ops.linear(h, self.w_in)
+    def forward(self, h, ctx: StepContext, line, writes_cache, position, projected=None):
+        U = projected[0] if projected is not None else ops.linear(h, self.w_in)
         state = ctx.cache.state_line(line)
         S, tail = state["S"], state["tail"]
         if not ctx.prefill and ops.ssm_step_fits(U, self.N, self.dv, self.inner // self.norm_groups, ctx.act_dtype):
@@ -125,6 +126,7 @@ class MatrixMemory(Mixer):
 
     graph_safe_prompts = True
     may_leave_product = True
+    reads_by_product = True
     takes_continuations = True
 
     def __init__(self, hidden_size: int, num_heads: int, key_dim: int, value_dim: int, gate_cap: float,
@@ -165,8 +167,8 @@ class MatrixMemory(Mixer):
     def tunables(self):
         return (("plain", self.w_o, {}),)
 
-    def forward(self, h, ctx: StepContext, line, writes_cache, position):
-        U = ops.linear(h, self.w_in)
+    def forward(self, h, ctx: StepContext, line, writes_cache, position, projected=None):
+        U = projected[0] if projected is not None else ops.linear(h, self.w_in)
         state = ctx.cache.state_line(line)
         if not ctx.prefill and ops.mixer_step_fits(U, self.dk, self.dv, ctx.act_dtype):
             y = ops.memory_step(U, self.i_off, self.f_off, self.z_off, self.i_bias, self.f_bias, self.cap, state["m"], state["S"],
