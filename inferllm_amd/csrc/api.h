@@ -441,6 +441,10 @@ int illm_moe_route(const float* z, const void* corr, int corr_dt, int T, int NE,
 int illm_moe_tile_rows(void);
 int illm_moe_group(const int32_t* idx, int NP, int NEr, int32_t* order, int32_t* tiles,
                    int max_tiles, int tile_rows, void* stream);
+// illm_moe_route (no groups) and illm_moe_group of up to 16 tokens, 16 choices and 64 outputs in one launch.
+int illm_moe_route_group(const float* z, const void* corr, int corr_dt, int T, int NE, int top, int32_t* idx, float* wt,
+                         int score_kind, float scale, int NEr, int32_t* order, int32_t* tiles, int max_tiles, int tile_rows,
+                         void* stream);
 
 // Y[p] = X[p / x_div] . W[e_p]^T for every grouped pair p (W [experts][N][K]); gated: W
 // [experts][2 N][K] = [gate | up] rows and Y[p] = silu(X Wg^T) * (X Wu^T).  Y [NP, N] of dt.

@@ -227,17 +227,20 @@ __device__ __forceinline__ float moe_plain_act(float v, int act_kind, bool round
 // the `top` largest choice scores (lowest index on ties) in falling order; weights are scale * s.
 // `groups` > 0: the outputs are that many equal groups of neighbours, of which only the `keep` with the
 // largest sums of their two largest choice scores (lowest index on ties) can be chosen from.
-#define MOE_EPL 8                                   // outputs a lane holds: up to 512 experts
+// EPL: outputs a lane holds, 1 for up to 64 (the exponentials of seven that are not there: 64 outputs, 6 chosen, 8 tokens
+// 5.2 -> 4.6 us, 2,964 6.7 -> 5.5), else MOE_EPL.
+#define MOE_EPL 8                                   // up to 512 experts
+template <int EPL>
 __device__ __forceinline__ void
 moe_route_row(const float* zr, const void* __restrict__ corr, int corr_dt, int NE, int top,
               int32_t* __restrict__ idx_row, float* __restrict__ wt_row, int32_t* idx_copy,
               int score_kind, float scale, int groups, int keep) {
-    __shared__ float choice[64 * MOE_EPL], group_score[64 * MOE_EPL];
+    __shared__ float choice[64 * EPL], group_score[64 * EPL];
     const int lane = threadIdx.x & 63;
-    float s[MOE_EPL], c[MOE_EPL];
+    float s[EPL], c[EPL];
     float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < MOE_EPL; ++i) {
+    for (int i = 0; i < EPL; ++i) {
         const int e = lane + 64 * i;
         s[i] = e < NE ? zr[e] : -INFINITY;
         mx = fmaxf(mx, s[i]);
@@ -245,13 +248,13 @@ moe_route_row(const float* zr, const void* __restrict__ corr, int corr_dt, int N
     mx = wave_max(mx);
     float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < MOE_EPL; ++i) {
+    for (int i = 0; i < EPL; ++i) {
         s[i] = lane + 64 * i < NE ? expf(s[i] - mx) : 0.f;
         sum += s[i];
     }
     sum = wave_sum(sum);
 #pragma unroll
-    for (int i = 0; i < MOE_EPL; ++i) {
+    for (int i = 0; i < EPL; ++i) {
         const int e = lane + 64 * i;
         // softmax over all outputs, or every output's own sigmoid
         s[i] = score_kind == MOE_SCORE_SIGMOID ? (e < NE ? 1.0f / (1.0f + expf(-zr[e])) : 0.f) : s[i] / sum;
@@ -260,7 +263,7 @@ moe_route_row(const float* zr, const void* __restrict__ corr, int corr_dt, int N
     if (groups > 0) {                                  // (the block is this one wave)
         const int size = NE / groups;
 #pragma unroll
-        for (int i = 0; i < MOE_EPL; ++i)
+        for (int i = 0; i < EPL; ++i)
             if (lane + 64 * i < NE) choice[lane + 64 * i] = c[i];
         __syncthreads();
         for (int g = lane; g < groups; g += 64) {
@@ -282,7 +285,7 @@ moe_route_row(const float* zr, const void* __restrict__ corr, int corr_dt, int N
         }
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < MOE_EPL; ++i) {
+        for (int i = 0; i < EPL; ++i) {
             const int e = lane + 64 * i;
             if (e < NE && choice[e / size] == 0.f) c[i] = -INFINITY;
         }
@@ -308,7 +311,7 @@ moe_route_row(const float* zr, const void* __restrict__ corr, int corr_dt, int N
         float best = -INFINITY;
         int be = 0x7fffffff;
 #pragma unroll
-        for (int i = 0; i < MOE_EPL; ++i) {
+        for (int i = 0; i < EPL; ++i) {
             const int e = lane + 64 * i;
             if (e < NE && (c[i] > best || (c[i] == best && e < be))) { best = c[i]; be = e; }
         }
@@ -319,7 +322,7 @@ moe_route_row(const float* zr, const void* __restrict__ corr, int corr_dt, int N
         }
         float w = 0.f;
 #pragma unroll
-        for (int i = 0; i < MOE_EPL; ++i)
+        for (int i = 0; i < EPL; ++i)
             if (lane + 64 * i == be) { w = s[i]; c[i] = -INFINITY; }
         w = wave_sum(w);                               // only the owner's lane holds a value
         if (lane == 0) {
@@ -330,25 +333,33 @@ moe_route_row(const float* zr, const void* __restrict__ corr, int corr_dt, int N
     }
 }
 
+template <int EPL>
 __global__ void __launch_bounds__(64)
 moe_route_kernel(const float* __restrict__ z, const void* __restrict__ corr, int corr_dt, int NE,
                  int top, int32_t* __restrict__ idx, float* __restrict__ wt, int score_kind, float scale,
                  int groups, int keep) {
     const size_t t = blockIdx.x;
-    moe_route_row(z + t * NE, corr, corr_dt, NE, top, idx + t * top, wt + t * top, nullptr, score_kind, scale, groups,
-                  keep);
+    moe_route_row<EPL>(z + t * NE, corr, corr_dt, NE, top, idx + t * top, wt + t * top, nullptr, score_kind, scale, groups,
+                       keep);
+}
+
+static bool moe_route_args(const void* corr, int corr_dt, int T, int NE, int top, int score_kind, int groups, int keep) {
+    return !(groups < 0 || (groups > 0 && (NE % groups || keep <= 0 || keep > groups || top > keep * (NE / groups)))) &&
+           (score_kind == MOE_SCORE_SOFTMAX || score_kind == MOE_SCORE_SIGMOID) && T >= 0 && NE > 0 && NE <= 64 * MOE_EPL &&
+           top > 0 && top <= NE && (!corr || illm_dtype_ok(corr_dt));
 }
 
 extern "C" int illm_moe_route(const float* z, const void* corr, int corr_dt, int T, int NE, int top,
                               int32_t* idx, float* wt, int score_kind, float scale, int groups, int keep,
                               void* stream) {
-    if (groups < 0 || (groups > 0 && (NE % groups || keep <= 0 || keep > groups || top > keep * (NE / groups))))
-        return ILLM_ERR_ARG;
-    if ((score_kind != MOE_SCORE_SOFTMAX && score_kind != MOE_SCORE_SIGMOID) || T < 0 || NE <= 0 || NE > 64 * MOE_EPL || top <= 0 || top > NE || (corr && !illm_dtype_ok(corr_dt)))
-        return ILLM_ERR_ARG;
+    if (!moe_route_args(corr, corr_dt, T, NE, top, score_kind, groups, keep)) return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
-    hipLaunchKernelGGL(moe_route_kernel, dim3(T), dim3(64), 0, (hipStream_t)stream, z, corr, corr_dt,
-                       NE, top, idx, wt, score_kind, scale, groups, keep);
+    if (NE <= 64)
+        hipLaunchKernelGGL(moe_route_kernel<1>, dim3(T), dim3(64), 0, (hipStream_t)stream, z, corr, corr_dt, NE, top, idx, wt,
+                           score_kind, scale, groups, keep);
+    else
+        hipLaunchKernelGGL(moe_route_kernel<MOE_EPL>, dim3(T), dim3(64), 0, (hipStream_t)stream, z, corr, corr_dt, NE, top, idx,
+                           wt, score_kind, scale, groups, keep);
     return illm_launch_status();
 }
 
@@ -408,6 +419,35 @@ __global__ void __launch_bounds__(1024)
 moe_group_kernel(const int32_t* __restrict__ idx, int NP, int NEr, int32_t* __restrict__ order,
                  int32_t* __restrict__ tiles, int max_tiles, int tile_rows) {
     moe_group_pairs(idx, NP, NEr, order, tiles, max_tiles, tile_rows);
+}
+
+// The choice and the grouping of up to 16 tokens in one launch, a wave a token: the pairs go from one to the other through LDS.
+// us in a graph, 64 outputs, 6 chosen, two kernels / this: 1 token
+// 6.4 / 5.6, 8 tokens 6.9 / 5.8, 16 tokens 7.2 / 7.1.
+#define MOE_FEW_TOKENS 16
+#define MOE_FEW_TOP 16
+__global__ void __launch_bounds__(64 * MOE_FEW_TOKENS)
+moe_route_group_kernel(const float* __restrict__ z, const void* __restrict__ corr, int corr_dt, int NE, int top, int32_t* __restrict__ idx,
+                       float* __restrict__ wt, int score_kind, float scale, int T, int NEr, int32_t* __restrict__ order,
+                       int32_t* __restrict__ tiles, int max_tiles, int tile_rows) {
+    __shared__ int32_t chosen[MOE_FEW_TOKENS * MOE_FEW_TOP];
+    const int t = wave_index();
+    if (t < T)
+        moe_route_row<1>(z + (size_t)t * NE, corr, corr_dt, NE, top, idx + t * top, wt + t * top, chosen + t * top, score_kind,
+                         scale, 0, 0);
+    __syncthreads();
+    moe_group_pairs(chosen, T * top, NEr, order, tiles, max_tiles, tile_rows);
+}
+
+extern "C" int illm_moe_route_group(const float* z, const void* corr, int corr_dt, int T, int NE, int top, int32_t* idx, float* wt,
+                                    int score_kind, float scale, int NEr, int32_t* order, int32_t* tiles, int max_tiles,
+                                    int tile_rows, void* stream) {
+    if (!moe_route_args(corr, corr_dt, T, NE, top, score_kind, 0, 0) || T < 1 || T > MOE_FEW_TOKENS || NE > 64 || top > MOE_FEW_TOP ||
+        NEr < 0 || NEr > MOE_MAX_EXPERTS || max_tiles < 0 || tile_rows <= 0)
+        return ILLM_ERR_ARG;
+    hipLaunchKernelGGL(moe_route_group_kernel, dim3(1), dim3(64 * T), 0, (hipStream_t)stream, z, corr, corr_dt, NE, top, idx, wt,
+                       score_kind, scale, T, NEr, order, tiles, max_tiles, tile_rows);
+    return illm_launch_status();
 }
 
 extern "C" int illm_moe_tile_rows(void) { return MOE_TILE; }
@@ -1150,12 +1190,13 @@ moe_combine_kernel(const void* __restrict__ h, int dt, const int32_t* __restrict
 
 // The same with V neighbouring columns a thread (16-byte loads from 16-byte addresses; E % V == 0, top <= MOE_COMBINE_TOP) and a
 // block a token: the gate's dot product is formed once a token, and all of a thread's rows are asked for
-// together (2,964 tokens of 2,048, 6 chosen: 157 -> 25 us; 8 tokens 7.0 -> 5.0).  Up to MOE_COMBINE_FEW tokens a
+// together (2,964 tokens of 2,048, 6 chosen: 157 -> 25 us; 8 tokens 7.0 -> 5.0; in a graph, with the choice's test ahead of each
+// load 19.0 and 3.6, without 17.3 and 2.7).  Up to MOE_COMBINE_FEW tokens a
 // block 256 V columns of a token, each with the gate's product for itself: tokens of 7,168, 8 chosen, one block
 // against several, by column first: 8 tokens 12.7, 14.4, 7.9 us; 128 tokens 37, 14.7, 9.4; 256 tokens in float32
 // 49, 17.8, 22.4.
 #define MOE_COMBINE_FEW 128
-template <int DT, int V>
+template <int DT, int V, int TOP>
 __global__ void __launch_bounds__(256)
 moe_combine_vec_kernel(const void* __restrict__ h, const int32_t* __restrict__ idx, const float* __restrict__ wt,
                        const void* __restrict__ Y, const void* __restrict__ shared, const void* __restrict__ sg,
@@ -1175,27 +1216,28 @@ moe_combine_vec_kernel(const void* __restrict__ h, const int32_t* __restrict__ i
         gate = 1.0f / (1.0f + expf(-d));
     }
     for (int i = (blockIdx.y * 256 + threadIdx.x) * V; i < E; i += gridDim.y * 256 * V) {
-        float acc[V], hv[V], v[V];
-        ldv<DT, V>(h, t * E + i, hv);
+        float acc[V];
 #pragma unroll
         for (int j = 0; j < V; ++j) acc[j] = 0.f;
-#pragma unroll 8
-        for (int k = 0; k < top; ++k) {
-            const int e = idx[t * top + k];                    // the same in all lanes
-            const float w = wt ? wt[t * top + k] : 1.f;
-            if (e < NEr) {
-                ldv<DT, V>(Y, (t * top + k) * E + i, v);
+        // (no load behind a branch: every choice's row, or h's for one that is no expert, is on its way before the first is used)
+        float r[TOP][V], w[TOP];
 #pragma unroll
-                for (int j = 0; j < V; ++j) acc[j] += w * v[j];
-            } else {
-#pragma unroll
-                for (int j = 0; j < V; ++j) acc[j] += w * hv[j];
-            }
+        for (int k = 0; k < TOP; ++k) {
+            const size_t p = t * top + min(k, top - 1);
+            const bool real = idx[p] < NEr;                    // the same in all lanes
+            w[k] = wt ? wt[p] : 1.f;
+            ldv<DT, V>(real ? Y : h, (real ? p : t) * E + i, r[k]);
         }
-        if (shared) {
-            ldv<DT, V>(shared, t * E + i, v);
+        float sv[V];
+        if (shared) ldv<DT, V>(shared, t * E + i, sv);
 #pragma unroll
-            for (int j = 0; j < V; ++j) acc[j] += gate * v[j];
+        for (int k = 0; k < TOP; ++k)
+            if (k < top)
+#pragma unroll
+                for (int j = 0; j < V; ++j) acc[j] += w[k] * r[k][j];
+        if (shared) {
+#pragma unroll
+            for (int j = 0; j < V; ++j) acc[j] += gate * sv[j];
         }
 #pragma unroll
         for (int j = 0; j < V; j += 4)
@@ -1213,12 +1255,15 @@ extern "C" int illm_moe_combine(const void* h, int dt, const int32_t* idx, const
     const uintptr_t at = (uintptr_t)h | (uintptr_t)Y | (uintptr_t)shared | (uintptr_t)out;
     if (top <= MOE_COMBINE_TOP && E % (dt == ILLM_BF16 ? 8 : 4) == 0 && at % 16 == 0) {
         const int V = dt == ILLM_BF16 ? 8 : 4, parts = T <= MOE_COMBINE_FEW ? (E + 256 * V - 1) / (256 * V) : 1;
-        if (dt == ILLM_BF16)
-            hipLaunchKernelGGL((moe_combine_vec_kernel<ILLM_BF16, 8>), dim3(T, parts), dim3(256), 0, (hipStream_t)stream, h,
-                               idx, wt, Y, shared, sg, sg_dt, out, E, top, NEr);
-        else
-            hipLaunchKernelGGL((moe_combine_vec_kernel<ILLM_F32, 4>), dim3(T, parts), dim3(256), 0, (hipStream_t)stream, h,
-                               idx, wt, Y, shared, sg, sg_dt, out, E, top, NEr);
+#define ILLM_COMBINE(DT, V, TOP)                                                                                          \
+    hipLaunchKernelGGL((moe_combine_vec_kernel<DT, V, TOP>), dim3(T, parts), dim3(256), 0, (hipStream_t)stream, h, idx, wt, Y, \
+                       shared, sg, sg_dt, out, E, top, NEr)
+        if (dt == ILLM_BF16) {
+            if (top <= 8) ILLM_COMBINE(ILLM_BF16, 8, 8);
+            else ILLM_COMBINE(ILLM_BF16, 8, 16);
+        } else if (top <= 8) ILLM_COMBINE(ILLM_F32, 4, 8);
+        else ILLM_COMBINE(ILLM_F32, 4, 16);
+#undef ILLM_COMBINE
         return illm_launch_status();
     }
     hipLaunchKernelGGL(moe_combine_kernel, dim3(T, (E + 255) / 256), dim3(256), 0, (hipStream_t)stream,

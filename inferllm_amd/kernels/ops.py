@@ -1965,10 +1965,8 @@ def _moe_tiling(dtype: torch.dtype, E: int, F: int, NP: int, n_exp: int):
     return mfma, rows, max(1, min(NP, NP // rows + n_exp))
 
 
-def _moe_group(idx: torch.Tensor, n_exp: int, dtype: torch.dtype, E: int, F: int, on16: bool = True):
-    """The pairs grouped by expert.  `on16`: the rows and the experts' matrices lie on 16-byte addresses, as the
-    tiles of 128 pairs and more want them (straight into LDS, 16 bytes a lane)."""
-    NP = idx.numel()
+def _moe_group_space(NP: int, device, n_exp: int, dtype: torch.dtype, E: int, F: int, on16: bool = True):
+    """Where NP pairs are to be grouped by expert: (order, tiles, most tiles, a tile's pairs, on the matrix cores)."""
     mfma, rows, max_tiles = _moe_tiling(dtype, E, F, NP, n_exp)
     if rows >= 128:
         if not on16:
@@ -1976,11 +1974,40 @@ def _moe_group(idx: torch.Tensor, n_exp: int, dtype: torch.dtype, E: int, F: int
         elif _moe_wide(E, F, NP, n_exp):
             rows = 192
         max_tiles = max(1, min(NP, NP // rows + n_exp))
-    order = torch.empty((NP,), dtype=torch.int32, device=idx.device)
-    tiles = torch.empty((3 * max_tiles + 1,), dtype=torch.int32, device=idx.device)
+    order = torch.empty((NP,), dtype=torch.int32, device=device)
+    tiles = torch.empty((3 * max_tiles + 1,), dtype=torch.int32, device=device)
+    return order, tiles, max_tiles, rows, mfma
+
+
+def _moe_group(idx: torch.Tensor, n_exp: int, dtype: torch.dtype, E: int, F: int, on16: bool = True):
+    """The pairs grouped by expert.  `on16`: the rows and the experts' matrices lie on 16-byte addresses, as the
+    tiles of 128 pairs and more want them (straight into LDS, 16 bytes a lane)."""
+    NP = idx.numel()
+    grouped = _moe_group_space(NP, idx.device, n_exp, dtype, E, F, on16)
+    order, tiles, max_tiles, rows, _ = grouped
     _check(_lib().illm_moe_group(_p(idx), NP, n_exp, _p(order), _p(tiles), max_tiles, rows,
                                  _stream()), "moe_group")
-    return order, tiles, max_tiles, rows, mfma
+    return grouped
+
+
+MOE_FEW = (16, 64, 16)     # tokens, outputs and choices a token of the kernel that chooses and groups
+
+
+def _moe_route_group(z: torch.Tensor, correction: Optional[torch.Tensor], top: int, score: str, scale: float, n_exp: int,
+                     dtype: torch.dtype, E: int, F: int):
+    """`moe_route` and `_moe_group` of few tokens in one kernel."""
+    _need(score in MOE_SCORES, f"moe_route: score {score!r}; known: {sorted(MOE_SCORES)}")
+    _gpu(z, correction)
+    T, NE = z.shape
+    _need(correction is None or correction.shape == (NE,), "moe_route: correction [outputs]")
+    idx = torch.empty((T, top), dtype=torch.int32, device=z.device)
+    wt = torch.empty((T, top), dtype=torch.float32, device=z.device)
+    grouped = _moe_group_space(T * top, z.device, n_exp, dtype, E, F)
+    order, tiles, max_tiles, rows, _ = grouped
+    _check(_lib().illm_moe_route_group(_p(z), _p(correction), _code(correction) if correction is not None else 0, T, NE, top,
+                                       _p(idx), _p(wt), MOE_SCORES[score], ctypes.c_float(scale), n_exp, _p(order), _p(tiles),
+                                       max_tiles, rows, _stream()), "moe_route")
+    return idx, wt, grouped
 
 
 def moe_plan(h: torch.Tensor, w_router: torch.Tensor, correction: Optional[torch.Tensor], top: int,
@@ -1992,9 +2019,12 @@ def moe_plan(h: torch.Tensor, w_router: torch.Tensor, correction: Optional[torch
     experts have an up matrix [F, E] alone."""
     E = h.shape[1]
     n_exp = w_gate_up.shape[0] if w_gate_up is not None else 0
-    idx, wt = moe_route(few_outputs_f32(h, w_router), correction, top, score, scale, groups)
-    grouped = (_moe_group(idx, n_exp, h.dtype, E, w_gate_up.shape[1] // (2 if gated else 1))
-               if n_exp else None)
+    z = few_outputs_f32(h, w_router)
+    F = w_gate_up.shape[1] // (2 if gated else 1) if n_exp else 0
+    if n_exp and not groups and all(1 <= n <= m for n, m in zip((h.shape[0], z.shape[1], top), MOE_FEW)):
+        return _moe_route_group(z, correction, top, score, scale, n_exp, h.dtype, E, F)
+    idx, wt = moe_route(z, correction, top, score, scale, groups)
+    grouped = _moe_group(idx, n_exp, h.dtype, E, F) if n_exp else None
     return idx, wt, grouped
 
 
