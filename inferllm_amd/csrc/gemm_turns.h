@@ -92,41 +92,45 @@ struct Turns {
         }
     }
     // The turn's products, once every wave's loads for the other group's and this group's next reads have arrived (all but
-    // the newest VM of this wave's) and the other group's products are on their way.
+    // the newest VM of this wave's) and the other group's products are on their way.  on: a group whose rows of X are not there
+    // leaves the products out (the same in all lanes).
     template <int VM, int NTH, int NB, int MTH, int MB>
-    __device__ __forceinline__ void multiply(const illm_u32x4_t (&w)[NTH][2]) {
+    __device__ __forceinline__ void multiply(const illm_u32x4_t (&w)[NTH][2], bool on) {
         __builtin_amdgcn_sched_barrier(0);
         turns_wait_loads<VM>();
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(0xc07f);                    // lgkmcnt(0)
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_setprio(1);
+        if (on) {
+            __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
+            for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-            for (int i = 0; i < NTH; ++i)
+                for (int i = 0; i < NTH; ++i)
 #pragma unroll
-                for (int j = 0; j < MTH; ++j)
-                    acc[NB + i][MB + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        *(const turns_bf16x8_t*)&w[i][kk], *(const turns_bf16x8_t*)&xf[j][kk], acc[NB + i][MB + j], 0, 0, 0);
-        __builtin_amdgcn_s_setprio(0);
+                    for (int j = 0; j < MTH; ++j)
+                        acc[NB + i][MB + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            *(const turns_bf16x8_t*)&w[i][kk], *(const turns_bf16x8_t*)&xf[j][kk], acc[NB + i][MB + j], 0, 0, 0);
+            __builtin_amdgcn_s_setprio(0);
+        }
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
     }
     // Stage s of set A (P = s % 2).  ld.x1(to) asks for part X1 of stage s + 1, ld.w0, ld.x0 and ld.w1 for parts of s + 2.
+    // on0, on1: whether any of the group's rows of X0 and of X1 are there.
     template <int P, class Loads>
     __device__ __forceinline__ void stage(illm_u32x4_t* x0a, illm_u32x4_t* x1a, illm_u32x4_t* w0a, illm_u32x4_t* w1a,
-                                          illm_u32x4_t* x1b, illm_u32x4_t* w0b, Loads& ld) {
+                                          illm_u32x4_t* x1b, illm_u32x4_t* w0b, Loads& ld, bool on0 = true, bool on1 = true) {
         read_x<MT0>(x0a); ld.x1(x1b);
-        multiply<ALL + CX1, NT0, 0, MT0, 0>(w0[P]);
+        multiply<ALL + CX1, NT0, 0, MT0, 0>(w0[P], on0);
         read_w(w1, w1a); ld.w0(w0a);
-        multiply<ALL + CW0, NT1, NT0, MT0, 0>(w1);
+        multiply<ALL + CW0, NT1, NT0, MT0, 0>(w1, on0);
         read_x<MT1>(x1a); ld.x0(x0a);
-        multiply<ALL + CX0, NT1, NT0, MT1, MT0>(w1);
+        multiply<ALL + CX0, NT1, NT0, MT1, MT0>(w1, on1);
         read_w(w0[1 - P], w0b); ld.w1(w1a);
-        multiply<ALL + CW1, NT0, 0, MT1, MT0>(w0[P]);
+        multiply<ALL + CW1, NT0, 0, MT1, MT0>(w0[P], on1);
     }
     // Before the first stage, with W0 X0 W1 X1 of stage 0 and W0 X0 W1 of stage 1 asked for in this order; the second
     // group starts a turn later.  end: every wave's barriers are then as many.

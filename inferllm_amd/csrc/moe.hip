@@ -971,8 +971,9 @@ moe_rows_mfma_lds_kernel(const bf16_t* __restrict__ X, int x_div, const bf16_t* 
 // into that L2 once.
 // A loop of two stages with one barrier each, both drained (four waves, tiles of 128 pairs by 128 rows of W, two blocks a
 // compute unit) -> this one; 64 experts of 1408 x 2048, 6 chosen, gate|up + down in us: 2,964 tokens 406 + 208 -> 289 + 149
-// (700 TFLOP/s; of the rows of 192 a third are padding), 1,000 tokens 199 + 97 -> 167 + 95, 64 tokens 174 + 73 -> 139 + 70
-// (bound by reading the experts); 8 experts of 8192 x 4096, 1,024 tokens, 2 chosen 478 + 285 -> 425 + 174.
+// (of the rows of 192 a third are padding), 1,000 tokens 199 + 97 -> 167 + 95, 64 tokens 174 + 73 -> 139 + 70
+// (bound by reading the experts); 8 experts of 8192 x 4096, 1,024 tokens, 2 chosen 478 + 285 -> 425 + 174.  A group of waves without
+// pairs in an expert's last tile leaves its products out: 2,964 tokens, both products 456 -> 434, 8 of 8192 x 4096 1,421 -> 1,282.
 template <int MT0, int MT1, int NTH, bool GATED>
 __global__ void __launch_bounds__(512, 2)
 moe_turns_kernel(const bf16_t* __restrict__ X, int x_div, const bf16_t* __restrict__ W,
@@ -1019,10 +1020,11 @@ moe_turns_kernel(const bf16_t* __restrict__ X, int x_div, const bf16_t* __restri
     ld.x1(x1a);
     ld.w0(w0b); ld.x0(x0b); ld.w1(w1b);
     t.start(w0a);
-    const int stages = K / 64;
+    const int stages = K / 64, there = n - t.wm * T::MT * 16;        // (an expert's last tile may hold few pairs)
+    const bool on0 = there > 0, on1 = there > MT0 * 16;
     for (int s = 0; s < stages; s += 2) {
-        t.template stage<0>(x0a, x1a, w0a, w1a, x1b, w0b, ld);
-        if (s + 1 < stages) t.template stage<1>(x0b, x1b, w0b, w1b, x1a, w0a, ld);
+        t.template stage<0>(x0a, x1a, w0a, w1a, x1b, w0b, ld, on0, on1);
+        if (s + 1 < stages) t.template stage<1>(x0b, x1b, w0b, w1b, x1a, w0a, ld, on0, on1);
     }
     t.end();
     // acc[i][j][v]: pair wm MT 16 + 16 j + r, the i-th tile's column turns_column(i, 4 q + v)
