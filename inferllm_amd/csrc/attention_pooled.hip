@@ -137,30 +137,40 @@ extern "C" int illm_qk_rotate_store(void* rows, int dt, int row_len, int k_off, 
 }
 
 // ---------------------------------------------------------------- pooled rows of completed blocks
-// grid (rows, nkv); 256 threads.  The row at position p completes block p / pool if (p + 1) % pool
+// grid (groups of POOL_ROWS rows, nkv); 256 threads.  The row at position p completes block p / pool if (p + 1) % pool
 // == 0: its block's keys and values, which the cache holds by now, are averaged in position order.
+#define POOL_ROWS 8                                // rows of a block: most complete nothing
+template <int DT>
 __global__ void __launch_bounds__(256)
 pool_store_kernel(const int32_t* __restrict__ row_pos, const int32_t* __restrict__ row_slot,
                   const void* __restrict__ kcache, const void* __restrict__ vcache,
-                  void* __restrict__ kpool, void* __restrict__ vpool, int dt,
+                  void* __restrict__ kpool, void* __restrict__ vpool,
                   const int32_t* __restrict__ page_table, int table_stride, int page_size, int nkv,
-                  int dk, int dv, int pool) {
-    const int t = blockIdx.x, g = blockIdx.y, d = threadIdx.x;
-    const int pos = row_pos[t];
-    if ((pos + 1) % pool != 0) return;
-    const int slot = row_slot[t], b = pos / pool;
+                  int dk, int dv, int pool, int T) {
+    const int g = blockIdx.y, d = threadIdx.x;
     const float inv = 1.0f / (float)pool;
-    if (d < dk) {
-        float s = 0.f;
-        for (int j = 0; j < pool; ++j)
-            s += ld_f(kcache, dt, cache_row_offset(page_table, table_stride, slot, b * pool + j, page_size, 0, nkv, g, dk) + d);
-        st_f(kpool, dt, cache_row_offset(page_table, table_stride, slot, b, page_size, 0, nkv, g, dk) + d, s * inv);
-    }
-    if (d < dv) {
-        float s = 0.f;
-        for (int j = 0; j < pool; ++j)
-            s += ld_f(vcache, dt, cache_row_offset(page_table, table_stride, slot, b * pool + j, page_size, 0, nkv, g, dv) + d);
-        st_f(vpool, dt, cache_row_offset(page_table, table_stride, slot, b, page_size, 0, nkv, g, dv) + d, s * inv);
+    for (int t = blockIdx.x * POOL_ROWS; t < min(T, (int)(blockIdx.x + 1) * POOL_ROWS); ++t) {
+        const int pos = row_pos[t];
+        if ((pos + 1) % pool != 0) continue;
+        const int slot = row_slot[t], b = pos / pool;
+        // eight rows asked for at a time (one after the other, a look into the page table ahead of each: 2,964 rows, 4 heads of 128,
+        // blocks of 8, a block a row: 27 us; eight rows a block 10; 64 rows 5.8 -> 4.4)
+        auto mean = [&](const void* cache, void* to, int n) __attribute__((always_inline)) {
+            float s = 0.f;
+            for (int j0 = 0; j0 < pool; j0 += 8) {
+                float v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    v[j] = ld_f(cache, DT, cache_row_offset(page_table, table_stride, slot, b * pool + min(j0 + j, pool - 1), page_size,
+                                                            0, nkv, g, n) + d);
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (j0 + j < pool) s += v[j];
+            }
+            st_f(to, DT, cache_row_offset(page_table, table_stride, slot, b, page_size, 0, nkv, g, n) + d, s * inv);
+        };
+        if (d < dk) mean(kcache, kpool, dk);
+        if (d < dv) mean(vcache, vpool, dv);
     }
 }
 
@@ -172,9 +182,13 @@ extern "C" int illm_pool_store(const int32_t* row_pos, const int32_t* row_slot, 
         page_size <= 0 || !illm_dtype_ok(dt))
         return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
-    hipLaunchKernelGGL(pool_store_kernel, dim3(T, nkv), dim3(256), 0, (hipStream_t)stream, row_pos,
-                       row_slot, kcache, vcache, kpool, vpool, dt, page_table, table_stride, page_size, nkv,
-                       dk, dv, pool);
+    const dim3 grid((T + POOL_ROWS - 1) / POOL_ROWS, nkv);
+    if (dt == ILLM_BF16)
+        hipLaunchKernelGGL(pool_store_kernel<ILLM_BF16>, grid, dim3(256), 0, (hipStream_t)stream, row_pos, row_slot, kcache, vcache,
+                           kpool, vpool, page_table, table_stride, page_size, nkv, dk, dv, pool, T);
+    else
+        hipLaunchKernelGGL(pool_store_kernel<ILLM_F32>, grid, dim3(256), 0, (hipStream_t)stream, row_pos, row_slot, kcache, vcache,
+                           kpool, vpool, page_table, table_stride, page_size, nkv, dk, dv, pool, T);
     return illm_launch_status();
 }
 
