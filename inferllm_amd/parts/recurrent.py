@@ -592,6 +592,7 @@ class GatedLinearRecurrence(Mixer):
 
     graph_safe_prompts = True
     takes_continuations = True
+    takes_projected = True
 
     def __init__(self, hidden_size: int, channels: int, blocks: int, conv: int, tensors=None):
         super().__init__(tensors)
@@ -634,17 +635,17 @@ class GatedLinearRecurrence(Mixer):
     def tunables(self):
         return (("plain", self.w_o, {}),)
 
-    def forward(self, h, ctx: StepContext, line, writes_cache, position):
+    def forward(self, h, ctx: StepContext, line, writes_cache, position, projected=None):
         C = self.C
-        U = ops.linear(h, self.w_in)
+        U, at = projected if projected is not None else (ops.linear(h, self.w_in), 0)
         state = ctx.cache.state_line(line)
         S, tail = state["S"], state["tail"]
-        u = ops.short_conv(U, C, C, self.conv_w, tail, ctx.row_slot, torch.float32, bias=self.conv_b,
+        u = ops.short_conv(U, at + C, C, self.conv_w, tail, ctx.row_slot, torch.float32, bias=self.conv_b,
                            in_bias=self.x_bias, update_tail=not ctx.prefill)
         if ctx.prefill:
-            ops.short_conv_tail(U, C, tail, ctx.cu_seqlens, ctx.seq_slot, ctx.n_seqs, self.taps,
+            ops.short_conv_tail(U, at + C, tail, ctx.cu_seqlens, ctx.seq_slot, ctx.n_seqs, self.taps,
                                 in_bias=self.x_bias)
         a, x = ops.lru_gates(u, self.w_gates, self.r_bias, self.i_bias, self.lam, LRU_RATE)
-        y = ops.lru_scan(a, x, S, U, 0, self.y_bias, ctx.cu_seqlens, ctx.seq_slot, ctx.n_seqs,
+        y = ops.lru_scan(a, x, S, U, at, self.y_bias, ctx.cu_seqlens, ctx.seq_slot, ctx.n_seqs,
                          ctx.max_rows if ctx.prefill else 1, ctx.act_dtype)
         return ops.linear(y, self.w_o)
