@@ -280,7 +280,7 @@ class GatedAttention(Mixer):
     may_leave_product = True
     reads_by_product = True
     takes_continuations = True
-    takes_projected = True            # (its own products at column 0)
+    takes_projected = projected_first = True
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, key_dim: int,
                  value_dim: int, softmax_scale: Optional[float] = None, softcap: float = 0.0,

@@ -144,8 +144,9 @@ class Mixer(Part):
 
     # True: the mixer reads its input through one stacked matrix `w_in` alone, and `forward` also takes
     # `projected` = (U, column): the rows' products with that matrix, made by whoever stacked it with others
-    # (`side_by_side`), from that column of U on.
+    # (`side_by_side`), from that column of U on; with `projected_first` only from column 0 on.
     takes_projected = False
+    projected_first = False
 
     def kv_spec(self) -> Optional[KVSpec]:
         """Keys/values the mixer keeps per token, or None."""

@@ -24,7 +24,8 @@ class SideBySide(Mixer):
     of its own sets `takes_normed_pairs` and gets the pieces as `ops.NormedPair`.
 
     Mixers that both read their input through one stacked matrix (`Mixer.takes_projected`) get theirs stacked
-    into one: a single product makes the columns of both.
+    into one: a single product makes the columns of both.  A right one whose columns must begin the rows
+    (`Mixer.projected_first`) keeps its product, and the left one too.
 
     `left_position`, `right_position`: `PartSpec`s of position encodings of the mixers' own, in place of the
     block's.
@@ -69,7 +70,7 @@ class SideBySide(Mixer):
         for m, own in zip((self.left, self.right), self.own_positions):
             m.decode_copies, m.position = self.decode_copies, own if own is not None else self.position
             m.load(tensors)
-        if self.left.takes_projected and self.right.takes_projected:
+        if self.left.takes_projected and self.right.takes_projected and not self.right.projected_first:
             a, b = ops.plain_weight(self.left.w_in), ops.plain_weight(self.right.w_in)
             if a.dtype == b.dtype:
                 # (rows of zeros up to a multiple of 8, so that the right mixer's columns are as aligned as alone)
