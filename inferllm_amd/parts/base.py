@@ -175,6 +175,8 @@ class Norm(Part):
     adds_planes = False
     # the norm that a block takes of the same rows beside this one, set by the block (None: no other)
     beside = None
+    # whether that block reads rows that were prepared for its norms (`ops.linear_sum`), set by the block
+    reads_prepared = False
 
     def rms_params(self):
         """(weight, eps) if the norm is a plain RMS norm that a product's kernel may take over

@@ -27,6 +27,10 @@ class PreNormBlock(Block):
     takes_next_norm = True
     takes_prepared_rows = True
 
+    def __init__(self, mixer, feed_forward, mixer_norm, feed_forward_norm, position, tensors=None):
+        super().__init__(mixer, feed_forward, mixer_norm, feed_forward_norm, position, tensors)
+        mixer_norm.reads_prepared = mixer.takes_normed_rows
+
     @staticmethod
     def _enter(norm, part, x, pending, ctx):
         """The input of `part`: the normed rows of x (+ pending), by a kernel or prepared."""
@@ -64,9 +68,10 @@ class ParallelBlock(Block):
     float32: as a pair, if that norm says it adds pairs in its own kernel (`Norm.adds_pairs`), else
     as their float32 sum (`ops.sum_rows`).  Two parts that may leave their last products to the block
     (`Part.may_leave_product`) do so: of few rows the two products are one kernel, which adds to the stream and prepares the
-    norm that follows.  Two parts that read the rows by one product each (`Part.reads_by_product`) have those in one kernel
-    as well, of rows prepared like that without a norm's kernel ahead of it.  8 sequences, us a
-    layer in a step: the sum 14.3 + its norm 4.9 -> 14.4, the first products 10.3 + 9.7 -> 15.
+    norms that follow, where the next block reads rows prepared for them (`Norm.reads_prepared`).  Two parts that read the
+    rows by one product each (`Part.reads_by_product`) have those in one kernel as well, of rows prepared like that without a
+    norm's kernel ahead of it.  8 sequences, us a layer in a step: the sum 14.3 + its norm 4.9 -> 14.4, the first products
+    10.3 + 9.7 -> 15.
     A feed-forward that returns None (a layer without one) leaves the mixer's output alone.
     """
 
@@ -82,6 +87,15 @@ class ParallelBlock(Block):
         self.by_products = getattr(mixer, "reads_by_product", False) and getattr(feed_forward, "reads_by_product", False)
         if feed_forward_norm is not None:
             mixer_norm.beside = feed_forward_norm
+        mixer_norm.reads_prepared = self.by_products
+
+    @staticmethod
+    def _norms_to_prepare(next_norm):
+        """Weights and eps of the norms that the next block takes of these rows, if it reads them prepared."""
+        if not getattr(next_norm, "reads_prepared", False):
+            return None, None
+        params = [n.rms_params() if n is not None else None for n in (next_norm, next_norm.beside)]
+        return params if params[1] is not None or next_norm.beside is None else (None, None)
 
     def _parts(self, h, h2, ctx: StepContext, line, writes_cache):
         """The two parts' outputs."""
@@ -116,8 +130,7 @@ class ParallelBlock(Block):
         a, f = self._parts(h, h2, ctx, line, writes_cache)
         if isinstance(a, ops.Product):
             if isinstance(f, ops.Product) and ops.linear_sum_fits(a, f):
-                norms = [n.rms_params() if n is not None else None for n in (next_norm, getattr(next_norm, "beside", None))]
-                return ops.linear_sum(a, f, x, *norms)
+                return ops.linear_sum(a, f, x, *self._norms_to_prepare(next_norm))
             a = a.tensor()
         if isinstance(f, ops.Product):
             f = f.tensor()
