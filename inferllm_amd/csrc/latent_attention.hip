@@ -293,17 +293,69 @@ latent_absorb_q_kernel(void* __restrict__ y, int dt, int ncols, const void* __re
     for (int e = threadIdx.x; e < dr; e += blockDim.x) st_f(qa, qa_dt, dst + R + e, qs[dn + e]);
 }
 
-// The same for bfloat16 W_uk with R % 8 == 0, grid (B, H or H + 1, chunks of COLS latent dims): a thread holds 8 neighbouring
-// latent dims (one 16-byte load a row of W_uk) of every 16th plain dim (512 dims a block: every 4th), 8 rows asked for ahead of the query's way through LDS;
-// the groups' sums are added through LDS in group order.  Bound by trips to memory one after another: with the store, 16
-// heads of 128 x 512, blocks of a head's 512 dims that asked for four rows of W_uk at a time took 5.0 us for one row and 7.2
-// for 8, this 3.9 and 6.2.  More blocks than the chip takes at once (64 rows: 10.7 us) keep the 512 dims a block: 9.7.
-template <bool FUSED, int COLS>
+// The same for bfloat16 W_uk with R % 8 == 0 and R <= 512: a thread holds 8 neighbouring latent
+// dims (one 16-byte load a row of W_uk) and takes every (256 / (R / 8))-th plain dim; the groups'
+// sums are added through LDS in group order.  Taken where the kernel after this would have more blocks than the chip takes at once.
+template <bool FUSED>
 __global__ void __launch_bounds__(256)
 latent_absorb_q_bf16_kernel(void* __restrict__ y, int dt, int ncols,
                             const bf16_t* __restrict__ wuk, void* __restrict__ qa, int qa_dt, int H,
                             int dn, int dr, int R, LatentStore st) {
-    constexpr int LANES = COLS / 8, GROUPS = 256 / LANES, AHEAD = 8;
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    float* qs = sm;                       // [dn + dr]
+    float* part = sm + dn + dr;           // [groups][R]
+    const int b = blockIdx.x, h = blockIdx.y;
+    if (FUSED && h == H) {
+        latent_store_row(b, y, dt, ncols, H, dn, dr, R, st.rot, st.cos_sin, st.max_pos, st.nw, st.nw_dt,
+                         st.eps, st.row_pos, st.row_slot, nullptr, st.cache, st.page_table,
+                         st.table_stride, st.page_size, st.ring, nullptr, nullptr, st.cache_t, false);
+        return;
+    }
+    const size_t src = (size_t)b * ncols + (size_t)h * (dn + dr);
+    for (int d = threadIdx.x; d < dn + dr; d += 256) qs[d] = ld_f(y, dt, src + d);
+    __syncthreads();
+    if (FUSED) rotate_in_lds(qs, dn, st, b);
+    const int per_row = R / 8, groups = 256 / per_row;
+    const int c = threadIdx.x % per_row, g = threadIdx.x / per_row;
+    float acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+    if (g < groups) {
+        const bf16_t* wp = wuk + (size_t)h * dn * R + c * 8;
+#pragma unroll 4
+        for (int d = g; d < dn; d += groups) {
+            const uint4 u = *(const uint4*)(wp + (size_t)d * R);
+            const float q = qs[d];
+            const uint32_t uw[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                acc[2 * i] += q * __uint_as_float(uw[i] << 16);
+                acc[2 * i + 1] += q * __uint_as_float(uw[i] & 0xffff0000u);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) part[(size_t)g * R + c * 8 + i] = acc[i];
+    }
+    __syncthreads();
+    const size_t dst = ((size_t)b * H + h) * (size_t)(R + dr);
+    for (int r = threadIdx.x; r < R; r += 256) {
+        float a = 0.f;
+        for (int gg = 0; gg < groups; ++gg) a += part[(size_t)gg * R + r];
+        st_f(qa, qa_dt, dst + r, a);
+    }
+    for (int e = threadIdx.x; e < dr; e += 256) st_f(qa, qa_dt, dst + R + e, qs[dn + e]);
+}
+
+// Up to 512 heads of rows: grid (B, H or H + 1, chunks of 128 latent dims), a thread's 8 dims of every 16th plain dim, 8 rows of
+// W_uk asked for ahead of the query's way through LDS.  Bound by trips to memory one after another.  With the store, 16
+// heads of 128 + 64, us, the kernel above / this: 8 rows of 192 dims 5.1 / 4.4, 320 6.6 / 5.7, 512 7.3 / 6.3; 33 rows
+// 5.4 / 5.5, 6.9 / 6.3, 7.8 / 7.6; 64 rows 6.0 / 7.2, 7.8 / 8.9, 9.6 / 10.4.
+template <bool FUSED>
+__global__ void __launch_bounds__(256)
+latent_absorb_q_few_kernel(void* __restrict__ y, int dt, int ncols,
+                            const bf16_t* __restrict__ wuk, void* __restrict__ qa, int qa_dt, int H,
+                            int dn, int dr, int R, LatentStore st) {
+    constexpr int COLS = 128, LANES = COLS / 8, GROUPS = 256 / LANES, AHEAD = 8;
     extern __shared__ __attribute__((aligned(16))) float qs[];           // [dn + dr]
     __shared__ __attribute__((aligned(16))) float part[GROUPS][COLS];
     const int b = blockIdx.x, h = blockIdx.y, r0 = blockIdx.z * COLS;
@@ -367,11 +419,11 @@ static int launch_absorb_q(void* y, int dt, int ncols, const void* wuk, int w_dt
     const dim3 grid(B, FUSED ? H + 1 : H);
     if (w_dt == ILLM_BF16 && R % 8 == 0 && R <= 512 && R >= 8 && (dn + dr) * sizeof(float) <= 40 * 1024 && (uintptr_t)wuk % 16 == 0) {
         if ((long long)B * H <= 512)
-            hipLaunchKernelGGL((latent_absorb_q_bf16_kernel<FUSED, 128>), dim3(grid.x, grid.y, (R + 127) / 128), dim3(256),
+            hipLaunchKernelGGL(latent_absorb_q_few_kernel<FUSED>, dim3(grid.x, grid.y, (R + 127) / 128), dim3(256),
                                (dn + dr) * sizeof(float), stream, y, dt, ncols, (const bf16_t*)wuk, qa, qa_dt, H, dn, dr, R, st);
         else
-            hipLaunchKernelGGL((latent_absorb_q_bf16_kernel<FUSED, 512>), grid, dim3(256), (dn + dr) * sizeof(float), stream, y, dt,
-                               ncols, (const bf16_t*)wuk, qa, qa_dt, H, dn, dr, R, st);
+            hipLaunchKernelGGL(latent_absorb_q_bf16_kernel<FUSED>, grid, dim3(256), ((dn + dr) + (256 / (R / 8)) * R) * sizeof(float),
+                               stream, y, dt, ncols, (const bf16_t*)wuk, qa, qa_dt, H, dn, dr, R, st);
         return illm_launch_status();
     }
     hipLaunchKernelGGL(latent_absorb_q_kernel<FUSED>, grid, dim3(256), (size_t)(dn + dr) * sizeof(float),
