@@ -137,40 +137,55 @@ extern "C" int illm_qk_rotate_store(void* rows, int dt, int row_len, int k_off, 
 }
 
 // ---------------------------------------------------------------- pooled rows of completed blocks
-// grid (groups of POOL_ROWS rows, nkv); 256 threads.  The row at position p completes block p / pool if (p + 1) % pool
-// == 0: its block's keys and values, which the cache holds by now, are averaged in position order.
-#define POOL_ROWS 8                                // rows of a block: most complete nothing
-template <int DT>
+// grid (groups of `rows` rows, nkv); 256 threads.  The row at position p completes block p / pool if (p + 1) % pool
+// == 0: its block's keys and values, which the cache holds by now, are averaged in position order.  A thread takes V neighbouring
+// columns of a row's key or value (V 1: any sizes and addresses; a block a row then), eight rows of the cache asked for at a time, so
+// that a block's means are one trip to memory however many of its rows complete one.  Bound by that trip.  4 heads of 128, blocks of
+// 8, us, a block a row and a column a thread / eight rows one after the other / this: 2,964 rows of 8 prompts 14.6 / 10.6 / 5.8; single
+// tokens of 8 sequences that complete a block together 5.9 / 18.5 / 3.4, of 1,024 19.9 / 30.6 / 5.1; prompts with blocks of 1 18.3 / 55.8
+// / 5.1, of 3 14.7 / 23.6 / 5.4.
+template <int DT, int V>
 __global__ void __launch_bounds__(256)
 pool_store_kernel(const int32_t* __restrict__ row_pos, const int32_t* __restrict__ row_slot,
                   const void* __restrict__ kcache, const void* __restrict__ vcache,
                   void* __restrict__ kpool, void* __restrict__ vpool,
                   const int32_t* __restrict__ page_table, int table_stride, int page_size, int nkv,
-                  int dk, int dv, int pool, int T) {
-    const int g = blockIdx.y, d = threadIdx.x;
+                  int dk, int dv, int pool, int T, int rows) {
+    const int g = blockIdx.y, t0 = blockIdx.x * rows, units = (dk + dv) / V;
     const float inv = 1.0f / (float)pool;
-    for (int t = blockIdx.x * POOL_ROWS; t < min(T, (int)(blockIdx.x + 1) * POOL_ROWS); ++t) {
-        const int pos = row_pos[t];
+    for (int u = threadIdx.x; u < rows * units; u += 256) {
+        const int t = t0 + u / units, col = (u % units) * V;
+        if (t >= T) return;
+        const int pos = row_pos[t], slot = row_slot[t];
         if ((pos + 1) % pool != 0) continue;
-        const int slot = row_slot[t], b = pos / pool;
-        // eight rows asked for at a time (one after the other, a look into the page table ahead of each: 2,964 rows, 4 heads of 128,
-        // blocks of 8, a block a row: 27 us; eight rows a block 10; 64 rows 5.8 -> 4.4)
-        auto mean = [&](const void* cache, void* to, int n) __attribute__((always_inline)) {
-            float s = 0.f;
-            for (int j0 = 0; j0 < pool; j0 += 8) {
-                float v[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    v[j] = ld_f(cache, DT, cache_row_offset(page_table, table_stride, slot, b * pool + min(j0 + j, pool - 1), page_size,
-                                                            0, nkv, g, n) + d);
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (j0 + j < pool) s += v[j];
-            }
-            st_f(to, DT, cache_row_offset(page_table, table_stride, slot, b, page_size, 0, nkv, g, n) + d, s * inv);
+        const bool key = col < dk;
+        const int n = key ? dk : dv, d = key ? col : col - dk, b = pos / pool;
+        const void* const cache = key ? kcache : vcache;
+        auto at = [&](int p) __attribute__((always_inline)) {
+            return cache_row_offset(page_table, table_stride, slot, p, page_size, 0, nkv, g, n) + d;
         };
-        if (d < dk) mean(kcache, kpool, dk);
-        if (d < dv) mean(vcache, vpool, dv);
+        float s[V];
+#pragma unroll
+        for (int e = 0; e < V; ++e) s[e] = 0.f;
+        int j = 0;
+        auto take = [&](auto count) __attribute__((always_inline)) {
+            constexpr int N = decltype(count)::value;
+            float v[N][V];
+#pragma unroll
+            for (int i = 0; i < N; ++i) ldv<DT, V>(cache, at(b * pool + j + i), v[i]);
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+#pragma unroll
+                for (int e = 0; e < V; ++e) s[e] += v[i][e];
+            j += N;
+        };
+        while (j + 8 <= pool) take(std::integral_constant<int, 8>());
+        if (j + 4 <= pool) take(std::integral_constant<int, 4>());
+        if (j + 2 <= pool) take(std::integral_constant<int, 2>());
+        if (j < pool) take(std::integral_constant<int, 1>());
+#pragma unroll
+        for (int e = 0; e < V; ++e) s[e] *= inv;
+        stv<DT, V>(key ? kpool : vpool, at(b), s);
     }
 }
 
@@ -182,13 +197,19 @@ extern "C" int illm_pool_store(const int32_t* row_pos, const int32_t* row_slot, 
         page_size <= 0 || !illm_dtype_ok(dt))
         return ILLM_ERR_ARG;
     if (T == 0) return ILLM_OK;
-    const dim3 grid((T + POOL_ROWS - 1) / POOL_ROWS, nkv);
-    if (dt == ILLM_BF16)
-        hipLaunchKernelGGL(pool_store_kernel<ILLM_BF16>, grid, dim3(256), 0, (hipStream_t)stream, row_pos, row_slot, kcache, vcache,
-                           kpool, vpool, page_table, table_stride, page_size, nkv, dk, dv, pool, T);
-    else
-        hipLaunchKernelGGL(pool_store_kernel<ILLM_F32>, grid, dim3(256), 0, (hipStream_t)stream, row_pos, row_slot, kcache, vcache,
-                           kpool, vpool, page_table, table_stride, page_size, nkv, dk, dv, pool, T);
+    const int wide = dt == ILLM_BF16 ? 8 : 4;
+    const bool vec = (dk | dv) % wide == 0 && ((uintptr_t)kcache | (uintptr_t)vcache | (uintptr_t)kpool | (uintptr_t)vpool) % 16 == 0;
+    const int rows = vec ? 8 : 1;
+    const dim3 grid((T + rows - 1) / rows, nkv);
+#define GO(DT, V)                                                                                                              \
+    hipLaunchKernelGGL((pool_store_kernel<DT, V>), grid, dim3(256), 0, (hipStream_t)stream, row_pos, row_slot, kcache, vcache, \
+                       kpool, vpool, page_table, table_stride, page_size, nkv, dk, dv, pool, T, rows)
+    if (dt == ILLM_BF16) {
+        if (vec) GO(ILLM_BF16, 8);
+        else GO(ILLM_BF16, 1);
+    } else if (vec) GO(ILLM_F32, 4);
+    else GO(ILLM_F32, 1);
+#undef GO
     return illm_launch_status();
 }
 

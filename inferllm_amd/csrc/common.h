@@ -205,6 +205,36 @@ static inline int illm_launch_status() {
 
 static inline bool illm_dtype_ok(int dt) { return dt == ILLM_F32 || dt == ILLM_BF16; }
 
+// V neighbouring elements as float32, and back (stv): bfloat16 V = 8 (16 bytes), float32 V = 4, or V = 1.
+template <int DT, int V>
+__device__ __forceinline__ void ldv(const void* p, size_t i, float* o) {
+    if (V == 8) {
+        const uint4 u = *(const uint4*)((const bf16_t*)p + i);
+        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            o[2 * j] = __uint_as_float(w[j] << 16);
+            o[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
+        }
+    } else if (V == 4) {
+        const float4 f = *(const float4*)((const float*)p + i);
+        o[0] = f.x; o[1] = f.y; o[2] = f.z; o[3] = f.w;
+    } else {
+        o[0] = DT == ILLM_BF16 ? bf16_to_f32(((const bf16_t*)p)[i]) : ((const float*)p)[i];
+    }
+}
+
+template <int DT, int V>
+__device__ __forceinline__ void stv(void* p, size_t i, const float* v) {
+    if (V == 8)
+        *(uint4*)((bf16_t*)p + i) = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
+                                               pack_bf16x2(v[6], v[7]));
+    else if (V == 4)
+        *(float4*)((float*)p + i) = make_float4(v[0], v[1], v[2], v[3]);
+    else
+        st_f(p, DT, i, v[0]);
+}
+
 // Where position `pos` of the sequence in `slot` lies in a paged cache line laid
 // out as [page][kv head][row in page][head_dim].  `ring` > 0: the first `kept` logical pages of
 // a sequence stay and of the later ones only the last `ring` are kept (a window).

@@ -462,25 +462,6 @@ extern "C" int illm_moe_group(const int32_t* idx, int NP, int NEr, int32_t* orde
 }
 
 // ---------------------------------------------------------------- the experts' products
-// V elements of a row as float32: bfloat16 V = 8 (one 16-byte load), float32 V = 4, or V = 1.
-template <int DT, int V>
-__device__ __forceinline__ void ldv(const void* p, size_t i, float* o) {
-    if (V == 8) {
-        const uint4 u = *(const uint4*)((const bf16_t*)p + i);
-        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            o[2 * j] = __uint_as_float(w[j] << 16);
-            o[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
-        }
-    } else if (V == 4) {
-        const float4 f = *(const float4*)((const float*)p + i);
-        o[0] = f.x; o[1] = f.y; o[2] = f.z; o[3] = f.w;
-    } else {
-        o[0] = DT == ILLM_BF16 ? bf16_to_f32(((const bf16_t*)p)[i]) : ((const float*)p)[i];
-    }
-}
-
 // grid (tiles, column groups).  X rows: pair p reads row p / x_div of X (x_div = top for the
 // tokens' rows, 1 for rows that are per pair already).  GATED: W holds [gate (N) | up (N)] rows per
 // expert and Y = silu(X Wg^T) * (X Wu^T); else Y = X W^T.  Y rows are per pair.  A wave takes two

@@ -32,3 +32,36 @@ def test_means_of_completed_blocks(lens, pool, dk, dv, dtype):
     on = [t.to(DEV) for t in (pos, slot, *caches, *pooled, table)]
     ops.pool_store(*on, page, nkv, dk, dv, pool)
     assert torch.equal(on[4].cpu(), want[0]) and torch.equal(on[5].cpu(), want[1])
+
+
+@pytest.mark.parametrize("T, pool, dk, dv, shift", [(9, 8, 128, 128, 0), (17, 5, 64, 8, 0), (8, 13, 256, 256, 0), (33, 3, 36, 20, 0),
+                                                    (9, 7, 128, 64, 1), (8, 1, 7, 250, 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_sequences_that_complete_a_block_together(T, pool, dk, dv, shift, dtype):
+    """One token of every sequence, each the last of its block (a block of the launch has up to 8 means to form), eight or four
+    columns a thread and one, rows that do not lie on 16 bytes."""
+    nkv, page = 2, 16
+    per = -(-3 * pool // page)
+    g = torch.Generator().manual_seed(T + pool)
+
+    def rows(n, fill=None):
+        t = torch.randn(T * per * nkv * page * n + shift, generator=g) if fill is None else torch.full((T * per * nkv * page * n + shift,), fill)
+        return t.to(dtype)[shift:].view(T * per, nkv, page, n)
+    table = torch.randperm(T * per, generator=g).int().view(T, per)
+    caches, pooled = [rows(n) for n in (dk, dv)], [rows(n, 7.0) for n in (dk, dv)]
+    pos, slot = torch.tensor([pool * (1 + i % 3) - 1 for i in range(T)]).int(), torch.randperm(T, generator=g).int()
+    want = [p.clone() for p in pooled]
+    for p, s in zip(pos.tolist(), slot.tolist()):
+        for c, w in zip(caches, want):
+            a = torch.zeros(nkv, c.shape[-1])
+            for j in range(p + 1 - pool, p + 1):
+                a += c[table[s, j // page], :, j % page].float()
+            b = p // pool
+            w[table[s, b // page], :, b % page] = (a * (torch.tensor(1.0) / pool)).to(dtype)
+
+    def put(t):                                   # (a view that begins `shift` elements into its memory)
+        flat = torch.empty(t.numel() + shift, dtype=t.dtype, device=DEV)
+        return flat[shift:].view(t.shape).copy_(t)
+    on = [pos.to(DEV), slot.to(DEV), *map(put, caches), *map(put, pooled), table.to(DEV)]
+    ops.pool_store(*on, page, nkv, dk, dv, pool)
+    assert torch.equal(on[4].cpu(), want[0]) and torch.equal(on[5].cpu(), want[1])
