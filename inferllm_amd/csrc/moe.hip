@@ -1174,7 +1174,8 @@ moe_combine_kernel(const void* __restrict__ h, int dt, const int32_t* __restrict
 // The same with V neighbouring columns a thread (16-byte loads from 16-byte addresses; E % V == 0, top <= MOE_COMBINE_TOP) and a
 // block a token: the gate's dot product is formed once a token, and all of a thread's rows are asked for
 // together (2,964 tokens of 2,048, 6 chosen: 157 -> 25 us; 8 tokens 7.0 -> 5.0; in a graph, with the choice's test ahead of each
-// load 19.0 and 3.6, without 17.3 and 2.7).  Up to MOE_COMBINE_FEW tokens a
+// load 19.0 and 3.6, without 17.3 and 2.7; of one or two choices no more are asked for than two: 2,964 tokens, one chosen, with eight
+// 11.0, with two 9.1).  Up to MOE_COMBINE_FEW tokens a
 // block 256 V columns of a token, each with the gate's product for itself: tokens of 7,168, 8 chosen, one block
 // against several, by column first: 8 tokens 12.7, 14.4, 7.9 us; 128 tokens 37, 14.7, 9.4; 256 tokens in float32
 // 49, 17.8, 22.4.
@@ -1242,9 +1243,11 @@ extern "C" int illm_moe_combine(const void* h, int dt, const int32_t* idx, const
     hipLaunchKernelGGL((moe_combine_vec_kernel<DT, V, TOP>), dim3(T, parts), dim3(256), 0, (hipStream_t)stream, h, idx, wt, Y, \
                        shared, sg, sg_dt, out, E, top, NEr)
         if (dt == ILLM_BF16) {
-            if (top <= 8) ILLM_COMBINE(ILLM_BF16, 8, 8);
+            if (top <= 2) ILLM_COMBINE(ILLM_BF16, 8, 2);
+            else if (top <= 8) ILLM_COMBINE(ILLM_BF16, 8, 8);
             else ILLM_COMBINE(ILLM_BF16, 8, 16);
-        } else if (top <= 8) ILLM_COMBINE(ILLM_F32, 4, 8);
+        } else if (top <= 2) ILLM_COMBINE(ILLM_F32, 4, 2);
+        else if (top <= 8) ILLM_COMBINE(ILLM_F32, 4, 8);
         else ILLM_COMBINE(ILLM_F32, 4, 16);
 #undef ILLM_COMBINE
         return illm_launch_status();

@@ -64,3 +64,8 @@ def test_combine_with_choices_that_are_no_experts(T, E, top, NEr, dtype, weights
         gate = torch.sigmoid((h.double() * sg.double()).sum(1, keepdim=True))
         want, size = want + gate * sh.double(), size + 8 * sh.double().abs()         # (the gate's own sum of E products)
     assert bool(((got.double() - want).abs() <= (top + 4 + (E if shared else 0)) * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("T, E, top, dtype", [(3, 264, 2, torch.bfloat16), (131, 2056, 1, torch.bfloat16), (9, 12, 2, torch.float32)])
+def test_combine_of_one_or_two_choices(T, E, top, dtype):
+    test_combine_with_choices_that_are_no_experts(T, E, top, 4, dtype, True, True)
