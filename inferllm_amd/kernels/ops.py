@@ -2443,9 +2443,30 @@ def memory_finish(o: torch.Tensor, em: torch.Tensor, weight: torch.Tensor, Z: to
     return out
 
 
-def mixer_step_fits(U: torch.Tensor, dk: int, dv: int, act_dtype: torch.dtype) -> bool:
-    """Whether csrc/mixer_steps.hip takes single tokens of these projections and head sizes."""
-    return U.is_cuda and U.dtype == act_dtype and U.is_contiguous() and U.shape[0] <= 65535 and 0 < dk <= 256 and 0 < dv <= 256
+# Up to so many heads of rows (rows x heads) the one kernel of a mixer's step is the faster way: a block takes a head of a row with 16
+# waves however small its state [dk, dv], so with many heads the kernels of their own, which share blocks, catch up, the sooner
+# the smaller the state; a wave's lanes also form the decays of gated linear attention alone, `rank` terms in a row each.
+# us, kernels of their own / one, at that many heads:
+#   matrix memory      32 x 32: 512 10.8 / 8.3, 1,024 12.2 / 12.5;  32 x 64: 1,024 16.6 / 13.0, 4,096 32.9 / 38.3;
+#                      64 x 128: 4,096 83.5 / 53.5;  128 x 128: 8,192 299 / 224
+#   gated linear       rank 16  32 x 64: 1,024 19.9 / 11.8, 4,096 30.9 / 36.0;  64 x 128: 4,096 62.6 / 50.8, 8,192 106 / 115
+#   attention          rank 32  64 x 64: 1,024 23.3 / 16.1, 4,096 43.9 / 48.5;  rank 64  64 x 128: 512 21.1 / 18.5, 1,024 28.9 / 32.1;
+#                      rank 128  128 x 128: 16 16.9 / 17.9, 2,048 78 / 120;  rank 256  64 x 128: 2,048 75 / 163, 8,192 141 / 644
+#   state-space        16 x 128: 256 11.4 / 11.2, 512 12.5 / 13.7;  64 x 64: 512 13.9 / 13.2, 1,024 16.5 / 18.3;
+#                      128 x 64: 4,096 60.6 / 57.3, 8,192 110 / 130;  128 x 128: 8,192 235 / 214
+def mixer_step_heads(kind: str, dk: int, dv: int, rank: int = 0) -> int:
+    size = dk * dv
+    if kind == "state_space":
+        return size // 2 if size >= 8192 else max(256, size // 8)
+    if rank > 64:
+        return 0
+    return 512 if rank > 32 else max(512, size // 4) if rank > 16 else max(512, size // 2)
+
+
+def mixer_step_fits(U: torch.Tensor, H: int, dk: int, dv: int, act_dtype: torch.dtype, kind: str, rank: int = 0) -> bool:
+    """Whether csrc/mixer_steps.hip takes single tokens of these projections and head sizes and is the faster way."""
+    return (U.is_cuda and U.dtype == act_dtype and U.is_contiguous() and U.shape[0] <= 65535 and 0 < dk <= 256 and 0 < dv <= 256
+            and U.shape[0] * H <= mixer_step_heads(kind, dk, dv, rank))
 
 
 def memory_step(U: torch.Tensor, i_off: int, f_off: int, z_off: int, i_bias: torch.Tensor, f_bias: torch.Tensor, cap: float,
@@ -2470,8 +2491,8 @@ def memory_step(U: torch.Tensor, i_off: int, f_off: int, z_off: int, i_bias: tor
 def gla_step_fits(U: torch.Tensor, a_off: int, w_a2, dk: int, dv: int, act_dtype: torch.dtype) -> bool:
     """Whether `gla_step` takes these: as `mixer_step_fits`, the decays' inner numbers in whole groups of four."""
     w = plain_weight(w_a2)
-    return (mixer_step_fits(U, dk, dv, act_dtype) and w.dtype == U.dtype and w.is_contiguous()
-            and (w.shape[1] | a_off | U.shape[1]) % 4 == 0 and _on16(U, w))
+    return (mixer_step_fits(U, w.shape[0] // dk, dk, dv, act_dtype, "gated_linear", w.shape[1]) and w.dtype == U.dtype
+            and w.is_contiguous() and (w.shape[1] | a_off | U.shape[1]) % 4 == 0 and _on16(U, w))
 
 
 def gla_step(U: torch.Tensor, q_off: int, k_off: int, v_off: int, z_off: int, a_off: int, w_a2, a2_bias: torch.Tensor,
@@ -2494,9 +2515,9 @@ def gla_step(U: torch.Tensor, q_off: int, k_off: int, v_off: int, z_off: int, a_
     return out
 
 
-def ssm_step_fits(U: torch.Tensor, N: int, dv: int, part: int, act_dtype: torch.dtype) -> bool:
+def ssm_step_fits(U: torch.Tensor, H: int, N: int, dv: int, part: int, act_dtype: torch.dtype) -> bool:
     """Whether `ssm_step` takes these: as `mixer_step_fits`, the norm's parts of at most 2,048 columns."""
-    return mixer_step_fits(U, N, dv, act_dtype) and part <= 2048
+    return mixer_step_fits(U, H, N, dv, act_dtype, "state_space") and part <= 2048
 
 
 def ssm_step(U: torch.Tensor, x_off: int, dt_off: int, z_off: int, conv_w: torch.Tensor, conv_b: torch.Tensor,

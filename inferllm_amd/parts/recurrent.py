@@ -88,7 +88,7 @@ class StateSpaceDuality(Mixer):
         U = projected[0] if projected is not None else ops.linear(h, self.w_in)
         state = ctx.cache.state_line(line)
         S, tail = state["S"], state["tail"]
-        if not ctx.prefill and ops.ssm_step_fits(U, self.N, self.dv, self.inner // self.norm_groups, ctx.act_dtype):
+        if not ctx.prefill and ops.ssm_step_fits(U, self.H, self.N, self.dv, self.inner // self.norm_groups, ctx.act_dtype):
             y = ops.ssm_step(U, self.inner, 2 * self.inner + 2 * self.G * self.N, 0, self.conv_w, self.conv_b, tail, S, ctx.row_slot,
                              self.a_log, self.dt_bias, self.D, self.norm_w, self.norm_groups, self.eps, self.G, self.H, self.N,
                              self.dv)
@@ -170,7 +170,7 @@ class MatrixMemory(Mixer):
     def forward(self, h, ctx: StepContext, line, writes_cache, position, projected=None):
         U = projected[0] if projected is not None else ops.linear(h, self.w_in)
         state = ctx.cache.state_line(line)
-        if not ctx.prefill and ops.mixer_step_fits(U, self.dk, self.dv, ctx.act_dtype):
+        if not ctx.prefill and ops.mixer_step_fits(U, self.H, self.dk, self.dv, ctx.act_dtype, "memory"):
             y = ops.memory_step(U, self.i_off, self.f_off, self.z_off, self.i_bias, self.f_bias, self.cap, state["m"], state["S"],
                                 ctx.row_slot, self.norm_w, self.H, self.dk, self.dv, self.eps)
             return self.leave(y, self.w_o)
@@ -245,7 +245,13 @@ class GatedLinearAttention(Mixer):
             y = ops.gla_step(U, 0, H * dk, 2 * H * dk, self.g_off, self.a_off, self.w_a2, self.a2_bias, self.tau, S, ctx.row_slot,
                              self.norm_w, H, dk, dv, self.eps)
             return ops.linear(y, self.w_o)
-        Z = ops.linear(U[:, self.a_off:].contiguous(), self.w_a2)
+        inner = U[:, self.a_off:].contiguous()
+        if ctx.prefill:
+            Z = ops.linear(inner, self.w_a2)
+        elif inner.shape[0] <= ops.SKINNY_MAX_ROWS:          # (single tokens' decays from float32 sums, as the one kernel has them)
+            Z = ops.linear(inner, self.w_a2, torch.float32)
+        else:
+            Z = ops.gemm_generic(inner, ops.plain_weight(self.w_a2), torch.float32)
         qn, kn, vv, weight, dec = ops.gla_prepare(U, 0, H * dk, 2 * H * dk, Z, self.a2_bias, self.tau, H, dk, dv)
         o = ops.delta_scan(qn, kn, vv, weight, dec, S, ctx.cu_seqlens, ctx.seq_slot, ctx.n_seqs,
                            ctx.max_rows if ctx.prefill else 1, correct=False)
