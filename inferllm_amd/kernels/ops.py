@@ -1393,12 +1393,15 @@ def qkv_rope_store(x, w_qkv, cos_sin: torch.Tensor,
 
 # csrc/gemm_short.hip takes q|k|v of 17 to 256 rows with rotation and cache store, and gate|up of 129 to 192 (to 160 with more than
 # SHORT_OUTPUTS columns each) with the activation.  us, weights cold, the vendor GEMM and the elementwise kernel -> these:
-#   q|k|v    6144 x 4096   96 rows 33 -> 19 (of it host time), 144 43 -> 24, 192 38 -> 26, 256 45 -> 34
-#            12288 x 4096  17 rows 36 -> 23, 96 36 -> 29, 160 43 -> 36, 256 55 -> 51
-#            15360 x 5120  17 rows 38 -> 33, 160 54 -> 48, 256 71 -> 67;  10240 x 8192  40 rows 46 -> 37, 160 77 -> 48, 256 95 -> 67
-#   gate|up  2 x 11008 x 4096  144 rows 60 -> 49, 192 65 -> 55, 224 68 -> 62, 256 64 -> 87 (128, the fused kernel of few rows: 45 -> 44)
-#            2 x 14336 x 4096  144 rows 68 -> 62, 192 76 -> 69, 224 76 -> 91;  2 x 13824 x 5120  160 rows 79 -> 76, 192 85 -> 83
-#            2 x 28672 x 8192  144 rows 204 -> 193, 160 206 -> 198, 192 214 -> 227
+#   q|k|v    6144 x 4096   17 rows 20 -> 16, 64 22 -> 18, 144 43 -> 24, 192 38 -> 27, 256 44 -> 34
+#            12288 x 4096  17 rows 29 -> 25, 64 31 -> 27, 160 43 -> 39, 256 55 -> 52
+#            15360 x 5120  17 rows 37 -> 35, 160 57 -> 53, 256 70 -> 67;  10240 x 8192  17 rows 41 -> 37, 160 70 -> 47, 256 92 -> 65
+#   gate|up  2 x 11008 x 4096  144 rows 59 -> 53, 192 64 -> 57, 224 68 -> 62, 256 64 -> 87 (128, the fused kernel of few rows: 45 -> 44)
+#            2 x 14336 x 4096  144 rows 63 -> 65, 160 62 -> 67, 192 70 -> 71 (in a prompt's step, us a layer: 160 rows 176 either way, 192
+#            189 -> 186);  2 x 13824 x 5120  160 rows 78 -> 79, 192 85 -> 86;  2 x 28672 x 8192  144 rows 228 -> 199, 192 238 -> 224
+#            2 x 5632 x 2048  144 rows 29 -> 23, 192 29 -> 26;  2 x 5376 x 2048  144 rows 22.3 -> 22.6, 176 23 -> 25, 192 29 -> 25
+#            2 x 8192 x 1024  144 rows 20 -> 20, 176 19 -> 22;  2 x 1024 x 512  144 rows 9.3 -> 9.9, 176 9.6 -> 10.7
+# (Small gate|up matrices gain nothing or lose a little; they keep the activation on the float32 sums.)
 SHORT_QKV, SHORT_GATE_UP, SHORT_OUTPUTS = 256, 192, 1 << 14
 
 
@@ -1427,8 +1430,19 @@ def qkv_short_pays(M: int, K: int) -> bool:
     return M >= (SHORT_STEPS if K <= 4096 else SHORT_STEPS_K)
 
 
+def qkv_short_rows(N: int, K: int) -> int:
+    """Up to how many rows csrc/gemm_short.hip is the faster way for q|k|v [N, K]: of small and of narrow matrices the vendor GEMM has
+    the whole in its caches, and its time hardly grows with the rows.  us, vendor GEMM and elementwise kernel / this, weights
+    cold:  768 x 768  64 rows 10.1 / 8.5, 112 9.7 / 10.6, 256 9.9 / 14.8;  1280 x 8192  64 rows 24.9 / 18.4, 144 23.6 / 27.1;
+    3072 x 2048  144 rows 15.7 / 15.5, 208 16.6 / 18.2;  4096 x 2048  160 rows 19.8 / 18.2, 224 16.9 / 20.7;  6144 x 2048  160 rows
+    20.9 / 19.7, 208 20.0 / 22.2;  7680 x 2560  208 rows 27.1 / 27.7, 256 36.6 / 30.1;  3072 x 4096  224 rows 25.1 / 23.3."""
+    if (N >= 3072 and K >= 3072) or N * K >= 15 << 20:
+        return SHORT_QKV
+    return 160 if N >= 1536 and N * K >= 1 << 20 else 96
+
+
 def gate_up_short_fits(x, w_gate_up) -> bool:
-    """Whether csrc/gemm_short.hip takes the gate and up products of these rows and is the faster way."""
+    """Whether csrc/gemm_short.hip takes the gate and up products of these rows."""
     return (_short_fits(x, w_gate_up, "gate_up") and w_gate_up.plain.shape[0] % 16 == 0
             and ROWS_MAX < x.shape[0] <= (SHORT_GATE_UP if w_gate_up.plain.shape[0] <= 2 * SHORT_OUTPUTS else 160))
 

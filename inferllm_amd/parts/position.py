@@ -108,7 +108,7 @@ class Rotary(PositionEncoding):
 
     def project_qkv(self, h, w_qkv, ctx: StepContext, nh, nkv, hd, kcache, vcache, group):
         if kcache is not None and self.pairing == "half" and self.rotary_dim == hd and kcache.dtype == h.dtype:
-            short = ops.qkv_short_fits(h, w_qkv, hd)
+            short = ops.qkv_short_fits(h, w_qkv, hd) and h.shape[0] <= ops.qkv_short_rows(*w_qkv.shape)
             if not ctx.prefill and ops.qkv_rope_store_fits(h, w_qkv, hd) and not (short and ops.qkv_short_pays(*h.shape)):
                 return ops.qkv_rope_store(h, w_qkv, self.table(ctx.device), ctx.row_pos, ctx.row_slot,
                                           kcache, vcache, group.table, group.page_size, group.ring,

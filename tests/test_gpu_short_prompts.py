@@ -104,3 +104,9 @@ def test_cut_products_of_wide_blocks(M, N, K, splits):
     assert planes.shape == (splits, M, N)
     want, room = (x.double() @ w.double().t(), K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()))
     assert bool(((planes.double().sum(0) - want).abs() <= room).all())
+
+
+def test_small_and_narrow_matrices_of_a_short_prompt_stay_with_the_vendor_gemm():
+    """(N, K) and the rows up to which q|k|v goes to the kernel: each side measured faster there."""
+    assert [ops.qkv_short_rows(N, K) for N, K in ((768, 768), (1280, 8192), (1536, 1024), (4096, 2048), (6144, 2048), (7680, 2560),
+                                                   (3072, 4096), (12288, 4096))] == [96, 96, 160, 160, 160, 256, 256, 256]
