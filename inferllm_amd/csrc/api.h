@@ -246,15 +246,15 @@ int illm_gemm_turns_gate_up(const void* X, const void* W, void* Y, int M, int F,
 int illm_gemm_turns_tiles(int M, int F, int* shape);
 // Up to 256 rows (csrc/gemm_short.hip) from the tiled copies of gate|up (F % 8 == 0) and of q|k|v, less than 4 GiB of either,
 // bfloat16 on 16-byte addresses, K % 64 == 0: the product in float32 planes P [splits][M][W's rows], then the activation, or the
-// rotation with q, k and v into Y [M, (nh + 2 nkv) hd] and k and v to where illm_rope_store stores them.  tb, splits: tiles a block
-// takes (to 14, with M rows 26 - 2 ceil(M / 32)) and parts of K; tb 0: the kernel's choice, illm_gemm_short_splits the parts.
+// rotation with q, k and v into Y [M, (nh + 2 nkv) hd] and k and v to where illm_rope_store stores them.  splits:
+// illm_gemm_short_splits.
 int illm_gemm_short_splits(int M, int rows, int K);
 int illm_gemm_short_gate_up(const void* X, const void* Wt, void* P, size_t p_bytes, void* Y, int M, int F, int K, float limit,
-                            float alpha, int tb, int splits, void* stream);
+                            float alpha, void* stream);
 int illm_gemm_short_qkv(const void* X, const void* Wt, void* P, size_t p_bytes, void* Y, int M, int K, const float* cos_sin,
                         int max_pos, const int32_t* row_pos, const int32_t* row_slot, const int32_t* slot_len, void* kcache,
                         void* vcache, const int32_t* page_table, int table_stride, int page_size, int ring, int nh, int nkv,
-                        int hd, int tb, int splits, void* stream);
+                        int hd, void* stream);
 // The sum of two products of at most 16 rows, float32 Y = X . W^T + X2 . W2^T, from the tiled copies (K, K2 % 128 == 0).
 int illm_gemm_skinny_sum_parts(int M, int N, int K, int K2);
 int illm_gemm_skinny_sum(const void* X, const void* Wt, int K, const void* X2, const void* W2t, int K2, float* Y, int M,

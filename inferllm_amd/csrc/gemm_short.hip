@@ -7,10 +7,12 @@
 // A block takes all rows, up to 14 tiles of W and a part of K, 64 k a stage, two or three stages ahead, one barrier a stage.  X and W
 // go straight from memory into LDS, W in operand order.  The rows are two groups of waves', the tiles WN waves' of each.
 //
-// What bounds it: a compute unit brings in some 38 GB/s of X (from L2) and W (from memory) together, whatever is under way (two or three
-// stages), so a part of K is what keeps X small, and its planes are paid for it: 160 rows, us, whole K a block with rotation or
-// activation behind the sums / K in two with the planes' kernel / the vendor GEMM with theirs: 12288 x 4096 50 / 35.5 / 43.3,
-// 22016 x 4096 54 / 49.6 / 57.9.
+// X (from L2) costs a block as much as W (from memory), so a part of K is what keeps X small, and its planes are paid for it: 160
+// rows, us, whole K a block with rotation or activation behind the sums / K in two with the planes' kernel / the vendor GEMM with
+// theirs: 12288 x 4096 50 / 35.5 / 43.3, 22016 x 4096 54 / 49.6 / 57.9.
+// What a stage waits for is open.  It takes as long as its bytes of X and W at some 38 GB/s a compute unit, with two or three stages under
+// way; that is neither memory's rate nor L2's (loads alone bring 120 to 146 GB/s from L2 into LDS, and in gemm_tiles.hip 60 % of a
+// stage remains with W in L2).
 #include <math.h>
 
 #include "api.h"
@@ -200,7 +202,10 @@ qkv_planes_kernel(const float* __restrict__ P, bf16_t* __restrict__ Y, int S, in
 struct ShortShape { int tb, splits; };
 
 // Tiles a block and parts of K: the least of what a compute unit's rounds of blocks bring in and of the planes, written and
-// read at the rate of all 256.
+// read at the rate of all 256.  Both rates are fits: 64 to 256 rows of 12288 x 4096, 6144 x 4096 and 15360 x 5120 take 0.85 to
+// 1.27 of what they give, and the choice is within 3 % of the best of a dozen others.  Where two are near each other it changes with
+// the rows: 12288 x 4096, us, 6 tiles and 2 parts / 12 and 4: 96 rows 29.0 / 31.5, 112 31.8 / 32.6, 128 32.6 / 33.5, 144 35.5 /
+// 35.8, 160 36.0 / 36.9, 161 38.6 / 37.3, 192 40.6 / 40.2, 224 44.8 / 45.3.
 static ShortShape short_shape(int M, int tiles, int K) {
     const int mt = (M + 31) / 32, most = min(14, 26 - 2 * mt);
     ShortShape best = {2, 1};
@@ -236,14 +241,10 @@ static int launch_short(const bf16_t* X, const bf16_t* Wt, float* P, int M, int 
     return ILLM_ERR_ARG;
 }
 
-static int short_planes(const void* X, const void* Wt, float* P, size_t p_bytes, int M, int K, int tiles, int tb, int splits,
-                        ShortShape* taken, hipStream_t st) {
-    ShortShape shape = short_shape(M, tiles, K);
-    if (tb > 0) shape = {tb, splits};
-    const int every = K / 64, per = (every + shape.splits - 1) / shape.splits;
-    if (shape.splits < 1 || (long long)(shape.splits - 1) * per >= every || shape.tb > min(14, 26 - 2 * ((M + 31) / 32)) ||
-        (size_t)shape.splits * M * tiles * 64 > p_bytes)
-        return ILLM_ERR_ARG;
+static int short_planes(const void* X, const void* Wt, float* P, size_t p_bytes, int M, int K, int tiles, ShortShape* taken,
+                        hipStream_t st) {
+    const ShortShape shape = short_shape(M, tiles, K);
+    if ((size_t)shape.splits * M * tiles * 64 > p_bytes) return ILLM_ERR_ARG;
     *taken = shape;
     const bf16_t *x = (const bf16_t*)X, *w = (const bf16_t*)Wt;
     switch ((M + 31) / 32) {
@@ -268,11 +269,11 @@ extern "C" int illm_gemm_short_splits(int M, int rows, int K) {
 }
 
 extern "C" int illm_gemm_short_gate_up(const void* X, const void* Wt, void* P, size_t p_bytes, void* Y, int M, int F, int K,
-                                       float limit, float alpha, int tb, int splits, void* stream) {
-    if (F <= 0 || F % 8 || !short_args(X, Wt, P, Y, M, 2LL * F, K) || !(limit >= 0.f) || tb < 0) return ILLM_ERR_ARG;
+                                       float limit, float alpha, void* stream) {
+    if (F <= 0 || F % 8 || !short_args(X, Wt, P, Y, M, 2LL * F, K) || !(limit >= 0.f)) return ILLM_ERR_ARG;
     const int tiles = F / 8;
     ShortShape shape;
-    const int rc = short_planes(X, Wt, (float*)P, p_bytes, M, K, tiles, tb, splits, &shape, (hipStream_t)stream);
+    const int rc = short_planes(X, Wt, (float*)P, p_bytes, M, K, tiles, &shape, (hipStream_t)stream);
     if (rc != ILLM_OK) return rc;
     hipLaunchKernelGGL(gate_up_planes_kernel, dim3((tiles + 255) / 256, M), dim3(256), 0, (hipStream_t)stream, (const float*)P,
                        (bf16_t*)Y, shape.splits, M, tiles, limit, alpha);
@@ -282,15 +283,14 @@ extern "C" int illm_gemm_short_gate_up(const void* X, const void* Wt, void* P, s
 extern "C" int illm_gemm_short_qkv(const void* X, const void* Wt, void* P, size_t p_bytes, void* Y, int M, int K,
                                    const float* cos_sin, int max_pos, const int32_t* row_pos, const int32_t* row_slot,
                                    const int32_t* slot_len, void* kcache, void* vcache, const int32_t* page_table,
-                                   int table_stride, int page_size, int ring, int nh, int nkv, int hd, int tb, int splits,
-                                   void* stream) {
+                                   int table_stride, int page_size, int ring, int nh, int nkv, int hd, void* stream) {
     if (nh <= 0 || nkv <= 0 || hd <= 0 || hd % 16 || (nh + 2LL * nkv) * hd > 1 << 26 || !cos_sin || max_pos <= 0 || !row_pos ||
-        !row_slot || !kcache || !vcache || !page_table || table_stride <= 0 || page_size <= 0 || ring < 0 || tb < 0)
+        !row_slot || !kcache || !vcache || !page_table || table_stride <= 0 || page_size <= 0 || ring < 0)
         return ILLM_ERR_ARG;
     const int N = (nh + 2 * nkv) * hd, tiles = N / 16;
     if (!short_args(X, Wt, P, Y, M, N, K)) return ILLM_ERR_ARG;
     ShortShape shape;
-    const int rc = short_planes(X, Wt, (float*)P, p_bytes, M, K, tiles, tb, splits, &shape, (hipStream_t)stream);
+    const int rc = short_planes(X, Wt, (float*)P, p_bytes, M, K, tiles, &shape, (hipStream_t)stream);
     if (rc != ILLM_OK) return rc;
     const GsQkv t = {cos_sin, row_pos, row_slot, slot_len, (bf16_t*)kcache, (bf16_t*)vcache, page_table, table_stride, page_size,
                      ring, nh, nkv, hd};

@@ -755,7 +755,8 @@ extern "C" int illm_gemm_skinny_pair(const void* X, const void* Wt, void* Y, int
     // One tile a block: with two, X is read half as often, but fewer waves have loads under way (us at 8 rows, cold, the two products
     // apart / one tile / two: 10304 and 8192 x 2048 19.6 / 17.1 / 21.4, 5120 and 8192 x 2048 17.9 / 14.7 / 14.5, 3648 and 2304 x 2048
     // 11.9 / 8.9 / 9.4, 2560 and 2176 x 512 7.0 / 4.4 / 5.4, 12288 and 16384 x 4096 47.2 / 43.6 / 44.9; at 16 rows the first 23.7 / 20.2 /
-    // 24.0, the second 21.8 / 17.0 / 15.0, the last 54.5 / 53.3 / 49.0).
+    // 24.0, the second 21.8 / 17.0 / 15.0, the last 54.5 / 53.3 / 49.0; 20480 and 16384 x 4096 at 8 rows 60.6 / 52.8 / 56.0, 12 62.0 /
+    // 56.3 / 58.3, 16 66.2 / 68.8 / 61.2: a row has the same bits whatever the others, so that the shape cannot go by their number).
     const int from = (N + 15) / 16, blocks = from + (N2 + 15) / 16;
     const int waves = clamp_waves((SK_WAVES_ON_CHIP_TILED + blocks / 2) / blocks, 1, 1, 4, K);
     const SkPair two = {(const bf16_t*)X2, (const bf16_t*)W2t, Y2, N2, from};

@@ -122,8 +122,8 @@ gemm_tiles_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, fl
     }
 }
 
-// Columns a block takes.  A compute unit brings in about 38 GB/s of X (from L2) and W together: of 128 columns X is read
-// half as often, for twice the planes, which pays where a part of K is then at least 16 stages long.  us with the norm that
+// Columns a block takes.  X (from L2) costs a block as much as W (see gemm_short.hip): of 128 columns X is read half as often,
+// for twice the planes, which pays where a part of K is then at least 16 stages long.  us with the norm that
 // adds the planes, matrices cold, 160 / 256 rows, 64 -> 128 columns: 4096 x 11008 37.5 / 46.2 -> 34.9 / 43.4, 4096 x 14336
 // 43.6 / 53.6 -> 39.4 / 48.6, 8192 x 28672 155 / 192 -> 124 / 146; with parts of 8 stages 4096 x 4096 19.4 / 25.3 -> 21.6 / 27.6,
 // 2048 x 8192 19.4 / 24.9 -> 22.0 / 27.5.  (Within the 4 GiB of a load's offset.)

@@ -1473,7 +1473,7 @@ def qkv_short(x, w_qkv: "Weight", cos_sin: torch.Tensor, row_pos: torch.Tensor, 
     _check(_lib().illm_gemm_short_qkv(
         _p(x), _p(w_qkv.tiled), _p(planes), planes.numel() * 4, _p(y), M, K, _p(cos_sin), cos_sin.shape[0], _p(row_pos),
         _p(row_slot), _p(slot_len), _p(kcache), _p(vcache), _p(page_table), page_table.shape[1], page_size, ring, nh, nkv, hd,
-        0, 0, _stream()), "qkv_short")
+        _stream()), "qkv_short")
     return y
 
 
@@ -1564,7 +1564,7 @@ def gate_up_act(x, w_gate_up, limit: float = 0.0) -> torch.Tensor:
         planes = _short_planes(x, F2)
         y = torch.empty((M, F2 // 2), dtype=x.dtype, device=x.device)
         _check(_lib().illm_gemm_short_gate_up(_p(x), _p(w_gate_up.tiled), _p(planes), planes.numel() * 4, _p(y), M, F2 // 2, K,
-                                              ctypes.c_float(limit), ctypes.c_float(SWISH_ALPHA), 0, 0, _stream()),
+                                              ctypes.c_float(limit), ctypes.c_float(SWISH_ALPHA), _stream()),
                "gate_up_act (a short prompt's rows)")
         return y
     if gate_up_turns_fits(x, w_gate_up):
