@@ -733,8 +733,8 @@ attn_cap_rows_bf16_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __
         for (int s = 0; s < 2 * KT; ++s)
             sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const cap_bf16x8_t*)(ks + col * KLD + 16 * s + 8 * half),
                                                          *(const cap_bf16x8_t*)&qr[s], sc, 0, 0, 0);
-        // a tile that all of the wave's rows see whole needs no masks (chunks of 1,024: 8 sequences of 1,024 to 61 rows, 16 heads of
-        // 128 92 -> 66 us, one of 1,500 90 -> 58)
+        // a tile that all of the wave's rows see whole needs no masks (chunks of 1,024 without a bias by distance: 8 sequences of 1,024
+        // to 61 rows, 16 heads of 128 90 -> 66 us, one of 1,500 90 -> 58; with one, 91 us, every tile has them)
         const bool whole = k0 + MK - 1 <= wq_lo && q0 + 32 * wave + 31 < len && (window <= 0 || k0 > wq_hi - window) &&
                            (chunk <= 0 || (k0 >= wc_lo && wq_hi - wc_lo < chunk));
         float tm = NEG_INF;

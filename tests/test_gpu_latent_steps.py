@@ -45,3 +45,17 @@ def test_wide_latents(B, H, Rk, dr, dv, window, dn, monkeypatch):
         assert bool(torch.isfinite(got).all()), nsplit
         # a weight's and a result's rounding, 2^-9 each
         assert float((got - want).norm() / want.norm()) < 2 ** -7, nsplit
+
+
+@pytest.mark.parametrize("R_", [8, 24, 64, 200, 320, 512])
+@pytest.mark.parametrize("B", [32, 33])
+def test_queries_on_either_side_of_512_heads_of_rows(B, R_):
+    from inferllm_amd.kernels import ops
+    g, H, dn, dr, bf = torch.Generator().manual_seed(B + R_), 16, 72, 12, torch.bfloat16
+    y = torch.randn(B, H * (dn + dr) + R_ + dr + H, generator=g).to(bf)
+    wuk = (torch.randn(H * dn, R_, generator=g) * R_ ** -0.5).to(bf)
+    got = ops.latent_absorb_q(y.cuda(), wuk.cuda(), H, dn, dr, R_, torch.float32).double().cpu()
+    want = R.latent_absorb_q(y, wuk, H, dn, dr, R_, torch.float32).double()
+    # float32 sums of dn products in another order: 2 dn 2^-24 of the sum of their sizes
+    size = R.latent_absorb_q(y.abs(), wuk.abs(), H, dn, dr, R_, torch.float32).double()
+    assert bool(((got - want).abs() <= 2 * dn * 2.0 ** -24 * size).all())

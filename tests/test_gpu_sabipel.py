@@ -536,6 +536,25 @@ def _attention_cases(dtype):
             _near(got, want[last], tol)
 
 
+@pytest.mark.parametrize("slopes", [False, True])
+@pytest.mark.parametrize("chunk", [64, 96, 128])
+def test_tiles_that_all_rows_of_a_wave_see_whole_in_chunks(chunk, slopes):
+    """Chunks of whole tiles of keys and more, rows that begin and end a wave's within them, without and with a bias by distance."""
+    from inferllm_amd.kernels import ops
+    g, nh, nkv, dk, dv, bf = torch.Generator().manual_seed(chunk), 4, 2, 64, 32, torch.bfloat16
+    lens, starts, slots, page = [300, 65, 1, 130], [0, 0, 127, 61], [2, 0, 1, 3], 64
+    T, per = sum(lens), 5
+    table = torch.randperm(4 * per, generator=g).view(4, per).to(torch.int32)
+    cu, seq_slot, _ = _packed(lens, slots)
+    rows = torch.randn(T, nh * dk, generator=g).to(bf)
+    kc, vc = (torch.randn(4 * per, nkv, page, n, generator=g).to(bf) for n in (dk, dv))
+    sl = torch.pow(2.0, -8.0 * torch.arange(1, nh + 1) / nh).float() if slopes else None
+    ins = (rows, cu, seq_slot, torch.tensor(starts, dtype=torch.int32), kc, vc, table)
+    tail = (page, 0, 4, max(lens), nh, nkv, dk, dv, 0.3, 0.0, 0)
+    want = R.attn_cap_rows(*ins, *tail, sl, chunk)
+    _near(ops.attn_cap_rows(*(t.cuda() for t in ins), *tail, sl.cuda() if slopes else None, chunk), want, 2e-2)
+
+
 def test_pair_embedding_and_gelu_against_plain_torch():
     from inferllm_amd.kernels import ops
     g = torch.Generator().manual_seed(9)
